@@ -1866,6 +1866,7 @@ __global__ __launch_bounds__(64 * ROWS) void expert_scale_wave_kernel(
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 template <int DT> struct Mfma32x32x16;
@@ -2604,6 +2605,286 @@ __global__ __launch_bounds__(64 * WM * WN, TM * TN >= 16 ? 1 : 2) void dense_gem
 }
 
 #undef MOE_A2A_INTERLEAVE
+
+// ---------------------------------------------------------------- dense product, 256 columns per tile
+//
+// The same product for tiles large enough to keep the matrix cores busy. A workgroup of eight waves
+// (two per SIMD) owns 32 * TM rows x 64 * TN columns; a wave owns TM bands of 16 rows (every second band
+// of the tile) x TN columns of 16 and uses v_mfma_f32_16x16x32. What shaped it:
+//  - Power. With every matrix core busy on ordinary data the clock, not the pipe, sets the rate: from
+//    registers alone 32x32x16 runs at 1.80 PFLOP/s and 16x16x32 at 2.06 (2.4 of either on zeros), because it
+//    reads and writes an accumulator half as often per product.
+//  - Rows go from memory to LDS directly (buffer_load ... lds): no registers, no ds_write, and what is
+//    saved there is clock for the matrix cores.
+//  - Two groups of four waves take turns ("phases", a barrier apart): while one group multiplies, the other
+//    reads its next fragments (32 elements of K) and asks for rows. A wave thus needs one set of fragments,
+//    and no memory instruction ever stands between two MFMAs of the group that owns the matrix cores.
+//  - Phases have to be even: rows of one operand are requested in the first slice of a step and rows of the
+//    other in the second. All of them in one phase cost 12 % (324 against 363 us at 8192 x 8192 x 3712).
+//  - Lookahead: 160 KB hold five half-steps of 32 KB. One operand (A, or B with LONG_B) gets three buffers
+//    and is asked for two steps ahead, the other two buffers and one step; with two of each, rows that start
+//    off the 128-byte lines (K = 3696) ran 17 % longer (399 against 340 us).
+//  - Rows that start off the lines take one and three quarter times the line requests: AHEAD then brings the
+//    lines into L2 before (operands out of HBM, K = 3696: 390 -> 372 us; on aligned rows it costs 1 to 2 %).
+// Measured at 8192 x 8192 (bf16, uniform values, clocks settled): K = 3696 395 us with dense_gemm_kernel's
+// 256 x 256 tile, 340 here (1.46 PFLOP/s); K = 4096 x 4096 x 4096 107 and 90; K = 8192 795 and 702.
+//
+// Order of K: MFMA q of a step takes inputs 32 q .. 32 q + 31. The instruction adds them as two runs of 16 in
+// that order, so a row count that selects this kernel or another changes no bit of the result.
+// LDS rows are 128 bytes, the eight 16-byte vectors of a row XORed with bits 1..3 of the row number, as above;
+// a direct load writes 1 KB (eight rows) in lane order, so the lane picks the vector that belongs at its place.
+
+// 16 bytes per lane from a buffer into LDS at `base` + OFF + 16 * lane (the place travels in m0, so the
+// instruction is written out; the wait for it is the caller's, through vmcnt).
+template <int OFF>
+__device__ __forceinline__ void load_to_lds(unsigned base, int voffset, b128 rsrc, int soffset) {
+  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
+               ::"s"(base), "n"(OFF), "v"(voffset), "s"(rsrc), "s"(soffset) : "memory", "scc");
+}
+// the descriptor of such a load, as __builtin_amdgcn_make_buffer_rsrc lays it out
+__device__ __forceinline__ b128 buffer_words(const void* p, int bytes) {
+  const uint64_t a = (uint64_t)p;
+  return b128{(unsigned)a, (unsigned)(a >> 32) & 0xffffu, (unsigned)bytes, (unsigned)BUFFER_RAW_32BIT};
+}
+
+template <int I, int END, typename F>
+__device__ __forceinline__ void unrolled(F&& f) {  // f(0), f(1), ... with constants
+  if constexpr (I < END) {
+    f(std::integral_constant<int, I>{});
+    unrolled<I + 1, END>(f);
+  }
+}
+
+constexpr int WAIT_LDS_ONLY = 0xC07F;  // s_waitcnt lgkmcnt(0), the other counters left alone
+
+template <int DT> struct Mfma16x16x32;
+template <> struct Mfma16x16x32<MOE_A2A_BF16> {
+  static __device__ __forceinline__ f32x4 mma(b128 a, b128 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+};
+template <> struct Mfma16x16x32<MOE_A2A_F16> {
+  static __device__ __forceinline__ f32x4 mma(b128 a, b128 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+};
+
+constexpr int phased_rows(int TM) { return 32 * TM; }
+constexpr int phased_cols(int TN) { return 64 * TN; }
+constexpr size_t phased_lds_bytes(int TM, int TN, bool long_b) {
+  return (size_t)((long_b ? 2 : 3) * phased_rows(TM) + (long_b ? 3 : 2) * phased_cols(TN)) * 128;
+}
+
+template <int DT, int TM, int TN, bool LONG_B, bool AHEAD>
+__global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
+    const b128* __restrict__ A, const b128* __restrict__ B, const uint16_t* __restrict__ bias,
+    uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n) {
+  constexpr int BM = phased_rows(TM), BN = phased_cols(TN), GROUP_M = 4;
+  constexpr int LA = BM / 64, LB = BN / 64;  // direct loads (8 rows each) of a wave per step
+  constexpr int NA = LONG_B ? 2 : 3, NB = LONG_B ? 3 : 2;
+  constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, B_AT = NA * A_BYTES;
+  extern __shared__ b128 tile_lds[];  // [NA][BM * 8], [NB][BN * 8]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int row_vecs = K / 8, row_bytes = K * 2, steps = (K + GEMM_KSTEP - 1) / GEMM_KSTEP;
+  const int tail_vecs = row_vecs - (steps - 1) * 8;
+  const bool first_group = wave < 4;
+
+  const int logical = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int per_group = GROUP_M * tiles_n, group = logical / per_group, in = logical - group * per_group;
+  const int group_rows = min(GROUP_M, tiles_m - group * GROUP_M);
+  const int tn = in / group_rows, tm = group * GROUP_M + in - tn * group_rows;
+  const int n0 = tn * BN, rows_left = M - tm * BM;
+  uint16_t* c_tile = C + (size_t)tm * BM * N;
+
+  // As in dense_gemm_kernel: rows past the end of a matrix read as zeros (they lie past the extent), and
+  // so do the vectors past the end of a row in the last step and everything past the last step.
+  const b128 abuf = buffer_words(A + (size_t)tm * BM * row_vecs, min(BM, rows_left) * row_bytes);
+  const b128 bbuf = buffer_words(B + (size_t)n0 * row_vecs, min(BN, N - n0) * row_bytes);
+  constexpr int OUT_OF_RANGE = 0x40000000;
+  const int sub = lane >> 3;
+  auto vec_of = [&](int row) { return (lane & 7) ^ ((row >> 1) & 7); };
+  auto a_row = [&](int i) { return (wave * LA + i) * 8 + sub; };
+  auto b_row = [&](int i) { return (wave * LB + i) * 8 + sub; };
+  int aoff[LA], boff[LB];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) aoff[i] = a_row(i) * row_bytes + vec_of(a_row(i)) * 16;
+#pragma unroll
+  for (int i = 0; i < LB; ++i) boff[i] = b_row(i) * row_bytes + vec_of(b_row(i)) * 16;
+  auto a_range = [&](int step) __attribute__((always_inline)) {  // before the rows of a step near the end are asked for
+    if (step == steps - 1) {
+#pragma unroll
+      for (int i = 0; i < LA; ++i) aoff[i] += vec_of(a_row(i)) >= tail_vecs ? OUT_OF_RANGE : 0;
+    } else if (step >= steps) {
+#pragma unroll
+      for (int i = 0; i < LA; ++i) aoff[i] = OUT_OF_RANGE;
+    }
+  };
+  auto b_range = [&](int step) __attribute__((always_inline)) {
+    if (step == steps - 1) {
+#pragma unroll
+      for (int i = 0; i < LB; ++i) boff[i] += vec_of(b_row(i)) >= tail_vecs ? OUT_OF_RANGE : 0;
+    } else if (step >= steps) {
+#pragma unroll
+      for (int i = 0; i < LB; ++i) boff[i] = OUT_OF_RANGE;
+    }
+  };
+
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) b128*)tile_lds;
+  const unsigned a_base = lds0 + wave * LA * 1024, b_base = lds0 + B_AT + wave * LB * 1024;
+  int a_soff = 0, b_soff = 0;          // byte of a row at which the next requested step begins
+  unsigned a_fill = 0, b_fill = 0;     // buffer (as a byte offset) that the next requested step goes to
+  unsigned a_use = 0, b_use = 0;       // buffer of the step being multiplied
+  auto next_a = [](unsigned at) { return at == (NA - 1) * A_BYTES ? 0u : at + A_BYTES; };
+  auto next_b = [](unsigned at) { return at == (NB - 1) * B_BYTES ? 0u : at + B_BYTES; };
+  auto load_a = [&]() __attribute__((always_inline)) {
+    unrolled<0, LA>([&](auto c) __attribute__((always_inline)) {
+      constexpr int i = decltype(c)::value;
+      load_to_lds<i * 1024>(a_base + a_fill, aoff[i], abuf, a_soff);
+    });
+    a_fill = next_a(a_fill);
+    a_soff += GEMM_KSTEP * 2;
+  };
+  auto load_b = [&]() __attribute__((always_inline)) {
+    unrolled<0, LB>([&](auto c) __attribute__((always_inline)) {
+      constexpr int i = decltype(c)::value;
+      load_to_lds<i * 1024>(b_base + b_fill, boff[i], bbuf, b_soff);
+    });
+    b_fill = next_b(b_fill);
+    b_soff += GEMM_KSTEP * 2;
+  };
+
+  // AHEAD: a wave touches, four steps ahead, one line each of the rows this workgroup fetches into L2 for its
+  // neighbours as well: of the GROUP_M x 8 tiles that an XCD works on at a time, the 8 with the same rows of
+  // A share those out, and the GROUP_M with the same rows of B. What comes back is not used, but the register
+  // it comes back to stays taken until the last of these loads has been waited for.
+  constexpr int AHEAD_STEPS = 4;
+  [[maybe_unused]] uint32_t touched = 0;
+  [[maybe_unused]] int touch_off = 0;
+  [[maybe_unused]] const b128 touch_buf = first_group ? abuf : bbuf;
+  if constexpr (AHEAD) {
+    constexpr int A_EACH = BM / 8 / 4, B_EACH = BN / GROUP_M / 4;  // rows of a wave of either group
+    const int row = first_group ? (tn & 7) * (BM / 8) + wave * A_EACH + lane
+                                : (tm & (GROUP_M - 1)) * (BN / GROUP_M) + (wave - 4) * B_EACH + lane;
+    touch_off = lane < (first_group ? A_EACH : B_EACH) ? row * row_bytes : OUT_OF_RANGE;
+  }
+  auto touch = [&](int step) __attribute__((always_inline)) {
+    if constexpr (AHEAD)
+      asm volatile("buffer_load_dword %0, %1, %2, %3 offen"
+                   : "+v"(touched) : "v"(touch_off), "s"(touch_buf), "s"(min(step, steps - 1) * (GEMM_KSTEP * 2)) : "memory");
+  };
+
+  // fragment of a slice: row r of the band, vector 4 * slice + q of the step
+  const int r = lane & 15, q = lane >> 4, swz = (r >> 1) & 7;
+  const char* const lds = (const char*)tile_lds;
+  const char* a_frag[2];
+  const char* b_frag[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    a_frag[s] = lds + (wm * 16 + r) * 128 + ((s * 4 + q) ^ swz) * 16;
+    b_frag[s] = lds + B_AT + (wn * TN * 16 + r) * 128 + ((s * 4 + q) ^ swz) * 16;
+  }
+  b128 af[TM], bf[TN];
+  f32x4 acc[TM][TN] = {};
+  auto read_frags = [&](int slice) __attribute__((always_inline)) {
+    const char* ap = a_frag[slice] + a_use;
+    const char* bp = b_frag[slice] + b_use;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) bf[j] = *(const b128*)(bp + j * (16 * 128));
+#pragma unroll
+    for (int i = 0; i < TM; ++i) af[i] = *(const b128*)(ap + i * (32 * 128));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&]() __attribute__((always_inline)) {  // this wave's turn at the matrix cores
+    __builtin_amdgcn_s_waitcnt(WAIT_LDS_ONLY);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = Mfma16x16x32<DT>::mma(bf[j], af[i], acc[i][j]);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // Step s reads its buffers in both of its slices. In the first it asks for step s + 1 of the operand with
+  // two buffers (the buffer of step s - 1: the other group has read its last slice in the phase before), in
+  // the second for step s + 2 of the operand with three. Before the barrier that ends the second reading
+  // phase the wave waits for all of its loads but the ones just made: step s + 1 is then in LDS for everybody
+  // one barrier later, when the first group gets there.
+  auto one_step = [&](int step) __attribute__((always_inline)) {
+    read_frags(0);
+    if constexpr (LONG_B) load_a(); else load_b();
+    multiply();
+    read_frags(1);
+    if constexpr (LONG_B) load_b(); else load_a();
+    touch(step + AHEAD_STEPS);
+    a_use = next_a(a_use);
+    b_use = next_b(b_use);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LONG_B ? LB : LA) + (AHEAD ? 1 : 0)) : "memory");
+    multiply();
+  };
+  a_range(0);
+  b_range(0);
+  load_a();
+  load_b();
+  if constexpr (LONG_B) { b_range(1); load_b(); } else { a_range(1); load_a(); }
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LONG_B ? LB : LA) : "memory");
+  if (!first_group) asm volatile("s_barrier" ::: "memory");  // one phase behind
+  int step = 0;
+  for (; step + 3 < steps; ++step) one_step(step);  // (what it asks for lies before the last step)
+  for (; step < steps; ++step) {
+    a_range(step + (LONG_B ? 1 : 2));
+    b_range(step + (LONG_B ? 2 : 1));
+    one_step(step);
+  }
+  if (first_group) asm volatile("s_barrier" ::: "memory");
+  // (the loads past the last step write zeros)
+  if constexpr (AHEAD) asm volatile("s_waitcnt vmcnt(0)" : "+v"(touched)::"memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+
+  // Out through LDS as in dense_gemm_kernel, a band of 16 rows at a time: a lane holds columns
+  // j * 16 + q * 4 + 0..3 of row r, and a store instruction writes whole 128-byte pieces of rows.
+  {
+    constexpr int VR = TN * 2, PITCH = TN * 32 + 16, ROWS_PER_READ = 64 / VR;
+    char* park = (char*)tile_lds + wave * (16 * PITCH);
+    const int ncol = n0 + wn * TN * 16;
+    uint32_t bias2[TN][2] = {};
+    if (bias) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        if (ncol + j * 16 < N) __builtin_memcpy(bias2[j], bias + ncol + j * 16 + q * 4, 8);
+    }
+    const int rrow = lane / VR, rvec = lane % VR;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const f32x4& c = acc[i][j];
+        uint32_t two[2] = {Pair16<DT>::canonical(Pair16<DT>::round(c[0], c[1])),
+                           Pair16<DT>::canonical(Pair16<DT>::round(c[2], c[3]))};
+        if (bias) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            two[e] = Pair16<DT>::canonical(Pair16<DT>::round(
+                __fadd_rn(Pair16<DT>::lo(two[e]), Pair16<DT>::lo(bias2[j][e])),
+                __fadd_rn(Pair16<DT>::hi(two[e]), Pair16<DT>::hi(bias2[j][e]))));
+        }
+        __builtin_memcpy(park + r * PITCH + (j * 16 + q * 4) * 2, two, 8);
+      }
+#pragma unroll
+      for (int p = 0; p < 16 / ROWS_PER_READ; ++p) {
+        const int row = p * ROWS_PER_READ + rrow;
+        const b128 v = *(const b128*)(park + row * PITCH + rvec * 16);
+        const int m = i * 32 + wm * 16 + row, n = ncol + rvec * 8;
+        if (m < rows_left && n < N) *(b128*)(c_tile + (size_t)m * N + n) = v;
+      }
+    }
+  }
+}
 
 // ---------------------------------------------------------------- exchange stand-in
 
@@ -3385,26 +3666,19 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
 #endif
 constexpr int MOE_A2A_NOT_DENSE = 1;  // (internal) the shape is left to the next kernel
 
-// Which tile the dense kernel uses for an M x N x K product: 256 x 256 (one workgroup per compute
-// unit, the highest rate per unit once every unit has work for several tiles), 128 x 128 (two
-// workgroups per unit, about 0.8 of that rate, but four times the tiles: fuller last round, and
-// one workgroup's prologue and epilogue overlap the other's MFMAs, which decides short K) or
-// 64 x 128 (for outputs that even 128 x 128 tiles cannot spread over the 256 units).
-// The costs are in units of a 128 x 128 tile's work at the big tile's rate; the constants are
-// fits to measurements on an MI355X (rows 64 .. 8192, K 256 .. 4608).
-int dense_tile_rows(long long M, long long N, int K) {
+// Which tile an M x N x K product is cut into: 64 x 128 (dense_gemm_kernel) for outputs that this height
+// spreads over the 256 units once, 128 x 128 (phased_gemm_kernel, two workgroups per unit) while tiles of
+// 256 x 256 would leave more than a third of the units without work, else 256 x 256 (phased, one workgroup
+// per unit), whose rate per unit is half as high again. Measured with 256 / 128 rows, us: 2048 x 4096 x 1024
+// (128 big tiles) 24.1 / 21.5; 1024 x 8192 x 2048 (128) 38.6 / 35.7; 2048 x 2880 x 360 (96) 15.4 / 11.6;
+// 4096 x 4096 x 512 (256) 22.2 / 27.4; 8192 x 8192 x 3696 (1024) 407 / 622.
+int dense_tile_rows(long long M, long long N) {
   if (MOE_A2A_DENSE_TILE) return MOE_A2A_DENSE_TILE;
-  constexpr double UNITS = 256.0;
-  const double steps = (K + GEMM_KSTEP - 1) / GEMM_KSTEP;
-  const double big = (double)((M + 255) / 256) * (double)((N + 255) / 256);
-  const double mid = (double)((M + 127) / 128) * (double)((N + 127) / 128);
-  const double low = (double)((M + 63) / 64) * (double)((N + 127) / 128);
+  constexpr long long UNITS = 256;
+  const long long low = ((M + 63) / 64) * ((N + 127) / 128);
   if (low <= UNITS) return 64;
-  // a last round that is partly empty costs about half of what it leaves idle (the busy units
-  // run faster meanwhile); per tile, fixed work worth 3 steps (big) and 1 step (mid)
-  const double big_cost = 4.0 * 0.5 * (big / UNITS + ceil(big / UNITS)) * (steps + 3.0) / steps;
-  const double mid_cost = 1.25 * fmax(mid / UNITS, 1.0) * (steps + 1.0) / steps;
-  return big_cost <= mid_cost ? 256 : 128;
+  const long long big = ((M + 255) / 256) * ((N + 255) / 256);
+  return big > UNITS * 5 / 8 ? 256 : 128;
 }
 
 constexpr size_t dense_lds_bytes(int BM, int BN) { return 2 * (size_t)(BM + BN) * 8 * sizeof(b128); }
@@ -3422,10 +3696,12 @@ int allow_large_lds() {
   auto allow = [&](const void* kernel, size_t bytes) {
     ok = ok && hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
   };
-  allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 4, 4, false>, dense_lds_bytes(256, 256));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 4, 4, false>, dense_lds_bytes(256, 256));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, false, false>, phased_lds_bytes(8, 4, false));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, false, false>, phased_lds_bytes(8, 4, false));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, false, true>, phased_lds_bytes(8, 4, false));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, false, true>, phased_lds_bytes(8, 4, false));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 4, 2, false, false>, phased_lds_bytes(4, 2, false));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 4, 2, false, false>, phased_lds_bytes(4, 2, false));
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 4, 4, true>, dense_lds_bytes(256, 256));
@@ -3449,27 +3725,28 @@ int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, i
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
   if (!all_aligned(16, a, b, c) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
   if ((long long)K * 2 * 256 >= (1 << 30)) return MOE_A2A_NOT_DENSE;  // 32-bit byte offsets inside a tile's rows
-  const int tile = dense_tile_rows(M, N, K);
+  const int tile = dense_tile_rows(M, N);
   const int BM = tile, BN = tile == 64 ? 128 : tile;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + BN - 1) / BN;
   if (tiles_m * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
-  const size_t lds_bytes = dense_lds_bytes(BM, BN);
   const int grid = (int)(tiles_m * tiles_n);
   if (const int rc = allow_large_lds()) return rc;
-#define LAUNCH_D(DT, TM, TN)                                                             \
-  dense_gemm_kernel<DT, 2, 2, TM, TN, false><<<grid, 256, lds_bytes, st>>>(              \
-      (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n, \
-      nullptr, 0, 0, 0)
-#define LAUNCH_DT(DT)                         \
-  do {                                        \
-    if (tile == 256) LAUNCH_D(DT, 4, 4);      \
-    else if (tile == 128) LAUNCH_D(DT, 2, 2); \
-    else LAUNCH_D(DT, 1, 2);                  \
+#define LAUNCH_P(DT, TM, TN, AHEAD)                                                              \
+  phased_gemm_kernel<DT, TM, TN, false, AHEAD><<<grid, 512, phased_lds_bytes(TM, TN, false), st>>>( \
+      (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n)
+#define LAUNCH_DT(DT)                                                                            \
+  do {                                                                                           \
+    if (tile == 256 && K * 2 % 128 != 0) LAUNCH_P(DT, 8, 4, true);                               \
+    else if (tile == 256) LAUNCH_P(DT, 8, 4, false);                                             \
+    else if (tile == 128) LAUNCH_P(DT, 4, 2, false);                                             \
+    else dense_gemm_kernel<DT, 2, 2, 1, 2, false><<<grid, 256, dense_lds_bytes(64, 128), st>>>(  \
+        (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, \
+        (int)tiles_n, nullptr, 0, 0, 0);                                                         \
   } while (0)
   if (dtype == MOE_A2A_BF16) LAUNCH_DT(MOE_A2A_BF16);
   else LAUNCH_DT(MOE_A2A_F16);
 #undef LAUNCH_DT
-#undef LAUNCH_D
+#undef LAUNCH_P
   return launch_status();
 }
 

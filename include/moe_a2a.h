@@ -363,11 +363,11 @@ int moe_a2a_expert_gemm(const moe_a2a_shape* shape, const void* expert_x,
  * float32 with one rounding to the 16-bit type; a bias is then added to that
  * rounded value and the sum rounded again, which is what the two torch
  * statements do. bias may be NULL.
- * One of three kernels runs, picked from the shape alone (so a shape always
+ * One of four kernels runs, picked from the shape alone (so a shape always
  * gives the same bits): for m <= 64, k >= 449 (eight steps of 64 elements) and
  * n <= 24448 (fewer than 192 tiles of 128 columns), a kernel whose
  * workgroups own 32 columns and split k over their waves (partial sums added in
- * a fixed order); else a kernel bound by the matrix cores, whose workgroups own
+ * a fixed order); else kernels bound by the matrix cores, whose workgroups own
  * output tiles of 256 x 256, 128 x 128 or 64 x 128 (the largest that still
  * gives every compute unit work; all three add the same terms in the same
  * order); for shapes beyond their index ranges, the kernel of

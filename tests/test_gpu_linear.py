@@ -196,3 +196,26 @@ def test_random_shapes_of_small_integers_are_exact(m, n, k):
     assert np.abs(want).max() <= 256 and np.abs(prod).max() <= 256
     assert np.array_equal(out[1:m + 1].float().cpu().numpy(), want.astype(np.float32))
     assert (out[0] == 777.0).all() and (out[m + 1] == 777.0).all()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("k", [8, 64, 72, 128, 136, 192, 264, 320])
+@pytest.mark.parametrize("m,n", [(3329, 3104), (1100, 4128)], ids=["256", "128"])
+def test_products_of_one_to_five_steps(m, n, k, dt):
+    """The kernel behind the tiles of 256 x 256 and 128 x 128 asks for rows up to two steps of 64 ahead and
+    runs its last three steps apart: every number of steps around that, with a whole and a cut last one, and
+    last tiles of one row and of 32 columns. Small integers are exact in every order."""
+    print(f"linear steps m={m} n={n} k={k} {dt}", flush=True)
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(m + k)
+    x = torch.randint(-1, 2, (m, k), device=DEV, generator=gen)
+    w = torch.randint(-1, 2, (n, k), device=DEV, generator=gen)
+    pad = torch.full((m + 2, k), float("nan"), dtype=dt, device=DEV)
+    pad[1:m + 1] = x.to(dt)
+    wpad = torch.full((n + 2, k), float("nan"), dtype=dt, device=DEV)
+    wpad[1:n + 1] = w.to(dt)
+    out = torch.full((m + 2, n), 777.0, dtype=dt, device=DEV)
+    gemm_rs.local_product((pad[1:m + 1], wpad[1:n + 1], None), out=out[1:m + 1])
+    want = x.double() @ w.double().T
+    assert torch.equal(out[1:m + 1].double(), want)
+    assert (out[0] == 777.0).all() and (out[m + 1] == 777.0).all()
