@@ -24,7 +24,21 @@ _DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    """The address as an int (the argument types say that it is a pointer)."""
+    return None if t is None else t.data_ptr()
+
+
+def _pointers(tensors):
+    return (C.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
+def _ref(shape):
+    """`C.byref(shape)`, made once per shape."""
+    try:
+        return shape.ref
+    except AttributeError:
+        shape.ref = C.byref(shape)
+        return shape.ref
 
 
 def _rows(buf: torch.Tensor, meta: torch.Tensor, hidden_dim: int) -> int:
@@ -35,101 +49,107 @@ class CtypesBinding:
     name = "ctypes"
 
     def __init__(self):
-        _lib.load()
+        lib = _lib.load()
+        self._functions = {name: getattr(lib, name) for name in _lib.SIGNATURES}
+
+    def _call(self, name, *args):
+        status = self._functions[name](*args)
+        if status:
+            _lib.check(status, name)
 
     def version(self) -> str:
         return _lib.load().moe_a2a_version().decode()
 
     def dispatch_send(self, shape, x, indices, num_tokens, send_buf, send_meta, send_counts, send_slot, stream):
-        _lib.call("moe_a2a_dispatch_send", C.byref(shape), _ptr(x), _ptr(indices), num_tokens, _ptr(send_buf),
-                  _ptr(send_meta), _ptr(send_counts), _ptr(send_slot), C.c_void_p(stream))
+        self._call("moe_a2a_dispatch_send", _ref(shape), _ptr(x), _ptr(indices), num_tokens, _ptr(send_buf),
+                  _ptr(send_meta), _ptr(send_counts), _ptr(send_slot), stream)
 
     def plan_send(self, shape, indices, num_tokens, rank_counts, rank_offsets, expert_counts, dst_slot,
                   src_entry, stream):
-        _lib.call("moe_a2a_plan_send", C.byref(shape), _ptr(indices), num_tokens, _ptr(rank_counts),
-                  _ptr(rank_offsets), _ptr(expert_counts), _ptr(dst_slot), _ptr(src_entry), C.c_void_p(stream))
+        self._call("moe_a2a_plan_send", _ref(shape), _ptr(indices), num_tokens, _ptr(rank_counts),
+                  _ptr(rank_offsets), _ptr(expert_counts), _ptr(dst_slot), _ptr(src_entry), stream)
 
     def dispatch_recv(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens, expert_x,
                       expert_meta, send_back_plan, stream, row_position=None):
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
-        args = (C.byref(shape), _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
+        args = (_ref(shape), _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
                 min(rows_hint, capacity), capacity, _ptr(expert_num_tokens), _ptr(expert_x), _ptr(expert_meta),
                 _ptr(send_back_plan))
         if row_position is None:
-            _lib.call("moe_a2a_dispatch_recv", *args, C.c_void_p(stream))
+            self._call("moe_a2a_dispatch_recv", *args, stream)
         else:  # long streams: positions from a planning launch
             if row_position.numel() < capacity:
                 raise ValueError("row_position must hold one int per row of the receive buffers")
-            _lib.call("moe_a2a_dispatch_recv_long", *args, _ptr(row_position), C.c_void_p(stream))
+            self._call("moe_a2a_dispatch_recv_long", *args, _ptr(row_position), stream)
 
     def combine_send(self, shape, expert_y, expert_meta, expert_num_tokens, rows_hint, send_buf, send_meta,
                      send_counts, send_back_plan, stream):
         capacity = _rows(send_buf, send_meta, shape.hidden_dim)
-        _lib.call("moe_a2a_combine_send", C.byref(shape), _ptr(expert_y), _ptr(expert_meta),
+        self._call("moe_a2a_combine_send", _ref(shape), _ptr(expert_y), _ptr(expert_meta),
                   _ptr(expert_num_tokens), min(rows_hint, capacity), capacity, _ptr(send_buf), _ptr(send_meta),
-                  _ptr(send_counts), _ptr(send_back_plan), C.c_void_p(stream))
+                  _ptr(send_counts), _ptr(send_back_plan), stream)
 
     def combine_recv(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, weights, num_tokens, out_tokens,
                      accumulate, stream, entry_row=None):
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
-        args = (C.byref(shape), _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
+        args = (_ref(shape), _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
                 min(rows_hint, capacity), capacity, _ptr(weights), num_tokens, _ptr(out_tokens),
                 int(bool(accumulate)), _DT[out_tokens.dtype])
         if entry_row is None:
-            _lib.call("moe_a2a_combine_recv", *args, C.c_void_p(stream))
+            self._call("moe_a2a_combine_recv", *args, stream)
         else:  # long streams: rows looked up in a (token, k) -> row table
             if entry_row.numel() < num_tokens * shape.experts_per_token:
                 raise ValueError("entry_row must hold num_tokens * experts_per_token ints")
-            _lib.call("moe_a2a_combine_recv_long", *args, _ptr(entry_row), C.c_void_p(stream))
+            self._call("moe_a2a_combine_recv_long", *args, _ptr(entry_row), stream)
 
     def expert_scale(self, shape, expert_x, expert_num_tokens, rows_hint, expert_y, stream):
-        _lib.call("moe_a2a_expert_scale", C.byref(shape), _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
-                  _DT[expert_x.dtype], _DT[expert_y.dtype], _ptr(expert_y), C.c_void_p(stream))
+        self._call("moe_a2a_expert_scale", _ref(shape), _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
+                  _DT[expert_x.dtype], _DT[expert_y.dtype], _ptr(expert_y), stream)
 
     def expert_gemm(self, shape, expert_x, expert_num_tokens, rows_hint, weights, bias, expert_y, stream):
-        _lib.call("moe_a2a_expert_gemm", C.byref(shape), _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
+        self._call("moe_a2a_expert_gemm", _ref(shape), _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
                   _ptr(weights), _ptr(bias), weights.shape[2], weights.shape[1], _DT[expert_x.dtype],
-                  _ptr(expert_y), C.c_void_p(stream))
+                  _ptr(expert_y), stream)
 
     def linear(self, input, weight, bias, output, stream):
         m, k = input.shape
-        _lib.call("moe_a2a_linear", _ptr(input), _ptr(weight), _ptr(bias), m, weight.shape[0], k, _DT[input.dtype],
-                  _ptr(output), C.c_void_p(stream))
+        self._call("moe_a2a_linear", _ptr(input), _ptr(weight), _ptr(bias), m, weight.shape[0], k, _DT[input.dtype],
+                  _ptr(output), stream)
 
     def exchange_local(self, world_size, hidden_dim, send_buf, send_meta, send_counts, dst_rank, recv_buf,
                        recv_meta, recv_counts, src_rank, rows_hint, stream):
-        _lib.call("moe_a2a_exchange_local", world_size, hidden_dim, _ptr(send_buf), _ptr(send_meta),
+        self._call("moe_a2a_exchange_local", world_size, hidden_dim, _ptr(send_buf), _ptr(send_meta),
                   _ptr(send_counts), dst_rank, _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts), src_rank,
                   rows_hint, _rows(send_buf, send_meta, hidden_dim), _rows(recv_buf, recv_meta, hidden_dim),
-                  C.c_void_p(stream))
+                  stream)
 
     # ---- the compact expert-major layout (rows of the experts back to back)
 
     def dispatch_recv_compact(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens,
                               expert_offsets, expert_x, expert_meta, send_back_plan, stream):
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
-        _lib.call("moe_a2a_dispatch_recv_compact", C.byref(shape), _ptr(recv_buf), _ptr(recv_meta),
+        self._call("moe_a2a_dispatch_recv_compact", _ref(shape), _ptr(recv_buf), _ptr(recv_meta),
                   _ptr(recv_counts), min(rows_hint, capacity), capacity, _ptr(expert_num_tokens),
                   _ptr(expert_offsets), _ptr(expert_x), _ptr(expert_meta),
-                  _rows(expert_x, expert_meta, shape.hidden_dim), _ptr(send_back_plan), C.c_void_p(stream))
+                  _rows(expert_x, expert_meta, shape.hidden_dim), _ptr(send_back_plan), stream)
 
     def expert_scale_compact(self, shape, expert_x, expert_num_tokens, rows_hint, expert_y, stream):
-        _lib.call("moe_a2a_expert_scale_compact", C.byref(shape), _ptr(expert_x), _ptr(expert_num_tokens),
+        self._call("moe_a2a_expert_scale_compact", _ref(shape), _ptr(expert_x), _ptr(expert_num_tokens),
                   rows_hint, min(expert_x.shape[0], expert_y.shape[0]), _DT[expert_x.dtype], _DT[expert_y.dtype],
-                  _ptr(expert_y), C.c_void_p(stream))
+                  _ptr(expert_y), stream)
 
     def expert_gemm_compact(self, shape, expert_x, expert_num_tokens, rows_hint, weights, bias, expert_y, stream):
-        _lib.call("moe_a2a_expert_gemm_compact", C.byref(shape), _ptr(expert_x), _ptr(expert_num_tokens),
+        self._call("moe_a2a_expert_gemm_compact", _ref(shape), _ptr(expert_x), _ptr(expert_num_tokens),
                   rows_hint, min(expert_x.shape[0], expert_y.shape[0]), _ptr(weights), _ptr(bias),
-                  weights.shape[2], weights.shape[1], _DT[expert_x.dtype], _ptr(expert_y), C.c_void_p(stream))
+                  weights.shape[2], weights.shape[1], _DT[expert_x.dtype], _ptr(expert_y), stream)
 
     def combine_send_compact(self, shape, expert_y, expert_meta, expert_num_tokens, rows_hint, send_buf,
                              send_meta, send_counts, send_back_plan, stream):
         capacity = _rows(send_buf, send_meta, shape.hidden_dim)
-        _lib.call("moe_a2a_combine_send_compact", C.byref(shape), _ptr(expert_y), _ptr(expert_meta),
+        self._call("moe_a2a_combine_send_compact", _ref(shape), _ptr(expert_y), _ptr(expert_meta),
                   _ptr(expert_num_tokens), min(rows_hint, capacity),
                   _rows(expert_y, expert_meta, shape.hidden_dim), capacity, _ptr(send_buf), _ptr(send_meta),
-                  _ptr(send_counts), _ptr(send_back_plan), C.c_void_p(stream))
+                  _ptr(send_counts), _ptr(send_back_plan), stream)
 
     def gather_sources(self, hidden_dim, send_bufs, send_metas, send_counts):
         """The per-source pointer tables of `exchange_gather`, built once for buffers that stay where
@@ -140,12 +160,27 @@ class CtypesBinding:
                 min(_rows(b, m, hidden_dim) for b, m in zip(send_bufs, send_metas)),
                 (list(send_bufs), list(send_metas), list(send_counts)))
 
+    def local_dispatch(self, shape, xs, indices, compact, entry_row, expert_num_tokens, expert_offsets, rows, meta,
+                       standin, stream):
+        tokens = (C.c_int32 * len(xs))(*[i.shape[0] for i in indices])
+        din, dout = (_DT[xs[0].dtype], _DT[rows.dtype]) if standin else (-1, -1)
+        self._call("moe_a2a_local_dispatch", _ref(shape), _pointers(xs), _pointers(indices), tokens,
+                   rows.shape[0] if compact else 0, din, dout, _ptr(entry_row), _ptr(expert_num_tokens),
+                   _ptr(expert_offsets), rows.data_ptr(), _ptr(meta), stream)
+
+    def local_combine(self, shape, rows, entry_row, weights, tokens, outs, only_rank, accumulate, stream):
+        """`weights` and `outs` may hold None for ranks other than `only_rank`; `tokens` are all ranks'."""
+        ranks = len(tokens)
+        self._call("moe_a2a_local_combine", _ref(shape), rows.data_ptr(), entry_row.data_ptr(),
+                   (C.c_void_p * ranks)(*map(_ptr, weights)), (C.c_int32 * ranks)(*tokens),
+                   (C.c_void_p * ranks)(*map(_ptr, outs)), only_rank, int(bool(accumulate)), _DT[rows.dtype], stream)
+
     def exchange_gather(self, world_size, hidden_dim, sources, dst_rank, recv_buf, recv_meta, recv_counts,
                         rows_hint, stream):
         (bufs, metas, counts), send_capacity, _ = sources
-        _lib.call("moe_a2a_exchange_gather_local", world_size, hidden_dim, bufs, metas, counts, dst_rank,
+        self._call("moe_a2a_exchange_gather_local", world_size, hidden_dim, bufs, metas, counts, dst_rank,
                   _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts), rows_hint, send_capacity,
-                  _rows(recv_buf, recv_meta, hidden_dim), C.c_void_p(stream))
+                  _rows(recv_buf, recv_meta, hidden_dim), stream)
 
 
 class ExtBinding:
@@ -158,7 +193,11 @@ class ExtBinding:
 
     @staticmethod
     def _shape(shape) -> list:
-        return [getattr(shape, f) for f, _ in _lib.Shape._fields_]
+        try:
+            return shape.fields
+        except AttributeError:
+            shape.fields = [getattr(shape, f) for f, _ in _lib.Shape._fields_]
+            return shape.fields
 
     def version(self) -> str:
         return self._m.a2a_version()
@@ -220,6 +259,16 @@ class ExtBinding:
                              send_meta, send_counts, send_back_plan, stream):
         self._m.a2a_combine_send_compact(self._shape(shape), expert_y, expert_meta, expert_num_tokens, rows_hint,
                                          send_buf, send_meta, send_counts, send_back_plan, stream)
+
+    def local_dispatch(self, shape, xs, indices, compact, entry_row, expert_num_tokens, expert_offsets, rows, meta,
+                       standin, stream):
+        self._m.a2a_local_dispatch(self._shape(shape), xs, indices, compact, entry_row, expert_num_tokens,
+                                   expert_offsets, rows, meta, standin, stream)
+
+    def local_combine(self, shape, rows, entry_row, weights, tokens, outs, only_rank, accumulate, stream):
+        if only_rank >= 0:
+            raise ValueError("one rank's result of several goes through the ctypes binding")
+        self._m.a2a_local_combine(self._shape(shape), rows, entry_row, weights, outs, bool(accumulate), stream)
 
     def gather_sources(self, hidden_dim, send_bufs, send_metas, send_counts):
         return (list(send_bufs), list(send_metas), list(send_counts))

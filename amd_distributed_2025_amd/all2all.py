@@ -13,7 +13,8 @@ recv_meta, rows_hint)`. `LocalExchange` is the one-GPU stand-in for the
 reference's `all_to_all_single` calls: the ranks of a job run as threads of one
 process, meet in `deliver` as processes meet in a collective, and the segments
 move by device copies. `run_lockstep` starts such a job. `LocalWorld` steps all
-ranks of a job from one thread, half by half, with the same copies.
+ranks of a job from one thread, half by half, with the same copies. A job of one
+rank has nothing to exchange: its `dispatch` and `combine` are one pass each.
 
 All device work goes through the C ABI in `libmoe_a2a.so`, bound either with
 ctypes or through the torch extension (`binding="ext"`); torch only owns
@@ -41,6 +42,9 @@ META_DIM = 5
 LONG_STREAM_ROWS = {"dispatch": 8192, "combine": 4096}
 
 
+# what moe_a2a_local_dispatch takes
+LOCAL_MAX_RANKS, LOCAL_MAX_EXPERTS, LOCAL_MAX_K = 64, 1024, 64
+
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
@@ -54,6 +58,9 @@ def _stream(device) -> int:
 
 
 def _need(t: torch.Tensor, dtype: torch.dtype, device, what: str) -> torch.Tensor:
+    # (one test for the usual case: what a call costs on the host is what a small job costs)
+    if t.dtype is dtype and t.get_device() == device.index and t.is_contiguous():
+        return t
     if t.dtype != dtype:
         raise TypeError(f"{what}: expected {dtype}, got {t.dtype}")
     if t.device != device:
@@ -102,20 +109,28 @@ class HIPAllToAll:
             self.max_rows_in = min(self.max_rows_in, self.compact_rows)
         self.expert_offsets = None  # compact layout: int32[nle + 1], written by dispatch_recv
         self._ws = {}
+        self._kept = {}       # what _buf made them for: name -> (shape, dtype)
+        self._send_views = {} # token count -> what dispatch_send returns for it
         # dispatch_recv leaves a plan of where combine_send will put every row; combine_send uses
         # it when it is handed the very tensors that dispatch_recv returned
         self.reuse_placement = reuse_placement
         self._planned_for = None
         self.long_stream_rows = None  # an int overrides both thresholds of LONG_STREAM_ROWS
+        # A job of one rank exchanges with itself, so dispatch() and combine() can move rows straight to
+        # their experts and back (moe_a2a_local_dispatch / _combine). Not where a token could have more
+        # entries than there are experts (its copies could overflow the receive buffers of the halves, which
+        # this path does not have), nor beyond the limits of those entry points.
+        self._direct = (world_size == 1 and reuse_placement and cfg.experts_per_token <= min(cfg.num_experts, LOCAL_MAX_K)
+                        and cfg.num_experts <= LOCAL_MAX_EXPERTS)
+        self._dispatched_for = None  # (expert_meta, expert_num_tokens, tokens) of such a dispatch
 
     # ------------------------------------------------------------------ workspace
 
-    def _buf(self, name: str, shape: Sequence[int], dtype: torch.dtype) -> torch.Tensor:
-        t = self._ws.get(name)
-        if t is None or tuple(t.shape) != tuple(shape) or t.dtype != dtype:
-            t = torch.empty(tuple(shape), dtype=dtype, device=self.device)
-            self._ws[name] = t
-        return t
+    def _buf(self, name: str, shape: Tuple[int, ...], dtype: torch.dtype) -> torch.Tensor:
+        if self._kept.get(name) != (shape, dtype):
+            self._ws[name] = torch.empty(shape, dtype=dtype, device=self.device)
+            self._kept[name] = (shape, dtype)
+        return self._ws[name]
 
     def workspace_bytes(self) -> int:
         """Device memory of the buffers this object has made so far."""
@@ -158,8 +173,14 @@ class HIPAllToAll:
         meta = self._buf("send_meta", (self.max_rows_out, META_DIM), torch.int32)
         slots = self._buf("send_slot", (self.max_rows_out,), torch.int32) if want_slots else None
         self.binding.dispatch_send(self.shape, dp_x, indices, T, buf, meta, counts, slots, _stream(self.device))
-        out = (counts, buf[:S], meta[:S])
-        return out + (slots[:S],) if want_slots else out
+        if want_slots:
+            return counts, buf[:S], meta[:S], slots[:S]
+        out = self._send_views.get(T)
+        if out is None:
+            if len(self._send_views) >= 64:
+                self._send_views.clear()
+            out = self._send_views[T] = (counts, buf[:S], meta[:S])
+        return out
 
     def plan_send(self, indices: torch.Tensor):
         """Counts, offsets and index maps of the send order, without moving rows.
@@ -206,6 +227,7 @@ class HIPAllToAll:
             self.binding.dispatch_recv(self.shape, recv_buf, recv_meta, recv_counts, hint, num, ex, em, plan,
                                        _stream(self.device), pos)
         self._planned_for = None if plan is None else (em.data_ptr(), num.data_ptr())
+        self._dispatched_for = None
         self._rows_in_hint = hint
         return num, ex, em
 
@@ -342,18 +364,75 @@ class HIPAllToAll:
         if self.exchange is None:
             raise RuntimeError("dispatch() of a job with several ranks needs the exchange its ranks share "
                                "(LocalExchange on one GPU); or use the halves, or LocalWorld")
+        if self._direct and type(self.exchange) is LocalExchange and self.exchange.world_size == 1:
+            S = indices.shape[0] * self.cfg.experts_per_token
+            if self.layout == "padded" or S <= self.compact_rows:
+                return self._direct_dispatch(dp_x, indices, S)
         counts, buf, meta = self.dispatch_send(dp_x, indices)
         rc, rb, rm, hint = self.exchange.deliver(self, "dispatch", counts, buf, meta)
         return self.dispatch_recv(rc, rb, rm, hint)
+
+    def _direct_dispatch(self, dp_x, indices, S: int):
+        """A job of one rank: what the halves and the exchange between them give, in one pass over the rows."""
+        cfg = self.cfg
+        T, K = indices.shape
+        if K != cfg.experts_per_token or dp_x.shape != (T, cfg.hidden_dim):
+            raise ValueError("dispatch: shapes of dp_x / indices do not match the config")
+        _need(dp_x, cfg.in_dtype, self.device, "dp_x")
+        _need(indices, torch.int32, self.device, "indices")
+        E, compact = cfg.num_experts, self.layout == "compact"
+        num = self._buf("expert_num_tokens", (E,), torch.int32)
+        rows = (self.compact_rows,) if compact else (E, self.max_recv)
+        ex = self._buf("expert_x", rows + (cfg.hidden_dim,), cfg.in_dtype)
+        em = self._buf("expert_meta", rows + (META_DIM,), torch.int32)
+        if compact:
+            self.expert_offsets = self._buf("expert_offsets", (E + 1,), torch.int32)
+        where = self._buf("row_of_entry", (self.max_rows_out,), torch.int32)
+        self.binding.local_dispatch(self.shape, (dp_x,), (indices,), compact, where, num,
+                                    self.expert_offsets if compact else None, ex, em, False, _stream(self.device))
+        self._planned_for = None
+        self._dispatched_for = (em.data_ptr(), num.data_ptr(), T)
+        self._rows_in_hint = S
+        return num, ex, em
 
     def combine(self, out_tokens, weights, expert_meta, expert_y, expert_num_tokens):
         """all2all/reference.py:151-234 with the exchange delegated to `self.exchange`."""
         if self.exchange is None:
             raise RuntimeError("combine() of a job with several ranks needs the exchange its ranks share "
                                "(LocalExchange on one GPU); or use the halves, or LocalWorld")
+        if self._dispatched_for is not None and self._direct_combine(out_tokens, weights, expert_meta, expert_y,
+                                                                     expert_num_tokens):
+            return out_tokens
         counts, buf, meta = self.combine_send(expert_meta, expert_y, expert_num_tokens)
         rc, rb, rm, _ = self.exchange.deliver(self, "combine", counts, buf, meta)
         return self.combine_recv(out_tokens, weights, rc, rb, rm, accumulate=True)
+
+    def _direct_combine(self, out_tokens, weights, expert_meta, expert_y, expert_num_tokens) -> bool:
+        """The way back of `_direct_dispatch`; False where the tensors are not the ones it returned (the
+        halves then read the rows' places from `expert_meta`)."""
+        cfg = self.cfg
+        T = weights.shape[0]
+        if (self._dispatched_for != (expert_meta.data_ptr(), expert_num_tokens.data_ptr(), T)
+                or type(self.exchange) is not LocalExchange):
+            return False
+        shape, K = expert_y.shape, cfg.experts_per_token
+        if len(shape) == 2 if self.layout == "padded" else len(shape) != 2:
+            return False
+        if len(shape) == 2:
+            if shape[0] < T * K or shape[1] != cfg.hidden_dim:
+                return False
+        elif shape != (self.num_local_experts, self.max_recv, cfg.hidden_dim):
+            return False
+        if weights.shape[1] != K:
+            return False
+        _need(expert_y, cfg.out_dtype, self.device, "expert_y")
+        _need(out_tokens, cfg.out_dtype, self.device, "out_tokens")
+        _need(weights, torch.float32, self.device, "weights")
+        if out_tokens.shape[0] < T or out_tokens.shape[1] != cfg.hidden_dim:
+            raise ValueError("combine: out_tokens must hold num_tokens rows of hidden_dim")
+        self.binding.local_combine(self.shape, expert_y, self._ws["row_of_entry"], (weights,), (T,), (out_tokens,), -1,
+                                   True, _stream(self.device))
+        return True
 
 
 def exchange_leg(src: HIPAllToAll, dst: HIPAllToAll, send_counts, send_buf, send_meta,

@@ -1751,6 +1751,22 @@ __global__ __launch_bounds__(BLK) void combine_recv_kernel(
 
 // ---------------------------------------------------------------- simulated expert
 
+// .to(out_dtype), then times `scale` = (1 + rank) in float32, rounded once (all2all/reference.py:262)
+template <typename V, int DIN, int DOUT>
+__device__ __forceinline__ V standin_expert(V v, float scale) {
+  constexpr int N = Words<V>::N;
+  uint32_t h[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    const uint32_t w = get_word(v, e);
+    const uint32_t o = Pair16<DOUT>::round(Pair16<DIN>::lo(w), Pair16<DIN>::hi(w));
+    const float lo = rounded_here(__fmul_rn(Pair16<DOUT>::lo(o), scale));
+    const float hi = rounded_here(__fmul_rn(Pair16<DOUT>::hi(o), scale));
+    h[e] = Pair16<DOUT>::canonical(Pair16<DOUT>::round(lo, hi));
+  }
+  return from_words<V>(h);
+}
+
 template <typename V, int NV, int DIN, int DOUT>
 __global__ __launch_bounds__(BLOCK) void expert_scale_kernel(
     const V* __restrict__ expert_x, const int* __restrict__ expert_num_tokens, int nle,
@@ -1769,20 +1785,7 @@ __global__ __launch_bounds__(BLOCK) void expert_scale_kernel(
     const size_t row = compact_rows > 0 ? (size_t)g : (size_t)le * max_recv + (g - pre[le]);
     Payload<V, NV> p;
     p.load(expert_x + row * row_vecs, base, row_vecs);
-    p.map([scale](V v) {
-      constexpr int N = Words<V>::N;
-      uint32_t h[N];
-#pragma unroll
-      for (int e = 0; e < N; ++e) {
-        const uint32_t w = get_word(v, e);
-        // .to(out_dtype), then times (1 + rank) in float32, rounded once
-        const uint32_t o = Pair16<DOUT>::round(Pair16<DIN>::lo(w), Pair16<DIN>::hi(w));
-        const float lo = rounded_here(__fmul_rn(Pair16<DOUT>::lo(o), scale));
-        const float hi = rounded_here(__fmul_rn(Pair16<DOUT>::hi(o), scale));
-        h[e] = Pair16<DOUT>::canonical(Pair16<DOUT>::round(lo, hi));
-      }
-      return from_words<V>(h);
-    });
+    p.map([scale](V v) { return standin_expert<V, DIN, DOUT>(v, scale); });
     p.store(expert_y + row * row_vecs, base, row_vecs);
   }
 }
@@ -1807,19 +1810,7 @@ __global__ __launch_bounds__(64 * ROWS) void expert_scale_wave_kernel(
     WavePayload<b128, NVW> p;
     p.load(expert_x + row * row_vecs, base, row_vecs, lane);
 #pragma unroll
-    for (int j = 0; j < NVW; ++j) {
-      uint32_t h[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t w = p.v[j][e];
-        // .to(out_dtype), then times (1 + rank) in float32, rounded once
-        const uint32_t o = Pair16<DOUT>::round(Pair16<DIN>::lo(w), Pair16<DIN>::hi(w));
-        const float lo = rounded_here(__fmul_rn(Pair16<DOUT>::lo(o), scale));
-        const float hi = rounded_here(__fmul_rn(Pair16<DOUT>::hi(o), scale));
-        h[e] = Pair16<DOUT>::canonical(Pair16<DOUT>::round(lo, hi));
-      }
-      p.v[j] = from_words<b128>(h);
-    }
+    for (int j = 0; j < NVW; ++j) p.v[j] = standin_expert<b128, DIN, DOUT>(p.v[j], scale);
     p.template store<(MOE_A2A_NT_STANDIN != 0)>(expert_y + row * row_vecs, base, row_vecs, lane);
   }
 }
@@ -2956,6 +2947,375 @@ __global__ __launch_bounds__(BLOCK) void exchange_gather_kernel(
   }
 }
 
+// ---------------------------------------------------------------- jobs whose ranks share the GPU
+//
+// Where every rank of a job lives on this GPU there is nothing to exchange: a token's row can go straight
+// to its experts' rows and come straight back. Three kernels replace the five stages and two exchanges:
+//   local_plan_kernel      the expert-buffer row of every (rank, token, k) entry (entry_row), in the order in
+//                          which the stages would have put it there: by source rank, token and k inside an
+//                          expert. Left out for one rank with up to LOCAL_RANK_ENTRIES entries, whose mover
+//                          ranks them itself (a launch costs more than that scan).
+//   local_dispatch_kernel  one workgroup per (token, chunk of its row) reads the chunk once and stores it to
+//                          all of the token's expert rows, as it is or through the stand-in expert.
+//   local_combine_kernel   one workgroup per (token, chunk): gathers the token's expert rows and adds them up
+//                          in arrival order. Rows come back by destination rank, expert and position, so
+//                          arrival order is the order of the expert-buffer rows themselves, in both layouts.
+// Bound by memory: a row is written once to its expert and read once from there, where the stages and
+// copies moved it six times.
+
+constexpr int LOCAL_MAX_RANKS = 64;
+constexpr int LOCAL_MAX_EXPERTS = 1024;     // counters of the plan in LDS
+constexpr int LOCAL_MAX_K = 64;             // entries of a token, one per lane
+constexpr int LOCAL_RANK_BITS = 11;
+constexpr int LOCAL_RANK_ENTRIES = 1 << LOCAL_RANK_BITS;  // eight keys per lane of the mover's workgroup
+
+struct LocalSources {
+  const void* x[LOCAL_MAX_RANKS];
+  const int* indices[LOCAL_MAX_RANKS];
+  int first[LOCAL_MAX_RANKS + 1];  // number of the rank's first token, counted over all ranks
+};
+struct LocalResults {
+  const float* weights[LOCAL_MAX_RANKS];
+  void* out[LOCAL_MAX_RANKS];
+  int first[LOCAL_MAX_RANKS + 1];
+};
+
+// the rank that token number t (the same for every lane of the wave) belongs to
+template <typename Table>
+__device__ __forceinline__ int rank_of_token(const Table& tab, int W, int t) {
+  if (W == 1) return 0;
+  const int lane = threadIdx.x & 63;
+  return __popcll(__ballot(lane < W && tab.first[lane] <= t)) - 1;
+}
+
+constexpr int LPLAN_BLOCK = 1024, LPLAN_WAVES = LPLAN_BLOCK / 64;
+
+// One workgroup per 1024 entries. Entries before the tile go through an LDS histogram per expert; inside the
+// tile an entry's place among the lanes of its wave with the same expert comes from one ballot per bit of
+// the expert number, the waves are ordered by a prefix over their counts (as in plan_recv_kernel).
+//   compact        row = rows of lower experts + position, else expert * max_recv + position
+//   expert_limit   entries at or past that position in their expert are dropped (row -1), as the padded
+//                  buffers of all2all/reference.py:123-136 have no room for them
+//   rank_limit     > 0: entries past that many of their destination rank are dropped (what its receive
+//                  buffer holds). Reached only by tokens that name an expert more than once.
+// Entries with an expert outside [0, E) have no row. The last workgroup writes the rows per expert.
+__global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
+    LocalSources src, int W, int S, int K, int E, int nle, int expert_bits, int rank_bits, bool compact, int max_recv,
+    int expert_limit, int rank_limit, int* __restrict__ entry_row, int* __restrict__ expert_num_tokens,
+    int* __restrict__ expert_offsets) {
+  extern __shared__ int plan_lds[];            // before[E], total[E], in_wave[LPLAN_WAVES][E]
+  int* const before = plan_lds;
+  int* const total = plan_lds + E;
+  int* const in_wave = plan_lds + 2 * E;
+  __shared__ int first_entry[LOCAL_MAX_RANKS + 1];
+  __shared__ const int* keys_of[LOCAL_MAX_RANKS];
+  __shared__ int rank_in_wave_of[LPLAN_WAVES][LOCAL_MAX_RANKS];
+  __shared__ int rank_before[LOCAL_MAX_RANKS];
+  __shared__ int red[LPLAN_WAVES];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const unsigned long long lanes_below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  const int begin = blockIdx.x * LPLAN_BLOCK;
+  const bool last = blockIdx.x == gridDim.x - 1;
+  if (tid <= W) first_entry[tid] = src.first[tid] * K;
+  if (tid < W) keys_of[tid] = src.indices[tid];
+  for (int j = tid; j < (2 + LPLAN_WAVES) * E; j += LPLAN_BLOCK) plan_lds[j] = 0;
+  for (int j = tid; j < LPLAN_WAVES * LOCAL_MAX_RANKS; j += LPLAN_BLOCK) (&rank_in_wave_of[0][0])[j] = 0;
+  __syncthreads();
+  auto key_at = [&](int i) {  // expert id of entry i < S
+    int r = 0;
+    for (int step = rank_bits ? 1 << (rank_bits - 1) : 0; step > 0; step >>= 1)
+      if (r + step < W && first_entry[r + step] <= i) r += step;
+    return keys_of[r][i - first_entry[r]];
+  };
+  const int i = begin + tid;
+  const int e = i < S ? key_at(i) : -1;
+  const int scanned = compact ? S : begin;
+  for (int b = 0; b < scanned; b += SCAN_UNROLL * LPLAN_BLOCK) {
+    int e2[SCAN_UNROLL];
+#pragma unroll
+    for (int u = 0; u < SCAN_UNROLL; ++u) e2[u] = key_at(min(b + tid + u * LPLAN_BLOCK, scanned - 1));
+#pragma unroll
+    for (int u = 0; u < SCAN_UNROLL; ++u) {
+      const int i2 = b + tid + u * LPLAN_BLOCK;
+      if (i2 < scanned && (uint32_t)e2[u] < (uint32_t)E) {
+        if (compact) atomicAdd(&total[e2[u]], 1);
+        if (i2 < begin) atomicAdd(&before[e2[u]], 1);
+      }
+    }
+  }
+  const bool ok = (uint32_t)e < (uint32_t)E;
+  unsigned long long same = __ballot(ok);
+  for (int b = 0; b < expert_bits; ++b) {
+    const bool set = (e >> b) & 1;
+    const unsigned long long with_bit = __ballot(set);
+    same &= set ? with_bit : ~with_bit;
+  }
+  const int in_wave_before = __popcll(same & lanes_below);
+  if (ok && in_wave_before == 0) in_wave[wave * E + e] = __popcll(same);
+  const int dst = ok ? e / nle : 0;
+  int rank_lane_before = 0;
+  if (rank_limit > 0) {
+    unsigned long long peers = __ballot(ok);
+    for (int b = 0; b < rank_bits; ++b) {
+      const bool set = (dst >> b) & 1;
+      const unsigned long long with_bit = __ballot(set);
+      peers &= set ? with_bit : ~with_bit;
+    }
+    rank_lane_before = __popcll(peers & lanes_below);
+    if (ok && rank_lane_before == 0) rank_in_wave_of[wave][dst] = __popcll(peers);
+  }
+  __syncthreads();
+  int pos = 0;
+  if (ok) {
+    pos = before[e] + in_wave_before;
+    for (int w = 0; w < wave; ++w) pos += in_wave[w * E + e];
+  }
+  bool keep = ok && pos < expert_limit;
+  if (rank_limit > 0) {
+    if (tid < W) {
+      int n = 0;
+      for (int j = 0; j < nle; ++j) n += before[tid * nle + j];
+      rank_before[tid] = n;
+    }
+    __syncthreads();
+    if (ok) {
+      int n = rank_before[dst] + rank_lane_before;
+      for (int w = 0; w < wave; ++w) n += rank_in_wave_of[w][dst];
+      keep = keep && n < rank_limit;
+    }
+  }
+  if (compact) {  // exclusive prefix of the rows per expert (E <= 1024: one expert per lane)
+    const int mine = tid < E ? total[tid] : 0;
+    const int incl = wave_inclusive_scan(mine);
+    if (lane == 63) red[wave] = incl;
+    __syncthreads();
+    int off = incl - mine;
+    for (int w = 0; w < wave; ++w) off += red[w];
+    if (tid < E) total[tid] = off;
+    if (last && tid < E && expert_offsets) {
+      expert_offsets[tid] = off;
+      if (tid == E - 1) expert_offsets[E] = off + mine;
+    }
+    if (last && tid < E && expert_num_tokens) expert_num_tokens[tid] = mine;
+    __syncthreads();
+  } else if (last && expert_num_tokens) {
+    for (int j = tid; j < E; j += LPLAN_BLOCK) {
+      int n = before[j];
+      for (int w = 0; w < LPLAN_WAVES; ++w) n += in_wave[w * E + j];
+      expert_num_tokens[j] = n;
+    }
+  }
+  if (i < S) entry_row[i] = !keep ? -1 : compact ? total[e] + pos : e * max_recv + pos;
+}
+
+// DIN / DOUT >= 0: rows leave as `row.to(out) * (1 + rank of the expert)` (all2all/reference.py:262).
+// RANKED: entry_row is worked out here (one rank, S <= LOCAL_RANK_ENTRIES) and workgroup 0 counts the
+// rows per expert; else it is read.
+template <typename V, int NV, int DIN, int DOUT, bool RANKED>
+__global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
+    LocalSources src, int W, int T, int K, int E, int nle, uint32_t magic, int row_vecs, int chunks, bool compact,
+    int max_recv, int expert_limit, int* __restrict__ entry_row, int* __restrict__ expert_num_tokens,
+    int* __restrict__ expert_offsets, V* __restrict__ rows, int* __restrict__ meta) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  int q = blockIdx.x;
+  if constexpr (RANKED) {
+    if (q == 0) {
+      __shared__ int hist[LOCAL_MAX_EXPERTS];
+      __shared__ int red[NWAVES];
+      constexpr int EACH = LOCAL_MAX_EXPERTS / BLOCK;
+      const int S = T * K;
+      int key[SCAN_UNROLL];
+#pragma unroll
+      for (int u = 0; u < SCAN_UNROLL; ++u) key[u] = src.indices[0][min(tid + u * BLOCK, S - 1)];
+      for (int j = tid; j < E; j += BLOCK) hist[j] = 0;
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < SCAN_UNROLL; ++u)
+        if (tid + u * BLOCK < S && (uint32_t)key[u] < (uint32_t)E) atomicAdd(&hist[key[u]], 1);
+      __syncthreads();
+      int own[EACH], sum = 0;
+#pragma unroll
+      for (int j = 0; j < EACH; ++j) {
+        own[j] = tid * EACH + j < E ? hist[tid * EACH + j] : 0;
+        sum += own[j];
+      }
+      const int incl = wave_inclusive_scan(sum);
+      if (lane == 63) red[wave] = incl;
+      __syncthreads();
+      int off = incl - sum;
+      for (int w = 0; w < wave; ++w) off += red[w];
+#pragma unroll
+      for (int j = 0; j < EACH; ++j) {
+        const int e = tid * EACH + j;
+        if (e < E) {
+          if (expert_num_tokens) expert_num_tokens[e] = own[j];
+          if (expert_offsets) {
+            expert_offsets[e] = off;
+            if (e == E - 1) expert_offsets[E] = off + own[j];
+          }
+        }
+        off += own[j];
+      }
+      return;
+    }
+    --q;
+  }
+  const int t = chunks == 1 ? q : q / chunks, c = q - t * chunks;
+  const int r = rank_of_token(src, W, t), local_t = t - src.first[r];
+  const int* __restrict__ indices = src.indices[r] + (size_t)local_t * K;
+  const int base = c * (BLOCK * NV);
+  const int own = indices[min(lane, K - 1)];
+  int row_of = -1;
+  int key[SCAN_UNROLL];
+  if constexpr (RANKED) {
+#pragma unroll
+    for (int u = 0; u < SCAN_UNROLL; ++u) key[u] = src.indices[0][min(tid + u * BLOCK, T * K - 1)];
+  } else {
+    row_of = entry_row[(size_t)t * K + min(lane, K - 1)];
+  }
+  Payload<V, NV> p;
+  p.load((const V*)src.x[r] + (size_t)local_t * row_vecs, base, row_vecs);
+
+  if constexpr (RANKED) {
+    // a key's place in (expert, entry) order; ids outside [0, E) come last
+    constexpr int FAN = 8, PAIRS = FAN / 2;
+    __shared__ int part[2][NWAVES][PAIRS];
+    const int S = T * K;
+    auto composite = [&](int e, int i) { return ((uint32_t)e < (uint32_t)E ? e : E) << LOCAL_RANK_BITS | i; };
+#pragma unroll
+    for (int u = 0; u < SCAN_UNROLL; ++u) {
+      const int i2 = tid + u * BLOCK;
+      key[u] = i2 < S ? composite(key[u], i2) : INT_MAX;
+    }
+    for (int g0 = 0, parity = 0; g0 < K; g0 += FAN, parity ^= 1) {
+      int cnt[FAN];
+#pragma unroll
+      for (int g = 0; g < FAN; ++g) {
+        const int k = min(g0 + g, K - 1);
+        const int mine = composite(__builtin_amdgcn_readlane(own, k), t * K + k);
+        // compact: everything ahead of it; padded: what is ahead of it in its own expert
+        const int from = compact ? 0 : mine & ~(LOCAL_RANK_ENTRIES - 1);
+        cnt[g] = 0;
+#pragma unroll
+        for (int u = 0; u < SCAN_UNROLL; ++u) cnt[g] += (int)((uint32_t)(key[u] - from) < (uint32_t)(mine - from));
+      }
+#pragma unroll
+      for (int h = 0; h < PAIRS; ++h) {
+        const int sum = wave_sum(cnt[h] | (cnt[h + PAIRS] << 16));
+        if (lane == 0) part[parity][wave][h] = sum;
+      }
+      lds_barrier();  // (each half of `part` is next written behind the barrier after this one)
+      if (lane >= g0 && lane < min(g0 + FAN, K)) {
+        const int g = lane - g0, h = g & (PAIRS - 1);
+        int both = 0;
+#pragma unroll
+        for (int w = 0; w < NWAVES; ++w) both += part[parity][w][h];
+        const int n = g < PAIRS ? both & 0xffff : (int)((unsigned)both >> 16);
+        const bool keep = (uint32_t)own < (uint32_t)E && (compact || n < expert_limit);
+        row_of = !keep ? -1 : compact ? n : own * max_recv + n;
+      }
+    }
+    if (c == 0 && wave == 0 && lane < K) entry_row[(size_t)t * K + lane] = row_of;
+  }
+
+  for (int k = 0; k < K; ++k) {
+    const int row = __builtin_amdgcn_readlane(row_of, k);
+    if (row < 0) continue;
+    V* __restrict__ to = rows + (size_t)row * row_vecs;
+    if constexpr (DIN >= 0) {
+      const int e = __builtin_amdgcn_readlane(own, k);
+      const float scale = (float)(1 + (nle == 1 ? e : (int)__umulhi((uint32_t)e, magic)));
+      Payload<V, NV> y = p;
+      y.map([scale](V v) { return standin_expert<V, DIN, DOUT>(v, scale); });
+      y.store(to, base, row_vecs);
+    } else {
+      p.store(to, base, row_vecs);
+    }
+  }
+  if (c == 0 && meta) {
+    for (int m0 = 0; m0 < K * META; m0 += BLOCK) {  // (the same trips for every lane: they shuffle)
+      const int m = m0 + tid, k = min(m / META, K - 1), f = m - k * META;
+      const int row = __shfl(row_of, k, 64), e = __shfl(own, k, 64);
+      if (m < K * META && row >= 0) meta[(size_t)row * META + f] = f == 0 ? e : f == 1 ? r : f == 2 ? local_t : f == 3 ? k : 0;
+    }
+  }
+}
+
+// MANY: more than eight entries per token.
+template <typename V, int DT, int NV, bool MANY>
+__global__ __launch_bounds__(BLOCK) void local_combine_kernel(
+    LocalResults dst, int W, int first_token, int K, int row_vecs, int chunks, const V* __restrict__ rows,
+    const int* __restrict__ entry_row, int accumulate) {
+  constexpr int N = Words<V>::N, BATCH = 8;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int q = blockIdx.x;
+  const int item = chunks == 1 ? q : q / chunks, c = q - item * chunks;
+  const int t = first_token + item;
+  const int r = rank_of_token(dst, W, t), local_t = t - dst.first[r];
+  const int base = c * (BLOCK * NV);
+  V* __restrict__ orow = (V*)dst.out[r] + (size_t)local_t * row_vecs;
+  // entry of this lane; lanes repeat the entries in runs of 8 unless there are more
+  const int k = MANY ? lane : lane & (BATCH - 1);
+  const bool there = k < K;
+  const int loaded = entry_row[(size_t)t * K + min(k, K - 1)];
+  const float w_loaded = dst.weights[r][(size_t)local_t * K + min(k, K - 1)];
+  PairAcc<DT> acc[NV][N];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    V o{};
+    if (accumulate) o = orow[min(base + j * BLOCK + tid, row_vecs - 1)];
+#pragma unroll
+    for (int e = 0; e < N; ++e) acc[j][e].set(get_word(o, e));
+  }
+  const int mine = there && loaded >= 0 ? loaded : INT_MAX;
+  const int n = __popcll(__ballot(mine != INT_MAX && lane < (MANY ? 64 : BATCH)));
+  // place of this lane's row among the token's rows (all different), then rows and weights in order
+  int place = 0;
+  if constexpr (MANY) {
+    for (int b = 0; b < K; ++b) place += (int)(__builtin_amdgcn_readlane(mine, b) < mine);
+  } else {
+#define MOE_A2A_ROT(S) place += (int)(__builtin_amdgcn_update_dpp(0, mine, 0x120 + S, 0xf, 0xf, false) < mine)
+    MOE_A2A_ROT(1); MOE_A2A_ROT(2); MOE_A2A_ROT(3); MOE_A2A_ROT(4); MOE_A2A_ROT(5); MOE_A2A_ROT(6); MOE_A2A_ROT(7);
+#undef MOE_A2A_ROT
+  }
+  const int to = (MANY ? place : (lane & ~(BATCH - 1)) | place) << 2;  // (lanes without a row all get place n, which nothing reads)
+  const int ordered_row = __builtin_amdgcn_ds_permute(to, mine);
+  const int ordered_w = __builtin_amdgcn_ds_permute(to, __float_as_int(w_loaded));
+  for (int a0 = 0; a0 < n; a0 += BATCH) {
+    V v[BATCH][NV];
+    float w[BATCH];
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u) {
+      const int from = min(a0 + u, n - 1);  // (loaded again past the last one, and not used)
+      const int row = __builtin_amdgcn_readlane(ordered_row, from);
+      w[u] = __int_as_float(__builtin_amdgcn_readlane(ordered_w, from));
+#pragma unroll
+      for (int j = 0; j < NV; ++j)
+        v[u][j] = rows[(size_t)row * row_vecs + min(base + j * BLOCK + tid, row_vecs - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u) {
+      if (a0 + u < n) {
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+          for (int e = 0; e < N; ++e) acc[j][e].step(get_word(v[u][j], e), w[u]);
+      }
+    }
+    if (!MANY) break;
+  }
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int idx = base + j * BLOCK + tid;
+    if (idx < row_vecs) {
+      uint32_t h[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) h[e] = acc[j][e].word();
+      orow[idx] = from_words<V>(h);
+    }
+  }
+}
+
 // ---------------------------------------------------------------- host side
 
 struct Geometry {
@@ -3095,7 +3455,7 @@ long long group_items(long long rows, const Geometry& g) {
 
 extern "C" {
 
-const char* moe_a2a_version(void) { return "moe_a2a 0.6 gfx950"; }
+const char* moe_a2a_version(void) { return "moe_a2a 0.7 gfx950"; }
 
 #ifndef MOE_A2A_BUILD_ID
 #define MOE_A2A_BUILD_ID "unknown"
@@ -3681,6 +4041,7 @@ int dense_tile_rows(long long M, long long N) {
   return big > UNITS * 5 / 8 ? 256 : 128;
 }
 
+constexpr size_t local_plan_lds_bytes(int experts) { return (size_t)(2 + LPLAN_WAVES) * experts * sizeof(int); }
 constexpr size_t dense_lds_bytes(int BM, int BN) { return 2 * (size_t)(BM + BN) * 8 * sizeof(b128); }
 constexpr size_t skinny_lds_bytes(int tj, int waves) { return (size_t)waves * (32 + 32 * tj) * 8 * sizeof(b128); }
 
@@ -3712,6 +4073,7 @@ int allow_large_lds() {
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8>, skinny_lds_bytes(2, 8));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8>, skinny_lds_bytes(2, 8));
+  allow((const void*)local_plan_kernel, local_plan_lds_bytes(LOCAL_MAX_EXPERTS));
   if (!ok) return MOE_A2A_ELAUNCH;
   allowed[gpu] = true;
   return MOE_A2A_OK;
@@ -3960,5 +4322,156 @@ int moe_a2a_exchange_gather_local(int32_t world_size, int32_t hidden_dim, const 
   return launch_status();
 }
 
+
+}  // extern "C"
+
+namespace {
+
+bool local_supported(const moe_a2a_shape* s) {
+  return s->world_size <= LOCAL_MAX_RANKS && s->num_experts <= LOCAL_MAX_EXPERTS && s->experts_per_token <= LOCAL_MAX_K;
+}
+
+}  // namespace
+
+extern "C" {
+
+int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const int32_t* const* indices,
+                           const int32_t* num_tokens, int32_t compact_rows, int32_t in_dtype, int32_t out_dtype,
+                           int32_t* entry_row, int32_t* expert_num_tokens, int32_t* expert_offsets,
+                           void* expert_rows, int32_t* expert_meta, void* stream) {
+  if (!shape_ok(s) || !local_supported(s) || !x || !indices || !num_tokens || compact_rows < 0 || !expert_rows)
+    return MOE_A2A_EINVAL;
+  const bool standin = in_dtype >= 0 || out_dtype >= 0;
+  if (standin && ((in_dtype != MOE_A2A_F16 && in_dtype != MOE_A2A_BF16) ||
+                  (out_dtype != MOE_A2A_F16 && out_dtype != MOE_A2A_BF16)))
+    return MOE_A2A_EINVAL;
+  const int W = s->world_size, K = s->experts_per_token, E = s->num_experts;
+  LocalSources src;
+  bool all16 = aligned(expert_rows, 16);
+  long long tokens = 0;
+  for (int r = 0; r < W; ++r) {
+    if (num_tokens[r] < 0 || num_tokens[r] > s->max_num_tokens || (num_tokens[r] > 0 && (!x[r] || !indices[r])))
+      return MOE_A2A_EINVAL;
+    if (!aligned(x[r], 2)) return MOE_A2A_EALIGN;
+    all16 = all16 && aligned(x[r], 16);
+    src.x[r] = x[r];
+    src.indices[r] = indices[r];
+    src.first[r] = (int)tokens;
+    tokens += num_tokens[r];
+    if (tokens * K > INT_MAX / 2) return MOE_A2A_EINVAL;
+  }
+  src.first[W] = (int)tokens;
+  const int S = (int)(tokens * K);
+  if (!aligned(expert_rows, 2)) return MOE_A2A_EALIGN;
+  if (S > 0 && !entry_row) return MOE_A2A_EINVAL;
+  const bool compact = compact_rows > 0;
+  if (compact && compact_rows < S) return MOE_A2A_EINVAL;
+  Geometry g;
+  row_geometry(g, s->hidden_dim, all16);
+  g.nle = E / W;
+  g.max_recv = s->max_num_tokens * W;
+  g.magic = g.nle == 1 ? 0u : (uint32_t)(0xffffffffu / (uint32_t)g.nle) + 1u;
+  if ((long long)E * g.max_recv > INT_MAX || !items_fit(tokens, g.chunks)) return MOE_A2A_EINVAL;
+  // what the padded expert buffers and a rank's receive buffer have room for (the second only matters
+  // where a token can have more entries on a rank than the rank has experts)
+  const int expert_limit = compact && !standin ? INT_MAX : g.max_recv;
+  const int rank_limit = K > g.nle && g.nle > 1 ? (int)std::min<long long>((long long)g.max_recv * g.nle, INT_MAX) : 0;
+  hipStream_t st = (hipStream_t)stream;
+  // One rank with few entries: its mover ranks them (LOCAL_RANK_ENTRIES keys, eight per lane)
+  const bool ranked = W == 1 && S > 0 && S <= LOCAL_RANK_ENTRIES && rank_limit == 0;
+  if (!ranked) {
+    int expert_bits = 0, rank_bits = 0;
+    while ((1 << expert_bits) < E) ++expert_bits;
+    while ((1 << rank_bits) < W) ++rank_bits;
+    if (const int rc = allow_large_lds()) return rc;
+    const int tiles = std::max(1, (S + LPLAN_BLOCK - 1) / LPLAN_BLOCK);
+    local_plan_kernel<<<tiles, LPLAN_BLOCK, local_plan_lds_bytes(E), st>>>(
+        src, W, S, K, E, g.nle, expert_bits, rank_bits, compact, g.max_recv, expert_limit, rank_limit, entry_row,
+        expert_num_tokens, expert_offsets);
+    if (S == 0) return launch_status();
+  }
+  const int grid = (ranked ? 1 : 0) + (int)(tokens * g.chunks);
+#define LAUNCH_T(V, NV, DI, DO, RANKED)                                                                    \
+  local_dispatch_kernel<V, NV, DI, DO, RANKED><<<grid, BLOCK, 0, st>>>(                                    \
+      src, W, (int)tokens, K, E, g.nle, g.magic, g.row_vecs, g.chunks, compact, g.max_recv, expert_limit,  \
+      entry_row, expert_num_tokens, expert_offsets, (V*)expert_rows, expert_meta)
+#define LAUNCH(V, NV)                                                                                      \
+  do {                                                                                                     \
+    if (!standin) {                                                                                        \
+      if (ranked) LAUNCH_T(V, NV, -1, -1, true);                                                           \
+      else LAUNCH_T(V, NV, -1, -1, false);                                                                 \
+    } else if (ranked) {                                                                                   \
+      if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_BF16, true); \
+      else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_F16, true); \
+      else if (in_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_BF16, true);                  \
+      else LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_F16, true);                                               \
+    } else {                                                                                               \
+      if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_BF16, false); \
+      else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_F16, false); \
+      else if (in_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_BF16, false);                 \
+      else LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_F16, false);                                              \
+    }                                                                                                      \
+  } while (0)
+  MOE_A2A_FOR_ROW_KERNEL(g, LAUNCH);
+#undef LAUNCH
+#undef LAUNCH_T
+  return launch_status();
+}
+
+int moe_a2a_local_combine(const moe_a2a_shape* s, const void* expert_rows, const int32_t* entry_row,
+                          const float* const* weights, const int32_t* num_tokens, void* const* out_tokens,
+                          int32_t only_rank, int32_t accumulate, int32_t dtype, void* stream) {
+  if (!shape_ok(s) || !local_supported(s) || !weights || !num_tokens || !out_tokens || only_rank >= s->world_size ||
+      (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16))
+    return MOE_A2A_EINVAL;
+  const int W = s->world_size, K = s->experts_per_token;
+  LocalResults dst;
+  bool all16 = aligned(expert_rows, 16);
+  long long tokens = 0;
+  for (int r = 0; r < W; ++r) {
+    if (num_tokens[r] < 0 || num_tokens[r] > s->max_num_tokens) return MOE_A2A_EINVAL;
+    const bool wanted = (only_rank < 0 || r == only_rank) && num_tokens[r] > 0;
+    if (wanted && (!weights[r] || !out_tokens[r])) return MOE_A2A_EINVAL;
+    if (wanted && !aligned(out_tokens[r], 2)) return MOE_A2A_EALIGN;
+    all16 = all16 && (!wanted || aligned(out_tokens[r], 16));
+    dst.weights[r] = weights[r];
+    dst.out[r] = out_tokens[r];
+    dst.first[r] = (int)tokens;
+    tokens += num_tokens[r];
+    if (tokens * K > INT_MAX / 2) return MOE_A2A_EINVAL;
+  }
+  dst.first[W] = (int)tokens;
+  const int first = only_rank < 0 ? 0 : dst.first[only_rank];
+  const long long items = only_rank < 0 ? tokens : num_tokens[only_rank];
+  if (items == 0) return MOE_A2A_OK;
+  if (!expert_rows || !entry_row) return MOE_A2A_EINVAL;
+  if (!aligned(expert_rows, 2)) return MOE_A2A_EALIGN;
+  Geometry g;
+  row_geometry(g, s->hidden_dim, all16);
+  // one column of vectors per lane (eight rows of it in flight), two for rows of 257 to 512 vectors
+  const int nv = g.row_vecs > 2 * BLOCK ? 1 : g.row_vecs > BLOCK ? 2 : 1;
+  const int chunks = (g.row_vecs + BLOCK * nv - 1) / (BLOCK * nv);
+  if (!items_fit(items, chunks)) return MOE_A2A_EINVAL;
+  const int grid = (int)(items * chunks);
+  hipStream_t st = (hipStream_t)stream;
+#define LAUNCH(V, DT, NV, MANY)                                                                            \
+  local_combine_kernel<V, DT, NV, MANY><<<grid, BLOCK, 0, st>>>(dst, W, first, K, g.row_vecs, chunks,      \
+                                                                (const V*)expert_rows, entry_row, accumulate)
+#define PICK(V, DT)                                                                                        \
+  do {                                                                                                     \
+    if (K <= 8) { if (nv == 1) LAUNCH(V, DT, 1, false); else LAUNCH(V, DT, 2, false); }                    \
+    else { if (nv == 1) LAUNCH(V, DT, 1, true); else LAUNCH(V, DT, 2, true); }                             \
+  } while (0)
+  if (g.vec16) {
+    if (dtype == MOE_A2A_BF16) PICK(b128, MOE_A2A_BF16);
+    else PICK(b128, MOE_A2A_F16);
+  } else {
+    if (dtype == MOE_A2A_BF16) PICK(uint16_t, MOE_A2A_BF16);
+    else PICK(uint16_t, MOE_A2A_F16);
+  }
+#undef PICK
+#undef LAUNCH
+  return launch_status();
+}
 
 }  // extern "C"

@@ -408,3 +408,72 @@ void a2a_combine_send_compact(std::vector<int64_t> shape, torch::Tensor expert_y
                                       ints_or_null(send_back_plan), stream_of(stream)),
          "moe_a2a_combine_send_compact");
 }
+
+// ---- jobs whose ranks share the GPU
+
+void a2a_local_dispatch(const std::vector<int64_t>& shape, const std::vector<torch::Tensor>& x,
+                        const std::vector<torch::Tensor>& indices, bool compact,
+                        c10::optional<torch::Tensor> entry_row, c10::optional<torch::Tensor> expert_num_tokens,
+                        c10::optional<torch::Tensor> expert_offsets, torch::Tensor expert_rows,
+                        c10::optional<torch::Tensor> expert_meta, bool standin, int64_t stream) {
+  const moe_a2a_shape s = shape_of(shape);
+  const int64_t W = s.world_size, K = s.experts_per_token, H = std::max<int64_t>(s.hidden_dim, 1);
+  TORCH_CHECK(W >= 1 && W <= 64, "world_size: 1 to 64 ranks on one GPU");
+  TORCH_CHECK((int64_t)x.size() == W && (int64_t)indices.size() == W, "one x and one indices per rank");
+  const auto dt = rows_type(x[0], "x"), out = rows_type(expert_rows, "expert_rows");
+  TORCH_CHECK(standin || dt == out, "expert_rows: rows are moved as they are");
+  const void* xs[64];
+  const int32_t* ids[64];
+  int32_t tokens[64];
+  int64_t total = 0;
+  for (int64_t r = 0; r < W; ++r) {
+    TORCH_CHECK(indices[r].dim() == 2 && indices[r].size(1) == K, "indices[r]: expected [tokens, K]");
+    tokens[r] = to_i32(indices[r].size(0), "tokens");
+    need(x[r], "x[r]", dt, tokens[r] * H, &expert_rows);
+    need(indices[r], "indices[r]", torch::kInt32, tokens[r] * K, &expert_rows);
+    xs[r] = x[r].data_ptr();
+    ids[r] = ints(indices[r]);
+    total += tokens[r] * K;
+  }
+  const int64_t room = expert_rows.numel() / H;
+  need(expert_rows, "expert_rows", out, compact ? total * H : (int64_t)s.num_experts * s.max_num_tokens * W * H);
+  if (entry_row.has_value()) need(*entry_row, "entry_row", torch::kInt32, total, &expert_rows);
+  if (expert_num_tokens.has_value()) need(*expert_num_tokens, "expert_num_tokens", torch::kInt32, s.num_experts, &expert_rows);
+  if (expert_offsets.has_value()) need(*expert_offsets, "expert_offsets", torch::kInt32, s.num_experts + 1, &expert_rows);
+  if (expert_meta.has_value())
+    need(*expert_meta, "expert_meta", torch::kInt32,
+         (compact ? total : (int64_t)s.num_experts * s.max_num_tokens * W) * MOE_A2A_META_DIM, &expert_rows);
+  status(moe_a2a_local_dispatch(&s, xs, ids, tokens, compact ? to_i32(room, "rows of expert_rows") : 0,
+                                standin ? dtype_code(dt) : -1, standin ? dtype_code(out) : -1,
+                                ints_or_null(entry_row), ints_or_null(expert_num_tokens), ints_or_null(expert_offsets),
+                                expert_rows.data_ptr(), ints_or_null(expert_meta), stream_of(stream)),
+         "moe_a2a_local_dispatch");
+}
+
+void a2a_local_combine(const std::vector<int64_t>& shape, torch::Tensor expert_rows, torch::Tensor entry_row,
+                       const std::vector<torch::Tensor>& weights, const std::vector<torch::Tensor>& out_tokens,
+                       bool accumulate, int64_t stream) {
+  const moe_a2a_shape s = shape_of(shape);
+  const int64_t W = s.world_size, K = s.experts_per_token;
+  TORCH_CHECK(W >= 1 && W <= 64, "world_size: 1 to 64 ranks on one GPU");
+  TORCH_CHECK((int64_t)weights.size() == W && (int64_t)out_tokens.size() == W, "one weights and one out_tokens per rank");
+  const auto dt = rows_type(expert_rows, "expert_rows");
+  need(expert_rows, "expert_rows", dt, 0);
+  const float* ws[64];
+  void* outs[64];
+  int32_t tokens[64];
+  int64_t total = 0;
+  for (int64_t r = 0; r < W; ++r) {
+    TORCH_CHECK(weights[r].dim() == 2 && weights[r].size(1) == K, "weights[r]: expected [tokens, K]");
+    tokens[r] = to_i32(weights[r].size(0), "tokens");
+    need(weights[r], "weights[r]", torch::kFloat32, tokens[r] * K, &expert_rows);
+    need(out_tokens[r], "out_tokens[r]", dt, tokens[r] * (int64_t)s.hidden_dim, &expert_rows);
+    ws[r] = weights[r].data_ptr<float>();
+    outs[r] = out_tokens[r].data_ptr();
+    total += tokens[r] * K;
+  }
+  need(entry_row, "entry_row", torch::kInt32, total, &expert_rows);
+  status(moe_a2a_local_combine(&s, expert_rows.data_ptr(), ints(entry_row), ws, tokens, outs, -1, accumulate ? 1 : 0,
+                               dtype_code(dt), stream_of(stream)),
+         "moe_a2a_local_combine");
+}

@@ -9,15 +9,19 @@ seeds the harness would give those ranks); `custom_kernel` then steps the whole
 job through `LocalWorld` on the caller's device and returns the caller's rows.
 With `world_size == 1` nothing has to be registered.
 
-A harness calls the entry point again and again on jobs of one shape. The first
-call of a job (a shape and the token counts of its ranks) runs launch by launch
-and reads the exchanged counts back to size its launches; from the second call
-on the job is a HIP graph captured once (one per rank asked for: a call needs
-every rank's dispatch, experts and send-back, but only the caller's return
-exchange and weighted sum): the inputs are copied into buffers the
-graph reads, the graph is replayed, the result is copied out. The graph's
-launches are sized by the counts of the first call; sizes are a matter of speed
-only, every kernel moves what the device-side counts of the call at hand say.
+The ranks share the GPU, so a job is three launches whatever its size
+(`moe_a2a_local_dispatch`, `moe_a2a_local_combine`): where every entry's row goes,
+every rank's rows to their experts and through the stand-in expert, and the
+weighted sums of the ranks asked for. Nothing is read back, staged or kept
+between calls; buffers come from torch's allocator, so calls from several
+threads and streams do not meet. A job beyond the limits of those entry points
+(64 ranks, 1024 experts, 64 entries per token) steps through `LocalWorld`: the
+first call of a job (a shape and the token counts of its ranks) launch by launch,
+reading the exchanged counts back to size its launches, and from the second call
+on as a HIP graph captured once (one per rank asked for) that reads its inputs
+from buffers they are copied into. The graph's launches are sized by the counts
+of the first call; sizes are a matter of speed only, every kernel moves what the
+device-side counts of the call at hand say.
 """
 from __future__ import annotations
 
@@ -25,7 +29,8 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
-from .all2all import LocalWorld
+from . import _binding, _lib
+from .all2all import LOCAL_MAX_EXPERTS, LOCAL_MAX_K, LOCAL_MAX_RANKS, LocalWorld, _need, _stream
 from .task import MoEConfig, RankTestData, input_t, output_t
 
 _peers: Optional[Sequence[input_t]] = None
@@ -103,6 +108,52 @@ def _world_for(cfg: MoEConfig, world_size: int, device: torch.device) -> _World:
     return w
 
 
+def _fits_direct(cfg: MoEConfig, world_size: int) -> bool:
+    return (world_size <= LOCAL_MAX_RANKS and cfg.num_experts <= LOCAL_MAX_EXPERTS
+            and cfg.experts_per_token <= LOCAL_MAX_K)
+
+
+def _run_direct(cfg: MoEConfig, world_size: int, everyone: Sequence[RankTestData], device: torch.device,
+                only: Optional[int] = None) -> List[torch.Tensor]:
+    """One step of the job; `only=r` leaves out the other ranks' weighted sums (and returns rank r's alone)."""
+    if cfg.num_experts % world_size:
+        raise ValueError("num_experts must be a multiple of world_size")
+    K, H = cfg.experts_per_token, cfg.hidden_dim
+    xs, ids, weights, tokens = [], [], [], []
+    for d in everyone:
+        x, i, w = d.x, d.indices, d.weights
+        T = i.shape[0]
+        if i.shape[1] != K or x.shape != (T, H) or w.shape != (T, K):
+            raise ValueError("shapes of x / indices / weights do not match the config")
+        xs.append(_need(x, cfg.in_dtype, device, "x"))
+        ids.append(_need(i, torch.int32, device, "indices"))
+        weights.append(_need(w, torch.float32, device, "weights"))
+        tokens.append(T)
+    entries = sum(tokens) * K
+    stream = _stream(device)
+    shape = _lib.Shape(world_size, 0, cfg.num_experts, K, H, cfg.max_num_tokens)
+    c = _binding.get("ctypes")
+    rows = torch.empty((max(entries, 1), H), dtype=cfg.out_dtype, device=device)
+    where = torch.empty((max(entries, 1),), dtype=torch.int32, device=device)
+    c.local_dispatch(shape, xs, ids, True, where, None, None, rows, None, True, stream)
+    if only is None:
+        out = torch.empty((sum(tokens), H), dtype=cfg.out_dtype, device=device)
+        ys = list(out.split(tokens))
+        c.local_combine(shape, rows, where, weights, tokens, ys, -1, False, stream)
+        return ys
+    y = torch.empty((tokens[only], H), dtype=cfg.out_dtype, device=device)
+    c.local_combine(shape, rows, where, weights, tokens, [y if r == only else None for r in range(world_size)], only,
+                    False, stream)
+    return [y]
+
+
+def _there(d: RankTestData, device: torch.device) -> RankTestData:
+    index = device.index
+    if d.x.get_device() == index and d.indices.get_device() == index and d.weights.get_device() == index:
+        return d
+    return d.to(device)
+
+
 def custom_kernel_job(inputs: Sequence[input_t]) -> list:
     """Every rank's `custom_kernel` result from ONE step of the job: what W processes calling
     `custom_kernel` at the same time produce together. `inputs[r]` is rank r's tuple."""
@@ -112,8 +163,11 @@ def custom_kernel_job(inputs: Sequence[input_t]) -> list:
         raise RuntimeError("custom_kernel needs its inputs on a GPU; this path has no CPU fallback")
     if len(inputs) != world_size:
         raise ValueError(f"a job of world_size={world_size} needs {world_size} inputs, got {len(inputs)}")
+    everyone = [_there(d[1], device) for d in inputs]
     with torch.cuda.device(device):
-        ys = _world_for(cfg, world_size, device).run([d[1].to(device) for d in inputs])
+        if _fits_direct(cfg, world_size):
+            return _run_direct(cfg, world_size, everyone, device)
+        ys = _world_for(cfg, world_size, device).run(everyone)
         return [y.clone() for y in ys]
 
 
@@ -129,7 +183,9 @@ def custom_kernel(data: input_t) -> output_t:
             raise RuntimeError(
                 f"world_size={world_size}: register the job's per-rank inputs with set_peer_inputs() first"
             )
-        everyone = [rank_data if r == rank else _peers[r][1].to(device) for r in range(world_size)]
+        everyone = [rank_data if r == rank else _there(_peers[r][1], device) for r in range(world_size)]
     with torch.cuda.device(device):
+        if _fits_direct(cfg, world_size):
+            return _run_direct(cfg, world_size, everyone, device, only=rank)[0]
         ys = _world_for(cfg, world_size, device).run(everyone, only=rank)
         return ys[rank].clone()

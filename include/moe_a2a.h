@@ -66,7 +66,7 @@ typedef struct moe_a2a_shape {
 } moe_a2a_shape;
 
 /* Library version / build probe. Returns a static string such as
- * "moe_a2a 0.6 gfx950"; the number changes with the ABI. Never NULL. */
+ * "moe_a2a 0.7 gfx950"; the number changes with the ABI. Never NULL. */
 const char* moe_a2a_version(void);
 
 /* Identifies the sources this library was built from: the first 16 hex digits of
@@ -500,6 +500,58 @@ int moe_a2a_exchange_gather_local(int32_t world_size, int32_t hidden_dim,
                                   void* recv_buf, int32_t* recv_meta, int32_t* recv_counts,
                                   int32_t rows_hint, int32_t send_capacity_rows,
                                   int32_t recv_capacity_rows, void* stream);
+
+/*
+ * Jobs whose ranks all live on this GPU (a job of one rank among them): tokens
+ * go straight to their experts' rows and come straight back, with no send
+ * buffers, no exchange and no receive buffers in between. Rows land where
+ * dispatch_send, the exchange and dispatch_recv would have put them, and come
+ * back in the order in which combine_send, the exchange and combine_recv would
+ * have delivered them (all2all/reference.py:68-234), so results are the same
+ * bits.
+ *
+ *   x, indices, num_tokens   host arrays of world_size entries, one per rank:
+ *                 device pointers to the rank's rows [num_tokens[r], H] and expert
+ *                 ids int32[num_tokens[r], K], and the rank's token count
+ *   compact_rows  0: expert_rows is [num_experts, max_num_tokens * world_size, H];
+ *                 else the experts' rows lie back to back in a buffer of
+ *                 compact_rows rows (at least the entries of all ranks)
+ *   in_dtype, out_dtype   both -1: rows are moved as they are. Else rows of in_dtype
+ *                 arrive as the stand-in expert's result, `row.to(out_dtype) *
+ *                 (1 + rank of the expert)` (all2all/reference.py:262)
+ *   entry_row     int32[K * sum of num_tokens] out: the row of every (rank, token,
+ *                 k) entry in expert_rows, -1 for an entry that has none (an id
+ *                 outside [0, num_experts), or no room; as the padded buffers the
+ *                 stand-in form keeps max_num_tokens * world_size rows per expert)
+ *   expert_num_tokens   int32[num_experts] out, or NULL
+ *   expert_offsets      int32[num_experts + 1] out, or NULL (compact layout only)
+ *   expert_meta   int32[rows, 5] out (expert, source rank, token, k, 0), or NULL
+ * Limits: world_size <= 64, num_experts <= 1024, experts_per_token <= 64
+ * (MOE_A2A_EINVAL). One launch for one rank with up to 2048 entries, else two.
+ * The first call on a GPU sets kernel attributes: make it outside a graph capture.
+ */
+int moe_a2a_local_dispatch(const moe_a2a_shape* shape, const void* const* x,
+                           const int32_t* const* indices, const int32_t* num_tokens,
+                           int32_t compact_rows, int32_t in_dtype, int32_t out_dtype,
+                           int32_t* entry_row, int32_t* expert_num_tokens,
+                           int32_t* expert_offsets, void* expert_rows, int32_t* expert_meta,
+                           void* stream);
+
+/*
+ * The way back: out_tokens[r][t] (+)= expert_rows[entry_row[...]].float() *
+ * weights[r][t, k] in arrival order, rounded to `dtype` after every addend
+ * (all2all/reference.py:224-232).
+ *
+ *   weights, out_tokens   host arrays of world_size device pointers: float32
+ *                 [num_tokens[r], K] and rows [num_tokens[r], H]
+ *   only_rank     that rank's tokens alone (the other entries of the two arrays may
+ *                 be NULL), or -1 for every rank
+ *   accumulate    0: the sum starts from zero and out_tokens is only written
+ */
+int moe_a2a_local_combine(const moe_a2a_shape* shape, const void* expert_rows,
+                          const int32_t* entry_row, const float* const* weights,
+                          const int32_t* num_tokens, void* const* out_tokens,
+                          int32_t only_rank, int32_t accumulate, int32_t dtype, void* stream);
 
 #ifdef __cplusplus
 }
