@@ -1889,6 +1889,15 @@ constexpr int GEMM_KSTEP = 64;   // input elements per step: 8 vectors of 16 byt
 #endif
 constexpr int GEMM_DEPTH = MOE_A2A_GEMM_DEPTH;  // steps between a load and its use
 
+// The step of K at which the product of group g starts (it goes round from there). Rows a multiple of 4 KB
+// apart put the same step of every row on the same few memory channels, and workgroups that walk K side by
+// side then all ask those: 256-row panels read at 4.6 TB/s with rows of 8 KB and 4.3 with 12 KB, at 6.1 with
+// the panels started apart (5.1 and 5.6 with 4 KB; nothing between with 2, 6 and 14 KB). A function of the
+// group alone, so every kernel adds up a group's products in the same order.
+__device__ __forceinline__ int first_kstep(int g, int groups, int K) {
+  return K % 2048 ? 0 : (int)((long long)g * (K / GEMM_KSTEP) / groups);
+}
+
 // x [groups, max_rows, K], w [groups, N, K], bias [groups, N] or null, y [groups, max_rows, N];
 // rows_of_group null: every group has max_rows rows (a plain dense product when groups == 1).
 // GW waves per workgroup, 32 output columns each: every workgroup of an expert pulls the expert's
@@ -1985,6 +1994,11 @@ __global__ __launch_bounds__(64 * GW, GW > 4 ? 1 : TJ <= 2 ? MOE_A2A_GEMM_OCC : 
     const int le = __builtin_amdgcn_readfirstlane(home[0]);
     const int rows = __builtin_amdgcn_readfirstlane(home[3]);
     const int t0 = (rb - __builtin_amdgcn_readfirstlane(home[1])) * TOK;  // first token of the block (t0 < rows)
+    const int first_step = first_kstep(le, nle, K);
+    auto k_bytes = [=](int at) {  // byte of a row at which step number `at` of the walk begins
+      const int k = at + first_step;
+      return (k >= steps ? k - steps : k) * (GEMM_KSTEP * 2);
+    };
     // buffer row of the expert's first row
     const size_t row0 = compact ? (size_t)__builtin_amdgcn_readfirstlane(home[2]) : (size_t)le * max_recv;
     const int n0 = ct * (GW * 32) + __builtin_amdgcn_readfirstlane(wave) * 32;  // first output column of this wave
@@ -2024,11 +2038,11 @@ __global__ __launch_bounds__(64 * GW, GW > 4 ? 1 : TJ <= 2 ? MOE_A2A_GEMM_OCC : 
     b128 wv[D][4], xv[D][XL];
     auto load_w = [&](int set, int step) {
       const int at = min(step, steps - 1);  // past the end: the last step again, unused
-      const bool last = at == steps - 1;
+      const bool last = at == steps - 1;  // (rows of whole steps, the only ones that start elsewhere, have nothing past their end)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         wv[set][i] = __builtin_amdgcn_raw_buffer_load_b128(wbuf, woff[i] + (last ? wpast[i & 1] : 0),
-                                                           at * (GEMM_KSTEP * 2), 0);
+                                                           k_bytes(at), 0);
     };
     auto load_x = [&](int set, int step) {
       const int at = min(step, steps - 1);
@@ -2039,7 +2053,7 @@ __global__ __launch_bounds__(64 * GW, GW > 4 ? 1 : TJ <= 2 ? MOE_A2A_GEMM_OCC : 
       for (int i = 0; i < XL; ++i)
         if (loader && i * XROWS < live)
           xv[set][i] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, xoff[i] + (last ? xpast : 0),
-                                                             at * (GEMM_KSTEP * 2), 0);
+                                                             k_bytes(at), 0);
     };
     auto park_x = [&](int set) {
 #pragma unroll
@@ -2251,19 +2265,14 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
 
 // ---------------------------------------------------------------- dense product (many rows)
 //
-// C[M, N] = A[M, K] @ B[N, K]^T for thousands of rows: bound by the matrix cores, not by memory,
-// so the kernel is built around operand reuse. A workgroup owns a BM x BN tile of C (256 x 256
-// with four waves: a wave owns 128 x 128, sixteen 32 x 32 MFMA tiles, 256 accumulator registers,
-// one wave per SIMD) and walks K in steps of 64 elements. Per step the workgroup copies BM + BN
-// rows of 128 bytes into LDS once (through registers, two LDS buffers, one barrier per step), and
-// every wave reads each operand fragment it needs once per 16-element slice of the step for a
-// whole row or column of its MFMA tiles: 8 LDS reads for 16 MFMAs, issued one slice ahead.
-// With one wave per SIMD nothing hides a wave's own stalls, so the loop body is laid out by hand
-// (sched_group_barrier): exactly one memory instruction between two MFMAs, and every slice of a
-// step carries the same mix (8 fragment reads, 4 LDS stores, 4 global loads). Sixteen loads or
-// stores issued back to back make the wave wait for the queues of the memory pipes, which its
-// three neighbours fill at the same moment, and the matrix core idles meanwhile (measured at
-// 8192 x 8192 x 3584: 587 us -> 482 us with the interleaving, -> 466 us with the even mix).
+// C[M, N] = A[M, K] @ B[N, K]^T for outputs that tiles of 256 columns (phased_gemm_kernel) would spread over
+// too few compute units. A workgroup of four waves owns a BM x BN tile of C (64 x 128) and walks K in steps of
+// 64 elements. Per step the workgroup copies BM + BN rows of 128 bytes into LDS once (through registers, two LDS
+// buffers, one barrier per step), and every wave reads each operand fragment it needs once per 16-element slice
+// of the step for a whole row or column of its MFMA tiles, issued one slice ahead.
+// The loop body is laid out by hand (sched_group_barrier): memory instructions spread over the MFMAs, and every
+// slice of a step carries the same mix. Loads or stores issued back to back make the wave wait for the queues of
+// the memory pipes, which its neighbours fill at the same moment, and the matrix core idles meanwhile.
 // LDS rows are 128 bytes with the eight 16-byte vectors of a row XORed with bits 1..3 of the
 // row number (reads of 32 rows at one vector hit every bank equally); a thread stores linearly and
 // picks the global vector that belongs at its place, so the stores are conflict-free too.
@@ -2274,7 +2283,7 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
 // the 32 workgroups an XCD runs at a time share 4 row panels of A and 8 of B in its L2.
 
 template <int DT, int WM, int WN, int TM, int TN, bool GROUPED>
-__global__ __launch_bounds__(64 * WM * WN, TM * TN >= 16 ? 1 : 2) void dense_gemm_kernel(
+__global__ __launch_bounds__(64 * WM * WN, 2) void dense_gemm_kernel(
     const b128* __restrict__ A, const b128* __restrict__ B, const uint16_t* __restrict__ bias,
     uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
     const int* __restrict__ rows_of_group, int groups, int max_rows, int compact) {
@@ -2340,6 +2349,7 @@ __global__ __launch_bounds__(64 * WM * WN, TM * TN >= 16 ? 1 : 2) void dense_gem
   const b128* b_tile;         // the tile's first row of B (column n0 of the product)
   uint16_t* c_tile;           // the tile's first row of C
   const uint16_t* bias_row;   // the bias of the tile's group, or null
+  [[maybe_unused]] int k_first = 0;  // the step of K at which the tile starts
   if constexpr (GROUPED) {
     // whole rounds of the launch are renumbered so that an XCD works on consecutive pairs
     // (the column tiles of one row tile share its rows in that XCD's L2)
@@ -2370,6 +2380,7 @@ __global__ __launch_bounds__(64 * WM * WN, TM * TN >= 16 ? 1 : 2) void dense_gem
     rows_left = __builtin_amdgcn_readfirstlane(grp_home[3]) - t0;
     a_tile = A + (row0 + t0) * row_vecs;
     b_tile = B + ((size_t)g * N + n0) * row_vecs;
+    k_first = first_kstep(g, groups, K);
     c_tile = C + (row0 + t0) * N;
     bias_row = bias ? bias + (size_t)g * N : nullptr;
   } else {
@@ -2405,7 +2416,8 @@ __global__ __launch_bounds__(64 * WM * WN, TM * TN >= 16 ? 1 : 2) void dense_gem
   static_assert(LA % 2 == 0 && LB % 2 == 0, "quarters");
   auto load_quarter = [&](int q, int step) __attribute__((always_inline)) {
     const int at = min(step, steps - 1);  // (past the end: the last step again, never used)
-    const int soff = at * (GEMM_KSTEP * 2), off = coff + (at == steps - 1 ? cpast : 0);
+    const int k = GROUPED && at + k_first >= steps ? at + k_first - steps : at + k_first;
+    const int soff = k * (GEMM_KSTEP * 2), off = coff + (at == steps - 1 ? cpast : 0);
     if (q < 2) {
 #pragma unroll
       for (int i = q * (LA / 2); i < (q + 1) * (LA / 2); ++i)
@@ -2444,9 +2456,7 @@ __global__ __launch_bounds__(64 * WM * WN, TM * TN >= 16 ? 1 : 2) void dense_gem
   };
   // (GROUPED) bands of 32 rows of this wave's part of the tile that hold rows of the group: the
   // last row tile of a group computes only those, in a copy of the loop with that one condition
-  // (not for the 256 x 256 tile, whose registers have no room for the copy's state: it is used
-  // where groups have many rows, and an empty band is a small part of them)
-  constexpr bool SKIP_BANDS = GROUPED && TM * TN < 16;
+  constexpr bool SKIP_BANDS = GROUPED;
   [[maybe_unused]] const int live_bands = min(max((rows_left - wm * TM * 32 + 31) / 32, 0), TM);
   auto mfmas = [&](int set, auto ragged) __attribute__((always_inline)) {
 #pragma unroll
@@ -2478,32 +2488,18 @@ __global__ __launch_bounds__(64 * WM * WN, TM * TN >= 16 ? 1 : 2) void dense_gem
   load_quarter(0, 2);
   __syncthreads();
   read_frags(0, 0, 0);
-  // One memory instruction between two MFMAs: a wave that issues its loads or stores back to back
-  // waits for the queues of the memory pipes and issues no MFMA meanwhile. A slice holds TM * TN
-  // MFMAs, TM + TN fragment reads and one quarter's stores and loads; the 256 x 256 tile has its
-  // measured order (read, store, read, load), smaller tiles spread theirs over the leading MFMAs.
+  // A wave that issues its loads or stores back to back waits for the queues of the memory pipes and issues no
+  // MFMA meanwhile: a slice's TM + TN fragment reads and one quarter's stores and loads are spread over its
+  // TM * TN MFMAs.
   constexpr int N_MFMA = TM * TN, N_QUARTER = (LA > LB ? LA : LB) / 2;
   constexpr int READS_EACH = (TM + TN + N_MFMA - 1) / N_MFMA, MOVES_EACH = (N_QUARTER + N_MFMA - 1) / N_MFMA;
 #define MOE_A2A_INTERLEAVE()                                            \
-  if constexpr (N_MFMA == 16 && N_QUARTER == 4) {                       \
-    _Pragma("unroll") for (int q = 0; q < 4; ++q) {                     \
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                \
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                \
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                \
-      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);                \
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                \
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                \
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                \
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                \
-    }                                                                   \
-  } else {                                                              \
     _Pragma("unroll") for (int q = 0; q < N_MFMA; ++q) {                \
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                \
       __builtin_amdgcn_sched_group_barrier(0x100, READS_EACH, 0);       \
       __builtin_amdgcn_sched_group_barrier(0x200, MOVES_EACH, 0);       \
       __builtin_amdgcn_sched_group_barrier(0x020, MOVES_EACH, 0);       \
     }                                                                   \
-  }                                                                     \
   __builtin_amdgcn_sched_barrier(0);
   auto one_step = [&](int step, int cur, auto ragged) __attribute__((always_inline)) {  // cur = step & 1, a constant where this is called
     read_frags(1, cur, 1);
@@ -2612,11 +2608,17 @@ __global__ __launch_bounds__(64 * WM * WN, TM * TN >= 16 ? 1 : 2) void dense_gem
 //    and no memory instruction ever stands between two MFMAs of the group that owns the matrix cores.
 //  - Phases have to be even: rows of one operand are requested in the first slice of a step and rows of the
 //    other in the second. All of them in one phase cost 12 % (324 against 363 us at 8192 x 8192 x 3712).
-//  - Lookahead: 160 KB hold five half-steps of 32 KB. One operand (A, or B with LONG_B) gets three buffers
-//    and is asked for two steps ahead, the other two buffers and one step; with two of each, rows that start
-//    off the 128-byte lines (K = 3696) ran 17 % longer (399 against 340 us).
+//  - Lookahead: 160 KB hold five half-steps of 32 KB. One operand gets three buffers and is asked for two steps
+//    ahead, the other two buffers and one step; with two of each, rows that start off the 128-byte lines
+//    (K = 3696) ran 17 % longer (399 against 340 us). Steps of 32 elements in a ring of five buffers look
+//    farther ahead but ask for half lines: 425 against 380 us at K = 4096.
 //  - Rows that start off the lines take one and three quarter times the line requests: AHEAD then brings the
 //    lines into L2 before (operands out of HBM, K = 3696: 390 -> 372 us; on aligned rows it costs 1 to 2 %).
+//  - GROUPED (the experts' products): a group's weights are read for a few hundred rows only, and what a
+//    compute unit can fetch, about 49 KB a microsecond with most lines on their way from HBM, bounds it. The
+//    fewer tiles the better: up to 320 rows per tile (two buffers of each operand fit), spread evenly over the
+//    tiles of a group, and only the bands of 32 rows that there are get fetched and multiplied. 32 groups x 256
+//    rows, 2048 x 4096: 208 us with dense_gemm_kernel's 128 x 128 tiles, 156 here; 1024 rows 407 -> 254.
 // Measured at 8192 x 8192 (bf16, uniform values, clocks settled): K = 3696 395 us with dense_gemm_kernel's
 // 256 x 256 tile, 340 here (1.46 PFLOP/s); K = 4096 x 4096 x 4096 107 and 90; K = 8192 795 and 702.
 //
@@ -2662,17 +2664,98 @@ template <> struct Mfma16x16x32<MOE_A2A_F16> {
 
 constexpr int phased_rows(int TM) { return 32 * TM; }
 constexpr int phased_cols(int TN) { return 64 * TN; }
-constexpr size_t phased_lds_bytes(int TM, int TN, bool long_b) {
-  return (size_t)((long_b ? 2 : 3) * phased_rows(TM) + (long_b ? 3 : 2) * phased_cols(TN)) * 128;
+constexpr size_t phased_lds_bytes(int TM, int TN, int NA, int NB) {
+  return (size_t)(NA * phased_rows(TM) + NB * phased_cols(TN)) * 128;
 }
 
-template <int DT, int TM, int TN, bool LONG_B, bool AHEAD>
+// Tiles of a grouped product: A is [groups, max_rows, K], B [groups, N, K], C [groups, max_rows, N], and group g
+// has rows_of_group[g] rows (read here, clamped to max_rows). A group's rows are spread evenly over the fewest
+// tiles of BM rows, in whole bands of 32; tiles are numbered by group, column tile and row tile, so that
+// neighbours share the group's weights. compact: A and C hold the groups' rows back to back in buffers of
+// max_rows rows. The rows ahead of a group are a prefix over the counts, and a group only has the rows that
+// still fit the buffers (counts that add up to more never send a load or a store past their end).
+struct GroupTile {
+  int total;       // tiles of the product; the rest holds for a tile below that
+  int group, tn;   // group and column tile
+  int rows;        // rows of the tile, at least 1
+  size_t row_at;   // its first row in A and C
+};
+
+// Every thread sums the tiles of a run of groups, a scan over the workgroup (NT lanes) places the runs, and the
+// thread whose run holds the tile walks it to find the group. `lds` is 20 ints that nobody else uses until the
+// barrier after the call.
+template <int NT, int BM>
+__device__ __forceinline__ GroupTile find_group_tile(int tile, const int* __restrict__ rows_of_group, int groups,
+                                                     int max_rows, int tiles_n, bool compact, int* lds) {
+  constexpr int NW = NT / 64;
+  static_assert(NW <= 8, "20 ints");
+  int* const red = lds;
+  int* const red_rows = lds + 8;
+  int* const home = lds + 16;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  auto rows_of = [=](int g) { return min(max(rows_of_group[g], 0), max_rows); };
+  auto kept_of = [=](int g, int ahead) {
+    const int n = rows_of(g);
+    return compact ? min(ahead + n, max_rows) - min(ahead, max_rows) : n;
+  };
+  auto tiles_for = [=](int rows) { return (rows + BM - 1) / BM * tiles_n; };
+  const int per = (groups + NT - 1) / NT, run_first = min(tid * per, groups), run_end = min(run_first + per, groups);
+  int run_rows = 0, run_tiles = 0;
+  for (int g = run_first; g < run_end; ++g) run_rows += rows_of(g);
+  const int inc_rows = wave_inclusive_scan(run_rows);
+  if (lane == 63) red_rows[wave] = inc_rows;
+  lds_barrier();
+  int run_ahead = inc_rows - run_rows;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) run_ahead += w < wave ? red_rows[w] : 0;
+  for (int g = run_first, ahead = run_ahead; g < run_end; ahead += rows_of(g), ++g) run_tiles += tiles_for(kept_of(g, ahead));
+  const int inc = wave_inclusive_scan(run_tiles);
+  if (lane == 63) red[wave] = inc;
+  lds_barrier();
+  int run_begin = inc - run_tiles, total = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    run_begin += w < wave ? red[w] : 0;
+    total += red[w];
+  }
+  GroupTile at;
+  at.total = __builtin_amdgcn_readfirstlane(total);
+  if (tile >= at.total) return at;
+  // (an XCD works on a run of consecutive tiles)
+  const int logical = xcd_contiguous(tile, at.total);
+  if (run_begin <= logical && logical < run_begin + run_tiles) {
+    int g = run_first, first = run_begin, ahead = run_ahead;
+    for (;; ++g) {
+      const int n = tiles_for(kept_of(g, ahead));
+      if (logical < first + n) break;
+      first += n;
+      ahead += rows_of(g);
+    }
+    const int kept = kept_of(g, ahead), n = (kept + BM - 1) / BM, height = ((kept + n - 1) / n + 31) / 32 * 32;
+    const int tn = (logical - first) / n, t0 = (logical - first - tn * n) * height;
+    home[0] = g;
+    home[1] = tn;
+    home[2] = (compact ? min(ahead, max_rows) : 0) + t0;
+    home[3] = min(height, kept - t0);
+  }
+  lds_barrier();
+  at.group = __builtin_amdgcn_readfirstlane(home[0]);
+  at.tn = __builtin_amdgcn_readfirstlane(home[1]);
+  at.row_at = (compact ? 0 : (size_t)at.group * max_rows) + __builtin_amdgcn_readfirstlane(home[2]);
+  at.rows = __builtin_amdgcn_readfirstlane(home[3]);
+  return at;
+}
+
+template <int DT, int TM, int TN, int NA, int NB, bool AHEAD, bool GROUPED>
 __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
     const b128* __restrict__ A, const b128* __restrict__ B, const uint16_t* __restrict__ bias,
-    uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n) {
+    uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
+    const int* __restrict__ rows_of_group, int groups, int max_rows, int compact) {
   constexpr int BM = phased_rows(TM), BN = phased_cols(TN), GROUP_M = 4;
   constexpr int LA = BM / 64, LB = BN / 64;  // direct loads (8 rows each) of a wave per step
-  constexpr int NA = LONG_B ? 2 : 3, NB = LONG_B ? 3 : 2;
+  constexpr bool TIGHT = NA == 2 && NB == 2;  // two buffers of either operand
+  static_assert(BM % 64 == 0 && (TIGHT ? !AHEAD : NA >= 2 && NB >= 2 && NA + NB == 5), "whole loads, and a schedule for the buffers");
+  constexpr bool B_FIRST = NB <= NA;  // the operand with fewer buffers is asked for in the first slice of a step
   constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, B_AT = NA * A_BYTES;
   extern __shared__ b128 tile_lds[];  // [NA][BM * 8], [NB][BN * 8]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2681,22 +2764,47 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   const int tail_vecs = row_vecs - (steps - 1) * 8;
   const bool first_group = wave < 4;
 
-  const int logical = xcd_contiguous(blockIdx.x, gridDim.x);
-  const int per_group = GROUP_M * tiles_n, group = logical / per_group, in = logical - group * per_group;
-  const int group_rows = min(GROUP_M, tiles_m - group * GROUP_M);
-  const int tn = in / group_rows, tm = group * GROUP_M + in - tn * group_rows;
-  const int n0 = tn * BN, rows_left = M - tm * BM;
-  uint16_t* c_tile = C + (size_t)tm * BM * N;
+  int tile = blockIdx.x;
+  [[maybe_unused]] int total_tiles = 0;
+  do {  // (one pass unless GROUPED, whose launch strides over the tiles: its size is a matter of speed only)
+  int n0, rows_left;         // first column of the tile; rows of the matrix from the tile's first one on
+  size_t row_at, b_at;       // the tile's first rows of A and C, and of B
+  const uint16_t* bias_row;  // the bias of the tile's group, or null
+  [[maybe_unused]] int tn, tm, k_first = 0;
+  if constexpr (GROUPED) {
+    lds_barrier();  // the tile before is out of LDS
+    const GroupTile at = find_group_tile<512, BM>(tile, rows_of_group, groups, max_rows, tiles_n, compact, (int*)tile_lds);
+    if (tile >= at.total) return;
+    lds_barrier();
+    total_tiles = at.total;
+    n0 = at.tn * BN;
+    rows_left = at.rows;
+    row_at = at.row_at;
+    b_at = (size_t)at.group * N + n0;
+    k_first = first_kstep(at.group, groups, K) * (GEMM_KSTEP * 2);
+    bias_row = bias ? bias + (size_t)at.group * N : nullptr;
+  } else {
+    const int logical = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int per_group = GROUP_M * tiles_n, group = logical / per_group, in = logical - group * per_group;
+    const int group_rows = min(GROUP_M, tiles_m - group * GROUP_M);
+    tn = in / group_rows, tm = group * GROUP_M + in - tn * group_rows;
+    n0 = tn * BN;
+    rows_left = M - tm * BM;
+    row_at = (size_t)tm * BM;
+    b_at = n0;
+    bias_row = bias;
+  }
+  uint16_t* c_tile = C + row_at * N;
 
   // As in dense_gemm_kernel: rows past the end of a matrix read as zeros (they lie past the extent), and
   // so do the vectors past the end of a row in the last step and everything past the last step.
-  const b128 abuf = buffer_words(A + (size_t)tm * BM * row_vecs, min(BM, rows_left) * row_bytes);
-  const b128 bbuf = buffer_words(B + (size_t)n0 * row_vecs, min(BN, N - n0) * row_bytes);
+  const b128 abuf = buffer_words(A + row_at * row_vecs, min(BM, rows_left) * row_bytes);
+  const b128 bbuf = buffer_words(B + b_at * row_vecs, min(BN, N - n0) * row_bytes);
   constexpr int OUT_OF_RANGE = 0x40000000;
   const int sub = lane >> 3;
   auto vec_of = [&](int row) { return (lane & 7) ^ ((row >> 1) & 7); };
-  auto a_row = [&](int i) { return (wave * LA + i) * 8 + sub; };
-  auto b_row = [&](int i) { return (wave * LB + i) * 8 + sub; };
+  auto a_row = [&](int i) { return (i * 8 + wave) * 8 + sub; };
+  auto b_row = [&](int i) { return (i * 8 + wave) * 8 + sub; };
   int aoff[LA], boff[LB];
 #pragma unroll
   for (int i = 0; i < LA; ++i) aoff[i] = a_row(i) * row_bytes + vec_of(a_row(i)) * 16;
@@ -2722,8 +2830,9 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   };
 
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) b128*)tile_lds;
-  const unsigned a_base = lds0 + wave * LA * 1024, b_base = lds0 + B_AT + wave * LB * 1024;
-  int a_soff = 0, b_soff = 0;          // byte of a row at which the next requested step begins
+  const unsigned a_base = lds0 + wave * 1024, b_base = lds0 + B_AT + wave * 1024;
+  // byte of a row at which the next requested step begins
+  int a_soff = GROUPED ? k_first : 0, b_soff = a_soff;
   unsigned a_fill = 0, b_fill = 0;     // buffer (as a byte offset) that the next requested step goes to
   unsigned a_use = 0, b_use = 0;       // buffer of the step being multiplied
   auto next_a = [](unsigned at) { return at == (NA - 1) * A_BYTES ? 0u : at + A_BYTES; };
@@ -2731,18 +2840,20 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   auto load_a = [&]() __attribute__((always_inline)) {
     unrolled<0, LA>([&](auto c) __attribute__((always_inline)) {
       constexpr int i = decltype(c)::value;
-      load_to_lds<i * 1024>(a_base + a_fill, aoff[i], abuf, a_soff);
+      load_to_lds<i * 8192>(a_base + a_fill, aoff[i], abuf, a_soff);
     });
     a_fill = next_a(a_fill);
     a_soff += GEMM_KSTEP * 2;
+    if (GROUPED && k_first && a_soff == row_bytes) a_soff = 0;
   };
   auto load_b = [&]() __attribute__((always_inline)) {
     unrolled<0, LB>([&](auto c) __attribute__((always_inline)) {
       constexpr int i = decltype(c)::value;
-      load_to_lds<i * 1024>(b_base + b_fill, boff[i], bbuf, b_soff);
+      load_to_lds<i * 8192>(b_base + b_fill, boff[i], bbuf, b_soff);
     });
     b_fill = next_b(b_fill);
     b_soff += GEMM_KSTEP * 2;
+    if (GROUPED && k_first && b_soff == row_bytes) b_soff = 0;
   };
 
   // AHEAD: a wave touches, four steps ahead, one line each of the rows this workgroup fetches into L2 for its
@@ -2752,8 +2863,10 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   constexpr int AHEAD_STEPS = 4;
   [[maybe_unused]] uint32_t touched = 0;
   [[maybe_unused]] int touch_off = 0;
-  [[maybe_unused]] const b128 touch_buf = first_group ? abuf : bbuf;
-  if constexpr (AHEAD) {
+  [[maybe_unused]] const b128 touch_buf = !GROUPED && first_group ? abuf : bbuf;
+  if constexpr (AHEAD && GROUPED) {
+    touch_off = lane < BN / 8 ? (wave * (BN / 8) + lane) * row_bytes : OUT_OF_RANGE;
+  } else if constexpr (AHEAD) {
     constexpr int A_EACH = BM / 8 / 4, B_EACH = BN / GROUP_M / 4;  // rows of a wave of either group
     const int row = first_group ? (tn & 7) * (BM / 8) + wave * A_EACH + lane
                                 : (tm & (GROUP_M - 1)) * (BN / GROUP_M) + (wave - 4) * B_EACH + lane;
@@ -2777,59 +2890,99 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   }
   b128 af[TM], bf[TN];
   f32x4 acc[TM][TN] = {};
-  auto read_frags = [&](int slice) __attribute__((always_inline)) {
+  auto read_frags = [&](auto bands, int slice) __attribute__((always_inline)) {
     const char* ap = a_frag[slice] + a_use;
     const char* bp = b_frag[slice] + b_use;
 #pragma unroll
     for (int j = 0; j < TN; ++j) bf[j] = *(const b128*)(bp + j * (16 * 128));
 #pragma unroll
-    for (int i = 0; i < TM; ++i) af[i] = *(const b128*)(ap + i * (32 * 128));
+    for (int i = 0; i < decltype(bands)::value; ++i) af[i] = *(const b128*)(ap + i * (32 * 128));
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto multiply = [&]() __attribute__((always_inline)) {  // this wave's turn at the matrix cores
+  // this wave's turn at the matrix cores; `begin` and `end` are what it does first and last in it
+  auto multiply = [&](auto bands, auto begin, auto end) __attribute__((always_inline)) {
     __builtin_amdgcn_s_waitcnt(WAIT_LDS_ONLY);
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
+    begin();
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < decltype(bands)::value; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = Mfma16x16x32<DT>::mma(bf[j], af[i], acc[i][j]);
     __builtin_amdgcn_sched_barrier(0);
+    end();
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // Step s reads its buffers in both of its slices. In the first it asks for step s + 1 of the operand with
-  // two buffers (the buffer of step s - 1: the other group has read its last slice in the phase before), in
-  // the second for step s + 2 of the operand with three. Before the barrier that ends the second reading
-  // phase the wave waits for all of its loads but the ones just made: step s + 1 is then in LDS for everybody
-  // one barrier later, when the first group gets there.
-  auto one_step = [&](int step) __attribute__((always_inline)) {
-    read_frags(0);
-    if constexpr (LONG_B) load_a(); else load_b();
-    multiply();
-    read_frags(1);
-    if constexpr (LONG_B) load_b(); else load_a();
+  // Step s reads its buffers in both of its slices. In the first it asks for the operand with fewer buffers, n
+  // of them: step s + n - 1, into the buffer of step s - 1 (the other group has read its last slice in the phase
+  // before); in the second likewise for the other operand. Before the barrier that ends the second reading phase
+  // the wave waits for everything that step s + 1 needs, which is all but the youngest loads: step s + 1 is then
+  // in LDS for everybody one barrier later, when the first group gets there.
+  auto nothing = []() __attribute__((always_inline)) {};
+  auto one_slice_pair = [&](auto bands, int step) __attribute__((always_inline)) {
+    read_frags(bands, 0);
+    if constexpr (B_FIRST) load_b(); else load_a();
+    multiply(bands, nothing, nothing);
+    read_frags(bands, 1);
+    if constexpr (B_FIRST) load_a(); else load_b();
     touch(step + AHEAD_STEPS);
     a_use = next_a(a_use);
     b_use = next_b(b_use);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LONG_B ? LB : LA) + (AHEAD ? 1 : 0)) : "memory");
-    multiply();
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((B_FIRST ? LA : LB) + (AHEAD ? 1 : 0)) : "memory");
+    multiply(bands, nothing, nothing);
   };
-  a_range(0);
-  b_range(0);
-  load_a();
-  load_b();
-  if constexpr (LONG_B) { b_range(1); load_b(); } else { a_range(1); load_a(); }
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LONG_B ? LB : LA) : "memory");
+  // With two buffers of either operand the rows of step s + 1 can only go to the buffers of step s - 1, and have
+  // to be there when the first group has multiplied step s: both groups wait in the phase before that, the first
+  // behind its MFMAs, the second behind its last reads. Rows of B, which come from farther away, are asked for
+  // first; the second group asks for rows of A at the start of its turn, a phase earlier than it could else.
+  auto one_tight_step = [&](auto bands) __attribute__((always_inline)) {
+    read_frags(bands, 0);
+    load_b();
+    multiply(bands, [&]() __attribute__((always_inline)) { if (!first_group) load_a(); }, nothing);
+    read_frags(bands, 1);
+    if (first_group) load_a();
+    a_use = next_a(a_use);
+    b_use = next_b(b_use);
+    if (!first_group) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    multiply(bands, nothing,
+             [&]() __attribute__((always_inline)) { if (first_group) asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); });
+  };
+  unrolled<0, 2>([&](auto c) __attribute__((always_inline)) {
+    constexpr int at = decltype(c)::value;
+    if constexpr (at < NA - 1) { a_range(at); load_a(); }
+    if constexpr (at < NB - 1) { b_range(at); load_b(); }
+  });
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NA - 2) * LA + (NB - 2) * LB) : "memory");
   if (!first_group) asm volatile("s_barrier" ::: "memory");  // one phase behind
-  int step = 0;
-  for (; step + 3 < steps; ++step) one_step(step);  // (what it asks for lies before the last step)
-  for (; step < steps; ++step) {
-    a_range(step + (LONG_B ? 1 : 2));
-    b_range(step + (LONG_B ? 2 : 1));
-    one_step(step);
+  auto walk_k = [&](auto bands) __attribute__((always_inline)) {
+    int step = 0;
+    if constexpr (TIGHT) {
+      for (; step + 2 < steps; ++step) one_tight_step(bands);
+      for (; step < steps; ++step) {
+        a_range(step + 1);
+        b_range(step + 1);
+        one_tight_step(bands);
+      }
+    } else {
+      for (; step + 3 < steps; ++step) one_slice_pair(bands, step);  // (what it asks for lies before the last step)
+      for (; step < steps; ++step) {
+        a_range(step + NA - 1);
+        b_range(step + NB - 1);
+        one_slice_pair(bands, step);
+      }
+    }
+  };
+  // A group's tile multiplies only the bands of 32 rows that it has: a copy of the loop per number of them (a
+  // condition on every band inside one loop takes registers that the loop needs)
+  if constexpr (GROUPED) {
+    const int live = (min(rows_left, BM) + 31) / 32;
+    unrolled<1, TM + 1>([&](auto bands) __attribute__((always_inline)) { if (live == decltype(bands)::value) walk_k(bands); });
+  } else {
+    walk_k(std::integral_constant<int, TM>{});
   }
   if (first_group) asm volatile("s_barrier" ::: "memory");
   // (the loads past the last step write zeros)
@@ -2844,12 +2997,14 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
     char* park = (char*)tile_lds + wave * (16 * PITCH);
     const int ncol = n0 + wn * TN * 16;
     uint32_t bias2[TN][2] = {};
-    if (bias) {
+    if (bias_row) {
 #pragma unroll
       for (int j = 0; j < TN; ++j)
-        if (ncol + j * 16 < N) __builtin_memcpy(bias2[j], bias + ncol + j * 16 + q * 4, 8);
+        if (ncol + j * 16 < N) __builtin_memcpy(bias2[j], bias_row + ncol + j * 16 + q * 4, 8);
     }
-    const int rrow = lane / VR, rvec = lane % VR;
+    int rrow = lane / VR, rvec = lane % VR;
+    // (the places of all bands are worked out here: ahead of the loop over tiles they would take 60 registers)
+    asm volatile("" : "+v"(rrow), "+v"(rvec));
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -2857,7 +3012,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
         const f32x4& c = acc[i][j];
         uint32_t two[2] = {Pair16<DT>::canonical(Pair16<DT>::round(c[0], c[1])),
                            Pair16<DT>::canonical(Pair16<DT>::round(c[2], c[3]))};
-        if (bias) {
+        if (bias_row) {
 #pragma unroll
           for (int e = 0; e < 2; ++e)
             two[e] = Pair16<DT>::canonical(Pair16<DT>::round(
@@ -2875,6 +3030,8 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
       }
     }
   }
+  tile += gridDim.x;
+  } while (GROUPED && tile < total_tiles);
 }
 
 // ---------------------------------------------------------------- exchange stand-in
@@ -4057,18 +4214,22 @@ int allow_large_lds() {
   auto allow = [&](const void* kernel, size_t bytes) {
     ok = ok && hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
   };
-  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, false, false>, phased_lds_bytes(8, 4, false));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, false, false>, phased_lds_bytes(8, 4, false));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, false, true>, phased_lds_bytes(8, 4, false));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, false, true>, phased_lds_bytes(8, 4, false));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 4, 2, false, false>, phased_lds_bytes(4, 2, false));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 4, 2, false, false>, phased_lds_bytes(4, 2, false));
+  auto allow_grouped = [&](auto dtype) {
+    constexpr int DT = decltype(dtype)::value;
+    allow((const void*)phased_gemm_kernel<DT, 10, 4, 2, 2, false, true>, phased_lds_bytes(10, 4, 2, 2));
+    allow((const void*)phased_gemm_kernel<DT, 8, 4, 2, 3, false, true>, phased_lds_bytes(8, 4, 2, 3));
+    allow((const void*)phased_gemm_kernel<DT, 6, 4, 2, 3, false, true>, phased_lds_bytes(6, 4, 2, 3));
+  };
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 2, false, false>, phased_lds_bytes(8, 4, 3, 2));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 2, false, false>, phased_lds_bytes(8, 4, 3, 2));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 2, true, false>, phased_lds_bytes(8, 4, 3, 2));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 2, true, false>, phased_lds_bytes(8, 4, 3, 2));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 4, 2, 3, 2, false, false>, phased_lds_bytes(4, 2, 3, 2));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 4, 2, 3, 2, false, false>, phased_lds_bytes(4, 2, 3, 2));
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 4, 4, true>, dense_lds_bytes(256, 256));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 4, 4, true>, dense_lds_bytes(256, 256));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 2, 2, true>, dense_lds_bytes(128, 128));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 2, 2, true>, dense_lds_bytes(128, 128));
+  allow_grouped(std::integral_constant<int, MOE_A2A_BF16>{});
+  allow_grouped(std::integral_constant<int, MOE_A2A_F16>{});
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8>, skinny_lds_bytes(2, 8));
@@ -4094,8 +4255,9 @@ int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, i
   const int grid = (int)(tiles_m * tiles_n);
   if (const int rc = allow_large_lds()) return rc;
 #define LAUNCH_P(DT, TM, TN, AHEAD)                                                              \
-  phased_gemm_kernel<DT, TM, TN, false, AHEAD><<<grid, 512, phased_lds_bytes(TM, TN, false), st>>>( \
-      (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n)
+  phased_gemm_kernel<DT, TM, TN, 3, 2, AHEAD, false><<<grid, 512, phased_lds_bytes(TM, TN, 3, 2), st>>>( \
+      (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n, \
+      nullptr, 0, 0, 0)
 #define LAUNCH_DT(DT)                                                                            \
   do {                                                                                           \
     if (tile == 256 && K * 2 % 128 != 0) LAUNCH_P(DT, 8, 4, true);                               \
@@ -4115,13 +4277,38 @@ int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, i
 #ifndef MOE_A2A_GROUPED_DENSE_MIN_ROWS
 #define MOE_A2A_GROUPED_DENSE_MIN_ROWS 56  // rows per group (from the caller's row count) from which tiles are used
 #endif
-#ifndef MOE_A2A_GROUPED_DENSE_BIG_ROWS
-#define MOE_A2A_GROUPED_DENSE_BIG_ROWS 768  // ... and from which they are 256 x 256 instead of 128 x 128
-#endif
+// How a grouped product with `rows` rows in an average group is cut: the height of its tiles in bands of 32
+// rows (10, 8, 6: phased_gemm_kernel, 256 columns; 2: dense_gemm_kernel, 64 x 128). A tile costs what a compute
+// unit has to fetch for it, (rows + columns) x 128 bytes per step of K: that, and not the matrix cores, bounds
+// these kernels (measured on 32 groups of 256 rows, 137 GFLOP: 163 us, 145 without the MFMAs, 119 without the
+// loads; a unit fetches about 49 KB a microsecond). Tiles run in rounds over the units. A group is taken to have
+// one standard deviation of uniform routing more rows than the average: it decides how many tiles most groups
+// need. 320 rows leave room for two buffers of each operand only and get 15 % on top.
+// Measured, us (rows: 320, 256, 192, 64 x 128): 32 groups x 256 rows, N 2048, K 4096: 156 188 171 -; N 4096, K
+// 2048: 164 173 183 -; 512 rows: 266 276 259 -; 128 rows: 133 111 108 -; 16 x 1024 rows, N 4096, K 2048: 261 254
+// 260 -; 8 x 200, N 7168, K 2048: 73 62 88 -; 16 x 150, 2880 x 2880: 87 73 71 136; 8 x 64, N 2048, K 7168: 168 117
+// 112 75; 4 x 300, N 2048, K 4096: 97 64 58 43; 4 x 1000, N 512, K 7168: 169 119 104 70.
+int grouped_tile_bands(long long rows, int groups, int N) {
+  constexpr long long UNITS = 256;
+  const long long most = std::max<long long>(1, rows + (long long)std::sqrt((double)rows));
+  int best_bands = 0;
+  double best = 0;
+  for (const int bands : {8, 6, 10, 2}) {
+    const long long high = bands * 32, wide = bands == 2 ? 128 : 256, n = (most + high - 1) / high;
+    const long long height = std::min(high, ((most + n - 1) / n + 31) / 32 * 32);
+    const long long rounds = (n * groups * ((N + wide - 1) / wide) + UNITS - 1) / UNITS;
+    const double cost = (double)rounds * (height + wide) * (bands == 10 ? 1.15 : 1.0);
+    if (!best_bands || cost < best) {
+      best = cost;
+      best_bands = bands;
+    }
+  }
+  return best_bands;
+}
 
 // The grouped product when groups have hundreds of rows: the weights are then read for enough
 // rows that the matrix cores, not the stream of weights, bound the work, and the dense kernel's
-// tiles (each weight row read once per 128 or 256 rows, operands shared by four waves through
+// tiles (each weight row read once per 64 to 320 rows, operands shared by the workgroup's waves through
 // LDS) do better than the kernel that is built around streaming. MOE_A2A_NOT_DENSE otherwise.
 int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void* w, const void* bias, void* y,
                          int groups, long long max_rows, long long rows_hint, int N, int K, int dtype,
@@ -4131,36 +4318,30 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
   if (!rows_of_group || rows_hint < (long long)MOE_A2A_GROUPED_DENSE_MIN_ROWS * groups) return MOE_A2A_NOT_DENSE;
   if ((long long)K * 2 * 256 >= (1 << 30) || max_rows > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
-#ifndef MOE_A2A_GROUPED_DENSE_TILE
-#define MOE_A2A_GROUPED_DENSE_TILE 0  // (measurements) 256, 128 or 64: that tile height for every launch
-#endif
-  // 256 x 256 when groups have rows for several bands of them; 64 x 128 when tiles of 128 x 128
-  // would not give every compute unit one
-  const int tile = MOE_A2A_GROUPED_DENSE_TILE ? MOE_A2A_GROUPED_DENSE_TILE
-                   : rows_hint >= (long long)MOE_A2A_GROUPED_DENSE_BIG_ROWS * groups ? 256
-                   : (rows_hint / 128 + groups) * ((N + 127) / 128) <= 256 ? 64 : 128;
-  const int BM = tile, BN = tile == 64 ? 128 : tile;
+  const int bands = grouped_tile_bands(rows_hint / groups, groups, N);
+  const int BM = bands * 32, BN = bands == 2 ? 128 : 256;
   const long long tiles_n = (N + BN - 1) / BN;
   // every group can end in a partly filled row tile; the kernel strides over what the hint misses
   const long long pairs = (rows_hint / BM + groups) * tiles_n;
   if ((max_rows / BM + 1) * groups * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
-  const int grid = mover_blocks(pairs);
-  const size_t lds_bytes = dense_lds_bytes(BM, BN);
+  const int grid = mover_blocks((pairs + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
   if (const int rc = allow_large_lds()) return rc;
-#define LAUNCH_GD(DT, TM, TN)                                                                 \
-  dense_gemm_kernel<DT, 2, 2, TM, TN, true><<<grid, 256, lds_bytes, st>>>(                    \
-      (const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, 0, N, K, 0, (int)tiles_n,        \
-      rows_of_group, groups, (int)max_rows, compact)
-  if (dtype == MOE_A2A_BF16) {
-    if (tile == 256) LAUNCH_GD(MOE_A2A_BF16, 4, 4);
-    else if (tile == 128) LAUNCH_GD(MOE_A2A_BF16, 2, 2);
-    else LAUNCH_GD(MOE_A2A_BF16, 1, 2);
-  } else {
-    if (tile == 256) LAUNCH_GD(MOE_A2A_F16, 4, 4);
-    else if (tile == 128) LAUNCH_GD(MOE_A2A_F16, 2, 2);
-    else LAUNCH_GD(MOE_A2A_F16, 1, 2);
-  }
-#undef LAUNCH_GD
+  auto launch = [&](auto dtype_const) {
+    constexpr int DT = decltype(dtype_const)::value;
+    auto phased = [&](auto kernel, size_t lds_bytes) {
+      kernel<<<grid, 512, lds_bytes, st>>>((const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, 0, N, K,
+                                           0, (int)tiles_n, rows_of_group, groups, (int)max_rows, compact);
+    };
+    if (bands == 10) phased(phased_gemm_kernel<DT, 10, 4, 2, 2, false, true>, phased_lds_bytes(10, 4, 2, 2));
+    else if (bands == 8) phased(phased_gemm_kernel<DT, 8, 4, 2, 3, false, true>, phased_lds_bytes(8, 4, 2, 3));
+    else if (bands == 6) phased(phased_gemm_kernel<DT, 6, 4, 2, 3, false, true>, phased_lds_bytes(6, 4, 2, 3));
+    else
+      dense_gemm_kernel<DT, 2, 2, 1, 2, true><<<grid, 256, dense_lds_bytes(64, 128), st>>>(
+          (const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, 0, N, K, 0, (int)tiles_n, rows_of_group,
+          groups, (int)max_rows, compact);
+  };
+  if (dtype == MOE_A2A_BF16) launch(std::integral_constant<int, MOE_A2A_BF16>{});
+  else launch(std::integral_constant<int, MOE_A2A_F16>{});
   return launch_status();
 }
 

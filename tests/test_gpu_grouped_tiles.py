@@ -1,0 +1,56 @@
+"""The tiles of the grouped product (`moe_a2a_expert_gemm` and its compact form): 64 x 128 and 192, 256 or 320
+rows x 256 columns, which of them from the caller's row count. The row count must change no bit of the result,
+and K may start anywhere in a group's walk (rows a multiple of 4 KB apart do)."""
+import pytest
+import torch
+
+from amd_distributed_2025_amd import HIPAllToAll, MoEConfig
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# rows per group -> tile, by groups (see grouped_tile_bands): N = 7168 is 28 tiles of 256 columns
+ROWS_FOR_TILE = {3: {56: "64 x 128", 150: "256", 200: "192"}, 5: {300: "320"}}
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("groups,counts", [
+    (3, [1, 193, 257]), (3, [700, 0, 31]), (3, [192, 256, 320]), (3, [64, 65, 63]),
+    (5, [321, 1, 0, 33, 640]), (5, [320, 319, 289, 288, 641]),
+])
+@pytest.mark.parametrize("K", [8, 200, 2048, 2112])  # one short step; a tail; a walk that starts apart; one that does not
+def test_every_tile_gives_the_same_bits(groups, counts, K, bias, dt):
+    print(f"tiles groups={groups} counts={counts} K={K} bias={bias} {dt}", flush=True)
+    N, T = 7168, 704
+    a = HIPAllToAll(MoEConfig(groups, 1, K, T, dt, dt), 0, 1, device=torch.device(DEV))
+    g = torch.Generator(device=DEV).manual_seed(K + sum(counts))
+    x = torch.randn(groups, T, K, generator=g, device=DEV).to(dt)
+    w = (torch.randn(groups, N, K, generator=g, device=DEV) / K ** 0.5).to(dt)
+    b = torch.randn(groups, N, generator=g, device=DEV).to(dt) if bias else None
+    num = torch.tensor(counts, dtype=torch.int32, device=DEV)
+    flat = torch.cat([x[e, :c] for e, c in enumerate(counts)] + [x[0, :5]]).contiguous()  # (and rows of nobody)
+
+    def run(rows, hint):
+        out = torch.full((*rows.shape[:-1], N), 7.0, dtype=dt, device=DEV)
+        return a.expert_gemm(rows, num, w, b, rows_hint=hint, out=out)
+
+    base = run(x, 0)  # the streaming kernel
+    ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt]  # of one rounding, to either side
+    for e, c in enumerate(counts):
+        want = x[e, :c].double() @ w[e].double().T
+        # K float32 sums and a rounding; with a bias a second one, and the first is of the sum without it
+        bound = ulp * want.abs() + 2.0 ** -24 * K * (x[e, :c].double().abs() @ w[e].double().abs().T)
+        if bias:
+            want = want + b[e].double()
+            bound = (1 + ulp) * bound + ulp * want.abs()
+        assert ((base[e, :c].double() - want).abs() <= bound + 2.0 ** -24).all(), f"group {e}"
+        assert (base[e, c:] == 7).all()
+    for rows in ROWS_FOR_TILE[groups]:
+        got = run(x, rows * groups)
+        assert torch.equal(got, base), f"row count {rows} per group"
+        got = run(flat, rows * groups)
+        at = 0
+        for e, c in enumerate(counts):
+            assert torch.equal(got[at:at + c], base[e, :c]), f"compact, row count {rows} per group, group {e}"
+            at += c
+        assert (got[at:] == 7).all()
