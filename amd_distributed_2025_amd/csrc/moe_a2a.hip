@@ -1853,7 +1853,8 @@ __global__ __launch_bounds__(64 * ROWS) void expert_scale_wave_kernel(
 // Tiles are numbered over (expert, block of tokens) by a prefix over the device-side counts, so a
 // hot expert is spread over as many workgroups as it has blocks and an empty one costs nothing.
 // Every block of an expert re-reads the expert's weights: TJ = 4 (128 tokens) is used when the
-// caller's row count says blocks of 64 would not hold most experts.
+// caller's row count says blocks of 64 would not hold most experts, TJ = 1 (32 tokens, 64 columns per
+// workgroup) when experts have a handful of rows.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -1882,7 +1883,7 @@ template <> struct Mfma32x32x16<MOE_A2A_F16> {
 #define MOE_A2A_GEMM_DEPTH 2
 #endif
 constexpr int BUFFER_RAW_32BIT = 0x00020000;  // word 3 of a gfx9 buffer descriptor: raw buffer of 32-bit data
-constexpr int GEMM_COLS = 128;   // output columns per workgroup, 32 per wave
+constexpr int GEMM_COLS = 128;   // output columns per workgroup (of four waves), 32 per wave
 constexpr int GEMM_KSTEP = 64;   // input elements per step: 8 vectors of 16 bytes per row
 #ifndef MOE_A2A_GEMM_DEPTH4
 #define MOE_A2A_GEMM_DEPTH4 3  // with blocks of 128 tokens (two workgroups per unit: 655 against 675 us at C4)
@@ -1903,13 +1904,13 @@ __device__ __forceinline__ int first_kstep(int g, int groups, int K) {
 // GW waves per workgroup, 32 output columns each: every workgroup of an expert pulls the expert's
 // token rows through its own L1, so wider workgroups halve that traffic (GW = 8: one workgroup of
 // 512 lanes per compute unit instead of two of 256).
-template <int DT, int TJ, int GW>
-__global__ __launch_bounds__(64 * GW, GW > 4 ? 1 : TJ <= 2 ? MOE_A2A_GEMM_OCC : MOE_A2A_GEMM_OCC4) void expert_gemm_kernel(
+// TJ = 1: two waves per workgroup, and either many of those per unit (D = 2) or few with twice the lookahead.
+template <int DT, int TJ, int GW, int D>
+__global__ __launch_bounds__(64 * GW, GW > 4 || D > 3 ? 1 : TJ == 1 ? 4 : TJ == 2 ? MOE_A2A_GEMM_OCC : MOE_A2A_GEMM_OCC4) void expert_gemm_kernel(
     const b128* __restrict__ expert_x, const int* __restrict__ expert_num_tokens,
     const b128* __restrict__ weights, const uint16_t* __restrict__ bias, uint16_t* __restrict__ expert_y,
     int nle, int max_recv, int N, int K, int col_tiles, int compact) {
   constexpr int TOK = TJ * 32;               // tokens per block
-  constexpr int D = TJ >= 4 ? MOE_A2A_GEMM_DEPTH4 : GEMM_DEPTH;
   __shared__ b128 xs[D][TOK * 8];            // D steps of TOK tokens x 8 vectors
   constexpr int THREADS = 64 * GW;
   // the token rows of a step are fetched and parked by all lanes when their number divides the
@@ -2027,7 +2028,7 @@ __global__ __launch_bounds__(64 * GW, GW > 4 ? 1 : TJ <= 2 ? MOE_A2A_GEMM_OCC : 
       wslot[i] = row * 8 + slot;
       if (i < 2) wpast[i] = vec >= tail_vecs ? OUT_OF_RANGE : 0;  // (loads i and i + 2 take the same vector)
     }
-    constexpr int XROWS = LOADERS / 8;  // token rows one load of the workgroup covers: 32 or 64
+    constexpr int XROWS = LOADERS / 8;  // token rows one load of the workgroup covers: 16, 32 or 64
     const bool loader = LOADERS == THREADS || tid < LOADERS;  // (whole waves)
     const int xrow = tid >> 3, xvec = slot ^ ((xrow >> 1) & 7);  // (XROWS * i does not change bits 1..3)
     const int xpast = xvec >= tail_vecs ? OUT_OF_RANGE : 0;
@@ -2048,7 +2049,8 @@ __global__ __launch_bounds__(64 * GW, GW > 4 ? 1 : TJ <= 2 ? MOE_A2A_GEMM_OCC : 
       const int at = min(step, steps - 1);
       const bool last = at == steps - 1;
       // (load i holds tokens XROWS * i .. of the block: a load without a valid token is neither
-      // issued nor parked, and a tile of 32 tokens without one is not multiplied)
+      // issued nor parked, and a tile of 32 tokens without one is not multiplied; what is left in the place
+      // of a token that was not parked only reaches the results of that token, which are not stored)
 #pragma unroll
       for (int i = 0; i < XL; ++i)
         if (loader && i * XROWS < live)
@@ -4130,7 +4132,16 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
   // per-lane byte offsets inside a block of tokens and inside a wave's 32 weight rows are 32-bit
   if ((long long)K * 2 * 128 >= (1 << 30) || max_rows > INT_MAX / 2) return MOE_A2A_EINVAL;
-  const int tj = rows_hint > (long long)MOE_A2A_GEMM_ROWS_FOR_128 * groups ? 4 : 2;
+  // Up to eight rows per group: blocks of 32 rows on workgroups of 64 columns. Twice as many of them share the
+  // stream of weights out more evenly, and where there are too few to keep it in flight (up to two per unit, of
+  // the groups that uniform routing would hit) each looks four steps ahead. Measured, us, blocks of 64 rows on
+  // 128 columns / two steps / four (rows per group, groups, N x K): 2.25, 64, 2048 x 1024 52.6 / 44.4 / -; the same,
+  // 1024 x 2048 44.8 / 44.5 / -; 4, 8, 7168 x 2048 45.6 / 42.2 / -; 2, 64, 512 x 7168 98.1 / 89.4 / 71.6; 1, 4,
+  // 2048 x 7168 85.8 / 73.0 / 38.2; 4, 8, 1024 x 2048 21.6 / 18.5 / 14.1; at 24 rows 53.4 / 56.2.
+  const bool few = rows_hint <= 8ll * groups && (max_rows / 32 + 1) * groups * ((N + 63) / 64) <= INT_MAX / 2;
+  const double hit = groups * (1.0 - std::exp(-(double)rows_hint / groups));
+  const bool far_ahead = hit * ((N + 63) / 64) <= 512;
+  const int tj = few ? 1 : rows_hint > (long long)MOE_A2A_GEMM_ROWS_FOR_128 * groups ? 4 : 2;
   // every group can end in a partly filled block of tokens; the kernel strides over what the hint misses
   const long long row_blocks = rows_hint / (tj * 32) + groups;
   // Workgroups of up to 256 columns (8 waves, one workgroup per compute unit) pull an expert's
@@ -4143,7 +4154,7 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
 #define MOE_A2A_GEMM_WIDE_MIN_TILES 512
 #endif
   constexpr int UNITS = 256;  // compute units of an MI355X
-  int gw = 4;
+  int gw = few ? 2 : 4;
   if (tj == 4 && row_blocks * ((N + 255) / 256) >= MOE_A2A_GEMM_WIDE_MIN_TILES) {
     const long long blocks = std::max<long long>(groups, (rows_hint + 127) / 128);
     double best = -1.0;
@@ -4158,18 +4169,20 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   const int col_tiles = (N + cols - 1) / cols;
   if ((max_rows / 64 + 1) * groups * col_tiles > INT_MAX / 2) return MOE_A2A_EINVAL;
   const int grid = mover_blocks(row_blocks * col_tiles);
-#define LAUNCH_G(DT, TJ, GW)                                                                          \
-  expert_gemm_kernel<DT, TJ, GW><<<grid, 64 * GW, 0, st>>>((const b128*)x, rows_of_group, (const b128*)w, \
-                                                           (const uint16_t*)bias, (uint16_t*)y, groups,  \
-                                                           (int)max_rows, N, K, col_tiles, compact)
-#define LAUNCH_GW(DT)                                 \
-  do {                                                \
-    if (tj == 2) LAUNCH_G(DT, 2, 4);                  \
-    else if (gw == 8) LAUNCH_G(DT, 4, 8);             \
-    else if (gw == 7) LAUNCH_G(DT, 4, 7);             \
-    else if (gw == 6) LAUNCH_G(DT, 4, 6);             \
-    else if (gw == 5) LAUNCH_G(DT, 4, 5);             \
-    else LAUNCH_G(DT, 4, 4);                          \
+#define LAUNCH_G(DT, TJ, GW, D)                                                                       \
+  expert_gemm_kernel<DT, TJ, GW, D><<<grid, 64 * GW, 0, st>>>((const b128*)x, rows_of_group, (const b128*)w, \
+                                                              (const uint16_t*)bias, (uint16_t*)y, groups,  \
+                                                              (int)max_rows, N, K, col_tiles, compact)
+#define LAUNCH_GW(DT)                                             \
+  do {                                                            \
+    if (few && far_ahead) LAUNCH_G(DT, 1, 2, 4);                  \
+    else if (few) LAUNCH_G(DT, 1, 2, 2);                          \
+    else if (tj == 2) LAUNCH_G(DT, 2, 4, GEMM_DEPTH);             \
+    else if (gw == 8) LAUNCH_G(DT, 4, 8, MOE_A2A_GEMM_DEPTH4);    \
+    else if (gw == 7) LAUNCH_G(DT, 4, 7, MOE_A2A_GEMM_DEPTH4);    \
+    else if (gw == 6) LAUNCH_G(DT, 4, 6, MOE_A2A_GEMM_DEPTH4);    \
+    else if (gw == 5) LAUNCH_G(DT, 4, 5, MOE_A2A_GEMM_DEPTH4);    \
+    else LAUNCH_G(DT, 4, 4, MOE_A2A_GEMM_DEPTH4);                 \
   } while (0)
   if (dtype == MOE_A2A_BF16) LAUNCH_GW(MOE_A2A_BF16);
   else LAUNCH_GW(MOE_A2A_F16);

@@ -1,6 +1,7 @@
-"""The tiles of the grouped product (`moe_a2a_expert_gemm` and its compact form): 64 x 128 and 192, 256 or 320
-rows x 256 columns, which of them from the caller's row count. The row count must change no bit of the result,
-and K may start anywhere in a group's walk (rows a multiple of 4 KB apart do)."""
+"""The tiles of the grouped product (`moe_a2a_expert_gemm` and its compact form): blocks of 32, 64 or 128 rows that
+stream the weights, 64 x 128 and 192, 256 or 320 rows x 256 columns, which of them from the caller's row count.
+The row count must change no bit of the result, and K may start anywhere in a group's walk (rows a multiple of
+4 KB apart do)."""
 import pytest
 import torch
 
@@ -9,7 +10,8 @@ from amd_distributed_2025_amd import HIPAllToAll, MoEConfig
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 # rows per group -> tile, by groups (see grouped_tile_bands): N = 7168 is 28 tiles of 256 columns
-ROWS_FOR_TILE = {3: {56: "64 x 128", 150: "256", 200: "192"}, 5: {300: "320"}}
+ROWS_FOR_TILE = {3: {20: "stream 64", 50: "stream 128", 56: "64 x 128", 150: "256", 200: "192"},
+                 5: {8: "stream 32, two steps ahead", 20: "stream 64", 300: "320"}}
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
@@ -34,7 +36,7 @@ def test_every_tile_gives_the_same_bits(groups, counts, K, bias, dt):
         out = torch.full((*rows.shape[:-1], N), 7.0, dtype=dt, device=DEV)
         return a.expert_gemm(rows, num, w, b, rows_hint=hint, out=out)
 
-    base = run(x, 0)  # the streaming kernel
+    base = run(x, 0)  # streams in blocks of 32 rows, four steps ahead
     ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt]  # of one rounding, to either side
     for e, c in enumerate(counts):
         want = x[e, :c].double() @ w[e].double().T
