@@ -1854,7 +1854,7 @@ __global__ __launch_bounds__(64 * ROWS) void expert_scale_wave_kernel(
 // hot expert is spread over as many workgroups as it has blocks and an empty one costs nothing.
 // Every block of an expert re-reads the expert's weights: TJ = 4 (128 tokens) is used when the
 // caller's row count says blocks of 64 would not hold most experts, TJ = 1 (32 tokens, 64 columns per
-// workgroup) when experts have a handful of rows.
+// workgroup) when experts have a handful of rows or there are few workgroups.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -4132,15 +4132,20 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
   // per-lane byte offsets inside a block of tokens and inside a wave's 32 weight rows are 32-bit
   if ((long long)K * 2 * 128 >= (1 << 30) || max_rows > INT_MAX / 2) return MOE_A2A_EINVAL;
-  // Up to eight rows per group: blocks of 32 rows on workgroups of 64 columns. Twice as many of them share the
-  // stream of weights out more evenly, and where there are too few to keep it in flight (up to two per unit, of
-  // the groups that uniform routing would hit) each looks four steps ahead. Measured, us, blocks of 64 rows on
-  // 128 columns / two steps / four (rows per group, groups, N x K): 2.25, 64, 2048 x 1024 52.6 / 44.4 / -; the same,
-  // 1024 x 2048 44.8 / 44.5 / -; 4, 8, 7168 x 2048 45.6 / 42.2 / -; 2, 64, 512 x 7168 98.1 / 89.4 / 71.6; 1, 4,
-  // 2048 x 7168 85.8 / 73.0 / 38.2; 4, 8, 1024 x 2048 21.6 / 18.5 / 14.1; at 24 rows 53.4 / 56.2.
-  const bool few = rows_hint <= 8ll * groups && (max_rows / 32 + 1) * groups * ((N + 63) / 64) <= INT_MAX / 2;
-  const double hit = groups * (1.0 - std::exp(-(double)rows_hint / groups));
-  const bool far_ahead = hit * ((N + 63) / 64) <= 512;
+  // Blocks of 32 rows on workgroups of 64 columns where they do better than 64 x 128. (1) Up to eight rows per
+  // group: twice as many workgroups share the stream of weights out more evenly. (2) Too few workgroups to keep
+  // that stream in flight, at most two per unit: each then looks four steps ahead. They are counted as uniform
+  // routing would have it: the groups that get a row, or half a block on top of whole ones. Measured, us, blocks
+  // of 64 on 128 columns / of 32 on 64, two steps / four (rows per group, groups, N x K): 2.25, 64, 2048 x 1024 52.6
+  // / 44.4 / -; the same, 1024 x 2048 44.8 / 44.5 / -; 4, 8, 7168 x 2048 45.6 / 42.2 / -; 2, 64, 512 x 7168 98.1 /
+  // 89.4 / 71.6; 1, 4, 2048 x 7168 85.8 / 73.0 / 38.2; 4, 8, 1024 x 2048 21.6 / 18.5 / 14.1; 20, 4, 2048 x 7168 86.3 /
+  // - / 39.7; 30, 8, 1024 x 4096 45.1 / - / 23.9; 40, 8, 2048 x 7168 101.5 / - / 58.8; but 24, 64, 1024 x 2048 53.4 /
+  // 56.2 / 62.1 and 40, 32, 1024 x 512 11.5 / - / 12.4.
+  const double average = (double)rows_hint / groups;
+  const double blocks_of_32 = groups * std::max(1.0 - std::exp(-average), average / 32 + 0.5);
+  const bool counts_fit_32 = (max_rows / 32 + 1) * groups * ((N + 63) / 64) <= INT_MAX / 2;
+  const bool far_ahead = counts_fit_32 && blocks_of_32 * ((N + 63) / 64) <= 512;
+  const bool few = counts_fit_32 && (far_ahead || average <= 8);
   const int tj = few ? 1 : rows_hint > (long long)MOE_A2A_GEMM_ROWS_FOR_128 * groups ? 4 : 2;
   // every group can end in a partly filled block of tokens; the kernel strides over what the hint misses
   const long long row_blocks = rows_hint / (tj * 32) + groups;
@@ -4175,7 +4180,7 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
                                                               (int)max_rows, N, K, col_tiles, compact)
 #define LAUNCH_GW(DT)                                             \
   do {                                                            \
-    if (few && far_ahead) LAUNCH_G(DT, 1, 2, 4);                  \
+    if (far_ahead) LAUNCH_G(DT, 1, 2, 4);                         \
     else if (few) LAUNCH_G(DT, 1, 2, 2);                          \
     else if (tj == 2) LAUNCH_G(DT, 2, 4, GEMM_DEPTH);             \
     else if (gw == 8) LAUNCH_G(DT, 4, 8, MOE_A2A_GEMM_DEPTH4);    \

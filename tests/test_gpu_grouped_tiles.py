@@ -10,7 +10,7 @@ from amd_distributed_2025_amd import HIPAllToAll, MoEConfig
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 # rows per group -> tile, by groups (see grouped_tile_bands): N = 7168 is 28 tiles of 256 columns
-ROWS_FOR_TILE = {3: {20: "stream 64", 50: "stream 128", 56: "64 x 128", 150: "256", 200: "192"},
+ROWS_FOR_TILE = {3: {20: "stream 32, four steps ahead", 50: "stream 128", 56: "64 x 128", 150: "256", 200: "192"},
                  5: {8: "stream 32, two steps ahead", 20: "stream 64", 300: "320"}}
 
 
