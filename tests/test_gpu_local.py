@@ -86,6 +86,9 @@ def test_combine_of_other_tensors_takes_the_halves():
     (2, 8, 8, 64, [40, 33], "twins"), (4, 8, 4, 72, [50, 2, 50, 31], "twins"), (2, 2, 4, 64, [20, 20], "twins"),
     (8, 256, 8, 520, [160] * 8, "ids"), (64, 128, 3, 64, [2] * 64, None), (1, 16, 4, 264, [70], "ids"),
     (1, 32, 12, 264, [300], None), (3, 9, 2, 7168, [11, 1, 40], None),
+    # ranked by the mover: experts with more entries than room, ids outside the range, up to 2048 entries and just above
+    (1, 4, 4, 264, [64], "twins"), (2, 16, 4, 72, [60, 50], "twins"), (8, 64, 8, 520, [32] * 8, "ids"),
+    (8, 64, 8, 64, [32] * 7 + [33], None), (7, 63, 9, 96, [32, 1, 60, 7, 33, 64, 30], None),
 ])
 def test_custom_kernel_matches_the_halves(W, E, K, H, tokens, spoil, din, dout):
     print(f"job W={W} E={E} K={K} H={H} {tokens[:4]} {spoil} {din}", flush=True)
