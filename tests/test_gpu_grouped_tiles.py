@@ -56,3 +56,17 @@ def test_every_tile_gives_the_same_bits(groups, counts, K, bias, dt):
             assert torch.equal(got[at:at + c], base[e, :c]), f"compact, row count {rows} per group, group {e}"
             at += c
         assert (got[at:] == 7).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (33, 96, 4096), (64, 2080, 2048), (8, 1024, 6144), (64, 64, 8192)])
+def test_few_rows_whose_walks_of_K_start_apart(M, N, K):
+    """`moe_a2a_linear` on at most 64 rows of a multiple of 2048 inputs: small integers, whose sums every order
+    gives exactly (|sums| <= K < 2^24, and those a bfloat16 cannot hold are rounded once)."""
+    from amd_distributed_2025_amd import gemm_rs
+
+    print(f"linear M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randint(-1, 2, (M, K), generator=g, device=DEV).bfloat16()
+    w = torch.randint(-1, 2, (N, K), generator=g, device=DEV).bfloat16()
+    got = gemm_rs.local_product((x, w, None))
+    assert torch.equal(got, (x.double() @ w.double().T).float().bfloat16())
