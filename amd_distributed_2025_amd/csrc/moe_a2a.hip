@@ -3274,28 +3274,31 @@ __global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
 }
 
 // DIN / DOUT >= 0: rows leave as `row.to(out) * (1 + rank of the expert)` (all2all/reference.py:262).
-// RANKED: entry_row is worked out here (W <= LOCAL_RANKED_RANKS, S <= LOCAL_RANK_ENTRIES), and workgroup 0 counts
+// RANKED > 0: entry_row is worked out here (W <= RANKED, S <= LOCAL_RANK_ENTRIES), and workgroup 0 counts
 // the rows per expert where the caller wants to know them; else it is read.
-// Measured with a plan launch / ranked here: 8 ranks x 16 tokens, 2 experts of 8 each, hidden 6144 42.0 / 38.2 us a
-// job, 124 / 93 the first on new inputs.
-template <typename V, int NV, int DIN, int DOUT, bool RANKED>
+// Measured with a plan launch / ranked here: 8 ranks x 16 tokens, 2 experts of 8 each, hidden 6144 41.7 / 38 us a
+// job, of which the kernels take 5.8 + 4.7 / 8.1.
+template <typename V, int NV, int DIN, int DOUT, int RANKED>
 __global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
     LocalSources src, int W, int T, int K, int E, int nle, uint32_t magic, int row_vecs, int chunks, bool compact,
     int max_recv, int expert_limit, int* __restrict__ entry_row, int* __restrict__ expert_num_tokens,
     int* __restrict__ expert_offsets, V* __restrict__ rows, int* __restrict__ meta) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   int q = blockIdx.x;
-  [[maybe_unused]] auto key_at = [&](int i) {  // expert id of entry i, counted over all ranks
+  // expert id of entry i, counted over all ranks (the table is walked at fixed places: one load of it serves all
+  // keys of a lane, where a loop of W trips made each key wait for it W times, 5 us)
+  [[maybe_unused]] auto key_at = [&](int i) {
     const int* from = src.indices[0];
     int first = 0;
-    for (int r = 1; r < W; ++r) {
-      const int f = src.first[r] * K;
+#pragma unroll
+    for (int r = 1; r < RANKED; ++r) {
+      const int f = r < W ? src.first[r] * K : INT_MAX;
       from = f <= i ? src.indices[r] : from;
       first = f <= i ? f : first;
     }
     return from[i - first];
   };
-  if (RANKED && (expert_num_tokens || expert_offsets)) {
+  if (RANKED > 0 && (expert_num_tokens || expert_offsets)) {
     if (q == 0) {
       __shared__ int hist[LOCAL_MAX_EXPERTS];
       __shared__ int red[NWAVES];
@@ -3344,7 +3347,7 @@ __global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
   const int own = indices[min(lane, K - 1)];
   int row_of = -1;
   int key[SCAN_UNROLL];
-  if constexpr (RANKED) {
+  if constexpr (RANKED > 0) {
 #pragma unroll
     for (int u = 0; u < SCAN_UNROLL; ++u) key[u] = key_at(min(tid + u * BLOCK, T * K - 1));
   } else {
@@ -3353,7 +3356,7 @@ __global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
   Payload<V, NV> p;
   p.load((const V*)src.x[r] + (size_t)local_t * row_vecs, base, row_vecs);
 
-  if constexpr (RANKED) {
+  if constexpr (RANKED > 0) {
     // a key's place in (expert, entry) order; ids outside [0, E) come last
     // Two 16-bit counts travel in a word. With the stand-in (jobs: compact rows, and still no more than max_recv
     // of an expert's entries are kept) an entry needs two, everything ahead of it and what of that is in its own
@@ -4572,7 +4575,7 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
                   (out_dtype != MOE_A2A_F16 && out_dtype != MOE_A2A_BF16)))
     return MOE_A2A_EINVAL;
   const int W = s->world_size, K = s->experts_per_token, E = s->num_experts;
-  LocalSources src;
+  LocalSources src{};
   bool all16 = aligned(expert_rows, 16);
   long long tokens = 0;
   for (int r = 0; r < W; ++r) {
@@ -4621,25 +4624,23 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
   local_dispatch_kernel<V, NV, DI, DO, RANKED><<<grid, BLOCK, 0, st>>>(                                    \
       src, W, (int)tokens, K, E, g.nle, g.magic, g.row_vecs, g.chunks, compact, g.max_recv, expert_limit,  \
       entry_row, expert_num_tokens, expert_offsets, (V*)expert_rows, expert_meta)
+#define LAUNCH_R(V, NV, RANKED)                                                                            \
+  do {                                                                                                     \
+    if (!standin) LAUNCH_T(V, NV, -1, -1, RANKED);                                                         \
+    else if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_BF16, RANKED); \
+    else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_F16, RANKED); \
+    else if (in_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_BF16, RANKED);                  \
+    else LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_F16, RANKED);                                               \
+  } while (0)
 #define LAUNCH(V, NV)                                                                                      \
   do {                                                                                                     \
-    if (!standin) {                                                                                        \
-      if (ranked) LAUNCH_T(V, NV, -1, -1, true);                                                           \
-      else LAUNCH_T(V, NV, -1, -1, false);                                                                 \
-    } else if (ranked) {                                                                                   \
-      if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_BF16, true); \
-      else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_F16, true); \
-      else if (in_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_BF16, true);                  \
-      else LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_F16, true);                                               \
-    } else {                                                                                               \
-      if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_BF16, false); \
-      else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_F16, false); \
-      else if (in_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_BF16, false);                 \
-      else LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_F16, false);                                              \
-    }                                                                                                      \
+    if (!ranked) LAUNCH_R(V, NV, 0);                                                                       \
+    else if (W == 1) LAUNCH_R(V, NV, 1);                                                                   \
+    else LAUNCH_R(V, NV, LOCAL_RANKED_RANKS);                                                              \
   } while (0)
   MOE_A2A_FOR_ROW_KERNEL(g, LAUNCH);
 #undef LAUNCH
+#undef LAUNCH_R
 #undef LAUNCH_T
   return launch_status();
 }
