@@ -2273,7 +2273,7 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
 // ---------------------------------------------------------------- dense product (many rows)
 //
 // C[M, N] = A[M, K] @ B[N, K]^T for outputs that tiles of 256 columns (phased_gemm_kernel) would spread over
-// too few compute units. A workgroup of four waves owns a BM x BN tile of C (64 x 128) and walks K in steps of
+// too few compute units. A workgroup of four waves owns a BM x BN tile of C (64 or 128 x 128) and walks K in steps of
 // 64 elements. Per step the workgroup copies BM + BN rows of 128 bytes into LDS once (through registers, two LDS
 // buffers, one barrier per step), and every wave reads each operand fragment it needs once per 16-element slice
 // of the step for a whole row or column of its MFMA tiles, issued one slice ahead.
@@ -4232,7 +4232,7 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
 constexpr int MOE_A2A_NOT_DENSE = 1;  // (internal) the shape is left to the next kernel
 
 // Which tile an M x N x K product is cut into: 64 x 128 (dense_gemm_kernel) for outputs that this height
-// spreads over the 256 units once, 128 x 128 (phased_gemm_kernel, two workgroups per unit) while tiles of
+// spreads over the 256 units once, 128 x 128 (phased_gemm_kernel, two workgroups per unit, or dense) while tiles of
 // 256 x 256 would leave more than a third of the units without work, else 256 x 256 (phased, one workgroup
 // per unit), whose rate per unit is half as high again. Measured with 256 / 128 rows, us: 2048 x 4096 x 1024
 // (128 big tiles) 24.1 / 21.5; 1024 x 8192 x 2048 (128) 38.6 / 35.7; 2048 x 2880 x 360 (96) 15.4 / 11.6;
@@ -4275,7 +4275,9 @@ int allow_large_lds() {
   allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 4, 2, 3, 2, false, false>, phased_lds_bytes(4, 2, 3, 2));
   allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 4, 2, 3, 2, false, false>, phased_lds_bytes(4, 2, 3, 2));
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
+  allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
+  allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
   allow_grouped(std::integral_constant<int, MOE_A2A_BF16>{});
   allow_grouped(std::integral_constant<int, MOE_A2A_F16>{});
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
@@ -4306,18 +4308,25 @@ int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, i
   phased_gemm_kernel<DT, TM, TN, 3, 2, AHEAD, false><<<grid, 512, phased_lds_bytes(TM, TN, 3, 2), st>>>( \
       (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n, \
       nullptr, 0, 0, 0)
+  // Tiles of 128 x 128, at most one per unit: nobody is there to work while phased_gemm_kernel's waves wait for each
+  // other, and dense_gemm_kernel, which waits less, is ahead (phased / dense, us: 1586 x 2432 x 1536 20.3 / 17.8; 1024
+  // x 4096 x 4096 44.2 / 38.2; 600 x 6144 x 7168 96.5 / 69.5; with 273 tiles, 1586 x 2688 x 1536, 21.9 / 24.1).
+#define LAUNCH_D(DT, TM, TN, LDS)                                                                \
+  dense_gemm_kernel<DT, 2, 2, TM, TN, false><<<grid, 256, LDS, st>>>(                            \
+      (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n, \
+      nullptr, 0, 0, 0)
 #define LAUNCH_DT(DT)                                                                            \
   do {                                                                                           \
     if (tile == 256 && K * 2 % 128 != 0) LAUNCH_P(DT, 8, 4, true);                               \
     else if (tile == 256) LAUNCH_P(DT, 8, 4, false);                                             \
-    else if (tile == 128) LAUNCH_P(DT, 4, 2, false);                                             \
-    else dense_gemm_kernel<DT, 2, 2, 1, 2, false><<<grid, 256, dense_lds_bytes(64, 128), st>>>(  \
-        (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, \
-        (int)tiles_n, nullptr, 0, 0, 0);                                                         \
+    else if (tile == 128 && grid > 256) LAUNCH_P(DT, 4, 2, false);                               \
+    else if (tile == 128) LAUNCH_D(DT, 2, 2, dense_lds_bytes(128, 128));                         \
+    else LAUNCH_D(DT, 1, 2, dense_lds_bytes(64, 128));                                           \
   } while (0)
   if (dtype == MOE_A2A_BF16) LAUNCH_DT(MOE_A2A_BF16);
   else LAUNCH_DT(MOE_A2A_F16);
 #undef LAUNCH_DT
+#undef LAUNCH_D
 #undef LAUNCH_P
   return launch_status();
 }

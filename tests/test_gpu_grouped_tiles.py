@@ -70,3 +70,19 @@ def test_few_rows_whose_walks_of_K_start_apart(M, N, K):
     w = torch.randint(-1, 2, (N, K), generator=g, device=DEV).bfloat16()
     got = gemm_rs.local_product((x, w, None))
     assert torch.equal(got, (x.double() @ w.double().T).float().bfloat16())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("M,N,K", [(1586, 2432, 200), (2048, 2048, 64), (1025, 2080, 8), (2047, 2080, 136)])
+def test_one_round_of_square_tiles(M, N, K, dt):
+    """128 x 128 tiles on both sides of one per unit (247, 256, 153, 272 of them), small integers, whose sums
+    both types hold."""
+    from amd_distributed_2025_amd import gemm_rs
+
+    print(f"linear M={M} N={N} K={K} {dt}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randint(-1, 2, (M, K), generator=g, device=DEV).to(dt)
+    w = torch.randint(-1, 2, (N, K), generator=g, device=DEV).to(dt)
+    b = torch.randint(-9, 10, (N,), generator=g, device=DEV).to(dt)
+    got = gemm_rs.local_product((x, w, b))
+    assert torch.equal(got.double(), x.double() @ w.double().T + b.double())
