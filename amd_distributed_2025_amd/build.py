@@ -22,6 +22,7 @@ from pathlib import Path
 PKG_DIR = Path(__file__).resolve().parent
 REPO_DIR = PKG_DIR.parent
 SOURCE = PKG_DIR / "csrc" / "moe_a2a.hip"
+HEADERS = [PKG_DIR / "csrc" / "tile_rules.h", REPO_DIR / "include" / "moe_a2a.h"]
 LIBRARY = PKG_DIR / "libmoe_a2a.so"
 EXT_SOURCE = PKG_DIR / "csrc" / "moe_a2a_torch.cpp"
 EXT_DIR = PKG_DIR / "_ext"
@@ -59,7 +60,8 @@ def source_id() -> str:
     import hashlib
 
     h = hashlib.sha256(SOURCE.read_bytes())
-    h.update((REPO_DIR / "include" / "moe_a2a.h").read_bytes())
+    for header in HEADERS:
+        h.update(header.read_bytes())
     return h.hexdigest()[:16]
 
 

@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "moe_a2a.h"
+#include "tile_rules.h"
 
 // Device memory of moe_a2a_dispatch_recv_static: the send-back plan of one call, held by the
 // library so that the caller brings no buffer for it. Every GPU the library runs on has its own
@@ -2019,7 +2020,6 @@ __global__ __launch_bounds__(64 * GW, GW > 4 || D > 3 ? 1 : TJ == 1 ? 4 : TJ == 
         (void*)(weights + ((size_t)le * N + nw) * row_vecs), 0, 32 * row_bytes, BUFFER_RAW_32BIT);
     const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(expert_x + (row0 + t0) * row_vecs), 0, min(live, TOK) * row_bytes, BUFFER_RAW_32BIT);
-    constexpr int OUT_OF_RANGE = 0x40000000;
     int woff[4], wslot[4], xoff[XL], wpast[2];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -2175,7 +2175,6 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
       (void*)(Wt + (size_t)n0 * row_vecs), 0, 32 * row_bytes, BUFFER_RAW_32BIT);
   const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(X + (size_t)t0 * row_vecs), 0, min(live, TOK) * row_bytes, BUFFER_RAW_32BIT);
-  constexpr int OUT_OF_RANGE = 0x40000000;
   // load i of a lane: row sub + 8 * i, the vector that belongs in physical slot `slot` of that row
   const int sub = lane >> 3, slot = lane & 7;
   auto vec_of = [&](int row) { return slot ^ ((row >> 1) & 7); };
@@ -2410,7 +2409,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void dense_gemm_kernel(
       (void*)a_tile, 0, min(BM, rows_left) * row_bytes, BUFFER_RAW_32BIT);
   const __amdgpu_buffer_rsrc_t bbuf = __builtin_amdgcn_make_buffer_rsrc(
       (void*)b_tile, 0, min(BN, N - n0) * row_bytes, BUFFER_RAW_32BIT);
-  constexpr int OUT_OF_RANGE = 0x40000000;
   // copy i of a thread: LDS place p = tid + i * NT, that is row p / 8 (rows NT / 8 apart, which
   // leaves bits 1..3 of the row number alone) and the vector that belongs in physical slot p % 8
   const int crow = tid >> 3, cvec = (tid & 7) ^ ((crow >> 1) & 7);
@@ -2807,7 +2805,6 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   // so do the vectors past the end of a row in the last step and everything past the last step.
   const b128 abuf = buffer_words(A + row_at * row_vecs, min(BM, rows_left) * row_bytes);
   const b128 bbuf = buffer_words(B + b_at * row_vecs, min(BN, N - n0) * row_bytes);
-  constexpr int OUT_OF_RANGE = 0x40000000;
   const int sub = lane >> 3;
   auto vec_of = [&](int row) { return (lane & 7) ^ ((row >> 1) & 7); };
   auto a_row = [&](int i) { return (i * 8 + wave) * 8 + sub; };
@@ -4161,7 +4158,7 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;  // whole wave tiles of columns, whole 16-byte vectors
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
   // per-lane byte offsets inside a block of tokens and inside a wave's 32 weight rows are 32-bit
-  if ((long long)K * 2 * 128 >= (1 << 30) || max_rows > INT_MAX / 2) return MOE_A2A_EINVAL;
+  if (!tile_rows_in_range(128, K) || max_rows > INT_MAX / 2) return MOE_A2A_EINVAL;
   // Blocks of 32 rows on workgroups of 64 columns where they do better than 64 x 128. (1) Up to eight rows per
   // group: twice as many workgroups share the stream of weights out more evenly. (2) Too few workgroups to keep
   // that stream in flight, at most two per unit: each then looks four steps ahead. They are counted as uniform
@@ -4297,7 +4294,7 @@ int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, i
   if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
   if (!all_aligned(16, a, b, c) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
-  if ((long long)K * 2 * 256 >= (1 << 30)) return MOE_A2A_NOT_DENSE;  // 32-bit byte offsets inside a tile's rows
+  if (!tile_rows_in_range(256, K)) return MOE_A2A_NOT_DENSE;  // 32-bit byte offsets inside a tile's rows
   const int tile = dense_tile_rows(M, N);
   const int BM = tile, BN = tile == 64 ? 128 : tile;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + BN - 1) / BN;
@@ -4334,35 +4331,6 @@ int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, i
 #ifndef MOE_A2A_GROUPED_DENSE_MIN_ROWS
 #define MOE_A2A_GROUPED_DENSE_MIN_ROWS 56  // rows per group (from the caller's row count) from which tiles are used
 #endif
-// How a grouped product with `rows` rows in an average group is cut: the height of its tiles in bands of 32
-// rows (10, 8, 6: phased_gemm_kernel, 256 columns; 2: dense_gemm_kernel, 64 x 128). A tile costs what a compute
-// unit has to fetch for it, (rows + columns) x 128 bytes per step of K: that, and not the matrix cores, bounds
-// these kernels (measured on 32 groups of 256 rows, 137 GFLOP: 163 us, 145 without the MFMAs, 119 without the
-// loads; a unit fetches about 49 KB a microsecond). Tiles run in rounds over the units. A group is taken to have
-// one standard deviation of uniform routing more rows than the average: it decides how many tiles most groups
-// need. 320 rows leave room for two buffers of each operand only and get 15 % on top.
-// Measured, us (rows: 320, 256, 192, 64 x 128): 32 groups x 256 rows, N 2048, K 4096: 156 188 171 -; N 4096, K
-// 2048: 164 173 183 -; 512 rows: 266 276 259 -; 128 rows: 133 111 108 -; 16 x 1024 rows, N 4096, K 2048: 261 254
-// 260 -; 8 x 200, N 7168, K 2048: 73 62 88 -; 16 x 150, 2880 x 2880: 87 73 71 136; 8 x 64, N 2048, K 7168: 168 117
-// 112 75; 4 x 300, N 2048, K 4096: 97 64 58 43; 4 x 1000, N 512, K 7168: 169 119 104 70.
-int grouped_tile_bands(long long rows, int groups, int N) {
-  constexpr long long UNITS = 256;
-  const long long most = std::max<long long>(1, rows + (long long)std::sqrt((double)rows));
-  int best_bands = 0;
-  double best = 0;
-  for (const int bands : {8, 6, 10, 2}) {
-    const long long high = bands * 32, wide = bands == 2 ? 128 : 256, n = (most + high - 1) / high;
-    const long long height = std::min(high, ((most + n - 1) / n + 31) / 32 * 32);
-    const long long rounds = (n * groups * ((N + wide - 1) / wide) + UNITS - 1) / UNITS;
-    const double cost = (double)rounds * (height + wide) * (bands == 10 ? 1.15 : 1.0);
-    if (!best_bands || cost < best) {
-      best = cost;
-      best_bands = bands;
-    }
-  }
-  return best_bands;
-}
-
 // The grouped product when groups have hundreds of rows: the weights are then read for enough
 // rows that the matrix cores, not the stream of weights, bound the work, and the dense kernel's
 // tiles (each weight row read once per 64 to 320 rows, operands shared by the workgroup's waves through
@@ -4374,8 +4342,9 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
   if (!rows_of_group || rows_hint < (long long)MOE_A2A_GROUPED_DENSE_MIN_ROWS * groups) return MOE_A2A_NOT_DENSE;
-  if ((long long)K * 2 * 256 >= (1 << 30) || max_rows > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
-  const int bands = grouped_tile_bands(rows_hint / groups, groups, N);
+  if (max_rows > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
+  const int bands = grouped_tile_bands(rows_hint / groups, groups, N, K);
+  if (!bands) return MOE_A2A_NOT_DENSE;
   const int BM = bands * 32, BN = bands == 2 ? 128 : 256;
   const long long tiles_n = (N + BN - 1) / BN;
   // every group can end in a partly filled row tile; the kernel strides over what the hint misses
@@ -4417,7 +4386,7 @@ int launch_skinny_gemm(const void* x, const void* w, const void* bias, void* y, 
   if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
-  if (M > 64 || (long long)K * 2 * 128 >= (1 << 30)) return MOE_A2A_NOT_DENSE;
+  if (M > 64 || !tile_rows_in_range(128, K)) return MOE_A2A_NOT_DENSE;
   const int wide_tiles = (N + GEMM_COLS - 1) / GEMM_COLS;
   const int steps = (K + GEMM_KSTEP - 1) / GEMM_KSTEP;
   if (wide_tiles >= MOE_A2A_SKINNY_MAX_TILES || steps < 2 * NWAVES) return MOE_A2A_NOT_DENSE;
