@@ -32,20 +32,14 @@ def _pointers(tensors):
     return (C.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
 
 
-def _ref(shape):
-    """`C.byref(shape)`, made once per shape."""
-    try:
-        return shape.ref
-    except AttributeError:
-        shape.ref = C.byref(shape)
-        return shape.ref
-
-
 def _rows(buf: torch.Tensor, meta: torch.Tensor, hidden_dim: int) -> int:
     return min(buf.numel() // max(hidden_dim, 1), meta.numel() // META_DIM)
 
 
 class CtypesBinding:
+    """(A `Shape` is passed as it is: ctypes takes its address for the call. A `byref` object kept on the shape would
+    refer back to it, and such cycles are never collected.)"""
+
     name = "ctypes"
 
     def __init__(self):
@@ -61,18 +55,18 @@ class CtypesBinding:
         return _lib.load().moe_a2a_version().decode()
 
     def dispatch_send(self, shape, x, indices, num_tokens, send_buf, send_meta, send_counts, send_slot, stream):
-        self._call("moe_a2a_dispatch_send", _ref(shape), _ptr(x), _ptr(indices), num_tokens, _ptr(send_buf),
+        self._call("moe_a2a_dispatch_send", shape, _ptr(x), _ptr(indices), num_tokens, _ptr(send_buf),
                   _ptr(send_meta), _ptr(send_counts), _ptr(send_slot), stream)
 
     def plan_send(self, shape, indices, num_tokens, rank_counts, rank_offsets, expert_counts, dst_slot,
                   src_entry, stream):
-        self._call("moe_a2a_plan_send", _ref(shape), _ptr(indices), num_tokens, _ptr(rank_counts),
+        self._call("moe_a2a_plan_send", shape, _ptr(indices), num_tokens, _ptr(rank_counts),
                   _ptr(rank_offsets), _ptr(expert_counts), _ptr(dst_slot), _ptr(src_entry), stream)
 
     def dispatch_recv(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens, expert_x,
                       expert_meta, send_back_plan, stream, row_position=None):
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
-        args = (_ref(shape), _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
+        args = (shape, _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
                 min(rows_hint, capacity), capacity, _ptr(expert_num_tokens), _ptr(expert_x), _ptr(expert_meta),
                 _ptr(send_back_plan))
         if row_position is None:
@@ -85,14 +79,14 @@ class CtypesBinding:
     def combine_send(self, shape, expert_y, expert_meta, expert_num_tokens, rows_hint, send_buf, send_meta,
                      send_counts, send_back_plan, stream):
         capacity = _rows(send_buf, send_meta, shape.hidden_dim)
-        self._call("moe_a2a_combine_send", _ref(shape), _ptr(expert_y), _ptr(expert_meta),
+        self._call("moe_a2a_combine_send", shape, _ptr(expert_y), _ptr(expert_meta),
                   _ptr(expert_num_tokens), min(rows_hint, capacity), capacity, _ptr(send_buf), _ptr(send_meta),
                   _ptr(send_counts), _ptr(send_back_plan), stream)
 
     def combine_recv(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, weights, num_tokens, out_tokens,
                      accumulate, stream, entry_row=None):
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
-        args = (_ref(shape), _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
+        args = (shape, _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
                 min(rows_hint, capacity), capacity, _ptr(weights), num_tokens, _ptr(out_tokens),
                 int(bool(accumulate)), _DT[out_tokens.dtype])
         if entry_row is None:
@@ -103,11 +97,11 @@ class CtypesBinding:
             self._call("moe_a2a_combine_recv_long", *args, _ptr(entry_row), stream)
 
     def expert_scale(self, shape, expert_x, expert_num_tokens, rows_hint, expert_y, stream):
-        self._call("moe_a2a_expert_scale", _ref(shape), _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
+        self._call("moe_a2a_expert_scale", shape, _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
                   _DT[expert_x.dtype], _DT[expert_y.dtype], _ptr(expert_y), stream)
 
     def expert_gemm(self, shape, expert_x, expert_num_tokens, rows_hint, weights, bias, expert_y, stream):
-        self._call("moe_a2a_expert_gemm", _ref(shape), _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
+        self._call("moe_a2a_expert_gemm", shape, _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
                   _ptr(weights), _ptr(bias), weights.shape[2], weights.shape[1], _DT[expert_x.dtype],
                   _ptr(expert_y), stream)
 
@@ -128,25 +122,25 @@ class CtypesBinding:
     def dispatch_recv_compact(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens,
                               expert_offsets, expert_x, expert_meta, send_back_plan, stream):
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
-        self._call("moe_a2a_dispatch_recv_compact", _ref(shape), _ptr(recv_buf), _ptr(recv_meta),
+        self._call("moe_a2a_dispatch_recv_compact", shape, _ptr(recv_buf), _ptr(recv_meta),
                   _ptr(recv_counts), min(rows_hint, capacity), capacity, _ptr(expert_num_tokens),
                   _ptr(expert_offsets), _ptr(expert_x), _ptr(expert_meta),
                   _rows(expert_x, expert_meta, shape.hidden_dim), _ptr(send_back_plan), stream)
 
     def expert_scale_compact(self, shape, expert_x, expert_num_tokens, rows_hint, expert_y, stream):
-        self._call("moe_a2a_expert_scale_compact", _ref(shape), _ptr(expert_x), _ptr(expert_num_tokens),
+        self._call("moe_a2a_expert_scale_compact", shape, _ptr(expert_x), _ptr(expert_num_tokens),
                   rows_hint, min(expert_x.shape[0], expert_y.shape[0]), _DT[expert_x.dtype], _DT[expert_y.dtype],
                   _ptr(expert_y), stream)
 
     def expert_gemm_compact(self, shape, expert_x, expert_num_tokens, rows_hint, weights, bias, expert_y, stream):
-        self._call("moe_a2a_expert_gemm_compact", _ref(shape), _ptr(expert_x), _ptr(expert_num_tokens),
+        self._call("moe_a2a_expert_gemm_compact", shape, _ptr(expert_x), _ptr(expert_num_tokens),
                   rows_hint, min(expert_x.shape[0], expert_y.shape[0]), _ptr(weights), _ptr(bias),
                   weights.shape[2], weights.shape[1], _DT[expert_x.dtype], _ptr(expert_y), stream)
 
     def combine_send_compact(self, shape, expert_y, expert_meta, expert_num_tokens, rows_hint, send_buf,
                              send_meta, send_counts, send_back_plan, stream):
         capacity = _rows(send_buf, send_meta, shape.hidden_dim)
-        self._call("moe_a2a_combine_send_compact", _ref(shape), _ptr(expert_y), _ptr(expert_meta),
+        self._call("moe_a2a_combine_send_compact", shape, _ptr(expert_y), _ptr(expert_meta),
                   _ptr(expert_num_tokens), min(rows_hint, capacity),
                   _rows(expert_y, expert_meta, shape.hidden_dim), capacity, _ptr(send_buf), _ptr(send_meta),
                   _ptr(send_counts), _ptr(send_back_plan), stream)
@@ -164,14 +158,14 @@ class CtypesBinding:
                        standin, stream):
         tokens = (C.c_int32 * len(xs))(*[i.shape[0] for i in indices])
         din, dout = (_DT[xs[0].dtype], _DT[rows.dtype]) if standin else (-1, -1)
-        self._call("moe_a2a_local_dispatch", _ref(shape), _pointers(xs), _pointers(indices), tokens,
+        self._call("moe_a2a_local_dispatch", shape, _pointers(xs), _pointers(indices), tokens,
                    rows.shape[0] if compact else 0, din, dout, _ptr(entry_row), _ptr(expert_num_tokens),
                    _ptr(expert_offsets), rows.data_ptr(), _ptr(meta), stream)
 
     def local_combine(self, shape, rows, entry_row, weights, tokens, outs, only_rank, accumulate, stream):
         """`weights` and `outs` may hold None for ranks other than `only_rank`; `tokens` are all ranks'."""
         ranks = len(tokens)
-        self._call("moe_a2a_local_combine", _ref(shape), rows.data_ptr(), entry_row.data_ptr(),
+        self._call("moe_a2a_local_combine", shape, rows.data_ptr(), entry_row.data_ptr(),
                    (C.c_void_p * ranks)(*map(_ptr, weights)), (C.c_int32 * ranks)(*tokens),
                    (C.c_void_p * ranks)(*map(_ptr, outs)), only_rank, int(bool(accumulate)), _DT[rows.dtype], stream)
 

@@ -231,3 +231,34 @@ def test_unknown_binding_is_refused():
         _binding.get("cffi")
     assert _binding.get("ctypes").version().startswith("moe_a2a")
     assert _binding.get("ext").version() == _binding.get("ctypes").version()
+
+
+def _arguments(method, shape):
+    """None for every tensor, 1 for every number: refused before anything is launched."""
+    import inspect
+
+    names = list(inspect.signature(method).parameters)[1:]
+    numbers = {"num_tokens", "rows_hint", "stream", "only_rank"}
+    return [shape] + [1 if n in numbers else None for n in names]
+
+
+@pytest.mark.parametrize("binding", ["ctypes", "ext"])
+def test_a_shape_does_not_outlive_its_calls(binding):
+    """One is made per call of `custom_kernel`: none may be kept by the call, or by itself."""
+    import gc
+    import weakref
+
+    from amd_distributed_2025_amd import _binding
+
+    b = _binding.get(binding)
+
+    def call():
+        shape = _lib.Shape(1, 0, 8, 2, 16, 4)
+        for method in (b.dispatch_send, b.plan_send):
+            with pytest.raises((_lib.MoeA2AError, RuntimeError, TypeError)):
+                method(*_arguments(method, shape))
+        return weakref.ref(shape)
+
+    shapes = [call() for _ in range(20)]
+    gc.collect()
+    assert not any(ref() is not None for ref in shapes)
