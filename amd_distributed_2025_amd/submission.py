@@ -137,8 +137,9 @@ def _run_direct(cfg: MoEConfig, world_size: int, everyone: Sequence[RankTestData
     where = torch.empty((max(entries, 1),), dtype=torch.int32, device=device)
     c.local_dispatch(shape, xs, ids, True, where, None, None, rows, None, True, stream)
     if only is None:
-        out = torch.empty((sum(tokens), H), dtype=cfg.out_dtype, device=device)
-        ys = list(out.split(tokens))
+        # (a tensor of its own for each rank: views of one would keep all results as long as any of them; empty_like
+        # takes 1.2 us of the host, empty with sizes and a device 1.8)
+        ys = [torch.empty_like(x, dtype=cfg.out_dtype) for x in xs]
         c.local_combine(shape, rows, where, weights, tokens, ys, -1, False, stream)
         return ys
     y = torch.empty((tokens[only], H), dtype=cfg.out_dtype, device=device)

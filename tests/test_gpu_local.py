@@ -126,3 +126,12 @@ def test_job_in_a_captured_graph_and_on_two_streams():
         assert all(torch.equal(a, b) for a, b in zip(other, want[1]))
         for y in captured:
             y.fill_(3.0)
+
+
+@pytest.mark.parametrize("tokens", [[16] * 4, [1, 30, 7, 2]])
+def test_results_of_a_job_share_no_storage(tokens):
+    """A caller that keeps or saves one rank's result keeps that result alone."""
+    cfg = config(16, 2, 264, max(tokens))
+    ys = custom_kernel_job([(cfg, rank_data(cfg, t, r), r, 4) for r, t in enumerate(tokens)])
+    assert len({y.untyped_storage().data_ptr() for y in ys}) == 4
+    assert all(y.untyped_storage().nbytes() == y.numel() * y.element_size() for y in ys)
