@@ -4275,6 +4275,8 @@ int allow_large_lds() {
     allow((const void*)phased_gemm_kernel<DT, 10, 4, 2, 2, false, true>, phased_lds_bytes(10, 4, 2, 2));
     allow((const void*)phased_gemm_kernel<DT, 8, 4, 2, 3, false, true>, phased_lds_bytes(8, 4, 2, 3));
     allow((const void*)phased_gemm_kernel<DT, 6, 4, 2, 3, false, true>, phased_lds_bytes(6, 4, 2, 3));
+    allow((const void*)dense_gemm_kernel<DT, 2, 2, 2, 2, true>, dense_lds_bytes(128, 128));
+    allow((const void*)dense_gemm_kernel<DT, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
   };
   allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 2, false, false>, phased_lds_bytes(8, 4, 3, 2));
   allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 2, false, false>, phased_lds_bytes(8, 4, 3, 2));
@@ -4288,8 +4290,6 @@ int allow_large_lds() {
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
   allow_grouped(std::integral_constant<int, MOE_A2A_BF16>{});
   allow_grouped(std::integral_constant<int, MOE_A2A_F16>{});
-  allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8>, skinny_lds_bytes(2, 8));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8>, skinny_lds_bytes(2, 8));
   allow((const void*)local_plan_kernel, local_plan_lds_bytes(LOCAL_MAX_EXPERTS));
@@ -4354,9 +4354,9 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
   if (!rows_of_group || rows_hint < (long long)MOE_A2A_GROUPED_DENSE_MIN_ROWS * groups) return MOE_A2A_NOT_DENSE;
   if (max_rows > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
-  const int bands = grouped_tile_bands(rows_hint / groups, groups, N, K);
+  const int bands = grouped_tile_bands(rows_hint, groups, N, K);
   if (!bands) return MOE_A2A_NOT_DENSE;
-  const int BM = bands * 32, BN = bands == 2 ? 128 : 256;
+  const int BM = bands * 32, BN = bands <= 4 ? 128 : 256;
   const long long tiles_n = (N + BN - 1) / BN;
   // every group can end in a partly filled row tile; the kernel strides over what the hint misses
   const long long pairs = (rows_hint / BM + groups) * tiles_n;
@@ -4365,17 +4365,17 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   if (const int rc = allow_large_lds()) return rc;
   auto launch = [&](auto dtype_const) {
     constexpr int DT = decltype(dtype_const)::value;
-    auto phased = [&](auto kernel, size_t lds_bytes) {
-      kernel<<<grid, 512, lds_bytes, st>>>((const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, 0, N, K,
-                                           0, (int)tiles_n, rows_of_group, groups, (int)max_rows, compact);
+    auto start = [&](auto kernel, int lanes, size_t lds_bytes) {
+      kernel<<<grid, lanes, lds_bytes, st>>>((const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, 0, N, K,
+                                             0, (int)tiles_n, rows_of_group, groups, (int)max_rows, compact);
     };
+    auto phased = [&](auto kernel, size_t lds_bytes) { start(kernel, 512, lds_bytes); };
+    auto dense = [&](auto kernel, size_t lds_bytes) { start(kernel, 256, lds_bytes); };
     if (bands == 10) phased(phased_gemm_kernel<DT, 10, 4, 2, 2, false, true>, phased_lds_bytes(10, 4, 2, 2));
     else if (bands == 8) phased(phased_gemm_kernel<DT, 8, 4, 2, 3, false, true>, phased_lds_bytes(8, 4, 2, 3));
     else if (bands == 6) phased(phased_gemm_kernel<DT, 6, 4, 2, 3, false, true>, phased_lds_bytes(6, 4, 2, 3));
-    else
-      dense_gemm_kernel<DT, 2, 2, 1, 2, true><<<grid, 256, dense_lds_bytes(64, 128), st>>>(
-          (const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, 0, N, K, 0, (int)tiles_n, rows_of_group,
-          groups, (int)max_rows, compact);
+    else if (bands == 4) dense(dense_gemm_kernel<DT, 2, 2, 2, 2, true>, dense_lds_bytes(128, 128));
+    else dense(dense_gemm_kernel<DT, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
   };
   if (dtype == MOE_A2A_BF16) launch(std::integral_constant<int, MOE_A2A_BF16>{});
   else launch(std::integral_constant<int, MOE_A2A_F16>{});

@@ -12,29 +12,64 @@ constexpr int OUT_OF_RANGE = 0x40000000;
 
 bool tile_rows_in_range(long long rows, long long K) { return rows * K * 2 < OUT_OF_RANGE; }
 
-// How a grouped product with `rows` rows in an average group is cut: the height of its tiles in bands of 32
-// rows (10, 8, 6: phased_gemm_kernel, 256 columns; 2: dense_gemm_kernel, 64 x 128), 0 where rows of K are too long
-// for any. A tile costs what a compute
-// unit has to fetch for it, (rows + columns) x 128 bytes per step of K: that, and not the matrix cores, bounds
-// these kernels (measured on 32 groups of 256 rows, 137 GFLOP: 163 us, 145 without the MFMAs, 119 without the
-// loads; a unit fetches about 49 KB a microsecond). Tiles run in rounds over the units. A group is taken to have
-// one standard deviation of uniform routing more rows than the average: it decides how many tiles most groups
-// need. 320 rows leave room for two buffers of each operand only and get 15 % on top.
-// Measured, us (rows: 320, 256, 192, 64 x 128): 32 groups x 256 rows, N 2048, K 4096: 156 188 171 -; N 4096, K
-// 2048: 164 173 183 -; 512 rows: 266 276 259 -; 128 rows: 133 111 108 -; 16 x 1024 rows, N 4096, K 2048: 261 254
-// 260 -; 8 x 200, N 7168, K 2048: 73 62 88 -; 16 x 150, 2880 x 2880: 87 73 71 136; 8 x 64, N 2048, K 7168: 168 117
-// 112 75; 4 x 300, N 2048, K 4096: 97 64 58 43; 4 x 1000, N 512, K 7168: 169 119 104 70.
-int grouped_tile_bands(long long rows, int groups, int N, int K) {
-  constexpr long long UNITS = 256;
-  const long long most = std::max<long long>(1, rows + (long long)std::sqrt((double)rows));
+// How a grouped product is cut: the height of its tiles in bands of 32 rows (10, 8, 6: phased_gemm_kernel, 256
+// columns; 4, 2: dense_gemm_kernel, 128 columns), 0 where rows of K are too long for any. `rows_hint` rows over all
+// groups are taken to be spread as uniform routing spreads them: a group's number is normal around the average.
+//
+// A tile costs per step of K what its unit has to fetch, in rows of 128 bytes (a unit fetches one in 2.6 ns, the
+// matrix cores are faster in every case that was measured). A step takes no less than HBM needs for the weights,
+// which every round of tiles over the units asks for anew: 256 x 256 columns in the time of 490 rows, two
+// workgroups of 128 columns on every unit in that of 530. What else was measured and stands in the factors: two
+// workgroups on a unit fetch 1.3 times as slowly as one; the two buffers of 320 rows cost 1.38; the first loads and
+// the results of a tile take as long as six steps, of two with two workgroups on a unit, which overlap them.
+// Factors and floors are those that lose least, and their neighbours lose hardly more: 697 shapes of 2 to 128 groups,
+// 50 to 1024 rows, N and K of 512 to 8192, all five tiles timed on each. The choice is 1.5 % behind the best of them
+// and the streaming kernel on average, more than a tenth on 31. (Counting rounds x (height + columns) alone, without
+// the tile of 128 x 128, it was 6.4 % behind, and more than a tenth on 155.) Among them, us with 320 / 256 / 192 / 128 /
+// 64 rows: 32 groups of 63 rows, 7168 x 7168 770 / 613 / 604 / 576 / 708; 8 of 64, 4096 x 4096 104 / 78 / 76 / 52 / 65;
+// 32 of 100, 2048 x 4096 126 / 105 / 104 / 119 / 146; 32 of 256, 4096 x 2048 161 / 176 / 182 / 203 / 240.
+struct GroupTiles {
+  double each;    // tiles of a group, on average
+  double surely;  // as many as nearly every group has
+  double height;  // rows of a tall one
+};
+
+GroupTiles tiles_of_groups(double rows, int groups, int high) {
+  if (rows > 16.0 * high) return {rows / high + 0.5, rows / high, (double)high};
+  const double deviation = std::max(1e-3, std::sqrt(rows * (1.0 - 1.0 / groups)));
+  GroupTiles t = {1.0, 1.0, 0.0};
+  for (int k = 1;; ++k) {
+    const double need_more = 0.5 * std::erfc(((double)k * high + 0.5 - rows) / (deviation * std::sqrt(2.0)));
+    if (need_more > 0.95) t.surely = k + 1;
+    if (need_more < 1e-3) break;
+    t.each += need_more;
+  }
+  t.height = std::min((double)high, (rows + deviation) / t.surely);
+  return t;
+}
+
+int grouped_tile_bands(long long rows_hint, int groups, int N, int K) {
+  constexpr double UNITS = 256, FEW = 0.01;  // (of a round: tiles that only some draws of the rows have)
+  const double rows = (double)rows_hint / groups, steps = (K + 63) / 64;
   int best_bands = 0;
   double best = 0;
-  for (const int bands : {8, 6, 10, 2}) {
-    const long long high = bands * 32, wide = bands == 2 ? 128 : 256, n = (most + high - 1) / high;
-    if (!tile_rows_in_range(std::max<long long>(high, 256), K)) continue;
-    const long long height = std::min(high, ((most + n - 1) / n + 31) / 32 * 32);
-    const long long rounds = (n * groups * ((N + wide - 1) / wide) + UNITS - 1) / UNITS;
-    const double cost = (double)rounds * (height + wide) * (bands == 10 ? 1.15 : 1.0);
+  for (const int bands : {6, 8, 2, 4, 10}) {  // (where two cost the same the first is faster, by up to 3 and 13 %)
+    const int high = bands * 32, wide = bands <= 4 ? 128 : 256;
+    if (!tile_rows_in_range(std::max(high, 256), K)) continue;
+    const GroupTiles t = tiles_of_groups(rows, groups, high);
+    const double one_each = (double)groups * ((N + wide - 1) / wide) / UNITS;
+    const double rounds = std::max(t.surely * one_each, t.each * one_each - FEW);
+    double cost;
+    if (wide == 256) {  // one workgroup per unit
+      const double fetch = (t.height + 256) * (bands == 10 ? 1.38 : 1.0), weights = 490 / t.each;
+      const double whole = std::floor(rounds), rest = rounds - whole;
+      cost = whole * std::max(fetch, weights) + (rest > 0 ? std::max(fetch, rest * weights) : 0);
+      cost *= 1 + 6 / steps;
+    } else {  // two per unit, and one in the last round if they are odd
+      const double each = std::ceil(rounds), pairs = std::floor(each / 2);
+      cost = pairs * std::max(1.3 * 2 * (t.height + 128), 530 / t.each) + (each - 2 * pairs) * (t.height + 128);
+      cost *= 1 + 2 / steps;
+    }
     if (!best_bands || cost < best) {
       best = cost;
       best_bands = bands;

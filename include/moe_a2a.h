@@ -334,8 +334,8 @@ int moe_a2a_expert_scale(const moe_a2a_shape* shape, const void* expert_x,
  * follows the rows, not the experts. rows_hint (the rows the caller expects
  * over all experts) picks the kernel and sizes the launch, and changes no bit
  * of the result: from 56 rows per expert on average, output tiles of 192, 256 or
- * 320 rows x 256 columns (64 x 128 when those would be too few for the GPU) of
- * the kernels behind moe_a2a_linear, numbered over the experts; below, a kernel
+ * 320 rows x 256 columns or of 64 or 128 rows x 128 columns (whichever keeps the
+ * GPU busiest) of the kernels behind moe_a2a_linear, numbered over the experts; below, a kernel
  * built around streaming every weight once, in blocks of 32, 64 or 128 tokens
  * and workgroups 64 to 256 columns wide. The first call on a GPU
  * sets kernel attributes (tiles can use more LDS than a kernel gets by default):

@@ -1,6 +1,6 @@
 """The tiles of the grouped product (`moe_a2a_expert_gemm` and its compact form): blocks of 32, 64 or 128 rows that
-stream the weights, 64 x 128 and 192, 256 or 320 rows x 256 columns, which of them from the caller's row count.
-The row count must change no bit of the result, and K may start anywhere in a group's walk (rows a multiple of
+stream the weights, 64 x 128, 128 x 128 and 192, 256 or 320 rows x 256 columns, which of them from the caller's row
+count. The row count must change no bit of the result, and K may start anywhere in a group's walk (rows a multiple of
 4 KB apart do)."""
 import pytest
 import torch
@@ -9,9 +9,10 @@ from amd_distributed_2025_amd import HIPAllToAll, MoEConfig
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-# rows per group -> tile, by groups (see grouped_tile_bands): N = 7168 is 28 tiles of 256 columns
-ROWS_FOR_TILE = {3: {20: "stream 32, four steps ahead", 50: "stream 128", 56: "64 x 128", 150: "256", 200: "192"},
-                 5: {8: "stream 32, two steps ahead", 20: "stream 64", 300: "320"}}
+# rows per group -> kernel and rows of a tile, by groups, at N = 7168 and K of 2048 or 2112 (csrc/tile_rules.h;
+# test_tile_rules.py holds the tiles to that)
+ROWS_FOR_TILE = {3: {20: "stream 32, four steps ahead", 50: "stream 128", 60: 64, 100: 128, 150: 192, 600: 256, 800: 320},
+                 5: {8: "stream 32, two steps ahead", 20: "stream 64", 100: 192, 230: 256, 300: 320}}
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
