@@ -2151,7 +2151,7 @@ __global__ __launch_bounds__(64 * GW, GW > 4 || D > 3 ? 1 : TJ == 1 ? 4 : TJ == 
 // partial sums in registers. At the end the partial sums meet in LDS and are added in a fixed
 // order (wave 0 + 1 + 2 + ...), so results do not depend on scheduling.
 
-template <int DT, int TJ, int KW>
+template <int DT, int TJ, int KW, bool APART>
 __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
     const b128* __restrict__ X, const b128* __restrict__ Wt, const uint16_t* __restrict__ bias,
     uint16_t* __restrict__ Y, int M, int N, int K, int col_units) {
@@ -2165,11 +2165,11 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
   const int tail_vecs = row_vecs - (steps - 1) * 8;
   const int rb = blockIdx.x / col_units, cu = blockIdx.x - rb * col_units;
   const int t0 = rb * TOK, n0 = cu * 32, live = M - t0;
-  // Where rows lie a multiple of 4 KB apart (see first_kstep) workgroups start apart too, by whole turns of the
-  // waves, so that a wave keeps its steps: 8 x 8192 x 8192 34.1 -> 25.6 us, 1 x 4096 x 4096 12.4 -> 9.5, 64 x 8192 x 8192
+  // APART: where rows lie a multiple of 4 KB apart (see first_kstep) workgroups start apart too, by whole turns of
+  // the waves, so that a wave keeps its steps (elsewhere going round would cost 0.8 %: 64 x 7168 x 2304 11.29 us, 11.20 without): 8 x 8192 x 8192 34.1 -> 25.6 us, 1 x 4096 x 4096 12.4 -> 9.5, 64 x 8192 x 8192
   // 41 -> 38, 16 x 16384 x 2048 16.0 -> 14.6.
   static_assert(32 % KW == 0, "whole turns in the steps of 2048 inputs");
-  const int first_step = K % 2048 ? 0 : (int)((long long)cu * (steps / KW) / col_units) * KW;
+  const int first_step = APART ? (int)((long long)cu * (steps / KW) / col_units) * KW : 0;
 
   const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(Wt + (size_t)n0 * row_vecs), 0, 32 * row_bytes, BUFFER_RAW_32BIT);
@@ -2185,7 +2185,7 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
   auto load = [&](int set, int step) {
     const int at = min(step, steps - 1);  // past the end: the last step again, unused
     const bool last = at == steps - 1;
-    const int k = at + first_step, soff = (k >= steps ? k - steps : k) * (GEMM_KSTEP * 2);
+    const int k = at + first_step, soff = (APART && k >= steps ? k - steps : k) * (GEMM_KSTEP * 2);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = sub + 8 * i, vec = vec_of(row);
@@ -4290,8 +4290,10 @@ int allow_large_lds() {
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
   allow_grouped(std::integral_constant<int, MOE_A2A_BF16>{});
   allow_grouped(std::integral_constant<int, MOE_A2A_F16>{});
-  allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8>, skinny_lds_bytes(2, 8));
-  allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8>, skinny_lds_bytes(2, 8));
+  allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8, true>, skinny_lds_bytes(2, 8));
+  allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8, false>, skinny_lds_bytes(2, 8));
+  allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8, true>, skinny_lds_bytes(2, 8));
+  allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8, false>, skinny_lds_bytes(2, 8));
   allow((const void*)local_plan_kernel, local_plan_lds_bytes(LOCAL_MAX_EXPERTS));
   if (!ok) return MOE_A2A_ELAUNCH;
   allowed[gpu] = true;
@@ -4407,9 +4409,14 @@ int launch_skinny_gemm(const void* x, const void* w, const void* bias, void* y, 
   const int waves = MOE_A2A_SKINNY_WAVES ? MOE_A2A_SKINNY_WAVES : steps >= 24 ? 8 : 4;
   const int tj = M <= 32 ? 1 : 2;
   if (const int rc = allow_large_lds()) return rc;
-#define LAUNCH_K(DT, TJ, KW)                                                              \
-  skinny_gemm_kernel<DT, TJ, KW><<<grid, 64 * KW, skinny_lds_bytes(TJ, KW), st>>>(        \
+#define LAUNCH_KA(DT, TJ, KW, APART)                                                      \
+  skinny_gemm_kernel<DT, TJ, KW, APART><<<grid, 64 * KW, skinny_lds_bytes(TJ, KW), st>>>( \
       (const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, M, N, K, N / 32)
+#define LAUNCH_K(DT, TJ, KW)                               \
+  do {                                                     \
+    if (K % 2048 == 0) LAUNCH_KA(DT, TJ, KW, true);        \
+    else LAUNCH_KA(DT, TJ, KW, false);                     \
+  } while (0)
 #define LAUNCH_KW(DT)                                      \
   do {                                                     \
     if (waves == 8 && tj == 2) LAUNCH_K(DT, 2, 8);         \
@@ -4421,6 +4428,7 @@ int launch_skinny_gemm(const void* x, const void* w, const void* bias, void* y, 
   else LAUNCH_KW(MOE_A2A_F16);
 #undef LAUNCH_KW
 #undef LAUNCH_K
+#undef LAUNCH_KA
   return launch_status();
 }
 
