@@ -99,12 +99,17 @@ def test_small_integers_sum_exactly(H, dt):
                               want.astype(np.float32))
 
 
+# rows per expert (of five) -> rows of a tile, by (in_dim, out_dim); test_tile_rules.py holds the tiles to that
+TILES_OF_NARROW = {(96, 160): {56: 64, 768: 64, 3000: 128, 10000: 256}, (200, 64): {56: 64, 768: 64, 10000: 128},
+                   (128, 128): {56: 64, 768: 64, 10000: 128}}
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("in_dim,out_dim", [(96, 160), (200, 64), (128, 128)])
+@pytest.mark.parametrize("in_dim,out_dim", TILES_OF_NARROW)
 def test_bias_and_unequal_widths_on_every_kernel(in_dim, out_dim, dt):
     """[nle, out_dim, in_dim] weights with a bias, small integers (every order of the sum agrees, and
-    both roundings are exact): the streaming kernel (row count 0) and the tiles of 64 x 128 / 128 x 128
-    and 256 x 256 (row counts of 56 and 768 per expert) all give the integers of `x @ w.T + b`."""
+    both roundings are exact): the streaming kernel (row count 0) and the tiles that `TILES_OF_NARROW`
+    lists for counts of rows per expert all give the integers of `x @ w.T + b`."""
     print(f"bias in={in_dim} out={out_dim} {dt}", flush=True)
     rng = np.random.default_rng(in_dim * 7 + out_dim)
     W, nle, max_tokens = 1, 5, 300
@@ -116,7 +121,7 @@ def test_bias_and_unequal_widths_on_every_kernel(in_dim, out_dim, dt):
     ex, wt, bt = (torch.from_numpy(v).to(dt).to(DEV) for v in (x, w, b))
     num = torch.tensor(counts, dtype=torch.int32, device=DEV)
     name = dtype_name(dt)
-    for hint in (0, 56 * nle, 768 * nle):
+    for hint in [0] + [rows * nle for rows in TILES_OF_NARROW[in_dim, out_dim]]:
         out = torch.empty(nle, max_tokens, out_dim, dtype=dt, device=DEV)
         out.view(torch.int16).fill_(SENTINEL)
         got = a.expert_gemm(ex, num, wt, bias=bt, rows_hint=hint, out=out)
@@ -267,17 +272,17 @@ def test_wide_workgroups_of_every_width(H, width):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("nle,H,max_tokens,counts", [
-    # about 160 rows per expert and more: tiles of 128 x 128 (ragged last tiles in both directions, an empty
-    # expert, exact multiples of the tile, one row)
+    # ragged last tiles in both directions, an empty expert, exact multiples of the tile, few rows: the row counts
+    # below take tiles of 64, 128 and 192 rows, and of 192 and 256
     (6, 416, 400, [384, 0, 5, 400, 131, 256]),
     (5, 7168, 300, [290, 213, 0, 256, 129]),
-    # about 768 rows and more: tiles of 256 x 256
+    # several tiles per expert: of 64 and 192 rows, and of 64, 128 and 192
     (3, 320, 1100, [1100, 770, 513]),
     (2, 1024, 1030, [1025, 1024]),
 ])
 def test_tiles_for_experts_with_hundreds_of_rows(nle, H, max_tokens, counts, dt):
-    """From about 160 rows per expert (judged from the row count the caller passes) the product runs on the
-    dense kernel's tiles, found over the experts from the device-side counts. The row count only picks the
+    """From 56 rows per expert (judged from the row count the caller passes) the product runs on tiles, found
+    over the experts from the device-side counts. The row count only picks the
     kernel and sizes the launch: every value of it gives the same bits, those of the streaming kernel
     (hint 0) included, within the float32 bound, and rows past the counts stay untouched."""
     print(f"gemm tiles nle={nle} H={H} counts={counts} {dt}", flush=True)
@@ -352,9 +357,9 @@ def _random_layouts(seed, count):
 
 @pytest.mark.parametrize("nle,H,max_tokens,counts", _random_layouts(77, 14))
 def test_random_layouts_give_the_same_bits_on_every_kernel(nle, H, max_tokens, counts):
-    """Random numbers of experts, row lengths and ragged counts: the streaming kernel (row count 0), tiles of
-    64 x 128 or 128 x 128 (a row count of 56 per expert or the true one) and tiles of 256 x 256 (768 per
-    expert) give the same bits, inside the float32 bound, and leave the rows past the counts alone."""
+    """Random numbers of experts, row lengths and ragged counts: the streaming kernel (row count 0) and the
+    tiles that the true row count (56 per expert at least) and one of 768 per expert pick give the same bits,
+    inside the float32 bound, and leave the rows past the counts alone."""
     print(f"gemm random layout nle={nle} H={H} T={max_tokens} rows={sum(counts)}", flush=True)
     a, cfg = rank_object(1, nle, H, max_tokens, torch.bfloat16)
     base = random_case(a, cfg, 1, counts, seed=nle * 1000 + H, hint=0, check_experts=[0, nle - 1])

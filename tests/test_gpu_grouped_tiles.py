@@ -20,6 +20,7 @@ ROWS_FOR_TILE = {3: {20: "stream 32, four steps ahead", 50: "stream 128", 60: 64
 @pytest.mark.parametrize("groups,counts", [
     (3, [1, 193, 257]), (3, [700, 0, 31]), (3, [192, 256, 320]), (3, [64, 65, 63]),
     (5, [321, 1, 0, 33, 640]), (5, [320, 319, 289, 288, 641]),
+    (5, [704, 704, 650, 704, 704]),  # more rows than any of the row counts: workgroups take a second tile, some a third
 ])
 @pytest.mark.parametrize("K", [8, 200, 2048, 2112])  # one short step; a tail; a walk that starts apart; one that does not
 def test_every_tile_gives_the_same_bits(groups, counts, K, bias, dt):

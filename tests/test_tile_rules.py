@@ -5,6 +5,7 @@ from pathlib import Path
 
 import pytest
 
+from tests.test_gpu_expert_gemm import TILES_OF_NARROW
 from tests.test_gpu_grouped_tiles import ROWS_FOR_TILE
 
 CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
@@ -66,3 +67,14 @@ def test_the_tiles_that_the_gpu_tests_mean(rules, K):
             if isinstance(tile, int):
                 assert 32 * rules.bands(rows * groups, groups, 7168, K) == tile, (groups, rows)
     assert {t for tiles in ROWS_FOR_TILE.values() for t in tiles.values() if isinstance(t, int)} == {64, 128, 192, 256, 320}
+    for (in_dim, out_dim), tiles in TILES_OF_NARROW.items():
+        assert {rows: 32 * rules.bands(rows * 5, 5, out_dim, in_dim) for rows in tiles} == tiles
+
+
+def test_the_second_tiles_that_the_gpu_tests_mean():
+    """A launch has a workgroup for every tile of `rows_hint` rows and one more row of tiles per group: with the row
+    counts of ROWS_FOR_TILE for five groups, [704, 704, 650, 704, 704] is more than that for every tall tile."""
+    for rows, tile in ROWS_FOR_TILE[5].items():
+        if isinstance(tile, int):
+            workgroups = rows * 5 // tile + 5
+            assert 5 * -(-650 // tile) > workgroups, (rows, tile)
