@@ -255,7 +255,11 @@ class HIPAllToAll:
         layer), `weights` [nle, out_dim, in_dim] with the input index contiguous, `bias` [nle,
         out_dim] or None, all of one 16-bit type; returns [nle, max_recv, out_dim] (a workspace
         buffer per out_dim unless `out` is given; never the input's memory). Limits of the
-        kernels: out_dim % 32 == 0 and in_dim % 8 == 0."""
+        kernels: out_dim % 32 == 0 and in_dim % 8 == 0.
+
+        The order in which float32 sums are formed depends on the shape and, where in_dim is a multiple
+        of 2048, on which of the rank's experts it is: the same expert can give other last bits in a job
+        of another number of ranks. `rows_hint` changes no bit."""
         nle = self.num_local_experts
         dt = expert_x.dtype
         if dt not in _binding._DT:

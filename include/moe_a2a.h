@@ -347,6 +347,10 @@ int moe_a2a_expert_scale(const moe_a2a_shape* shape, const void* expert_x,
  * order plus the roundings allow around the exact value, and are exact when
  * every order gives the same float32 sum (identity and signed permutation
  * weights, small integers).
+ * Where in_dim is a multiple of 2048, a local expert's sums start at input
+ * in_dim * le / nle (rounded down to 64) and go round from there; elsewhere at
+ * input 0. So the same expert and rows can give other last bits on another number
+ * of ranks, or as another local expert.
  */
 int moe_a2a_expert_gemm(const moe_a2a_shape* shape, const void* expert_x,
                         const int32_t* expert_num_tokens, int32_t rows_hint,
@@ -364,7 +368,9 @@ int moe_a2a_expert_gemm(const moe_a2a_shape* shape, const void* expert_x,
  * rounded value and the sum rounded again, which is what the two torch
  * statements do. bias may be NULL.
  * One of four kernels runs, picked from the shape alone (so a shape always
- * gives the same bits): for m <= 64, k >= 449 (eight steps of 64 elements) and
+ * gives the same bits; a slice of the weight's rows is another shape, and where
+ * m <= 64 and k is a multiple of 2048 the first of these kernels also starts its
+ * sums at an input that depends on the column's place among n): for m <= 64, k >= 449 (eight steps of 64 elements) and
  * n <= 24448 (fewer than 192 tiles of 128 columns), a kernel whose
  * workgroups own 32 columns and split k over their waves (partial sums added in
  * a fixed order); else kernels bound by the matrix cores, whose workgroups own
