@@ -2166,8 +2166,9 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
   const int rb = blockIdx.x / col_units, cu = blockIdx.x - rb * col_units;
   const int t0 = rb * TOK, n0 = cu * 32, live = M - t0;
   // APART: where rows lie a multiple of 4 KB apart (see first_kstep) workgroups start apart too, by whole turns of
-  // the waves, so that a wave keeps its steps (elsewhere going round would cost 0.8 %: 64 x 7168 x 2304 11.29 us, 11.20 without): 8 x 8192 x 8192 34.1 -> 25.6 us, 1 x 4096 x 4096 12.4 -> 9.5, 64 x 8192 x 8192
-  // 41 -> 38, 16 x 16384 x 2048 16.0 -> 14.6.
+  // the waves, so that a wave keeps its steps: 8 x 8192 x 8192 34.1 -> 25.6 us, 1 x 4096 x 4096 12.4 -> 9.5, 64 x
+  // 8192 x 8192 41 -> 38, 16 x 16384 x 2048 16.0 -> 14.6. Elsewhere going round costs 0.8 % (64 x 7168 x 2304 11.29 us,
+  // 11.20 without).
   static_assert(32 % KW == 0, "whole turns in the steps of 2048 inputs");
   const int first_step = APART ? (int)((long long)cu * (steps / KW) / col_units) * KW : 0;
 
@@ -2272,7 +2273,8 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
 // ---------------------------------------------------------------- dense product (many rows)
 //
 // C[M, N] = A[M, K] @ B[N, K]^T for outputs that tiles of 256 columns (phased_gemm_kernel) would spread over
-// too few compute units. A workgroup of four waves owns a BM x BN tile of C (64 or 128 x 128) and walks K in steps of
+// too few compute units, and for experts' rows (GROUPED) also where those would leave much of a last round idle. A
+// workgroup of four waves owns a BM x BN tile of C (64 or 128 x 128) and walks K in steps of
 // 64 elements. Per step the workgroup copies BM + BN rows of 128 bytes into LDS once (through registers, two LDS
 // buffers, one barrier per step), and every wave reads each operand fragment it needs once per 16-element slice
 // of the step for a whole row or column of its MFMA tiles, issued one slice ahead.
@@ -2619,11 +2621,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void dense_gemm_kernel(
 //    farther ahead but ask for half lines: 425 against 380 us at K = 4096.
 //  - Rows that start off the lines take one and three quarter times the line requests: AHEAD then brings the
 //    lines into L2 before (operands out of HBM, K = 3696: 390 -> 372 us; on aligned rows it costs 1 to 2 %).
-//  - GROUPED (the experts' products): a group's weights are read for a few hundred rows only, and what a
-//    compute unit can fetch, about 49 KB a microsecond with most lines on their way from HBM, bounds it. The
-//    fewer tiles the better: up to 320 rows per tile (two buffers of each operand fit), spread evenly over the
+//  - GROUPED (the experts' products): a group's weights are read for a few hundred rows only, most lines come
+//    from HBM, and the loads bound it. The fewer tiles the better: up to 320 rows per tile, spread evenly over the
 //    tiles of a group, and only the bands of 32 rows that there are get fetched and multiplied. 32 groups x 256
-//    rows, 2048 x 4096: 208 us with dense_gemm_kernel's 128 x 128 tiles, 156 here; 1024 rows 407 -> 254.
+//    rows, 2048 x 4096: 208 us with dense_gemm_kernel's 128 x 128 tiles, 153 to 160 here (145 without the MFMAs, 96
+//    without the loads); 1024 rows 407 -> 254. A unit fetches 4.2 MB in that time, 27 KB a microsecond with 90 lines
+//    under way on average: with two buffers of each operand nothing is asked for while a step's last rows are
+//    waited for. (Tiles of 192 rows, three buffers of B: 37 KB a microsecond, but half as much again to fetch.)
 // Measured at 8192 x 8192 (bf16, uniform values, clocks settled): K = 3696 395 us with dense_gemm_kernel's
 // 256 x 256 tile, 340 here (1.46 PFLOP/s); K = 4096 x 4096 x 4096 107 and 90; K = 8192 795 and 702.
 //
@@ -4344,10 +4348,9 @@ int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, i
 #ifndef MOE_A2A_GROUPED_DENSE_MIN_ROWS
 #define MOE_A2A_GROUPED_DENSE_MIN_ROWS 56  // rows per group (from the caller's row count) from which tiles are used
 #endif
-// The grouped product when groups have hundreds of rows: the weights are then read for enough
-// rows that the matrix cores, not the stream of weights, bound the work, and the dense kernel's
-// tiles (each weight row read once per 64 to 320 rows, operands shared by the workgroup's waves through
-// LDS) do better than the kernel that is built around streaming. MOE_A2A_NOT_DENSE otherwise.
+// The grouped product from some dozens of rows per group: the dense kernels' tiles (each weight row read once per 64
+// to 320 rows, operands shared by the workgroup's waves through LDS) do as well as or better than the kernel that is
+// built around streaming the weights. MOE_A2A_NOT_DENSE otherwise.
 int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void* w, const void* bias, void* y,
                          int groups, long long max_rows, long long rows_hint, int N, int K, int dtype,
                          hipStream_t st, int compact = 0) {

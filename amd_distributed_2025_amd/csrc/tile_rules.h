@@ -16,12 +16,14 @@ bool tile_rows_in_range(long long rows, long long K) { return rows * K * 2 < OUT
 // columns; 4, 2: dense_gemm_kernel, 128 columns), 0 where rows of K are too long for any. `rows_hint` rows over all
 // groups are taken to be spread as uniform routing spreads them: a group's number is normal around the average.
 //
-// A tile costs per step of K what its unit has to fetch, in rows of 128 bytes (a unit fetches one in 2.6 ns, the
-// matrix cores are faster in every case that was measured). A step takes no less than HBM needs for the weights,
+// A tile costs per step of K what its unit has to fetch, in rows of 128 bytes, about 3 ns each (32 groups of 256 rows,
+// 2048 x 4096, tiles of 192 rows: 37 KB a microsecond and unit, 40 without the MFMAs; the MFMAs without the loads take
+// 0.55 to 0.7 of the time on every tall tile). A step takes no less than HBM needs for the weights,
 // which every round of tiles over the units asks for anew: 256 x 256 columns in the time of 490 rows, two
 // workgroups of 128 columns on every unit in that of 530. What else was measured and stands in the factors: two
-// workgroups on a unit fetch 1.3 times as slowly as one; the two buffers of 320 rows cost 1.38; the first loads and
-// the results of a tile take as long as six steps, of two with two workgroups on a unit, which overlap them.
+// workgroups on a unit fetch 1.3 times as slowly as one; tiles of 320 rows, which have room for two buffers of either
+// operand only and wait for every load once a step, 1.38 times (26 KB a microsecond, 29 without the MFMAs); the first
+// loads and the results of a tile take as long as six steps, of two with two workgroups on a unit, which overlap them.
 // Factors and floors are those that lose least, and their neighbours lose hardly more: 697 shapes of 2 to 128 groups,
 // 50 to 1024 rows, N and K of 512 to 8192, all five tiles timed on each. The choice is 1.5 % behind the best of them
 // and the streaming kernel on average, more than a tenth on 31. (Counting rounds x (height + columns) alone, without
