@@ -91,4 +91,5 @@ def check(status: int, what: str) -> None:
 
 
 def call(name: str, *args) -> None:
+    """One entry point by name, for callers without a binding object; raises on a nonzero status."""
     check(getattr(load(), name)(*args), name)

@@ -18,7 +18,7 @@ bool tile_rows_in_range(long long rows, long long K) { return rows * K * 2 < OUT
 //
 // A tile costs per step of K what its unit has to fetch, in rows of 128 bytes, about 3 ns each (32 groups of 256 rows,
 // 2048 x 4096, tiles of 192 rows: 37 KB a microsecond and unit, 40 without the MFMAs; the MFMAs without the loads take
-// 0.55 to 0.7 of the time on every tall tile). A step takes no less than HBM needs for the weights,
+// 0.5 to 0.7 of the time on every tall tile). A step takes no less than HBM needs for the weights,
 // which every round of tiles over the units asks for anew: 256 x 256 columns in the time of 490 rows, two
 // workgroups of 128 columns on every unit in that of 530. What else was measured and stands in the factors: two
 // workgroups on a unit fetch 1.3 times as slowly as one; tiles of 320 rows, which have room for two buffers of either
