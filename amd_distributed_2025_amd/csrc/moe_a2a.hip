@@ -2623,11 +2623,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void dense_gemm_kernel(
 //    lines into L2 before (operands out of HBM, K = 3696: 390 -> 372 us; on aligned rows it costs 1 to 2 %).
 //  - GROUPED (the experts' products): a group's weights are read for a few hundred rows only, most lines come
 //    from HBM, and the loads bound it. The fewer tiles the better: up to 320 rows per tile, spread evenly over the
-//    tiles of a group, and only the bands of 32 rows that there are get fetched and multiplied. 32 groups x 256
-//    rows, 2048 x 4096: 208 us with dense_gemm_kernel's 128 x 128 tiles, 153 to 160 here (145 without the MFMAs, 96
-//    without the loads); 1024 rows 407 -> 254. A unit fetches 4.2 MB in that time, 27 KB a microsecond with 90 lines
-//    under way on average: with two buffers of each operand nothing is asked for while a step's last rows are
-//    waited for. (Tiles of 192 rows, three buffers of B: 37 KB a microsecond, but half as much again to fetch.)
+//    tiles of a group, and only the bands of 32 rows that there are get fetched and multiplied. Beside two buffers
+//    of 320 rows of A there is room for five halves of B (128 columns each): the ring of halves keeps half a
+//    step of weights under way while the rows of the next step are waited for, and rows of A have a whole step to
+//    arrive. 32 groups x 256 rows, 2048 x 4096: 208 us with dense_gemm_kernel's 128 x 128 tiles, 151 with two whole
+//    buffers of either operand, which leave nothing under way then, 137 here (131 without the MFMAs, 99 without the
+//    loads, 107 with the weights alone, which is their rate out of HBM in this pattern); 4096 x 2048 161 -> 147.
 // Measured at 8192 x 8192 (bf16, uniform values, clocks settled): K = 3696 395 us with dense_gemm_kernel's
 // 256 x 256 tile, 340 here (1.46 PFLOP/s); K = 4096 x 4096 x 4096 107 and 90; K = 8192 795 and 702.
 //
@@ -2674,8 +2675,8 @@ template <> struct Mfma16x16x32<MOE_A2A_F16> {
 
 constexpr int phased_rows(int TM) { return 32 * TM; }
 constexpr int phased_cols(int TN) { return 64 * TN; }
-constexpr size_t phased_lds_bytes(int TM, int TN, int NA, int NB) {
-  return (size_t)(NA * phased_rows(TM) + NB * phased_cols(TN)) * 128;
+constexpr size_t phased_lds_bytes(int TM, int TN, int NA, int HB) {  // NA buffers of A, HB half buffers of B
+  return (size_t)(NA * phased_rows(TM) + HB * phased_cols(TN) / 2) * 128;
 }
 
 // Tiles of a grouped product: A is [groups, max_rows, K], B [groups, N, K], C [groups, max_rows, N], and group g
@@ -2756,19 +2757,21 @@ __device__ __forceinline__ GroupTile find_group_tile(int tile, const int* __rest
   return at;
 }
 
-template <int DT, int TM, int TN, int NA, int NB, bool AHEAD, bool GROUPED>
+template <int DT, int TM, int TN, int NA, int HB, bool AHEAD, bool GROUPED>
 __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
     const b128* __restrict__ A, const b128* __restrict__ B, const uint16_t* __restrict__ bias,
     uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
     const int* __restrict__ rows_of_group, int groups, int max_rows, int compact) {
   constexpr int BM = phased_rows(TM), BN = phased_cols(TN), GROUP_M = 4;
   constexpr int LA = BM / 64, LB = BN / 64;  // direct loads (8 rows each) of a wave per step
-  constexpr bool TIGHT = NA == 2 && NB == 2;  // two buffers of either operand
-  static_assert(BM % 64 == 0 && (TIGHT ? !AHEAD : NA >= 2 && NB >= 2 && NA + NB == 5), "whole loads, and a schedule for the buffers");
+  constexpr bool HALVES = HB % 2 != 0;  // B goes to a ring of HB halves (BN / 2 columns each) instead of NB whole buffers
+  constexpr int NB = HB / 2;
+  static_assert(BM % 64 == 0 && (HALVES ? NA == 2 && HB == 5 && !AHEAD : NA >= 2 && NB >= 2 && NA + NB == 5),
+                "whole loads, and a schedule for the buffers");
   static_assert(!(AHEAD && GROUPED), "tiles that share rows across an XCD");
   constexpr bool B_FIRST = NB <= NA;  // the operand with fewer buffers is asked for in the first slice of a step
-  constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, B_AT = NA * A_BYTES;
-  extern __shared__ b128 tile_lds[];  // [NA][BM * 8], [NB][BN * 8]
+  constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, HALF_BYTES = B_BYTES / 2, B_AT = NA * A_BYTES;
+  extern __shared__ b128 tile_lds[];  // [NA][BM * 8], [HB][BN * 4]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 2, wn = wave & 3;
   const int row_vecs = K / 8, row_bytes = K * 2, steps = (K + GEMM_KSTEP - 1) / GEMM_KSTEP;
@@ -2829,13 +2832,13 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
       for (int i = 0; i < LA; ++i) aoff[i] = OUT_OF_RANGE;
     }
   };
-  auto b_range = [&](int step) __attribute__((always_inline)) {
+  auto b_range = [&](int step, int from, int to) __attribute__((always_inline)) {
     if (step == steps - 1) {
 #pragma unroll
-      for (int i = 0; i < LB; ++i) boff[i] += vec_of(b_row(i)) >= tail_vecs ? OUT_OF_RANGE : 0;
+      for (int i = from; i < to; ++i) boff[i] += vec_of(b_row(i)) >= tail_vecs ? OUT_OF_RANGE : 0;
     } else if (step >= steps) {
 #pragma unroll
-      for (int i = 0; i < LB; ++i) boff[i] = OUT_OF_RANGE;
+      for (int i = from; i < to; ++i) boff[i] = OUT_OF_RANGE;
     }
   };
 
@@ -2844,9 +2847,13 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   // byte of a row at which the next requested step begins
   int a_soff = GROUPED ? k_first : 0, b_soff = a_soff;
   unsigned a_fill = 0, b_fill = 0;     // buffer (as a byte offset) that the next requested step goes to
-  unsigned a_use = 0, b_use = 0;       // buffer of the step being multiplied
+  // buffer of the step being multiplied (HALVES: the place of the half that holds this wave's columns)
+  unsigned a_use = 0, b_use = HALVES ? (wn >> 1) * HALF_BYTES : 0;
+  [[maybe_unused]] int half_soff[2] = {b_soff, b_soff};
   auto next_a = [](unsigned at) { return at == (NA - 1) * A_BYTES ? 0u : at + A_BYTES; };
-  auto next_b = [](unsigned at) { return at == (NB - 1) * B_BYTES ? 0u : at + B_BYTES; };
+  auto next_b = [](unsigned at) {
+    return at + B_BYTES < HB * HALF_BYTES ? at + B_BYTES : at + B_BYTES - HB * HALF_BYTES;
+  };
   auto load_a = [&]() __attribute__((always_inline)) {
     unrolled<0, LA>([&](auto c) __attribute__((always_inline)) {
       constexpr int i = decltype(c)::value;
@@ -2865,6 +2872,19 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
     b_soff += GEMM_KSTEP * 2;
     if (GROUPED && k_first && b_soff == row_bytes) b_soff = 0;
   };
+
+  auto load_half = [&](auto half) __attribute__((always_inline)) {  // the next step's columns of a half
+    constexpr int h = decltype(half)::value;
+    unrolled<0, LB / 2>([&](auto c) __attribute__((always_inline)) {
+      constexpr int i = decltype(c)::value;
+      load_to_lds<i * 8192>(b_base + b_fill, boff[h * (LB / 2) + i], bbuf, half_soff[h]);
+    });
+    b_fill = b_fill == (HB - 1) * HALF_BYTES ? 0u : b_fill + HALF_BYTES;
+    half_soff[h] += GEMM_KSTEP * 2;
+    if (GROUPED && k_first && half_soff[h] == row_bytes) half_soff[h] = 0;
+  };
+  constexpr std::integral_constant<int, 0> lower{};
+  constexpr std::integral_constant<int, 1> upper{};
 
   // AHEAD: a wave touches, four steps ahead, one line each of the rows this workgroup fetches into L2 for its
   // neighbours as well: of the GROUP_M x 8 tiles that an XCD works on at a time, the 8 with the same rows of
@@ -2905,7 +2925,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     a_frag[s] = lds + (wm * 16 + r) * 128 + ((s * 4 + q) ^ swz) * 16;
-    b_frag[s] = lds + B_AT + (wn * TN * 16 + r) * 128 + ((s * 4 + q) ^ swz) * 16;
+    b_frag[s] = lds + B_AT + ((HALVES ? wn & 1 : wn) * TN * 16 + r) * 128 + ((s * 4 + q) ^ swz) * 16;
   }
   b128 af[TM], bf[TN];
   f32x4 acc[TM][TN] = {};
@@ -2954,43 +2974,58 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((B_FIRST ? LA : LB) + (AHEAD ? 1 : 0)) : "memory");
     multiply(bands, nothing, nothing);
   };
-  // With two buffers of either operand the rows of step s + 1 can only go to the buffers of step s - 1, and have
-  // to be there when the first group has multiplied step s: both groups wait in the phase before that, the first
-  // behind its MFMAs, the second behind its last reads. Rows of B, which come from farther away, are asked for
-  // first; the second group asks for rows of A at the start of its turn, a phase earlier than it could else.
-  auto one_tight_step = [&](auto bands) __attribute__((always_inline)) {
+  // With five halves of B, step s + 1's upper half and step s + 2's lower one go to the places of step s - 1's halves,
+  // and step s + 1's rows of A to the buffer of step s - 1. Step s + 1 has to be there when the first group has
+  // multiplied step s: both groups wait in the phase before that, the first behind its MFMAs, the second behind its
+  // last reads, for all but the lower half of step s + 2, the youngest loads.
+  auto one_step_of_halves = [&](auto bands) __attribute__((always_inline)) {
+    constexpr int YOUNGER = LB / 2;  // loads of a wave that may be under way when a step ends
     read_frags(bands, 0);
-    load_b();
-    multiply(bands, [&]() __attribute__((always_inline)) { if (!first_group) load_a(); }, nothing);
+    load_half(upper);
+    load_a();
+    multiply(bands, nothing, nothing);
     read_frags(bands, 1);
-    if (first_group) load_a();
+    load_half(lower);
     a_use = next_a(a_use);
     b_use = next_b(b_use);
-    if (!first_group) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    multiply(bands, nothing,
-             [&]() __attribute__((always_inline)) { if (first_group) asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); });
+    if (!first_group) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER) : "memory");
+    multiply(bands, nothing, [&]() __attribute__((always_inline)) {
+      if (first_group) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER) : "memory");
+    });
   };
-  unrolled<0, 2>([&](auto c) __attribute__((always_inline)) {
-    constexpr int at = decltype(c)::value;
-    if constexpr (at < NA - 1) { a_range(at); load_a(); }
-    if constexpr (at < NB - 1) { b_range(at); load_b(); }
-  });
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NA - 2) * LA + (NB - 2) * LB) : "memory");
+  if constexpr (HALVES) {
+    b_range(0, 0, LB);
+    load_half(lower);
+    load_half(upper);
+    a_range(0);
+    load_a();
+    b_range(1, 0, LB / 2);
+    load_half(lower);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LB / 2) : "memory");
+  } else {
+    unrolled<0, 2>([&](auto c) __attribute__((always_inline)) {
+      constexpr int at = decltype(c)::value;
+      if constexpr (at < NA - 1) { a_range(at); load_a(); }
+      if constexpr (at < NB - 1) { b_range(at, 0, LB); load_b(); }
+    });
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NA - 2) * LA + (NB - 2) * LB) : "memory");
+  }
   if (!first_group) asm volatile("s_barrier" ::: "memory");  // one phase behind
   auto walk_k = [&](auto bands) __attribute__((always_inline)) {
     int step = 0;
-    if constexpr (TIGHT) {
-      for (; step + 2 < steps; ++step) one_tight_step(bands);
+    if constexpr (HALVES) {
+      for (; step + 3 < steps; ++step) one_step_of_halves(bands);
       for (; step < steps; ++step) {
         a_range(step + 1);
-        b_range(step + 1);
-        one_tight_step(bands);
+        b_range(step + 1, LB / 2, LB);
+        b_range(step + 2, 0, LB / 2);
+        one_step_of_halves(bands);
       }
     } else {
       for (; step + 3 < steps; ++step) one_slice_pair(bands, step);  // (what it asks for lies before the last step)
       for (; step < steps; ++step) {
         a_range(step + NA - 1);
-        b_range(step + NB - 1);
+        b_range(step + NB - 1, 0, LB);
         one_slice_pair(bands, step);
       }
     }
@@ -4276,18 +4311,18 @@ int allow_large_lds() {
   };
   auto allow_grouped = [&](auto dtype) {
     constexpr int DT = decltype(dtype)::value;
-    allow((const void*)phased_gemm_kernel<DT, 10, 4, 2, 2, false, true>, phased_lds_bytes(10, 4, 2, 2));
-    allow((const void*)phased_gemm_kernel<DT, 8, 4, 2, 3, false, true>, phased_lds_bytes(8, 4, 2, 3));
-    allow((const void*)phased_gemm_kernel<DT, 6, 4, 2, 3, false, true>, phased_lds_bytes(6, 4, 2, 3));
+    allow((const void*)phased_gemm_kernel<DT, 10, 4, 2, 5, false, true>, phased_lds_bytes(10, 4, 2, 5));
+    allow((const void*)phased_gemm_kernel<DT, 8, 4, 2, 6, false, true>, phased_lds_bytes(8, 4, 2, 6));
+    allow((const void*)phased_gemm_kernel<DT, 6, 4, 2, 6, false, true>, phased_lds_bytes(6, 4, 2, 6));
     allow((const void*)dense_gemm_kernel<DT, 2, 2, 2, 2, true>, dense_lds_bytes(128, 128));
     allow((const void*)dense_gemm_kernel<DT, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
   };
-  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 2, false, false>, phased_lds_bytes(8, 4, 3, 2));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 2, false, false>, phased_lds_bytes(8, 4, 3, 2));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 2, true, false>, phased_lds_bytes(8, 4, 3, 2));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 2, true, false>, phased_lds_bytes(8, 4, 3, 2));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 4, 2, 3, 2, false, false>, phased_lds_bytes(4, 2, 3, 2));
-  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 4, 2, 3, 2, false, false>, phased_lds_bytes(4, 2, 3, 2));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 4, false, false>, phased_lds_bytes(8, 4, 3, 4));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 4, false, false>, phased_lds_bytes(8, 4, 3, 4));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 4, true, false>, phased_lds_bytes(8, 4, 3, 4));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 4, true, false>, phased_lds_bytes(8, 4, 3, 4));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 4, 2, 3, 4, false, false>, phased_lds_bytes(4, 2, 3, 4));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 4, 2, 3, 4, false, false>, phased_lds_bytes(4, 2, 3, 4));
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
@@ -4319,7 +4354,7 @@ int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, i
   const int grid = (int)(tiles_m * tiles_n);
   if (const int rc = allow_large_lds()) return rc;
 #define LAUNCH_P(DT, TM, TN, AHEAD)                                                              \
-  phased_gemm_kernel<DT, TM, TN, 3, 2, AHEAD, false><<<grid, 512, phased_lds_bytes(TM, TN, 3, 2), st>>>( \
+  phased_gemm_kernel<DT, TM, TN, 3, 4, AHEAD, false><<<grid, 512, phased_lds_bytes(TM, TN, 3, 4), st>>>( \
       (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n, \
       nullptr, 0, 0, 0)
   // Tiles of 128 x 128, at most one per unit: nobody is there to work while phased_gemm_kernel's waves wait for each
@@ -4376,9 +4411,9 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
     };
     auto phased = [&](auto kernel, size_t lds_bytes) { start(kernel, 512, lds_bytes); };
     auto dense = [&](auto kernel, size_t lds_bytes) { start(kernel, 256, lds_bytes); };
-    if (bands == 10) phased(phased_gemm_kernel<DT, 10, 4, 2, 2, false, true>, phased_lds_bytes(10, 4, 2, 2));
-    else if (bands == 8) phased(phased_gemm_kernel<DT, 8, 4, 2, 3, false, true>, phased_lds_bytes(8, 4, 2, 3));
-    else if (bands == 6) phased(phased_gemm_kernel<DT, 6, 4, 2, 3, false, true>, phased_lds_bytes(6, 4, 2, 3));
+    if (bands == 10) phased(phased_gemm_kernel<DT, 10, 4, 2, 5, false, true>, phased_lds_bytes(10, 4, 2, 5));
+    else if (bands == 8) phased(phased_gemm_kernel<DT, 8, 4, 2, 6, false, true>, phased_lds_bytes(8, 4, 2, 6));
+    else if (bands == 6) phased(phased_gemm_kernel<DT, 6, 4, 2, 6, false, true>, phased_lds_bytes(6, 4, 2, 6));
     else if (bands == 4) dense(dense_gemm_kernel<DT, 2, 2, 2, 2, true>, dense_lds_bytes(128, 128));
     else dense(dense_gemm_kernel<DT, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
   };

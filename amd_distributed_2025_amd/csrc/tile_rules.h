@@ -21,15 +21,15 @@ bool tile_rows_in_range(long long rows, long long K) { return rows * K * 2 < OUT
 // 0.5 to 0.7 of the time on every tall tile). A step takes no less than HBM needs for the weights,
 // which every round of tiles over the units asks for anew: 256 x 256 columns in the time of 490 rows, two
 // workgroups of 128 columns on every unit in that of 530. What else was measured and stands in the factors: two
-// workgroups on a unit fetch 1.3 times as slowly as one; tiles of 320 rows, which have room for two buffers of either
-// operand only and wait for every load once a step, 1.38 times (26 KB a microsecond, 29 without the MFMAs); the first
+// workgroups on a unit fetch 1.3 times as slowly as one; tiles of 320 rows, which have room for half a step of weights
+// beyond the next one, 1.15 times (30 KB a microsecond, 32 without the MFMAs); the first
 // loads and the results of a tile take as long as six steps, of two with two workgroups on a unit, which overlap them.
 // Factors and floors are those that lose least, and their neighbours lose hardly more: 697 shapes of 2 to 128 groups,
 // 50 to 1024 rows, N and K of 512 to 8192, all five tiles timed on each. The choice is 1.5 % behind the best of them
 // and the streaming kernel on average, more than a tenth on 31. (Counting rounds x (height + columns) alone, without
 // the tile of 128 x 128, it was 6.4 % behind, and more than a tenth on 155.) Among them, us with 320 / 256 / 192 / 128 /
-// 64 rows: 32 groups of 63 rows, 7168 x 7168 770 / 613 / 604 / 576 / 708; 8 of 64, 4096 x 4096 104 / 78 / 76 / 52 / 65;
-// 32 of 100, 2048 x 4096 126 / 105 / 104 / 119 / 146; 32 of 256, 4096 x 2048 161 / 176 / 182 / 203 / 240.
+// 64 rows: 32 groups of 63 rows, 7168 x 7168 640 / 613 / 604 / 576 / 708; 8 of 64, 4096 x 4096 89 / 78 / 76 / 52 / 65;
+// 32 of 100, 2048 x 4096 112 / 105 / 104 / 119 / 146; 32 of 256, 4096 x 2048 147 / 176 / 182 / 203 / 240.
 struct GroupTiles {
   double each;    // tiles of a group, on average
   double surely;  // as many as nearly every group has
@@ -63,7 +63,7 @@ int grouped_tile_bands(long long rows_hint, int groups, int N, int K) {
     const double rounds = std::max(t.surely * one_each, t.each * one_each - FEW);
     double cost;
     if (wide == 256) {  // one workgroup per unit
-      const double fetch = (t.height + 256) * (bands == 10 ? 1.38 : 1.0), weights = 490 / t.each;
+      const double fetch = (t.height + 256) * (bands == 10 ? 1.15 : 1.0), weights = 490 / t.each;
       const double whole = std::floor(rounds), rest = rounds - whole;
       cost = whole * std::max(fetch, weights) + (rest > 0 ? std::max(fetch, rest * weights) : 0);
       cost *= 1 + 6 / steps;

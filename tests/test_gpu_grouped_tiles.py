@@ -60,6 +60,28 @@ def test_every_tile_gives_the_same_bits(groups, counts, K, bias, dt):
         assert (got[at:] == 7).all()
 
 
+FEW_STEPS = [64, 128, 136, 192, 328, 392]  # one to seven steps of 64, the last one whole or not
+
+
+@pytest.mark.parametrize("K", FEW_STEPS)
+def test_few_steps_on_the_ring_of_half_steps(K):
+    """320 rows: weights go round a ring of five half steps. Walks shorter than the ring, as long, and longer,
+    on small integers, whose sums every order gives exactly; tiles of one to ten bands of 32 rows."""
+    print(f"ring of halves K={K}", flush=True)
+    counts, N = [289, 330, 61], 7168
+    a = HIPAllToAll(MoEConfig(3, 1, K, 704, torch.bfloat16, torch.bfloat16), 0, 1, device=torch.device(DEV))
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x = torch.randint(-1, 2, (3, 704, K), generator=g, device=DEV).bfloat16()
+    w = torch.randint(-1, 2, (3, N, K), generator=g, device=DEV).bfloat16()
+    num = torch.tensor(counts, dtype=torch.int32, device=DEV)
+    for rows in (1, 32, 65, 97, 129, 161, 193, 225, 257, 320):
+        num[2] = rows
+        out = a.expert_gemm(x, num, w, None, rows_hint=800 * 3, out=torch.full((3, 704, N), 7.0, dtype=x.dtype, device=DEV))
+        for e, c in enumerate([*counts[:2], rows]):
+            assert torch.equal(out[e, :c], (x[e, :c].double() @ w[e].double().T).float().bfloat16()), (rows, e)
+            assert (out[e, c:] == 7).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (33, 96, 4096), (64, 2080, 2048), (8, 1024, 6144), (64, 64, 8192)])
 def test_few_rows_whose_walks_of_K_start_apart(M, N, K):
     """`moe_a2a_linear` on at most 64 rows of a multiple of 2048 inputs: small integers, whose sums every order

@@ -7,7 +7,7 @@ from pathlib import Path
 import pytest
 
 from tests.test_gpu_expert_gemm import TILES_OF_NARROW
-from tests.test_gpu_grouped_tiles import ROWS_FOR_TILE
+from tests.test_gpu_grouped_tiles import FEW_STEPS, ROWS_FOR_TILE
 
 CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
 
@@ -72,6 +72,11 @@ def test_the_tiles_that_the_gpu_tests_mean(rules, K):
     assert {t for tiles in ROWS_FOR_TILE.values() for t in tiles.values() if isinstance(t, int)} == {64, 128, 192, 256, 320}
     for (in_dim, out_dim), tiles in TILES_OF_NARROW.items():
         assert {rows: 32 * rules.bands(rows * 5, 5, out_dim, in_dim) for rows in tiles} == tiles
+
+
+@pytest.mark.parametrize("K", FEW_STEPS)
+def test_the_tile_that_the_ring_of_half_steps_is_tested_on(rules, K):
+    assert rules.bands(800 * 3, 3, 7168, K) == 10
 
 
 def test_the_second_tiles_that_the_gpu_tests_mean():
