@@ -59,30 +59,36 @@ constexpr int NUM_XCD = 8;
 // struct whose copies become memcpy calls that can pin a local in memory.)
 typedef unsigned int b128 __attribute__((ext_vector_type(4)));
 
-// Streaming (nontemporal) stores do not write-allocate in L2, which makes the
-// writing kernel about a quarter faster, but a kernel that reads the rows right
-// afterwards then fetches them from HBM and loses more than the writer gained.
-// So they are used only for the two buffers whose next reader is the exchange
-// (in a multi-GPU job: the fabric), not for expert_x / expert_y, which the
-// expert computation reads next on the same device.
-#ifndef MOE_A2A_NT_SEND   /* stage 1 -> send buffer */
-#define MOE_A2A_NT_SEND 1
+// How a row is stored.
+// STREAM (nontemporal) does not write-allocate in L2, which makes the writing kernel about a quarter faster, but a
+// kernel that reads the rows right afterwards then fetches them from HBM and loses more than the writer gained. So
+// the row movers use it only for the two buffers whose next reader is the exchange (in a multi-GPU job: the
+// fabric), not for expert_x / expert_y, which the expert computation reads next on the same device.
+// THROUGH (device scope) writes on past L2 while the kernel runs. What a plain store leaves dirty there is written
+// back when the kernel ends, with nothing else going on: the 29 MB that stage 2 writes at the headline shape
+// (8 ranks, 2048 rows of 14 KB) cost 15.8 us plain, 14.7 through; the stand-in's rows of a whole job 44.5 and 42.9.
+// The readers lose nothing: the L2s of the XCDs do not serve each other, so they come from behind L2 either way.
+enum Store { PLAIN, THROUGH, STREAM };
+#ifndef MOE_A2A_STORE_SEND   /* stage 1 -> send buffer */
+#define MOE_A2A_STORE_SEND STREAM
 #endif
-#ifndef MOE_A2A_NT_RECV   /* stage 2 -> expert_x */
-#define MOE_A2A_NT_RECV 0
+#ifndef MOE_A2A_STORE_RECV   /* stage 2 -> expert_x */
+#define MOE_A2A_STORE_RECV THROUGH
 #endif
-#ifndef MOE_A2A_NT_CSEND  /* stage 3 -> send-back buffer */
-#define MOE_A2A_NT_CSEND 1
+#ifndef MOE_A2A_STORE_CSEND  /* stage 3 -> send-back buffer */
+#define MOE_A2A_STORE_CSEND STREAM
 #endif
-#ifndef MOE_A2A_NT_STANDIN /* expert and exchange stand-ins */
-#define MOE_A2A_NT_STANDIN 0
+#ifndef MOE_A2A_STORE_STANDIN /* expert and exchange stand-ins */
+#define MOE_A2A_STORE_STANDIN THROUGH
 #endif
 #ifndef MOE_A2A_NT_LOAD
 #define MOE_A2A_NT_LOAD 0
 #endif
-template <bool NT, typename V>
+template <Store HOW, typename V>
 __device__ __forceinline__ void row_store(V* p, const V& v) {
-  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  if constexpr (HOW == STREAM) __builtin_nontemporal_store(v, p);
+  else if constexpr (HOW == THROUGH && sizeof(V) == sizeof(b128))
+    __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) b128*)p, v, "agent");
   else *p = v;
 }
 template <typename P>
@@ -228,16 +234,16 @@ struct Payload {
 #pragma unroll
     for (int j = 0; j < NV; ++j) v[j] = stream_load(row + min(base + j * BLOCK + (int)threadIdx.x, row_vecs - 1));
   }
-  template <bool NT>
+  template <Store HOW>
   __device__ __forceinline__ void store_as(V* __restrict__ row, int base, int row_vecs) const {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int idx = base + j * BLOCK + threadIdx.x;
-      if (idx < row_vecs) row_store<NT>(row + idx, v[j]);
+      if (idx < row_vecs) row_store<HOW>(row + idx, v[j]);
     }
   }
   __device__ __forceinline__ void store(V* __restrict__ row, int base, int row_vecs) const {
-    store_as<(MOE_A2A_NT_STANDIN != 0)>(row, base, row_vecs);
+    store_as<MOE_A2A_STORE_STANDIN>(row, base, row_vecs);
   }
   template <typename F>
   __device__ __forceinline__ void map(F f) {
@@ -304,12 +310,12 @@ struct WavePayload {
 #pragma unroll
     for (int j = 0; j < NVW; ++j) v[j] = stream_load(row + min(base + j * 64 + lane, row_vecs - 1));
   }
-  template <bool NT>
+  template <Store HOW>
   __device__ __forceinline__ void store(V* __restrict__ row, int base, int row_vecs, int lane) const {
 #pragma unroll
     for (int j = 0; j < NVW; ++j) {
       const int idx = base + j * 64 + lane;
-      if (idx < row_vecs) row_store<NT>(row + idx, v[j]);
+      if (idx < row_vecs) row_store<HOW>(row + idx, v[j]);
     }
   }
 };
@@ -457,7 +463,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_send_kernel(
     const int slot = rows_reduce(cnt, part, parity, wave, lane);
 
     if (valid) {
-      p.template store<(MOE_A2A_NT_SEND != 0)>(send_buf + (size_t)slot * row_vecs, base, row_vecs, lane);
+      p.template store<MOE_A2A_STORE_SEND>(send_buf + (size_t)slot * row_vecs, base, row_vecs, lane);
       if (c == 0) {
         if (lane < META) {
           int m = lane == 0 ? e : lane == 1 ? rank : lane == 2 ? t : lane == 3 ? k : 0;
@@ -568,7 +574,7 @@ __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
           int slot = 0;
 #pragma unroll
           for (int w = 0; w < NWAVES; ++w) slot += half[w * FAN + g];
-          p.template store_as<(MOE_A2A_NT_SEND != 0)>(send_buf + (size_t)slot * row_vecs, base, row_vecs);
+          p.template store_as<MOE_A2A_STORE_SEND>(send_buf + (size_t)slot * row_vecs, base, row_vecs);
         }
       }
       if (c == 0 && tid < live * META) {
@@ -707,7 +713,7 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
 #pragma unroll
         for (int j = 0; j < NV; ++j)
           if (g < live && col + j * BLK < row_vecs)
-            row_store<(MOE_A2A_NT_SEND != 0)>(send_buf + (size_t)slot[g] * row_vecs + col + j * BLK, v[j]);
+            row_store<MOE_A2A_STORE_SEND>(send_buf + (size_t)slot[g] * row_vecs + col + j * BLK, v[j]);
       }
       if (c == 0 && tid < live * META) {
         const int g = tid / META, f = tid - g * META;
@@ -1054,7 +1060,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
       const int R = rows_known();
       if (i < R && (uint32_t)pos < (uint32_t)max_recv) {
         const size_t row = (size_t)floormod(e, nle, magic) * max_recv + pos;
-        p.template store<(MOE_A2A_NT_RECV != 0)>(expert_x + row * row_vecs, base, row_vecs, lane);
+        p.template store<MOE_A2A_STORE_RECV>(expert_x + row * row_vecs, base, row_vecs, lane);
         if (c == 0 && lane < META) expert_meta[row * META + lane] = m;
       }
       return R;
@@ -1094,7 +1100,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
 #pragma unroll
       for (int r = 0; r < ROWS; ++r) le = r == wave ? rle[r] : le;
       const size_t row = COMPACT ? (size_t)pos : (size_t)le * max_recv + pos;
-      p.template store<(MOE_A2A_NT_RECV != 0)>(expert_x + row * row_vecs, base, row_vecs, lane);
+      p.template store<MOE_A2A_STORE_RECV>(expert_x + row * row_vecs, base, row_vecs, lane);
       if (c == 0 && lane < META) expert_meta[row * META + lane] = m;
     }
     return R;
@@ -1348,7 +1354,7 @@ __global__ __launch_bounds__(64 * ROWS) void combine_send_kernel(
         const int src = max((int)__popcll(__ballot(run[0] <= j)) - 1, 0);
         const int slot = __builtin_amdgcn_readlane(run[1], src) + (j - __builtin_amdgcn_readlane(run[0], src));
         if (slot >= 0 && slot < capacity_rows) {
-          p.template store<(MOE_A2A_NT_CSEND != 0)>(send_buf + (size_t)slot * row_vecs, base, row_vecs, lane);
+          p.template store<MOE_A2A_STORE_CSEND>(send_buf + (size_t)slot * row_vecs, base, row_vecs, lane);
           if (c == 0 && lane < META) send_meta[(size_t)slot * META + lane] = m;
         }
       }
@@ -1420,7 +1426,7 @@ __global__ __launch_bounds__(64 * ROWS) void combine_send_kernel(
     const int slot = rows_reduce(cnt, part, parity, wave, lane);
 
     if (valid && slot < capacity_rows) {
-      p.template store<(MOE_A2A_NT_CSEND != 0)>(send_buf + (size_t)slot * row_vecs, base, row_vecs, lane);
+      p.template store<MOE_A2A_STORE_CSEND>(send_buf + (size_t)slot * row_vecs, base, row_vecs, lane);
       if (c == 0 && lane < META) send_meta[(size_t)slot * META + lane] = m;
     }
   }
@@ -1812,7 +1818,7 @@ __global__ __launch_bounds__(64 * ROWS) void expert_scale_wave_kernel(
     p.load(expert_x + row * row_vecs, base, row_vecs, lane);
 #pragma unroll
     for (int j = 0; j < NVW; ++j) p.v[j] = standin_expert<b128, DIN, DOUT>(p.v[j], scale);
-    p.template store<(MOE_A2A_NT_STANDIN != 0)>(expert_y + row * row_vecs, base, row_vecs, lane);
+    p.template store<MOE_A2A_STORE_STANDIN>(expert_y + row * row_vecs, base, row_vecs, lane);
   }
 }
 
@@ -2548,7 +2554,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void dense_gemm_kernel(
   // are 8-byte pieces of 32 different rows. Each wave parks one band of 32 rows at a time in a
   // region of its own (rows padded by 16 bytes so that they start in different banks; a wave's
   // LDS operations execute in order, so no barrier is needed inside it) and reads it back with
-  // 16 lanes per row: a store instruction then writes four 256-byte row segments.
+  // 16 lanes per row: a store instruction then writes four 256-byte row segments. They write through (Store):
+  // 1500 x 2304 x 360 8.7 -> 7.9 us, 1586 x 2432 x 1536 16.8 -> 15.8, with a kernel behind it that reads the result
+  // 21.2 -> 20.1; experts' products, plain / through / streaming: 7 x 57 rows, 2656 x 1152 13.4 / 13.2 / 13.3 and with
+  // the reader 18.7 / 18.5 / 19.6; 32 x 100 rows, 2720 x 1024 52.4 / 51.9 / 50.2 and 61.2 / 60.2 / 60.8.
   __syncthreads();  // every wave has read its last fragments: the operand tiles can be overwritten
   {
     constexpr int VR = TN * 4;            // 16-byte vectors per row of the wave's tile
@@ -2590,7 +2599,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void dense_gemm_kernel(
         const int row = p * ROWS_PER_READ + rrow;
         const b128 v = *(const b128*)(park + row * PITCH + rvec * 16);
         const int m = (wm * TM + i) * 32 + row, n = ncol + rvec * 8;
-        if (m < rows_left && n < N) *(b128*)(c_tile + (size_t)m * N + n) = v;
+        if (m < rows_left && n < N) row_store<THROUGH>((b128*)(c_tile + (size_t)m * N + n), v);
       }
     }
   }
@@ -3046,7 +3055,14 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
 
   // Out through LDS as in dense_gemm_kernel, a band of 16 rows at a time: a lane holds columns
   // j * 16 + q * 4 + 0..3 of row r, and a store instruction writes whole 128-byte pieces of rows.
+  // How they are stored (Store), measured as us of the product alone, plain / through / streaming, and with a kernel
+  // behind it that reads the result. Results of up to 64 MB go through: 2048 x 4096 x 256 9.8 / 8.3 / 9.1, with the
+  // reader 15.8 / 14.6 / 16.6; 4096 x 6144 x 512 32.2 / 30.6 / 31.0, 47.5 / 46.1 / 48.1. Larger ones are streamed
+  // where there is work to write them behind (8192 x 8192 x 3696 375 / 372 / 369, 416 / 413 / 415), and plain where
+  // that would cost the reader more than it gains (8192 x 8192 x 512 83 / 87 / 72, 123 / 127 / 128). Experts' results
+  // are streamed, which leaves L2 to the operands: 32 x 256 rows, 4096 x 2048 145 / 144 / 137, 180 / 183 / 177.
   {
+    const bool large = (long long)M * N > (32ll << 20), streams = GROUPED || (large && K >= 2048);
     constexpr int VR = TN * 2, PITCH = TN * 32 + 16, ROWS_PER_READ = 64 / VR;
     char* park = (char*)tile_lds + wave * (16 * PITCH);
     const int ncol = n0 + wn * TN * 16;
@@ -3080,7 +3096,12 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
         const int row = p * ROWS_PER_READ + rrow;
         const b128 v = *(const b128*)(park + row * PITCH + rvec * 16);
         const int m = i * 32 + wm * 16 + row, n = ncol + rvec * 8;
-        if (m < rows_left && n < N) *(b128*)(c_tile + (size_t)m * N + n) = v;
+        if (m < rows_left && n < N) {
+          b128* const to = (b128*)(c_tile + (size_t)m * N + n);
+          if (streams) row_store<STREAM>(to, v);
+          else if (large) row_store<PLAIN>(to, v);
+          else row_store<THROUGH>(to, v);
+        }
       }
     }
   }
