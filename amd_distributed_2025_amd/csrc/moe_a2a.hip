@@ -2778,6 +2778,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   static_assert(BM % 64 == 0 && (HALVES ? NA == 2 && HB == 5 && !AHEAD : NA >= 2 && NB >= 2 && NA + NB == 5),
                 "whole loads, and a schedule for the buffers");
   static_assert(!(AHEAD && GROUPED), "tiles that share rows across an XCD");
+  constexpr bool EARLY = !GROUPED;
   constexpr bool B_FIRST = NB <= NA;  // the operand with fewer buffers is asked for in the first slice of a step
   constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, HALF_BYTES = B_BYTES / 2, B_AT = NA * A_BYTES;
   extern __shared__ b128 tile_lds[];  // [NA][BM * 8], [HB][BN * 4]
@@ -2787,55 +2788,51 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   const int tail_vecs = row_vecs - (steps - 1) * 8;
   const bool first_group = wave < 4;
 
-  int tile = blockIdx.x;
-  [[maybe_unused]] int total_tiles = 0;
-  do {  // (one pass unless GROUPED, whose launch strides over the tiles: its size is a matter of speed only)
+  // A workgroup strides over the tiles (the size of the launch is a matter of speed only). EARLY: the first loads of
+  // its next tile go out before the results of the last one do, so that they arrive while those are written, and the
+  // accumulators are cleared meanwhile. A workgroup per tile / this: 8192 x 8192 x 512 84.5 / 79.0 us, x 3696 370.6 /
+  // 368.3, 4096 x 4096 x 4096 93.5 / 92.4, tiles of 128 x 128 at 3000 x 3000 x 1024 31.9 / 30.3. Experts' products have
+  // a workgroup per tile in general, and the registers for it would be spilled at 320 rows: 140 -> 146 us.
+  int tile = blockIdx.x, total_tiles = tiles_m * tiles_n;  // (GROUPED: counted by find_tile)
   int n0, rows_left;         // first column of the tile; rows of the matrix from the tile's first one on
   size_t row_at, b_at;       // the tile's first rows of A and C, and of B
   const uint16_t* bias_row;  // the bias of the tile's group, or null
   [[maybe_unused]] int tn, tm, k_first = 0;
-  if constexpr (GROUPED) {
-    lds_barrier();  // the tile before is out of LDS
-    const GroupTile at = find_group_tile<512, BM>(tile, rows_of_group, groups, max_rows, tiles_n, compact, (int*)tile_lds);
-    if (tile >= at.total) return;
-    lds_barrier();
-    total_tiles = at.total;
-    n0 = at.tn * BN;
-    rows_left = at.rows;
-    row_at = at.row_at;
-    b_at = (size_t)at.group * N + n0;
-    k_first = first_kstep(at.group, groups, K) * (GEMM_KSTEP * 2);
-    bias_row = bias ? bias + (size_t)at.group * N : nullptr;
-  } else {
-    const int logical = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int per_group = GROUP_M * tiles_n, group = logical / per_group, in = logical - group * per_group;
-    const int group_rows = min(GROUP_M, tiles_m - group * GROUP_M);
-    tn = in / group_rows, tm = group * GROUP_M + in - tn * group_rows;
-    n0 = tn * BN;
-    rows_left = M - tm * BM;
-    row_at = (size_t)tm * BM;
-    b_at = n0;
-    bias_row = bias;
-  }
-  uint16_t* c_tile = C + row_at * N;
+  auto find_tile = [&]() __attribute__((always_inline)) {  // (GROUPED: nobody uses LDS, and there is a tile if tile < total_tiles)
+    if constexpr (GROUPED) {
+      const GroupTile at = find_group_tile<512, BM>(tile, rows_of_group, groups, max_rows, tiles_n, compact, (int*)tile_lds);
+      total_tiles = at.total;
+      if (tile >= at.total) return;
+      lds_barrier();
+      n0 = at.tn * BN;
+      rows_left = at.rows;
+      row_at = at.row_at;
+      b_at = (size_t)at.group * N + n0;
+      k_first = first_kstep(at.group, groups, K) * (GEMM_KSTEP * 2);
+      bias_row = bias ? bias + (size_t)at.group * N : nullptr;
+    } else {
+      const int logical = xcd_contiguous(tile, total_tiles);
+      const int per_group = GROUP_M * tiles_n, group = logical / per_group, in = logical - group * per_group;
+      const int group_rows = min(GROUP_M, tiles_m - group * GROUP_M);
+      tn = in / group_rows, tm = group * GROUP_M + in - tn * group_rows;
+      n0 = tn * BN;
+      rows_left = M - tm * BM;
+      row_at = (size_t)tm * BM;
+      b_at = n0;
+      bias_row = bias;
+    }
+  };
 
   // As in dense_gemm_kernel: rows past the end of a matrix read as zeros (they lie past the extent), and
   // so do the vectors past the end of a row in the last step and everything past the last step.
-  const b128 abuf = buffer_words(A + row_at * row_vecs, min(BM, rows_left) * row_bytes);
-  const b128 bbuf = buffer_words(B + b_at * row_vecs, min(BN, N - n0) * row_bytes);
-  const int sub = lane >> 3;
-  auto vec_of = [&](int row) { return (lane & 7) ^ ((row >> 1) & 7); };
-  auto a_row = [&](int i) { return (i * 8 + wave) * 8 + sub; };
-  auto b_row = [&](int i) { return (i * 8 + wave) * 8 + sub; };
+  b128 abuf, bbuf;
+  // Load i of a wave takes rows i * 64 + wave * 8 .. + 7, and a lane the vector that belongs at its place: the same for all i.
+  auto vec_of = [=](int l) { return (l & 7) ^ (((wave * 8 + (l >> 3)) >> 1) & 7); };
   int aoff[LA], boff[LB];
-#pragma unroll
-  for (int i = 0; i < LA; ++i) aoff[i] = a_row(i) * row_bytes + vec_of(a_row(i)) * 16;
-#pragma unroll
-  for (int i = 0; i < LB; ++i) boff[i] = b_row(i) * row_bytes + vec_of(b_row(i)) * 16;
   auto a_range = [&](int step) __attribute__((always_inline)) {  // before the rows of a step near the end are asked for
     if (step == steps - 1) {
 #pragma unroll
-      for (int i = 0; i < LA; ++i) aoff[i] += vec_of(a_row(i)) >= tail_vecs ? OUT_OF_RANGE : 0;
+      for (int i = 0; i < LA; ++i) aoff[i] += vec_of(lane) >= tail_vecs ? OUT_OF_RANGE : 0;
     } else if (step >= steps) {
 #pragma unroll
       for (int i = 0; i < LA; ++i) aoff[i] = OUT_OF_RANGE;
@@ -2844,7 +2841,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   auto b_range = [&](int step, int from, int to) __attribute__((always_inline)) {
     if (step == steps - 1) {
 #pragma unroll
-      for (int i = from; i < to; ++i) boff[i] += vec_of(b_row(i)) >= tail_vecs ? OUT_OF_RANGE : 0;
+      for (int i = from; i < to; ++i) boff[i] += vec_of(lane) >= tail_vecs ? OUT_OF_RANGE : 0;
     } else if (step >= steps) {
 #pragma unroll
       for (int i = from; i < to; ++i) boff[i] = OUT_OF_RANGE;
@@ -2854,11 +2851,10 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) b128*)tile_lds;
   const unsigned a_base = lds0 + wave * 1024, b_base = lds0 + B_AT + wave * 1024;
   // byte of a row at which the next requested step begins
-  int a_soff = GROUPED ? k_first : 0, b_soff = a_soff;
-  unsigned a_fill = 0, b_fill = 0;     // buffer (as a byte offset) that the next requested step goes to
-  // buffer of the step being multiplied (HALVES: the place of the half that holds this wave's columns)
-  unsigned a_use = 0, b_use = HALVES ? (wn >> 1) * HALF_BYTES : 0;
-  [[maybe_unused]] int half_soff[2] = {b_soff, b_soff};
+  int a_soff, b_soff;
+  [[maybe_unused]] int half_soff[2];
+  unsigned a_fill, b_fill;  // buffer (as a byte offset) that the next requested step goes to
+  unsigned a_use, b_use;    // buffer of the step being multiplied (HALVES: the place of the half that holds this wave's columns)
   auto next_a = [](unsigned at) { return at == (NA - 1) * A_BYTES ? 0u : at + A_BYTES; };
   auto next_b = [](unsigned at) {
     return at + B_BYTES < HB * HALF_BYTES ? at + B_BYTES : at + B_BYTES - HB * HALF_BYTES;
@@ -2903,17 +2899,18 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   // repeating a row, 8192 x 8192 x 3696 took 2 % longer.)
   constexpr int AHEAD_STEPS = 4;
   typedef const __attribute__((address_space(1))) char* global_bytes;
-  [[maybe_unused]] const global_bytes touch_base = (global_bytes)(first_group ? A + row_at * row_vecs : B + b_at * row_vecs);
+  [[maybe_unused]] global_bytes touch_base = nullptr;
   [[maybe_unused]] unsigned touch_off = 0;
   [[maybe_unused]] uint32_t touched = 0;
   [[maybe_unused]] bool touches = false;
-  if constexpr (AHEAD) {
+  auto aim_touches = [&]() __attribute__((always_inline)) {
     constexpr int A_EACH = BM / 8 / 4, B_EACH = BN / GROUP_M / 4;  // rows of a wave of either group
+    touch_base = (global_bytes)(first_group ? A + row_at * row_vecs : B + b_at * row_vecs);
     const int a_row = min((tn & 7) * (BM / 8) + wave * A_EACH + lane, rows_left - 1);
     const int b_row = min((tm & (GROUP_M - 1)) * (BN / GROUP_M) + (wave - 4) * B_EACH + lane, N - n0 - 1);
     touches = lane < (first_group ? A_EACH : B_EACH);  // (lanes of every wave: its waits count the load)
     touch_off = (unsigned)(first_group ? a_row : b_row) * row_bytes;
-  }
+  };
   auto touch = [&](int step) __attribute__((always_inline)) {
     if constexpr (AHEAD) {
       global_bytes at = touch_base + min(step, steps - 1) * (GEMM_KSTEP * 2);
@@ -2937,7 +2934,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
     b_frag[s] = lds + B_AT + ((HALVES ? wn & 1 : wn) * TN * 16 + r) * 128 + ((s * 4 + q) ^ swz) * 16;
   }
   b128 af[TM], bf[TN];
-  f32x4 acc[TM][TN] = {};
+  f32x4 acc[TM][TN];
   auto read_frags = [&](auto bands, int slice) __attribute__((always_inline)) {
     const char* ap = a_frag[slice] + a_use;
     const char* bp = b_frag[slice] + b_use;
@@ -3002,24 +2999,37 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
       if (first_group) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER) : "memory");
     });
   };
-  if constexpr (HALVES) {
-    b_range(0, 0, LB);
-    load_half(lower);
-    load_half(upper);
-    a_range(0);
-    load_a();
-    b_range(1, 0, LB / 2);
-    load_half(lower);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LB / 2) : "memory");
-  } else {
-    unrolled<0, 2>([&](auto c) __attribute__((always_inline)) {
-      constexpr int at = decltype(c)::value;
-      if constexpr (at < NA - 1) { a_range(at); load_a(); }
-      if constexpr (at < NB - 1) { b_range(at, 0, LB); load_b(); }
-    });
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NA - 2) * LA + (NB - 2) * LB) : "memory");
-  }
-  if (!first_group) asm volatile("s_barrier" ::: "memory");  // one phase behind
+  constexpr int FIRST_YOUNGER = HALVES ? LB / 2 : (NA - 2) * LA + (NB - 2) * LB;  // of a tile's first loads, what its first step does without
+  auto begin_tile = [&]() __attribute__((always_inline)) {
+    abuf = buffer_words(A + row_at * row_vecs, min(BM, rows_left) * row_bytes);
+    bbuf = buffer_words(B + b_at * row_vecs, min(BN, N - n0) * row_bytes);
+    int at = lane;  // (worked out anew for each tile: kept over the loop the offsets would take registers that it needs)
+    asm volatile("" : "+v"(at));
+    const int off = (wave * 8 + (at >> 3)) * row_bytes + vec_of(at) * 16;
+#pragma unroll
+    for (int i = 0; i < LA; ++i) aoff[i] = off + i * 64 * row_bytes;
+#pragma unroll
+    for (int i = 0; i < LB; ++i) boff[i] = off + i * 64 * row_bytes;
+    a_soff = b_soff = half_soff[0] = half_soff[1] = GROUPED ? k_first : 0;
+    a_fill = b_fill = a_use = 0;
+    b_use = HALVES ? (wn >> 1) * HALF_BYTES : 0;
+    if constexpr (AHEAD) aim_touches();
+    if constexpr (HALVES) {
+      b_range(0, 0, LB);
+      load_half(lower);
+      load_half(upper);
+      a_range(0);
+      load_a();
+      b_range(1, 0, LB / 2);
+      load_half(lower);
+    } else {
+      unrolled<0, 2>([&](auto c) __attribute__((always_inline)) {
+        constexpr int at = decltype(c)::value;
+        if constexpr (at < NA - 1) { a_range(at); load_a(); }
+        if constexpr (at < NB - 1) { b_range(at, 0, LB); load_b(); }
+      });
+    }
+  };
   auto walk_k = [&](auto bands) __attribute__((always_inline)) {
     int step = 0;
     if constexpr (HALVES) {
@@ -3039,6 +3049,23 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
       }
     }
   };
+  find_tile();
+  if (tile >= total_tiles) return;
+  begin_tile();
+  auto clear = [&]() __attribute__((always_inline)) {  // (while the first loads are under way)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        acc[i][j] = f32x4{};
+        asm volatile("" : "+v"(acc[i][j]));
+      }
+  };
+  clear();
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FIRST_YOUNGER) : "memory");
+  for (;;) {
+  asm volatile("s_barrier" ::: "memory");
+  if (!first_group) asm volatile("s_barrier" ::: "memory");  // one phase behind
   // A group's tile multiplies only the bands of 32 rows that it has: a copy of the loop per number of them (a
   // condition on every band inside one loop takes registers that the loop needs)
   if constexpr (GROUPED) {
@@ -3061,17 +3088,28 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   // where there is work to write them behind (8192 x 8192 x 3696 375 / 372 / 369, 416 / 413 / 415), and plain where
   // that would cost the reader more than it gains (8192 x 8192 x 512 83 / 87 / 72, 123 / 127 / 128). Experts' results
   // are streamed, which leaves L2 to the operands: 32 x 256 rows, 4096 x 2048 145 / 144 / 137, 180 / 183 / 177.
-  {
-    const bool large = (long long)M * N > (32ll << 20), streams = GROUPED || (large && K >= 2048);
-    constexpr int VR = TN * 2, PITCH = TN * 32 + 16, ROWS_PER_READ = 64 / VR;
-    char* park = (char*)tile_lds + wave * (16 * PITCH);
-    const int ncol = n0 + wn * TN * 16;
-    uint32_t bias2[TN][2] = {};
-    if (bias_row) {
+  const bool large = (long long)M * N > (32ll << 20), streams = GROUPED || (large && K >= 2048);
+  constexpr int VR = TN * 2, PITCH = TN * 32 + 16, ROWS_PER_READ = 64 / VR, BAND_STORES = 16 / ROWS_PER_READ;
+  static_assert(8 * 16 * PITCH <= A_BYTES, "results leave through the last buffer of A, which a tile's first loads leave alone");
+  char* park = (char*)tile_lds + (NA - 1) * A_BYTES + wave * (16 * PITCH);
+  uint16_t* const c_tile = C + row_at * N;
+  const int ncol = n0 + wn * TN * 16, rows_out = rows_left;
+  const bool whole_columns = n0 + BN <= N, with_bias = bias_row != nullptr;
+  uint32_t bias2[TN][2] = {};
+  if (with_bias) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-        if (ncol + j * 16 < N) __builtin_memcpy(bias2[j], bias_row + ncol + j * 16 + q * 4, 8);
-    }
+    for (int j = 0; j < TN; ++j)
+      if (ncol + j * 16 < N) __builtin_memcpy(bias2[j], bias_row + ncol + j * 16 + q * 4, 8);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(bias2[j][0]), "+v"(bias2[j][1]));  // (waited for here, ahead of the loads below)
+  }
+  tile += gridDim.x;
+  const bool more = tile < total_tiles;
+  if (EARLY && more) {
+    find_tile();
+    begin_tile();
+  }
+  {
     int rrow = lane / VR, rvec = lane % VR;
     // (the places of all bands are worked out here: ahead of the loop over tiles they would take 60 registers)
     asm volatile("" : "+v"(rrow), "+v"(rvec));
@@ -3082,7 +3120,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
         const f32x4& c = acc[i][j];
         uint32_t two[2] = {Pair16<DT>::canonical(Pair16<DT>::round(c[0], c[1])),
                            Pair16<DT>::canonical(Pair16<DT>::round(c[2], c[3]))};
-        if (bias_row) {
+        if (with_bias) {
 #pragma unroll
           for (int e = 0; e < 2; ++e)
             two[e] = Pair16<DT>::canonical(Pair16<DT>::round(
@@ -3096,7 +3134,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
         const int row = p * ROWS_PER_READ + rrow;
         const b128 v = *(const b128*)(park + row * PITCH + rvec * 16);
         const int m = i * 32 + wm * 16 + row, n = ncol + rvec * 8;
-        if (m < rows_left && n < N) {
+        if (m < rows_out && n < N) {
           b128* const to = (b128*)(c_tile + (size_t)m * N + n);
           if (streams) row_store<STREAM>(to, v);
           else if (large) row_store<PLAIN>(to, v);
@@ -3105,8 +3143,23 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
       }
     }
   }
-  tile += gridDim.x;
-  } while (GROUPED && tile < total_tiles);
+  if (!more) return;
+  if constexpr (!EARLY) {
+    lds_barrier();  // the results are out of LDS
+    find_tile();
+    begin_tile();
+    clear();
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FIRST_YOUNGER) : "memory");
+    continue;
+  }
+  clear();
+  // The first step's rows: all but the youngest first loads and the stores behind them, of which there are as many as
+  // whole bands. (Loads and stores are counted in the order in which they were issued.)
+  constexpr int STORES = TM * BAND_STORES;
+  if (whole_columns && rows_out >= BM) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FIRST_YOUNGER + STORES) : "memory");
+  else if (whole_columns && rows_out >= BM / 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FIRST_YOUNGER + STORES / 2) : "memory");
+  else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FIRST_YOUNGER) : "memory");
+  }
 }
 
 // ---------------------------------------------------------------- exchange stand-in
@@ -4373,9 +4426,11 @@ int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, i
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + BN - 1) / BN;
   if (tiles_m * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
   const int grid = (int)(tiles_m * tiles_n);
+  // phased_gemm_kernel strides over its tiles: one workgroup per unit, or two of 128 x 128
+  const int phased_grid = std::min(grid, tile == 256 ? 256 : 512);
   if (const int rc = allow_large_lds()) return rc;
 #define LAUNCH_P(DT, TM, TN, AHEAD)                                                              \
-  phased_gemm_kernel<DT, TM, TN, 3, 4, AHEAD, false><<<grid, 512, phased_lds_bytes(TM, TN, 3, 4), st>>>( \
+  phased_gemm_kernel<DT, TM, TN, 3, 4, AHEAD, false><<<phased_grid, 512, phased_lds_bytes(TM, TN, 3, 4), st>>>( \
       (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n, \
       nullptr, 0, 0, 0)
   // Tiles of 128 x 128, at most one per unit: nobody is there to work while phased_gemm_kernel's waves wait for each

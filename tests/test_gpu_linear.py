@@ -219,3 +219,24 @@ def test_products_of_one_to_five_steps(m, n, k, dt):
     want = x.double() @ w.double().T
     assert torch.equal(out[1:m + 1].double(), want)
     assert (out[0] == 777.0).all() and (out[m + 1] == 777.0).all()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("k", [8, 64, 200, 448])
+@pytest.mark.parametrize("m,n", [(4100, 4128), (5120, 7200), (2100, 4128)], ids=["289 of 256", "580 of 256", "561 of 128"])
+def test_more_tiles_than_workgroups(m, n, k, bias, dt):
+    """Workgroups take a second and a third tile, whose first rows are asked for ahead of the results of the tile
+    before: whole and ragged tiles in front of them. Small integers, whose sums (|x @ w.T + b| <= 448 + 20 here at
+    most, and in fact far below 256) both types hold."""
+    print(f"linear m={m} n={n} k={k} bias={bias} {dt}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    x = torch.randint(-1, 2, (m, k), generator=g, device=DEV).to(dt)
+    w = torch.randint(-1, 2, (n, k), generator=g, device=DEV).to(dt)
+    b = torch.randint(-20, 21, (n,), generator=g, device=DEV).to(dt) if bias else None
+    want = x.float() @ w.float().T
+    assert want.abs().max() < 236
+    for _ in range(2):
+        out = torch.full((m, n), float("nan"), dtype=dt, device=DEV)
+        gemm_rs.local_product((x, w, b), out=out)
+        assert torch.equal(out.float(), want if b is None else want + b.float())
