@@ -275,6 +275,21 @@ class ExtBinding:
 
 
 _BINDINGS = {}
+_host_calls: Optional[dict] = None
+
+
+def host_calls() -> dict:
+    """What `csrc/host_calls.cpp` offers: `RankCalls`, `linear`, `job`. Empty where the extension has not been built
+    for this library: the Python code above the bindings then does every call by itself."""
+    global _host_calls
+    if _host_calls is None:
+        try:
+            from . import _ext
+
+            _host_calls = _ext.load().a2a_host_calls()
+        except (_lib.MoeA2AError, ImportError, AttributeError):
+            _host_calls = {}
+    return _host_calls
 
 
 def get(name: str):

@@ -70,7 +70,33 @@ def _need(t: torch.Tensor, dtype: torch.dtype, device, what: str) -> torch.Tenso
     return t
 
 
+class _PythonOnly:
+    """In the place of `RankCalls` (csrc/host_calls.cpp) where there is none: every call is refused."""
+
+    def __getattr__(self, name):
+        return _refused
+
+
+def _refused(*_):
+    return None
+
+
+def _rank_calls(shape: "_lib.Shape", cfg: MoEConfig, device):
+    make = _binding.host_calls().get("RankCalls")
+    if make is None or _raw_stream is None or device.index is None:
+        return _PythonOnly()
+    try:
+        return make(tuple(getattr(shape, f) for f, _ in _lib.Shape._fields_), cfg.in_dtype, cfg.out_dtype, device.index,
+                    _raw_stream)
+    except (TypeError, OverflowError):
+        return _PythonOnly()
+
+
 class HIPAllToAll:
+    """(The calls below are tried in native code first, `self._calls`, which refuses all but the plain forms; what
+    follows in each method takes every form, raises for the rest, and tells the native code which workspace buffers
+    the call used.)"""
+
     META_DIM = META_DIM  # global_exp, src_rank, src_token, src_k, pad
 
     def __init__(self, cfg: MoEConfig, rank: int, world_size: int, exchange=None, device=None,
@@ -91,6 +117,8 @@ class HIPAllToAll:
         self.binding = _binding.get(binding)  # raises if the native code has not been built
         self.shape = _lib.Shape(world_size, rank, cfg.num_experts, cfg.experts_per_token,
                                 cfg.hidden_dim, cfg.max_num_tokens)
+        self._calls = _rank_calls(self.shape, cfg, self.device)
+        self._learned = set()  # calls whose workspace buffers the native code knows
         # rows this rank can receive: every peer may route min(K, nle) entries of each token here
         self.max_rows_in = self.max_recv * min(cfg.experts_per_token, self.num_local_experts)
         self.max_rows_out = cfg.max_num_tokens * cfg.experts_per_token
@@ -115,6 +143,8 @@ class HIPAllToAll:
         # it when it is handed the very tensors that dispatch_recv returned
         self.reuse_placement = reuse_placement
         self._planned_for = None
+        self._plan_made_for = None  # what `_planned_for` is after a dispatch_recv
+        self._rows_in_hint = min(self.max_rows_in, self.max_rows_out)  # rows that arrived in the last dispatch
         self.long_stream_rows = None  # an int overrides both thresholds of LONG_STREAM_ROWS
         # A job of one rank exchanges with itself, so dispatch() and combine() can move rows straight to
         # their experts and back (moe_a2a_local_dispatch / _combine). Not where a token could have more
@@ -124,10 +154,40 @@ class HIPAllToAll:
                         and cfg.num_experts <= LOCAL_MAX_EXPERTS)
         self._dispatched_for = None  # (expert_meta, expert_num_tokens, tokens) of such a dispatch
 
+    @property
+    def long_stream_rows(self):
+        return self._long_stream_rows
+
+    @long_stream_rows.setter
+    def long_stream_rows(self, rows):
+        self._long_stream_rows = rows
+        self._forget()
+
+    @property
+    def reuse_placement(self):
+        return self._reuse_placement
+
+    @reuse_placement.setter
+    def reuse_placement(self, reuse):
+        self._reuse_placement = reuse
+        self._forget()
+
     # ------------------------------------------------------------------ workspace
+
+    def _forget(self) -> None:
+        """The native code's calls no longer use the buffers that they have learned."""
+        self._learned.clear()
+        self._calls.forget()
+
+    def _learn(self, key, method: str, *buffers) -> None:
+        if key not in self._learned:
+            self._learned.add(key)
+            getattr(self._calls, method)(*buffers)
 
     def _buf(self, name: str, shape: Tuple[int, ...], dtype: torch.dtype) -> torch.Tensor:
         if self._kept.get(name) != (shape, dtype):
+            if name in self._ws:
+                self._forget()
             self._ws[name] = torch.empty(shape, dtype=dtype, device=self.device)
             self._kept[name] = (shape, dtype)
         return self._ws[name]
@@ -161,6 +221,10 @@ class HIPAllToAll:
         """Group this rank's (token, k) entries by destination rank.
         Returns (send_counts int32[W], send_buf [T*K,H], send_meta [T*K,5])
         (+ send_slot int32[T*K] when `want_slots`)."""
+        if not want_slots:
+            T = self._calls.dispatch_send(dp_x, indices)
+            if T is not None:
+                return self._sent(T)
         cfg = self.cfg
         T, K = indices.shape
         if K != cfg.experts_per_token or dp_x.shape != (T, cfg.hidden_dim):
@@ -173,13 +237,18 @@ class HIPAllToAll:
         meta = self._buf("send_meta", (self.max_rows_out, META_DIM), torch.int32)
         slots = self._buf("send_slot", (self.max_rows_out,), torch.int32) if want_slots else None
         self.binding.dispatch_send(self.shape, dp_x, indices, T, buf, meta, counts, slots, _stream(self.device))
+        self._learn("send", "learn_send", counts, buf, meta)
         if want_slots:
             return counts, buf[:S], meta[:S], slots[:S]
+        return self._sent(T)
+
+    def _sent(self, T: int):
         out = self._send_views.get(T)
         if out is None:
             if len(self._send_views) >= 64:
                 self._send_views.clear()
-            out = self._send_views[T] = (counts, buf[:S], meta[:S])
+            S = T * self.cfg.experts_per_token
+            out = self._send_views[T] = (self._ws["send_counts"], self._ws["send_buf"][:S], self._ws["send_meta"][:S])
         return out
 
     def plan_send(self, indices: torch.Tensor):
@@ -202,6 +271,14 @@ class HIPAllToAll:
     def dispatch_recv(self, recv_counts, recv_buf, recv_meta, rows_hint: Optional[int] = None):
         """Received stream -> (expert_num_tokens[nle], expert_x[nle,max_recv,H],
         expert_meta[nle,max_recv,5]); rows past expert_num_tokens[le] are not written."""
+        hint = self._calls.dispatch_recv(recv_counts, recv_buf, recv_meta,
+                                         self.max_rows_out if rows_hint is None else rows_hint)
+        if hint is not None:
+            self._planned_for = self._plan_made_for
+            self._dispatched_for = None
+            self._rows_in_hint = hint
+            ws = self._ws
+            return ws["expert_num_tokens"], ws["expert_x"], ws["expert_meta"]
         cfg = self.cfg
         _need(recv_counts, torch.int32, self.device, "recv_counts")
         _need(recv_buf, cfg.in_dtype, self.device, "recv_buf")
@@ -226,13 +303,19 @@ class HIPAllToAll:
             pos = self._buf("row_position", (capacity,), torch.int32) if hint > self._long_from("dispatch") else None
             self.binding.dispatch_recv(self.shape, recv_buf, recv_meta, recv_counts, hint, num, ex, em, plan,
                                        _stream(self.device), pos)
-        self._planned_for = None if plan is None else (em.data_ptr(), num.data_ptr())
+        self._planned_for = self._plan_made_for = None if plan is None else (em.data_ptr(), num.data_ptr())
         self._dispatched_for = None
         self._rows_in_hint = hint
+        compact = self.layout == "compact"
+        self._learn("recv", "learn_recv", num, ex, em, self.expert_offsets if compact else None, plan,
+                    0x7fffffff if compact else self._long_from("dispatch"))
         return num, ex, em
 
     def expert_scale(self, expert_x, expert_num_tokens, rows_hint: Optional[int] = None):
         """Stand-in expert: `expert_x.to(out_dtype) * (1 + rank)` on the valid rows."""
+        ey = self._calls.expert_scale(expert_x, expert_num_tokens, self._rows_in_hint if rows_hint is None else rows_hint)
+        if ey is not None:
+            return ey
         cfg = self.cfg
         _need(expert_x, cfg.in_dtype, self.device, "expert_x")
         _need(expert_num_tokens, torch.int32, self.device, "expert_num_tokens")
@@ -242,6 +325,7 @@ class HIPAllToAll:
             self.binding.expert_scale_compact(self.shape, expert_x, expert_num_tokens, hint, ey, _stream(self.device))
         else:
             self.binding.expert_scale(self.shape, expert_x, expert_num_tokens, hint, ey, _stream(self.device))
+        self._learn("scale", "learn_scale", ey)
         return ey
 
     def expert_gemm(self, expert_x, expert_num_tokens, weights, bias=None, rows_hint: Optional[int] = None,
@@ -260,6 +344,11 @@ class HIPAllToAll:
         The order in which float32 sums are formed depends on the shape and, where in_dim is a multiple
         of 2048, on which of the rank's experts it is: the same expert can give other last bits in a job
         of another number of ranks. `rows_hint` changes no bit."""
+        if out is None:
+            got = self._calls.expert_gemm(expert_x, expert_num_tokens, weights, bias,
+                                          self._rows_in_hint if rows_hint is None else rows_hint)
+            if got is not None:
+                return got
         nle = self.num_local_experts
         dt = expert_x.dtype
         if dt not in _binding._DT:
@@ -281,7 +370,8 @@ class HIPAllToAll:
             if tuple(bias.shape) != (nle, out_dim):
                 raise ValueError(f"bias must be [{nle}, {out_dim}], got {tuple(bias.shape)}")
         hint = self._default_rows_in(rows_hint)
-        if out is None:
+        own = out is None
+        if own:
             name = f"expert_out_{out_dim}"
             if name in self._ws and self._ws[name].data_ptr() == expert_x.data_ptr():
                 name += "_b"  # a layer of equal width reading the buffer the one before it wrote
@@ -292,12 +382,18 @@ class HIPAllToAll:
                 raise ValueError(f"out must be {list(rows_shape) + [out_dim]} and not the input")
         gemm = self.binding.expert_gemm_compact if compact else self.binding.expert_gemm
         gemm(self.shape, expert_x, expert_num_tokens, hint, weights, bias, out, _stream(self.device))
+        if own:
+            self._learn(name, "learn_gemm", out, name.endswith("_b"))
         return out
 
     def combine_send(self, expert_meta, expert_y, expert_num_tokens, rows_hint: Optional[int] = None):
         """Expert-major results -> rows grouped by origin rank.
         Returns (back_counts int32[W], back_buf [max_rows_in,H], back_meta [max_rows_in,5]);
         the first sum(back_counts) rows are valid."""
+        if self._calls.combine_send(expert_meta, expert_y, expert_num_tokens,
+                                    self._rows_in_hint if rows_hint is None else rows_hint, self._planned_for):
+            ws = self._ws
+            return ws["back_counts"], ws["back_buf"], ws["back_meta"]
         cfg = self.cfg
         _need(expert_meta, torch.int32, self.device, "expert_meta")
         _need(expert_y, cfg.out_dtype, self.device, "expert_y")
@@ -321,6 +417,7 @@ class HIPAllToAll:
         send = self.binding.combine_send_compact if compact else self.binding.combine_send
         send(self.shape, expert_y, expert_meta, expert_num_tokens, min(hint, self.max_rows_in), buf, meta, counts,
              plan, _stream(self.device))
+        self._learn("back" if plan is None else "back by plan", "learn_back", counts, buf, meta, self._ws.get("send_back_plan"))
         return counts, buf, meta
 
     def combine_recv(self, out_tokens, weights, ret_counts, ret_buf, ret_meta, accumulate: bool = True,
@@ -335,6 +432,9 @@ class HIPAllToAll:
         src_k) pair may arrive more than once (the reference, all2all/reference.py:227-232, adds
         every arriving row) says so with `unique_pairs=False`; the rows are then found by scanning
         whatever the length, and every one of them is added."""
+        if unique_pairs and self._calls.combine_recv(out_tokens, weights, ret_counts, ret_buf, ret_meta, accumulate,
+                                                     self._long_from("combine")):
+            return out_tokens
         cfg = self.cfg
         _need(out_tokens, cfg.out_dtype, self.device, "out_tokens")
         _need(weights, torch.float32, self.device, "weights")
@@ -359,7 +459,7 @@ class HIPAllToAll:
     def _default_rows_in(self, rows_hint):
         if rows_hint is not None:
             return int(rows_hint)
-        return int(getattr(self, "_rows_in_hint", min(self.max_rows_in, self.max_rows_out)))
+        return int(self._rows_in_hint)
 
     # ------------------------------------------------------------------ reference surface
 
@@ -369,6 +469,13 @@ class HIPAllToAll:
             raise RuntimeError("dispatch() of a job with several ranks needs the exchange its ranks share "
                                "(LocalExchange on one GPU); or use the halves, or LocalWorld")
         if self._direct and type(self.exchange) is LocalExchange and self.exchange.world_size == 1:
+            T = self._calls.direct_dispatch(dp_x, indices)
+            if T is not None:
+                self._planned_for = None
+                self._dispatched_for = (*self._direct_key, T)
+                self._rows_in_hint = T * self.cfg.experts_per_token
+                ws = self._ws
+                return ws["expert_num_tokens"], ws["expert_x"], ws["expert_meta"]
             S = indices.shape[0] * self.cfg.experts_per_token
             if self.layout == "padded" or S <= self.compact_rows:
                 return self._direct_dispatch(dp_x, indices, S)
@@ -395,8 +502,10 @@ class HIPAllToAll:
         self.binding.local_dispatch(self.shape, (dp_x,), (indices,), compact, where, num,
                                     self.expert_offsets if compact else None, ex, em, False, _stream(self.device))
         self._planned_for = None
-        self._dispatched_for = (em.data_ptr(), num.data_ptr(), T)
+        self._direct_key = (em.data_ptr(), num.data_ptr())
+        self._dispatched_for = (*self._direct_key, T)
         self._rows_in_hint = S
+        self._learn("direct", "learn_direct", num, ex, em, where, self.expert_offsets if compact else None)
         return num, ex, em
 
     def combine(self, out_tokens, weights, expert_meta, expert_y, expert_num_tokens):
@@ -404,9 +513,13 @@ class HIPAllToAll:
         if self.exchange is None:
             raise RuntimeError("combine() of a job with several ranks needs the exchange its ranks share "
                                "(LocalExchange on one GPU); or use the halves, or LocalWorld")
-        if self._dispatched_for is not None and self._direct_combine(out_tokens, weights, expert_meta, expert_y,
-                                                                     expert_num_tokens):
-            return out_tokens
+        if self._dispatched_for is not None:
+            if (type(self.exchange) is LocalExchange
+                    and self._calls.direct_combine(out_tokens, weights, expert_meta, expert_y, expert_num_tokens,
+                                                   self._dispatched_for)):
+                return out_tokens
+            if self._direct_combine(out_tokens, weights, expert_meta, expert_y, expert_num_tokens):
+                return out_tokens
         counts, buf, meta = self.combine_send(expert_meta, expert_y, expert_num_tokens)
         rc, rb, rm, _ = self.exchange.deliver(self, "combine", counts, buf, meta)
         return self.combine_recv(out_tokens, weights, rc, rb, rm, accumulate=True)

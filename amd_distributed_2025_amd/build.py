@@ -7,7 +7,7 @@
 GPU is needed to build.
 
 `build_extension()` compiles the torch::Tensor wrappers of
-`csrc/moe_a2a_torch.cpp` with `torch.utils.cpp_extension.load_inline`, the way
+`csrc/moe_a2a_torch.cpp` and the native calls of `csrc/host_calls.cpp` with `torch.utils.cpp_extension.load_inline`, the way
 the reference's submissions build their kernels (all2all/hipv8.py:241-252), into
 `_ext/moe_a2a_torch.so`, linked against `libmoe_a2a.so`. The build directory is
 in the package so that the module travels with the tree.
@@ -25,6 +25,7 @@ SOURCE = PKG_DIR / "csrc" / "moe_a2a.hip"
 HEADERS = [PKG_DIR / "csrc" / "tile_rules.h", REPO_DIR / "include" / "moe_a2a.h"]
 LIBRARY = PKG_DIR / "libmoe_a2a.so"
 EXT_SOURCE = PKG_DIR / "csrc" / "moe_a2a_torch.cpp"
+CALLS_SOURCE = PKG_DIR / "csrc" / "host_calls.cpp"
 EXT_DIR = PKG_DIR / "_ext"
 EXT_NAME = "moe_a2a_torch"
 # the wrappers load_inline binds, one per entry point of the C ABI
@@ -32,6 +33,9 @@ EXT_FUNCTIONS = ["a2a_version", "a2a_dispatch_send", "a2a_plan_send", "a2a_dispa
                  "a2a_combine_recv", "a2a_expert_scale", "a2a_expert_gemm", "a2a_linear", "a2a_exchange_local",
                  "a2a_exchange_gather_local", "a2a_dispatch_recv_compact", "a2a_expert_scale_compact",
                  "a2a_expert_gemm_compact", "a2a_combine_send_compact", "a2a_local_dispatch", "a2a_local_combine"]
+
+# and the calls of the class surface in native code
+EXT_CALLS = ["a2a_host_calls"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -92,8 +96,8 @@ def build_extension(verbose: bool = False) -> Path:
     EXT_DIR.mkdir(exist_ok=True)
     load_inline(
         name=EXT_NAME,
-        cpp_sources=[EXT_SOURCE.read_text()],
-        functions=EXT_FUNCTIONS,
+        cpp_sources=[EXT_SOURCE.read_text(), CALLS_SOURCE.read_text()],
+        functions=EXT_FUNCTIONS + EXT_CALLS,
         extra_cflags=["-O2", "-std=c++17"],
         extra_include_paths=[str(REPO_DIR / "include")],
         # $ORIGIN/.. is the package directory as seen from _ext/ ($$ is ninja's escape for $)

@@ -18,7 +18,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 from . import _binding
-from .all2all import _stream
+from .all2all import _raw_stream, _stream
 
 input_t = Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]
 
@@ -53,6 +53,11 @@ def local_product(data: input_t, out: Optional[torch.Tensor] = None, binding: st
     """`matmul(input, weight.T)` rounded to the 16-bit type, then `+ bias` rounded again
     (gemm-rs/reference.py:54-57), as one launch. Returns [M, N]."""
     inp, weight, bias = data
+    if out is None and binding in ("ctypes", "ext") and _raw_stream is not None:
+        native = _binding.host_calls().get("linear")  # (refuses all but the plain forms)
+        got = native and native(_raw_stream, inp, weight, bias)
+        if got is not None:
+            return got
     if inp.dim() != 2 or weight.dim() != 2 or inp.shape[1] != weight.shape[1]:
         raise ValueError(f"input [M, K] and weight [N, K] expected, got {tuple(inp.shape)} and {tuple(weight.shape)}")
     if inp.dtype not in (torch.float16, torch.bfloat16):

@@ -30,7 +30,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 import torch
 
 from . import _binding, _lib
-from .all2all import LOCAL_MAX_EXPERTS, LOCAL_MAX_K, LOCAL_MAX_RANKS, LocalWorld, _need, _stream
+from .all2all import LOCAL_MAX_EXPERTS, LOCAL_MAX_K, LOCAL_MAX_RANKS, LocalWorld, _need, _raw_stream, _stream
 from .task import MoEConfig, RankTestData, input_t, output_t
 
 _peers: Optional[Sequence[input_t]] = None
@@ -148,6 +148,12 @@ def _run_direct(cfg: MoEConfig, world_size: int, everyone: Sequence[RankTestData
     return [y]
 
 
+def _native_job(cfg, world_size, inputs, own, rank, every_rank):
+    """`_run_direct` in native code (csrc/host_calls.cpp): one rank's result or all of them; None where it refuses."""
+    native = _binding.host_calls().get("job") if _raw_stream is not None else None
+    return native and native(_raw_stream, cfg, world_size, inputs, own, rank, every_rank)
+
+
 def _there(d: RankTestData, device: torch.device) -> RankTestData:
     index = device.index
     if d.x.get_device() == index and d.indices.get_device() == index and d.weights.get_device() == index:
@@ -159,6 +165,9 @@ def custom_kernel_job(inputs: Sequence[input_t]) -> list:
     """Every rank's `custom_kernel` result from ONE step of the job: what W processes calling
     `custom_kernel` at the same time produce together. `inputs[r]` is rank r's tuple."""
     cfg, first, _, world_size = inputs[0]
+    ys = _native_job(cfg, world_size, inputs, None, 0, True)
+    if ys is not None:
+        return ys
     device = first.x.device
     if device.type != "cuda":
         raise RuntimeError("custom_kernel needs its inputs on a GPU; this path has no CPU fallback")
@@ -174,6 +183,11 @@ def custom_kernel_job(inputs: Sequence[input_t]) -> list:
 
 def custom_kernel(data: input_t) -> output_t:
     cfg, rank_data, rank, world_size = data
+    peers = [data] if world_size == 1 else _peers
+    if peers is not None:
+        y = _native_job(cfg, world_size, peers, rank_data, rank, False)
+        if y is not None:
+            return y
     device = rank_data.x.device
     if device.type != "cuda":
         raise RuntimeError("custom_kernel needs its inputs on a GPU; this path has no CPU fallback")

@@ -1,0 +1,53 @@
+"""csrc/host_calls.cpp without a GPU: whatever is not a plain tensor on the rank's GPU is refused before anything is
+launched, and the class surface does without the extension."""
+import pytest
+import torch
+
+from amd_distributed_2025_amd import _binding, all2all
+
+ROWS, INTS = torch.zeros(4, 16, dtype=torch.bfloat16), torch.zeros(4, 2, dtype=torch.int32)
+ODD = [ROWS, INTS, None, 3, -1, 2 ** 70, "x", (1, 2), torch.zeros(0), torch.zeros(4, 16, device="meta"), torch.zeros(2, 2).to_sparse()]
+CALLS = {"dispatch_send": 2, "dispatch_recv": 4, "expert_scale": 3, "expert_gemm": 5, "combine_send": 5, "combine_recv": 7,
+         "direct_dispatch": 2, "direct_combine": 6}
+
+
+@pytest.fixture()
+def calls():
+    def stream(device):
+        raise AssertionError("nothing is launched")
+
+    c = _binding.host_calls()["RankCalls"]((1, 0, 8, 2, 16, 4), torch.bfloat16, torch.bfloat16, 0, stream)
+    meta = torch.zeros(8, 5, dtype=torch.int32)
+    num, ex = torch.zeros(8, dtype=torch.int32), torch.zeros(8, 4, 16, dtype=torch.bfloat16)
+    assert c.learn_send(num, ROWS, meta) and c.learn_recv(num, ex, meta, None, None, 100) and c.learn_scale(ex)
+    assert c.learn_back(num, ROWS, meta, None) and c.learn_direct(num, ex, meta, num, None) and c.learn_gemm(ex, False)
+    return c
+
+
+@pytest.mark.parametrize("name", CALLS)
+def test_calls_refuse_what_is_not_on_the_gpu(calls, name):
+    call = getattr(calls, name)
+    for shift in range(len(ODD)):
+        assert call(*[ODD[(i * 3 + shift) % len(ODD)] for i in range(CALLS[name])]) is None
+        assert call(*[ODD[shift]] * CALLS[name]) is None
+    for n in (0, CALLS[name] - 1, CALLS[name] + 1):
+        with pytest.raises(TypeError):
+            call(*[ROWS] * n)
+    calls.forget()
+    assert call(*[ROWS] * CALLS[name]) is None
+
+
+def test_functions_refuse_too():
+    f = _binding.host_calls()
+    for odd in ODD:
+        assert f["linear"](None, odd, ROWS, None) is None and f["linear"](None, ROWS, odd, odd) is None
+        assert f["job"](None, odd, 1, [odd], None, 0, True) is None
+        assert f["job"](None, odd, odd, odd, odd, odd, odd) is None
+    with pytest.raises(TypeError):
+        _binding.host_calls()["RankCalls"]((1, 0, 8), torch.bfloat16, torch.bfloat16, 0, None)
+
+
+def test_without_the_extension():
+    """Every call is refused, so that the Python code does it."""
+    none = all2all._PythonOnly()
+    assert none.dispatch_send(ROWS, INTS) is None and none.forget() is None and none.learn_send(1, 2, 3) is None
