@@ -2156,6 +2156,14 @@ __global__ __launch_bounds__(64 * GW, GW > 4 || D > 3 ? 1 : TJ == 1 ? 4 : TJ == 
 // turned into MFMA layout through LDS private to the wave: no barrier in the loop), and keeps
 // partial sums in registers. At the end the partial sums meet in LDS and are added in a fixed
 // order (wave 0 + 1 + 2 + ...), so results do not depend on scheduling.
+// What bounds it: with more than 32 rows, what a unit can take in (a workgroup of 64 x 7168 x 2304 fetches 442 KB,
+// two thirds of it token rows out of L2, and passes them all through LDS); with fewer, HBM or, on few columns, the
+// trips of a wave. Of both, what it does not have to do counts: with waits that leave the younger step under way (the
+// order of the loads is pinned, or the compiler waits for all of them), no loads past the last step, fragments read
+// ahead of the MFMAs, and the final sums shared out over all waves: 64 x 7168 x 2304 11.1 -> 9.7 us, x 4608 23.5 -> 19.8,
+// 64 x 2048 x 4608 16.2 -> 13.1, 16 x 7168 x 2304 8.8 -> 7.5, 1 x 4096 x 4096 9.4 -> 7.9, 64 x 8192 x 8192 36.5 -> 31.7.
+// (16 x 16384 x 2048 15.4 -> 15.6: one workgroup per unit instead of two, for the registers.) A third step under way
+// does not fit the registers beside 64 rows, and changes nothing with fewer.
 
 template <int DT, int TJ, int KW, bool APART>
 __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
@@ -2189,89 +2197,103 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
 
   f32x16 acc[TJ] = {};
   b128 wv[2][4], xv[2][XL];
-  auto load = [&](int set, int step) {
-    const int at = min(step, steps - 1);  // past the end: the last step again, unused
-    const bool last = at == steps - 1;
-    const int k = at + first_step, soff = (APART && k >= steps ? k - steps : k) * (GEMM_KSTEP * 2);
+  int woff[2];  // (rows 16 apart take the same vector)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = sub + 8 * i, vec = vec_of(row);
-      wv[set][i] = __builtin_amdgcn_raw_buffer_load_b128(
-          wbuf, row * row_bytes + vec * 16 + (last && vec >= tail_vecs ? OUT_OF_RANGE : 0), soff, 0);
-    }
+  for (int i = 0; i < 2; ++i) {
+    const int row = sub + 8 * i;
+    woff[i] = row * row_bytes + vec_of(row) * 16;
+  }
+  auto load = [&](int set, int step) __attribute__((always_inline)) {
+    const int k = step + first_step, soff = (APART && k >= steps ? k - steps : k) * (GEMM_KSTEP * 2);
+    int off[2];  // (past the end of the rows in the last step: out of range, zeros)
 #pragma unroll
-    for (int i = 0; i < XL; ++i) {
-      const int row = sub + 8 * i, vec = vec_of(row);
-      xv[set][i] = __builtin_amdgcn_raw_buffer_load_b128(
-          xbuf, row * row_bytes + vec * 16 + (last && vec >= tail_vecs ? OUT_OF_RANGE : 0), soff, 0);
-    }
+    for (int i = 0; i < 2; ++i) off[i] = woff[i] + (step == steps - 1 && vec_of(sub + 8 * i) >= tail_vecs ? OUT_OF_RANGE : 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      wv[set][i] = __builtin_amdgcn_raw_buffer_load_b128(wbuf, off[i & 1] + (i >> 1) * 16 * row_bytes, soff, 0);
+#pragma unroll
+    for (int i = 0; i < XL; ++i)
+      xv[set][i] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, off[i & 1] + (i >> 1) * 16 * row_bytes, soff, 0);
   };
   auto compute = [&](int set) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) wsl[wave][(sub + 8 * i) * 8 + slot] = wv[set][i];
 #pragma unroll
     for (int i = 0; i < XL; ++i) xsl[wave][(sub + 8 * i) * 8 + slot] = xv[set][i];
-    b128 a[4];
+    b128 a[4], tok[TJ][4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) a[q] = wsl[wave][r * 8 + ((kb * 4 + q) ^ read_swz)];
+    for (int q = 0; q < 4; ++q) {
+      a[q] = wsl[wave][r * 8 + ((kb * 4 + q) ^ read_swz)];
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) tok[j][q] = xsl[wave][(j * 32 + r) * 8 + ((kb * 4 + q) ^ read_swz)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int j = 0; j < TJ; ++j) {
-        if (j * 32 < live) {
-          const b128 tok = xsl[wave][(j * 32 + r) * 8 + ((kb * 4 + q) ^ read_swz)];
-          acc[j] = Mfma32x32x16<DT>::mma(a[q], tok, acc[j]);
-        }
-      }
+      for (int j = 0; j < TJ; ++j) acc[j] = Mfma32x32x16<DT>::mma(a[q], tok[j][q], acc[j]);
+    __builtin_amdgcn_sched_barrier(0);
   };
 
-  load(0, wave);
-  load(1, wave + KW);
-  for (int s = wave; s < steps; s += 2 * KW) {
+  // The wave's n steps (two at least: the launch sees to it), two of them under way. Nothing is asked for past the
+  // last one (a load out of range takes its turn in the address unit all the same: 0.7 us for the eight waves' loads of
+  // a step), and no load in the loop is conditional (the wait for a step has to know how many are younger).
+  const int n = (steps - wave + KW - 1) / KW;
+  auto load_step = [&](int set, int i) __attribute__((always_inline)) {
+    load(set, wave + i * KW);
+    __builtin_amdgcn_sched_barrier(0);  // (in this order, which the waits count on)
+  };
+  load_step(0, 0);
+  load_step(1, 1);
+  int i = 0;
+  for (; i + 4 <= n; i += 2) {
     compute(0);
-    load(0, s + 2 * KW);
-    if (s + KW < steps) compute(1);
-    load(1, s + 3 * KW);
+    load_step(0, i + 2);
+    compute(1);
+    load_step(1, i + 3);
+  }
+  compute(0);
+  if (n - i == 3) {
+    load_step(0, i + 2);
+    compute(1);
+    compute(0);
+  } else {
+    compute(1);
   }
 
-  // partial sums to LDS (a wave's region holds exactly its TJ x 16 floats per lane), then wave j
-  // adds up token tile j in the order of the waves and writes it out
-  float* mine = reinterpret_cast<float*>(xsl[wave]);
+  // Partial sums to LDS (a wave's region holds exactly its TJ x 16 floats per lane), 16 bytes at a time; then every wave
+  // adds up a share of the four quarters of the token tiles, each in the order of the waves, and writes it out.
+  f32x4* mine = reinterpret_cast<f32x4*>(xsl[wave]);
 #pragma unroll
   for (int j = 0; j < TJ; ++j)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) mine[(j * 16 + e) * 64 + lane] = acc[j][e];
+    for (int g = 0; g < 4; ++g) mine[(j * 4 + g) * 64 + lane] = f32x4{acc[j][g * 4], acc[j][g * 4 + 1], acc[j][g * 4 + 2], acc[j][g * 4 + 3]};
   __syncthreads();
-  if (wave < TJ && wave * 32 < live) {
-    const int j = wave;
-    float c[16];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      float sum = reinterpret_cast<const float*>(xsl[0])[(j * 16 + e) * 64 + lane];
+  for (int p = 0; p < (TJ * 4 + KW - 1) / KW; ++p) {
+    const int share = p * KW + wave, j = share % TJ, g = share / TJ;
+    if (g >= 4 || j * 32 >= live) continue;
+    f32x4 c = reinterpret_cast<const f32x4*>(xsl[0])[(j * 4 + g) * 64 + lane];
 #pragma unroll
-      for (int w = 1; w < KW; ++w)
-        sum = __fadd_rn(sum, reinterpret_cast<const float*>(xsl[w])[(j * 16 + e) * 64 + lane]);
-      c[e] = sum;
+    for (int w = 1; w < KW; ++w) {
+      const f32x4 more = reinterpret_cast<const f32x4*>(xsl[w])[(j * 4 + g) * 64 + lane];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) c[e] = __fadd_rn(c[e], more[e]);
     }
-    // this lane: token r of tile j, output columns n0 + g*8 + kb*4 + 0..3, g < 4
+    // this lane: token r of tile j, output columns n0 + g*8 + kb*4 + 0..3
     const int token = t0 + j * 32 + r;
     if (token < M) {
-      uint16_t* out = Y + (size_t)token * N + n0 + kb * 4;
+      uint32_t two[2] = {Pair16<DT>::canonical(Pair16<DT>::round(c[0], c[1])), Pair16<DT>::canonical(Pair16<DT>::round(c[2], c[3]))};
+      if (bias) {
+        uint32_t b2[2];
+        __builtin_memcpy(b2, bias + n0 + kb * 4 + g * 8, 8);
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        uint32_t two[2] = {Pair16<DT>::canonical(Pair16<DT>::round(c[g * 4 + 0], c[g * 4 + 1])),
-                           Pair16<DT>::canonical(Pair16<DT>::round(c[g * 4 + 2], c[g * 4 + 3]))};
-        if (bias) {
-          uint32_t b2[2];
-          __builtin_memcpy(b2, bias + n0 + kb * 4 + g * 8, 8);
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            two[h] = Pair16<DT>::canonical(Pair16<DT>::round(
-                __fadd_rn(Pair16<DT>::lo(two[h]), Pair16<DT>::lo(b2[h])),
-                __fadd_rn(Pair16<DT>::hi(two[h]), Pair16<DT>::hi(b2[h]))));
-        }
-        __builtin_memcpy(out + g * 8, two, 8);
+        for (int h = 0; h < 2; ++h)
+          two[h] = Pair16<DT>::canonical(Pair16<DT>::round(
+              __fadd_rn(Pair16<DT>::lo(two[h]), Pair16<DT>::lo(b2[h])),
+              __fadd_rn(Pair16<DT>::hi(two[h]), Pair16<DT>::hi(b2[h]))));
       }
+      __builtin_memcpy(Y + (size_t)token * N + n0 + kb * 4 + g * 8, two, 8);
     }
   }
 }

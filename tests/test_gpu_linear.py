@@ -240,3 +240,23 @@ def test_more_tiles_than_workgroups(m, n, k, bias, dt):
         out = torch.full((m, n), float("nan"), dtype=dt, device=DEV)
         gemm_rs.local_product((x, w, b), out=out)
         assert torch.equal(out.float(), want if b is None else want + b.float())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("m", [1, 32, 33, 64])
+@pytest.mark.parametrize("k", [512, 520, 768, 832, 1472, 1536, 1592, 2048, 2112, 2624, 3208, 4096])
+def test_few_rows_whatever_a_wave_has_to_walk(m, k, dt):
+    """Two to seven steps of 64 for each of the four or eight waves that share K, even and odd, the last one whole or
+    not, with a bias. Small integers, whose sums every order gives exactly and float32 holds; rounded once before the bias
+    and once after."""
+    n = 96
+    print(f"linear m={m} n={n} k={k} {dt}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + k)
+    x = torch.randint(-1, 2, (m, k), generator=g, device=DEV).to(dt)
+    w = torch.randint(-1, 2, (n, k), generator=g, device=DEV).to(dt)
+    b = torch.randint(-9, 10, (n,), generator=g, device=DEV).to(dt)
+    out = torch.full((m + 2, n), 777.0, dtype=dt, device=DEV)
+    gemm_rs.local_product((x, w, b), out=out[1:m + 1])
+    want = ((x.double() @ w.double().T).to(dt).double() + b.double()).to(dt)
+    assert torch.equal(out[1:m + 1], want)
+    assert (out[0] == 777.0).all() and (out[m + 1] == 777.0).all()
