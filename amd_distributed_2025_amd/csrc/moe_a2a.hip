@@ -1890,6 +1890,7 @@ template <> struct Mfma32x32x16<MOE_A2A_F16> {
 #define MOE_A2A_GEMM_DEPTH 2
 #endif
 constexpr int BUFFER_RAW_32BIT = 0x00020000;  // word 3 of a gfx9 buffer descriptor: raw buffer of 32-bit data
+constexpr int BUFFER_STREAM = 2;  // cache policy of a buffer load: nontemporal
 constexpr int GEMM_COLS = 128;   // output columns per workgroup (of four waves), 32 per wave
 constexpr int GEMM_KSTEP = 64;   // input elements per step: 8 vectors of 16 bytes per row
 #ifndef MOE_A2A_GEMM_DEPTH4
@@ -1911,8 +1912,9 @@ __device__ __forceinline__ int first_kstep(int g, int groups, int K) {
 // GW waves per workgroup, 32 output columns each: every workgroup of an expert pulls the expert's
 // token rows through its own L1, so wider workgroups halve that traffic (GW = 8: one workgroup of
 // 512 lanes per compute unit instead of two of 256).
+// STREAMED: the weights leave nothing behind in the caches (weights_past_the_cache, csrc/tile_rules.h).
 // TJ = 1: two waves per workgroup, and either many of those per unit (D = 2) or few with twice the lookahead.
-template <int DT, int TJ, int GW, int D>
+template <int DT, int TJ, int GW, int D, bool STREAMED>
 __global__ __launch_bounds__(64 * GW, GW > 4 || D > 3 ? 1 : TJ == 1 ? 4 : TJ == 2 ? MOE_A2A_GEMM_OCC : MOE_A2A_GEMM_OCC4) void expert_gemm_kernel(
     const b128* __restrict__ expert_x, const int* __restrict__ expert_num_tokens,
     const b128* __restrict__ weights, const uint16_t* __restrict__ bias, uint16_t* __restrict__ expert_y,
@@ -2049,7 +2051,7 @@ __global__ __launch_bounds__(64 * GW, GW > 4 || D > 3 ? 1 : TJ == 1 ? 4 : TJ == 
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         wv[set][i] = __builtin_amdgcn_raw_buffer_load_b128(wbuf, woff[i] + (last ? wpast[i & 1] : 0),
-                                                           k_bytes(at), 0);
+                                                           k_bytes(at), STREAMED ? BUFFER_STREAM : 0);
     };
     auto load_x = [&](int set, int step) {
       const int at = min(step, steps - 1);
@@ -2318,7 +2320,7 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
 // and consecutive numbers walk GROUP_M tile rows down before they step to the next tile column:
 // the 32 workgroups an XCD runs at a time share 4 row panels of A and 8 of B in its L2.
 
-template <int DT, int WM, int WN, int TM, int TN, bool GROUPED>
+template <int DT, int WM, int WN, int TM, int TN, bool GROUPED, bool STREAMED = false>
 __global__ __launch_bounds__(64 * WM * WN, 2) void dense_gemm_kernel(
     const b128* __restrict__ A, const b128* __restrict__ B, const uint16_t* __restrict__ bias,
     uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
@@ -2460,7 +2462,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void dense_gemm_kernel(
     } else {
 #pragma unroll
       for (int i = (q - 2) * (LB / 2); i < (q - 1) * (LB / 2); ++i)
-        gb[i] = __builtin_amdgcn_raw_buffer_load_b128(bbuf, off + i * rstep, soff, 0);
+        gb[i] = __builtin_amdgcn_raw_buffer_load_b128(bbuf, off + i * rstep, soff, STREAMED ? BUFFER_STREAM : 0);
     }
   };
   auto store_quarter = [&](int q, int buf) __attribute__((always_inline)) {
@@ -2671,10 +2673,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void dense_gemm_kernel(
 // 16 bytes per lane from a buffer into LDS at `base` + OFF + 16 * lane. The place travels in m0, which the compiler
 // sets (so that it knows what m0 holds); the instruction is written out, as the wait for it, through vmcnt, is the
 // caller's. One wait state between the two.
-template <int OFF>
+template <int OFF, bool STREAMED = false>
 __device__ __forceinline__ void load_to_lds(unsigned base, int voffset, b128 rsrc, int soffset) {
-  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               ::"{m0}"(base + OFF), "v"(voffset), "s"(rsrc), "s"(soffset) : "memory");
+  if constexpr (STREAMED)
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 ::"{m0}"(base + OFF), "v"(voffset), "s"(rsrc), "s"(soffset) : "memory");
+  else
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 ::"{m0}"(base + OFF), "v"(voffset), "s"(rsrc), "s"(soffset) : "memory");
 }
 // the descriptor of such a load, as __builtin_amdgcn_make_buffer_rsrc lays it out
 __device__ __forceinline__ b128 buffer_words(const void* p, int bytes) {
@@ -2788,7 +2794,7 @@ __device__ __forceinline__ GroupTile find_group_tile(int tile, const int* __rest
   return at;
 }
 
-template <int DT, int TM, int TN, int NA, int HB, bool AHEAD, bool GROUPED>
+template <int DT, int TM, int TN, int NA, int HB, bool AHEAD, bool GROUPED, bool STREAMED = false>
 __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
     const b128* __restrict__ A, const b128* __restrict__ B, const uint16_t* __restrict__ bias,
     uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
@@ -2893,7 +2899,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   auto load_b = [&]() __attribute__((always_inline)) {
     unrolled<0, LB>([&](auto c) __attribute__((always_inline)) {
       constexpr int i = decltype(c)::value;
-      load_to_lds<i * 8192>(b_base + b_fill, boff[i], bbuf, b_soff);
+      load_to_lds<i * 8192, STREAMED>(b_base + b_fill, boff[i], bbuf, b_soff);
     });
     b_fill = next_b(b_fill);
     b_soff += GEMM_KSTEP * 2;
@@ -2904,7 +2910,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
     constexpr int h = decltype(half)::value;
     unrolled<0, LB / 2>([&](auto c) __attribute__((always_inline)) {
       constexpr int i = decltype(c)::value;
-      load_to_lds<i * 8192>(b_base + b_fill, boff[h * (LB / 2) + i], bbuf, half_soff[h]);
+      load_to_lds<i * 8192, STREAMED>(b_base + b_fill, boff[h * (LB / 2) + i], bbuf, half_soff[h]);
     });
     b_fill = b_fill == (HB - 1) * HALF_BYTES ? 0u : b_fill + HALF_BYTES;
     half_soff[h] += GEMM_KSTEP * 2;
@@ -4347,10 +4353,16 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   const int col_tiles = (N + cols - 1) / cols;
   if ((max_rows / 64 + 1) * groups * col_tiles > INT_MAX / 2) return MOE_A2A_EINVAL;
   const int grid = mover_blocks(row_blocks * col_tiles);
-#define LAUNCH_G(DT, TJ, GW, D)                                                                       \
-  expert_gemm_kernel<DT, TJ, GW, D><<<grid, 64 * GW, 0, st>>>((const b128*)x, rows_of_group, (const b128*)w, \
-                                                              (const uint16_t*)bias, (uint16_t*)y, groups,  \
-                                                              (int)max_rows, N, K, col_tiles, compact)
+  const bool streamed = weights_past_the_cache(groups, N, K);
+#define LAUNCH_GS(DT, TJ, GW, D, S)                                                                   \
+  expert_gemm_kernel<DT, TJ, GW, D, S><<<grid, 64 * GW, 0, st>>>((const b128*)x, rows_of_group, (const b128*)w, \
+                                                                 (const uint16_t*)bias, (uint16_t*)y, groups,  \
+                                                                 (int)max_rows, N, K, col_tiles, compact)
+#define LAUNCH_G(DT, TJ, GW, D)                       \
+  do {                                                \
+    if (streamed) LAUNCH_GS(DT, TJ, GW, D, true);     \
+    else LAUNCH_GS(DT, TJ, GW, D, false);             \
+  } while (0)
 #define LAUNCH_GW(DT)                                             \
   do {                                                            \
     if (far_ahead) LAUNCH_G(DT, 1, 2, 4);                         \
@@ -4366,6 +4378,7 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   else LAUNCH_GW(MOE_A2A_F16);
 #undef LAUNCH_GW
 #undef LAUNCH_G
+#undef LAUNCH_GS
   return launch_status();
 }
 
@@ -4405,13 +4418,14 @@ int allow_large_lds() {
   auto allow = [&](const void* kernel, size_t bytes) {
     ok = ok && hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
   };
-  auto allow_grouped = [&](auto dtype) {
+  auto allow_grouped = [&](auto dtype, auto streamed) {
     constexpr int DT = decltype(dtype)::value;
-    allow((const void*)phased_gemm_kernel<DT, 10, 4, 2, 5, false, true>, phased_lds_bytes(10, 4, 2, 5));
-    allow((const void*)phased_gemm_kernel<DT, 8, 4, 2, 6, false, true>, phased_lds_bytes(8, 4, 2, 6));
-    allow((const void*)phased_gemm_kernel<DT, 6, 4, 2, 6, false, true>, phased_lds_bytes(6, 4, 2, 6));
-    allow((const void*)dense_gemm_kernel<DT, 2, 2, 2, 2, true>, dense_lds_bytes(128, 128));
-    allow((const void*)dense_gemm_kernel<DT, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
+    constexpr bool S = decltype(streamed)::value;
+    allow((const void*)phased_gemm_kernel<DT, 10, 4, 2, 5, false, true, S>, phased_lds_bytes(10, 4, 2, 5));
+    allow((const void*)phased_gemm_kernel<DT, 8, 4, 2, 6, false, true, S>, phased_lds_bytes(8, 4, 2, 6));
+    allow((const void*)phased_gemm_kernel<DT, 6, 4, 2, 6, false, true, S>, phased_lds_bytes(6, 4, 2, 6));
+    allow((const void*)dense_gemm_kernel<DT, 2, 2, 2, 2, true, S>, dense_lds_bytes(128, 128));
+    allow((const void*)dense_gemm_kernel<DT, 2, 2, 1, 2, true, S>, dense_lds_bytes(64, 128));
   };
   allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 4, false, false>, phased_lds_bytes(8, 4, 3, 4));
   allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 4, false, false>, phased_lds_bytes(8, 4, 3, 4));
@@ -4423,8 +4437,10 @@ int allow_large_lds() {
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
-  allow_grouped(std::integral_constant<int, MOE_A2A_BF16>{});
-  allow_grouped(std::integral_constant<int, MOE_A2A_F16>{});
+  allow_grouped(std::integral_constant<int, MOE_A2A_BF16>{}, std::false_type{});
+  allow_grouped(std::integral_constant<int, MOE_A2A_BF16>{}, std::true_type{});
+  allow_grouped(std::integral_constant<int, MOE_A2A_F16>{}, std::false_type{});
+  allow_grouped(std::integral_constant<int, MOE_A2A_F16>{}, std::true_type{});
   allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8, true>, skinny_lds_bytes(2, 8));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8, false>, skinny_lds_bytes(2, 8));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8, true>, skinny_lds_bytes(2, 8));
@@ -4501,22 +4517,29 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   if ((max_rows / BM + 1) * groups * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
   const int grid = mover_blocks((pairs + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
   if (const int rc = allow_large_lds()) return rc;
-  auto launch = [&](auto dtype_const) {
+  // (tiles of one row of tiles per group ask for its weights once; neighbours that ask for them too find them in L2)
+  const bool streamed = weights_past_the_cache(groups, N, K) && rows_hint <= (long long)groups * BM;
+  auto launch = [&](auto dtype_const, auto streamed_const) {
     constexpr int DT = decltype(dtype_const)::value;
+    constexpr bool S = decltype(streamed_const)::value;
     auto start = [&](auto kernel, int lanes, size_t lds_bytes) {
       kernel<<<grid, lanes, lds_bytes, st>>>((const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, 0, N, K,
                                              0, (int)tiles_n, rows_of_group, groups, (int)max_rows, compact);
     };
     auto phased = [&](auto kernel, size_t lds_bytes) { start(kernel, 512, lds_bytes); };
     auto dense = [&](auto kernel, size_t lds_bytes) { start(kernel, 256, lds_bytes); };
-    if (bands == 10) phased(phased_gemm_kernel<DT, 10, 4, 2, 5, false, true>, phased_lds_bytes(10, 4, 2, 5));
-    else if (bands == 8) phased(phased_gemm_kernel<DT, 8, 4, 2, 6, false, true>, phased_lds_bytes(8, 4, 2, 6));
-    else if (bands == 6) phased(phased_gemm_kernel<DT, 6, 4, 2, 6, false, true>, phased_lds_bytes(6, 4, 2, 6));
-    else if (bands == 4) dense(dense_gemm_kernel<DT, 2, 2, 2, 2, true>, dense_lds_bytes(128, 128));
-    else dense(dense_gemm_kernel<DT, 2, 2, 1, 2, true>, dense_lds_bytes(64, 128));
+    if (bands == 10) phased(phased_gemm_kernel<DT, 10, 4, 2, 5, false, true, S>, phased_lds_bytes(10, 4, 2, 5));
+    else if (bands == 8) phased(phased_gemm_kernel<DT, 8, 4, 2, 6, false, true, S>, phased_lds_bytes(8, 4, 2, 6));
+    else if (bands == 6) phased(phased_gemm_kernel<DT, 6, 4, 2, 6, false, true, S>, phased_lds_bytes(6, 4, 2, 6));
+    else if (bands == 4) dense(dense_gemm_kernel<DT, 2, 2, 2, 2, true, S>, dense_lds_bytes(128, 128));
+    else dense(dense_gemm_kernel<DT, 2, 2, 1, 2, true, S>, dense_lds_bytes(64, 128));
   };
-  if (dtype == MOE_A2A_BF16) launch(std::integral_constant<int, MOE_A2A_BF16>{});
-  else launch(std::integral_constant<int, MOE_A2A_F16>{});
+  auto launch_of = [&](auto dtype_const) {
+    if (streamed) launch(dtype_const, std::true_type{});
+    else launch(dtype_const, std::false_type{});
+  };
+  if (dtype == MOE_A2A_BF16) launch_of(std::integral_constant<int, MOE_A2A_BF16>{});
+  else launch_of(std::integral_constant<int, MOE_A2A_F16>{});
   return launch_status();
 }
 

@@ -12,6 +12,14 @@ constexpr int OUT_OF_RANGE = 0x40000000;
 
 bool tile_rows_in_range(long long rows, long long K) { return rows * K * 2 < OUT_OF_RANGE; }
 
+// Weights that the 256 MB behind L2 cannot hold are read with streaming (nontemporal) loads: they then push nothing out
+// of it on their way, which costs 5 to 10 % (us, plain / streaming, operands changing from call to call: 64 groups of 2
+// rows, 1024 x 2048, 268 MB 42.8 / 39.2, 2048 x 7168 134.9 / 119.7; 32 groups of 256 rows, 2048 x 4096 133.6 / 125.4,
+// of 100 rows 97.0 / 86.2; 32 of 63, 7168 x 7168 574 / 546). Smaller ones may still be there from the call before,
+// and streaming loads leave nothing behind: 32 groups, 1024 x 2048, 134 MB read again 20.2 / 25.6, 67 MB 12.4 / 14.4.
+// Where a group has several rows of tiles L2 has to keep its weights between them: 32 of 1000, 7168 x 2048 828 / 835.
+bool weights_past_the_cache(int groups, int N, int K) { return (double)groups * N * K * 2 >= 256.0 * (1 << 20); }
+
 // How a grouped product is cut: the height of its tiles in bands of 32 rows (10, 8, 6: phased_gemm_kernel, 256
 // columns; 4, 2: dense_gemm_kernel, 128 columns), 0 where rows of K are too long for any. `rows_hint` rows over all
 // groups are taken to be spread as uniform routing spreads them: a group's number is normal around the average.

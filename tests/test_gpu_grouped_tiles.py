@@ -82,6 +82,33 @@ def test_few_steps_on_the_ring_of_half_steps(K):
             assert (out[e, c:] == 7).all()
 
 
+# groups, K -> rows per group and the tile (0: a block that streams the weights) of weights of 256 MB and more at N = 7168,
+# which are read with loads that leave nothing in the caches: every kernel of the grouped product has such a form
+PAST_THE_CACHE = {(3, 6272): {20: 0, 50: 0, 60: 64, 100: 128, 150: 192}, (5, 3752): {8: 0, 30: 0, 230: 256, 300: 320}}
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("groups,K", PAST_THE_CACHE)
+def test_weights_that_the_cache_cannot_hold(groups, K, dt):
+    """Small integers, whose sums every order gives exactly (|sums| < 2^11 here, which float16 holds; bfloat16
+    rounds them once)."""
+    print(f"past the cache groups={groups} K={K} {dt}", flush=True)
+    N, T = 7168, 330
+    a = HIPAllToAll(MoEConfig(groups, 1, K, T, dt, dt), 0, 1, device=torch.device(DEV))
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x = torch.randint(-1, 2, (groups, T, K), generator=g, device=DEV).to(dt)
+    w = torch.randint(-1, 2, (groups, N, K), generator=g, device=DEV).to(dt)
+    b = torch.randint(-9, 10, (groups, N), generator=g, device=DEV).to(dt)
+    counts = [257, 0, 33, 321, 1][:groups]
+    num = torch.tensor(counts, dtype=torch.int32, device=DEV)
+    want = [((x[e, :c].double() @ w[e].double().T).to(dt).double() + b[e].double()).to(dt) for e, c in enumerate(counts)]
+    for rows in PAST_THE_CACHE[groups, K]:
+        out = a.expert_gemm(x, num, w, b, rows_hint=rows * groups, out=torch.full((groups, T, N), 7.0, dtype=dt, device=DEV))
+        for e, c in enumerate(counts):
+            assert torch.equal(out[e, :c], want[e]), (rows, e)
+            assert (out[e, c:] == 7).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 32, 2048), (33, 96, 4096), (64, 2080, 2048), (8, 1024, 6144), (64, 64, 8192)])
 def test_few_rows_whose_walks_of_K_start_apart(M, N, K):
     """`moe_a2a_linear` on at most 64 rows of a multiple of 2048 inputs: small integers, whose sums every order

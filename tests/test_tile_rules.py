@@ -7,7 +7,7 @@ from pathlib import Path
 import pytest
 
 from tests.test_gpu_expert_gemm import TILES_OF_NARROW
-from tests.test_gpu_grouped_tiles import FEW_STEPS, ROWS_FOR_TILE
+from tests.test_gpu_grouped_tiles import FEW_STEPS, PAST_THE_CACHE, ROWS_FOR_TILE
 
 CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
 
@@ -18,7 +18,8 @@ def rules(tmp_path_factory):
         pytest.skip("g++ not installed")
     src = tmp_path_factory.mktemp("rules") / "rules.cpp"
     src.write_text('#include "tile_rules.h"\n'
-                   'extern "C" int bands(long long rows_hint, int groups, int n, int k) { return grouped_tile_bands(rows_hint, groups, n, k); }\n')
+                   'extern "C" int bands(long long rows_hint, int groups, int n, int k) { return grouped_tile_bands(rows_hint, groups, n, k); }\n'
+                   'extern "C" int past(int groups, int n, int k) { return weights_past_the_cache(groups, n, k); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
                     str(src), "-o", str(lib)], check=True)
@@ -77,6 +78,15 @@ def test_the_tiles_that_the_gpu_tests_mean(rules, K):
 @pytest.mark.parametrize("K", FEW_STEPS)
 def test_the_tile_that_the_ring_of_half_steps_is_tested_on(rules, K):
     assert rules.bands(800 * 3, 3, 7168, K) == 10
+
+
+def test_weights_past_the_cache(rules):
+    """From 256 MB on (MB of 2^20 bytes), also where the product of the sizes does not fit 64 bits."""
+    assert rules.past(64, 1024, 2048) and not rules.past(64, 1024, 2040) and rules.past(2 ** 31 - 1, 2 ** 31 - 1, 2 ** 31 - 1)
+    for (groups, K), tiles in PAST_THE_CACHE.items():
+        assert rules.past(groups, 7168, K)
+        for rows, tile in tiles.items():
+            assert not tile or (32 * rules.bands(rows * groups, groups, 7168, K) == tile and rows <= tile)
 
 
 def test_the_second_tiles_that_the_gpu_tests_mean():
