@@ -175,16 +175,19 @@ PyObject* rank_forget(PyObject* self, PyObject*) {
     return nullptr;                                                       \
   }
 
-// A copy of the workspace with the tensors of one method filled in; arguments: tensors or None, in the order of `to`.
+// the workspace to change: a copy where a call in another thread is using it (calls come and go under the interpreter's lock)
+std::shared_ptr<Workspace> own(State& s) { return s.ws.use_count() == 1 ? s.ws : std::make_shared<Workspace>(*s.ws); }
+
+// The tensors of one method filled in; arguments: tensors or None, in the order of `to`.
 PyObject* learn(State& s, PyObject* const* a, std::initializer_list<Tensor Workspace::*> to, int64_t long_rows = -1) {
-  auto next = std::make_shared<Workspace>(*s.ws);
+  for (size_t i = 0; i < to.size(); ++i)
+    if (a[i] != Py_None && !plain(a[i])) REFUSE;
+  auto next = own(s);
   for (auto field : to) {
     if (*a == Py_None) {
       (*next).*field = Tensor();
     } else {
-      const Tensor* t = plain(*a);
-      if (!t) REFUSE;
-      (*next).*field = *t;
+      (*next).*field = *plain(*a);
     }
     ++a;
   }
@@ -311,7 +314,7 @@ PyObject* learn_gemm(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   State& s = state(self);
   const Tensor* out = plain(a[0]);
   if (!out || out->dim() < 2) REFUSE;
-  auto next = std::make_shared<Workspace>(*s.ws);
+  auto next = own(s);
   if (next->gemm.size() >= 16) next->gemm.clear();
   next->gemm.push_back({out->size(-1), a[1] == Py_True, *out});
   s.ws = std::move(next);

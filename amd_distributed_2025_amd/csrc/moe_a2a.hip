@@ -67,13 +67,12 @@ typedef unsigned int b128 __attribute__((ext_vector_type(4)));
 // THROUGH (device scope) writes on past L2 while the kernel runs. What a plain store leaves dirty there is written
 // back when the kernel ends, with nothing else going on: the 29 MB that stage 2 writes at the headline shape
 // (8 ranks, 2048 rows of 14 KB) cost 15.8 us plain, 14.7 through; the stand-in's rows of a whole job 44.5 and 42.9.
+// (Stage 2, whose waves write whole rows, is better off plain below 8 MB: 16 rows of 14 KB 4.1 / 5.5, 500 of 5.8 KB
+// 4.9 / 5.4, 1024 of 5.8 KB 6.3 / 5.8, 2048 of 5.8 KB 9.6 / 8.4.)
 // The readers lose nothing: the L2s of the XCDs do not serve each other, so they come from behind L2 either way.
 enum Store { PLAIN, THROUGH, STREAM };
 #ifndef MOE_A2A_STORE_SEND   /* stage 1 -> send buffer */
 #define MOE_A2A_STORE_SEND STREAM
-#endif
-#ifndef MOE_A2A_STORE_RECV   /* stage 2 -> expert_x */
-#define MOE_A2A_STORE_RECV THROUGH
 #endif
 #ifndef MOE_A2A_STORE_CSEND  /* stage 3 -> send-back buffer */
 #define MOE_A2A_STORE_CSEND STREAM
@@ -957,7 +956,7 @@ __global__ __launch_bounds__(RPLAN_BLOCK) void plan_recv_kernel(
 //                 the offsets.
 enum { RECV_SCAN = 0, RECV_POS = 1, RECV_COMPACT = 2 };
 
-template <typename V, int NVW, bool PLAN, int MODE>
+template <typename V, int NVW, bool PLAN, int MODE, Store HOW>
 __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
     const V* __restrict__ recv_buf, const int* __restrict__ recv_meta,
     const int* __restrict__ recv_counts, int W, int hint_rows, int capacity_rows, int nle,
@@ -1060,7 +1059,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
       const int R = rows_known();
       if (i < R && (uint32_t)pos < (uint32_t)max_recv) {
         const size_t row = (size_t)floormod(e, nle, magic) * max_recv + pos;
-        p.template store<MOE_A2A_STORE_RECV>(expert_x + row * row_vecs, base, row_vecs, lane);
+        p.template store<HOW>(expert_x + row * row_vecs, base, row_vecs, lane);
         if (c == 0 && lane < META) expert_meta[row * META + lane] = m;
       }
       return R;
@@ -1100,7 +1099,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
 #pragma unroll
       for (int r = 0; r < ROWS; ++r) le = r == wave ? rle[r] : le;
       const size_t row = COMPACT ? (size_t)pos : (size_t)le * max_recv + pos;
-      p.template store<MOE_A2A_STORE_RECV>(expert_x + row * row_vecs, base, row_vecs, lane);
+      p.template store<HOW>(expert_x + row * row_vecs, base, row_vecs, lane);
       if (c == 0 && lane < META) expert_meta[row * META + lane] = m;
     }
     return R;
@@ -3399,7 +3398,7 @@ __global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
     }
   }
   if (compact) {  // exclusive prefix of the rows per expert (E <= 1024: one expert per lane)
-    const int mine = tid < E ? total[tid] : 0;
+    const int mine = tid < E ? total_of(tid) : 0;
     const int incl = wave_inclusive_scan(mine);
     if (lane == 63) red[wave] = incl;
     __syncthreads();
@@ -3955,7 +3954,7 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
                                                     capacity_rows, g.nle, g.magic, expert_bits, row_position);
     const int grid = g.nle + mover_blocks(group_items(rows_hint, g));
 #define LAUNCH_P(V, NVW, PLAN)                                                              \
-  dispatch_recv_kernel<V, NVW, PLAN, RECV_POS><<<grid, 64 * ROWS, 0, st>>>(                 \
+  dispatch_recv_kernel<V, NVW, PLAN, RECV_POS, THROUGH><<<grid, 64 * ROWS, 0, st>>>(        \
       (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, capacity_rows,   \
       g.nle, g.magic, g.max_recv, g.row_vecs, g.wchunks, expert_num_tokens, (V*)expert_x,    \
       expert_meta, send_back_plan, row_position, nullptr)
@@ -3975,11 +3974,17 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   // the stream can hold at most nle * max_recv rows that fit the expert buffers
   if (!items_fit((long long)g.nle * g.max_recv, g.wchunks)) return MOE_A2A_EINVAL;
   const int grid = g.nle + mover_blocks(group_items(rows_hint, g));
-#define LAUNCH_P(V, NVW, PLAN, MODE)                                                        \
-  dispatch_recv_kernel<V, NVW, PLAN, MODE><<<grid, 64 * ROWS, 0, st>>>(                     \
+  const bool through = (long long)rows_hint * s->hidden_dim * 2 >= 8 << 20;  // (Store)
+#define LAUNCH_S(V, NVW, PLAN, MODE, HOW)                                                   \
+  dispatch_recv_kernel<V, NVW, PLAN, MODE, HOW><<<grid, 64 * ROWS, 0, st>>>(                     \
       (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, capacity_rows,   \
       g.nle, g.magic, compact_rows > 0 ? compact_rows : g.max_recv, g.row_vecs, g.wchunks,   \
       expert_num_tokens, (V*)expert_x, expert_meta, send_back_plan, nullptr, expert_offsets)
+#define LAUNCH_P(V, NVW, PLAN, MODE)                        \
+  do {                                                      \
+    if (through) LAUNCH_S(V, NVW, PLAN, MODE, THROUGH);     \
+    else LAUNCH_S(V, NVW, PLAN, MODE, PLAIN);               \
+  } while (0)
 #define LAUNCH(V, NVW)                                         \
   do {                                                         \
     if (compact_rows > 0) {                                    \
@@ -3993,6 +3998,7 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   MOE_A2A_FOR_WAVE_KERNEL(g, LAUNCH);
 #undef LAUNCH
 #undef LAUNCH_P
+#undef LAUNCH_S
   return launch_status();
 }
 
