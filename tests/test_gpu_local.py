@@ -135,3 +135,20 @@ def test_results_of_a_job_share_no_storage(tokens):
     ys = custom_kernel_job([(cfg, rank_data(cfg, t, r), r, 4) for r, t in enumerate(tokens)])
     assert len({y.untyped_storage().data_ptr() for y in ys}) == 4
     assert all(y.untyped_storage().nbytes() == y.numel() * y.element_size() for y in ys)
+
+
+@pytest.mark.parametrize("W,E,K,tokens,spoil", [
+    (5, 35, 3, [201, 7, 1, 350, 130], None), (9, 18, 1, [3, 0, 1, 2, 5, 0, 7, 1, 2], None),  # loads across two and more ranks
+    (4, 64, 7, [100, 33, 0, 171], "ids"), (2, 8, 8, [4000, 4191], None), (2, 8, 8, [4096, 4097], None),  # 65528 and 65544 entries
+    (2, 8, 8, [4000, 4400], "ids"), (64, 64, 3, [11] * 64, "twins"),
+])
+def test_planned_jobs(W, E, K, tokens, spoil):
+    """Jobs with a plan launch of their own: ranks that begin inside a load of four entries, both counts of an expert
+    in one word (up to 65535 entries) and in two."""
+    print(f"planned W={W} E={E} K={K} {tokens[:4]} {spoil}", flush=True)
+    cfg = config(E, K, 16, max(tokens))
+    data = [rank_data(cfg, t, 7 * r + K, spoil) for r, t in enumerate(tokens)]
+    want = [y.clone() for y in LocalWorld(cfg, W, device=DEV).run(data)]
+    ys = custom_kernel_job([(cfg, d, r, W) for r, d in enumerate(data)])
+    for r in range(W):
+        assert torch.equal(ys[r], want[r]), f"rank {r}"
