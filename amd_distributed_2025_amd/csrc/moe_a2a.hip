@@ -2149,8 +2149,8 @@ __global__ __launch_bounds__(64 * GW, GW > 4 || D > 3 ? 1 : TJ == 1 ? 4 : TJ == 
 
 // ---------------------------------------------------------------- product with few rows
 //
-// Y[M, N] = X[M, K] @ W[N, K]^T for at most 64 rows: the weights are streamed once and no tile
-// shape gives every compute unit work (M = 64, N = 7168: 56 tiles of 128 columns). Here a
+// Y[M, N] = X[M, K] @ W[N, K]^T where larger tiles would leave compute units without work (M = 64,
+// N = 7168: 56 tiles of 128 columns; M = 255, N = 1728: 56 of 64 x 128). Here a
 // workgroup owns only 32 output columns x one block of 32 or 64 tokens, and its KW waves (four,
 // eight for long K) split K: wave w takes steps w, w + KW, ... of 64 elements, streams
 // its own slices of the 32 weight rows and of the token rows (both 8 lanes per 128-byte line,
@@ -2169,7 +2169,7 @@ __global__ __launch_bounds__(64 * GW, GW > 4 || D > 3 ? 1 : TJ == 1 ? 4 : TJ == 
 template <int DT, int TJ, int KW, bool APART>
 __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
     const b128* __restrict__ X, const b128* __restrict__ Wt, const uint16_t* __restrict__ bias,
-    uint16_t* __restrict__ Y, int M, int N, int K, int col_units) {
+    uint16_t* __restrict__ Y, int M, int N, int K, int row_units, uint32_t row_magic) {
   constexpr int TOK = TJ * 32;
   constexpr int XL = TJ * 4;  // token loads per lane and step: TOK rows x 8 vectors over 64 lanes
   extern __shared__ b128 skinny_lds[];  // per wave: 32 weight rows, then TOK token rows, of 8 vectors
@@ -2178,14 +2178,22 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int row_vecs = K / 8, row_bytes = K * 2, steps = (K + GEMM_KSTEP - 1) / GEMM_KSTEP;
   const int tail_vecs = row_vecs - (steps - 1) * 8;
-  const int rb = blockIdx.x / col_units, cu = blockIdx.x - rb * col_units;
+  // Row blocks of the same columns run beside each other on one XCD: its L2 then has the weights for all but the first
+  // (us, row blocks numbered last / first: 140 x 3008 x 4680 28.3 / 21.1, 37 x 3968 x 936 5.7 / 4.75, 81 x 2176 x 7488
+  // 15.2 / 13.7). row_magic = ceil(2^32 / row_units): exact for the up to 10240 workgroups, and a division less to wait for.
+  int rb = 0, cu = blockIdx.x;
+  if (row_units > 1) {
+    const int logical = xcd_contiguous(blockIdx.x, N / 32 * row_units);
+    cu = __umulhi((uint32_t)logical, row_magic);
+    rb = logical - cu * row_units;
+  }
   const int t0 = rb * TOK, n0 = cu * 32, live = M - t0;
   // APART: where rows lie a multiple of 4 KB apart (see first_kstep) workgroups start apart too, by whole turns of
   // the waves, so that a wave keeps its steps: 8 x 8192 x 8192 34.1 -> 25.6 us, 1 x 4096 x 4096 12.4 -> 9.5, 64 x
   // 8192 x 8192 41 -> 38, 16 x 16384 x 2048 16.0 -> 14.6. Elsewhere going round costs 0.8 % (64 x 7168 x 2304 11.29 us,
   // 11.20 without).
   static_assert(32 % KW == 0, "whole turns in the steps of 2048 inputs");
-  const int first_step = APART ? (int)((long long)cu * (steps / KW) / col_units) * KW : 0;
+  const int first_step = APART ? (int)((uint32_t)cu * (steps / KW) / ((uint32_t)N / 32)) * KW : 0;
 
   const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(Wt + (size_t)n0 * row_vecs), 0, 32 * row_bytes, BUFFER_RAW_32BIT);
@@ -4424,25 +4432,7 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   return launch_status();
 }
 
-#ifndef MOE_A2A_DENSE_TILE
-#define MOE_A2A_DENSE_TILE 0  // (measurements) 256, 128 or 64: that tile height for every shape
-#endif
 constexpr int MOE_A2A_NOT_DENSE = 1;  // (internal) the shape is left to the next kernel
-
-// Which tile an M x N x K product is cut into: 64 x 128 (dense_gemm_kernel) for outputs that this height
-// spreads over the 256 units once, 128 x 128 (phased_gemm_kernel, two workgroups per unit, or dense) while tiles of
-// 256 x 256 would leave more than a third of the units without work, else 256 x 256 (phased, one workgroup
-// per unit), whose rate per unit is half as high again. Measured with 256 / 128 rows, us: 2048 x 4096 x 1024
-// (128 big tiles) 24.1 / 21.5; 1024 x 8192 x 2048 (128) 38.6 / 35.7; 2048 x 2880 x 360 (96) 15.4 / 11.6;
-// 4096 x 4096 x 512 (256) 22.2 / 27.4; 8192 x 8192 x 3696 (1024) 407 / 622.
-int dense_tile_rows(long long M, long long N) {
-  if (MOE_A2A_DENSE_TILE) return MOE_A2A_DENSE_TILE;
-  constexpr long long UNITS = 256;
-  const long long low = ((M + 63) / 64) * ((N + 127) / 128);
-  if (low <= UNITS) return 64;
-  const long long big = ((M + 255) / 256) * ((N + 255) / 256);
-  return big > UNITS * 5 / 8 ? 256 : 128;
-}
 
 constexpr size_t local_plan_lds_bytes(int experts) { return (size_t)(2 + LPLAN_WAVES) * experts * sizeof(int); }
 constexpr size_t dense_lds_bytes(int BM, int BN) { return 2 * (size_t)(BM + BN) * 8 * sizeof(b128); }
@@ -4493,39 +4483,30 @@ int allow_large_lds() {
   return MOE_A2A_OK;
 }
 
-// The dense kernel for products of more than a few rows; MOE_A2A_NOT_DENSE otherwise (the kernels
-// that split K over the waves of a workgroup or stream the weights once).
-int launch_dense_gemm(const void* a, const void* b, const void* bias, void* c, int M, int N, int K,
-                      int dtype, hipStream_t st) {
-  if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
-  if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
-  if (!all_aligned(16, a, b, c) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
-  if (!tile_rows_in_range(256, K)) return MOE_A2A_NOT_DENSE;  // 32-bit byte offsets inside a tile's rows
-  const int tile = dense_tile_rows(M, N);
-  const int BM = tile, BN = tile == 64 ? 128 : tile;
+// A plain product on tiles that workgroups own whole, as linear_way has chosen.
+int launch_linear_tiles(const void* a, const void* b, const void* bias, void* c, int M, int N, int K, int dtype,
+                        LinearWay way, hipStream_t st) {
+  const int BM = way == PHASED_256 ? 256 : way == TILES_64x128 ? 64 : 128, BN = way == PHASED_256 ? 256 : 128;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + BN - 1) / BN;
   if (tiles_m * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
   const int grid = (int)(tiles_m * tiles_n);
   // phased_gemm_kernel strides over its tiles: one workgroup per unit, or two of 128 x 128
-  const int phased_grid = std::min(grid, tile == 256 ? 256 : 512);
+  const int phased_grid = std::min(grid, way == PHASED_256 ? 256 : 512);
   if (const int rc = allow_large_lds()) return rc;
 #define LAUNCH_P(DT, TM, TN, AHEAD)                                                              \
   phased_gemm_kernel<DT, TM, TN, 3, 4, AHEAD, false><<<phased_grid, 512, phased_lds_bytes(TM, TN, 3, 4), st>>>( \
       (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n, \
       nullptr, 0, 0, 0)
-  // Tiles of 128 x 128, at most one per unit: nobody is there to work while phased_gemm_kernel's waves wait for each
-  // other, and dense_gemm_kernel, which waits less, is ahead (phased / dense, us: 1586 x 2432 x 1536 20.3 / 17.8; 1024
-  // x 4096 x 4096 44.2 / 38.2; 600 x 6144 x 7168 96.5 / 69.5; with 273 tiles, 1586 x 2688 x 1536, 21.9 / 24.1).
 #define LAUNCH_D(DT, TM, TN, LDS)                                                                \
   dense_gemm_kernel<DT, 2, 2, TM, TN, false><<<grid, 256, LDS, st>>>(                            \
       (const b128*)a, (const b128*)b, (const uint16_t*)bias, (uint16_t*)c, M, N, K, (int)tiles_m, (int)tiles_n, \
       nullptr, 0, 0, 0)
 #define LAUNCH_DT(DT)                                                                            \
   do {                                                                                           \
-    if (tile == 256 && K * 2 % 128 != 0) LAUNCH_P(DT, 8, 4, true);                               \
-    else if (tile == 256) LAUNCH_P(DT, 8, 4, false);                                             \
-    else if (tile == 128 && grid > 256) LAUNCH_P(DT, 4, 2, false);                               \
-    else if (tile == 128) LAUNCH_D(DT, 2, 2, dense_lds_bytes(128, 128));                         \
+    if (way == PHASED_256 && K * 2 % 128 != 0) LAUNCH_P(DT, 8, 4, true);                         \
+    else if (way == PHASED_256) LAUNCH_P(DT, 8, 4, false);                                       \
+    else if (way == PHASED_128) LAUNCH_P(DT, 4, 2, false);                                       \
+    else if (way == TILES_128x128) LAUNCH_D(DT, 2, 2, dense_lds_bytes(128, 128));                \
     else LAUNCH_D(DT, 1, 2, dense_lds_bytes(64, 128));                                           \
   } while (0)
   if (dtype == MOE_A2A_BF16) LAUNCH_DT(MOE_A2A_BF16);
@@ -4585,34 +4566,19 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   return launch_status();
 }
 
-#ifndef MOE_A2A_SKINNY_WAVES
-#define MOE_A2A_SKINNY_WAVES 0  // (measurements) 4 or 8: that many waves for every shape
-#endif
-#ifndef MOE_A2A_SKINNY_MAX_TILES
-#define MOE_A2A_SKINNY_MAX_TILES 192  // tiles of 128 columns below which K is split inside the workgroup
-#endif
-
-// Products of at most 64 rows whose tiles of 128 columns would leave compute units idle: 32
-// columns per workgroup, K split over its waves. MOE_A2A_NOT_DENSE when the grouped kernel is
-// the better fit.
-int launch_skinny_gemm(const void* x, const void* w, const void* bias, void* y, int M, int N, int K,
-                       int dtype, hipStream_t st) {
-  if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
-  if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
-  if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
-  if (M > 64 || !tile_rows_in_range(128, K)) return MOE_A2A_NOT_DENSE;
-  const int wide_tiles = (N + GEMM_COLS - 1) / GEMM_COLS;
+// A plain product on workgroups of 32 columns whose waves split K among them, tj x 32 rows each.
+int launch_linear_split(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int dtype, int tj,
+                        hipStream_t st) {
   const int steps = (K + GEMM_KSTEP - 1) / GEMM_KSTEP;
-  if (wide_tiles >= MOE_A2A_SKINNY_MAX_TILES || steps < 2 * NWAVES) return MOE_A2A_NOT_DENSE;
-  const int grid = N / 32;
+  const int row_units = (M + 32 * tj - 1) / (32 * tj), grid = N / 32 * row_units;
+  const uint32_t row_magic = row_units > 1 ? (uint32_t)(((1ull << 32) + row_units - 1) / row_units) : 0;
   // eight waves keep more of the stream in flight (measured 10 to 13 % less time from 28 steps
   // on); with few steps the four extra partial sums cost more than that
-  const int waves = MOE_A2A_SKINNY_WAVES ? MOE_A2A_SKINNY_WAVES : steps >= 24 ? 8 : 4;
-  const int tj = M <= 32 ? 1 : 2;
+  const int waves = steps >= 24 ? 8 : 4;
   if (const int rc = allow_large_lds()) return rc;
 #define LAUNCH_KA(DT, TJ, KW, APART)                                                      \
   skinny_gemm_kernel<DT, TJ, KW, APART><<<grid, 64 * KW, skinny_lds_bytes(TJ, KW), st>>>( \
-      (const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, M, N, K, N / 32)
+      (const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, M, N, K, row_units, row_magic)
 #define LAUNCH_K(DT, TJ, KW)                               \
   do {                                                     \
     if (K % 2048 == 0) LAUNCH_KA(DT, TJ, KW, true);        \
@@ -4631,6 +4597,18 @@ int launch_skinny_gemm(const void* x, const void* w, const void* bias, void* y, 
 #undef LAUNCH_K
 #undef LAUNCH_KA
   return launch_status();
+}
+
+int launch_linear(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int dtype, hipStream_t st) {
+  if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
+  if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
+  if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
+  const LinearWay way = linear_way(M, N, K);
+  int rc = MOE_A2A_NOT_DENSE;
+  if (way == SPLIT_32 || way == SPLIT_64) rc = launch_linear_split(x, w, bias, y, M, N, K, dtype, way == SPLIT_32 ? 1 : 2, st);
+  else if (way != STREAM_WEIGHTS) rc = launch_linear_tiles(x, w, bias, y, M, N, K, dtype, way, st);
+  if (rc != MOE_A2A_NOT_DENSE) return rc;
+  return launch_grouped_gemm(x, nullptr, w, bias, y, 1, M, M, N, K, dtype, st);
 }
 
 }  // namespace
@@ -4676,12 +4654,7 @@ int moe_a2a_linear(const void* input, const void* weight, const void* bias, int3
                    int32_t k, int32_t dtype, void* output, void* stream) {
   if (m < 0 || n < 1 || k < 1 || !weight || (m > 0 && (!input || !output))) return MOE_A2A_EINVAL;
   if (m == 0) return MOE_A2A_OK;
-  const int skinny = launch_skinny_gemm(input, weight, bias, output, m, n, k, dtype, (hipStream_t)stream);
-  if (skinny != MOE_A2A_NOT_DENSE) return skinny;
-  const int dense = launch_dense_gemm(input, weight, bias, output, m, n, k, dtype, (hipStream_t)stream);
-  if (dense != MOE_A2A_NOT_DENSE) return dense;
-  return launch_grouped_gemm(input, nullptr, weight, bias, output, 1, m, m, n, k, dtype,
-                             (hipStream_t)stream);
+  return launch_linear(input, weight, bias, output, m, n, k, dtype, (hipStream_t)stream);
 }
 
 int moe_a2a_exchange_local(int32_t world_size, int32_t hidden_dim, const void* send_buf,

@@ -1,6 +1,8 @@
 // Which tiles a product is cut into: plain arithmetic on its sizes, so that a host compiler can take it as well.
 #pragma once
 
+#include <limits.h>
+
 #include <algorithm>
 #include <cmath>
 
@@ -86,6 +88,66 @@ int grouped_tile_bands(long long rows_hint, int groups, int N, int K) {
     }
   }
   return best_bands;
+}
+
+// The kernel of a plain product [M, N, K].
+//
+// Up to 160 tiles of 256 x 256 a product takes, per step of K, what its workgroups wait for (about the same for every
+// round of them over the 256 units, and the longer the larger the tile) and what all of them fetch, in rows of 128
+// bytes, 0.7 ns for one row on every unit: rounds x `wait` + rows fetched. Small tiles fetch more and wait less. The
+// waits are those that lose least over 510 shapes (65 to 1500 rows, N 1024 to 8192, K 256 to 8192, all five timed on
+// each): the choice is 0.5 % behind the best of the five on average, by more than a tenth on 5 shapes; on 180 that had no
+// part in the fit (to 20000 rows, N from 32 to 36000) 0.4 %, on 2 shapes. By the number of tiles alone (64 x 128 up to
+// 256 of them, then 128 x 128) it was 13 % behind, by more than a quarter on 103. Among them, us with SPLIT_32 / SPLIT_64 /
+// 64 x 128 / 128 x 128 / PHASED_128:
+//   112 x 1920 x 1832   7.3 /  9.4 / 13.8 / 18.9 / 21.0     255 x 1728 x 3968  19.4 / 14.4 / 23.1 / 26.7 / 37.0
+//   867 x 1216 x 6104  70.0 / 61.1 / 43.5 / 56.1 / 63.9     547 x 2688 x 5376  61.1 / 44.2 / 31.3 / 35.0 / 49.2
+//   825 x 2624 x 1792  40.2 / 35.5 / 18.5 / 15.5 / 19.5     1586 x 2688 x 1536 phased / 128 x 128 21.9 / 24.1
+// Up to 64 rows the two that split K are ahead of the others as far as SPLIT_MAX_TILES, and the same comparison picks the
+// height: 59 x 512 x 4448 7.9 / 11.2, 59 x 896 x 6728 16.2 / 22.2 (60 shapes of 33 to 64 rows: 1 % behind the better one,
+// 64 rows high for all of them 13 %, more than a quarter on 15).
+//
+// From there on tiles of 256 x 256 win, whose rate per unit is half as high again as that of 128 x 128. Measured with
+// 256 / 128 rows: 2048 x 4096 x 1024 (128 big tiles) 24.1 / 21.5; 1024 x 8192 x 2048 (128) 38.6 / 35.7; 2048 x 2880 x
+// 360 (96) 15.4 / 11.6; 4096 x 4096 x 512 (256) 22.2 / 27.4; 8192 x 8192 x 3696 (1024) 407 / 622.
+enum LinearWay {
+  SPLIT_32, SPLIT_64,           // skinny_gemm_kernel, 32 or 64 rows x 32 columns
+  TILES_64x128, TILES_128x128,  // dense_gemm_kernel
+  PHASED_128, PHASED_256,       // phased_gemm_kernel, 128 x 128 or 256 x 256
+  STREAM_WEIGHTS                // expert_gemm_kernel, as one group
+};
+
+LinearWay linear_way(long long M, long long N, long long K) {
+  constexpr long long UNITS = 256, SPLIT_MIN_STEPS = 8;  // (two for each of four waves)
+  constexpr long long SPLIT_MAX_TILES = 192;             // of 128 columns, up to 64 rows
+  // (sizes of tiles as powers of two: a small product waits for every division here)
+  auto tiles = [&](int rows, int columns) { return ((M + (1 << rows) - 1) >> rows) * ((N + (1 << columns) - 1) >> columns); };
+  const bool can_split = (K + 63) / 64 >= SPLIT_MIN_STEPS;
+  const bool only_split = can_split && M <= 64 && (N + 127) / 128 < SPLIT_MAX_TILES;
+  if (!tile_rows_in_range(only_split ? 128 : 256, K)) return STREAM_WEIGHTS;
+  if (!only_split && tiles(8, 8) > UNITS * 5 / 8) return PHASED_256;
+  auto cost = [&](int rows, int columns, int wait, int more) {
+    const long long n = tiles(rows, columns);
+    return ((n + UNITS - 1) / UNITS * wait + more) * UNITS + n * ((1 << rows) + (1 << columns));
+  };
+  LinearWay best = PHASED_128;
+  long long least = LLONG_MAX;
+  auto consider = [&](LinearWay way, long long c) {
+    if (c < least) {
+      least = c;
+      best = way;
+    }
+  };
+  if (can_split) {
+    consider(SPLIT_32, cost(5, 5, 120, 0));
+    consider(SPLIT_64, cost(6, 5, 190, 0));
+  }
+  if (!only_split) {
+    consider(TILES_64x128, cost(6, 7, 380, 0));
+    consider(TILES_128x128, cost(7, 7, 550, 0));
+    consider(PHASED_128, cost(7, 7, 380, 280));
+  }
+  return best;
 }
 
 }  // namespace

@@ -369,15 +369,15 @@ int moe_a2a_expert_gemm(const moe_a2a_shape* shape, const void* expert_x,
  * statements do. bias may be NULL.
  * One of four kernels runs, picked from the shape alone (so a shape always
  * gives the same bits; a slice of the weight's rows is another shape, and where
- * m <= 64 and k is a multiple of 2048 the first of these kernels also starts its
- * sums at an input that depends on the column's place among n): for m <= 64, k >= 449 (eight steps of 64 elements) and
- * n <= 24448 (fewer than 192 tiles of 128 columns), a kernel whose
- * workgroups own 32 columns and split k over their waves (partial sums added in
- * a fixed order); else kernels bound by the matrix cores, whose workgroups own
- * output tiles of 256 x 256, 128 x 128 or 64 x 128 (the largest that still
- * gives every compute unit work; all three add the same terms in the same
- * order); for shapes beyond their index ranges, the kernel of
- * moe_a2a_expert_gemm with one group of m rows.
+ * k is a multiple of 2048 the first of these kernels also starts its sums at an
+ * input that depends on the column's place among n): for k >= 449 (eight steps
+ * of 64 elements), a kernel whose workgroups own 32 columns and 32 or 64 rows and
+ * split k over their waves (partial sums added in a fixed order), always for m <=
+ * 64 and n <= 24448 and else where larger tiles would leave compute units without
+ * work; kernels bound by the matrix cores, whose workgroups own output tiles of
+ * 256 x 256, 128 x 128 or 64 x 128 (all of them add the same terms in the same
+ * order); for shapes beyond their index ranges, the kernel of moe_a2a_expert_gemm
+ * with one group of m rows.
  * Limits: n a multiple of 32, k a multiple of 8, input / weight / output 16-byte
  * and bias 8-byte aligned (MOE_A2A_EINVAL / EALIGN). m == 0 is a no-op.
  * The first call on a GPU sets kernel attributes (tiles can use more LDS than a

@@ -260,3 +260,32 @@ def test_few_rows_whatever_a_wave_has_to_walk(m, k, dt):
     want = ((x.double() @ w.double().T).to(dt).double() + b.double()).to(dt)
     assert torch.equal(out[1:m + 1], want)
     assert (out[0] == 777.0).all() and (out[m + 1] == 777.0).all()
+
+
+# rows and columns that csrc/tile_rules.h gives to each way of cutting a product (tests/test_tile_rules.py asks it), from
+# eight steps of K on: last row blocks of one row and whole ones, last column tiles of 32 columns and whole ones
+WAYS = {"SPLIT_32": [(65, 96), (64, 4096), (96, 2720), (97, 32), (321, 480)],
+        "SPLIT_64": [(64, 7168), (129, 1728), (192, 2048), (449, 992)],
+        "TILES_64x128": [(547, 2688), (513, 3104), (193, 7200)],
+        "TILES_128x128": [(825, 2624), (769, 4128)]}
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("k", [512, 520, 1472, 1544, 2048, 4096])
+@pytest.mark.parametrize("way,m,n", [(way, *mn) for way, shapes in WAYS.items() for mn in shapes])
+def test_every_way_of_cutting_a_product(way, m, n, k, dt):
+    """Four and eight waves on a workgroup's K, a cut last step, rows 4 KB apart; several row blocks of 32 and of 64 rows
+    beside each other. Small integers, whose sums every order gives exactly and float32 holds; rounded once before the
+    bias and once after. Stray NaNs around the operands, sentinels around the result."""
+    print(f"linear {way} m={m} n={n} k={k} {dt}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    pad = torch.full((m + 2, k), float("nan"), dtype=dt, device=DEV)
+    pad[1:m + 1] = torch.randint(-1, 2, (m, k), generator=g, device=DEV).to(dt)
+    wpad = torch.full((n + 2, k), float("nan"), dtype=dt, device=DEV)
+    wpad[1:n + 1] = torch.randint(-1, 2, (n, k), generator=g, device=DEV).to(dt)
+    b = torch.randint(-9, 10, (n,), generator=g, device=DEV).to(dt)
+    out = torch.full((m + 2, n), 777.0, dtype=dt, device=DEV)
+    gemm_rs.local_product((pad[1:m + 1], wpad[1:n + 1], b), out=out[1:m + 1])
+    want = ((pad[1:m + 1].double() @ wpad[1:n + 1].double().T).to(dt).double() + b.double()).to(dt)
+    assert torch.equal(out[1:m + 1], want)
+    assert (out[0] == 777.0).all() and (out[m + 1] == 777.0).all()

@@ -8,6 +8,7 @@ import pytest
 
 from tests.test_gpu_expert_gemm import TILES_OF_NARROW
 from tests.test_gpu_grouped_tiles import FEW_STEPS, PAST_THE_CACHE, ROWS_FOR_TILE
+from tests.test_gpu_linear import WAYS
 
 CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
 
@@ -19,12 +20,14 @@ def rules(tmp_path_factory):
     src = tmp_path_factory.mktemp("rules") / "rules.cpp"
     src.write_text('#include "tile_rules.h"\n'
                    'extern "C" int bands(long long rows_hint, int groups, int n, int k) { return grouped_tile_bands(rows_hint, groups, n, k); }\n'
-                   'extern "C" int past(int groups, int n, int k) { return weights_past_the_cache(groups, n, k); }\n')
+                   'extern "C" int past(int groups, int n, int k) { return weights_past_the_cache(groups, n, k); }\n'
+                   'extern "C" int way(long long m, long long n, long long k) { return linear_way(m, n, k); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
                     str(src), "-o", str(lib)], check=True)
     dll = C.CDLL(str(lib))
     dll.bands.argtypes = [C.c_longlong, C.c_int, C.c_int, C.c_int]
+    dll.way.argtypes = [C.c_longlong] * 3
     return dll
 
 
@@ -96,3 +99,38 @@ def test_the_second_tiles_that_the_gpu_tests_mean():
         if isinstance(tile, int):
             workgroups = rows * 5 // tile + 5
             assert 5 * -(-650 // tile) > workgroups, (rows, tile)
+
+
+SPLIT_32, SPLIT_64, TILES_64x128, TILES_128x128, PHASED_128, PHASED_256, STREAM_WEIGHTS = range(7)  # LinearWay
+
+
+def test_the_ways_that_the_gpu_tests_mean(rules):
+    for name, shapes in WAYS.items():
+        for m, n in shapes:
+            for k in (512, 2048, 8192):
+                assert rules.way(m, n, k) == globals()[name], (m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k,way", [(112, 1920, 1832, SPLIT_32), (255, 1728, 3968, SPLIT_64), (64, 7168, 2304, SPLIT_64),
+                                       (59, 512, 4448, SPLIT_32), (867, 1216, 6104, TILES_64x128),
+                                       (547, 2688, 5376, TILES_64x128), (825, 2624, 1792, TILES_128x128),
+                                       (1586, 2688, 1536, PHASED_128), (2048, 2880, 360, PHASED_128),
+                                       (2048, 4096, 1024, PHASED_128), (4096, 4096, 512, PHASED_256)])
+def test_way_that_was_fastest_where_they_differ_most(rules, m, n, k, way):
+    assert rules.way(m, n, k) == way
+
+
+def test_ways_of_a_product_stay_in_the_range_of_their_kernels(rules):
+    """K is split from two steps for each of four waves on, and a way whose 32-bit offsets reach over `rows` rows is
+    picked only where rows of K elements end before the out-of-range offset. Large and extreme sizes have a way too."""
+    rows_of = {SPLIT_32: 128, SPLIT_64: 128, TILES_64x128: 256, TILES_128x128: 256, PHASED_128: 256, PHASED_256: 256}
+    for m in (1, 32, 33, 64, 65, 200, 1000, 5000, 2 ** 31 - 1):
+        for n in (32, 1024, 7168, 24448, 24480, 40000, 2 ** 31 - 32):
+            for k in (8, 448, 456, 7168, 2097144, 2097152, 4194296, 4194304, 2 ** 31 - 8):
+                way = rules.way(m, n, k)
+                assert way == STREAM_WEIGHTS or rows_of[way] * k * 2 < OUT_OF_RANGE, (m, n, k, way)
+                if way in (SPLIT_32, SPLIT_64):
+                    assert (k + 63) // 64 >= 8
+                    assert (n // 32) * ((m + 31) // 32) < 2 ** 31  # workgroups
+                if way == STREAM_WEIGHTS:
+                    assert k >= 2097152
