@@ -2826,7 +2826,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   // A workgroup strides over the tiles (the size of the launch is a matter of speed only). EARLY: the first loads of
   // its next tile go out before the results of the last one do, so that they arrive while those are written, and the
   // accumulators are cleared meanwhile. A workgroup per tile / this: 8192 x 8192 x 512 84.5 / 79.0 us, x 3696 370.6 /
-  // 368.3, 4096 x 4096 x 4096 93.5 / 92.4, tiles of 128 x 128 at 3000 x 3000 x 1024 31.9 / 30.3. Experts' products have
+  // 368.3, 4096 x 4096 x 4096 93.5 / 92.4. (Smaller tiles have no next one: linear_way.) Experts' products have
   // a workgroup per tile in general, and the registers for it would be spilled at 320 rows: 140 -> 146 us.
   int tile = blockIdx.x, total_tiles = tiles_m * tiles_n;  // (GROUPED: counted by find_tile)
   int n0, rows_left;         // first column of the tile; rows of the matrix from the tile's first one on
@@ -4464,7 +4464,9 @@ int allow_large_lds() {
   allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 4, true, false>, phased_lds_bytes(8, 4, 3, 4));
   allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 4, true, false>, phased_lds_bytes(8, 4, 3, 4));
   allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 4, 2, 3, 4, false, false>, phased_lds_bytes(4, 2, 3, 4));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 6, 2, 3, 4, false, false>, phased_lds_bytes(6, 2, 3, 4));
   allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 4, 2, 3, 4, false, false>, phased_lds_bytes(4, 2, 3, 4));
+  allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 6, 2, 3, 4, false, false>, phased_lds_bytes(6, 2, 3, 4));
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
@@ -4486,12 +4488,13 @@ int allow_large_lds() {
 // A plain product on tiles that workgroups own whole, as linear_way has chosen.
 int launch_linear_tiles(const void* a, const void* b, const void* bias, void* c, int M, int N, int K, int dtype,
                         LinearWay way, hipStream_t st) {
-  const int BM = way == PHASED_256 ? 256 : way == TILES_64x128 ? 64 : 128, BN = way == PHASED_256 ? 256 : 128;
+  const int BM = way == PHASED_256 ? 256 : way == PHASED_192 ? 192 : way == TILES_64x128 ? 64 : 128;
+  const int BN = way == PHASED_256 ? 256 : 128;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + BN - 1) / BN;
   if (tiles_m * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
   const int grid = (int)(tiles_m * tiles_n);
   // phased_gemm_kernel strides over its tiles: one workgroup per unit, or two of 128 x 128
-  const int phased_grid = std::min(grid, way == PHASED_256 ? 256 : 512);
+  const int phased_grid = std::min(grid, way == PHASED_128 ? 512 : 256);
   if (const int rc = allow_large_lds()) return rc;
 #define LAUNCH_P(DT, TM, TN, AHEAD)                                                              \
   phased_gemm_kernel<DT, TM, TN, 3, 4, AHEAD, false><<<phased_grid, 512, phased_lds_bytes(TM, TN, 3, 4), st>>>( \
@@ -4505,6 +4508,7 @@ int launch_linear_tiles(const void* a, const void* b, const void* bias, void* c,
   do {                                                                                           \
     if (way == PHASED_256 && K * 2 % 128 != 0) LAUNCH_P(DT, 8, 4, true);                         \
     else if (way == PHASED_256) LAUNCH_P(DT, 8, 4, false);                                       \
+    else if (way == PHASED_192) LAUNCH_P(DT, 6, 2, false);                                       \
     else if (way == PHASED_128) LAUNCH_P(DT, 4, 2, false);                                       \
     else if (way == TILES_128x128) LAUNCH_D(DT, 2, 2, dense_lds_bytes(128, 128));                \
     else LAUNCH_D(DT, 1, 2, dense_lds_bytes(64, 128));                                           \

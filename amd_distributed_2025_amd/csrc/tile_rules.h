@@ -107,14 +107,23 @@ int grouped_tile_bands(long long rows_hint, int groups, int N, int K) {
 // height: 59 x 512 x 4448 7.9 / 11.2, 59 x 896 x 6728 16.2 / 22.2 (60 shapes of 33 to 64 rows: 1 % behind the better one,
 // 64 rows high for all of them 13 %, more than a quarter on 15).
 //
-// From there on tiles of 256 x 256 win, whose rate per unit is half as high again as that of 128 x 128. Measured with
-// 256 / 128 rows: 2048 x 4096 x 1024 (128 big tiles) 24.1 / 21.5; 1024 x 8192 x 2048 (128) 38.6 / 35.7; 2048 x 2880 x
-// 360 (96) 15.4 / 11.6; 4096 x 4096 x 512 (256) 22.2 / 27.4; 8192 x 8192 x 3696 (1024) 407 / 622.
+// Between 256 tiles of 128 x 128 and 160 of 256 x 256 what counts is how many tiles the fullest unit has. 192 x 128 (192 +
+// 128 rows fetched, one workgroup per unit) makes one round of up to 384 tiles of 128 x 128, of which a quarter to a half
+// of the units would have two, and 256 x 256 one of those that would be three rounds of 128 x 128. Their waits (680, 1380)
+// lose least over 130 shapes of 360 to 8192 rows there (0.14 % behind the best of five on average, more than a tenth
+// on none; without these two 6.9 %, on 29; any 640 to 720 and 1300 to 1400 do as well). us with 128 x 128 / PHASED_128 /
+// PHASED_192 / PHASED_256:
+//   2048 x 2880 x 360    12.7 / 11.3 /  9.9 / 15.2     3532 x 1408 x 3824   69.5 / 67.9 / 46.5 / 73.3
+//   1586 x 2688 x 1536   23.4 / 21.7 / 20.1 / 29.2      685 x 7232 x 2800   49.5 / 46.2 / 33.5 / 53.1
+//   2048 x 4096 x 1024   21.4 / 19.1 / 29.0 / 23.3     1646 x 5056 x 2800   76.9 / 76.6 / 67.5 / 54.2
+//   1024 x 8192 x 2048   36.7 / 32.1 / 49.5 / 39.3     4225 x 2176 x 1896   58.4 / 57.1 / 51.8 / 42.4
+// From 160 tiles on 256 x 256 win, whose rate per unit is half as high again as that of 128 x 128: with 256 / 128 rows
+// 4096 x 4096 x 512 (256) 22.2 / 27.4; 8192 x 8192 x 3696 (1024) 407 / 622.
 enum LinearWay {
-  SPLIT_32, SPLIT_64,           // skinny_gemm_kernel, 32 or 64 rows x 32 columns
-  TILES_64x128, TILES_128x128,  // dense_gemm_kernel
-  PHASED_128, PHASED_256,       // phased_gemm_kernel, 128 x 128 or 256 x 256
-  STREAM_WEIGHTS                // expert_gemm_kernel, as one group
+  SPLIT_32, SPLIT_64,                  // skinny_gemm_kernel, 32 or 64 rows x 32 columns
+  TILES_64x128, TILES_128x128,         // dense_gemm_kernel
+  PHASED_128, PHASED_192, PHASED_256,  // phased_gemm_kernel, 128 x 128, 192 x 128 or 256 x 256
+  STREAM_WEIGHTS                       // expert_gemm_kernel, as one group
 };
 
 LinearWay linear_way(long long M, long long N, long long K) {
@@ -126,9 +135,11 @@ LinearWay linear_way(long long M, long long N, long long K) {
   const bool only_split = can_split && M <= 64 && (N + 127) / 128 < SPLIT_MAX_TILES;
   if (!tile_rows_in_range(only_split ? 128 : 256, K)) return STREAM_WEIGHTS;
   if (!only_split && tiles(8, 8) > UNITS * 5 / 8) return PHASED_256;
+  auto cost_of = [&](long long n, int rows_fetched, int wait, int more) {
+    return ((n + UNITS - 1) / UNITS * wait + more) * UNITS + n * rows_fetched;
+  };
   auto cost = [&](int rows, int columns, int wait, int more) {
-    const long long n = tiles(rows, columns);
-    return ((n + UNITS - 1) / UNITS * wait + more) * UNITS + n * ((1 << rows) + (1 << columns));
+    return cost_of(tiles(rows, columns), (1 << rows) + (1 << columns), wait, more);
   };
   LinearWay best = PHASED_128;
   long long least = LLONG_MAX;
@@ -146,6 +157,8 @@ LinearWay linear_way(long long M, long long N, long long K) {
     consider(TILES_64x128, cost(6, 7, 380, 0));
     consider(TILES_128x128, cost(7, 7, 550, 0));
     consider(PHASED_128, cost(7, 7, 380, 280));
+    consider(PHASED_192, cost_of((M + 191) / 192 * ((N + 127) >> 7), 192 + 128, 680, 0));
+    consider(PHASED_256, cost(8, 8, 1380, 0));
   }
   return best;
 }

@@ -375,8 +375,8 @@ int moe_a2a_expert_gemm(const moe_a2a_shape* shape, const void* expert_x,
  * split k over their waves (partial sums added in a fixed order), always for m <=
  * 64 and n <= 24448 and else where larger tiles would leave compute units without
  * work; kernels bound by the matrix cores, whose workgroups own output tiles of
- * 256 x 256, 128 x 128 or 64 x 128 (all of them add the same terms in the same
- * order); for shapes beyond their index ranges, the kernel of moe_a2a_expert_gemm
+ * 256 x 256, 192 x 128, 128 x 128 or 64 x 128 (all of them add the same terms in
+ * the same order); for shapes beyond their index ranges, the kernel of moe_a2a_expert_gemm
  * with one group of m rows.
  * Limits: n a multiple of 32, k a multiple of 8, input / weight / output 16-byte
  * and bias 8-byte aligned (MOE_A2A_EINVAL / EALIGN). m == 0 is a no-op.

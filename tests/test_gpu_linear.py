@@ -200,9 +200,9 @@ def test_random_shapes_of_small_integers_are_exact(m, n, k):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("k", [8, 64, 72, 128, 136, 192, 264, 320])
-@pytest.mark.parametrize("m,n", [(3329, 3104), (1100, 4128)], ids=["256", "128"])
+@pytest.mark.parametrize("m,n", [(3329, 3104), (1100, 4128), (1921, 3872)], ids=["256", "192", "128"])
 def test_products_of_one_to_five_steps(m, n, k, dt):
-    """The kernel behind the tiles of 256 x 256 and 128 x 128 asks for rows up to two steps of 64 ahead and
+    """The kernel behind the tiles of 256 x 256, 192 x 128 and 128 x 128 asks for rows up to two steps of 64 ahead and
     runs its last three steps apart: every number of steps around that, with a whole and a cut last one, and
     last tiles of one row and of 32 columns. Small integers are exact in every order."""
     print(f"linear steps m={m} n={n} k={k} {dt}", flush=True)
@@ -224,7 +224,7 @@ def test_products_of_one_to_five_steps(m, n, k, dt):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("k", [8, 64, 200, 448])
-@pytest.mark.parametrize("m,n", [(4100, 4128), (5120, 7200), (2100, 4128)], ids=["289 of 256", "580 of 256", "561 of 128"])
+@pytest.mark.parametrize("m,n", [(4100, 4128), (5120, 7200)], ids=["289 of 256", "580 of 256"])
 def test_more_tiles_than_workgroups(m, n, k, bias, dt):
     """Workgroups take a second and a third tile, whose first rows are asked for ahead of the results of the tile
     before: whole and ragged tiles in front of them. Small integers, whose sums (|x @ w.T + b| <= 448 + 20 here at
@@ -267,7 +267,10 @@ def test_few_rows_whatever_a_wave_has_to_walk(m, k, dt):
 WAYS = {"SPLIT_32": [(65, 96), (64, 4096), (96, 2720), (97, 32), (321, 480)],
         "SPLIT_64": [(64, 7168), (129, 1728), (192, 2048), (449, 992)],
         "TILES_64x128": [(547, 2688), (513, 3104), (193, 7200)],
-        "TILES_128x128": [(825, 2624), (769, 4128)]}
+        "TILES_128x128": [(825, 2624), (769, 4128)],
+        "PHASED_128": [(1024, 8192), (1921, 3872)],
+        "PHASED_192": [(1536, 3360), (2113, 2336), (2017, 2688), (1345, 4000)],
+        "PHASED_256": [(1646, 5056), (2305, 4000)]}
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])

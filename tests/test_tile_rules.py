@@ -101,7 +101,7 @@ def test_the_second_tiles_that_the_gpu_tests_mean():
             assert 5 * -(-650 // tile) > workgroups, (rows, tile)
 
 
-SPLIT_32, SPLIT_64, TILES_64x128, TILES_128x128, PHASED_128, PHASED_256, STREAM_WEIGHTS = range(7)  # LinearWay
+SPLIT_32, SPLIT_64, TILES_64x128, TILES_128x128, PHASED_128, PHASED_192, PHASED_256, STREAM_WEIGHTS = range(8)  # LinearWay
 
 
 def test_the_ways_that_the_gpu_tests_mean(rules):
@@ -114,7 +114,8 @@ def test_the_ways_that_the_gpu_tests_mean(rules):
 @pytest.mark.parametrize("m,n,k,way", [(112, 1920, 1832, SPLIT_32), (255, 1728, 3968, SPLIT_64), (64, 7168, 2304, SPLIT_64),
                                        (59, 512, 4448, SPLIT_32), (867, 1216, 6104, TILES_64x128),
                                        (547, 2688, 5376, TILES_64x128), (825, 2624, 1792, TILES_128x128),
-                                       (1586, 2688, 1536, PHASED_128), (2048, 2880, 360, PHASED_128),
+                                       (1586, 2688, 1536, PHASED_192), (2048, 2880, 360, PHASED_192),
+                                       (3532, 1408, 3824, PHASED_192), (1646, 5056, 2800, PHASED_256),
                                        (2048, 4096, 1024, PHASED_128), (4096, 4096, 512, PHASED_256)])
 def test_way_that_was_fastest_where_they_differ_most(rules, m, n, k, way):
     assert rules.way(m, n, k) == way
@@ -123,7 +124,7 @@ def test_way_that_was_fastest_where_they_differ_most(rules, m, n, k, way):
 def test_ways_of_a_product_stay_in_the_range_of_their_kernels(rules):
     """K is split from two steps for each of four waves on, and a way whose 32-bit offsets reach over `rows` rows is
     picked only where rows of K elements end before the out-of-range offset. Large and extreme sizes have a way too."""
-    rows_of = {SPLIT_32: 128, SPLIT_64: 128, TILES_64x128: 256, TILES_128x128: 256, PHASED_128: 256, PHASED_256: 256}
+    rows_of = {SPLIT_32: 128, SPLIT_64: 128, TILES_64x128: 256, TILES_128x128: 256, PHASED_128: 256, PHASED_192: 256, PHASED_256: 256}
     for m in (1, 32, 33, 64, 65, 200, 1000, 5000, 2 ** 31 - 1):
         for n in (32, 1024, 7168, 24448, 24480, 40000, 2 ** 31 - 32):
             for k in (8, 448, 456, 7168, 2097144, 2097152, 4194296, 4194304, 2 ** 31 - 8):
