@@ -79,11 +79,14 @@ bool stream_of(PyObject* raw_stream, PyObject* device, void** stream) {
   return !PyErr_Occurred();
 }
 
-template <typename F>
-bool launched(F call) {
+// The C ABI call with the interpreter's lock released. Its arguments are worked out before that, by the caller: the
+// address of a tensor that gives none (a lazily cloned one that cannot be copied, one that must not be written) is an
+// exception, which needs the lock on its way out.
+template <typename... Params, typename... Args>
+bool launched(int (*entry)(Params...), Args... args) {
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = call();
+  rc = entry(args...);
   Py_END_ALLOW_THREADS
   return rc == MOE_A2A_OK;
 }
@@ -217,10 +220,8 @@ PyObject* dispatch_send(PyObject* self, PyObject* const* a, Py_ssize_t n) {
     REFUSE;
   void* stream;
   if (!stream_of(s.raw_stream, s.device_index, &stream)) return nullptr;
-  if (!launched([&] {
-        return moe_a2a_dispatch_send(&s.shape, x->data_ptr(), ints(*idx), (int32_t)T, ws->send_buf.data_ptr(),
-                                     ints(ws->send_meta), ints(ws->send_counts), nullptr, stream);
-      }))
+  if (!launched(moe_a2a_dispatch_send, &s.shape, x->data_ptr(), ints(*idx), (int32_t)T, ws->send_buf.data_ptr(),
+                ints(ws->send_meta), ints(ws->send_counts), nullptr, stream))
     REFUSE;
   return PyLong_FromLongLong(T);
   END_HANDLE_TH_ERRORS
@@ -256,14 +257,12 @@ PyObject* dispatch_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   if (!compact && rows > ws->long_rows) REFUSE;
   void* stream;
   if (!stream_of(s.raw_stream, s.device_index, &stream)) return nullptr;
-  const bool ok = launched([&] {
-    if (compact)
-      return moe_a2a_dispatch_recv_compact(&s.shape, buf->data_ptr(), ints(*meta), ints(*counts), (int32_t)rows,
-                                           (int32_t)capacity, ints(ws->num), ints(ws->offsets), ws->expert_x.data_ptr(),
-                                           ints(ws->expert_meta), (int32_t)ws->expert_x.size(0), ints(ws->plan), stream);
-    return moe_a2a_dispatch_recv(&s.shape, buf->data_ptr(), ints(*meta), ints(*counts), (int32_t)rows, (int32_t)capacity,
-                                 ints(ws->num), ws->expert_x.data_ptr(), ints(ws->expert_meta), ints(ws->plan), stream);
-  });
+  const bool ok =
+      compact ? launched(moe_a2a_dispatch_recv_compact, &s.shape, buf->data_ptr(), ints(*meta), ints(*counts), (int32_t)rows,
+                         (int32_t)capacity, ints(ws->num), ints(ws->offsets), ws->expert_x.data_ptr(), ints(ws->expert_meta),
+                         (int32_t)ws->expert_x.size(0), ints(ws->plan), stream)
+              : launched(moe_a2a_dispatch_recv, &s.shape, buf->data_ptr(), ints(*meta), ints(*counts), (int32_t)rows,
+                         (int32_t)capacity, ints(ws->num), ws->expert_x.data_ptr(), ints(ws->expert_meta), ints(ws->plan), stream);
   if (!ok) REFUSE;
   return PyLong_FromLongLong(rows);
   END_HANDLE_TH_ERRORS
@@ -295,13 +294,11 @@ PyObject* expert_scale(PyObject* self, PyObject* const* a, Py_ssize_t n) {
     REFUSE;
   void* stream;
   if (!stream_of(s.raw_stream, s.device_index, &stream)) return nullptr;
-  const bool ok = launched([&] {
-    if (x->dim() == 2)
-      return moe_a2a_expert_scale_compact(&s.shape, x->data_ptr(), ints(*num), (int32_t)rows, (int32_t)x->size(0), code(s.in),
-                                          code(s.out), ws->expert_y.data_ptr(), stream);
-    return moe_a2a_expert_scale(&s.shape, x->data_ptr(), ints(*num), (int32_t)rows, code(s.in), code(s.out),
-                                ws->expert_y.data_ptr(), stream);
-  });
+  const bool ok =
+      x->dim() == 2 ? launched(moe_a2a_expert_scale_compact, &s.shape, x->data_ptr(), ints(*num), (int32_t)rows,
+                               (int32_t)x->size(0), code(s.in), code(s.out), ws->expert_y.data_ptr(), stream)
+                    : launched(moe_a2a_expert_scale, &s.shape, x->data_ptr(), ints(*num), (int32_t)rows, code(s.in), code(s.out),
+                               ws->expert_y.data_ptr(), stream);
   if (!ok) REFUSE;
   return THPVariable_Wrap(ws->expert_y);
   END_HANDLE_TH_ERRORS
@@ -349,13 +346,12 @@ PyObject* expert_gemm(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   void* stream;
   if (!stream_of(s.raw_stream, s.device_index, &stream)) return nullptr;
   const void* b = bias ? bias->data_ptr() : nullptr;
-  const bool ok = launched([&] {
-    if (x->dim() == 2)
-      return moe_a2a_expert_gemm_compact(&s.shape, x->data_ptr(), ints(*num), (int32_t)rows, (int32_t)x->size(0), w->data_ptr(),
-                                         b, (int32_t)in_dim, (int32_t)out_dim, code(dt), out->data_ptr(), stream);
-    return moe_a2a_expert_gemm(&s.shape, x->data_ptr(), ints(*num), (int32_t)rows, w->data_ptr(), b, (int32_t)in_dim,
-                               (int32_t)out_dim, code(dt), out->data_ptr(), stream);
-  });
+  const bool ok =
+      x->dim() == 2 ? launched(moe_a2a_expert_gemm_compact, &s.shape, x->data_ptr(), ints(*num), (int32_t)rows,
+                               (int32_t)x->size(0), w->data_ptr(), b, (int32_t)in_dim, (int32_t)out_dim, code(dt),
+                               out->data_ptr(), stream)
+                    : launched(moe_a2a_expert_gemm, &s.shape, x->data_ptr(), ints(*num), (int32_t)rows, w->data_ptr(), b,
+                               (int32_t)in_dim, (int32_t)out_dim, code(dt), out->data_ptr(), stream);
   if (!ok) REFUSE;
   return THPVariable_Wrap(*out);
   END_HANDLE_TH_ERRORS
@@ -391,14 +387,12 @@ PyObject* combine_send(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   void* stream;
   if (!stream_of(s.raw_stream, s.device_index, &stream)) return nullptr;
   const int32_t* plan = planned ? ints(ws->back_plan) : nullptr;
-  const bool ok = launched([&] {
-    if (compact)
-      return moe_a2a_combine_send_compact(&s.shape, y->data_ptr(), ints(*meta), ints(*num), (int32_t)rows,
-                                          (int32_t)std::min(y->size(0), meta->size(0)), (int32_t)capacity, ws->back_buf.data_ptr(),
-                                          ints(ws->back_meta), ints(ws->back_counts), plan, stream);
-    return moe_a2a_combine_send(&s.shape, y->data_ptr(), ints(*meta), ints(*num), (int32_t)rows, (int32_t)capacity,
-                                ws->back_buf.data_ptr(), ints(ws->back_meta), ints(ws->back_counts), plan, stream);
-  });
+  const bool ok =
+      compact ? launched(moe_a2a_combine_send_compact, &s.shape, y->data_ptr(), ints(*meta), ints(*num), (int32_t)rows,
+                         (int32_t)std::min(y->size(0), meta->size(0)), (int32_t)capacity, ws->back_buf.data_ptr(),
+                         ints(ws->back_meta), ints(ws->back_counts), plan, stream)
+              : launched(moe_a2a_combine_send, &s.shape, y->data_ptr(), ints(*meta), ints(*num), (int32_t)rows, (int32_t)capacity,
+                         ws->back_buf.data_ptr(), ints(ws->back_meta), ints(ws->back_counts), plan, stream);
   if (!ok) REFUSE;
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -428,11 +422,8 @@ PyObject* combine_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   void* stream;
   if (!stream_of(s.raw_stream, s.device_index, &stream)) return nullptr;
   const int32_t accumulate = a[5] == Py_True;
-  if (!launched([&] {
-        return moe_a2a_combine_recv(&s.shape, buf->data_ptr(), ints(*meta), ints(*counts), (int32_t)rows, (int32_t)capacity,
-                                    static_cast<const float*>(weights->data_ptr()), (int32_t)T, out->data_ptr(), accumulate,
-                                    code(s.out), stream);
-      }))
+  if (!launched(moe_a2a_combine_recv, &s.shape, buf->data_ptr(), ints(*meta), ints(*counts), (int32_t)rows, (int32_t)capacity,
+                static_cast<const float*>(weights->data_ptr()), (int32_t)T, out->data_ptr(), accumulate, code(s.out), stream))
     REFUSE;
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -464,11 +455,9 @@ PyObject* direct_dispatch(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   const void* xs[1] = {x->data_ptr()};
   const int32_t* ids[1] = {ints(*idx)};
   const int32_t tokens[1] = {(int32_t)T};
-  if (!launched([&] {
-        return moe_a2a_local_dispatch(&s.shape, xs, ids, tokens, compact ? (int32_t)ws->direct_x.size(0) : 0, -1, -1,
-                                      ints(ws->where), ints(ws->direct_num), ints(ws->direct_offsets), ws->direct_x.data_ptr(),
-                                      ints(ws->direct_meta), stream);
-      }))
+  if (!launched(moe_a2a_local_dispatch, &s.shape, xs, ids, tokens, compact ? (int32_t)ws->direct_x.size(0) : 0, -1, -1,
+                ints(ws->where), ints(ws->direct_num), ints(ws->direct_offsets), ws->direct_x.data_ptr(), ints(ws->direct_meta),
+                stream))
     REFUSE;
   return PyLong_FromLongLong(T);
   END_HANDLE_TH_ERRORS
@@ -495,9 +484,7 @@ PyObject* direct_combine(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   const float* ws_of[1] = {static_cast<const float*>(weights->data_ptr())};
   void* outs[1] = {out->data_ptr()};
   const int32_t tokens[1] = {(int32_t)T};
-  if (!launched([&] {
-        return moe_a2a_local_combine(&s.shape, y->data_ptr(), ints(ws->where), ws_of, tokens, outs, -1, 1, code(s.out), stream);
-      }))
+  if (!launched(moe_a2a_local_combine, &s.shape, y->data_ptr(), ints(ws->where), ws_of, tokens, outs, -1, 1, code(s.out), stream))
     REFUSE;
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
@@ -527,10 +514,8 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Py_DECREF(index);
   if (!have_stream) return nullptr;
   const Tensor out = at::empty({m, cols}, at::TensorOptions().dtype(dt).device(x->device()));
-  if (!launched([&] {
-        return moe_a2a_linear(x->data_ptr(), w->data_ptr(), bias ? bias->data_ptr() : nullptr, (int32_t)m, (int32_t)cols, (int32_t)k,
-                              code(dt), out.data_ptr(), stream);
-      }))
+  if (!launched(moe_a2a_linear, x->data_ptr(), w->data_ptr(), bias ? bias->data_ptr() : nullptr, (int32_t)m, (int32_t)cols,
+                (int32_t)k, code(dt), out.data_ptr(), stream))
     REFUSE;
   return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
@@ -635,10 +620,8 @@ PyObject* job(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const auto options = at::TensorOptions().device(x[0].device());
   const Tensor rows = at::empty({std::max<int64_t>(entries, 1), H}, options.dtype(out));
   const Tensor where = at::empty({std::max<int64_t>(entries, 1)}, options.dtype(at::kInt));
-  if (!launched([&] {
-        return moe_a2a_local_dispatch(&shape, xs, is, tokens, (int32_t)rows.size(0), code(in), code(out), ints(where), nullptr,
-                                      nullptr, rows.data_ptr(), nullptr, stream);
-      }))
+  if (!launched(moe_a2a_local_dispatch, &shape, xs, is, tokens, (int32_t)rows.size(0), code(in), code(out), ints(where), nullptr,
+                nullptr, rows.data_ptr(), nullptr, stream))
     REFUSE;
   // (a tensor of its own for each rank: views of one would keep all results as long as any of them)
   Tensor y[MAX_RANKS];
@@ -648,10 +631,8 @@ PyObject* job(PyObject*, PyObject* const* a, Py_ssize_t n) {
     y[r] = at::empty({tokens[r], H}, options.dtype(out));
     outs[r] = y[r].data_ptr();
   }
-  if (!launched([&] {
-        return moe_a2a_local_combine(&shape, rows.data_ptr(), ints(where), wts, tokens, outs, everyone ? -1 : (int32_t)own_rank, 0,
-                                     code(out), stream);
-      }))
+  if (!launched(moe_a2a_local_combine, &shape, rows.data_ptr(), ints(where), wts, tokens, outs, everyone ? -1 : (int32_t)own_rank,
+                0, code(out), stream))
     REFUSE;
   if (!everyone) return THPVariable_Wrap(y[own_rank]);
   PyObject* list = PyList_New(W);

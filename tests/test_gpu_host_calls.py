@@ -49,8 +49,15 @@ def strided(t):
     return torch.stack([t, t], dim=-1)[..., 0]
 
 
+def unreadable(t):
+    """A tensor that raises where its address is asked for, as a lazily cloned one does that cannot be copied."""
+    t = t.clone()
+    torch._C._set_throw_on_mutable_data_ptr(t)
+    return t
+
+
 # how an argument may come
-FORMS = {"plain": lambda t: t, "strided": strided, "cpu": lambda t: t.cpu(), "double": lambda t: t.double(), "half": lambda t: t.half(),
+FORMS = {"unreadable": unreadable, "plain": lambda t: t, "strided": strided, "cpu": lambda t: t.cpu(), "double": lambda t: t.double(), "half": lambda t: t.half(),
          "long": lambda t: t.long(), "subclass": lambda t: t.as_subclass(Sub), "parameter": lambda t: torch.nn.Parameter(t, requires_grad=False),
          "flat": lambda t: t.reshape(-1), "short": lambda t: t[:-1], "wide": lambda t: torch.cat([t, t], dim=-1), "tall": lambda t: torch.cat([t, t]),
          "none": lambda t: None, "list": lambda t: t.tolist(), "empty": lambda t: t[:0], "offset": lambda t: torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:].view(t.shape)}
