@@ -23,6 +23,7 @@
 #include <c10/core/impl/DeviceGuardImplInterface.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 
+#include <algorithm>
 #include <memory>
 #include <vector>
 
@@ -312,8 +313,12 @@ PyObject* learn_gemm(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   const Tensor* out = plain(a[0]);
   if (!out || out->dim() < 2) REFUSE;
   auto next = own(s);
-  if (next->gemm.size() >= 16) next->gemm.clear();
-  next->gemm.push_back({out->size(-1), a[1] == Py_True, *out});
+  // (one per width and place, as the rank object owns them: its names are these two)
+  const GemmOut made{out->size(-1), a[1] == Py_True, *out};
+  auto known = std::find_if(next->gemm.begin(), next->gemm.end(),
+                            [&](const GemmOut& g) { return g.out_dim == made.out_dim && g.second == made.second; });
+  if (known == next->gemm.end()) next->gemm.push_back(made);
+  else *known = made;
   s.ws = std::move(next);
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS

@@ -172,6 +172,25 @@ def test_forms_of_a_job_of_one_rank(layout, inter, form):
         assert same(*[outcome(lambda a=a: one_rank(a, d, FORMS[form], at, gemm)) for a in pair]), at
 
 
+def test_results_of_many_widths():
+    """Every width that the rank object has a buffer for, and both buffers where a layer reads the first of its width."""
+    d, a, plain = data(seed=6), rank("padded", True), rank("padded", False)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    num, ex, _ = plain.dispatch(d.x, d.indices)
+    widths = [32 * (i + 1) for i in range(18)]
+    weights = [torch.randn(E, n, H, generator=g, device=DEV).bfloat16() for n in widths]
+    square = torch.randn(E, H, H, generator=g, device=DEV).bfloat16()
+    for w in weights:
+        a.expert_gemm(ex, num, w)
+    first = a.expert_gemm(ex, num, square)
+    a.expert_gemm(first, num, square)
+    for w in weights:
+        got = a._calls.expert_gemm(ex, num, w, None, T * K)
+        assert got is not None and torch.equal(got, plain.expert_gemm(ex, num, w)), w.shape
+    second = a._calls.expert_gemm(a._calls.expert_gemm(ex, num, square, None, T * K), num, square, None, T * K)
+    assert second is not None and torch.equal(second, plain.expert_gemm(plain.expert_gemm(ex, num, square), num, square))
+
+
 def test_workspace_that_changes_and_options_set_later():
     """Other token counts, a buffer replaced by one of another shape, options changed between calls."""
     pair = [rank("padded", native, reuse_placement=True) for native in (True, False)]
