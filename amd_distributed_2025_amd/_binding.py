@@ -274,6 +274,7 @@ class ExtBinding:
                                           recv_meta, recv_counts, rows_hint, stream)
 
 
+KINDS = (CtypesBinding, ExtBinding)
 _BINDINGS = {}
 _host_calls: Optional[dict] = None
 

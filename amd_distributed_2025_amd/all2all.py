@@ -81,15 +81,27 @@ def _refused(*_):
     return None
 
 
-def _rank_calls(shape: "_lib.Shape", cfg: MoEConfig, device):
+def _rank_calls(shape: "_lib.Shape", cfg: MoEConfig, device, binding):
     make = _binding.host_calls().get("RankCalls")
-    if make is None or _raw_stream is None or device.index is None:
+    # (a binding of the caller's own is there to be called)
+    if make is None or _raw_stream is None or device.index is None or type(binding) not in _binding.KINDS:
         return _PythonOnly()
     try:
         return make(tuple(getattr(shape, f) for f, _ in _lib.Shape._fields_), cfg.in_dtype, cfg.out_dtype, device.index,
                     _raw_stream)
     except (TypeError, OverflowError):
         return _PythonOnly()
+
+
+def _option(name: str):
+    """An attribute that decides which buffers a call uses, or how: the native code learns these anew once it is set."""
+    key = "_" + name
+
+    def set_option(self, value):
+        setattr(self, key, value)
+        self._forget()
+
+    return property(lambda self: getattr(self, key), set_option)
 
 
 class HIPAllToAll:
@@ -114,11 +126,11 @@ class HIPAllToAll:
         self.device = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
         if self.device.type != "cuda":
             raise _lib.MoeA2AError("HIPAllToAll needs a GPU device; this path has no CPU fallback")
-        self.binding = _binding.get(binding)  # raises if the native code has not been built
+        self._learned = set()  # calls whose workspace buffers the native code knows
+        self._binding = _binding.get(binding)  # raises if the native code has not been built
         self.shape = _lib.Shape(world_size, rank, cfg.num_experts, cfg.experts_per_token,
                                 cfg.hidden_dim, cfg.max_num_tokens)
-        self._calls = _rank_calls(self.shape, cfg, self.device)
-        self._learned = set()  # calls whose workspace buffers the native code knows
+        self._calls = _rank_calls(self.shape, cfg, self.device, self._binding)
         # rows this rank can receive: every peer may route min(K, nle) entries of each token here
         self.max_rows_in = self.max_recv * min(cfg.experts_per_token, self.num_local_experts)
         self.max_rows_out = cfg.max_num_tokens * cfg.experts_per_token
@@ -128,8 +140,8 @@ class HIPAllToAll:
         # then returns 2-D expert_x / expert_meta, which expert_scale, expert_gemm and combine accept.
         if layout not in ("padded", "compact"):
             raise ValueError(f"layout must be 'padded' or 'compact', got {layout!r}")
-        self.layout = layout
-        self.compact_rows = self.max_rows_in if compact_rows is None else int(compact_rows)
+        self._layout = layout
+        self._compact_rows = self.max_rows_in if compact_rows is None else int(compact_rows)
         if layout == "compact":
             if self.compact_rows < 1:
                 raise ValueError("compact_rows must be at least 1")
@@ -141,11 +153,11 @@ class HIPAllToAll:
         self._send_views = {} # token count -> what dispatch_send returns for it
         # dispatch_recv leaves a plan of where combine_send will put every row; combine_send uses
         # it when it is handed the very tensors that dispatch_recv returned
-        self.reuse_placement = reuse_placement
+        self._reuse_placement = reuse_placement
         self._planned_for = None
         self._plan_made_for = None  # what `_planned_for` is after a dispatch_recv
         self._rows_in_hint = min(self.max_rows_in, self.max_rows_out)  # rows that arrived in the last dispatch
-        self.long_stream_rows = None  # an int overrides both thresholds of LONG_STREAM_ROWS
+        self._long_stream_rows = None  # an int overrides both thresholds of LONG_STREAM_ROWS
         # A job of one rank exchanges with itself, so dispatch() and combine() can move rows straight to
         # their experts and back (moe_a2a_local_dispatch / _combine). Not where a token could have more
         # entries than there are experts (its copies could overflow the receive buffers of the halves, which
@@ -154,23 +166,18 @@ class HIPAllToAll:
                         and cfg.num_experts <= LOCAL_MAX_EXPERTS)
         self._dispatched_for = None  # (expert_meta, expert_num_tokens, tokens) of such a dispatch
 
-    @property
-    def long_stream_rows(self):
-        return self._long_stream_rows
-
-    @long_stream_rows.setter
-    def long_stream_rows(self, rows):
-        self._long_stream_rows = rows
-        self._forget()
+    layout, compact_rows = _option("layout"), _option("compact_rows")
+    long_stream_rows, reuse_placement = _option("long_stream_rows"), _option("reuse_placement")
 
     @property
-    def reuse_placement(self):
-        return self._reuse_placement
+    def binding(self):
+        return self._binding
 
-    @reuse_placement.setter
-    def reuse_placement(self, reuse):
-        self._reuse_placement = reuse
-        self._forget()
+    @binding.setter
+    def binding(self, binding):
+        self._binding = binding
+        self._learned.clear()
+        self._calls = _rank_calls(self.shape, self.cfg, self.device, binding)
 
     # ------------------------------------------------------------------ workspace
 

@@ -212,6 +212,36 @@ def test_workspace_that_changes_and_options_set_later():
     assert "row_position" in pair[0]._ws and "entry_row" in pair[0]._ws
 
 
+class Recorder:
+    """A binding of the caller's own."""
+
+    def __init__(self, binding):
+        self._binding, self.calls = binding, []
+
+    def __getattr__(self, name):
+        call = getattr(self._binding, name)
+        return lambda *a: (self.calls.append(name), call(*a))[1]
+
+
+def test_layout_and_binding_set_later():
+    """Both are read at every call; a binding of the caller's own is the one that is called."""
+    d, pair = data(seed=8), [rank("padded", native) for native in (True, False)]
+    for change in (dict(), dict(layout="compact", compact_rows=T * K + 3), dict(compact_rows=T * K), dict(layout="padded"), dict(binding=_binding.get("ext"))):
+        for a in pair:
+            for name, value in change.items():
+                setattr(a, name, value)
+            if a is pair[1]:
+                a._calls = all2all._PythonOnly()
+        for _ in range(2):
+            got = [outcome(lambda a=a: halves(a, d)) + outcome(lambda a=a: one_rank(a, d)) for a in pair]
+            assert same(*got), change
+    own = pair[0].binding = Recorder(_binding.get("ctypes"))
+    for _ in range(2):
+        own.calls.clear()
+        assert same(outcome(lambda: one_rank(pair[0], d)), got[0][-6:])
+        assert own.calls == ["local_dispatch", "expert_scale", "local_combine"]
+
+
 @pytest.mark.parametrize("form", FORMS)
 @pytest.mark.parametrize("which", ["x", "indices", "weights"])
 def test_forms_of_a_job(form, which, monkeypatch):
