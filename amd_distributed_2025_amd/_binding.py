@@ -17,7 +17,7 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _lib, build
 
 META_DIM = 5
 _DT = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
@@ -281,14 +281,16 @@ _host_calls: Optional[dict] = None
 
 def host_calls() -> dict:
     """What `csrc/host_calls.cpp` offers: `RankCalls`, `linear`, `job`. Empty where the extension has not been built
-    for this library: the Python code above the bindings then does every call by itself."""
+    for this library or was built from other sources than those that are here: the Python code above the bindings then
+    does every call by itself."""
     global _host_calls
     if _host_calls is None:
         try:
             from . import _ext
 
-            _host_calls = _ext.load().a2a_host_calls()
-        except (_lib.MoeA2AError, ImportError, AttributeError):
+            ext = _ext.load()
+            _host_calls = ext.a2a_host_calls() if ext.a2a_extension_id() == build.extension_id() else {}
+        except (_lib.MoeA2AError, ImportError, AttributeError, OSError):  # (OSError: the sources are not here)
             _host_calls = {}
     return _host_calls
 

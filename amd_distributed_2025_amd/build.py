@@ -22,7 +22,8 @@ from pathlib import Path
 PKG_DIR = Path(__file__).resolve().parent
 REPO_DIR = PKG_DIR.parent
 SOURCE = PKG_DIR / "csrc" / "moe_a2a.hip"
-HEADERS = [PKG_DIR / "csrc" / "tile_rules.h", REPO_DIR / "include" / "moe_a2a.h"]
+ABI_HEADER = REPO_DIR / "include" / "moe_a2a.h"
+HEADERS = [PKG_DIR / "csrc" / "tile_rules.h", ABI_HEADER]
 LIBRARY = PKG_DIR / "libmoe_a2a.so"
 EXT_SOURCE = PKG_DIR / "csrc" / "moe_a2a_torch.cpp"
 CALLS_SOURCE = PKG_DIR / "csrc" / "host_calls.cpp"
@@ -34,8 +35,8 @@ EXT_FUNCTIONS = ["a2a_version", "a2a_dispatch_send", "a2a_plan_send", "a2a_dispa
                  "a2a_exchange_gather_local", "a2a_dispatch_recv_compact", "a2a_expert_scale_compact",
                  "a2a_expert_gemm_compact", "a2a_combine_send_compact", "a2a_local_dispatch", "a2a_local_combine"]
 
-# and the calls of the class surface in native code
-EXT_CALLS = ["a2a_host_calls"]
+# and the calls of the class surface in native code, and what they were built from
+EXT_CALLS = ["a2a_host_calls", "a2a_extension_id"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -59,14 +60,23 @@ def hipcc_path() -> str:
     raise RuntimeError("hipcc not found (looked at $HIPCC, PATH and /opt/rocm/bin)")
 
 
-def source_id() -> str:
-    """What `moe_a2a_build_id()` of a library built from the present sources returns."""
+def _hash(*files: Path) -> str:
     import hashlib
 
-    h = hashlib.sha256(SOURCE.read_bytes())
-    for header in HEADERS:
-        h.update(header.read_bytes())
+    h = hashlib.sha256()
+    for f in files:
+        h.update(f.read_bytes())
     return h.hexdigest()[:16]
+
+
+def source_id() -> str:
+    """What `moe_a2a_build_id()` of a library built from the present sources returns."""
+    return _hash(SOURCE, *HEADERS)
+
+
+def extension_id() -> str:
+    """What `a2a_extension_id()` of an extension built from the present sources returns."""
+    return _hash(EXT_SOURCE, CALLS_SOURCE, ABI_HEADER)
 
 
 def build_library(verbose: bool = False) -> Path:
@@ -96,7 +106,7 @@ def build_extension(verbose: bool = False) -> Path:
     EXT_DIR.mkdir(exist_ok=True)
     load_inline(
         name=EXT_NAME,
-        cpp_sources=[EXT_SOURCE.read_text(), CALLS_SOURCE.read_text()],
+        cpp_sources=[f'#define A2A_EXTENSION_ID "{extension_id()}"', EXT_SOURCE.read_text(), CALLS_SOURCE.read_text()],
         functions=EXT_FUNCTIONS + EXT_CALLS,
         extra_cflags=["-O2", "-std=c++17"],
         extra_include_paths=[str(REPO_DIR / "include")],

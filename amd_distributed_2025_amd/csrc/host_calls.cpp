@@ -686,6 +686,9 @@ PyType_Spec rank_spec = {"moe_a2a_torch.RankCalls", sizeof(RankCalls), 0, Py_TPF
 
 }  // namespace host_calls
 
+// what the extension was built from (build.extension_id): the Python code and these calls have to be of one state
+std::string a2a_extension_id() { return A2A_EXTENSION_ID; }
+
 // {"RankCalls": type, "linear": function, "job": function}
 py::dict a2a_host_calls() {
   using namespace host_calls;

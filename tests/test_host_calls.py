@@ -51,3 +51,18 @@ def test_without_the_extension():
     """Every call is refused, so that the Python code does it."""
     none = all2all._PythonOnly()
     assert none.dispatch_send(ROWS, INTS) is None and none.forget() is None and none.learn_send(1, 2, 3) is None
+
+
+def test_an_extension_of_other_sources_is_left_alone(monkeypatch, tmp_path):
+    """The calls are those that the Python code was written with, or none."""
+    from amd_distributed_2025_amd import _ext, build
+
+    assert _ext.load().a2a_extension_id() == build.extension_id()
+    other = tmp_path / "host_calls.cpp"
+    other.write_bytes(build.CALLS_SOURCE.read_bytes() + b"\n")
+    monkeypatch.setattr(build, "CALLS_SOURCE", other)
+    monkeypatch.setattr(_binding, "_host_calls", None)
+    assert _binding.host_calls() == {}
+    monkeypatch.setattr(build, "CALLS_SOURCE", tmp_path / "none.cpp")
+    monkeypatch.setattr(_binding, "_host_calls", None)
+    assert _binding.host_calls() == {}
