@@ -4403,7 +4403,7 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   const int col_tiles = (N + cols - 1) / cols;
   if ((max_rows / 64 + 1) * groups * col_tiles > INT_MAX / 2) return MOE_A2A_EINVAL;
   const int grid = mover_blocks(row_blocks * col_tiles);
-  const bool streamed = weights_past_the_cache(groups, N, K);
+  const bool streamed = weights_past_the_cache(groups, rows_hint, N, K);
 #define LAUNCH_GS(DT, TJ, GW, D, S)                                                                   \
   expert_gemm_kernel<DT, TJ, GW, D, S><<<grid, 64 * GW, 0, st>>>((const b128*)x, rows_of_group, (const b128*)w, \
                                                                  (const uint16_t*)bias, (uint16_t*)y, groups,  \
@@ -4545,7 +4545,7 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   const int grid = mover_blocks((pairs + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
   if (const int rc = allow_large_lds()) return rc;
   // (tiles of one row of tiles per group ask for its weights once; neighbours that ask for them too find them in L2)
-  const bool streamed = weights_past_the_cache(groups, N, K) && rows_hint <= (long long)groups * BM;
+  const bool streamed = weights_past_the_cache(groups, rows_hint, N, K) && rows_hint <= (long long)groups * BM;
   auto launch = [&](auto dtype_const, auto streamed_const) {
     constexpr int DT = decltype(dtype_const)::value;
     constexpr bool S = decltype(streamed_const)::value;

@@ -19,8 +19,19 @@ bool tile_rows_in_range(long long rows, long long K) { return rows * K * 2 < OUT
 // rows, 1024 x 2048, 268 MB 42.8 / 39.2, 2048 x 7168 134.9 / 119.7; 32 groups of 256 rows, 2048 x 4096 133.6 / 125.4,
 // of 100 rows 97.0 / 86.2; 32 of 63, 7168 x 7168 574 / 546). Smaller ones may still be there from the call before,
 // and streaming loads leave nothing behind: 32 groups, 1024 x 2048, 134 MB read again 20.2 / 25.6, 67 MB 12.4 / 14.4.
+// What counts is what is read: no more groups than there are rows. Where that is three quarters of the cache or more,
+// reading it again gains little, and other weights in between cost the most (groups, N x K, rows: the same groups call
+// after call, other groups, another matrix in between): 64, 1024 x 2048, 24 rows, 96 MB 20.4 / 25.9, 20.6 / 26.6, 26.5 /
+// 26.8; 8 rows 18.1 / 18.3, 18.4 / 23.5, 21.6 / 23.5; 128, 1024 x 4096, 16 rows, 128 MB 33.9 / 43.5, 45.5 / 45.2, 46.0 /
+// 45.5; but 64, 1024 x 2048, 48 rows, 192 MB 30.9 / 31.9, 31.2 / 32.1, 36.3 / 32.8; 63 rows 39.1 / 40.7, 39.3 / 40.8, 46.0 /
+// 41.7; and against the rule 64, 2048 x 7168, 8 rows, 224 MB 56.6 / 75.3, 77.6 / 76.7, 78.2 / 76.9; 256, 1024 x 1024, 64
+// rows, 128 MB 24.3 / 22.2, 24.2 / 24.0, 25.0 / 24.4.
 // Where a group has several rows of tiles L2 has to keep its weights between them: 32 of 1000, 7168 x 2048 828 / 835.
-bool weights_past_the_cache(int groups, int N, int K) { return (double)groups * N * K * 2 >= 256.0 * (1 << 20); }
+bool weights_past_the_cache(int groups, long long rows_hint, int N, int K) {
+  constexpr double CACHE = 256.0 * (1 << 20);
+  const double group = (double)N * K * 2;
+  return groups * group >= CACHE && (double)std::min<long long>(groups, rows_hint) * group >= CACHE * 3 / 4;
+}
 
 // How a grouped product is cut: the height of its tiles in bands of 32 rows (10, 8, 6: phased_gemm_kernel, 256
 // columns; 4, 2: dense_gemm_kernel, 128 columns), 0 where rows of K are too long for any. `rows_hint` rows over all

@@ -20,13 +20,14 @@ def rules(tmp_path_factory):
     src = tmp_path_factory.mktemp("rules") / "rules.cpp"
     src.write_text('#include "tile_rules.h"\n'
                    'extern "C" int bands(long long rows_hint, int groups, int n, int k) { return grouped_tile_bands(rows_hint, groups, n, k); }\n'
-                   'extern "C" int past(int groups, int n, int k) { return weights_past_the_cache(groups, n, k); }\n'
+                   'extern "C" int past(int groups, long long rows_hint, int n, int k) { return weights_past_the_cache(groups, rows_hint, n, k); }\n'
                    'extern "C" int way(long long m, long long n, long long k) { return linear_way(m, n, k); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
                     str(src), "-o", str(lib)], check=True)
     dll = C.CDLL(str(lib))
     dll.bands.argtypes = [C.c_longlong, C.c_int, C.c_int, C.c_int]
+    dll.past.argtypes = [C.c_int, C.c_longlong, C.c_int, C.c_int]
     dll.way.argtypes = [C.c_longlong] * 3
     return dll
 
@@ -84,11 +85,14 @@ def test_the_tile_that_the_ring_of_half_steps_is_tested_on(rules, K):
 
 
 def test_weights_past_the_cache(rules):
-    """From 256 MB on (MB of 2^20 bytes), also where the product of the sizes does not fit 64 bits."""
-    assert rules.past(64, 1024, 2048) and not rules.past(64, 1024, 2040) and rules.past(2 ** 31 - 1, 2 ** 31 - 1, 2 ** 31 - 1)
+    """From 256 MB on (MB of 2^20 bytes), also where the product of the sizes does not fit 64 bits, and from 192 MB in as
+    many groups as there are rows."""
+    big = 2 ** 31 - 1
+    assert rules.past(64, 64, 1024, 2048) and not rules.past(64, 64, 1024, 2040) and rules.past(big, big, big, big)
+    assert rules.past(64, 48, 1024, 2048) and not rules.past(64, 47, 1024, 2048) and not rules.past(256, 0, 7168, 7168)
     for (groups, K), tiles in PAST_THE_CACHE.items():
-        assert rules.past(groups, 7168, K)
         for rows, tile in tiles.items():
+            assert rules.past(groups, rows * groups, 7168, K)
             assert not tile or (32 * rules.bands(rows * groups, groups, 7168, K) == tile and rows <= tile)
 
 
