@@ -67,18 +67,29 @@ typedef unsigned int b128 __attribute__((ext_vector_type(4)));
 // THROUGH (device scope) writes on past L2 while the kernel runs. What a plain store leaves dirty there is written
 // back when the kernel ends, with nothing else going on: the 29 MB that stage 2 writes at the headline shape
 // (8 ranks, 2048 rows of 14 KB) cost 15.8 us plain, 14.7 through; the stand-in's rows of a whole job 44.5 and 42.9.
-// (Stage 2, whose waves write whole rows, is better off plain below 8 MB: 16 rows of 14 KB 4.1 / 5.5, 500 of 5.8 KB
-// 4.9 / 5.4, 1024 of 5.8 KB 6.3 / 5.8, 2048 of 5.8 KB 9.6 / 8.4.)
 // The readers lose nothing: the L2s of the XCDs do not serve each other, so they come from behind L2 either way.
+// With little to write back the longer way of each store costs more. Where the line lies, us of the kernel in a graph, plain
+// / through, and of the kernels of a job around it where that tells more:
+//  - stage 2, whose waves write whole rows: about 1000 of them, whatever their length, or 8 MB (10 rows of 5.8 KB 3.45 / 3.98,
+//    715 4.43 / 4.62, 1010 4.96 / 4.93, 1422 6.08 / 5.46; 483 of 14 KB 5.15 / 5.34, 715 5.88 / 5.86, 1010 6.68 / 6.09; 494 of
+//    2 KB 3.71 / 3.92, 2042 6.71 / 6.32; with stages 2 and 3 around the expert 1010 of 8 KB 16.3 / 17.3, 1169 16.8 / 16.5,
+//    1422 of 5.8 KB 16.6 / 15.9, 2042 of 2 KB 13.9 / 12.9).
+//  - stand-in expert and the dispatch of a job whose ranks share the GPU: 1 MB of rows (dispatch: 64 rows of 512 B 3.76 /
+//    3.92, 1.0 MB of them 4.37 / 4.59, 3.9 MB 7.80 / 7.70; 1 MB of 2 KB 3.95 / 4.04, 4 MB 4.77 / 4.63; 7 MB of 14 KB 5.09 /
+//    4.73. Expert: 0.5 MB of 512 B 2.25 / 2.18, 28 MB of 14 KB 9.84 / 7.21. One rank's dispatch, expert and combine: 0.1 MB
+//    of 5.8 KB 10.46 / 10.77, 0.7 MB 10.99 / 11.11, 1.4 MB 11.68 / 11.37, 2.8 MB 13.10 / 12.54).
+//  - exchange: 8 MB of rows for a rank (0.03 MB of 512 B 2.25 / 2.41, 3.9 MB 6.30 / 7.31; 8 MB of 2 KB 5.01 / 5.27, 16 MB 8.46
+//    / 7.80; 3.9 MB of 8 KB 3.18 / 3.31, 6.2 MB 3.67 / 3.61).
 enum Store { PLAIN, THROUGH, STREAM };
+constexpr int STAGE2_THROUGH_ROWS = 1024;
+constexpr long long STAGE2_THROUGH_BYTES = 8 << 20, JOB_THROUGH_BYTES = 1 << 20, EXCHANGE_THROUGH_BYTES = 8 << 20;
+// (a kernel for each kind: chosen inside one, the stores of 5.5 MB of rows took 0.3 us longer than either)
+template <typename V> constexpr Store THROUGH_OF = sizeof(V) == sizeof(b128) ? THROUGH : PLAIN;  // (of 16 bytes only)
 #ifndef MOE_A2A_STORE_SEND   /* stage 1 -> send buffer */
 #define MOE_A2A_STORE_SEND STREAM
 #endif
 #ifndef MOE_A2A_STORE_CSEND  /* stage 3 -> send-back buffer */
 #define MOE_A2A_STORE_CSEND STREAM
-#endif
-#ifndef MOE_A2A_STORE_STANDIN /* expert and exchange stand-ins */
-#define MOE_A2A_STORE_STANDIN THROUGH
 #endif
 #ifndef MOE_A2A_NT_LOAD
 #define MOE_A2A_NT_LOAD 0
@@ -234,15 +245,12 @@ struct Payload {
     for (int j = 0; j < NV; ++j) v[j] = stream_load(row + min(base + j * BLOCK + (int)threadIdx.x, row_vecs - 1));
   }
   template <Store HOW>
-  __device__ __forceinline__ void store_as(V* __restrict__ row, int base, int row_vecs) const {
+  __device__ __forceinline__ void store(V* __restrict__ row, int base, int row_vecs) const {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int idx = base + j * BLOCK + threadIdx.x;
       if (idx < row_vecs) row_store<HOW>(row + idx, v[j]);
     }
-  }
-  __device__ __forceinline__ void store(V* __restrict__ row, int base, int row_vecs) const {
-    store_as<MOE_A2A_STORE_STANDIN>(row, base, row_vecs);
   }
   template <typename F>
   __device__ __forceinline__ void map(F f) {
@@ -573,7 +581,7 @@ __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
           int slot = 0;
 #pragma unroll
           for (int w = 0; w < NWAVES; ++w) slot += half[w * FAN + g];
-          p.template store_as<MOE_A2A_STORE_SEND>(send_buf + (size_t)slot * row_vecs, base, row_vecs);
+          p.template store<MOE_A2A_STORE_SEND>(send_buf + (size_t)slot * row_vecs, base, row_vecs);
         }
       }
       if (c == 0 && tid < live * META) {
@@ -1773,7 +1781,7 @@ __device__ __forceinline__ V standin_expert(V v, float scale) {
   return from_words<V>(h);
 }
 
-template <typename V, int NV, int DIN, int DOUT>
+template <typename V, int NV, int DIN, int DOUT, Store HOW>
 __global__ __launch_bounds__(BLOCK) void expert_scale_kernel(
     const V* __restrict__ expert_x, const int* __restrict__ expert_num_tokens, int nle,
     int max_recv, float scale, int row_vecs, int chunks, V* __restrict__ expert_y, int compact_rows) {
@@ -1792,14 +1800,14 @@ __global__ __launch_bounds__(BLOCK) void expert_scale_kernel(
     Payload<V, NV> p;
     p.load(expert_x + row * row_vecs, base, row_vecs);
     p.map([scale](V v) { return standin_expert<V, DIN, DOUT>(v, scale); });
-    p.store(expert_y + row * row_vecs, base, row_vecs);
+    p.template store<HOW>(expert_y + row * row_vecs, base, row_vecs);
   }
 }
 
 // The same for at most 64 local experts and 16-byte vectors: a wave per (row,
 // chunk of 64 * NVW vectors), the expert prefix in one register per lane, the
 // row found with one ballot. No LDS table, no barrier.
-template <int NVW, int DIN, int DOUT>
+template <int NVW, int DIN, int DOUT, Store HOW>
 __global__ __launch_bounds__(64 * ROWS) void expert_scale_wave_kernel(
     const b128* __restrict__ expert_x, const int* __restrict__ expert_num_tokens, int nle,
     int max_recv, float scale, int row_vecs, int chunks, b128* __restrict__ expert_y, int compact_rows) {
@@ -1817,7 +1825,7 @@ __global__ __launch_bounds__(64 * ROWS) void expert_scale_wave_kernel(
     p.load(expert_x + row * row_vecs, base, row_vecs, lane);
 #pragma unroll
     for (int j = 0; j < NVW; ++j) p.v[j] = standin_expert<b128, DIN, DOUT>(p.v[j], scale);
-    p.template store<MOE_A2A_STORE_STANDIN>(expert_y + row * row_vecs, base, row_vecs, lane);
+    p.template store<HOW>(expert_y + row * row_vecs, base, row_vecs, lane);
   }
 }
 
@@ -3199,7 +3207,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
 
 // ---------------------------------------------------------------- exchange stand-in
 
-template <typename V, int NV>
+template <typename V, int NV, Store HOW>
 __global__ __launch_bounds__(BLOCK) void exchange_local_kernel(
     const V* __restrict__ send_buf, const int* __restrict__ send_meta,
     const int* __restrict__ send_counts, int dst_rank, V* __restrict__ recv_buf,
@@ -3217,7 +3225,7 @@ __global__ __launch_bounds__(BLOCK) void exchange_local_kernel(
     const int base = c * (BLOCK * NV);
     Payload<V, NV> p;
     p.load(send_buf + (size_t)(src_off + i) * row_vecs, base, row_vecs);
-    p.store(recv_buf + (size_t)(dst_off + i) * row_vecs, base, row_vecs);
+    p.template store<HOW>(recv_buf + (size_t)(dst_off + i) * row_vecs, base, row_vecs);
     if (c == 0 && tid < META)
       recv_meta[(size_t)(dst_off + i) * META + tid] = send_meta[(size_t)(src_off + i) * META + tid];
   }
@@ -3236,7 +3244,7 @@ struct GatherSources {
   const int* counts[GATHER_MAX_RANKS];
 };
 
-template <typename V, int NV>
+template <typename V, int NV, Store HOW>
 __global__ __launch_bounds__(BLOCK) void exchange_gather_kernel(
     GatherSources src, int W, int dst_rank, V* __restrict__ recv_buf, int* __restrict__ recv_meta,
     int* __restrict__ recv_counts, int row_vecs, int chunks, int send_capacity_rows,
@@ -3261,7 +3269,7 @@ __global__ __launch_bounds__(BLOCK) void exchange_gather_kernel(
     const int base = c * (BLOCK * NV);
     Payload<V, NV> p;
     p.load(send_buf + (size_t)(src_off + i) * row_vecs, base, row_vecs);
-    p.store(recv_buf + (size_t)(dst_off + i) * row_vecs, base, row_vecs);
+    p.template store<HOW>(recv_buf + (size_t)(dst_off + i) * row_vecs, base, row_vecs);
     if (c == 0 && tid < META)
       recv_meta[(size_t)(dst_off + i) * META + tid] = send_meta[(size_t)(src_off + i) * META + tid];
   }
@@ -3470,7 +3478,7 @@ __global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
 // the rows per expert where the caller wants to know them; else it is read.
 // Measured with a plan launch / ranked here: 8 ranks x 16 tokens, 2 experts of 8 each, hidden 6144 41.7 / 38 us a
 // job, of which the kernels take 5.8 + 4.7 / 8.1.
-template <typename V, int NV, int DIN, int DOUT, int RANKED>
+template <typename V, int NV, int DIN, int DOUT, int RANKED, Store HOW>
 __global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
     LocalSources src, int W, int T, int K, int E, int nle, uint32_t magic, int row_vecs, int chunks, bool compact,
     int max_recv, int expert_limit, int* __restrict__ entry_row, int* __restrict__ expert_num_tokens,
@@ -3608,9 +3616,9 @@ __global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
       const float scale = (float)(1 + (nle == 1 ? e : (int)__umulhi((uint32_t)e, magic)));
       Payload<V, NV> y = p;
       y.map([scale](V v) { return standin_expert<V, DIN, DOUT>(v, scale); });
-      y.store(to, base, row_vecs);
+      y.template store<HOW>(to, base, row_vecs);
     } else {
-      p.store(to, base, row_vecs);
+      p.template store<HOW>(to, base, row_vecs);
     }
   }
   if (c == 0 && meta) {
@@ -4018,7 +4026,8 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   // the stream can hold at most nle * max_recv rows that fit the expert buffers
   if (!items_fit((long long)g.nle * g.max_recv, g.wchunks)) return MOE_A2A_EINVAL;
   const int grid = g.nle + mover_blocks(group_items(rows_hint, g));
-  const bool through = (long long)rows_hint * s->hidden_dim * 2 >= 8 << 20;  // (Store)
+  const bool through =  // (Store)
+      rows_hint >= STAGE2_THROUGH_ROWS || (long long)rows_hint * s->hidden_dim * 2 >= STAGE2_THROUGH_BYTES;
 #define LAUNCH_S(V, NVW, PLAN, MODE, HOW)                                                   \
   dispatch_recv_kernel<V, NVW, PLAN, MODE, HOW><<<grid, 64 * ROWS, 0, st>>>(                     \
       (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, capacity_rows,   \
@@ -4272,6 +4281,7 @@ int launch_expert_scale(const moe_a2a_shape* s, const void* expert_x, const int3
   if (!items_fit(most_rows, g.chunks)) return MOE_A2A_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   const float scale = (float)(1 + s->rank);
+  const bool through = (long long)rows_hint * s->hidden_dim * 2 >= JOB_THROUGH_BYTES;  // (Store)
 #ifndef MOE_A2A_SCALE_WAVES
 #define MOE_A2A_SCALE_WAVES 1
 #endif
@@ -4280,10 +4290,15 @@ int launch_expert_scale(const moe_a2a_shape* s, const void* expert_x, const int3
     const int wchunks = (g.row_vecs + 64 * nvw - 1) / (64 * nvw);
     if (!items_fit(most_rows, wchunks)) return MOE_A2A_EINVAL;
     const int wgrid = mover_blocks(((long long)rows_hint * wchunks + ROWS - 1) / ROWS);
-#define LAUNCH_WT(NVW, DI, DO)                                                                 \
-  expert_scale_wave_kernel<NVW, DI, DO><<<wgrid, 64 * ROWS, 0, st>>>(                          \
+#define LAUNCH_WH(NVW, DI, DO, HOW)                                                            \
+  expert_scale_wave_kernel<NVW, DI, DO, HOW><<<wgrid, 64 * ROWS, 0, st>>>(                     \
       (const b128*)expert_x, expert_num_tokens, g.nle, g.max_recv, scale, g.row_vecs, wchunks,  \
       (b128*)expert_y, compact_rows)
+#define LAUNCH_WT(NVW, DI, DO)                                                                 \
+  do {                                                                                         \
+    if (through) LAUNCH_WH(NVW, DI, DO, THROUGH);                                              \
+    else LAUNCH_WH(NVW, DI, DO, PLAIN);                                                        \
+  } while (0)
 #define LAUNCH_W(NVW)                                                                          \
   do {                                                                                         \
     if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16)                                 \
@@ -4300,13 +4315,19 @@ int launch_expert_scale(const moe_a2a_shape* s, const void* expert_x, const int3
     else LAUNCH_W(4);
 #undef LAUNCH_W
 #undef LAUNCH_WT
+#undef LAUNCH_WH
     return launch_status();
   }
   const int grid = mover_blocks((long long)rows_hint * g.chunks);
-#define LAUNCH_T(V, NV, DI, DO)                                                              \
-  expert_scale_kernel<V, NV, DI, DO><<<grid, BLOCK, 0, st>>>(                                \
+#define LAUNCH_H(V, NV, DI, DO, HOW)                                                         \
+  expert_scale_kernel<V, NV, DI, DO, HOW><<<grid, BLOCK, 0, st>>>(                           \
       (const V*)expert_x, expert_num_tokens, g.nle, g.max_recv, scale, g.row_vecs, g.chunks, \
       (V*)expert_y, compact_rows)
+#define LAUNCH_T(V, NV, DI, DO)                                                              \
+  do {                                                                                       \
+    if (through) LAUNCH_H(V, NV, DI, DO, THROUGH_OF<V>);                                     \
+    else LAUNCH_H(V, NV, DI, DO, PLAIN);                                                     \
+  } while (0)
 #define LAUNCH(V, NV)                                                                         \
   do {                                                                                        \
     if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16)                                \
@@ -4321,6 +4342,7 @@ int launch_expert_scale(const moe_a2a_shape* s, const void* expert_x, const int3
   MOE_A2A_FOR_ROW_KERNEL(g, LAUNCH);
 #undef LAUNCH
 #undef LAUNCH_T
+#undef LAUNCH_H
   return launch_status();
 }
 
@@ -4678,13 +4700,20 @@ int moe_a2a_exchange_local(int32_t world_size, int32_t hidden_dim, const void* s
   row_geometry(g, hidden_dim, all_aligned(16, send_buf, recv_buf));
   if (!items_fit(rows_hint, g.chunks)) return MOE_A2A_EINVAL;
   const int grid = mover_blocks((long long)rows_hint * g.chunks);
+  const bool through = (long long)rows_hint * hidden_dim * 2 >= EXCHANGE_THROUGH_BYTES;  // (Store)
   hipStream_t st = (hipStream_t)stream;
-#define LAUNCH(V, NV)                                                                         \
-  exchange_local_kernel<V, NV><<<grid, BLOCK, 0, st>>>(                                       \
+#define LAUNCH_H(V, NV, HOW)                                                                  \
+  exchange_local_kernel<V, NV, HOW><<<grid, BLOCK, 0, st>>>(                                  \
       (const V*)send_buf, send_meta, send_counts, dst_rank, (V*)recv_buf, recv_meta,          \
       recv_counts, src_rank, g.row_vecs, g.chunks, send_capacity_rows, recv_capacity_rows)
+#define LAUNCH(V, NV)                                    \
+  do {                                                   \
+    if (through) LAUNCH_H(V, NV, THROUGH_OF<V>);         \
+    else LAUNCH_H(V, NV, PLAIN);                         \
+  } while (0)
   MOE_A2A_FOR_ROW_KERNEL(g, LAUNCH);
 #undef LAUNCH
+#undef LAUNCH_H
   return launch_status();
 }
 
@@ -4716,13 +4745,20 @@ int moe_a2a_exchange_gather_local(int32_t world_size, int32_t hidden_dim, const 
   if (!items_fit(rows_hint, g.chunks)) return MOE_A2A_EINVAL;
   // (the launch also delivers the counts, so it is made even when no row can move)
   const dim3 grid(std::min(mover_blocks((long long)rows_hint * g.chunks), 1 << 16), world_size);
+  const bool through = (double)rows_hint * world_size * hidden_dim * 2 >= EXCHANGE_THROUGH_BYTES;  // (Store)
   hipStream_t st = (hipStream_t)stream;
-#define LAUNCH(V, NV)                                                                          \
-  exchange_gather_kernel<V, NV><<<grid, BLOCK, 0, st>>>(src, world_size, dst_rank, (V*)recv_buf, \
-                                                        recv_meta, recv_counts, g.row_vecs, g.chunks, \
-                                                        send_capacity_rows, recv_capacity_rows)
+#define LAUNCH_H(V, NV, HOW)                                                                   \
+  exchange_gather_kernel<V, NV, HOW><<<grid, BLOCK, 0, st>>>(src, world_size, dst_rank, (V*)recv_buf, \
+                                                             recv_meta, recv_counts, g.row_vecs, g.chunks, \
+                                                             send_capacity_rows, recv_capacity_rows)
+#define LAUNCH(V, NV)                                    \
+  do {                                                   \
+    if (through) LAUNCH_H(V, NV, THROUGH_OF<V>);         \
+    else LAUNCH_H(V, NV, PLAIN);                         \
+  } while (0)
   MOE_A2A_FOR_ROW_KERNEL(g, LAUNCH);
 #undef LAUNCH
+#undef LAUNCH_H
   return launch_status();
 }
 
@@ -4794,11 +4830,17 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
         expert_num_tokens, expert_offsets);
     if (S == 0) return launch_status();
   }
+  const bool through = (long long)S * s->hidden_dim * 2 >= JOB_THROUGH_BYTES;  // (Store; with a plan's launch, that is with more entries, always)
   const int grid = (ranked && (expert_num_tokens || expert_offsets) ? 1 : 0) + (int)(tokens * g.chunks);
-#define LAUNCH_T(V, NV, DI, DO, RANKED)                                                                    \
-  local_dispatch_kernel<V, NV, DI, DO, RANKED><<<grid, BLOCK, 0, st>>>(                                    \
+#define LAUNCH_H(V, NV, DI, DO, RANKED, HOW)                                                               \
+  local_dispatch_kernel<V, NV, DI, DO, RANKED, HOW><<<grid, BLOCK, 0, st>>>(                               \
       src, W, (int)tokens, K, E, g.nle, g.magic, g.row_vecs, g.chunks, compact, g.max_recv, expert_limit,  \
       entry_row, expert_num_tokens, expert_offsets, (V*)expert_rows, expert_meta)
+#define LAUNCH_T(V, NV, DI, DO, RANKED)                                                                    \
+  do {                                                                                                     \
+    if (through) LAUNCH_H(V, NV, DI, DO, RANKED, THROUGH_OF<V>);                                           \
+    else LAUNCH_H(V, NV, DI, DO, RANKED, (RANKED > 0 ? PLAIN : THROUGH_OF<V>));                            \
+  } while (0)
 #define LAUNCH_R(V, NV, RANKED)                                                                            \
   do {                                                                                                     \
     if (!standin) LAUNCH_T(V, NV, -1, -1, RANKED);                                                         \
@@ -4817,6 +4859,7 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
 #undef LAUNCH
 #undef LAUNCH_R
 #undef LAUNCH_T
+#undef LAUNCH_H
   return launch_status();
 }
 
