@@ -82,13 +82,14 @@ def _refused(*_):
 
 
 def _rank_calls(shape: "_lib.Shape", cfg: MoEConfig, device, binding):
+    """The native calls of a rank object of this shape (world_size, rank, and the sizes of `cfg`)."""
     make = _binding.host_calls().get("RankCalls")
     # (a binding of the caller's own is there to be called)
     if make is None or _raw_stream is None or device.index is None or type(binding) not in _binding.KINDS:
         return _PythonOnly()
     try:
-        return make(tuple(getattr(shape, f) for f, _ in _lib.Shape._fields_), cfg.in_dtype, cfg.out_dtype, device.index,
-                    _raw_stream)
+        return make((shape.world_size, shape.rank, shape.num_experts, shape.experts_per_token, shape.hidden_dim,
+                     shape.max_num_tokens), cfg.in_dtype, cfg.out_dtype, device.index, _raw_stream)
     except (TypeError, OverflowError):
         return _PythonOnly()
 
@@ -105,9 +106,10 @@ def _option(name: str):
 
 
 class HIPAllToAll:
-    """(The calls below are tried in native code first, `self._calls`, which refuses all but the plain forms; what
-    follows in each method takes every form, raises for the rest, and tells the native code which workspace buffers
-    the call used.)"""
+    """(The calls below are tried in native code first, `self._calls`, which refuses all but the plain forms, and every
+    form until it knows the workspace buffers that the call uses. What follows in each method takes every form, raises
+    for the rest, and tells the native code which buffers those are; a call that has just done so is tried there again,
+    so that the first pass of an object costs no more than the others but for its allocations.)"""
 
     META_DIM = META_DIM  # global_exp, src_rank, src_token, src_k, pad
 
@@ -186,10 +188,13 @@ class HIPAllToAll:
         self._learned.clear()
         self._calls.forget()
 
-    def _learn(self, key, method: str, *buffers) -> None:
-        if key not in self._learned:
-            self._learned.add(key)
-            getattr(self._calls, method)(*buffers)
+    def _learn(self, key, method: str, *buffers) -> bool:
+        """Tell the native code which buffers a call uses; True if it did not know."""
+        if key in self._learned:
+            return False
+        self._learned.add(key)
+        getattr(self._calls, method)(*buffers)
+        return True
 
     def _buf(self, name: str, shape: Tuple[int, ...], dtype: torch.dtype) -> torch.Tensor:
         if self._kept.get(name) != (shape, dtype):
@@ -243,8 +248,9 @@ class HIPAllToAll:
         buf = self._buf("send_buf", (self.max_rows_out, cfg.hidden_dim), cfg.in_dtype)
         meta = self._buf("send_meta", (self.max_rows_out, META_DIM), torch.int32)
         slots = self._buf("send_slot", (self.max_rows_out,), torch.int32) if want_slots else None
-        self.binding.dispatch_send(self.shape, dp_x, indices, T, buf, meta, counts, slots, _stream(self.device))
-        self._learn("send", "learn_send", counts, buf, meta)
+        fresh = self._learn("send", "learn_send", counts, buf, meta)
+        if not (fresh and not want_slots and self._calls.dispatch_send(dp_x, indices) is not None):
+            self.binding.dispatch_send(self.shape, dp_x, indices, T, buf, meta, counts, slots, _stream(self.device))
         if want_slots:
             return counts, buf[:S], meta[:S], slots[:S]
         return self._sent(T)
@@ -298,24 +304,29 @@ class HIPAllToAll:
         nle = self.num_local_experts
         num = self._buf("expert_num_tokens", (nle,), torch.int32)
         plan = self._buf("send_back_plan", (2 * cfg.num_experts,), torch.int32) if self.reuse_placement else None
-        if self.layout == "compact":
+        compact, pos = self.layout == "compact", None
+        if compact:
             ex = self._buf("expert_x", (self.compact_rows, cfg.hidden_dim), cfg.in_dtype)
             em = self._buf("expert_meta", (self.compact_rows, META_DIM), torch.int32)
             self.expert_offsets = self._buf("expert_offsets", (nle + 1,), torch.int32)
-            self.binding.dispatch_recv_compact(self.shape, recv_buf, recv_meta, recv_counts, hint, num,
-                                               self.expert_offsets, ex, em, plan, _stream(self.device))
         else:
             ex = self._buf("expert_x", (nle, self.max_recv, cfg.hidden_dim), cfg.in_dtype)
             em = self._buf("expert_meta", (nle, self.max_recv, META_DIM), torch.int32)
             pos = self._buf("row_position", (capacity,), torch.int32) if hint > self._long_from("dispatch") else None
+        self._plan_made_for = None if plan is None else (em.data_ptr(), num.data_ptr())
+        fresh = self._learn("recv", "learn_recv", num, ex, em, self.expert_offsets if compact else None, plan,
+                            0x7fffffff if compact else self._long_from("dispatch"))
+        if fresh and self._calls.dispatch_recv(recv_counts, recv_buf, recv_meta, hint) is not None:
+            pass
+        elif compact:
+            self.binding.dispatch_recv_compact(self.shape, recv_buf, recv_meta, recv_counts, hint, num,
+                                               self.expert_offsets, ex, em, plan, _stream(self.device))
+        else:
             self.binding.dispatch_recv(self.shape, recv_buf, recv_meta, recv_counts, hint, num, ex, em, plan,
                                        _stream(self.device), pos)
-        self._planned_for = self._plan_made_for = None if plan is None else (em.data_ptr(), num.data_ptr())
+        self._planned_for = self._plan_made_for
         self._dispatched_for = None
         self._rows_in_hint = hint
-        compact = self.layout == "compact"
-        self._learn("recv", "learn_recv", num, ex, em, self.expert_offsets if compact else None, plan,
-                    0x7fffffff if compact else self._long_from("dispatch"))
         return num, ex, em
 
     def expert_scale(self, expert_x, expert_num_tokens, rows_hint: Optional[int] = None):
@@ -328,11 +339,13 @@ class HIPAllToAll:
         _need(expert_num_tokens, torch.int32, self.device, "expert_num_tokens")
         hint = self._default_rows_in(rows_hint)
         ey = self._buf("expert_y", tuple(expert_x.shape), cfg.out_dtype)
+        if (self._learn("scale", "learn_scale", ey)
+                and self._calls.expert_scale(expert_x, expert_num_tokens, hint) is not None):
+            return ey
         if expert_x.dim() == 2:  # the compact layout
             self.binding.expert_scale_compact(self.shape, expert_x, expert_num_tokens, hint, ey, _stream(self.device))
         else:
             self.binding.expert_scale(self.shape, expert_x, expert_num_tokens, hint, ey, _stream(self.device))
-        self._learn("scale", "learn_scale", ey)
         return ey
 
     def expert_gemm(self, expert_x, expert_num_tokens, weights, bias=None, rows_hint: Optional[int] = None,
@@ -377,20 +390,21 @@ class HIPAllToAll:
             if tuple(bias.shape) != (nle, out_dim):
                 raise ValueError(f"bias must be [{nle}, {out_dim}], got {tuple(bias.shape)}")
         hint = self._default_rows_in(rows_hint)
-        own = out is None
-        if own:
+        if out is None:
             name = f"expert_out_{out_dim}"
             if name in self._ws and self._ws[name].data_ptr() == expert_x.data_ptr():
                 name += "_b"  # a layer of equal width reading the buffer the one before it wrote
             out = self._buf(name, rows_shape + (out_dim,), dt)
+            if self._learn(name, "learn_gemm", out, name.endswith("_b")):
+                got = self._calls.expert_gemm(expert_x, expert_num_tokens, weights, bias, hint)
+                if got is not None:
+                    return got
         else:
             _need(out, dt, self.device, "out")
             if tuple(out.shape) != rows_shape + (out_dim,) or out.data_ptr() == expert_x.data_ptr():
                 raise ValueError(f"out must be {list(rows_shape) + [out_dim]} and not the input")
         gemm = self.binding.expert_gemm_compact if compact else self.binding.expert_gemm
         gemm(self.shape, expert_x, expert_num_tokens, hint, weights, bias, out, _stream(self.device))
-        if own:
-            self._learn(name, "learn_gemm", out, name.endswith("_b"))
         return out
 
     def combine_send(self, expert_meta, expert_y, expert_num_tokens, rows_hint: Optional[int] = None):
@@ -421,10 +435,12 @@ class HIPAllToAll:
         plan = None
         if self._planned_for == (expert_meta.data_ptr(), expert_num_tokens.data_ptr()):
             plan = self._ws["send_back_plan"]
+        if (self._learn("back" if plan is None else "back by plan", "learn_back", counts, buf, meta, self._ws.get("send_back_plan"))
+                and self._calls.combine_send(expert_meta, expert_y, expert_num_tokens, hint, self._planned_for)):
+            return counts, buf, meta
         send = self.binding.combine_send_compact if compact else self.binding.combine_send
         send(self.shape, expert_y, expert_meta, expert_num_tokens, min(hint, self.max_rows_in), buf, meta, counts,
              plan, _stream(self.device))
-        self._learn("back" if plan is None else "back by plan", "learn_back", counts, buf, meta, self._ws.get("send_back_plan"))
         return counts, buf, meta
 
     def combine_recv(self, out_tokens, weights, ret_counts, ret_buf, ret_meta, accumulate: bool = True,
@@ -506,13 +522,15 @@ class HIPAllToAll:
         if compact:
             self.expert_offsets = self._buf("expert_offsets", (E + 1,), torch.int32)
         where = self._buf("row_of_entry", (self.max_rows_out,), torch.int32)
-        self.binding.local_dispatch(self.shape, (dp_x,), (indices,), compact, where, num,
-                                    self.expert_offsets if compact else None, ex, em, False, _stream(self.device))
-        self._planned_for = None
+        offsets = self.expert_offsets if compact else None
         self._direct_key = (em.data_ptr(), num.data_ptr())
+        fresh = self._learn("direct", "learn_direct", num, ex, em, where, offsets)
+        if not (fresh and self._calls.direct_dispatch(dp_x, indices) is not None):
+            self.binding.local_dispatch(self.shape, (dp_x,), (indices,), compact, where, num, offsets, ex, em, False,
+                                        _stream(self.device))
+        self._planned_for = None
         self._dispatched_for = (*self._direct_key, T)
         self._rows_in_hint = S
-        self._learn("direct", "learn_direct", num, ex, em, where, self.expert_offsets if compact else None)
         return num, ex, em
 
     def combine(self, out_tokens, weights, expert_meta, expert_y, expert_num_tokens):

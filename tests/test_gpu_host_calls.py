@@ -6,6 +6,7 @@ import torch
 
 from amd_distributed_2025_amd import HIPAllToAll, LocalWorld, MoEConfig, RankTestData, custom_kernel, custom_kernel_job, gemm_rs, set_peer_inputs
 from amd_distributed_2025_amd import _binding, all2all
+from amd_distributed_2025_amd._lib import MoeA2AError
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
@@ -314,6 +315,30 @@ def test_native_calls_are_the_ones_that_run():
         got = one_rank(a, d)[-1]
     side.synchronize()
     assert torch.equal(got, want[0])
+
+
+@pytest.mark.parametrize("layout", ["padded", "compact"])
+def test_the_first_pass_is_native_too(layout):
+    """A new object launches nothing through its binding for plain calls."""
+    d, w = data(seed=4), torch.ones(E, H, H, device=DEV, dtype=torch.bfloat16)
+    for f in (halves, lambda a, d: one_rank(a, d, gemm=(w, w, None))):
+        a = rank(layout, True)
+        a._binding = own = Recorder(a._binding)  # (past the setter: the native calls stay)
+        assert same(outcome(lambda: f(a, d)), outcome(lambda: f(rank(layout, False), d))) and own.calls == []
+
+
+@pytest.mark.parametrize("layout", ["padded", "compact"])
+def test_a_call_that_fails_leaves_no_plan(layout):
+    """The buffers are known from then on, and that none of them is a plan."""
+    d, a = data(seed=4), rank(layout, True)
+    c, b, m = [t.clone() for t in a.dispatch_send(d.x, d.indices)]
+    a.dispatch_recv(c, b, m)
+    a.reuse_placement = False
+    with pytest.raises(MoeA2AError):
+        a.dispatch_recv(c, b, m, -1)
+    assert a._calls.dispatch_recv(c, b, m, T * K) == T * K
+    assert same(outcome(lambda: halves(a, d)), outcome(lambda: halves(rank(layout, False, reuse_placement=False), d)))
+    assert a._planned_for is None
 
 
 def test_wrapped_tensors_are_refused():
