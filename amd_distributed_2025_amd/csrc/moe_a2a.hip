@@ -2821,7 +2821,8 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   static_assert(BM % 64 == 0 && (HALVES ? NA == 2 && HB == 5 && !AHEAD : NA >= 2 && NB >= 2 && NA + NB == 5),
                 "whole loads, and a schedule for the buffers");
   static_assert(!(AHEAD && GROUPED), "tiles that share rows across an XCD");
-  constexpr bool EARLY = !GROUPED;
+  constexpr bool EARLY = !GROUPED && TM == 8;   // a workgroup has several tiles of 256 x 256,
+  constexpr bool ONE_TILE = !GROUPED && !EARLY;  // and one of the lower ones, of which there are fewer (linear_way)
   constexpr bool B_FIRST = NB <= NA;  // the operand with fewer buffers is asked for in the first slice of a step
   constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128, HALF_BYTES = B_BYTES / 2, B_AT = NA * A_BYTES;
   extern __shared__ b128 tile_lds[];  // [NA][BM * 8], [HB][BN * 4]
@@ -2834,7 +2835,7 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   // A workgroup strides over the tiles (the size of the launch is a matter of speed only). EARLY: the first loads of
   // its next tile go out before the results of the last one do, so that they arrive while those are written, and the
   // accumulators are cleared meanwhile. A workgroup per tile / this: 8192 x 8192 x 512 84.5 / 79.0 us, x 3696 370.6 /
-  // 368.3, 4096 x 4096 x 4096 93.5 / 92.4. (Smaller tiles have no next one: linear_way.) Experts' products have
+  // 368.3, 4096 x 4096 x 4096 93.5 / 92.4. Experts' products have
   // a workgroup per tile in general, and the registers for it would be spilled at 320 rows: 140 -> 146 us.
   int tile = blockIdx.x, total_tiles = tiles_m * tiles_n;  // (GROUPED: counted by find_tile)
   int n0, rows_left;         // first column of the tile; rows of the matrix from the tile's first one on
@@ -3131,7 +3132,8 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
   // where there is work to write them behind (8192 x 8192 x 3696 375 / 372 / 369, 416 / 413 / 415), and plain where
   // that would cost the reader more than it gains (8192 x 8192 x 512 83 / 87 / 72, 123 / 127 / 128). Experts' results
   // are streamed, which leaves L2 to the operands: 32 x 256 rows, 4096 x 2048 145 / 144 / 137, 180 / 183 / 177.
-  const bool large = (long long)M * N > (32ll << 20), streams = GROUPED || (large && K >= 2048);
+  // (Tiles of one per workgroup make no results of more than 21 MB: linear_way.)
+  const bool large = !ONE_TILE && (long long)M * N > (32ll << 20), streams = GROUPED || (large && K >= 2048);
   constexpr int VR = TN * 2, PITCH = TN * 32 + 16, ROWS_PER_READ = 64 / VR, BAND_STORES = 16 / ROWS_PER_READ;
   static_assert(8 * 16 * PITCH <= A_BYTES, "results leave through the last buffer of A, which a tile's first loads leave alone");
   char* park = (char*)tile_lds + (NA - 1) * A_BYTES + wave * (16 * PITCH);
@@ -3146,8 +3148,11 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
 #pragma unroll
     for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(bias2[j][0]), "+v"(bias2[j][1]));  // (waited for here, ahead of the loads below)
   }
-  tile += gridDim.x;
-  const bool more = tile < total_tiles;
+  bool more = false;
+  if constexpr (!ONE_TILE) {
+    tile += gridDim.x;
+    more = tile < total_tiles;
+  }
   if (EARLY && more) {
     find_tile();
     begin_tile();
@@ -4515,8 +4520,7 @@ int launch_linear_tiles(const void* a, const void* b, const void* bias, void* c,
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + BN - 1) / BN;
   if (tiles_m * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
   const int grid = (int)(tiles_m * tiles_n);
-  // phased_gemm_kernel strides over its tiles: one workgroup per unit, or two of 128 x 128
-  const int phased_grid = std::min(grid, way == PHASED_128 ? 512 : 256);
+  const int phased_grid = way == PHASED_256 ? std::min(grid, 256) : grid;  // (one per unit, which strides over its tiles)
   if (const int rc = allow_large_lds()) return rc;
 #define LAUNCH_P(DT, TM, TN, AHEAD)                                                              \
   phased_gemm_kernel<DT, TM, TN, 3, 4, AHEAD, false><<<phased_grid, 512, phased_lds_bytes(TM, TN, 3, 4), st>>>( \
