@@ -13,6 +13,26 @@ def bits(t: torch.Tensor) -> np.ndarray:
     return t.detach().cpu().contiguous().view(torch.int16).numpy().view(np.uint16)
 
 
+def reach_the_binding(monkeypatch, binding=None):
+    """Rank objects that are made from here on, and `local_product`, call the binding that they were asked for: plain forms
+    are otherwise done in native code ahead of any binding. Returns the names of its methods that get called."""
+    from amd_distributed_2025_amd import _binding
+
+    monkeypatch.setattr(_binding, "_host_calls", {})
+    called = set()
+    for kind in _binding.KINDS:
+        if binding not in (None, kind.name):
+            continue
+        for name, method in list(vars(kind).items()):
+            if callable(method) and not name.startswith("_"):
+                def seen(*args, _call=method, _name=name, **kw):
+                    called.add(_name)
+                    return _call(*args, **kw)
+
+                monkeypatch.setattr(kind, name, seen)
+    return called
+
+
 def from_bits(a: np.ndarray, dtype: torch.dtype) -> torch.Tensor:
     return torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).view(dtype)
 

@@ -11,7 +11,7 @@ from amd_distributed_2025_amd import HIPAllToAll, LocalWorld, WORKLOADS, generat
 from amd_distributed_2025_amd.all2all import LocalExchange, run_lockstep
 from amd_distributed_2025_amd.task import DTYPES, MoEConfig
 from oracle import moe_a2a_oracle as orc
-from tests.helpers import bits, from_bits, run_oracle
+from tests.helpers import bits, from_bits, reach_the_binding, run_oracle
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -29,11 +29,13 @@ def ref_kernel_body(ata, cfg, rank_data, rank, seen):
 
 @pytest.mark.parametrize("name,binding", [("C1", "ctypes"), ("C2", "ctypes"), ("C2", "ext"), ("C3", "ctypes")])
 @pytest.mark.parametrize("exact_hints", [False, True])
-def test_reference_class_surface_runs_ref_kernel(name, binding, exact_hints):
+def test_reference_class_surface_runs_ref_kernel(name, binding, exact_hints, monkeypatch):
     """Only `dispatch(dp_x, indices)` and `combine(out_tokens, weights, expert_meta, expert_y,
     expert_num_tokens)` are called, one thread per rank as the reference has one process per
     rank; every rank's result and the three returned layouts are checked."""
     print(f"class surface {name} {binding} exact_hints={exact_hints}", flush=True)
+    if binding == "ext":  # (with the other one the native calls do the plain forms)
+        called = reach_the_binding(monkeypatch, binding)
     world = generate_world(WORKLOADS[name], 2025)
     cfg, W = world[0][0], len(world)
     nle, max_recv = cfg.num_experts // W, cfg.max_num_tokens * W
@@ -62,6 +64,8 @@ def test_reference_class_surface_runs_ref_kernel(name, binding, exact_hints):
         assert np.array_equal(bits(rows), want[r].expert_rows), r
         assert np.array_equal(metas.cpu().numpy(), want[r].expert_meta_rows), r
         assert np.array_equal(bits(y), want[r].y), f"rank {r}: combined rows differ from the oracle"
+    if binding == "ext":
+        assert called >= {"dispatch_send", "dispatch_recv", "combine_send", "combine_recv"}
 
 
 def test_single_rank_job_needs_no_exchange_object():
@@ -99,18 +103,24 @@ TRACE_KEYS = ("send_counts", "send_buf", "send_meta", "send_slot", "recv_counts"
 
 
 @pytest.mark.parametrize("name", ["C2", "C3"])
-def test_extension_binding_gives_the_bits_of_the_ctypes_binding(name):
+def test_extension_binding_gives_the_bits_of_the_ctypes_binding(name, monkeypatch):
     """The whole job through the torch extension (torch::Tensor wrappers built by load_inline)
     and through ctypes: every intermediate of every rank is identical, and equals the oracle."""
     print(f"extension vs ctypes {name}", flush=True)
+    reach_the_binding(monkeypatch)
     world = generate_world(WORKLOADS[name], 77)
     cfg, W = world[0][0], len(world)
     dev = [d.to(DEV) for _, d, _, _ in world]
     via_ext = LocalWorld(cfg, W, device=DEV, binding="ext")
     via_ctypes = LocalWorld(cfg, W, device=DEV, binding="ctypes")
     assert via_ext.ranks[0].binding.name == "ext" and via_ctypes.ranks[0].binding.name == "ctypes"
-    ys_e = via_ext.run(dev)
-    ys_c = via_ctypes.run(dev)
+    ys = []
+    for world_of, binding in ((via_ext, "ext"), (via_ctypes, "ctypes")):
+        with monkeypatch.context() as m:
+            called = reach_the_binding(m, binding)
+            ys.append(world_of.run(dev))
+            assert called >= {"dispatch_send", "dispatch_recv", "expert_scale", "combine_send", "combine_recv"}
+    ys_e, ys_c = ys
     torch.cuda.synchronize()
     want = run_oracle(world)
     for r in range(W):

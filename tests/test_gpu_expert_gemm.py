@@ -13,7 +13,7 @@ import torch
 from amd_distributed_2025_amd import LocalWorld, WORKLOADS
 from amd_distributed_2025_amd.task import MoEConfig, dtype_name
 from oracle import moe_a2a_oracle as orc
-from tests.helpers import bits, from_bits
+from tests.helpers import bits, from_bits, reach_the_binding
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -212,14 +212,20 @@ def test_counts_above_the_padding_are_clamped():
     assert np.array_equal(got, want)
 
 
-def test_both_bindings_give_the_same_bits():
+def test_both_bindings_give_the_same_bits(monkeypatch):
+    """Each of them is called; the third result is the native call's."""
     W, nle, H, T = 2, 4, 256, 64
     counts = [128, 7, 0, 90]
     outs = []
     for binding in ("ctypes", "ext"):
-        a, cfg = rank_object(W, nle, H, T, torch.bfloat16, binding)
-        outs.append(run_gemm_same(a, cfg, W, counts, 9, None))
-    assert np.array_equal(outs[0], outs[1])
+        with monkeypatch.context() as m:
+            called = reach_the_binding(m, binding)
+            a, cfg = rank_object(W, nle, H, T, torch.bfloat16, binding)
+            outs.append(run_gemm_same(a, cfg, W, counts, 9, None))
+            assert called == {"expert_gemm"}
+    a, cfg = rank_object(W, nle, H, T, torch.bfloat16)
+    outs.append(run_gemm_same(a, cfg, W, counts, 9, None))
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
 
 
 def test_unsupported_shapes_raise():

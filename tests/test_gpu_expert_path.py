@@ -16,7 +16,7 @@ import torch
 from amd_distributed_2025_amd import LocalWorld, WORKLOADS, generate_world
 from amd_distributed_2025_amd.task import dtype_name
 from oracle import moe_a2a_oracle as orc
-from tests.helpers import bits, run_oracle
+from tests.helpers import bits, reach_the_binding, run_oracle
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -59,12 +59,14 @@ def world_on_gpu(name, seed):
 
 @pytest.mark.parametrize("binding", ["ctypes", "ext"])
 @pytest.mark.parametrize("name,inter", [("C2", 1024), ("C3", 4096), ("C3", 2048), ("C4", None)])
-def test_selection_experts_give_the_oracle_bits(name, inter, binding):
+def test_selection_experts_give_the_oracle_bits(name, inter, binding, monkeypatch):
     """One layer H -> H at C4; two layers H -> inter -> H (inter above, below and equal to H)
     elsewhere: every buffer and `y` bit for bit."""
     if name == "C4" and binding == "ext":
         pytest.skip("the large case runs once; the bindings are compared on the small ones")
     print(f"selection expert {name} inter={inter} {binding}", flush=True)
+    if binding == "ext":  # (with the other one the native calls do the plain forms)
+        reach_the_binding(monkeypatch, binding)
     world, cfg, dev = world_on_gpu(name, 11)
     W, H, dt = len(world), cfg.hidden_dim, cfg.in_dtype
     nle = cfg.num_experts // W

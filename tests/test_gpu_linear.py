@@ -9,9 +9,9 @@ import numpy as np
 import pytest
 import torch
 
-from amd_distributed_2025_amd import gemm_rs
+from amd_distributed_2025_amd import _binding, all2all, gemm_rs
 from oracle import moe_a2a_oracle as orc
-from tests.helpers import bits, from_bits
+from tests.helpers import bits, from_bits, reach_the_binding
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -107,11 +107,21 @@ def test_bias_is_added_to_the_rounded_product():
     assert np.array_equal(orc.linear(bits(x.cpu()), bits(w.cpu()), bits(bias.cpu()), name), bits(out.cpu()))
 
 
-def test_both_bindings_give_the_same_bits():
+def test_both_bindings_give_the_same_bits(monkeypatch):
+    """Each of them is called, and gives what the native call gives."""
     data = gemm_rs.generate_input(0, 8, 512, 4096, 12288, True, 663, device=DEV)
-    a = gemm_rs.local_product(data, binding="ctypes")
-    b = gemm_rs.local_product(data, binding="ext")
-    assert torch.equal(a, b)
+    native = _binding.host_calls()["linear"](all2all._raw_stream, *data)
+    assert native is not None  # (taken, not refused)
+    for binding in ("ctypes", "ext"):
+        with monkeypatch.context() as m:
+            called = reach_the_binding(m, binding)
+            assert torch.equal(gemm_rs.local_product(data, binding=binding), native)
+            assert called == {"linear"}
+    with monkeypatch.context() as m:
+        called = reach_the_binding(m, "ext")
+        out = torch.full_like(native, float("nan"))
+        assert gemm_rs.local_product(data, out=out, binding="ext") is out and torch.equal(out, native)
+        assert called == {"linear"}
 
 
 def test_arguments_are_checked():

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from amd_distributed_2025_amd import HIPAllToAll, LocalWorld, MoEConfig, RankTestData, custom_kernel, custom_kernel_job, set_peer_inputs
+from tests.helpers import reach_the_binding
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -42,8 +43,10 @@ def config(E, K, H, T, din=torch.bfloat16, dout=torch.bfloat16):
     (40, 9, 1032, 33, None), (64, 64, 128, 20, "ids"), (64, 33, 72, 90, None),  # more than eight entries per token
     (1024, 4, 96, 700, None), (16, 8, 512, 300, "twins"), (4, 4, 264, 64, "twins"),
 ])
-def test_one_rank_matches_the_halves(E, K, H, T, spoil, layout, binding):
+def test_one_rank_matches_the_halves(E, K, H, T, spoil, layout, binding, monkeypatch):
     print(f"one rank E={E} K={K} H={H} T={T} {spoil} {layout} {binding}", flush=True)
+    if binding == "ext":  # (with the other one the native calls do the plain forms)
+        called = reach_the_binding(monkeypatch, binding)
     cfg = config(E, K, H, T + 3)  # (room for more tokens than come)
     d = rank_data(cfg, T, 17 + K, spoil)
     direct = HIPAllToAll(cfg, 0, 1, device=DEV, layout=layout, binding=binding)
@@ -64,6 +67,9 @@ def test_one_rank_matches_the_halves(E, K, H, T, spoil, layout, binding):
     assert direct._dispatched_for is not None and halves._dispatched_for is None
     for what, p, q in zip(("counts", "rows", "meta", "result", "offsets"), *got):
         assert (p is None and q is None) or torch.equal(p, q), what
+    if binding == "ext":
+        halves_too = {"dispatch_send", "combine_recv"} | ({"dispatch_recv", "combine_send"} if layout == "padded" else {"dispatch_recv_compact", "combine_send_compact"})
+        assert called >= {"local_dispatch", "local_combine"} | halves_too
 
 
 def test_combine_of_other_tensors_takes_the_halves():

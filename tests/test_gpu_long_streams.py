@@ -8,7 +8,7 @@ import torch
 
 from amd_distributed_2025_amd import LocalWorld, WORKLOADS, generate_world
 from amd_distributed_2025_amd.all2all import LONG_STREAM_ROWS
-from tests.helpers import bits, run_oracle
+from tests.helpers import bits, reach_the_binding, run_oracle
 from tests.test_gpu_parity import DEV, EDGE, assert_rank_matches, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -44,9 +44,12 @@ def test_edge_shapes_through_the_long_stream_entry_points(name):
     run_long(generate_world(spec, 77))
 
 
-def test_extension_binding_and_loose_hints():
+def test_extension_binding_and_loose_hints(monkeypatch):
     world = generate_world(WORKLOADS["C3"], 5)
-    run_long(world, binding="ext")
+    with monkeypatch.context() as m:
+        called = reach_the_binding(m, "ext")
+        run_long(world, binding="ext")
+        assert called >= {"dispatch_recv", "combine_recv"}
     run_long(world, exact_hints=False, accumulate=True, reuse_placement=False)
 
 
