@@ -317,14 +317,68 @@ def test_native_calls_are_the_ones_that_run():
     assert torch.equal(got, want[0])
 
 
+class Answers:
+    """The native calls of a rank object; what each of them answered."""
+
+    def __init__(self, calls):
+        self._calls, self.got = calls, {}
+
+    def __getattr__(self, name):
+        call = getattr(self._calls, name)
+
+        def seen(*args):
+            got = call(*args)
+            if not name.startswith("learn_"):
+                self.got.setdefault(name, []).append(got is not None)
+            return got
+
+        return seen
+
+
+HALVES = {"dispatch_send", "dispatch_recv", "expert_scale", "combine_send", "combine_recv"}
+
+
 @pytest.mark.parametrize("layout", ["padded", "compact"])
-def test_the_first_pass_is_native_too(layout):
-    """A new object launches nothing through its binding for plain calls."""
+@pytest.mark.parametrize("reuse", [True, False])
+def test_every_call_is_native_from_the_first_pass_on(layout, reuse):
+    """A new object launches nothing through its binding for plain calls; from the second pass on no call is refused."""
     d, w = data(seed=4), torch.ones(E, H, H, device=DEV, dtype=torch.bfloat16)
-    for f in (halves, lambda a, d: one_rank(a, d, gemm=(w, w, None))):
-        a = rank(layout, True)
+    of_one = {"direct_dispatch", "direct_combine"} if reuse else HALVES - {"expert_scale"}
+    for f, names in ((halves, HALVES), (one_rank, of_one | {"expert_scale"}), (lambda a, d: one_rank(a, d, gemm=(w, w, None)), of_one | {"expert_gemm"})):
+        a, want = rank(layout, True, reuse_placement=reuse), outcome(lambda: f(rank(layout, False, reuse_placement=reuse), d))
         a._binding = own = Recorder(a._binding)  # (past the setter: the native calls stay)
-        assert same(outcome(lambda: f(a, d)), outcome(lambda: f(rank(layout, False), d))) and own.calls == []
+        assert same(outcome(lambda: f(a, d)), want)
+        a._calls = answers = Answers(a._calls)
+        assert same(outcome(lambda: f(a, d)), want)
+        assert set(own.calls) <= {"gather_sources", "exchange_gather"}  # (the exchange between the halves)
+        taken = {name for name, got in answers.got.items() if all(got)}
+        assert taken >= names and not any(any(got) for name, got in answers.got.items() if name not in names)
+
+
+def test_the_linear_product_and_the_job_are_native(monkeypatch):
+    answers = {}
+
+    def seen(name, call):
+        def f(*args):
+            got = call(*args)
+            answers.setdefault(name, []).append(got is not None)
+            return got
+
+        return f
+
+    monkeypatch.setattr(_binding, "_host_calls", {name: seen(name, call) for name, call in _binding.host_calls().items() if name != "RankCalls"})
+    x, w = torch.ones(20, 128, device=DEV).bfloat16(), torch.ones(96, 128, device=DEV).bfloat16()
+    for bias in (None, w[:, 0].contiguous()):
+        assert gemm_rs.local_product((x, w, bias)).shape == (20, 96)
+    inputs = [(config(), data(t, r), r, W) for r, t in enumerate([T, 3, 0, 7])]
+    custom_kernel_job(inputs)
+    set_peer_inputs(inputs)
+    try:
+        custom_kernel(inputs[1])
+    finally:
+        set_peer_inputs(None)
+    torch.cuda.synchronize()
+    assert answers == {"linear": [True, True], "job": [True, True]}
 
 
 @pytest.mark.parametrize("layout", ["padded", "compact"])
