@@ -57,16 +57,16 @@ def test_task_shapes(m, n, k, has_bias, seed):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-# up to 64 rows and from 8 steps of K: a workgroup's 4 or 8 waves split K among them, 32 or 64 rows at a time
+# from 8 steps of K, where tiles would leave units without work: a workgroup's 4 or 8 waves split K, 32 rows at a time
 @pytest.mark.parametrize("m,n,k", [(1, 32, 512), (64, 96, 520), (33, 2880, 1000), (16, 64, 1600), (64, 96, 1544),
-                                   (32, 32, 3000),
-                                   # else tiles of 64 x 128 (outputs that fill few compute units) ...
-                                   (1, 32, 8), (64, 64, 64), (65, 64, 520), (70, 96, 72), (129, 160, 360), (300, 2880, 200), (70, 64, 1000),
-                                   (200, 160, 1096),
-                                   # ... of 128 x 128 (short K, or too few tiles of 256 x 256 for every unit) ...
-                                   (3000, 2944, 72), (2050, 4128, 200), (4100, 2080, 8), (1000, 4128, 1096),
-                                   # ... and of 256 x 256; ragged last tiles in both directions and a K tail each
-                                   (3900, 4000, 1032)])
+                                   (32, 32, 3000), (65, 64, 520), (70, 64, 1000), (200, 160, 1096),
+                                   # tiles of 64 x 128 (short K, few rows) ...
+                                   (1, 32, 8), (64, 64, 64), (70, 96, 72), (129, 160, 360), (300, 2880, 200),
+                                   # ... of 192 x 128 ...
+                                   (1000, 4128, 1096),
+                                   # ... and of 256 x 256; ragged last tiles in both directions and a K tail each. (WAYS
+                                   # below has shapes of every way, and tests/test_tile_rules.py holds them to it.)
+                                   (3000, 2944, 72), (2050, 4128, 200), (4100, 2080, 8), (3900, 4000, 1032)])
 def test_small_integers_with_bias_are_exact(m, n, k, dt):
     print(f"linear integers m={m} n={n} k={k} {dt}", flush=True)
     rng = np.random.default_rng(m * n + k)
@@ -231,13 +231,20 @@ def test_products_of_one_to_five_steps(m, n, k, dt):
     assert (out[0] == 777.0).all() and (out[m + 1] == 777.0).all()
 
 
+# products of more tiles of 256 x 256 than units, and what the tiles are of which a workgroup has a next one: whole, of too
+# few columns, of 128 to 255 rows, of less (tests/test_tile_rules.py works it out)
+WITH_A_NEXT_TILE = {(4100, 4128): {"whole"}, (5120, 7200): {"whole", "columns"}, (4738, 4128): {"whole", "columns", "half"},
+                    (4736, 4128): {"whole", "columns", "half"}, (4863, 4128): {"whole", "columns", "half"},
+                    (4735, 4128): {"whole", "columns", "less"}, (4613, 4128): {"whole", "columns", "less"}}
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("k", [8, 64, 200, 448])
-@pytest.mark.parametrize("m,n", [(4100, 4128), (5120, 7200)], ids=["289 of 256", "580 of 256"])
+@pytest.mark.parametrize("m,n", WITH_A_NEXT_TILE, ids=["289 of 256", "580 of 256", *[f"{m}x{n}" for m, n in list(WITH_A_NEXT_TILE)[2:]]])
 def test_more_tiles_than_workgroups(m, n, k, bias, dt):
     """Workgroups take a second and a third tile, whose first rows are asked for ahead of the results of the tile
-    before: whole and ragged tiles in front of them. Small integers, whose sums (|x @ w.T + b| <= 448 + 20 here at
+    before, and waited for by counting the stores of that one: as many as whole bands, half as many, none. Small integers, whose sums (|x @ w.T + b| <= 448 + 20 here at
     most, and in fact far below 256) both types hold."""
     print(f"linear m={m} n={n} k={k} bias={bias} {dt}", flush=True)
     g = torch.Generator(device=DEV).manual_seed(m + n + k)

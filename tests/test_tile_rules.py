@@ -8,7 +8,7 @@ import pytest
 
 from tests.test_gpu_expert_gemm import TILES_OF_NARROW
 from tests.test_gpu_grouped_tiles import FEW_STEPS, PAST_THE_CACHE, ROWS_FOR_TILE
-from tests.test_gpu_linear import WAYS
+from tests.test_gpu_linear import WAYS, WITH_A_NEXT_TILE
 
 CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
 
@@ -113,6 +113,27 @@ def test_the_ways_that_the_gpu_tests_mean(rules):
         for m, n in shapes:
             for k in (512, 2048, 8192):
                 assert rules.way(m, n, k) == globals()[name], (m, n, k)
+
+
+@pytest.mark.parametrize("m,n", WITH_A_NEXT_TILE)
+def test_the_tiles_with_a_next_one_that_the_gpu_tests_mean(rules, m, n):
+    """phased_gemm_kernel: workgroup b of 256 takes tiles b, b + 256, ..., whose numbers run through an XCD's share of them
+    (xcd_contiguous) and then down four tile rows before the next tile column (GROUP_M)."""
+    assert all(rules.way(m, n, k) == PHASED_256 for k in (8, 64, 200, 448))
+    tiles_m, tiles_n = -(-m // 256), -(-n // 256)
+    total = tiles_m * tiles_n
+    kinds, places = set(), set()
+    for tile in range(total):
+        xcd, share, rest = tile % 8, total // 8, total % 8
+        number = xcd * share + min(xcd, rest) + tile // 8
+        group, inside = divmod(number, 4 * tiles_n)
+        column, row = divmod(inside, min(4, tiles_m - 4 * group))
+        row += 4 * group
+        places.add((row, column))
+        if tile + 256 < total:
+            rows = min(256, m - 256 * row)
+            kinds.add("columns" if 256 * (column + 1) > n else "whole" if rows == 256 else "half" if rows >= 128 else "less")
+    assert len(places) == total and kinds == WITH_A_NEXT_TILE[m, n]
 
 
 @pytest.mark.parametrize("m,n,k,way", [(112, 1920, 1832, SPLIT_32), (255, 1728, 3968, SPLIT_64), (64, 7168, 2304, SPLIT_64),
