@@ -4,7 +4,9 @@
 `ExtBinding` goes through the torch extension of `csrc/moe_a2a_torch.cpp`, the
 binding idiom of the reference's submissions (all2all/hipv8.py:230-252). Both
 offer the same methods with the same arguments — tensors, sizes and the stream
-handle — and both end in the same kernels, so results are identical. Neither has
+handle — and both end in the same kernels, so results are identical. Calls in plain
+forms do not get here: `host_calls()` has them done in native code, whichever
+binding was asked for. Neither binding has
 a fallback: a missing library or a nonzero status raises.
 
 Capacities (`capacity_rows` of the C ABI) are taken from the tensors: the rows a

@@ -17,7 +17,8 @@ ranks of a job from one thread, half by half, with the same copies. A job of one
 rank has nothing to exchange: its `dispatch` and `combine` are one pass each.
 
 All device work goes through the C ABI in `libmoe_a2a.so`, bound either with
-ctypes or through the torch extension (`binding="ext"`); torch only owns
+ctypes or through the torch extension (`binding="ext"`), and ahead of both, for
+plain forms, by the native calls of csrc/host_calls.cpp; torch only owns
 memory and streams. Buffers live in a per-object workspace allocated once, so
 the tensors returned by `dispatch` are views that stay valid until the next
 `dispatch` on the same object.

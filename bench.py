@@ -89,7 +89,8 @@ def parse_args():
                     help="routing weights of the main workload (default: the workload's own, softmax; the "
                          "reference draws rand, all2all/reference.py:37-43)")
     ap.add_argument("--binding", default="ctypes", choices=["ctypes", "ext"],
-                    help="how the host class reaches the C ABI: ctypes, or the torch extension built with load_inline")
+                    help="how the host class reaches the C ABI where its native calls leave a call to a binding: ctypes, or the "
+                         "torch extension built with load_inline")
     ap.add_argument("--no-extra-workloads", action="store_true",
                     help="skip the C5 block and the C4 block with the reference's input rules (fp16, rand weights)")
     ap.add_argument("--no-entry-points", action="store_true",
@@ -454,7 +455,8 @@ def main():
 
     # ---- the reference's class surface, launch by launch: every rank of the job in a thread of its own
     # calls dispatch() and combine() (all2all/reference.py:259-272 with the stand-in expert), through
-    # each binding; wall time of the whole job, nothing read back from the device in between
+    # objects of each binding (plain calls are the same native ones, the exchange goes through the binding); wall time of
+    # the whole job, nothing read back from the device in between
     def class_surface(binding):
         objs = {}
 

@@ -368,7 +368,9 @@ int moe_a2a_expert_gemm(const moe_a2a_shape* shape, const void* expert_x,
  * rounded value and the sum rounded again, which is what the two torch
  * statements do. bias may be NULL.
  * One of four kernels runs, picked from the shape alone (so a shape always
- * gives the same bits; a slice of the weight's rows is another shape, and where
+ * gives the same bits; other numbers of rows, above 64 too, or of columns are another
+ * shape, in which the same row may be added up in another order and differ in
+ * its last bits; a slice of the weight's rows is another shape as well, and where
  * k is a multiple of 2048 the first of these kernels also starts its sums at an
  * input that depends on the column's place among n): for k >= 449 (eight steps
  * of 64 elements), a kernel whose workgroups own 32 columns and 32 or 64 rows and
