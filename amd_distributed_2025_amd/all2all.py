@@ -130,6 +130,7 @@ class HIPAllToAll:
         if self.device.type != "cuda":
             raise _lib.MoeA2AError("HIPAllToAll needs a GPU device; this path has no CPU fallback")
         self._learned = set()  # calls whose workspace buffers the native code knows
+        self._copied = False   # copy.copy() has been made of it, or made it
         self._binding = _binding.get(binding)  # raises if the native code has not been built
         self.shape = _lib.Shape(world_size, rank, cfg.num_experts, cfg.experts_per_token,
                                 cfg.hidden_dim, cfg.max_num_tokens)
@@ -180,7 +181,15 @@ class HIPAllToAll:
     def binding(self, binding):
         self._binding = binding
         self._learned.clear()
-        self._calls = _rank_calls(self.shape, self.cfg, self.device, binding)
+        self._calls = _PythonOnly() if self._copied else _rank_calls(self.shape, self.cfg, self.device, binding)
+
+    def __copy__(self):
+        """A copy shares the workspace, and either object may replace a buffer that the other's native calls have learned:
+        the Python code, which looks a buffer up for every call, does the calls of both."""
+        twin = object.__new__(type(self))
+        self._copied, self._calls = True, _PythonOnly()
+        twin.__dict__.update(self.__dict__)
+        return twin
 
     # ------------------------------------------------------------------ workspace
 

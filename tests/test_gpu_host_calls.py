@@ -1,5 +1,7 @@
 """The calls of the class surface in native code (csrc/host_calls.cpp) against the Python code that takes every form:
 whatever the form of a call, both give the same result or raise the same error."""
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -241,6 +243,30 @@ def test_layout_and_binding_set_later():
         own.calls.clear()
         assert same(outcome(lambda: one_rank(pair[0], d)), got[0][-6:])
         assert own.calls == ["local_dispatch", "expert_scale", "local_combine"]
+
+
+def test_copies_share_a_workspace():
+    """A copy with another layout takes turns with the object it was made of."""
+    d = data()
+    a = HIPAllToAll(config(), 0, 1, device=DEV)
+    a.dispatch_recv(*a.dispatch_send(d.x, d.indices))
+    b = copy.copy(a)
+    b.layout = "compact"
+    b.binding = _binding.get("ext")
+    for _ in range(2):
+        for of, dims in ((a, 3), (b, 2), (a, 3)):
+            num, ex, em = of.dispatch_recv(*of.dispatch_send(d.x, d.indices))
+            assert ex.dim() == em.dim() == dims
+            fresh = HIPAllToAll(config(), 0, 1, device=DEV, layout=of.layout)
+            fnum, fex, fem = fresh.dispatch_recv(*fresh.dispatch_send(d.x, d.indices))
+            assert torch.equal(num, fnum)
+            for e, n in enumerate(num.tolist()):
+                at = slice(int(num[:e].sum()), int(num[:e].sum()) + n)
+                assert torch.equal(ex[e, :n], fex[e, :n]) if dims == 3 else torch.equal(ex[at], fex[at])
+            y, fy = torch.zeros(T, H, dtype=torch.bfloat16, device=DEV), torch.zeros(T, H, dtype=torch.bfloat16, device=DEV)
+            of.combine_recv(y, d.weights, *of.combine_send(em, of.expert_scale(ex, num), num))
+            fresh.combine_recv(fy, d.weights, *fresh.combine_send(fem, fresh.expert_scale(fex, fnum), fnum))
+            assert torch.equal(y, fy)
 
 
 @pytest.mark.parametrize("form", FORMS)

@@ -1,5 +1,7 @@
 """csrc/host_calls.cpp without a GPU: whatever is not a plain tensor on the rank's GPU is refused before anything is
 launched, and the class surface does without the extension."""
+import copy
+
 import pytest
 import torch
 
@@ -66,3 +68,14 @@ def test_an_extension_of_other_sources_is_left_alone(monkeypatch, tmp_path):
     monkeypatch.setattr(build, "CALLS_SOURCE", tmp_path / "none.cpp")
     monkeypatch.setattr(_binding, "_host_calls", None)
     assert _binding.host_calls() == {}
+
+
+def test_a_copied_object_and_its_copy_use_no_learned_buffers():
+    """They share a workspace: what one of them replaces the other's native calls would go on using."""
+    a = object.__new__(all2all.HIPAllToAll)
+    a.__dict__.update(_learned={"recv"}, _copied=False, _calls="native calls", _ws={}, _layout="padded")
+    b = copy.copy(a)
+    b.layout = "compact"
+    assert type(a._calls) is type(b._calls) is all2all._PythonOnly and b._ws is a._ws and a.layout == "padded"
+    b.binding = object()
+    assert type(b._calls) is all2all._PythonOnly
