@@ -26,6 +26,7 @@ the tensors returned by `dispatch` are views that stay valid until the next
 from __future__ import annotations
 
 import threading
+from operator import attrgetter
 from typing import Callable, List, Optional, Sequence, Tuple
 
 import torch
@@ -88,9 +89,11 @@ def _rank_calls(shape: "_lib.Shape", cfg: MoEConfig, device, binding):
     # (a binding of the caller's own is there to be called)
     if make is None or _raw_stream is None or device.index is None or type(binding) not in _binding.KINDS:
         return _PythonOnly()
+    sizes = (shape.num_experts, shape.experts_per_token, shape.hidden_dim, shape.max_num_tokens)
+    if sizes != (cfg.num_experts, cfg.experts_per_token, cfg.hidden_dim, cfg.max_num_tokens):
+        return _PythonOnly()  # (one of the two was set alone: the Python code checks by the one and launches by the other)
     try:
-        return make((shape.world_size, shape.rank, shape.num_experts, shape.experts_per_token, shape.hidden_dim,
-                     shape.max_num_tokens), cfg.in_dtype, cfg.out_dtype, device.index, _raw_stream)
+        return make((shape.world_size, shape.rank, *sizes), cfg.in_dtype, cfg.out_dtype, device.index, _raw_stream, cfg)
     except (TypeError, OverflowError):
         return _PythonOnly()
 
@@ -103,7 +106,19 @@ def _option(name: str):
         setattr(self, key, value)
         self._forget()
 
-    return property(lambda self: getattr(self, key), set_option)
+    return property(attrgetter(key), set_option)
+
+
+def _part(name: str):
+    """An attribute that the native calls were made from: they are made anew once it is set."""
+    key = "_" + name
+
+    def set_part(self, value):
+        setattr(self, key, value)
+        self._learned.clear()
+        self._calls = _PythonOnly() if self._copied else _rank_calls(self._shape, self._cfg, self.device, self._binding)
+
+    return property(attrgetter(key), set_part)
 
 
 class HIPAllToAll:
@@ -119,7 +134,7 @@ class HIPAllToAll:
                  compact_rows: Optional[int] = None):
         if cfg.num_experts % world_size:
             raise ValueError("num_experts must be a multiple of world_size")
-        self.cfg = cfg
+        self._cfg = cfg
         self.rank = rank
         self.world_size = world_size
         self.num_local_experts = cfg.num_experts // world_size
@@ -132,12 +147,12 @@ class HIPAllToAll:
         self._learned = set()  # calls whose workspace buffers the native code knows
         self._copied = False   # copy.copy() has been made of it, or made it
         self._binding = _binding.get(binding)  # raises if the native code has not been built
-        self.shape = _lib.Shape(world_size, rank, cfg.num_experts, cfg.experts_per_token,
-                                cfg.hidden_dim, cfg.max_num_tokens)
-        self._calls = _rank_calls(self.shape, cfg, self.device, self._binding)
+        self._shape = _lib.Shape(world_size, rank, cfg.num_experts, cfg.experts_per_token,
+                                 cfg.hidden_dim, cfg.max_num_tokens)
+        self._calls = _rank_calls(self._shape, cfg, self.device, self._binding)
         # rows this rank can receive: every peer may route min(K, nle) entries of each token here
-        self.max_rows_in = self.max_recv * min(cfg.experts_per_token, self.num_local_experts)
-        self.max_rows_out = cfg.max_num_tokens * cfg.experts_per_token
+        self._max_rows_in = self.max_recv * min(cfg.experts_per_token, self.num_local_experts)
+        self._max_rows_out = cfg.max_num_tokens * cfg.experts_per_token
         # "padded": the reference's expert buffers [nle, max_recv, H] (all2all/reference.py:123-136).
         # "compact": the experts' rows back to back in buffers of `compact_rows` rows (default: every
         # row the rank can receive), row pos of expert le at expert_offsets[le] + pos; dispatch()
@@ -145,12 +160,12 @@ class HIPAllToAll:
         if layout not in ("padded", "compact"):
             raise ValueError(f"layout must be 'padded' or 'compact', got {layout!r}")
         self._layout = layout
-        self._compact_rows = self.max_rows_in if compact_rows is None else int(compact_rows)
+        self._compact_rows = self._max_rows_in if compact_rows is None else int(compact_rows)
         if layout == "compact":
-            if self.compact_rows < 1:
+            if self._compact_rows < 1:
                 raise ValueError("compact_rows must be at least 1")
             # a rank that keeps at most compact_rows rows needs no room to receive or return more
-            self.max_rows_in = min(self.max_rows_in, self.compact_rows)
+            self._max_rows_in = min(self._max_rows_in, self._compact_rows)
         self.expert_offsets = None  # compact layout: int32[nle + 1], written by dispatch_recv
         self._ws = {}
         self._kept = {}       # what _buf made them for: name -> (shape, dtype)
@@ -160,7 +175,7 @@ class HIPAllToAll:
         self._reuse_placement = reuse_placement
         self._planned_for = None
         self._plan_made_for = None  # what `_planned_for` is after a dispatch_recv
-        self._rows_in_hint = min(self.max_rows_in, self.max_rows_out)  # rows that arrived in the last dispatch
+        self._rows_in_hint = min(self._max_rows_in, self._max_rows_out)  # rows that arrived in the last dispatch
         self._long_stream_rows = None  # an int overrides both thresholds of LONG_STREAM_ROWS
         # A job of one rank exchanges with itself, so dispatch() and combine() can move rows straight to
         # their experts and back (moe_a2a_local_dispatch / _combine). Not where a token could have more
@@ -172,16 +187,8 @@ class HIPAllToAll:
 
     layout, compact_rows = _option("layout"), _option("compact_rows")
     long_stream_rows, reuse_placement = _option("long_stream_rows"), _option("reuse_placement")
-
-    @property
-    def binding(self):
-        return self._binding
-
-    @binding.setter
-    def binding(self, binding):
-        self._binding = binding
-        self._learned.clear()
-        self._calls = _PythonOnly() if self._copied else _rank_calls(self.shape, self.cfg, self.device, binding)
+    max_rows_in, max_rows_out = _option("max_rows_in"), _option("max_rows_out")
+    binding, shape, cfg = _part("binding"), _part("shape"), _part("cfg")
 
     def __copy__(self):
         """A copy shares the workspace, and either object may replace a buffer that the other's native calls have learned:
@@ -210,6 +217,7 @@ class HIPAllToAll:
         if self._kept.get(name) != (shape, dtype):
             if name in self._ws:
                 self._forget()
+                self._send_views.clear()
             self._ws[name] = torch.empty(shape, dtype=dtype, device=self.device)
             self._kept[name] = (shape, dtype)
         return self._ws[name]
@@ -295,7 +303,7 @@ class HIPAllToAll:
         """Received stream -> (expert_num_tokens[nle], expert_x[nle,max_recv,H],
         expert_meta[nle,max_recv,5]); rows past expert_num_tokens[le] are not written."""
         hint = self._calls.dispatch_recv(recv_counts, recv_buf, recv_meta,
-                                         self.max_rows_out if rows_hint is None else rows_hint)
+                                         self._max_rows_out if rows_hint is None else rows_hint)
         if hint is not None:
             self._planned_for = self._plan_made_for
             self._dispatched_for = None
@@ -506,7 +514,7 @@ class HIPAllToAll:
             if T is not None:
                 self._planned_for = None
                 self._dispatched_for = (*self._direct_key, T)
-                self._rows_in_hint = T * self.cfg.experts_per_token
+                self._rows_in_hint = T * self._cfg.experts_per_token
                 ws = self._ws
                 return ws["expert_num_tokens"], ws["expert_x"], ws["expert_meta"]
             S = indices.shape[0] * self.cfg.experts_per_token

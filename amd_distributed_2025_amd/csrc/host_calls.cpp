@@ -71,6 +71,23 @@ bool same_address(PyObject* o, const Tensor& t) {
   return PyLong_CheckExact(o) && PyLong_AsVoidPtr(o) == t.data_ptr();
 }
 
+struct Names {
+  PyObject *num_experts, *experts_per_token, *hidden_dim, *max_num_tokens, *in_dtype, *out_dtype, *x, *indices, *weights;
+};
+Names names;
+
+bool type_of(PyObject* cfg, PyObject* name, ScalarType* dt) {
+  PyObject* o = PyObject_GetAttr(cfg, name);
+  if (!o) {
+    PyErr_Clear();
+    return false;
+  }
+  const bool ok = THPDtype_Check(o);
+  if (ok) *dt = reinterpret_cast<THPDtype*>(o)->scalar_type;
+  Py_DECREF(o);
+  return ok;
+}
+
 // the current stream of a device; false with an exception set
 bool stream_of(PyObject* raw_stream, PyObject* device, void** stream) {
   PyObject* r = PyObject_CallFunctionObjArgs(raw_stream, device, nullptr);
@@ -116,6 +133,7 @@ struct State {
   ScalarType in, out;
   std::shared_ptr<Workspace> ws = std::make_shared<Workspace>();
   PyObject *raw_stream = nullptr, *device_index = nullptr;
+  PyObject* cfg = nullptr;  // where the row types come from, if the rank object has said so
 };
 
 struct RankCalls {
@@ -128,11 +146,11 @@ State& state(PyObject* self) { return *reinterpret_cast<RankCalls*>(self)->s; }
 PyObject* rank_new(PyTypeObject* type, PyObject* args, PyObject*) {
   HANDLE_TH_ERRORS
   int32_t f[6];
-  PyObject *in, *out, *device, *raw;
-  if (!PyArg_ParseTuple(args, "(iiiiii)OOOO", &f[0], &f[1], &f[2], &f[3], &f[4], &f[5], &in, &out, &device, &raw)) return nullptr;
+  PyObject *in, *out, *device, *raw, *cfg = nullptr;
+  if (!PyArg_ParseTuple(args, "(iiiiii)OOOO|O", &f[0], &f[1], &f[2], &f[3], &f[4], &f[5], &in, &out, &device, &raw, &cfg)) return nullptr;
   if (!THPDtype_Check(in) || !THPDtype_Check(out) || !PyLong_CheckExact(device) || f[0] < 1) {
     PyErr_SetString(PyExc_TypeError, "RankCalls((world_size, rank, num_experts, experts_per_token, hidden_dim, "
-                                     "max_num_tokens), in_dtype, out_dtype, device_index, raw_stream)");
+                                     "max_num_tokens), in_dtype, out_dtype, device_index, raw_stream, cfg=None)");
     return nullptr;
   }
   PyObject* self = type->tp_alloc(type, 0);
@@ -151,6 +169,10 @@ PyObject* rank_new(PyTypeObject* type, PyObject* args, PyObject*) {
   s->raw_stream = raw;
   Py_INCREF(device);
   s->device_index = device;
+  if (cfg && cfg != Py_None) {
+    Py_INCREF(cfg);
+    s->cfg = cfg;
+  }
   return self;
   END_HANDLE_TH_ERRORS
 }
@@ -160,6 +182,7 @@ void rank_dealloc(PyObject* self) {
   if (s) {
     Py_XDECREF(s->raw_stream);
     Py_XDECREF(s->device_index);
+    Py_XDECREF(s->cfg);
     delete s;
   }
   PyTypeObject* type = Py_TYPE(self);
@@ -171,6 +194,15 @@ PyObject* rank_forget(PyObject* self, PyObject*) {
   state(self).ws = std::make_shared<Workspace>();
   Py_RETURN_NONE;
 }
+
+// Whether rows are there (`t`, a workspace buffer or an argument) and of the type that these calls were made for, which the
+// config still names: a caller may set its types between two calls, and the Python code then makes the buffers anew.
+bool known(const State& s, const Tensor& t, PyObject* name, ScalarType made_for) {
+  ScalarType now;
+  return t.defined() && t.scalar_type() == made_for && (!s.cfg || (type_of(s.cfg, name, &now) && now == made_for));
+}
+bool known_in(const State& s, const Tensor& t) { return known(s, t, names.in_dtype, s.in); }
+bool known_out(const State& s, const Tensor& t) { return known(s, t, names.out_dtype, s.out); }
 
 #define REFUSE Py_RETURN_NONE
 #define TAKES(N)                                                          \
@@ -214,7 +246,7 @@ PyObject* dispatch_send(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   State& s = state(self);
   const auto ws = s.ws;
   const Tensor *x = plain(a[0]), *idx = plain(a[1]);
-  if (!ws->send_buf.defined() || !x || !idx || idx->dim() != 2) REFUSE;
+  if (!known_in(s, ws->send_buf) || !x || !idx || idx->dim() != 2) REFUSE;
   const int64_t T = idx->size(0);
   if (T > s.shape.max_num_tokens || idx->size(1) != s.topk || !shaped(*x, T, s.hidden) || !dense(*x, s.in, s.device) ||
       !dense(*idx, at::kInt, s.device))
@@ -246,7 +278,7 @@ PyObject* dispatch_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   const auto ws = s.ws;
   const Tensor *counts = plain(a[0]), *buf = plain(a[1]), *meta = plain(a[2]);
   int64_t rows;
-  if (!ws->expert_x.defined() || !counts || !buf || !meta || !count(a[3], &rows)) REFUSE;
+  if (!known_in(s, ws->expert_x) || !counts || !buf || !meta || !count(a[3], &rows)) REFUSE;
   if (buf->dim() != 2 || buf->size(1) != s.hidden || meta->dim() != 2 || meta->size(1) != MOE_A2A_META_DIM ||
       counts->numel() < s.shape.world_size || !dense(*counts, at::kInt, s.device) || !dense(*buf, s.in, s.device) ||
       !dense(*meta, at::kInt, s.device))
@@ -289,7 +321,7 @@ PyObject* expert_scale(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   const auto ws = s.ws;
   const Tensor *x = plain(a[0]), *num = plain(a[1]);
   int64_t rows;
-  if (!ws->expert_y.defined() || !x || !num || !count(a[2], &rows)) REFUSE;
+  if (!x || !known_in(s, *x) || !known_out(s, ws->expert_y) || !num || !count(a[2], &rows)) REFUSE;
   if (!row_type(s.in) || !row_type(s.out) || !expert_rows(s, *x, s.hidden) || x->sizes() != ws->expert_y.sizes() ||
       num->numel() < s.nle || !dense(*x, s.in, s.device) || !dense(*num, at::kInt, s.device))
     REFUSE;
@@ -378,7 +410,7 @@ PyObject* combine_send(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   const auto ws = s.ws;
   const Tensor *meta = plain(a[0]), *y = plain(a[1]), *num = plain(a[2]);
   int64_t rows;
-  if (!ws->back_buf.defined() || !meta || !y || !num || !count(a[3], &rows)) REFUSE;
+  if (!known_out(s, ws->back_buf) || !meta || !y || !num || !count(a[3], &rows)) REFUSE;
   const bool compact = y->dim() == 2;
   if (!row_type(s.out) || !expert_rows(s, *y, s.hidden) || num->numel() < s.nle || !dense(*y, s.out, s.device) ||
       !dense(*meta, at::kInt, s.device) || !dense(*num, at::kInt, s.device) ||
@@ -417,7 +449,7 @@ PyObject* combine_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   State& s = state(self);
   const Tensor *out = plain(a[0]), *weights = plain(a[1]), *counts = plain(a[2]), *buf = plain(a[3]), *meta = plain(a[4]);
   int64_t long_rows;
-  if (!out || !weights || !counts || !buf || !meta || !PyBool_Check(a[5]) || !count(a[6], &long_rows)) REFUSE;
+  if (!out || !known_out(s, *out) || !weights || !counts || !buf || !meta || !PyBool_Check(a[5]) || !count(a[6], &long_rows)) REFUSE;
   if (!takes_results(s, *out, *weights) || buf->dim() != 2 || buf->size(1) != s.hidden || meta->dim() != 2 ||
       meta->size(1) != MOE_A2A_META_DIM || counts->numel() < s.shape.world_size || !dense(*counts, at::kInt, s.device) ||
       !dense(*buf, s.out, s.device) || !dense(*meta, at::kInt, s.device))
@@ -449,7 +481,7 @@ PyObject* direct_dispatch(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   State& s = state(self);
   const auto ws = s.ws;
   const Tensor *x = plain(a[0]), *idx = plain(a[1]);
-  if (!ws->where.defined() || !x || !idx || idx->dim() != 2) REFUSE;
+  if (!ws->where.defined() || !known_in(s, ws->direct_x) || !x || !idx || idx->dim() != 2) REFUSE;
   const int64_t T = idx->size(0);
   const bool compact = ws->direct_offsets.defined();
   if (T > s.shape.max_num_tokens || idx->size(1) != s.topk || !shaped(*x, T, s.hidden) || !dense(*x, s.in, s.device) ||
@@ -475,7 +507,7 @@ PyObject* direct_combine(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   State& s = state(self);
   const auto ws = s.ws;
   const Tensor *out = plain(a[0]), *weights = plain(a[1]), *meta = plain(a[2]), *y = plain(a[3]), *num = plain(a[4]);
-  if (!ws->where.defined() || !out || !weights || !meta || !y || !num || !PyTuple_CheckExact(a[5]) || PyTuple_GET_SIZE(a[5]) != 3) REFUSE;
+  if (!ws->where.defined() || !out || !known_out(s, *out) || !weights || !meta || !y || !num || !PyTuple_CheckExact(a[5]) || PyTuple_GET_SIZE(a[5]) != 3) REFUSE;
   if (!takes_results(s, *out, *weights) || !dense(*y, s.out, s.device)) REFUSE;
   const int64_t T = weights->size(0);
   int64_t tokens_dispatched;
@@ -526,11 +558,6 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-struct Names {
-  PyObject *num_experts, *experts_per_token, *hidden_dim, *max_num_tokens, *in_dtype, *out_dtype, *x, *indices, *weights;
-};
-Names names;
-
 bool number_of(PyObject* cfg, PyObject* name, int64_t* v) {  // false without an exception: not a plain count
   PyObject* o = PyObject_GetAttr(cfg, name);
   if (!o) {
@@ -540,18 +567,6 @@ bool number_of(PyObject* cfg, PyObject* name, int64_t* v) {  // false without an
   const bool ok = count(o, v);
   Py_DECREF(o);
   return ok;
-}
-
-bool type_of(PyObject* cfg, PyObject* name, ScalarType* dt) {
-  PyObject* o = PyObject_GetAttr(cfg, name);
-  if (!o) {
-    PyErr_Clear();
-    return false;
-  }
-  const bool ok = THPDtype_Check(o);
-  if (ok) *dt = reinterpret_cast<THPDtype*>(o)->scalar_type;
-  Py_DECREF(o);
-  return ok && row_type(*dt);
 }
 
 bool tensor_of(PyObject* data, PyObject* name, Tensor* t) {
@@ -581,6 +596,7 @@ PyObject* job(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!(PyList_CheckExact(inputs) || PyTuple_CheckExact(inputs)) || PySequence_Fast_GET_SIZE(inputs) != W) REFUSE;
   if (!number_of(cfg, names.num_experts, &E) || !number_of(cfg, names.experts_per_token, &K) || !number_of(cfg, names.hidden_dim, &H) ||
       !number_of(cfg, names.max_num_tokens, &max_tokens) || !type_of(cfg, names.in_dtype, &in) || !type_of(cfg, names.out_dtype, &out) ||
+      !row_type(in) || !row_type(out) ||
       E > MAX_EXPERTS || K > MAX_TOPK || E % W != 0)
     REFUSE;
   Tensor x[MAX_RANKS], ids[MAX_RANKS], weights[MAX_RANKS];

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from amd_distributed_2025_amd import HIPAllToAll, LocalWorld, MoEConfig, RankTestData, custom_kernel, custom_kernel_job, gemm_rs, set_peer_inputs
-from amd_distributed_2025_amd import _binding, all2all
+from amd_distributed_2025_amd import _binding, _lib, all2all
 from amd_distributed_2025_amd._lib import MoeA2AError
 
 pytestmark = pytest.mark.gpu
@@ -243,6 +243,39 @@ def test_layout_and_binding_set_later():
         own.calls.clear()
         assert same(outcome(lambda: one_rank(pair[0], d)), got[0][-6:])
         assert own.calls == ["local_dispatch", "expert_scale", "local_combine"]
+
+
+def test_config_and_bounds_set_later():
+    """Both are read at every call: the types that the config names, another config, the rows that the buffers have room for."""
+    d, pair = data(seed=9), [rank("padded", native) for native in (True, False)]
+    bf16, f16 = torch.bfloat16, torch.float16
+
+    def everything(a):
+        x, ys = d.x.to(a.cfg.in_dtype), [torch.zeros(T, H, dtype=a.cfg.out_dtype, device=DEV) for _ in range(2)]
+        sent = a.dispatch_send(x, d.indices)
+        num, ex, em = a.dispatch_recv(*[t.clone() for t in sent])
+        ey = a.expert_scale(ex, num)
+        back = a.combine_send(em, ey, num)
+        a.combine_recv(ys[0], d.weights, *[t.clone() for t in back])
+        num, ex, em = a.dispatch(x, d.indices)
+        a.combine(ys[1], d.weights, em, a.expert_scale(ex, num), num)
+        assert torch.equal(*ys)
+        return [*sent, *back, num, ex, em, ey, *ys]
+
+    for types in ((bf16, bf16), (bf16, f16), (f16, bf16), (bf16, bf16)):
+        for a in pair:
+            a.cfg.in_dtype, a.cfg.out_dtype = types
+        for _ in range(2):
+            assert same(*[outcome(lambda a=a: everything(a)) for a in pair]), types
+    for change in (dict(cfg=config(f16)), dict(max_rows_in=T * K + 8, max_rows_out=T * K + 1), dict(shape=_lib.Shape(1, 0, E, K, H, T))):
+        for a in pair:
+            for name, value in change.items():
+                setattr(a, name, value)
+        pair[1]._calls = all2all._PythonOnly()
+        for _ in range(2):
+            got = [outcome(lambda a=a: everything(a)) for a in pair]
+            assert same(*got), change
+    assert got[0][4].shape == (T * K + 8, H) and got[0][4].dtype == f16
 
 
 def test_copies_share_a_workspace():

@@ -5,7 +5,7 @@ import copy
 import pytest
 import torch
 
-from amd_distributed_2025_amd import _binding, all2all
+from amd_distributed_2025_amd import MoEConfig, _binding, _lib, all2all
 
 ROWS, INTS = torch.zeros(4, 16, dtype=torch.bfloat16), torch.zeros(4, 2, dtype=torch.int32)
 ODD = [ROWS, INTS, None, 3, -1, 2 ** 70, "x", (1, 2), torch.zeros(0), torch.zeros(4, 16, device="meta"), torch.zeros(2, 2).to_sparse()]
@@ -79,3 +79,18 @@ def test_a_copied_object_and_its_copy_use_no_learned_buffers():
     assert type(a._calls) is type(b._calls) is all2all._PythonOnly and b._ws is a._ws and a.layout == "padded"
     b.binding = object()
     assert type(b._calls) is all2all._PythonOnly
+
+
+def test_a_config_or_shape_of_other_sizes_gets_no_native_calls():
+    """(The Python code checks by the one and launches by the other.)"""
+    made = [MoEConfig(8, 2, 16, 4, torch.bfloat16, torch.bfloat16), _lib.Shape(1, 0, 8, 2, 16, 4)]
+    binding = object.__new__(_binding.CtypesBinding)
+    native, device = _binding.host_calls()["RankCalls"], torch.device("cuda", 0)
+    assert type(all2all._rank_calls(made[1], made[0], device, binding)) is native
+    assert type(all2all._rank_calls(_lib.Shape(1, 0, 8, 2, 32, 4), made[0], device, binding)) is all2all._PythonOnly
+    a = object.__new__(all2all.HIPAllToAll)
+    a.__dict__.update(_learned={"recv"}, _copied=False, _calls=None, _binding=binding, _cfg=made[0], _shape=made[1], device=device)
+    a.cfg = MoEConfig(8, 2, 32, 4, torch.bfloat16, torch.bfloat16)
+    assert type(a._calls) is all2all._PythonOnly and not a._learned
+    a.shape = _lib.Shape(1, 0, 8, 2, 32, 4)
+    assert type(a._calls) is native and a.cfg.hidden_dim == a.shape.hidden_dim == 32
