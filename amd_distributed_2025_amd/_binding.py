@@ -7,7 +7,8 @@ offer the same methods with the same arguments — tensors, sizes and the stream
 handle — and both end in the same kernels, so results are identical. Calls in plain
 forms do not get here: `host_calls()` has them done in native code, whichever
 binding was asked for. Neither binding has
-a fallback: a missing library or a nonzero status raises.
+a fallback: a missing library, a nonzero status or a tensor that holds less than the call
+addresses raises.
 
 Capacities (`capacity_rows` of the C ABI) are taken from the tensors: the rows a
 row buffer and its meta buffer were allocated with.
@@ -32,6 +33,21 @@ def _ptr(t: Optional[torch.Tensor]):
 
 def _pointers(tensors):
     return (C.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
+def _holds(what: str, t: torch.Tensor, elements: int) -> None:
+    """The kernels address a tensor by the shape of the call: one that holds less must not get there."""
+    if t.numel() < elements:
+        raise ValueError(f"{what}: holds {t.numel()} elements, the call needs {elements}")
+
+
+def _padded(shape) -> int:
+    """Rows of a rank's padded expert buffers."""
+    return shape.num_experts // shape.world_size * shape.max_num_tokens * shape.world_size
+
+
+def _holds_counts(shape, expert_num_tokens) -> None:
+    _holds("expert_num_tokens", expert_num_tokens, shape.num_experts // shape.world_size)
 
 
 def _rows(buf: torch.Tensor, meta: torch.Tensor, hidden_dim: int) -> int:
@@ -67,6 +83,7 @@ class CtypesBinding:
 
     def dispatch_recv(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens, expert_x,
                       expert_meta, send_back_plan, stream, row_position=None):
+        _holds("recv_counts", recv_counts, shape.world_size)
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
         args = (shape, _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
                 min(rows_hint, capacity), capacity, _ptr(expert_num_tokens), _ptr(expert_x), _ptr(expert_meta),
@@ -80,6 +97,9 @@ class CtypesBinding:
 
     def combine_send(self, shape, expert_y, expert_meta, expert_num_tokens, rows_hint, send_buf, send_meta,
                      send_counts, send_back_plan, stream):
+        _holds("expert_y", expert_y, _padded(shape) * shape.hidden_dim)
+        _holds("expert_meta", expert_meta, _padded(shape) * META_DIM)
+        _holds_counts(shape, expert_num_tokens)
         capacity = _rows(send_buf, send_meta, shape.hidden_dim)
         self._call("moe_a2a_combine_send", shape, _ptr(expert_y), _ptr(expert_meta),
                   _ptr(expert_num_tokens), min(rows_hint, capacity), capacity, _ptr(send_buf), _ptr(send_meta),
@@ -87,6 +107,9 @@ class CtypesBinding:
 
     def combine_recv(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, weights, num_tokens, out_tokens,
                      accumulate, stream, entry_row=None):
+        _holds("recv_counts", recv_counts, shape.world_size)
+        _holds("weights", weights, num_tokens * shape.experts_per_token)
+        _holds("out_tokens", out_tokens, num_tokens * shape.hidden_dim)
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
         args = (shape, _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts),
                 min(rows_hint, capacity), capacity, _ptr(weights), num_tokens, _ptr(out_tokens),
@@ -99,10 +122,16 @@ class CtypesBinding:
             self._call("moe_a2a_combine_recv_long", *args, _ptr(entry_row), stream)
 
     def expert_scale(self, shape, expert_x, expert_num_tokens, rows_hint, expert_y, stream):
+        _holds("expert_x", expert_x, _padded(shape) * shape.hidden_dim)
+        _holds("expert_y", expert_y, _padded(shape) * shape.hidden_dim)
+        _holds_counts(shape, expert_num_tokens)
         self._call("moe_a2a_expert_scale", shape, _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
                   _DT[expert_x.dtype], _DT[expert_y.dtype], _ptr(expert_y), stream)
 
     def expert_gemm(self, shape, expert_x, expert_num_tokens, rows_hint, weights, bias, expert_y, stream):
+        _holds("expert_x", expert_x, _padded(shape) * weights.shape[2])
+        _holds("expert_y", expert_y, _padded(shape) * weights.shape[1])
+        _holds_counts(shape, expert_num_tokens)
         self._call("moe_a2a_expert_gemm", shape, _ptr(expert_x), _ptr(expert_num_tokens), rows_hint,
                   _ptr(weights), _ptr(bias), weights.shape[2], weights.shape[1], _DT[expert_x.dtype],
                   _ptr(expert_y), stream)
@@ -123,6 +152,7 @@ class CtypesBinding:
 
     def dispatch_recv_compact(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens,
                               expert_offsets, expert_x, expert_meta, send_back_plan, stream):
+        _holds("recv_counts", recv_counts, shape.world_size)
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
         self._call("moe_a2a_dispatch_recv_compact", shape, _ptr(recv_buf), _ptr(recv_meta),
                   _ptr(recv_counts), min(rows_hint, capacity), capacity, _ptr(expert_num_tokens),
@@ -130,17 +160,23 @@ class CtypesBinding:
                   _rows(expert_x, expert_meta, shape.hidden_dim), _ptr(send_back_plan), stream)
 
     def expert_scale_compact(self, shape, expert_x, expert_num_tokens, rows_hint, expert_y, stream):
+        capacity = min(expert_x.shape[0], expert_y.shape[0])
+        _holds("expert_x", expert_x, capacity * shape.hidden_dim)
+        _holds("expert_y", expert_y, capacity * shape.hidden_dim)
+        _holds_counts(shape, expert_num_tokens)
         self._call("moe_a2a_expert_scale_compact", shape, _ptr(expert_x), _ptr(expert_num_tokens),
-                  rows_hint, min(expert_x.shape[0], expert_y.shape[0]), _DT[expert_x.dtype], _DT[expert_y.dtype],
+                  rows_hint, capacity, _DT[expert_x.dtype], _DT[expert_y.dtype],
                   _ptr(expert_y), stream)
 
     def expert_gemm_compact(self, shape, expert_x, expert_num_tokens, rows_hint, weights, bias, expert_y, stream):
+        _holds_counts(shape, expert_num_tokens)
         self._call("moe_a2a_expert_gemm_compact", shape, _ptr(expert_x), _ptr(expert_num_tokens),
                   rows_hint, min(expert_x.shape[0], expert_y.shape[0]), _ptr(weights), _ptr(bias),
                   weights.shape[2], weights.shape[1], _DT[expert_x.dtype], _ptr(expert_y), stream)
 
     def combine_send_compact(self, shape, expert_y, expert_meta, expert_num_tokens, rows_hint, send_buf,
                              send_meta, send_counts, send_back_plan, stream):
+        _holds_counts(shape, expert_num_tokens)
         capacity = _rows(send_buf, send_meta, shape.hidden_dim)
         self._call("moe_a2a_combine_send_compact", shape, _ptr(expert_y), _ptr(expert_meta),
                   _ptr(expert_num_tokens), min(rows_hint, capacity),

@@ -94,3 +94,68 @@ def test_a_config_or_shape_of_other_sizes_gets_no_native_calls():
     assert type(a._calls) is all2all._PythonOnly and not a._learned
     a.shape = _lib.Shape(1, 0, 8, 2, 32, 4)
     assert type(a._calls) is native and a.cfg.hidden_dim == a.shape.hidden_dim == 32
+
+
+class Recorded(_binding.CtypesBinding):
+    """The binding with nothing behind it: every call is noted."""
+
+    def __init__(self):
+        self.called = []
+
+    def _call(self, name, *args):
+        self.called.append(name)
+
+
+SHAPE = _lib.Shape(1, 0, 8, 2, 64, 12)  # (padded buffers of 96 rows, 24 in the compact layout)
+
+
+def _bf(*shape):
+    return torch.zeros(*shape, dtype=torch.bfloat16)
+
+
+def _int(*shape):
+    return torch.zeros(*shape, dtype=torch.int32)
+
+
+# method -> its arguments after the shape, and which of them may not be shorter (by place)
+SIZED = {
+    "dispatch_recv": ([_bf(24, 64), _int(24, 5), _int(1), 24, _int(8), _bf(8, 12, 64), _int(8, 12, 5), None, 0], [2]),
+    "dispatch_recv_compact": ([_bf(24, 64), _int(24, 5), _int(1), 24, _int(8), _int(9), _bf(24, 64), _int(24, 5), None, 0], [2]),
+    "expert_scale": ([_bf(8, 12, 64), _int(8), 24, _bf(8, 12, 64), 0], [0, 1, 3]),
+    "expert_scale_compact": ([_bf(24, 64), _int(8), 24, _bf(24, 64), 0], [1]),
+    "expert_gemm": ([_bf(8, 12, 64), _int(8), 24, _bf(8, 32, 64), None, _bf(8, 12, 32), 0], [0, 1, 5]),
+    "expert_gemm_compact": ([_bf(24, 64), _int(8), 24, _bf(8, 32, 64), None, _bf(24, 32), 0], [1]),
+    "combine_send": ([_bf(8, 12, 64), _int(8, 12, 5), _int(8), 24, _bf(24, 64), _int(24, 5), _int(1), None, 0], [0, 1, 2]),
+    "combine_send_compact": ([_bf(24, 64), _int(24, 5), _int(8), 24, _bf(24, 64), _int(24, 5), _int(1), None, 0], [2]),
+    "combine_recv": ([_bf(24, 64), _int(24, 5), _int(1), 24, torch.zeros(12, 2), 12, _bf(12, 64), True, 0], [2, 4, 6]),
+}
+
+
+@pytest.mark.parametrize("method", SIZED)
+def test_tensors_that_hold_less_than_a_call_addresses_are_refused(method):
+    args, sized = SIZED[method]
+    b = Recorded()
+    getattr(b, method)(SHAPE, *args)
+    assert len(b.called) == 1
+    for at in sized:
+        short = list(args)
+        short[at] = args[at][:-1]
+        with pytest.raises(ValueError, match="the call needs"):
+            getattr(b, method)(SHAPE, *short)
+    assert len(b.called) == 1
+
+
+@pytest.mark.parametrize("rows, taken", [(24, False), (96, True), (95, False)])
+def test_flat_expert_rows_are_held_to_the_padded_layout(rows, taken, monkeypatch):
+    """Rows without their dimensions go to the padded entry point, which addresses 96 of them: flat compact ones, 24,
+    had it write past the end of a buffer made for 24."""
+    monkeypatch.setattr(all2all, "_stream", lambda device: 0)
+    a, b = object.__new__(all2all.HIPAllToAll), Recorded()
+    a.__dict__.update(_calls=all2all._PythonOnly(), _learned=set(), _ws={}, _kept={}, _send_views={}, _binding=b, _shape=SHAPE,
+                      _cfg=MoEConfig(8, 2, 64, 12, torch.bfloat16, torch.bfloat16), _rows_in_hint=24, device=torch.device("cpu"))
+    if taken:
+        assert a.expert_scale(_bf(rows * 64), _int(8)).shape == (rows * 64,) and b.called == ["moe_a2a_expert_scale"]
+    else:
+        with pytest.raises(ValueError, match="the call needs"):
+            a.expert_scale(_bf(rows * 64), _int(8))
+        assert not b.called
