@@ -218,6 +218,21 @@ __device__ __forceinline__ int floormod(int e, int d, uint32_t magic) {
   return m < 0 ? m + d : m;
 }
 
+// key[u] = floormod(key[u], d, magic), with one branch for all of them.
+template <int U>
+__device__ __forceinline__ void floormod_each(int (&key)[U], int d, uint32_t magic) {
+  int all = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) all |= key[u];
+  if (__ballot((uint32_t)all >= 65536u) != 0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) key[u] = floormod(key[u], d, magic);
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) key[u] = d == 1 ? 0 : key[u] - (int)__umulhi((uint32_t)key[u], magic) * d;
+}
+
 // Inclusive [lo, hi] range of expert ids owned by the same destination as `e`.
 // Ids outside [0, E) name no destination: they form one class after all ranks
 // (compared as unsigned numbers, a negative id is just a large one), so the
@@ -290,8 +305,10 @@ __device__ __forceinline__ int count_keys(int n, const Keys& keys, Test test) {
     for (int u = 0; u < SCAN_UNROLL; ++u) idx[u] = min(i + u * BLK, n - 1);
     keys.fetch(idx, key);
 #pragma unroll
-    for (int u = 0; u < SCAN_UNROLL; ++u)
+    for (int u = 0; u < SCAN_UNROLL; ++u) {
+      if (b + u * BLK >= n) break;
       cnt += (i + u * BLK < n) ? (int)test(key[u], i + u * BLK) : 0;
+    }
   }
   return cnt;
 }
@@ -300,9 +317,10 @@ __device__ __forceinline__ int count_keys(int n, const Keys& keys, Test test) {
 struct StridedKeys {
   const int* __restrict__ base;
   int stride;
-  __device__ __forceinline__ void fetch(const int* idx, int* key) const {
+  template <int U>
+  __device__ __forceinline__ void fetch(const int (&idx)[U], int (&key)[U]) const {
 #pragma unroll
-    for (int u = 0; u < SCAN_UNROLL; ++u) key[u] = base[(size_t)idx[u] * stride];
+    for (int u = 0; u < U; ++u) key[u] = base[(size_t)idx[u] * stride];
   }
 };
 
@@ -333,11 +351,13 @@ struct WavePayload {
 // issue order, so the keys arrive first and the slot is ready while the payload
 // is still in flight):  RowsScan scan(n, keys);  ...issue payload...;
 // scan.finish(keys, test, cnt);
-template <typename Keys>
+// SHORT: scans that mostly end inside a batch leave it there (the branches cost 0.5 us where batches are full: 20.2 against
+// 19.2 for the 4800 rows of a skewed job in the compact layout).
+template <typename Keys, bool SHORT = false, int UNROLL = SCAN_UNROLL>
 struct RowsScan {
   static constexpr int STEP = 64 * ROWS;
   int n, b;  // keys that may be loaded; first key of the batch in flight (same for every lane)
-  int key[SCAN_UNROLL];
+  int key[UNROLL];
   // `n_load` keys are known to be readable; how many of them count is told to finish().
   __device__ __forceinline__ RowsScan(int n_load, const Keys& keys) : n(n_load), b(0) {
     if (n > 0) issue(keys);
@@ -346,16 +366,17 @@ struct RowsScan {
   // lanes whose keys fall past n load key n-1 and are masked in consume().
   __device__ __forceinline__ void issue(const Keys& keys) {
     const int i = b + threadIdx.x;
-    int idx[SCAN_UNROLL];
+    int idx[UNROLL];
 #pragma unroll
-    for (int u = 0; u < SCAN_UNROLL; ++u) idx[u] = min(i + u * STEP, n - 1);
+    for (int u = 0; u < UNROLL; ++u) idx[u] = min(i + u * STEP, n - 1);
     keys.fetch(idx, key);
   }
   template <typename Test>
   __device__ __forceinline__ void consume(Test test, int (&cnt)[ROWS]) const {
     const int i = b + threadIdx.x;
 #pragma unroll
-    for (int u = 0; u < SCAN_UNROLL; ++u) {
+    for (int u = 0; u < UNROLL; ++u) {
+      if (SHORT && b + u * STEP >= n) break;
       const int i2 = i + u * STEP;
       if (i2 < n) {
 #pragma unroll
@@ -374,7 +395,7 @@ struct RowsScan {
     const bool first = n > 0;
     n = min(n, n_valid);
     if (first) consume(test, cnt);
-    for (b += SCAN_UNROLL * STEP; b < n; b += SCAN_UNROLL * STEP) {
+    for (b += UNROLL * STEP; b < n; b += UNROLL * STEP) {
       issue(keys);
       consume(test, cnt);
     }
@@ -384,7 +405,7 @@ struct RowsScan {
   template <typename Test>
   __device__ __forceinline__ void extend(const Keys& keys, int from, int to, Test test, int (&cnt)[ROWS]) {
     n = to;
-    for (b = from; b < to; b += SCAN_UNROLL * STEP) {
+    for (b = from; b < to; b += UNROLL * STEP) {
       issue(keys);
       consume(test, cnt);
     }
@@ -420,8 +441,8 @@ __device__ __forceinline__ int rows_reduce(const int (&cnt)[ROWS], int* part, in
 
 template <typename V, int NVW>
 __global__ __launch_bounds__(64 * ROWS) void dispatch_send_kernel(
-    const V* __restrict__ x, const int* __restrict__ indices, int S, int K, int nle, int E, int W,
-    uint32_t magic, int rank, int row_vecs, int chunks, V* __restrict__ send_buf,
+    const V* __restrict__ x, const int* __restrict__ indices, int S, int K, int W, int movers, int chunks, int row_vecs,
+    int nle, int E, uint32_t magic, int rank, V* __restrict__ send_buf,
     int* __restrict__ send_meta, int* __restrict__ send_counts, int* __restrict__ send_slot) {
   __shared__ int part[2 * ROWS * ROWS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -436,7 +457,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_send_kernel(
   }
 
   const int groups = (S + ROWS - 1) / ROWS;
-  const int items = groups * chunks, movers = gridDim.x - W;
+  const int items = groups * chunks;
   int parity = 0;
   for (int q = xcd_contiguous(blockIdx.x - W, movers); q < items; q += movers, ++parity) {
     const int grp = chunks == 1 ? q : q / chunks, c = q - grp * chunks;
@@ -507,8 +528,8 @@ inline int fan_of(long long S) { return S <= MOE_A2A_FAN2_MAX_ENTRIES ? 2 : 8; }
 
 template <typename V, int NV, int FAN>
 __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
-    const V* __restrict__ x, const int* __restrict__ indices, int T, int K, int nle, int E, int W,
-    uint32_t magic, int rank, int row_vecs, int chunks, V* __restrict__ send_buf,
+    const V* __restrict__ x, const int* __restrict__ indices, int T, int K, int W, int chunks, int row_vecs, int nle,
+    int E, uint32_t magic, int rank, V* __restrict__ send_buf,
     int* __restrict__ send_meta, int* __restrict__ send_counts, int* __restrict__ send_slot) {
   __shared__ int part[2 * NWAVES * FAN];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -533,7 +554,9 @@ __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
     const int base = c * (BLOCK * NV);
     const int i0 = t * K;
 
-    // first batch of keys, then the row: the keys come back first
+    // the token's own expert ids (as in the kernel below), first batch of keys, then the row: the keys come back first
+    const bool all_own = K <= 64;
+    const int own0 = indices[i0 + min(all_own ? lane : lane & (FAN - 1), K - 1)];
     int key[SCAN_UNROLL];
 #pragma unroll
     for (int u = 0; u < SCAN_UNROLL; ++u) key[u] = indices[min(tid + u * BLOCK, S - 1)];
@@ -541,11 +564,13 @@ __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
     p.load(x + (size_t)t * row_vecs, base, row_vecs);
 
     for (int g0 = 0; g0 < K; g0 += FAN) {
+      int own = own0;
+      if (!all_own && g0 > 0) own = first_use(indices[i0 + min(g0 + (lane & (FAN - 1)), K - 1)]);
       int mine[FAN];
 #pragma unroll
       for (int g = 0; g < FAN; ++g) {
-        const int i = i0 + min(g0 + g, K - 1);
-        mine[g] = klass(indices[i]) * S + i;
+        const int k = min(g0 + g, K - 1);
+        mine[g] = klass(__builtin_amdgcn_readlane(own, all_own ? k : g)) * S + i0 + k;
       }
       int cnt[FAN];
 #pragma unroll
@@ -586,11 +611,13 @@ __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
       }
       if (c == 0 && tid < live * META) {
         const int g = tid / META, f = tid - g * META;
-        int slot = 0;
+        int slot = 0, e = 0;
 #pragma unroll
         for (int w = 0; w < NWAVES; ++w) slot += half[w * FAN + g];
+#pragma unroll
+        for (int gg = 0; gg < FAN; ++gg) e = gg == g ? __builtin_amdgcn_readlane(own, all_own ? min(g0 + gg, K - 1) : gg) : e;
         const int i = i0 + g0 + g;
-        const int m = f == 0 ? indices[i] : f == 1 ? rank : f == 2 ? t : f == 3 ? g0 + g : 0;
+        const int m = f == 0 ? e : f == 1 ? rank : f == 2 ? t : f == 3 ? g0 + g : 0;
         send_meta[(size_t)slot * META + f] = m;
         if (f == 0 && send_slot) send_slot[i] = slot;
       }
@@ -611,8 +638,8 @@ __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
 
 template <typename V, int BLK, int NV, bool POW2, int FAN>
 __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
-    const V* __restrict__ x, const int* __restrict__ indices, int T, int K, int nle, int E, int W,
-    uint32_t magic, int nle_shift, int order_bits, int rank, int row_vecs, int chunks,
+    const V* __restrict__ x, const int* __restrict__ indices, int T, int K, int W, int chunks, int row_vecs, int E,
+    uint32_t magic, int nle_shift, int order_bits, int rank,
     V* __restrict__ send_buf, int* __restrict__ send_meta, int* __restrict__ send_counts,
     int* __restrict__ send_slot) {
   constexpr int NW = BLK / 64;
@@ -647,10 +674,11 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
     const int col = c * (BLK * NV) + tid;  // this lane's first vector; the others BLK apart
     const int i0 = t * K;
 
-    // the token's own expert ids, FAN at a time: lane l of every wave holds entry g0 + l % FAN. One
-    // vector load issued ahead of the keys (as uniform loads they become scalar loads that are
+    // the token's own expert ids: lane l of every wave holds entry l, or entry g0 + l % FAN of a token with more than
+    // 64. One vector load issued ahead of the keys (as uniform loads they become scalar loads that are
     // waited for one by one in the middle of the ranking)
-    const int own0 = indices[i0 + min(lane & (FAN - 1), K - 1)];
+    const bool all_own = K <= 64;
+    const int own0 = indices[i0 + min(all_own ? lane : lane & (FAN - 1), K - 1)];
     int key[KEYS];
 #pragma unroll
     for (int u = 0; u < KEYS; ++u) key[u] = indices[min(tid + u * BLK, S - 1)];
@@ -662,12 +690,12 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
       // (a later group waits for its ids inside the branch: a wait at the place where the two paths
       // meet would cover the first group's row as well, which is requested behind its ids)
       int own = own0;
-      if (g0 > 0) own = first_use(indices[i0 + min(g0 + (lane & (FAN - 1)), K - 1)]);
+      if (!all_own && g0 > 0) own = first_use(indices[i0 + min(g0 + (lane & (FAN - 1)), K - 1)]);
       int mine[FAN];
 #pragma unroll
       for (int g = 0; g < FAN; ++g) {
-        const int i = i0 + min(g0 + g, K - 1);
-        mine[g] = composite(__builtin_amdgcn_readlane(own, g), i);
+        const int k = min(g0 + g, K - 1);
+        mine[g] = composite(__builtin_amdgcn_readlane(own, all_own ? k : g), i0 + k);
       }
       int cnt[FAN];
 #pragma unroll
@@ -675,6 +703,7 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
       auto consume = [&](const int (&k)[KEYS], int b) {
 #pragma unroll
         for (int u = 0; u < KEYS; ++u) {
+          if (b + u * BLK >= S) break;  // (with few entries that is most of the batch)
           const int i2 = b + tid + u * BLK;
           const int ck = i2 < S ? composite(k[u], i2) : INT_MAX;
 #pragma unroll
@@ -724,15 +753,95 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
       }
       if (c == 0 && tid < live * META) {
         const int g = tid / META, f = tid - g * META;
-        int mine_slot = 0;
+        int mine_slot = 0, e = 0;
 #pragma unroll
-        for (int gg = 0; gg < FAN; ++gg) mine_slot = gg == g ? slot[gg] : mine_slot;
+        for (int gg = 0; gg < FAN; ++gg) {
+          mine_slot = gg == g ? slot[gg] : mine_slot;
+          e = gg == g ? __builtin_amdgcn_readlane(own, all_own ? min(g0 + gg, K - 1) : gg) : e;
+        }
         const int i = i0 + g0 + g;
-        const int e = __shfl(own, g, 64);  // (lanes 0 .. FAN-1 of wave 0 are among the active ones)
         const int m = f == 0 ? e : f == 1 ? rank : f == 2 ? t : f == 3 ? g0 + g : 0;
         send_meta[(size_t)mine_slot * META + f] = m;
         if (f == 0 && send_slot) send_slot[i] = mine_slot;
       }
+    }
+  }
+}
+
+// The fan-out of a job with few entries: every wave holds all their keys (KEYS per lane) and ranks entries of its own
+// (wave, wave + 4, ...), so that one barrier makes the slots known, where the kernels above add partial counts over the
+// waves, for two entries at a time. Such a job is bound by the chain of steps from the launch to the last store, and what
+// counts in it is the code that a wave runs through: KEYS is the smallest of 2, 4, 8, 12 and 16 that holds the entries, and
+// nothing in the scan is skipped by a branch (with up to 16 keys per lane skipped in this way 3.23 us instead of 2.57 for
+// the 32 entries of 12 KB below, 2.83 with up to 8). us, one launch after another in a graph, before / here: 72 entries
+// of 1 KB, 6 per token 4.38 / 2.77, 32 of 12 KB, 2 per token 3.92 / 2.57, 500 of 5.8 KB, 4 per token 3.85 / 3.30, 720 of
+// 2 KB, 8 per token 5.27 / 3.61, 800 of 14 KB, 8 per token 6.17 / 4.66. Beyond 1024 entries the keys of all waves go through
+// the unit's one path to L1 too often; and tokens with fewer than four entries and much to move are better off with a wave
+// per entry (900 of 14 KB, 2 per token 5.26 / 5.70).
+constexpr int FEW_ENTRIES = 64 * 16;
+constexpr int FEW_MAX_K = 64;            // a lane of the wave for each
+constexpr long long FEW_BYTES = 8 << 20; // (of tokens with fewer than MOE_A2A_FANOUT_MIN_K entries)
+
+template <typename V, int KEYS, bool POW2>
+__global__ __launch_bounds__(BLOCK) void dispatch_few_kernel(
+    const V* __restrict__ x, const int* __restrict__ indices, int T, int K, int W, int chunks, int row_vecs, int E,
+    uint32_t magic, int nle_shift, int order_bits, int rank,
+    V* __restrict__ send_buf, int* __restrict__ send_meta, int* __restrict__ send_counts,
+    int* __restrict__ send_slot) {
+  __shared__ int slots[FEW_MAX_K], ids[FEW_MAX_K];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int S = T * K;
+  auto klass = [&](int e) {
+    const int d = POW2 ? e >> nle_shift : (int)__umulhi((uint32_t)e, magic);
+    return (uint32_t)e >= (uint32_t)E ? W : d;
+  };
+  // (as above)
+  auto composite = [&](int e, int i) { return (klass(e) << order_bits) | i; };
+  int key[KEYS];
+  auto fetch = [&] {
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) key[u] = indices[min(lane + u * 64, S - 1)];
+  };
+
+  if ((int)blockIdx.x < W) {
+    if (wave > 0) return;
+    fetch();
+    int n = 0;
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) n += __popcll(__ballot(lane + u * 64 < S && klass(key[u]) == (int)blockIdx.x));
+    if (lane == 0) send_counts[blockIdx.x] = n;
+    return;
+  }
+
+  const int q = blockIdx.x - W;
+  const int t = chunks == 1 ? q : q / chunks, c = q - t * chunks;
+  const int i0 = t * K, col = c * BLOCK + tid;
+  const int own = indices[i0 + min(lane, K - 1)];
+  fetch();
+  const V v = stream_load(x + (size_t)t * row_vecs + min(col, row_vecs - 1));
+#pragma unroll
+  for (int u = 0; u < KEYS; ++u)
+    key[u] = lane + u * 64 < S ? composite(key[u], lane + u * 64) : INT_MAX;
+  for (int k = wave; k < K; k += NWAVES) {
+    const int mine = composite(__builtin_amdgcn_readlane(own, k), i0 + k);
+    int slot = 0;
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) slot += __popcll(__ballot(key[u] < mine));
+    if (lane == 0) slots[k] = slot;
+  }
+  if (wave == 0 && lane < K) ids[lane] = own;
+  lds_barrier();
+  const int slot_of = slots[min(lane, K - 1)];
+  for (int k = 0; k < K; ++k) {
+    const int slot = __builtin_amdgcn_readlane(slot_of, k);
+    if (col < row_vecs) row_store<MOE_A2A_STORE_SEND>(send_buf + (size_t)slot * row_vecs + col, v);
+  }
+  if (c == 0) {
+    for (int m = tid; m < K * META; m += BLOCK) {
+      const int k = m / META, f = m - k * META;
+      const int slot = slots[k];
+      send_meta[(size_t)slot * META + f] = f == 0 ? ids[k] : f == 1 ? rank : f == 2 ? t : f == 3 ? k : 0;
+      if (f == 0 && send_slot) send_slot[i0 + k] = slot;
     }
   }
 }
@@ -964,68 +1073,94 @@ __global__ __launch_bounds__(RPLAN_BLOCK) void plan_recv_kernel(
 //                 the offsets.
 enum { RECV_SCAN = 0, RECV_POS = 1, RECV_COMPACT = 2 };
 
+// A workgroup that plans expert blockIdx.x: its rows, where every source's run of them starts inside the expert and in the
+// send-back stream, and in the compact layout where the expert starts.
+template <bool COMPACT, int UNROLL>
+__device__ __forceinline__ void plan_expert(
+    const int* __restrict__ recv_meta, const int* __restrict__ recv_counts, int W, int hint_rows, int nle, int capacity_rows,
+    uint32_t magic, int* __restrict__ expert_num_tokens, int* __restrict__ plan, int* __restrict__ expert_offsets) {
+  // Its keys go out with the counts, as far as the hint says that they can be read. A lane per source counts by the
+  // ballots of 64 rows, cut to the rows of its source.
+  __shared__ int sums[ROWS][2][64];  // per wave and source: rows of this expert, rows of lower experts
+  constexpr int BLK = 64 * ROWS;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int me = blockIdx.x, first_of_wave = __builtin_amdgcn_readfirstlane(wave) * 64;
+  const int raw_count = recv_counts[min(lane, W - 1)];
+  int e2[UNROLL];
+  auto fetch = [&](int b, int end) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) e2[u] = recv_meta[(size_t)min(b + tid + u * BLK, end - 1) * META];
+  };
+  const int early = min(hint_rows, UNROLL * BLK);
+  if (early > 0) fetch(0, early);
+  const int mine = lane < W ? min(max(first_use(raw_count), 0), capacity_rows) : 0;
+  const int incl = wave_inclusive_scan(mine);
+  const int R = min(__builtin_amdgcn_readlane(incl, 63), capacity_rows);
+  int here = 0, below = 0;
+  auto count = [&](int b, int end) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int row0 = b + u * BLK + first_of_wave;
+      if (row0 >= end) break;
+      const int le2 = floormod(e2[u], nle, magic);
+      const bool there = row0 + lane < end;
+      auto lanes_from = [&](int row) {
+        const int n = row - row0;
+        return n <= 0 ? ~0ull : n >= 64 ? 0ull : ~0ull << n;
+      };
+      const unsigned long long own = lanes_from(incl - mine) & ~lanes_from(incl);
+      here += __popcll(__ballot(there && le2 == me) & own);
+      below += __popcll(__ballot(there && le2 < me) & own);
+    }
+  };
+  count(0, min(early, R));
+  for (int b = early; b < R; b += UNROLL * BLK) {
+    fetch(b, R);
+    count(b, R);
+  }
+  sums[wave][0][lane] = here;
+  sums[wave][1][lane] = below;
+  lds_barrier();
+  if (wave == 0) {
+#pragma unroll
+    for (int w = 1; w < ROWS; ++w) {
+      here += sums[w][0][lane];
+      below += sums[w][1][lane];
+    }
+    const int upto = wave_inclusive_scan(here);
+    if (lane < W) {
+      int* out = plan + ((size_t)me * W + lane) * PLAN_INTS;
+      out[0] = upto - here;
+      out[1] = (incl - mine) + below;
+    }
+    if (lane == 63) expert_num_tokens[me] = upto;
+    if constexpr (COMPACT) {  // rows of lower experts, from every source: where this expert's rows start
+      const int lower = wave_sum(below), mine_all = __builtin_amdgcn_readlane(upto, 63);
+      if (lane == 0) {
+        expert_offsets[me] = lower;
+        if (me == nle - 1) expert_offsets[nle] = lower + mine_all;
+      }
+    }
+  }
+}
+
 template <typename V, int NVW, bool PLAN, int MODE, Store HOW>
 __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
     const V* __restrict__ recv_buf, const int* __restrict__ recv_meta,
-    const int* __restrict__ recv_counts, int W, int hint_rows, int capacity_rows, int nle,
-    uint32_t magic, int max_recv, int row_vecs, int chunks, int* __restrict__ expert_num_tokens,
+    const int* __restrict__ recv_counts, int W, int hint_rows, int movers, int chunks, int row_vecs, int nle,
+    int capacity_rows, uint32_t magic, int max_recv, int* __restrict__ expert_num_tokens,
     V* __restrict__ expert_x, int* __restrict__ expert_meta, int* __restrict__ plan,
     const int* __restrict__ row_pos, int* __restrict__ expert_offsets) {
   constexpr bool POS = MODE == RECV_POS, COMPACT = MODE == RECV_COMPACT;
+  constexpr int UNROLL = HOW == PLAIN ? 4 : SCAN_UNROLL;  // (PLAIN: at most 1024 rows, mostly)
   __shared__ int part[2 * ROWS * ROWS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const StridedKeys key{recv_meta, META};
 
   if constexpr (PLAN) {
     if ((int)blockIdx.x < nle) {
-      __shared__ int seg_end[64];  // rows received from sources 0..s
-      __shared__ int hist[64][2];  // per source: rows of this expert, rows of lower experts
-      const int me = blockIdx.x;
-      const int mine = lane < W ? min(max(recv_counts[lane], 0), capacity_rows) : 0;
-      const int incl = wave_inclusive_scan(mine);
-      const int R = min(__builtin_amdgcn_readlane(incl, 63), capacity_rows);
-      if (wave == 0 && lane < W) {
-        seg_end[lane] = incl;
-        hist[lane][0] = 0;
-        hist[lane][1] = 0;
-      }
-      lds_barrier();
-      constexpr int BLK = 64 * ROWS;
-      for (int b = 0; b < R; b += SCAN_UNROLL * BLK) {
-        int e2[SCAN_UNROLL];
-#pragma unroll
-        for (int u = 0; u < SCAN_UNROLL; ++u)
-          e2[u] = recv_meta[(size_t)min(b + tid + u * BLK, R - 1) * META];
-#pragma unroll
-        for (int u = 0; u < SCAN_UNROLL; ++u) {
-          const int i2 = b + tid + u * BLK;
-          const int le2 = floormod(e2[u], nle, magic);
-          if (i2 < R && le2 <= me) {
-            int src = 0;
-            for (int s = 0; s + 1 < W; ++s) src += (int)(seg_end[s] <= i2);
-            atomicAdd(&hist[src][le2 < me ? 1 : 0], 1);
-          }
-        }
-      }
-      lds_barrier();
-      if (wave == 0) {
-        const int here = lane < W ? hist[lane][0] : 0;
-        const int below = lane < W ? hist[lane][1] : 0;
-        const int upto = wave_inclusive_scan(here);
-        if (lane < W) {
-          int* out = plan + ((size_t)me * W + lane) * PLAN_INTS;
-          out[0] = upto - here;
-          out[1] = (incl - mine) + below;
-        }
-        if (lane == 63) expert_num_tokens[me] = upto;
-        if constexpr (COMPACT) {  // rows of lower experts, from every source: where this expert's rows start
-          const int lower = wave_sum(below), mine_all = __builtin_amdgcn_readlane(upto, 63);
-          if (lane == 0) {
-            expert_offsets[me] = lower;
-            if (me == nle - 1) expert_offsets[nle] = lower + mine_all;
-          }
-        }
-      }
+      plan_expert<COMPACT, UNROLL>(recv_meta, recv_counts, W, hint_rows, nle, capacity_rows, magic, expert_num_tokens, plan,
+                                   expert_offsets);
       return;
     }
   }
@@ -1047,7 +1182,6 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
     return;
   }
 
-  const int movers = gridDim.x - nle;
   int parity = 0;
   // One (group, chunk) item. `limit` rows may be read; R is evaluated after the
   // loads are issued (it is already known on every pass but the first).
@@ -1080,7 +1214,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
     if (c == 0 && lane < META) m = recv_meta[(size_t)ic * META + lane];
     // only rows before the group's last row can precede any of its rows in its expert; the rows of
     // lower experts, which the compact layout puts ahead of it, lie anywhere in the stream
-    RowsScan<StridedKeys> scan(COMPACT ? limit : min(i0 + ROWS - 1, limit), key);
+    RowsScan<StridedKeys, !COMPACT, UNROLL> scan(COMPACT ? limit : min(i0 + ROWS - 1, limit), key);
     WavePayload<V, NVW> p;
     p.load(recv_buf + (size_t)ic * row_vecs, base, row_vecs, lane);
 
@@ -1136,6 +1270,74 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
   }
   const int items = (R + ROWS - 1) / ROWS * chunks;
   for (; q < items; q += movers) move(q, R, [&] { return R; });
+}
+
+// The same for a short stream: every wave ranks a row of its own against all keys it needs (KEYS per lane, the fewest that
+// hold hint_rows), with nothing to wait for but its own loads. As in dispatch_few_kernel the code that a wave runs through is
+// what counts. us, one launch after another in a graph, before / here: 72 rows of 1 KB 3.33 / 2.54, 32 of 12 KB 3.87 / 3.09,
+// 500 of 5.8 KB 4.11 / 3.44, 600 of 8 KB 4.45 / 4.11, 800 of 14 KB 6.17 / 5.75.
+template <typename V, int NVW, int KEYS, bool COMPACT>
+__global__ __launch_bounds__(64 * ROWS) void dispatch_recv_few_kernel(
+    const V* __restrict__ recv_buf, const int* __restrict__ recv_meta,
+    const int* __restrict__ recv_counts, int W, int hint_rows, int movers, int chunks, int row_vecs, int nle,
+    int capacity_rows, uint32_t magic, int max_recv, int* __restrict__ expert_num_tokens,
+    V* __restrict__ expert_x, int* __restrict__ expert_meta, int* __restrict__ plan, int* __restrict__ expert_offsets) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if ((int)blockIdx.x < nle) {
+    plan_expert<COMPACT, KEYS / ROWS>(recv_meta, recv_counts, W, hint_rows, nle, capacity_rows, magic, expert_num_tokens, plan,
+                            expert_offsets);
+    return;
+  }
+  int R = -1;  // not known yet
+  const int raw_count = recv_counts[min(lane, W - 1)];
+  auto rows_arrived = [&] {
+    const int my_count = lane < W ? min(max(first_use(raw_count), 0), capacity_rows) : 0;
+    return min(wave_sum(my_count), capacity_rows);
+  };
+  for (int q = ((int)blockIdx.x - nle) * ROWS + wave;; q += movers * ROWS) {
+    const int i = chunks == 1 ? q : q / chunks, c = q - i * chunks;
+    if (R < 0 && i >= hint_rows) R = rows_arrived();
+    if (R >= 0 && i >= R) return;
+    const int base = c * (64 * NVW);
+    const int e = recv_meta[(size_t)i * META];
+    // keys that may be read, and of them the ones that can precede the row
+    const int limit = R < 0 ? hint_rows : R;
+    int n = COMPACT ? limit : min(i + 1, limit);
+    int key[KEYS];
+    auto fetch = [&](int b) {
+#pragma unroll
+      for (int u = 0; u < KEYS; ++u) key[u] = recv_meta[(size_t)min(b + u * 64 + lane, n - 1) * META];
+    };
+    fetch(0);
+    int m = 0;
+    if (c == 0 && lane < META) m = recv_meta[(size_t)i * META + lane];
+    WavePayload<V, NVW> p;
+    p.load(recv_buf + (size_t)i * row_vecs, base, row_vecs, lane);
+    if (R < 0) R = rows_arrived();
+    if (i >= R) return;
+    const int le = floormod(e, nle, magic);
+    int pos = 0;
+    auto count = [&](int b, int end) {
+      floormod_each(key, nle, magic);
+#pragma unroll
+      for (int u = 0; u < KEYS; ++u) {
+        const int j = b + u * 64 + lane, le2 = key[u];
+        pos += __popcll(__ballot(((le2 == le) & (j < i)) | (COMPACT && (le2 < le) & (j < end))));
+      }
+    };
+    count(0, min(n, R));
+    int b = min(n, 64 * KEYS);
+    if constexpr (COMPACT) n = R;
+    for (; b < n; b += 64 * KEYS) {
+      fetch(b);
+      count(b, n);
+    }
+    if (pos < max_recv) {
+      const size_t row = COMPACT ? (size_t)pos : (size_t)le * max_recv + pos;
+      p.template store<PLAIN>(expert_x + row * row_vecs, base, row_vecs, lane);
+      if (c == 0 && lane < META) expert_meta[row * META + lane] = m;
+    }
+  }
 }
 
 // ---------------------------------------------------------------- expert-major stream helpers
@@ -1307,10 +1509,10 @@ struct WaveStreamKeys {
 
 template <typename V, int NVW, bool SMALL, bool PLAN>
 __global__ __launch_bounds__(64 * ROWS) void combine_send_kernel(
-    const V* __restrict__ expert_y, const int* __restrict__ expert_meta,
-    const int* __restrict__ expert_num_tokens, int nle, int max_recv, int W, int row_vecs,
-    int chunks, int capacity_rows, V* __restrict__ send_buf, int* __restrict__ send_meta,
-    int* __restrict__ send_counts, const int* __restrict__ plan, int compact_rows) {
+    const int* __restrict__ expert_num_tokens, const int* __restrict__ plan,
+    const int* __restrict__ expert_meta, const V* __restrict__ expert_y, int nle, int W, int chunks, int max_recv,
+    int compact_rows, int row_vecs, int capacity_rows, V* __restrict__ send_buf, int* __restrict__ send_meta,
+    int* __restrict__ send_counts) {
   static_assert(!PLAN || SMALL, "the planned path keeps the expert prefix in registers");
   __shared__ int part[2 * ROWS * ROWS];
   __shared__ int pre[SMALL ? 1 : MAX_LOCAL_EXPERTS + 1];
@@ -1552,12 +1754,11 @@ __global__ __launch_bounds__(BLOCK) void return_map_kernel(
   }
 }
 
-template <typename V, int DT, int BLK, int NV, bool MAPPED>
+template <typename V, int DT, int BLK, int NV, bool MAPPED, int UNROLL>
 __global__ __launch_bounds__(BLK) void combine_recv_kernel(
-    const V* __restrict__ recv_buf, const int* __restrict__ recv_meta,
-    const int* __restrict__ recv_counts, int W, int hint_rows, int capacity_rows,
-    const float* __restrict__ weights, int T, int K, int row_vecs, int chunks, V* __restrict__ out, int accumulate,
-    const int* __restrict__ entry_row) {
+    const int* __restrict__ recv_meta, const int* __restrict__ recv_counts, const float* __restrict__ weights, int W,
+    int hint_rows, int T, int K, int chunks, int capacity_rows, const V* __restrict__ recv_buf, int row_vecs,
+    int accumulate, V* __restrict__ out, const int* __restrict__ entry_row) {
   constexpr int N = Words<V>::N;
   constexpr int FAST = 8;  // addends ordered in registers
   __shared__ int hit_row[COMBINE_CAP], hit_k[COMBINE_CAP];
@@ -1578,10 +1779,10 @@ __global__ __launch_bounds__(BLK) void combine_recv_kernel(
 
   // rows [lo, hi) of the arriving stream: note the ones addressed to token t
   auto scan = [&](int t, int lo, int hi) {
-    for (int b = lo; b < hi; b += SCAN_UNROLL * BLK) {
-      int key[SCAN_UNROLL], kk[SCAN_UNROLL];
+    for (int b = lo; b < hi; b += UNROLL * BLK) {
+      int key[UNROLL], kk[UNROLL];
 #pragma unroll
-      for (int u = 0; u < SCAN_UNROLL; ++u) {
+      for (int u = 0; u < UNROLL; ++u) {
         // src_token and src_k with one 8-byte load (4-byte aligned, which global loads accept);
         // fetching src_k for the hits alone with a dependent load costs more than it saves
         int tk[2];
@@ -1591,7 +1792,7 @@ __global__ __launch_bounds__(BLK) void combine_recv_kernel(
       }
       if (R < 0) R = rows_arrived();
 #pragma unroll
-      for (int u = 0; u < SCAN_UNROLL; ++u) {
+      for (int u = 0; u < UNROLL; ++u) {
         const int row = b + tid + u * BLK;
         // (an arriving row whose k names no weight of the token is not an addend)
         if (row < min(hi, R) && key[u] == t && (uint32_t)kk[u] < (uint32_t)K) {
@@ -1644,7 +1845,7 @@ __global__ __launch_bounds__(BLK) void combine_recv_kernel(
       }
     } else if (R < 0) {
       // first item: one batch below the readable bound goes out before R is known
-      const int spec = min(hint_rows, SCAN_UNROLL * BLK);
+      const int spec = min(hint_rows, UNROLL * BLK);
       scan(t, 0, spec);
       if (R < 0) R = rows_arrived();
       scan(t, spec, R);
@@ -1760,6 +1961,113 @@ __global__ __launch_bounds__(BLK) void combine_recv_kernel(
       }
     }
     lds_barrier();  // the LDS lists are reused by the next item
+  }
+}
+
+// The same for a short stream (hint_rows <= 64 * KEYS): every wave looks through all of it by itself. The rows of 64 keys
+// that are the token's come out of a ballot in arrival order, so there is nothing to sort and no other wave to wait for.
+// ADDENDS: rows under way at a time. us, one launch after another in a graph, before / here: 72 rows of 1 KB, 6 per token
+// 3.73 / 3.06, 32 of 12 KB 3.62 / 2.79, 240 of 2 KB 3.69 / 2.92, 500 of 5.8 KB 4.37 / 3.88.
+constexpr int COMBINE_FEW_ROWS = 64 * 8;
+template <int DT, int NV, int KEYS, int ADDENDS>
+__global__ __launch_bounds__(BLOCK) void combine_recv_few_kernel(
+    const int* __restrict__ recv_meta, const int* __restrict__ recv_counts, const float* __restrict__ weights, int W,
+    int hint_rows, int K, int chunks, int capacity_rows, const b128* __restrict__ recv_buf, int row_vecs,
+    int accumulate, b128* __restrict__ out) {
+  constexpr int N = Words<b128>::N, LIST = 64;
+  __shared__ int hits[NWAVES][LIST][2];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int t = chunks == 1 ? (int)blockIdx.x : (int)blockIdx.x / chunks, c = (int)blockIdx.x - t * chunks;
+  const int base = c * (BLOCK * NV);
+  const int raw_count = recv_counts[min(lane, W - 1)];
+  const float my_weight = weights[(size_t)t * K + min(lane, K - 1)];
+  int tk[KEYS][2];
+  auto fetch = [&](int b, int end) {
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) __builtin_memcpy(tk[u], recv_meta + (size_t)min(b + u * 64 + lane, end - 1) * META + 2, 8);
+  };
+  fetch(0, hint_rows);
+  b128* __restrict__ orow = out + (size_t)t * row_vecs;
+  PairAcc<DT> acc[NV][N];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    b128 o{};
+    if (accumulate) o = orow[min(base + j * BLOCK + tid, row_vecs - 1)];
+#pragma unroll
+    for (int e = 0; e < N; ++e) acc[j][e].set(o[e]);
+  }
+  const int my_count = lane < W ? min(max(first_use(raw_count), 0), capacity_rows) : 0;
+  const int R = min(wave_sum(my_count), capacity_rows);
+  int n = 0;
+  auto note = [&](int b, int end) {
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) {
+      const int row = b + u * 64 + lane;
+      // (an arriving row whose k names no weight of the token is not an addend)
+      const bool hit = row < end && tk[u][0] == t && (uint32_t)tk[u][1] < (uint32_t)K;
+      const unsigned long long all = __ballot(hit);
+      const int at = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(all >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)all, 0));
+      if (hit && at < LIST) {
+        hits[wave][at][0] = row;
+        hits[wave][at][1] = tk[u][1];
+      }
+      n += __popcll(all);
+    }
+  };
+  note(0, min(hint_rows, R));
+  for (int b = hint_rows; b < R; b += KEYS * 64) {
+    fetch(b, R);
+    note(b, R);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  if (n <= LIST) {
+    for (int a0 = 0; a0 < n; a0 += ADDENDS) {
+      const int p = min(a0 + (lane & (ADDENDS - 1)), n - 1);
+      const int hit_row = hits[wave][p][0];
+      const int hit_weight = __builtin_amdgcn_ds_bpermute(hits[wave][p][1] << 2, __float_as_int(my_weight));
+      b128 v[ADDENDS][NV];
+      float w[ADDENDS];
+#pragma unroll
+      for (int u = 0; u < ADDENDS; ++u) {
+        // (row 0 exists: loaded for the places past n and not used)
+        const int row = a0 + u < n ? __builtin_amdgcn_readlane(hit_row, u) : 0;
+        w[u] = __int_as_float(__builtin_amdgcn_readlane(hit_weight, u));
+#pragma unroll
+        for (int j = 0; j < NV; ++j) v[u][j] = recv_buf[(size_t)row * row_vecs + min(base + j * BLOCK + tid, row_vecs - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < ADDENDS; ++u) {
+        if (a0 + u < n) {
+#pragma unroll
+          for (int j = 0; j < NV; ++j)
+#pragma unroll
+            for (int e = 0; e < N; ++e) acc[j][e].step(v[u][j][e], w[u]);
+        }
+      }
+    }
+  } else {  // more addends than the list holds: walk the stream in order
+    for (int i = 0; i < R; ++i) {
+      if (recv_meta[(size_t)i * META + 2] != t) continue;
+      const int k = recv_meta[(size_t)i * META + 3];
+      if (k < 0 || k >= K) continue;
+      const float w = weights[(size_t)t * K + k];
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        const b128 v = recv_buf[(size_t)i * row_vecs + min(base + j * BLOCK + tid, row_vecs - 1)];
+#pragma unroll
+        for (int e = 0; e < N; ++e) acc[j][e].step(v[e], w);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    const int idx = base + j * BLOCK + tid;
+    if (idx < row_vecs) {
+      uint32_t h[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) h[e] = acc[j][e].word();
+      orow[idx] = from_words<b128>(h);
+    }
   }
 }
 
@@ -3890,6 +4198,32 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
   Geometry f = g;
   f.nv = 1;
   f.chunks = (f.row_vecs + BLOCK - 1) / BLOCK;
+  // (a job without tokens goes to the kernels below, which then read nothing)
+  if (S > 0 && S <= FEW_ENTRIES && s->experts_per_token <= FEW_MAX_K && (long long)num_tokens * f.chunks <= 1 << 20 &&
+      (s->experts_per_token >= MOE_A2A_FANOUT_MIN_K || S * s->hidden_dim * 2 <= FEW_BYTES)) {
+    int order_bits = 1, nle_shift = 0;
+    while ((1 << order_bits) < S) ++order_bits;
+    while ((1 << nle_shift) < g.nle) ++nle_shift;
+    const int few_grid = s->world_size + num_tokens * f.chunks;
+#define LAUNCH_K(V, KEYS, POW2)                                                                  \
+  dispatch_few_kernel<V, KEYS, POW2><<<few_grid, BLOCK, 0, st>>>(                                \
+      (const V*)x, indices, num_tokens, s->experts_per_token, s->world_size, f.chunks,           \
+      f.row_vecs, s->num_experts, g.magic, nle_shift, order_bits, s->rank,                       \
+      (V*)send_buf, send_meta, send_counts, send_slot)
+#define LAUNCH(V, POW2)                                  \
+  do {                                                   \
+    if (S <= 64 * 2) LAUNCH_K(V, 2, POW2);               \
+    else if (S <= 64 * 4) LAUNCH_K(V, 4, POW2);          \
+    else if (S <= 64 * 8) LAUNCH_K(V, 8, POW2);          \
+    else if (S <= 64 * 12) LAUNCH_K(V, 12, POW2);        \
+    else LAUNCH_K(V, 16, POW2);                          \
+  } while (0)
+    if ((g.nle & (g.nle - 1)) == 0) { if (f.vec16) LAUNCH(b128, true); else LAUNCH(uint16_t, true); }
+    else { if (f.vec16) LAUNCH(b128, false); else LAUNCH(uint16_t, false); }
+#undef LAUNCH
+#undef LAUNCH_K
+    return launch_status();
+  }
   if (s->experts_per_token >= MOE_A2A_FANOUT_MIN_K && (s->world_size + 2ll) * S <= INT_MAX &&
       items_fit(num_tokens, f.chunks)) {
     const int fan = fan_of(S);
@@ -3911,8 +4245,8 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
       while ((1 << nle_shift) < g.nle) ++nle_shift;
 #define LAUNCH_W(V, NV, POW2, FAN)                                                             \
   dispatch_fanout_wide_kernel<V, WIDE, NV, POW2, FAN><<<wgrid, WIDE, 0, st>>>(                 \
-      (const V*)x, indices, num_tokens, s->experts_per_token, g.nle, s->num_experts,           \
-      s->world_size, g.magic, nle_shift, order_bits, s->rank, f.row_vecs, wchunks,             \
+      (const V*)x, indices, num_tokens, s->experts_per_token, s->world_size, wchunks,          \
+      f.row_vecs, s->num_experts, g.magic, nle_shift, order_bits, s->rank,                     \
       (V*)send_buf, send_meta, send_counts, send_slot)
 #define LAUNCH_WF(V, NV, POW2)                       \
   do {                                               \
@@ -3934,8 +4268,8 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
     const int fgrid = s->world_size + mover_blocks((long long)num_tokens * f.chunks);
 #define LAUNCH_F(V, FAN)                                                                       \
   dispatch_fanout_kernel<V, 1, FAN><<<fgrid, BLOCK, 0, st>>>(                                  \
-      (const V*)x, indices, num_tokens, s->experts_per_token, g.nle, s->num_experts,           \
-      s->world_size, g.magic, s->rank, f.row_vecs, f.chunks, (V*)send_buf, send_meta,          \
+      (const V*)x, indices, num_tokens, s->experts_per_token, s->world_size, f.chunks,         \
+      f.row_vecs, g.nle, s->num_experts, g.magic, s->rank, (V*)send_buf, send_meta,            \
       send_counts, send_slot)
 #define LAUNCH(V)                         \
   do {                                    \
@@ -3951,8 +4285,9 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
   const int grid = s->world_size + mover_blocks(group_items(S, g));
 #define LAUNCH(V, NVW)                                                                         \
   dispatch_send_kernel<V, NVW><<<grid, 64 * ROWS, 0, st>>>(                                    \
-      (const V*)x, indices, (int)S, s->experts_per_token, g.nle, s->num_experts, s->world_size, \
-      g.magic, s->rank, g.row_vecs, g.wchunks, (V*)send_buf, send_meta, send_counts, send_slot)
+      (const V*)x, indices, (int)S, s->experts_per_token, s->world_size, grid - s->world_size, \
+      g.wchunks, g.row_vecs, g.nle, s->num_experts, g.magic, s->rank, (V*)send_buf, send_meta, \
+      send_counts, send_slot)
   MOE_A2A_FOR_WAVE_KERNEL(g, LAUNCH);
 #undef LAUNCH
   return launch_status();
@@ -4012,9 +4347,9 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
     const int grid = g.nle + mover_blocks(group_items(rows_hint, g));
 #define LAUNCH_P(V, NVW, PLAN)                                                              \
   dispatch_recv_kernel<V, NVW, PLAN, RECV_POS, THROUGH><<<grid, 64 * ROWS, 0, st>>>(        \
-      (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, capacity_rows,   \
-      g.nle, g.magic, g.max_recv, g.row_vecs, g.wchunks, expert_num_tokens, (V*)expert_x,    \
-      expert_meta, send_back_plan, row_position, nullptr)
+      (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, grid - g.nle,    \
+      g.wchunks, g.row_vecs, g.nle, capacity_rows, g.magic, g.max_recv, expert_num_tokens,   \
+      (V*)expert_x, expert_meta, send_back_plan, row_position, nullptr)
 #define LAUNCH(V, NVW)                     \
   do {                                     \
     if (planned) LAUNCH_P(V, NVW, true);   \
@@ -4030,13 +4365,40 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   }
   // the stream can hold at most nle * max_recv rows that fit the expert buffers
   if (!items_fit((long long)g.nle * g.max_recv, g.wchunks)) return MOE_A2A_EINVAL;
+  if (planned && rows_hint > 0 && rows_hint <= FEW_ENTRIES) {  // (planned: at most 64 ranks)
+    const int few_grid = g.nle + mover_blocks(((long long)rows_hint * g.wchunks + ROWS - 1) / ROWS);
+#define LAUNCH_K(V, NVW, KEYS, COMPACT)                                                      \
+  dispatch_recv_few_kernel<V, NVW, KEYS, COMPACT><<<few_grid, 64 * ROWS, 0, st>>>(           \
+      (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint,                  \
+      few_grid - g.nle, g.wchunks, g.row_vecs, g.nle, capacity_rows, g.magic,                \
+      compact_rows > 0 ? compact_rows : g.max_recv, expert_num_tokens, (V*)expert_x,         \
+      expert_meta, send_back_plan, expert_offsets)
+#define LAUNCH_C(V, NVW, COMPACT)                                       \
+  do {                                                                  \
+    if (rows_hint <= 64 * 4) LAUNCH_K(V, NVW, 4, COMPACT);              \
+    else if (rows_hint <= 64 * 8) LAUNCH_K(V, NVW, 8, COMPACT);         \
+    else if (rows_hint <= 64 * 12) LAUNCH_K(V, NVW, 12, COMPACT);       \
+    else LAUNCH_K(V, NVW, 16, COMPACT);                                 \
+  } while (0)
+#define LAUNCH(V, NVW)                                   \
+  do {                                                   \
+    if (compact_rows > 0) LAUNCH_C(V, NVW, true);        \
+    else LAUNCH_C(V, NVW, false);                        \
+  } while (0)
+    MOE_A2A_FOR_WAVE_KERNEL(g, LAUNCH);
+#undef LAUNCH
+#undef LAUNCH_C
+#undef LAUNCH_K
+    return launch_status();
+  }
   const int grid = g.nle + mover_blocks(group_items(rows_hint, g));
   const bool through =  // (Store)
       rows_hint >= STAGE2_THROUGH_ROWS || (long long)rows_hint * s->hidden_dim * 2 >= STAGE2_THROUGH_BYTES;
 #define LAUNCH_S(V, NVW, PLAN, MODE, HOW)                                                   \
   dispatch_recv_kernel<V, NVW, PLAN, MODE, HOW><<<grid, 64 * ROWS, 0, st>>>(                     \
-      (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, capacity_rows,   \
-      g.nle, g.magic, compact_rows > 0 ? compact_rows : g.max_recv, g.row_vecs, g.wchunks,   \
+      (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, grid - g.nle,    \
+      g.wchunks, g.row_vecs, g.nle, capacity_rows, g.magic,                                  \
+      compact_rows > 0 ? compact_rows : g.max_recv,                                          \
       expert_num_tokens, (V*)expert_x, expert_meta, send_back_plan, nullptr, expert_offsets)
 #define LAUNCH_P(V, NVW, PLAN, MODE)                        \
   do {                                                      \
@@ -4133,9 +4495,9 @@ int launch_combine_send(const moe_a2a_shape* s, const void* expert_y, const int3
   hipStream_t st = (hipStream_t)stream;
 #define LAUNCH_S(V, NVW, SMALL, PLAN)                                                          \
   combine_send_kernel<V, NVW, SMALL, PLAN><<<grid, 64 * ROWS, 0, st>>>(                       \
-      (const V*)expert_y, expert_meta, expert_num_tokens, g.nle, g.max_recv, s->world_size,    \
-      g.row_vecs, g.wchunks, capacity_rows, (V*)send_buf, send_meta, send_counts,              \
-      send_back_plan, compact_rows)
+      expert_num_tokens, send_back_plan, expert_meta, (const V*)expert_y, g.nle,               \
+      s->world_size, g.wchunks, g.max_recv, compact_rows, g.row_vecs, capacity_rows,           \
+      (V*)send_buf, send_meta, send_counts)
 #define LAUNCH(V, NVW)                                   \
   do {                                                   \
     if (planned) LAUNCH_S(V, NVW, true, true);           \
@@ -4184,16 +4546,46 @@ int launch_combine_recv(const moe_a2a_shape* s, const void* recv_buf, const int3
     return_map_kernel<<<mgrid, BLOCK, 0, st>>>(recv_meta, recv_counts, W, rows_hint, capacity_rows,
                                                num_tokens, K, entry_row);
   }
+  // Up to 512 rows every wave looks through the stream by itself (combine_recv_few_kernel); above that the waves share the
+  // scan (601 rows of 8 KB: 4.17 us shared, 4.68 by each wave), with code for what there is of it up to 1024.
+  if (!mapped && g.vec16 && rows_hint > 0 && rows_hint <= COMBINE_FEW_ROWS && W <= 64 && K <= FEW_MAX_K &&
+      (long long)num_tokens * chunks <= 1 << 20) {
+    const int few_grid = num_tokens * chunks;
+#define LAUNCH_A(DT, NV, KEYS, ADDENDS)                                                         \
+  combine_recv_few_kernel<DT, NV, KEYS, ADDENDS><<<few_grid, BLOCK, 0, st>>>(                \
+      recv_meta, recv_counts, weights, W, rows_hint, K, chunks, capacity_rows, (const b128*)recv_buf, \
+      g.row_vecs, accumulate, (b128*)out_tokens)
+#define LAUNCH_K(DT, NV, KEYS)                                                                  \
+  do {                                                                                       \
+    if (K <= 4) LAUNCH_A(DT, NV, KEYS, 4);                                                   \
+    else LAUNCH_A(DT, NV, KEYS, 8);                                                          \
+  } while (0)
+#define LAUNCH(DT, NV)                                                                       \
+  do {                                                                                       \
+    if (rows_hint <= 64 * 4) LAUNCH_K(DT, NV, 4);                                            \
+    else LAUNCH_K(DT, NV, 8);                                                                \
+  } while (0)
+    if (dtype == MOE_A2A_BF16) { if (nv == 1) LAUNCH(MOE_A2A_BF16, 1); else LAUNCH(MOE_A2A_BF16, 2); }
+    else { if (nv == 1) LAUNCH(MOE_A2A_F16, 1); else LAUNCH(MOE_A2A_F16, 2); }
+#undef LAUNCH
+#undef LAUNCH_K
+#undef LAUNCH_A
+    return launch_status();
+  }
 #define LAUNCH(V, DT, BLK, NV)                                                               \
   do {                                                                                       \
     if (mapped)                                                                              \
-      combine_recv_kernel<V, DT, BLK, NV, true><<<grid, BLK, 0, st>>>(                       \
-          (const V*)recv_buf, recv_meta, recv_counts, W, rows_hint, capacity_rows, weights,  \
-          num_tokens, K, g.row_vecs, chunks, (V*)out_tokens, accumulate, entry_row);         \
+      combine_recv_kernel<V, DT, BLK, NV, true, SCAN_UNROLL><<<grid, BLK, 0, st>>>(          \
+          recv_meta, recv_counts, weights, W, rows_hint, num_tokens, K, chunks,              \
+          capacity_rows, (const V*)recv_buf, g.row_vecs, accumulate, (V*)out_tokens, entry_row); \
+    else if (rows_hint <= 4 * BLK)                                                              \
+      combine_recv_kernel<V, DT, BLK, NV, false, 4><<<grid, BLK, 0, st>>>(                   \
+          recv_meta, recv_counts, weights, W, rows_hint, num_tokens, K, chunks,              \
+          capacity_rows, (const V*)recv_buf, g.row_vecs, accumulate, (V*)out_tokens, nullptr); \
     else                                                                                     \
-      combine_recv_kernel<V, DT, BLK, NV, false><<<grid, BLK, 0, st>>>(                      \
-          (const V*)recv_buf, recv_meta, recv_counts, W, rows_hint, capacity_rows, weights,  \
-          num_tokens, K, g.row_vecs, chunks, (V*)out_tokens, accumulate, nullptr);           \
+      combine_recv_kernel<V, DT, BLK, NV, false, SCAN_UNROLL><<<grid, BLK, 0, st>>>(         \
+          recv_meta, recv_counts, weights, W, rows_hint, num_tokens, K, chunks,              \
+          capacity_rows, (const V*)recv_buf, g.row_vecs, accumulate, (V*)out_tokens, nullptr); \
   } while (0)
 #define PICK_SHAPE(V, DT)                       \
   do {                                          \

@@ -1,0 +1,83 @@
+"""Jobs whose streams are short: the kernels that hold every key of a stream in one wave (stages 1, 2 and 4), at the numbers of
+entries where another number of keys per lane or another kernel takes over, against the oracle bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from amd_distributed_2025_amd import HIPAllToAll, LocalWorld, MoEConfig, generate_world
+from oracle import moe_a2a_oracle as orc
+from tests.helpers import bits, run_oracle
+from tests.test_gpu_parity import run_and_compare
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def job(world_size, num_experts, topk, hidden, tokens, routing="uniform", dtype="bf16", seed=5):
+    return generate_world(dict(world_size=world_size, num_experts=num_experts, experts_per_token=topk, hidden_dim=hidden,
+                               max_num_tokens=tokens, num_tokens="full", routing=routing, weights="softmax", dtype=dtype), seed)
+
+
+@pytest.mark.parametrize("entries", [1, 64, 127, 128, 129, 256, 257, 512, 513, 768, 769, 1024, 1025])
+def test_numbers_of_entries(entries):
+    """One entry per token, two ranks: as many rows leave as there are tokens and about as many arrive."""
+    print(f"entries {entries}", flush=True)
+    run_and_compare(job(2, 6, 1, 72, entries))
+
+
+@pytest.mark.parametrize("hidden", [64, 2048, 2056, 4104, 37])
+@pytest.mark.parametrize("world_size,num_experts,topk,tokens", [(4, 24, 5, 100), (8, 64, 8, 32), (4, 8, 3, 170), (2, 64, 64, 4)])
+@pytest.mark.parametrize("routing", ["uniform", "zipf"])
+def test_shapes(world_size, num_experts, topk, tokens, hidden, routing):
+    print(f"shape {world_size} {num_experts} {topk} {tokens} {hidden} {routing}", flush=True)
+    world = job(world_size, num_experts, topk, hidden, tokens, routing, "fp16" if hidden == 2048 else "bf16")
+    _, want = run_and_compare(world)
+    lw = LocalWorld(world[0][0], world_size, device=DEV, layout="compact")
+    ys = lw.run([d.to(DEV) for _, d, _, _ in world])
+    torch.cuda.synchronize()
+    for r, t in enumerate(want):
+        n = int(t.expert_num_tokens.sum())
+        assert np.array_equal(bits(lw.trace[r]["expert_x"][:n]), t.expert_rows), r
+        assert np.array_equal(lw.trace[r]["expert_meta"][:n].cpu().numpy(), t.expert_meta_rows), r
+        assert np.array_equal(bits(ys[r]), t.y), r
+
+
+@pytest.mark.parametrize("hint", [1, 60, 250, 256, 300, 512, 600])
+@pytest.mark.parametrize("layout", ["padded", "compact"])
+def test_a_stream_longer_than_the_hint(layout, hint):
+    """The hint picks the kernel; the rows behind it are moved all the same."""
+    print(f"hint {hint} {layout}", flush=True)
+    world = job(4, 32, 6, 24, 95, "zipf")
+    want = run_oracle(world)
+    lw = LocalWorld(world[0][0], 4, device=DEV, layout=layout)
+    counts_of = lw._exchange_hints
+    lw._exchange_hints = lambda phase, sent: [[max(1, hint // 4) for _ in row] for row in counts_of(phase, sent)]
+    ys = lw.run([d.to(DEV) for _, d, _, _ in world])
+    torch.cuda.synchronize()
+    for r, t in enumerate(want):
+        assert np.array_equal(lw.trace[r]["expert_num_tokens"].cpu().numpy(), t.expert_num_tokens), r
+        assert np.array_equal(bits(lw.trace[r]["back_buf"][: int(t.expert_num_tokens.sum())]), t.back_buf), r
+        assert np.array_equal(bits(ys[r]), t.y), r
+
+
+@pytest.mark.parametrize("arrive", [3, 64, 65, 250])
+@pytest.mark.parametrize("accumulate", [True, False])
+def test_rows_of_one_token(arrive, accumulate):
+    """More rows of one token than the list of a wave holds (64) are added up in arrival order too."""
+    print(f"rows of one token {arrive} {accumulate}", flush=True)
+    T, K, H = 4, 3, 200
+    rng = np.random.default_rng(arrive)
+    cfg = MoEConfig(8, K, H, 128, torch.bfloat16, torch.bfloat16)
+    a = HIPAllToAll(cfg, 0, 2, device=DEV)
+    meta = np.zeros((arrive + 5, 5), np.int32)
+    meta[:, 2], meta[:, 3] = np.where(np.arange(arrive + 5) < arrive, 1, 2), rng.integers(-1, K + 1, arrive + 5)
+    buf = torch.from_numpy(rng.standard_normal((arrive + 5, H)).astype(np.float32)).bfloat16()
+    weights = rng.random((T, K), np.float32)
+    y = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).bfloat16()
+    counts = torch.tensor([arrive, 5], dtype=torch.int32)
+    names = (meta[:, 3] >= 0) & (meta[:, 3] < K)  # (a row whose k names no weight is not added)
+    want = orc.combine_recv(bits(buf)[names], meta[names], weights, T, "bf16", y_init=bits(y) if accumulate else None)
+    got = a.combine_recv(y.to(DEV), torch.from_numpy(weights).to(DEV), counts.to(DEV), buf.to(DEV),
+                         torch.from_numpy(meta).to(DEV), accumulate=accumulate)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(got), want)
