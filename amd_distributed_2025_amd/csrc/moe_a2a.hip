@@ -3594,8 +3594,8 @@ __global__ __launch_bounds__(BLOCK) void exchange_gather_kernel(
 // to its experts' rows and come straight back. Three kernels replace the five stages and two exchanges:
 //   local_plan_kernel      the expert-buffer row of every (rank, token, k) entry (entry_row), in the order in
 //                          which the stages would have put it there: by source rank, token and k inside an
-//                          expert. Left out for up to LOCAL_RANKED_RANKS ranks with LOCAL_RANK_ENTRIES entries
-//                          between them, whose mover ranks them itself (a launch costs more than that scan).
+//                          expert. Left out for up to LOCAL_FEW_RANKS ranks with LOCAL_RANK_ENTRIES entries
+//                          between them, whose mover ranks them itself (local_dispatch_few_kernel).
 //   local_dispatch_kernel  one workgroup per (token, chunk of its row) reads the chunk once and stores it to
 //                          all of the token's expert rows, as it is or through the stand-in expert.
 //   local_combine_kernel   one workgroup per (token, chunk): gathers the token's expert rows and adds them up
@@ -3607,27 +3607,50 @@ __global__ __launch_bounds__(BLOCK) void exchange_gather_kernel(
 constexpr int LOCAL_MAX_RANKS = 64;
 constexpr int LOCAL_MAX_EXPERTS = 1024;     // counters of the plan in LDS
 constexpr int LOCAL_MAX_K = 64;             // entries of a token, one per lane
-constexpr int LOCAL_RANKED_RANKS = 8;
+constexpr int LOCAL_FEW_RANKS = 8;          // a table that a wave holds in scalar registers
 constexpr int LOCAL_RANK_BITS = 11;
-constexpr int LOCAL_RANK_ENTRIES = 1 << LOCAL_RANK_BITS;  // eight keys per lane of the mover's workgroup
+constexpr int LOCAL_RANK_ENTRIES = 1 << LOCAL_RANK_BITS;  // 32 keys per lane of a wave
 
+// Tables of R ranks, passed by value. Jobs of up to eight ranks pass eight entries: a launch with 1.3 KB of arguments takes
+// the host 4.6 us where one with a few words takes 3.0, and eight entries are read at once and picked from by compares,
+// where a table of 64 costs each wave a load of `first` by lane and then one by rank.
+template <int R>
 struct LocalSources {
-  const void* x[LOCAL_MAX_RANKS];
-  const int* indices[LOCAL_MAX_RANKS];
-  int first[LOCAL_MAX_RANKS + 1];  // number of the rank's first token, counted over all ranks
+  const void* x[R];
+  const int* indices[R];
+  int first[R + 1];  // number of the rank's first token, counted over all ranks (up to [W]; INT_MAX behind it)
 };
+template <int R>
 struct LocalResults {
-  const float* weights[LOCAL_MAX_RANKS];
-  void* out[LOCAL_MAX_RANKS];
-  int first[LOCAL_MAX_RANKS + 1];
+  const float* weights[R];
+  void* out[R];
+  int first[R + 1];
 };
 
 // the rank that token number t (the same for every lane of the wave) belongs to
-template <typename Table>
-__device__ __forceinline__ int rank_of_token(const Table& tab, int W, int t) {
-  if (W == 1) return 0;
-  const int lane = threadIdx.x & 63;
-  return __popcll(__ballot(lane < W && tab.first[lane] <= t)) - 1;
+template <int R>
+__device__ __forceinline__ int rank_of_token(const int (&first)[R + 1], int W, int t) {
+  if constexpr (R <= LOCAL_FEW_RANKS) {
+    int r = 0;
+#pragma unroll
+    for (int s = 1; s < R; ++s) r += (int)(first[s] <= t);
+    return r;
+  } else {
+    const int lane = threadIdx.x & 63;
+    return __popcll(__ballot(lane < W && first[lane] <= t)) - 1;
+  }
+}
+// table[r], with r the same for every lane
+template <int R, typename T>
+__device__ __forceinline__ T of_rank(const T* table, int r) {
+  if constexpr (R <= LOCAL_FEW_RANKS) {
+    T v = table[0];
+#pragma unroll
+    for (int s = 1; s < R; ++s) v = s == r ? table[s] : v;
+    return v;
+  } else {
+    return table[r];
+  }
 }
 
 constexpr int LPLAN_BLOCK = 1024, LPLAN_WAVES = LPLAN_BLOCK / 64;
@@ -3641,8 +3664,9 @@ constexpr int LPLAN_BLOCK = 1024, LPLAN_WAVES = LPLAN_BLOCK / 64;
 //   rank_limit     > 0: entries past that many of their destination rank are dropped (what its receive
 //                  buffer holds). Reached only by tokens that name an expert more than once.
 // Entries with an expert outside [0, E) have no row. The last workgroup writes the rows per expert.
+template <int R>
 __global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
-    LocalSources src, int W, int S, int K, int E, int nle, int expert_bits, int rank_bits, bool compact, int max_recv,
+    LocalSources<R> src, int W, int S, int K, int E, int nle, int expert_bits, int rank_bits, bool compact, int max_recv,
     int expert_limit, int rank_limit, int* __restrict__ entry_row, int* __restrict__ expert_num_tokens,
     int* __restrict__ expert_offsets) {
   extern __shared__ int plan_lds[];            // before[E], total[E], in_wave[LPLAN_WAVES][E]
@@ -3786,46 +3810,96 @@ __global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
   if (i < S) entry_row[i] = !keep ? -1 : compact ? total[e] + pos : e * max_recv + pos;
 }
 
-// DIN / DOUT >= 0: rows leave as `row.to(out) * (1 + rank of the expert)` (all2all/reference.py:262).
-// RANKED > 0: entry_row is worked out here (W <= RANKED, S <= LOCAL_RANK_ENTRIES), and workgroup 0 counts
-// the rows per expert where the caller wants to know them; else it is read.
-// Measured with a plan launch / ranked here: 8 ranks x 16 tokens, 2 experts of 8 each, hidden 6144 41.7 / 38 us a
-// job, of which the kernels take 5.8 + 4.7 / 8.1.
-template <typename V, int NV, int DIN, int DOUT, int RANKED, Store HOW>
-__global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
-    LocalSources src, int W, int T, int K, int E, int nle, uint32_t magic, int row_vecs, int chunks, bool compact,
-    int max_recv, int expert_limit, int* __restrict__ entry_row, int* __restrict__ expert_num_tokens,
-    int* __restrict__ expert_offsets, V* __restrict__ rows, int* __restrict__ meta) {
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  int q = blockIdx.x;
-  // expert id of entry i, counted over all ranks (the table is walked at fixed places: one load of it serves all
-  // keys of a lane, where a loop of W trips made each key wait for it W times, 5 us)
-  [[maybe_unused]] auto key_at = [&](int i) {
-    const int* from = src.indices[0];
-    int first = 0;
-#pragma unroll
-    for (int r = 1; r < RANKED; ++r) {
-      const int f = r < W ? src.first[r] * K : INT_MAX;
-      from = f <= i ? src.indices[r] : from;
-      first = f <= i ? f : first;
+// The token's row, held by the workgroup, to its K places: row_of and own hold the places and experts of entries, one per
+// lane. DIN / DOUT >= 0: rows leave as `row.to(out) * (1 + rank of the expert)` (all2all/reference.py:262).
+template <int DIN, int DOUT, Store HOW, typename V, int NV>
+__device__ __forceinline__ void local_rows_out(const Payload<V, NV>& p, int base, int row_vecs, int K, int row_of, int own, int nle,
+                                               uint32_t magic, V* __restrict__ rows) {
+  for (int k = 0; k < K; ++k) {
+    const int row = __builtin_amdgcn_readlane(row_of, k);
+    if (row < 0) continue;
+    V* __restrict__ to = rows + (size_t)row * row_vecs;
+    if constexpr (DIN >= 0) {
+      const int e = __builtin_amdgcn_readlane(own, k);
+      const float scale = (float)(1 + (nle == 1 ? e : (int)__umulhi((uint32_t)e, magic)));
+      Payload<V, NV> y = p;
+      y.map([scale](V v) { return standin_expert<V, DIN, DOUT>(v, scale); });
+      y.template store<HOW>(to, base, row_vecs);
+    } else {
+      p.template store<HOW>(to, base, row_vecs);
     }
-    return from[i - first];
+  }
+}
+__device__ __forceinline__ void local_meta_out(int K, int row_of, int own, int r, int local_t, int* __restrict__ meta) {
+  for (int m0 = 0; m0 < K * META; m0 += BLOCK) {  // (the same trips for every lane: they shuffle)
+    const int m = m0 + threadIdx.x, k = min(m / META, K - 1), f = m - k * META;
+    const int row = __shfl(row_of, k, 64), e = __shfl(own, k, 64);
+    if (m < K * META && row >= 0) meta[(size_t)row * META + f] = f == 0 ? e : f == 1 ? r : f == 2 ? local_t : f == 3 ? k : 0;
+  }
+}
+
+template <typename V, int NV, int DIN, int DOUT, Store HOW, int R>
+__global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
+    const int* __restrict__ entry_row, V* __restrict__ rows, int* __restrict__ meta, int W, int K, int chunks, int row_vecs,
+    int nle, uint32_t magic, LocalSources<R> src) {
+  const int lane = threadIdx.x & 63;
+  const int q = blockIdx.x;
+  const int t = chunks == 1 ? q : q / chunks, c = q - t * chunks;
+  const int row_of = entry_row[(size_t)t * K + min(lane, K - 1)];
+  const int r = rank_of_token<R>(src.first, W, t), local_t = t - of_rank<R>(src.first, r);
+  const int base = c * (BLOCK * NV);
+  const int own = of_rank<R>(src.indices, r)[(size_t)local_t * K + min(lane, K - 1)];
+  Payload<V, NV> p;
+  p.load((const V*)of_rank<R>(src.x, r) + (size_t)local_t * row_vecs, base, row_vecs);
+  local_rows_out<DIN, DOUT, HOW>(p, base, row_vecs, K, row_of, own, nle, magic, rows);
+  if (c == 0 && meta) local_meta_out(K, row_of, own, r, local_t, meta);
+}
+
+// The same without a plan, for few entries of few ranks: every wave holds all keys (KEYS per lane) and ranks entries of its own
+// (wave, wave + 4, ...), as dispatch_few_kernel does; workgroup 0 counts the rows per expert where the caller wants
+// to know them. x0 and indices0 are rank 0's, which is all that a job of one rank has (R = 1).
+// A plan's launch costs more than the scan, and the chain from launch to last store is what bounds these jobs. us of a whole
+// job in a graph with partial counts added up over the waves and tables of 64 ranks / here: 8 ranks x 16 tokens x 2, hidden
+// 6144 10.9 / 7.9, x 30 x 4, 2880 11.9 / 10.3, x 7 x 6, 7168 13.5 / 9.3, x 24 x 8, 4096 13.0 / 12.4 (16.2 with keys that every
+// wave picks up by itself); one rank's dispatch, expert and combine, 16 tokens x 2, hidden 256 10.5 / 9.3, 180 x 8, 4096 18.9 /
+// 17.7.
+template <typename V, int DIN, int DOUT, Store HOW, int R, int KEYS>
+__global__ __launch_bounds__(BLOCK) void local_dispatch_few_kernel(
+    const void* x0, const int* indices0, int T, int K, int E, int chunks, int row_vecs, bool counts, bool compact, int max_recv,
+    int expert_limit, int nle, uint32_t magic, int W, int* __restrict__ entry_row, int* __restrict__ expert_num_tokens,
+    int* __restrict__ expert_offsets, V* __restrict__ rows, int* __restrict__ meta, LocalSources<R> src) {
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int S = T * K;
+  // expert id of entry i, counted over all ranks
+  auto key_at = [&](int i) {
+    const int* from = indices0;
+    if constexpr (R > 1) {
+      int first = 0;
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        const int f = r < W ? src.first[r] * K : INT_MAX;
+        from = f <= i ? src.indices[r] : from;
+        first = f <= i ? f : first;
+      }
+      from -= first;
+    }
+    return from[i];
   };
-  if (RANKED > 0 && (expert_num_tokens || expert_offsets)) {
+  int q = blockIdx.x;
+  if (counts) {
     if (q == 0) {
       __shared__ int hist[LOCAL_MAX_EXPERTS];
       __shared__ int red[NWAVES];
-      constexpr int EACH = LOCAL_MAX_EXPERTS / BLOCK;
-      const int S = T * K;
-      int key[SCAN_UNROLL];
+      constexpr int EACH = LOCAL_MAX_EXPERTS / BLOCK, MINE = KEYS / NWAVES;
+      int key[MINE];
 #pragma unroll
-      for (int u = 0; u < SCAN_UNROLL; ++u) key[u] = key_at(min(tid + u * BLOCK, S - 1));
+      for (int u = 0; u < MINE; ++u) key[u] = key_at(min(tid + u * BLOCK, S - 1));
       for (int j = tid; j < E; j += BLOCK) hist[j] = 0;
-      __syncthreads();
+      lds_barrier();
 #pragma unroll
-      for (int u = 0; u < SCAN_UNROLL; ++u)
+      for (int u = 0; u < MINE; ++u)
         if (tid + u * BLOCK < S && (uint32_t)key[u] < (uint32_t)E) atomicAdd(&hist[key[u]], 1);
-      __syncthreads();
+      lds_barrier();
       int own[EACH], sum = 0;
 #pragma unroll
       for (int j = 0; j < EACH; ++j) {
@@ -3834,7 +3908,7 @@ __global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
       }
       const int incl = wave_inclusive_scan(sum);
       if (lane == 63) red[wave] = incl;
-      __syncthreads();
+      lds_barrier();
       int off = incl - sum;
       for (int w = 0; w < wave; ++w) off += red[w];
 #pragma unroll
@@ -3854,113 +3928,100 @@ __global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
     --q;
   }
   const int t = chunks == 1 ? q : q / chunks, c = q - t * chunks;
-  const int r = rank_of_token(src, W, t), local_t = t - src.first[r];
-  const int* __restrict__ indices = src.indices[r] + (size_t)local_t * K;
-  const int base = c * (BLOCK * NV);
-  const int own = indices[min(lane, K - 1)];
-  int row_of = -1;
-  int key[SCAN_UNROLL];
-  if constexpr (RANKED > 0) {
+  int r = 0, local_t = t;
+  const void* x = x0;
+  const int* indices = indices0;
+  if constexpr (R > 1) {
+    r = rank_of_token<R>(src.first, W, t);
+    local_t = t - of_rank<R>(src.first, r);
+    x = of_rank<R>(src.x, r);
+    indices = of_rank<R>(src.indices, r);
+  }
+  const int base = c * BLOCK;
+  const int own = indices[(size_t)local_t * K + min(lane, K - 1)];
+  // The waves load a quarter of the keys each and share them through LDS where the ranks' pointers have to be picked from
+  // for every key, and where there are many
+  constexpr bool SHARED = R > 1 || KEYS > 4;
+  constexpr int LOADED = SHARED ? KEYS / NWAVES : KEYS;
+  int loaded[LOADED], key[KEYS];
+  const int mine0 = SHARED ? tid : lane;
 #pragma unroll
-    for (int u = 0; u < SCAN_UNROLL; ++u) key[u] = key_at(min(tid + u * BLOCK, T * K - 1));
+  for (int u = 0; u < LOADED; ++u) loaded[u] = key_at(min(mine0 + u * (SHARED ? BLOCK : 64), S - 1));
+  Payload<V, 1> p;
+  p.load((const V*)x + (size_t)local_t * row_vecs, base, row_vecs);
+
+  // a key's place in (expert, entry) order; ids outside [0, E) come last
+  __shared__ int places[LOCAL_MAX_K];
+  auto composite = [&](int e, int i) { return ((uint32_t)e < (uint32_t)E ? e : E) << LOCAL_RANK_BITS | i; };
+#pragma unroll
+  for (int u = 0; u < LOADED; ++u) {
+    const int i = mine0 + u * (SHARED ? BLOCK : 64);
+    loaded[u] = i < S ? composite(loaded[u], i) : INT_MAX;
+  }
+  if constexpr (SHARED) {  // (in whatever order: a key holds its place)
+    __shared__ b128 all[KEYS * 16];
+#pragma unroll
+    for (int u = 0; u < LOADED; ++u) ((int*)all)[tid + u * BLOCK] = loaded[u];
+    lds_barrier();
+#pragma unroll
+    for (int u = 0; u < KEYS / 4; ++u) {
+      const b128 four = all[lane + u * 64];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) key[u * 4 + v] = (int)four[v];
+    }
   } else {
-    row_of = entry_row[(size_t)t * K + min(lane, K - 1)];
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) key[u] = loaded[u];
   }
-  Payload<V, NV> p;
-  p.load((const V*)src.x[r] + (size_t)local_t * row_vecs, base, row_vecs);
-
-  if constexpr (RANKED > 0) {
-    // a key's place in (expert, entry) order; ids outside [0, E) come last
-    // Two 16-bit counts travel in a word. With the stand-in (jobs: compact rows, and still no more than max_recv
-    // of an expert's entries are kept) an entry needs two, everything ahead of it and what of that is in its own
-    // expert; without, one of them, and a word serves two entries.
-    constexpr bool BOTH = DIN >= 0;
-    constexpr int FAN = 8, SUMS = BOTH ? FAN : FAN / 2;
-    __shared__ int part[2][NWAVES][SUMS];
-    const int S = T * K;
-    auto composite = [&](int e, int i) { return ((uint32_t)e < (uint32_t)E ? e : E) << LOCAL_RANK_BITS | i; };
+  for (int k = wave; k < K; k += NWAVES) {
+    const int e = __builtin_amdgcn_readlane(own, k);
+    const int mine = composite(e, t * K + k), from = mine & ~(LOCAL_RANK_ENTRIES - 1);
+    int pos = 0, lower = 0;  // entries ahead of it in its expert, and of lower experts
 #pragma unroll
-    for (int u = 0; u < SCAN_UNROLL; ++u) {
-      const int i2 = tid + u * BLOCK;
-      key[u] = i2 < S ? composite(key[u], i2) : INT_MAX;
+    for (int u = 0; u < KEYS; ++u) pos += __popcll(__ballot((uint32_t)(key[u] - from) < (uint32_t)(mine - from)));
+    if (compact) {
+#pragma unroll
+      for (int u = 0; u < KEYS; ++u) lower += __popcll(__ballot(key[u] < from));
     }
-    for (int g0 = 0, parity = 0; g0 < K; g0 += FAN, parity ^= 1) {
-      int cnt[FAN];
-#pragma unroll
-      for (int g = 0; g < FAN; ++g) {
-        const int k = min(g0 + g, K - 1);
-        const int mine = composite(__builtin_amdgcn_readlane(own, k), t * K + k);
-        const int from = mine & ~(LOCAL_RANK_ENTRIES - 1);
-        cnt[g] = 0;
-#pragma unroll
-        for (int u = 0; u < SCAN_UNROLL; ++u) {
-          if constexpr (BOTH)
-            cnt[g] += (int)(key[u] < mine) + ((int)((uint32_t)(key[u] - from) < (uint32_t)(mine - from)) << 16);
-          else
-            cnt[g] += (int)((uint32_t)(key[u] - (compact ? 0 : from)) < (uint32_t)(mine - (compact ? 0 : from)));
-        }
-      }
-#pragma unroll
-      for (int h = 0; h < SUMS; ++h) {
-        const int sum = wave_sum(BOTH ? cnt[h] : cnt[h] | (cnt[h + FAN - SUMS] << 16));
-        if (lane == 0) part[parity][wave][h] = sum;
-      }
-      lds_barrier();  // (each half of `part` is next written behind the barrier after this one)
-      if (lane >= g0 && lane < min(g0 + FAN, K)) {
-        const int g = lane - g0;
-        int sums = 0;
-#pragma unroll
-        for (int w = 0; w < NWAVES; ++w) sums += part[parity][w][g & (SUMS - 1)];
-        const int low = sums & 0xffff, high = (int)((unsigned)sums >> 16);
-        const int ahead = BOTH || g < SUMS ? low : high, pos = BOTH ? high : ahead;
-        const bool keep = (uint32_t)own < (uint32_t)E && pos < expert_limit;
-        row_of = !keep ? -1 : compact ? ahead : own * max_recv + pos;
-      }
-    }
-    if (c == 0 && wave == 0 && lane < K) entry_row[(size_t)t * K + lane] = row_of;
+    const bool keep = (uint32_t)e < (uint32_t)E && pos < expert_limit;
+    if (lane == 0) places[k] = !keep ? -1 : compact ? lower + pos : e * max_recv + pos;
   }
-
-  for (int k = 0; k < K; ++k) {
-    const int row = __builtin_amdgcn_readlane(row_of, k);
-    if (row < 0) continue;
-    V* __restrict__ to = rows + (size_t)row * row_vecs;
-    if constexpr (DIN >= 0) {
-      const int e = __builtin_amdgcn_readlane(own, k);
-      const float scale = (float)(1 + (nle == 1 ? e : (int)__umulhi((uint32_t)e, magic)));
-      Payload<V, NV> y = p;
-      y.map([scale](V v) { return standin_expert<V, DIN, DOUT>(v, scale); });
-      y.template store<HOW>(to, base, row_vecs);
-    } else {
-      p.template store<HOW>(to, base, row_vecs);
-    }
-  }
-  if (c == 0 && meta) {
-    for (int m0 = 0; m0 < K * META; m0 += BLOCK) {  // (the same trips for every lane: they shuffle)
-      const int m = m0 + tid, k = min(m / META, K - 1), f = m - k * META;
-      const int row = __shfl(row_of, k, 64), e = __shfl(own, k, 64);
-      if (m < K * META && row >= 0) meta[(size_t)row * META + f] = f == 0 ? e : f == 1 ? r : f == 2 ? local_t : f == 3 ? k : 0;
-    }
+  lds_barrier();
+  const int row_of = places[min(lane, K - 1)];
+  local_rows_out<DIN, DOUT, HOW>(p, base, row_vecs, K, row_of, own, nle, magic, rows);
+  if (c == 0) {
+    if (wave == 0 && lane < K) entry_row[(size_t)t * K + lane] = row_of;
+    if (meta) local_meta_out(K, row_of, own, r, local_t, meta);
   }
 }
 
 // MANY: more than eight entries per token.
-template <typename V, int DT, int NV, bool MANY>
+// weights0 and out0 are rank 0's, which is all that a job of one rank has (R = 1).
+template <typename V, int DT, int NV, bool MANY, int R>
 __global__ __launch_bounds__(BLOCK) void local_combine_kernel(
-    LocalResults dst, int W, int first_token, int K, int row_vecs, int chunks, const V* __restrict__ rows,
-    const int* __restrict__ entry_row, int accumulate) {
+    const int* __restrict__ entry_row, const float* weights0, const V* __restrict__ rows, void* out0, int K, int chunks,
+    int row_vecs, int first_token, int accumulate, int W, LocalResults<R> dst) {
   constexpr int N = Words<V>::N, BATCH = 8;
   const int tid = threadIdx.x, lane = tid & 63;
   const int q = blockIdx.x;
   const int item = chunks == 1 ? q : q / chunks, c = q - item * chunks;
   const int t = first_token + item;
-  const int r = rank_of_token(dst, W, t), local_t = t - dst.first[r];
+  int local_t = t;
+  const float* weights = weights0;
+  void* out = out0;
+  if constexpr (R > 1) {
+    const int r = rank_of_token<R>(dst.first, W, t);
+    local_t = t - of_rank<R>(dst.first, r);
+    weights = of_rank<R>(dst.weights, r);
+    out = of_rank<R>(dst.out, r);
+  }
   const int base = c * (BLOCK * NV);
-  V* __restrict__ orow = (V*)dst.out[r] + (size_t)local_t * row_vecs;
+  V* __restrict__ orow = (V*)out + (size_t)local_t * row_vecs;
   // entry of this lane; lanes repeat the entries in runs of 8 unless there are more
   const int k = MANY ? lane : lane & (BATCH - 1);
   const bool there = k < K;
   const int loaded = entry_row[(size_t)t * K + min(k, K - 1)];
-  const float w_loaded = dst.weights[r][(size_t)local_t * K + min(k, K - 1)];
+  const float w_loaded = weights[(size_t)local_t * K + min(k, K - 1)];
   PairAcc<DT> acc[NV][N];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -4898,7 +4959,8 @@ int allow_large_lds() {
   allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8, false>, skinny_lds_bytes(2, 8));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8, true>, skinny_lds_bytes(2, 8));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8, false>, skinny_lds_bytes(2, 8));
-  allow((const void*)local_plan_kernel, local_plan_lds_bytes(LOCAL_MAX_EXPERTS));
+  allow((const void*)local_plan_kernel<LOCAL_FEW_RANKS>, local_plan_lds_bytes(LOCAL_MAX_EXPERTS));
+  allow((const void*)local_plan_kernel<LOCAL_MAX_RANKS>, local_plan_lds_bytes(LOCAL_MAX_EXPERTS));
   if (!ok) return MOE_A2A_ELAUNCH;
   allowed[gpu] = true;
   return MOE_A2A_OK;
@@ -5182,7 +5244,6 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
                   (out_dtype != MOE_A2A_F16 && out_dtype != MOE_A2A_BF16)))
     return MOE_A2A_EINVAL;
   const int W = s->world_size, K = s->experts_per_token, E = s->num_experts;
-  LocalSources src{};
   bool all16 = aligned(expert_rows, 16);
   long long tokens = 0;
   for (int r = 0; r < W; ++r) {
@@ -5190,13 +5251,21 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
       return MOE_A2A_EINVAL;
     if (!aligned(x[r], 2)) return MOE_A2A_EALIGN;
     all16 = all16 && aligned(x[r], 16);
-    src.x[r] = x[r];
-    src.indices[r] = indices[r];
-    src.first[r] = (int)tokens;
     tokens += num_tokens[r];
     if (tokens * K > INT_MAX / 2) return MOE_A2A_EINVAL;
   }
-  src.first[W] = (int)tokens;
+  auto sources = [&](auto table) {
+    int first = 0;
+    for (int r = 0; r < W; ++r) {
+      table.x[r] = x[r];
+      table.indices[r] = indices[r];
+      table.first[r] = first;
+      first += num_tokens[r];
+    }
+    table.first[W] = first;
+    for (int r = W + 1; r < (int)(sizeof(table.first) / sizeof(int)); ++r) table.first[r] = INT_MAX;
+    return table;
+  };
   const int S = (int)(tokens * K);
   if (!aligned(expert_rows, 2)) return MOE_A2A_EALIGN;
   if (S > 0 && !entry_row) return MOE_A2A_EINVAL;
@@ -5213,49 +5282,79 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
   const int expert_limit = compact && !standin ? INT_MAX : g.max_recv;
   const int rank_limit = K > g.nle && g.nle > 1 ? (int)std::min<long long>((long long)g.max_recv * g.nle, INT_MAX) : 0;
   hipStream_t st = (hipStream_t)stream;
-  // Few ranks with few entries: the mover ranks them (LOCAL_RANK_ENTRIES keys, eight per lane)
-  const bool ranked = W <= LOCAL_RANKED_RANKS && S > 0 && S <= LOCAL_RANK_ENTRIES && rank_limit == 0;
-  if (!ranked) {
-    int expert_bits = 0, rank_bits = 0;
-    while ((1 << expert_bits) < E) ++expert_bits;
-    while ((1 << rank_bits) < W) ++rank_bits;
-    if (const int rc = allow_large_lds()) return rc;
-    const int tiles = std::max(1, (S + LPLAN_BLOCK - 1) / LPLAN_BLOCK);
-    local_plan_kernel<<<tiles, LPLAN_BLOCK, local_plan_lds_bytes(E), st>>>(
-        src, W, S, K, E, g.nle, expert_bits, rank_bits, compact, g.max_recv, expert_limit, rank_limit, entry_row,
-        expert_num_tokens, expert_offsets);
-    if (S == 0) return launch_status();
-  }
-  const bool through = (long long)S * s->hidden_dim * 2 >= JOB_THROUGH_BYTES;  // (Store; with a plan's launch, that is with more entries, always)
-  const int grid = (ranked && (expert_num_tokens || expert_offsets) ? 1 : 0) + (int)(tokens * g.chunks);
-#define LAUNCH_H(V, NV, DI, DO, RANKED, HOW)                                                               \
-  local_dispatch_kernel<V, NV, DI, DO, RANKED, HOW><<<grid, BLOCK, 0, st>>>(                               \
-      src, W, (int)tokens, K, E, g.nle, g.magic, g.row_vecs, g.chunks, compact, g.max_recv, expert_limit,  \
-      entry_row, expert_num_tokens, expert_offsets, (V*)expert_rows, expert_meta)
-#define LAUNCH_T(V, NV, DI, DO, RANKED)                                                                    \
+  const bool through = (long long)S * s->hidden_dim * 2 >= JOB_THROUGH_BYTES;  // (Store)
+  // Few ranks with few entries: the mover ranks them
+  const int few_chunks = (g.row_vecs + BLOCK - 1) / BLOCK;
+  if (W <= LOCAL_FEW_RANKS && S > 0 && S <= LOCAL_RANK_ENTRIES && rank_limit == 0 && items_fit(tokens, few_chunks)) {
+    const bool counts = expert_num_tokens || expert_offsets;
+    const int grid = (counts ? 1 : 0) + (int)(tokens * few_chunks);
+#define LAUNCH_H(V, DI, DO, HOW, R, KEYS)                                                                  \
+  local_dispatch_few_kernel<V, DI, DO, HOW, R, KEYS><<<grid, BLOCK, 0, st>>>(                              \
+      x[0], indices[0], (int)tokens, K, E, few_chunks, g.row_vecs, counts, compact, g.max_recv, expert_limit, \
+      g.nle, g.magic, W, entry_row, expert_num_tokens, expert_offsets, (V*)expert_rows, expert_meta,       \
+      sources(LocalSources<R>{}))
+#define LAUNCH_T(V, DI, DO, R, KEYS)                                                                       \
   do {                                                                                                     \
-    if (through) LAUNCH_H(V, NV, DI, DO, RANKED, THROUGH_OF<V>);                                           \
-    else LAUNCH_H(V, NV, DI, DO, RANKED, (RANKED > 0 ? PLAIN : THROUGH_OF<V>));                            \
+    if (through) LAUNCH_H(V, DI, DO, THROUGH_OF<V>, R, KEYS);                                              \
+    else LAUNCH_H(V, DI, DO, PLAIN, R, KEYS);                                                              \
   } while (0)
-#define LAUNCH_R(V, NV, RANKED)                                                                            \
+#define LAUNCH_S(V, R, KEYS)                                                                               \
   do {                                                                                                     \
-    if (!standin) LAUNCH_T(V, NV, -1, -1, RANKED);                                                         \
-    else if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_BF16, RANKED); \
-    else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_F16, RANKED); \
-    else if (in_dtype == MOE_A2A_F16) LAUNCH_T(V, NV, MOE_A2A_F16, MOE_A2A_BF16, RANKED);                  \
-    else LAUNCH_T(V, NV, MOE_A2A_BF16, MOE_A2A_F16, RANKED);                                               \
+    if (!standin) LAUNCH_T(V, -1, -1, R, KEYS);                                                            \
+    else if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_T(V, MOE_A2A_BF16, MOE_A2A_BF16, R, KEYS); \
+    else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_T(V, MOE_A2A_F16, MOE_A2A_F16, R, KEYS); \
+    else if (in_dtype == MOE_A2A_F16) LAUNCH_T(V, MOE_A2A_F16, MOE_A2A_BF16, R, KEYS);                     \
+    else LAUNCH_T(V, MOE_A2A_BF16, MOE_A2A_F16, R, KEYS);                                                  \
   } while (0)
-#define LAUNCH(V, NV)                                                                                      \
+#define LAUNCH_K(V, R)                                                                                     \
   do {                                                                                                     \
-    if (!ranked) LAUNCH_R(V, NV, 0);                                                                       \
-    else if (W == 1) LAUNCH_R(V, NV, 1);                                                                   \
-    else LAUNCH_R(V, NV, LOCAL_RANKED_RANKS);                                                              \
+    if (S <= 64 * 4) LAUNCH_S(V, R, 4);                                                                    \
+    else if (S <= 64 * 16) LAUNCH_S(V, R, 16);                                                             \
+    else LAUNCH_S(V, R, 32);                                                                               \
   } while (0)
-  MOE_A2A_FOR_ROW_KERNEL(g, LAUNCH);
+#define LAUNCH(V)                                                                                          \
+  do {                                                                                                     \
+    if (W == 1) LAUNCH_K(V, 1);                                                                            \
+    else LAUNCH_K(V, LOCAL_FEW_RANKS);                                                                     \
+  } while (0)
+    if (g.vec16) LAUNCH(b128);
+    else LAUNCH(uint16_t);
 #undef LAUNCH
-#undef LAUNCH_R
+#undef LAUNCH_K
+#undef LAUNCH_S
 #undef LAUNCH_T
 #undef LAUNCH_H
+    return launch_status();
+  }
+  int expert_bits = 0, rank_bits = 0;
+  while ((1 << expert_bits) < E) ++expert_bits;
+  while ((1 << rank_bits) < W) ++rank_bits;
+  if (const int rc = allow_large_lds()) return rc;
+  const int tiles = std::max(1, (S + LPLAN_BLOCK - 1) / LPLAN_BLOCK);
+  auto launch = [&](auto table) {
+    constexpr int R = sizeof(table.x) / sizeof(table.x[0]);
+    local_plan_kernel<R><<<tiles, LPLAN_BLOCK, local_plan_lds_bytes(E), st>>>(
+        table, W, S, K, E, g.nle, expert_bits, rank_bits, compact, g.max_recv, expert_limit, rank_limit, entry_row,
+        expert_num_tokens, expert_offsets);
+    if (S == 0) return;
+    const int grid = (int)(tokens * g.chunks);
+#define LAUNCH_H(V, NV, DI, DO)                                                                            \
+  local_dispatch_kernel<V, NV, DI, DO, THROUGH_OF<V>, R><<<grid, BLOCK, 0, st>>>(                          \
+      entry_row, (V*)expert_rows, expert_meta, W, K, g.chunks, g.row_vecs, g.nle, g.magic, table)
+#define LAUNCH(V, NV)                                                                                      \
+  do {                                                                                                     \
+    if (!standin) LAUNCH_H(V, NV, -1, -1);                                                                 \
+    else if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_H(V, NV, MOE_A2A_BF16, MOE_A2A_BF16); \
+    else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_H(V, NV, MOE_A2A_F16, MOE_A2A_F16); \
+    else if (in_dtype == MOE_A2A_F16) LAUNCH_H(V, NV, MOE_A2A_F16, MOE_A2A_BF16);                          \
+    else LAUNCH_H(V, NV, MOE_A2A_BF16, MOE_A2A_F16);                                                       \
+  } while (0)
+    MOE_A2A_FOR_ROW_KERNEL(g, LAUNCH);
+#undef LAUNCH
+#undef LAUNCH_H
+  };
+  if (W <= LOCAL_FEW_RANKS) launch(sources(LocalSources<LOCAL_FEW_RANKS>{}));
+  else launch(sources(LocalSources<LOCAL_MAX_RANKS>{}));
   return launch_status();
 }
 
@@ -5266,23 +5365,31 @@ int moe_a2a_local_combine(const moe_a2a_shape* s, const void* expert_rows, const
       (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16))
     return MOE_A2A_EINVAL;
   const int W = s->world_size, K = s->experts_per_token;
-  LocalResults dst;
   bool all16 = aligned(expert_rows, 16);
   long long tokens = 0;
+  int first = 0;  // token that the launch starts with
   for (int r = 0; r < W; ++r) {
     if (num_tokens[r] < 0 || num_tokens[r] > s->max_num_tokens) return MOE_A2A_EINVAL;
     const bool wanted = (only_rank < 0 || r == only_rank) && num_tokens[r] > 0;
     if (wanted && (!weights[r] || !out_tokens[r])) return MOE_A2A_EINVAL;
     if (wanted && !aligned(out_tokens[r], 2)) return MOE_A2A_EALIGN;
     all16 = all16 && (!wanted || aligned(out_tokens[r], 16));
-    dst.weights[r] = weights[r];
-    dst.out[r] = out_tokens[r];
-    dst.first[r] = (int)tokens;
+    if (r == only_rank) first = (int)tokens;
     tokens += num_tokens[r];
     if (tokens * K > INT_MAX / 2) return MOE_A2A_EINVAL;
   }
-  dst.first[W] = (int)tokens;
-  const int first = only_rank < 0 ? 0 : dst.first[only_rank];
+  auto results = [&](auto table) {
+    int at = 0;
+    for (int r = 0; r < W; ++r) {
+      table.weights[r] = weights[r];
+      table.out[r] = out_tokens[r];
+      table.first[r] = at;
+      at += num_tokens[r];
+    }
+    table.first[W] = at;
+    for (int r = W + 1; r < (int)(sizeof(table.first) / sizeof(int)); ++r) table.first[r] = INT_MAX;
+    return table;
+  };
   const long long items = only_rank < 0 ? tokens : num_tokens[only_rank];
   if (items == 0) return MOE_A2A_OK;
   if (!expert_rows || !entry_row) return MOE_A2A_EINVAL;
@@ -5295,9 +5402,16 @@ int moe_a2a_local_combine(const moe_a2a_shape* s, const void* expert_rows, const
   if (!items_fit(items, chunks)) return MOE_A2A_EINVAL;
   const int grid = (int)(items * chunks);
   hipStream_t st = (hipStream_t)stream;
+#define LAUNCH_R(V, DT, NV, MANY, R)                                                                       \
+  local_combine_kernel<V, DT, NV, MANY, R><<<grid, BLOCK, 0, st>>>(                                        \
+      entry_row, weights[0], (const V*)expert_rows, out_tokens[0], K, chunks, g.row_vecs, first, accumulate, W, \
+      results(LocalResults<R>{}))
 #define LAUNCH(V, DT, NV, MANY)                                                                            \
-  local_combine_kernel<V, DT, NV, MANY><<<grid, BLOCK, 0, st>>>(dst, W, first, K, g.row_vecs, chunks,      \
-                                                                (const V*)expert_rows, entry_row, accumulate)
+  do {                                                                                                     \
+    if (W == 1) LAUNCH_R(V, DT, NV, MANY, 1);                                                              \
+    else if (W <= LOCAL_FEW_RANKS) LAUNCH_R(V, DT, NV, MANY, LOCAL_FEW_RANKS);                             \
+    else LAUNCH_R(V, DT, NV, MANY, LOCAL_MAX_RANKS);                                                       \
+  } while (0)
 #define PICK(V, DT)                                                                                        \
   do {                                                                                                     \
     if (K <= 8) { if (nv == 1) LAUNCH(V, DT, 1, false); else LAUNCH(V, DT, 2, false); }                    \
@@ -5312,6 +5426,7 @@ int moe_a2a_local_combine(const moe_a2a_shape* s, const void* expert_rows, const
   }
 #undef PICK
 #undef LAUNCH
+#undef LAUNCH_R
   return launch_status();
 }
 

@@ -1,12 +1,13 @@
-"""Jobs whose streams are short: the kernels that hold every key of a stream in one wave (stages 1, 2 and 4), at the numbers of
+"""Jobs whose streams are short: the kernels that hold every key of a stream in one wave (stages 1, 2 and 4, and jobs on one GPU), at the numbers of
 entries where another number of keys per lane or another kernel takes over, against the oracle bit for bit."""
 import numpy as np
 import pytest
 import torch
 
-from amd_distributed_2025_amd import HIPAllToAll, LocalWorld, MoEConfig, generate_world
+from amd_distributed_2025_amd import HIPAllToAll, LocalWorld, MoEConfig, custom_kernel_job, generate_world
 from oracle import moe_a2a_oracle as orc
 from tests.helpers import bits, run_oracle
+from tests.test_gpu_local import config, rank_data
 from tests.test_gpu_parity import run_and_compare
 
 pytestmark = pytest.mark.gpu
@@ -81,3 +82,17 @@ def test_rows_of_one_token(arrive, accumulate):
                          torch.from_numpy(meta).to(DEV), accumulate=accumulate)
     torch.cuda.synchronize()
     assert np.array_equal(bits(got), want)
+
+
+@pytest.mark.parametrize("tokens", [[256], [257], [1024], [1025], [2048], [0, 255, 1], [0, 100, 0, 157], [300, 0, 724, 0],
+                                    [0, 0, 0, 0, 0, 0, 3, 1022], [100, 0, 948, 0, 1000]])
+def test_jobs_on_one_gpu(tokens):
+    """Entries where another number of keys per lane takes over, and ranks without tokens, one entry per token."""
+    print(f"jobs {tokens}", flush=True)
+    W = len(tokens)
+    cfg = config(3 * W, 1, 40, max(tokens))
+    data = [rank_data(cfg, t, 11 * r) for r, t in enumerate(tokens)]
+    want = [y.clone() for y in LocalWorld(cfg, W, device=DEV).run(data)]
+    ys = custom_kernel_job([(cfg, d, r, W) for r, d in enumerate(data)])
+    for r in range(W):
+        assert torch.equal(ys[r], want[r]), f"rank {r}"
