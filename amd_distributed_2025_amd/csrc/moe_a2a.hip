@@ -846,6 +846,117 @@ __global__ __launch_bounds__(BLOCK) void dispatch_few_kernel(
   }
 }
 
+// The fan-out of a long stream: a workgroup owns ROWS consecutive tokens, a wave each, and ranks all of their entries in one
+// pass over the keys, which costs the same for one entry as for 64: a lane counts its keys by destination in bytes packed
+// into two words (up to 8 destinations, up to 255 keys per lane), apart for the keys ahead of the workgroup's first entry
+// and the others. From these come where every destination's rows begin and how many of them lie ahead; the workgroup's own
+// entries, one per lane of every wave, add the lanes before them with the same destination. The kernels above compare every
+// key with every entry of one token, which grows with the square of the stream. What bounds this one is the stores of the
+// rows, below some 4 KB per token the passes over the keys (4 bytes and nine instructions each, 2 KB ahead). us, before / here:
+// 2787 tokens of 4 KB, 4 per token 33.4 / 14.6 (the rows alone 10.4 at 5.3 TB/s), 4096 of 14 KB, 8 per token 118.9 / 102.5
+// (99.7), 4096 of 512 bytes, 8 per token 109 / 23.6, 1500 of 1 KB, 6 per token 17.6 / 7.3, 700 of 3.4 KB, 5 per token 8.1 / 5.6,
+// 3626 of 8150 bytes, moved by elements, 3 per token 109 / 37.
+constexpr int BLOCK_RANKS = 8;
+constexpr int BLOCK_MAX_ENTRIES = 255 * BLOCK;  // keys that 256 lanes count in bytes
+
+template <typename V, int NVW, bool POW2>
+__global__ __launch_bounds__(64 * ROWS) void dispatch_block_kernel(
+    const V* __restrict__ x, const int* __restrict__ indices, int T, int K, int W, int chunks, int row_vecs, int E,
+    uint32_t magic, int nle_shift, int rank,
+    V* __restrict__ send_buf, int* __restrict__ send_meta, int* __restrict__ send_counts,
+    int* __restrict__ send_slot) {
+  static_assert(64 * ROWS == BLOCK, "a wave per token");
+  constexpr int KEYS = 8, BATCH = KEYS * BLOCK, WORDS = 4;  // 16-bit pairs: destinations 0 and 2, 1 and 3, 4 and 6, 5 and 7
+  __shared__ int part[ROWS][2 * WORDS];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int S = T * K;
+  const int q = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int grp = chunks == 1 ? q : q / chunks, c = q - grp * chunks;
+  const int t0 = grp * ROWS, i0 = t0 * K, own = min(ROWS, T - t0) * K;  // (own <= 64)
+  auto klass = [&](int e) {
+    const int d = POW2 ? e >> nle_shift : (int)__umulhi((uint32_t)e, magic);
+    return (uint32_t)e >= (uint32_t)E ? BLOCK_RANKS : d;
+  };
+  const int mine = indices[i0 + min(lane, own - 1)];
+  int key[KEYS];
+  auto fetch = [&](int b) {
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) key[u] = indices[min(b + tid + u * BLOCK, S - 1)];
+  };
+  fetch(0);
+  issued_here();
+  const int t = t0 + wave, base = c * (64 * NVW);
+  WavePayload<V, NVW> p;
+  p.load(x + (size_t)min(t, T - 1) * row_vecs, base, row_vecs, lane);
+
+  uint32_t ahead[2] = {}, others[2] = {};  // destinations 0..3 and 4..7, a byte each
+  auto count = [&](uint32_t (&n)[2], int b, int from, int to) {  // the batch's keys in [from, to)
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) {
+      const int i = b + tid + u * BLOCK;
+      const int d = (i >= from) & (i < to) ? klass(key[u]) : BLOCK_RANKS;
+      const uint32_t one = 1u << ((d & 3) * 8);
+      n[0] += d < 4 ? one : 0;
+      n[1] += (uint32_t)(d - 4) < 4u ? one : 0;
+    }
+  };
+  for (int b = 0; b < S; b += BATCH) {
+    if (b > 0) fetch(b);
+    if (b < i0) count(ahead, b, 0, i0);
+    if (b + BATCH > i0) count(others, b, i0, S);
+  }
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    const int a0 = wave_sum((int)(ahead[w] & 0x00ff00ffu)), a1 = wave_sum((int)((ahead[w] >> 8) & 0x00ff00ffu));
+    const int o0 = wave_sum((int)(others[w] & 0x00ff00ffu)), o1 = wave_sum((int)((others[w] >> 8) & 0x00ff00ffu));
+    if (lane == 0) {
+      part[wave][w * 2] = a0;
+      part[wave][w * 2 + 1] = a1;
+      part[wave][WORDS + w * 2] = o0;
+      part[wave][WORDS + w * 2 + 1] = o1;
+    }
+  }
+  lds_barrier();
+  // lane d: entries of destination d ahead of the workgroup's, and all of them
+  const int word = (lane >> 2 & 1) * 2 + (lane & 1), half = (lane >> 1 & 1) * 16;
+  int before = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < ROWS; ++w) {
+    before += part[w][word] >> half & 0xffff;
+    total += part[w][WORDS + word] >> half & 0xffff;
+  }
+  const bool is_rank = lane < W;
+  before = is_rank ? before : 0;
+  total = is_rank ? total + before : 0;
+  const int upto = wave_inclusive_scan(total), all_before = wave_inclusive_scan(before);
+  // (entries without a destination come last: in lane BLOCK_RANKS, behind all ranks)
+  const int first = lane < BLOCK_RANKS ? upto - total + before : upto + i0 - all_before;
+  if (blockIdx.x == 0 && wave == 0 && is_rank) send_counts[lane] = total;
+  const int d = lane < own ? klass(mine) : -1;
+  int slot = __shfl(first, d < 0 ? 0 : d, 64);
+#pragma unroll
+  for (int r = 0; r <= BLOCK_RANKS; ++r) {
+    const unsigned long long same = __ballot(d == r);
+    slot += d == r ? __popcll(same & ((1ull << lane) - 1)) : 0;
+  }
+
+  if (t >= T) return;
+  for (int k = 0; k < K; ++k) {
+    const int to = __builtin_amdgcn_readlane(slot, wave * K + k);
+    p.template store<MOE_A2A_STORE_SEND>(send_buf + (size_t)to * row_vecs, base, row_vecs, lane);
+  }
+  if (c == 0) {
+    for (int b = 0; b < K * META; b += 64) {
+      const int m = b + lane, k = min(m / META, K - 1), f = m - k * META;
+      const int to = __shfl(slot, wave * K + k, 64), e = __shfl(mine, wave * K + k, 64);
+      if (m < K * META) {
+        send_meta[(size_t)to * META + f] = f == 0 ? e : f == 1 ? rank : f == 2 ? t : f == 3 ? k : 0;
+        if (f == 0 && send_slot) send_slot[t * K + k] = to;
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------- send plan (counts, offsets, maps)
 //
 // The stable counting sort of stage 1 made explicit, for callers that want the
@@ -4283,6 +4394,44 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
     else { if (f.vec16) LAUNCH(b128, false); else LAUNCH(uint16_t, false); }
 #undef LAUNCH
 #undef LAUNCH_K
+    return launch_status();
+  }
+  // Longer streams go to the kernel that ranks four tokens in one pass over the keys, but for two kinds of short ones, where
+  // a pass is little beside the rows and the kernels below store them faster: fewer than four entries per token up to
+  // 1280 of them (600 tokens of 14 KB, 2 per token 6.2 / 6.4 us), and long rows as long as a pass over the keys is short
+  // beside the rows of a token, which the tokens and the vectors of a row measure: before / here 8 per token of 14 KB, 1024
+  // tokens 26.2 / 27.8, 1400 34.3 / 36.9, 1800 43.7 / 48.9, 4096 118.9 / 102.5; 4 of 10 KB, 1000 tokens 10.7 / 11.1, 1500
+  // 16.2 / 16.3; 6 of 13.7 KB, 600 tokens 12.0 / 13.0; but 3 of 9.2 KB, 500 tokens 5.6 / 5.4, and rows moved by elements 18.1 /
+  // 10.2 (6 of 4111, 500 tokens).
+  const bool few_entries = s->experts_per_token < MOE_A2A_FANOUT_MIN_K && S <= 1280;
+  const bool long_rows = s->experts_per_token >= MOE_A2A_FANOUT_MIN_K && f.vec16 && f.row_vecs > 2 * BLOCK &&
+                         num_tokens <= 3 * f.row_vecs;
+  if (S > 0 && S <= BLOCK_MAX_ENTRIES && s->world_size <= BLOCK_RANKS && s->experts_per_token * ROWS <= 64 && !few_entries &&
+      !long_rows) {
+    Geometry b = g;
+    const int groups = (num_tokens + ROWS - 1) / ROWS;
+    // Rows are cut into pieces of two vectors per lane where there are few workgroups otherwise, else of four: pieces of 2 / 4 /
+    // whole rows: 250 tokens of 5.8 KB, 8 per token 4.8 / 5.1 / 5.5 us, 1440 of 7.4 KB, 4 per token 11.6 / 12.3 / 12.1, 4096 of
+    // 14 KB, 8 per token 129 / 102 / 106. With one entry a piece would do little but rank: 2000 of 14 KB 13.4 / 10.7 / 9.6.
+    if (b.vec16 && s->experts_per_token > 1) b.nvw = std::min(b.nvw, groups <= 400 ? 2 : 4);
+    b.wchunks = (b.row_vecs + 64 * b.nvw - 1) / (64 * b.nvw);
+    int nle_shift = 0;
+    while ((1 << nle_shift) < g.nle) ++nle_shift;
+    const bool pow2 = (g.nle & (g.nle - 1)) == 0;
+    const int block_grid = groups * b.wchunks;
+#define LAUNCH_B(V, NVW, POW2)                                                                \
+  dispatch_block_kernel<V, NVW, POW2><<<block_grid, 64 * ROWS, 0, st>>>(                      \
+      (const V*)x, indices, num_tokens, s->experts_per_token, s->world_size, b.wchunks,       \
+      b.row_vecs, s->num_experts, g.magic, nle_shift, s->rank, (V*)send_buf, send_meta,       \
+      send_counts, send_slot)
+#define LAUNCH(V, NVW)                            \
+  do {                                            \
+    if (pow2) LAUNCH_B(V, NVW, true);             \
+    else LAUNCH_B(V, NVW, false);                 \
+  } while (0)
+    MOE_A2A_FOR_WAVE_KERNEL(b, LAUNCH);
+#undef LAUNCH
+#undef LAUNCH_B
     return launch_status();
   }
   if (s->experts_per_token >= MOE_A2A_FANOUT_MIN_K && (s->world_size + 2ll) * S <= INT_MAX &&
