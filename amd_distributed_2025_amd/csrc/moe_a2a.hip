@@ -3228,6 +3228,157 @@ __device__ __forceinline__ GroupTile find_group_tile(int tile, const int* __rest
   return at;
 }
 
+// ---------------------------------------------------------------- grouped product, few tiles
+//
+// The experts' product where its tiles leave a unit with one or two workgroups: nothing then hides the way of a step's
+// rows from memory but the steps that are already under way. Four waves fetch the rows of a tile of 32 TM x 32 TN straight
+// into a ring of DEPTH steps in LDS (64 to 144 KB of them) and multiply a quarter of the tile each. One barrier per step:
+// behind it step s + 1 is there for everybody, and everybody holds the fragments of step s, so that its place is free for
+// step s + DEPTH, and the fragments of step s + 1 are read beside the MFMAs of step s (without that, and with all of a tile's
+// 32 columns on one wave, 1 row in 1024 x 7168 took 27.6 us instead of 17.1).
+// LDS rows, fragments and the order of K are those of phased_gemm_kernel.
+// What bounds it: with few tiles the chain of a step (barrier, fragments, two MFMAs: 0.14 us), with more HBM (5 to 6 TB/s
+// from 400 tiles on), on 64 x 128 the fragments' way out of LDS. us, expert_gemm_kernel or dense_gemm_kernel / here: 7 of 48
+// groups with a row, 832 x 3840 21.7 / 11.3; 2 of 8, 2048 x 4096 23.0 / 11.8; 4 groups of 1 row, 2048 x 7168 38.1 / 22.5; 8 of
+// 70, 2048 x 4096 42.4 / 32.3; 7 of 197, 832 x 6528 66.3 / 42.4; 19 of 2, 6272 x 3360 157.0 / 120.6.
+
+constexpr size_t ring_lds_bytes(int TM, int TN, int DEPTH) { return (size_t)DEPTH * (TM + TN) * 32 * 128; }
+
+template <int DT, int TM, int TN, int DEPTH, bool STREAMED>
+__global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
+    const b128* __restrict__ A, const b128* __restrict__ B, const int* __restrict__ rows_of_group,
+    const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int N, int K, int tiles_n, int groups, int max_rows, int compact) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, LA = TM, LB = TN;  // direct loads (8 rows each) of a wave per step
+  constexpr int STEP_BYTES = (BM + BN) * 128, B_AT = BM * 128, RING_BYTES = DEPTH * STEP_BYTES;
+  constexpr int YOUNGER = (LA + LB) * (DEPTH - 2);  // a wave's loads that may be under way when step s + 1 has to be there
+  static_assert(DEPTH >= 3 && YOUNGER + LA + LB < 64, "loads that the wait can count");
+  extern __shared__ b128 tile_lds[];  // [DEPTH][(BM + BN) * 8]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int row_vecs = K / 8, row_bytes = K * 2, steps = (K + GEMM_KSTEP - 1) / GEMM_KSTEP;
+  const int tail_vecs = row_vecs - (steps - 1) * 8;
+  // load i of a wave takes rows i * 32 + wave * 8 .. + 7 of an operand, a lane the vector that belongs at its place
+  const int vec = (lane & 7) ^ ((wave * 4 + (lane >> 4)) & 7);
+  const int off = (wave * 8 + (lane >> 3)) * row_bytes + vec * 16;
+  const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) b128*)tile_lds + wave * 1024;
+  // fragment of a slice of 32 inputs: row r of a band of 16, vector 4 * slice + q of the step
+  const int r = lane & 15, q = lane >> 4, swz = (r >> 1) & 7;
+
+  for (int tile = blockIdx.x;; tile += gridDim.x) {
+    const GroupTile at = find_group_tile<256, BM>(tile, rows_of_group, groups, max_rows, tiles_n, compact, (int*)tile_lds);
+    if (tile >= at.total) return;
+    lds_barrier();
+    const int n0 = at.tn * BN;
+    const int k_first = first_kstep(at.group, groups, K) * (GEMM_KSTEP * 2);
+    const b128 abuf = buffer_words(A + at.row_at * row_vecs, min(BM, at.rows) * row_bytes);
+    const b128 bbuf = buffer_words(B + ((size_t)at.group * N + n0) * row_vecs, min(BN, N - n0) * row_bytes);
+    int past = 0, soff = k_first;  // past the end of the rows in their last step, and everywhere behind it: out of range
+    unsigned fill = 0, use = 0;
+    auto range = [&](int step) __attribute__((always_inline)) {  // before a step near the end is asked for
+      if (step == steps - 1) past = vec >= tail_vecs ? OUT_OF_RANGE : 0;
+      else if (step >= steps) past = OUT_OF_RANGE;
+    };
+    auto load = [&]() __attribute__((always_inline)) {
+      unrolled<0, LA>([&](auto c) __attribute__((always_inline)) {
+        constexpr int i = decltype(c)::value;
+        load_to_lds<i * 4096>(base + fill, off + i * 32 * row_bytes + past, abuf, soff);
+      });
+      unrolled<0, LB>([&](auto c) __attribute__((always_inline)) {
+        constexpr int i = decltype(c)::value;
+        load_to_lds<B_AT + i * 4096, STREAMED>(base + fill, off + i * 32 * row_bytes + past, bbuf, soff);
+      });
+      fill = fill == RING_BYTES - STEP_BYTES ? 0u : fill + STEP_BYTES;
+      soff += GEMM_KSTEP * 2;
+      if (k_first && soff == row_bytes) soff = 0;
+    };
+#pragma unroll 1
+    for (int step = 0; step < DEPTH; ++step) {
+      range(step);
+      load();
+    }
+    f32x4 acc[TM][TN] = {};
+    b128 af[2][2][TM], bf[2][2][TN];  // [set][slice]
+    const bool multiplies = wm * (BM / 2) < at.rows && n0 + wn * (BN / 2) < N;  // (the same for the whole wave)
+    auto read_frags = [&](auto set) __attribute__((always_inline)) {  // of the step in `use`
+      constexpr int f = decltype(set)::value;
+      const char* as = (const char*)tile_lds + use + (wm * (BM / 2) + r) * 128;
+      const char* bs = (const char*)tile_lds + use + B_AT + (wn * (BN / 2) + r) * 128;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int v = ((s * 4 + q) ^ swz) * 16;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) bf[f][s][j] = *(const b128*)(bs + j * (16 * 128) + v);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) af[f][s][i] = *(const b128*)(as + i * (16 * 128) + v);
+      }
+      use = use == RING_BYTES - STEP_BYTES ? 0u : use + STEP_BYTES;
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    auto one_step = [&](auto set, auto other) __attribute__((always_inline)) {
+      constexpr int f = decltype(set)::value;
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER) : "memory");
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      load();
+      if (multiplies) {
+        read_frags(other);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = Mfma16x16x32<DT>::mma(bf[f][s][j], af[f][s][i], acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER + LA + LB) : "memory");
+    lds_barrier();
+    if (multiplies) read_frags(even);
+    int step = 0;
+    for (; step + DEPTH + 2 < steps; step += 2) {  // (what these ask for lies before the last step)
+      one_step(even, odd);
+      one_step(odd, even);
+    }
+    for (; step < steps; step += 2) {
+      range(step + DEPTH);
+      one_step(even, odd);
+      if (step + 1 == steps) break;
+      range(step + 1 + DEPTH);
+      one_step(odd, even);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the loads past the last step write zeros)
+    __syncthreads();
+
+    // this lane: row r of a band, columns q * 4 + 0..3 of 16
+    if (multiplies) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int n = n0 + wn * (BN / 2) + j * 16 + q * 4;
+        if (n >= N) continue;
+        uint32_t bias2[2] = {};
+        if (bias) __builtin_memcpy(bias2, bias + (size_t)at.group * N + n, 8);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const int m = wm * (BM / 2) + i * 16 + r;
+          const f32x4& c = acc[i][j];
+          uint32_t two[2] = {Pair16<DT>::canonical(Pair16<DT>::round(c[0], c[1])),
+                             Pair16<DT>::canonical(Pair16<DT>::round(c[2], c[3]))};
+          if (bias) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+              two[e] = Pair16<DT>::canonical(Pair16<DT>::round(
+                  __fadd_rn(Pair16<DT>::lo(two[e]), Pair16<DT>::lo(bias2[e])),
+                  __fadd_rn(Pair16<DT>::hi(two[e]), Pair16<DT>::hi(bias2[e]))));
+          }
+          if (m < at.rows) __builtin_memcpy(C + (at.row_at + m) * N + n, two, 8);
+        }
+      }
+    }
+  }
+}
+
 template <int DT, int TM, int TN, int NA, int HB, bool AHEAD, bool GROUPED, bool STREAMED = false>
 __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
     const b128* __restrict__ A, const b128* __restrict__ B, const uint16_t* __restrict__ bias,
@@ -4999,6 +5150,7 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   // 89.4 / 71.6; 1, 4, 2048 x 7168 85.8 / 73.0 / 38.2; 4, 8, 1024 x 2048 21.6 / 18.5 / 14.1; 20, 4, 2048 x 7168 86.3 /
   // - / 39.7; 30, 8, 1024 x 4096 45.1 / - / 23.9; 40, 8, 2048 x 7168 101.5 / - / 58.8; but 24, 64, 1024 x 2048 53.4 /
   // 56.2 / 62.1 and 40, 32, 1024 x 512 11.5 / - / 12.4.
+  // (What of these has 24 steps of K or a workgroup per unit at most is ring_gemm_kernel's: grouped_ring.)
   const double average = (double)rows_hint / groups;
   const double blocks_of_32 = groups * std::max(1.0 - std::exp(-average), average / 32 + 0.5);
   const bool counts_fit_32 = (max_rows / 32 + 1) * groups * ((N + 63) / 64) <= INT_MAX / 2;
@@ -5086,6 +5238,10 @@ int allow_large_lds() {
     allow((const void*)phased_gemm_kernel<DT, 8, 4, 2, 6, false, true, S>, phased_lds_bytes(8, 4, 2, 6));
     allow((const void*)phased_gemm_kernel<DT, 6, 4, 2, 6, false, true, S>, phased_lds_bytes(6, 4, 2, 6));
     allow((const void*)dense_gemm_kernel<DT, 2, 2, 2, 2, true, S>, dense_lds_bytes(128, 128));
+    allow((const void*)ring_gemm_kernel<DT, 1, 1, 8, S>, ring_lds_bytes(1, 1, 8));
+    allow((const void*)ring_gemm_kernel<DT, 1, 2, 6, S>, ring_lds_bytes(1, 2, 6));
+    allow((const void*)ring_gemm_kernel<DT, 2, 2, 4, S>, ring_lds_bytes(2, 2, 4));
+    allow((const void*)ring_gemm_kernel<DT, 2, 4, 6, S>, ring_lds_bytes(2, 4, 6));
     allow((const void*)dense_gemm_kernel<DT, 2, 2, 1, 2, true, S>, dense_lds_bytes(64, 128));
   };
   allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 4, false, false>, phased_lds_bytes(8, 4, 3, 4));
@@ -5113,6 +5269,38 @@ int allow_large_lds() {
   if (!ok) return MOE_A2A_ELAUNCH;
   allowed[gpu] = true;
   return MOE_A2A_OK;
+}
+
+// The grouped product on ring_gemm_kernel, in the tiles that grouped_ring has chosen. MOE_A2A_NOT_DENSE where it has too many.
+int launch_grouped_ring(const void* x, const int32_t* rows_of_group, const void* w, const void* bias, void* y, int groups,
+                        long long max_rows, long long rows_hint, int N, int K, int dtype, hipStream_t st, int compact, RingTile way) {
+  const int BM = way == RING_32x32 || way == RING_32x64 ? 32 : 64, BN = way == RING_32x32 ? 32 : way == RING_64x128 ? 128 : 64;
+  const long long tiles_n = (N + BN - 1) / BN;
+  // every group can end in a partly filled row tile; the kernel strides over what the hint misses
+  const long long pairs = (rows_hint / BM + groups) * tiles_n;
+  if ((max_rows / BM + 1) * groups * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
+  const int grid = mover_blocks((pairs + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
+  if (const int rc = allow_large_lds()) return rc;
+  const bool streamed = weights_past_the_cache(groups, rows_hint, N, K) && rows_hint <= (long long)groups * BM;
+  auto launch = [&](auto dtype_const, auto streamed_const) {
+    constexpr int DT = decltype(dtype_const)::value;
+    constexpr bool S = decltype(streamed_const)::value;
+    auto start = [&](auto kernel, int depth) {
+      kernel<<<grid, 256, ring_lds_bytes(BM / 32, BN / 32, depth), st>>>((const b128*)x, (const b128*)w, rows_of_group, (const uint16_t*)bias,
+                                                                         (uint16_t*)y, N, K, (int)tiles_n, groups, (int)max_rows, compact);
+    };
+    if (way == RING_32x32) start(ring_gemm_kernel<DT, 1, 1, 8, S>, 8);
+    else if (way == RING_32x64) start(ring_gemm_kernel<DT, 1, 2, 6, S>, 6);
+    else if (way == RING_64x64) start(ring_gemm_kernel<DT, 2, 2, 4, S>, 4);
+    else start(ring_gemm_kernel<DT, 2, 4, 6, S>, 6);
+  };
+  auto launch_of = [&](auto dtype_const) {
+    if (streamed) launch(dtype_const, std::true_type{});
+    else launch(dtype_const, std::false_type{});
+  };
+  if (dtype == MOE_A2A_BF16) launch_of(std::integral_constant<int, MOE_A2A_BF16>{});
+  else launch_of(std::integral_constant<int, MOE_A2A_F16>{});
+  return launch_status();
 }
 
 // A plain product on tiles that workgroups own whole, as linear_way has chosen.
@@ -5153,7 +5341,7 @@ int launch_linear_tiles(const void* a, const void* b, const void* bias, void* c,
 #ifndef MOE_A2A_GROUPED_DENSE_MIN_ROWS
 #define MOE_A2A_GROUPED_DENSE_MIN_ROWS 56  // rows per group (from the caller's row count) from which tiles are used
 #endif
-// The grouped product from some dozens of rows per group: the dense kernels' tiles (each weight row read once per 64
+// The grouped product where its tiles are few (launch_grouped_ring), and from some dozens of rows per group: the dense kernels' tiles (each weight row read once per 64
 // to 320 rows, operands shared by the workgroup's waves through LDS) do as well as or better than the kernel that is
 // built around streaming the weights. MOE_A2A_NOT_DENSE otherwise.
 int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void* w, const void* bias, void* y,
@@ -5162,6 +5350,10 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
+  if (const RingTile ring = rows_of_group && max_rows <= INT_MAX / 2 ? grouped_ring(rows_hint, groups, N, K) : NO_RING) {
+    const int rc = launch_grouped_ring(x, rows_of_group, w, bias, y, groups, max_rows, rows_hint, N, K, dtype, st, compact, ring);
+    if (rc != MOE_A2A_NOT_DENSE) return rc;
+  }
   if (!rows_of_group || rows_hint < (long long)MOE_A2A_GROUPED_DENSE_MIN_ROWS * groups) return MOE_A2A_NOT_DENSE;
   if (max_rows > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
   const int bands = grouped_tile_bands(rows_hint, groups, N, K);

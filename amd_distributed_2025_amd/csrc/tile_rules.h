@@ -101,6 +101,40 @@ int grouped_tile_bands(long long rows_hint, int groups, int N, int K) {
   return best_bands;
 }
 
+// Tiles of ring_gemm_kernel (rows x columns), or none, for a grouped product. Groups with a row, and their row tiles, are
+// counted as uniform routing would have them.
+//
+// Up to 40 rows per group, where expert_gemm_kernel streams the weights otherwise: from 24 steps of K on, which a ring of six
+// has to be started for only once, and with fewer as long as every unit has one tile at most. 32 x 32 up to a tile per unit,
+// else 32 x 64. From 56 rows on, where dense_gemm_kernel's tiles are the others, and between: as long as no unit has a second
+// tile of 64 x 128 and some are left over (with 256 of few steps two workgroups of the other on a unit are ahead), on 64 x 64
+// while there is a unit for each, on 32 x 64 below 56 rows. us, the others / 32 x 32 / 32 x 64 / 64 x 64 / 64 x 128 (rows, groups, N x K):
+//    1 each in 5 of 41, 576 x 3520  19.8 / 10.5 / 12.3 / 15.0 / 22.2     1 each in 5 of 45, 2144 x 1344  13.2 / 10.6 /  8.0 /  8.6 / 11.8
+//   22, 7, 768 x 6656               35.8 / 19.6 / 27.1 / 30.8 / 45.5     12, 36, 5728 x 2432              183 /  167 /  152 /  155 /  176
+//   46, 8, 1024 x 3648              22.7 / 21.0 / 18.0 / 22.3 / 32.1     52, 9, 2304 x 5568              66.4 / 76.9 / 64.7 / 61.5 / 53.2
+//  143, 6, 960 x 2400               27.2 / 28.2 / 22.8 / 17.7 / 27.3     282, 4, 1472 x 4992             46.0 / 72.6 / 58.8 / 42.8 / 37.9
+// and where the others stay: 2, 53, 2240 x 512 23.3 / 35.8 / 29.4; 2.25, 64, 2048 x 1024 45.3 / - / 51.3; 51, 48, 1856 x 1184 54.5 / - /
+// 75.7 / 58.3 / 67.6; 68, 41, 512 x 640 12.7 / 23.1 / 17.1 / 16.0 / 19.7. Over 100 products (0.1 to 300 rows, N and K of 512 to 7168) the
+// choice takes 0.85 of the others' time (geometric mean; the best of all five 0.83) and 1.04 at most.
+enum RingTile { NO_RING = 0, RING_32x32, RING_32x64, RING_64x64, RING_64x128 };
+
+RingTile grouped_ring(long long rows_hint, int groups, int N, int K) {
+  constexpr double UNITS = 256;
+  if (!tile_rows_in_range(128, K)) return NO_RING;
+  const double rows = (double)rows_hint / groups, hit = 1.0 - std::exp(-rows);
+  auto tiles = [&](int high, int wide) {
+    const double of_a_group = rows < 0.7 ? hit : std::max(hit, rows / high + 0.5);
+    return of_a_group * groups * ((N + wide - 1) / wide);
+  };
+  if (rows <= 40) {
+    if (tiles(32, 32) <= UNITS) return RING_32x32;
+    return (K + 63) / 64 >= 24 || tiles(32, 64) <= UNITS ? RING_32x64 : NO_RING;
+  }
+  if (tiles(64, 128) > UNITS * 15 / 16) return NO_RING;
+  if (rows < 56) return tiles(32, 64) <= UNITS ? RING_32x64 : RING_64x128;
+  return tiles(64, 64) <= UNITS ? RING_64x64 : RING_64x128;
+}
+
 // The kernel of a plain product [M, N, K].
 //
 // Up to 160 tiles of 256 x 256 a product takes, per step of K, what its workgroups wait for (about the same for every

@@ -1,0 +1,60 @@
+"""Grouped products of few tiles (`ring_gemm_kernel`): every tile it is launched with, on walks of K shorter than the ring, as
+long, and longer, with rows and columns that end inside a tile."""
+import pytest
+import torch
+
+from amd_distributed_2025_amd import HIPAllToAll, MoEConfig
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# tile (RingTile) -> groups, out_dim, rows per group that the caller promises (test_tile_rules.py holds the rule to that)
+RING_TILES = {1: (3, 96, 8), 2: (5, 3872, 9), 3: (3, 160, 70), 4: (6, 2080, 80)}
+RING_STEPS = [8, 64, 136, 256, 320, 328, 384, 448, 512, 520, 1000, 2048]  # from 24 steps on the streaming kernel has some fewer
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("K", RING_STEPS)
+@pytest.mark.parametrize("tile", RING_TILES)
+def test_rings_on_small_integers(tile, K, bias, dt):
+    """Small integers, whose sums every order gives exactly (below 2^11 but for a rounding of bfloat16)."""
+    groups, N, rows = RING_TILES[tile]
+    print(f"ring tile={tile} K={K} bias={bias} {dt}", flush=True)
+    T = 100
+    a = HIPAllToAll(MoEConfig(groups, 1, K, T, dt, dt), 0, 1, device=torch.device(DEV))
+    g = torch.Generator(device=DEV).manual_seed(K + tile)
+    counts = [65, 0, 97, 1, 100, 32][:groups]
+    x = torch.randint(-1, 2, (groups, T, K), generator=g, device=DEV).to(dt)
+    w = torch.randint(-1, 2, (groups, N, K), generator=g, device=DEV).to(dt)
+    b = torch.randint(-9, 10, (groups, N), generator=g, device=DEV).to(dt) if bias else None
+    num = torch.tensor(counts, dtype=torch.int32, device=DEV)
+    flat = torch.cat([x[e, :c] for e, c in enumerate(counts)] + [x[0, :5]]).contiguous()  # (and rows of nobody)
+    hint = rows * groups
+    out = a.expert_gemm(x, num, w, b, rows_hint=hint, out=torch.full((groups, T, N), 7.0, dtype=dt, device=DEV))
+    packed = a.expert_gemm(flat, num, w, b, rows_hint=hint, out=torch.full((len(flat), N), 7.0, dtype=dt, device=DEV))
+    at = 0
+    for e, c in enumerate(counts):
+        want = (x[e, :c].double() @ w[e].double().T).to(dt)
+        if bias:
+            want = (want.double() + b[e].double()).to(dt)
+        assert torch.equal(out[e, :c], want), e
+        assert (out[e, c:] == 7).all()
+        assert torch.equal(packed[at:at + c], want), e
+        at += c
+    assert (packed[at:] == 7).all()
+
+
+@pytest.mark.parametrize("tile", RING_TILES)
+def test_rings_keep_the_bits(tile):
+    """The row count picks the tile and changes no bit: against a count at which none of these runs."""
+    groups, N, rows = RING_TILES[tile]
+    print(f"ring bits tile={tile}", flush=True)
+    for K in (1544, 2048, 2112):
+        a = HIPAllToAll(MoEConfig(groups, 1, K, 130, torch.bfloat16, torch.bfloat16), 0, 1, device=torch.device(DEV))
+        g = torch.Generator(device=DEV).manual_seed(K)
+        x = torch.randn(groups, 130, K, generator=g, device=DEV).bfloat16()
+        w = (torch.randn(groups, N, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+        num = torch.tensor([130, 31, 64, 0, 66, 2][:groups], dtype=torch.int32, device=DEV)
+        got, base = (a.expert_gemm(x, num, w, None, rows_hint=hint, out=torch.zeros(groups, 130, N, dtype=x.dtype, device=DEV))
+                     for hint in (rows * groups, 30000 * groups))
+        assert torch.equal(got, base), K

@@ -9,6 +9,7 @@ import pytest
 from tests.test_gpu_expert_gemm import TILES_OF_NARROW
 from tests.test_gpu_grouped_tiles import FEW_STEPS, PAST_THE_CACHE, ROWS_FOR_TILE
 from tests.test_gpu_linear import WAYS, WITH_A_NEXT_TILE
+from tests.test_gpu_ring_tiles import RING_STEPS, RING_TILES
 
 CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
 
@@ -21,6 +22,7 @@ def rules(tmp_path_factory):
     src.write_text('#include "tile_rules.h"\n'
                    'extern "C" int bands(long long rows_hint, int groups, int n, int k) { return grouped_tile_bands(rows_hint, groups, n, k); }\n'
                    'extern "C" int past(int groups, long long rows_hint, int n, int k) { return weights_past_the_cache(groups, rows_hint, n, k); }\n'
+                   'extern "C" int ring(long long rows_hint, int groups, int n, int k) { return grouped_ring(rows_hint, groups, n, k); }\n'
                    'extern "C" int way(long long m, long long n, long long k) { return linear_way(m, n, k); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
@@ -28,6 +30,7 @@ def rules(tmp_path_factory):
     dll = C.CDLL(str(lib))
     dll.bands.argtypes = [C.c_longlong, C.c_int, C.c_int, C.c_int]
     dll.past.argtypes = [C.c_int, C.c_longlong, C.c_int, C.c_int]
+    dll.ring.argtypes = [C.c_longlong, C.c_int, C.c_int, C.c_int]
     dll.way.argtypes = [C.c_longlong] * 3
     return dll
 
@@ -160,3 +163,22 @@ def test_ways_of_a_product_stay_in_the_range_of_their_kernels(rules):
                     assert (n // 32) * ((m + 31) // 32) < 2 ** 31  # workgroups
                 if way == STREAM_WEIGHTS:
                     assert k >= 2097152
+
+
+@pytest.mark.parametrize("tile", RING_TILES)
+def test_rings_that_the_gpu_tests_mean(rules, tile):
+    groups, n, rows = RING_TILES[tile]
+    for k in [*RING_STEPS, 1544, 2112]:
+        few_steps = tile == 2 and k < 24 * 64 - 56
+        assert rules.ring(rows * groups, groups, n, k) == (0 if few_steps else tile), k
+    assert rules.ring(30000 * groups, groups, n, 2048) == 0
+
+
+@pytest.mark.parametrize("rows_hint,groups,n,k,tile", [
+    (7, 48, 832, 3840, 1), (2, 8, 4096, 2048, 1), (4, 4, 2048, 7168, 1), (144, 64, 1024, 2048, 2), (425, 36, 5728, 2432, 2),
+    (368, 8, 1024, 3648, 2), (858, 6, 960, 2400, 3), (1379, 7, 832, 6528, 4), (468, 9, 2304, 5568, 4),
+    (144, 64, 2048, 1024, 0), (118, 53, 2240, 512, 0), (2792, 41, 512, 640, 0), (2468, 48, 1856, 1184, 0), (8192, 32, 2048, 4096, 0),
+    (0, 3, 7168, 200, 1), (7, 48, 832, 1 << 23, 0),
+])
+def test_ring_that_was_fastest(rules, rows_hint, groups, n, k, tile):
+    assert rules.ring(rows_hint, groups, n, k) == tile
