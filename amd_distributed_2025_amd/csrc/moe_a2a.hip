@@ -3151,7 +3151,7 @@ constexpr size_t phased_lds_bytes(int TM, int TN, int NA, int HB) {  // NA buffe
 }
 
 // Tiles of a grouped product: A is [groups, max_rows, K], B [groups, N, K], C [groups, max_rows, N], and group g
-// has rows_of_group[g] rows (read here, clamped to max_rows). A group's rows are spread evenly over the fewest
+// has rows_of_group[g] rows (read here, clamped to max_rows; null: max_rows). A group's rows are spread evenly over the fewest
 // tiles of BM rows, in whole bands of 32; tiles are numbered by group, column tile and row tile, so that
 // neighbours share the group's weights. compact: A and C hold the groups' rows back to back in buffers of
 // max_rows rows. The rows ahead of a group are a prefix over the counts, and a group only has the rows that
@@ -3175,7 +3175,7 @@ __device__ __forceinline__ GroupTile find_group_tile(int tile, const int* __rest
   int* const red_rows = lds + 8;
   int* const home = lds + 16;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  auto rows_of = [=](int g) { return min(max(rows_of_group[g], 0), max_rows); };
+  auto rows_of = [=](int g) { return rows_of_group ? min(max(rows_of_group[g], 0), max_rows) : max_rows; };
   auto kept_of = [=](int g, int ahead) {
     const int n = rows_of(g);
     return compact ? min(ahead + n, max_rows) - min(ahead, max_rows) : n;
@@ -3228,9 +3228,9 @@ __device__ __forceinline__ GroupTile find_group_tile(int tile, const int* __rest
   return at;
 }
 
-// ---------------------------------------------------------------- grouped product, few tiles
+// ---------------------------------------------------------------- products of few tiles
 //
-// The experts' product where its tiles leave a unit with one or two workgroups: nothing then hides the way of a step's
+// The experts' product, or a plain one, where its tiles leave a unit with one or two workgroups: nothing then hides the way of a step's
 // rows from memory but the steps that are already under way. Four waves fetch the rows of a tile of 32 TM x 32 TN straight
 // into a ring of DEPTH steps in LDS (64 to 144 KB of them) and multiply a quarter of the tile each. One barrier per step:
 // behind it step s + 1 is there for everybody, and everybody holds the fragments of step s, so that its place is free for
@@ -5271,7 +5271,8 @@ int allow_large_lds() {
   return MOE_A2A_OK;
 }
 
-// The grouped product on ring_gemm_kernel, in the tiles that grouped_ring has chosen. MOE_A2A_NOT_DENSE where it has too many.
+// A product on ring_gemm_kernel, in the tiles that grouped_ring or linear_ring has chosen (rows_of_group null: max_rows rows in
+// every group). MOE_A2A_NOT_DENSE where it has too many.
 int launch_grouped_ring(const void* x, const int32_t* rows_of_group, const void* w, const void* bias, void* y, int groups,
                         long long max_rows, long long rows_hint, int N, int K, int dtype, hipStream_t st, int compact, RingTile way) {
   const int BM = way == RING_32x32 || way == RING_32x64 ? 32 : 64, BN = way == RING_32x32 ? 32 : way == RING_64x128 ? 128 : 64;
@@ -5428,6 +5429,10 @@ int launch_linear(const void* x, const void* w, const void* bias, void* y, int M
   if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
+  if (const RingTile ring = linear_ring(M, N, K)) {
+    const int rc = launch_grouped_ring(x, nullptr, w, bias, y, 1, M, M, N, K, dtype, st, 0, ring);
+    if (rc != MOE_A2A_NOT_DENSE) return rc;
+  }
   const LinearWay way = linear_way(M, N, K);
   int rc = MOE_A2A_NOT_DENSE;
   if (way == SPLIT_32 || way == SPLIT_64) rc = launch_linear_split(x, w, bias, y, M, N, K, dtype, way == SPLIT_32 ? 1 : 2, st);

@@ -171,7 +171,8 @@ enum LinearWay {
   STREAM_WEIGHTS                       // expert_gemm_kernel, as one group
 };
 
-LinearWay linear_way(long long M, long long N, long long K) {
+// `*least_cost`: what the choice costs by that comparison, where there was one.
+LinearWay linear_way(long long M, long long N, long long K, long long* least_cost = nullptr) {
   constexpr long long UNITS = 256, SPLIT_MIN_STEPS = 8;  // (two for each of four waves)
   constexpr long long SPLIT_MAX_TILES = 192;             // of 128 columns, up to 64 rows
   // (sizes of tiles as powers of two: a small product waits for every division here)
@@ -205,7 +206,27 @@ LinearWay linear_way(long long M, long long N, long long K) {
     consider(PHASED_192, cost_of((M + 191) / 192 * ((N + 127) >> 7), 192 + 128, 680, 0));
     consider(PHASED_256, cost(8, 8, 1380, 0));
   }
+  if (least_cost) *least_cost = least;
   return best;
+}
+
+// Whether a plain product goes to ring_gemm_kernel instead. With K too short to be split it is ahead on tiles of 32 x 32 as
+// long as every unit has one at most. Above, tiles of 64 x 64, which it has under way for longer than dense_gemm_kernel and which fetch
+// no more than skinny_gemm_kernel does, fill a gap between those two; a wait of 300 in the comparison above finds them (280 to 320 choose
+// the same of 95 shapes), from 12 steps on (shorter ones are as fast elsewhere). us, linear_way's choice / here:
+//   137 x 4320 x 5440  47.9 / 25.7     200 x 4096 x 4096  36.9 / 21.4     82 x 6592 x 2816  27.1 / 16.9
+//   494 x 2048 x 2176  20.1 / 13.4     128 x 8192 x 2048  21.2 / 14.9    195 x 3008 x 832    7.7 /  7.5
+// and on 32 x 32: 15 x 5888 x 448 5.5 / 4.7, 80 x 2176 x 448 5.6 / 4.8, 4 x 7104 x 280 5.0 / 4.4; but 33 x 4608 x 352 5.3 / 5.5.
+// Elsewhere the others stay: 255 x 1728 x 3968 14.7 / 21.6, 349 x 4032 x 2752 26.8 / 25.4, 358 x 6976 x 2096 27.7 / 39.0.
+RingTile linear_ring(long long M, long long N, long long K) {
+  constexpr long long UNITS = 256, WAIT = 300;
+  const long long steps = (K + 63) / 64;
+  if (steps < 8) return (M + 31) / 32 * ((N + 31) / 32) <= UNITS ? RING_32x32 : NO_RING;
+  if (steps < 12 || M <= 64) return NO_RING;
+  const long long n = (M + 63) / 64 * ((N + 63) / 64);
+  long long least = 0;  // (more than a unit's tile each, or one of the largest tiles: not compared)
+  if (n > UNITS || linear_way(M, N, K, &least) == STREAM_WEIGHTS) return NO_RING;
+  return WAIT * UNITS + n * (64 + 64) < least ? RING_64x64 : NO_RING;
 }
 
 }  // namespace

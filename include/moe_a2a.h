@@ -368,7 +368,7 @@ int moe_a2a_expert_gemm(const moe_a2a_shape* shape, const void* expert_x,
  * float32 with one rounding to the 16-bit type; a bias is then added to that
  * rounded value and the sum rounded again, which is what the two torch
  * statements do. bias may be NULL.
- * One of four kernels runs, picked from the shape alone (so a shape always
+ * One of five kernels runs, picked from the shape alone (so a shape always
  * gives the same bits; other numbers of rows, above 64 too, or of columns are another
  * shape, in which the same row may be added up in another order and differ in
  * its last bits; a slice of the weight's rows is another shape as well, and where
@@ -379,7 +379,9 @@ int moe_a2a_expert_gemm(const moe_a2a_shape* shape, const void* expert_x,
  * 64 and n <= 24448 and else where larger tiles would leave compute units without
  * work; kernels bound by the matrix cores, whose workgroups own output tiles of
  * 256 x 256, 192 x 128, 128 x 128 or 64 x 128 (all of them add the same terms in
- * the same order); for shapes beyond their index ranges, the kernel of moe_a2a_expert_gemm
+ * the same order); where tiles of 64 x 64 (of 32 x 32 for k <= 448) are at most one
+ * per compute unit and the others would take longer, the kernel that
+ * moe_a2a_expert_gemm has for few tiles, in that order too; for shapes beyond their index ranges, the kernel of moe_a2a_expert_gemm
  * with one group of m rows.
  * Limits: n a multiple of 32, k a multiple of 8, input / weight / output 16-byte
  * and bias 8-byte aligned (MOE_A2A_EINVAL / EALIGN). m == 0 is a no-op.

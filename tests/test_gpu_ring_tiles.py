@@ -3,7 +3,7 @@ long, and longer, with rows and columns that end inside a tile."""
 import pytest
 import torch
 
-from amd_distributed_2025_amd import HIPAllToAll, MoEConfig
+from amd_distributed_2025_amd import HIPAllToAll, MoEConfig, gemm_rs
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -58,3 +58,24 @@ def test_rings_keep_the_bits(tile):
         got, base = (a.expert_gemm(x, num, w, None, rows_hint=hint, out=torch.zeros(groups, 130, N, dtype=x.dtype, device=DEV))
                      for hint in (rows * groups, 30000 * groups))
         assert torch.equal(got, base), K
+
+
+RING_LINEAR = [(1, 32, 8), (31, 64, 64), (33, 96, 136), (100, 2016, 448), (256, 1024, 320),
+               (65, 7168, 768), (129, 4320, 1000), (200, 4064, 4096), (511, 2048, 1544), (250, 3936, 777 * 8)]
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("m,n,k", RING_LINEAR)
+def test_plain_products(m, n, k, dt):
+    """Small integers again, with stray NaNs around the operands and sentinels around the result."""
+    print(f"ring linear {m} {n} {k} {dt}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    x, w = torch.full((m + 2, k), float("nan"), dtype=dt, device=DEV), torch.full((n + 2, k), float("nan"), dtype=dt, device=DEV)
+    x[1:m + 1] = torch.randint(-1, 2, (m, k), generator=g, device=DEV).to(dt)
+    w[1:n + 1] = torch.randint(-1, 2, (n, k), generator=g, device=DEV).to(dt)
+    b = torch.randint(-9, 10, (n,), generator=g, device=DEV).to(dt)
+    out = torch.full((m + 2, n), 777.0, dtype=dt, device=DEV)
+    gemm_rs.local_product((x[1:m + 1], w[1:n + 1], b), out=out[1:m + 1])
+    want = ((x[1:m + 1].double() @ w[1:n + 1].double().T).to(dt).double() + b.double()).to(dt)
+    assert torch.equal(out[1:m + 1], want)
+    assert (out[0] == 777).all() and (out[m + 1] == 777).all()

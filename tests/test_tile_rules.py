@@ -23,6 +23,7 @@ def rules(tmp_path_factory):
                    'extern "C" int bands(long long rows_hint, int groups, int n, int k) { return grouped_tile_bands(rows_hint, groups, n, k); }\n'
                    'extern "C" int past(int groups, long long rows_hint, int n, int k) { return weights_past_the_cache(groups, rows_hint, n, k); }\n'
                    'extern "C" int ring(long long rows_hint, int groups, int n, int k) { return grouped_ring(rows_hint, groups, n, k); }\n'
+                   'extern "C" int linear_ring_of(long long m, long long n, long long k) { return linear_ring(m, n, k); }\n'
                    'extern "C" int way(long long m, long long n, long long k) { return linear_way(m, n, k); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
@@ -31,6 +32,7 @@ def rules(tmp_path_factory):
     dll.bands.argtypes = [C.c_longlong, C.c_int, C.c_int, C.c_int]
     dll.past.argtypes = [C.c_int, C.c_longlong, C.c_int, C.c_int]
     dll.ring.argtypes = [C.c_longlong, C.c_int, C.c_int, C.c_int]
+    dll.linear_ring_of.argtypes = [C.c_longlong] * 3
     dll.way.argtypes = [C.c_longlong] * 3
     return dll
 
@@ -182,3 +184,15 @@ def test_rings_that_the_gpu_tests_mean(rules, tile):
 ])
 def test_ring_that_was_fastest(rules, rows_hint, groups, n, k, tile):
     assert rules.ring(rows_hint, groups, n, k) == tile
+
+
+@pytest.mark.parametrize("m,n,k,tile", [
+    (137, 4320, 5440, 3), (200, 4096, 4096, 3), (82, 6592, 2816, 3), (494, 2048, 2176, 3), (195, 3008, 832, 3),
+    (255, 1728, 3968, 0), (349, 4032, 2752, 0), (160, 4544, 512, 0), (64, 7168, 2304, 0), (8192, 8192, 3696, 0), (2048, 2880, 360, 0),
+    (15, 5888, 448, 1), (80, 2176, 448, 1), (33, 4608, 352, 0), (1, 32, 8, 1), (100, 4096, 1 << 22, 0),
+])
+def test_plain_products_on_rings(rules, m, n, k, tile):
+    assert rules.linear_ring_of(m, n, k) == tile
+    from tests.test_gpu_ring_tiles import RING_LINEAR
+    for rows, columns, inputs in RING_LINEAR:
+        assert rules.linear_ring_of(rows, columns, inputs), (rows, columns, inputs)
