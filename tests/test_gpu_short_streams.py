@@ -96,3 +96,16 @@ def test_jobs_on_one_gpu(tokens):
     ys = custom_kernel_job([(cfg, d, r, W) for r, d in enumerate(data)])
     for r in range(W):
         assert torch.equal(ys[r], want[r]), f"rank {r}"
+
+
+@pytest.mark.parametrize("world_size", [1, 3])
+@pytest.mark.parametrize("hidden", [2064, 4104, 5000, 7168, 1001])
+def test_jobs_whose_lanes_move_several_vectors(world_size, hidden):
+    """More than 1024 entries and two workgroups per unit: lanes move one, two or four vectors of a row."""
+    print(f"several vectors {world_size} {hidden}", flush=True)
+    cfg = config(4 * world_size, 2, hidden, 600)
+    data = [rank_data(cfg, 540 if world_size == 1 else t, 7 * r) for r, t in enumerate([200, 341, 0][:world_size])]
+    want = [y.clone() for y in LocalWorld(cfg, world_size, device=DEV).run(data)]
+    ys = custom_kernel_job([(cfg, d, r, world_size) for r, d in enumerate(data)])
+    for r in range(world_size):
+        assert torch.equal(ys[r], want[r]), f"rank {r}"
