@@ -3230,8 +3230,8 @@ __device__ __forceinline__ GroupTile find_group_tile(int tile, const int* __rest
 
 // ---------------------------------------------------------------- products of few tiles
 //
-// The experts' product, or a plain one, where its tiles leave a unit with one or two workgroups: nothing then hides the way of a step's
-// rows from memory but the steps that are already under way. Four waves fetch the rows of a tile of 32 TM x 32 TN straight
+// The experts' product, or a plain one, where its tiles leave a unit with one or two workgroups (and some with long walks of K,
+// grouped_ring): nothing then hides the way of a step's rows from memory but the steps that are already under way. Four waves fetch the rows of a tile of 32 TM x 32 TN straight
 // into a ring of DEPTH steps in LDS (64 to 144 KB of them) and multiply a quarter of the tile each. One barrier per step:
 // behind it step s + 1 is there for everybody, and everybody holds the fragments of step s, so that its place is free for
 // step s + DEPTH, and the fragments of step s + 1 are read beside the MFMAs of step s (without that, and with all of a tile's
@@ -5144,19 +5144,16 @@ int launch_grouped_gemm(const void* x, const int32_t* rows_of_group, const void*
   if (!tile_rows_in_range(128, K) || max_rows > INT_MAX / 2) return MOE_A2A_EINVAL;
   // Blocks of 32 rows on workgroups of 64 columns where they do better than 64 x 128. (1) Up to eight rows per
   // group: twice as many workgroups share the stream of weights out more evenly. (2) Too few workgroups to keep
-  // that stream in flight, at most two per unit: each then looks four steps ahead. They are counted as uniform
-  // routing would have it: the groups that get a row, or half a block on top of whole ones. Measured, us, blocks
+  // that stream in flight, at most two per unit: each then looks four steps ahead (streams_far_ahead). Measured, us, blocks
   // of 64 on 128 columns / of 32 on 64, two steps / four (rows per group, groups, N x K): 2.25, 64, 2048 x 1024 52.6
   // / 44.4 / -; the same, 1024 x 2048 44.8 / 44.5 / -; 4, 8, 7168 x 2048 45.6 / 42.2 / -; 2, 64, 512 x 7168 98.1 /
   // 89.4 / 71.6; 1, 4, 2048 x 7168 85.8 / 73.0 / 38.2; 4, 8, 1024 x 2048 21.6 / 18.5 / 14.1; 20, 4, 2048 x 7168 86.3 /
   // - / 39.7; 30, 8, 1024 x 4096 45.1 / - / 23.9; 40, 8, 2048 x 7168 101.5 / - / 58.8; but 24, 64, 1024 x 2048 53.4 /
   // 56.2 / 62.1 and 40, 32, 1024 x 512 11.5 / - / 12.4.
-  // (What of these has 24 steps of K or a workgroup per unit at most is ring_gemm_kernel's: grouped_ring.)
-  const double average = (double)rows_hint / groups;
-  const double blocks_of_32 = groups * std::max(1.0 - std::exp(-average), average / 32 + 0.5);
+  // (Some of these are ring_gemm_kernel's by now: grouped_ring.)
   const bool counts_fit_32 = (max_rows / 32 + 1) * groups * ((N + 63) / 64) <= INT_MAX / 2;
-  const bool far_ahead = counts_fit_32 && blocks_of_32 * ((N + 63) / 64) <= 512;
-  const bool few = counts_fit_32 && (far_ahead || average <= 8);
+  const bool far_ahead = counts_fit_32 && streams_far_ahead(rows_hint, groups, N);
+  const bool few = counts_fit_32 && (far_ahead || rows_hint <= 8ll * groups);
   const int tj = few ? 1 : rows_hint > (long long)MOE_A2A_GEMM_ROWS_FOR_128 * groups ? 4 : 2;
   // every group can end in a partly filled block of tokens; the kernel strides over what the hint misses
   const long long row_blocks = rows_hint / (tj * 32) + groups;

@@ -101,38 +101,56 @@ int grouped_tile_bands(long long rows_hint, int groups, int N, int K) {
   return best_bands;
 }
 
+// Whether expert_gemm_kernel has so few blocks (32 rows on 64 columns, at most two per unit) that each looks four steps ahead.
+// They are counted as uniform routing would have it: the groups that get a row, or half a block on top of whole ones.
+bool streams_far_ahead(long long rows_hint, int groups, int N) {
+  const double average = (double)rows_hint / groups;
+  return groups * std::max(1.0 - std::exp(-average), average / 32 + 0.5) * ((N + 63) / 64) <= 512;
+}
+
 // Tiles of ring_gemm_kernel (rows x columns), or none, for a grouped product. Groups with a row, and their row tiles, are
-// counted as uniform routing would have them.
+// counted as uniform routing would have them, and `of_*` is how many tiles that makes per unit.
 //
-// Up to 40 rows per group, where expert_gemm_kernel streams the weights otherwise: from 24 steps of K on, which a ring of six
-// has to be started for only once, and with fewer as long as every unit has one tile at most. 32 x 32 up to a tile per unit,
-// else 32 x 64. From 56 rows on, where dense_gemm_kernel's tiles are the others, and between: as long as no unit has a second
-// tile of 64 x 128 and some are left over (with 256 of few steps two workgroups of the other on a unit are ahead), on 64 x 64
-// while there is a unit for each, on 32 x 64 below 56 rows. us, the others / 32 x 32 / 32 x 64 / 64 x 64 / 64 x 128 (rows, groups, N x K):
-//    1 each in 5 of 41, 576 x 3520  19.8 / 10.5 / 12.3 / 15.0 / 22.2     1 each in 5 of 45, 2144 x 1344  13.2 / 10.6 /  8.0 /  8.6 / 11.8
-//   22, 7, 768 x 6656               35.8 / 19.6 / 27.1 / 30.8 / 45.5     12, 36, 5728 x 2432              183 /  167 /  152 /  155 /  176
-//   46, 8, 1024 x 3648              22.7 / 21.0 / 18.0 / 22.3 / 32.1     52, 9, 2304 x 5568              66.4 / 76.9 / 64.7 / 61.5 / 53.2
-//  143, 6, 960 x 2400               27.2 / 28.2 / 22.8 / 17.7 / 27.3     282, 4, 1472 x 4992             46.0 / 72.6 / 58.8 / 42.8 / 37.9
-// and where the others stay: 2, 53, 2240 x 512 23.3 / 35.8 / 29.4; 2.25, 64, 2048 x 1024 45.3 / - / 51.3; 51, 48, 1856 x 1184 54.5 / - /
-// 75.7 / 58.3 / 67.6; 68, 41, 512 x 640 12.7 / 23.1 / 17.1 / 16.0 / 19.7. Over 100 products (0.1 to 300 rows, N and K of 512 to 7168) the
-// choice takes 0.85 of the others' time (geometric mean; the best of all five 0.83) and 1.04 at most.
+// As long as every unit has one tile at most a ring is ahead of expert_gemm_kernel, on 32 x 32 up to 40 rows per group, on 32 x 64
+// where those are too many, and from 56 rows on of dense_gemm_kernel, on 64 x 64 and then 64 x 128 (of which nearly a unit's worth pays
+// from 40 rows on). With more tiles the kernel that streams the weights looks four steps ahead up to two blocks per unit and is as fast
+// or faster. Beyond, where it does not, walks of K that are long beside the start of a ring are ahead: of 48 steps with up to three
+// tiles per unit (between three and four the last round is nearly empty), of 24 with five or more, on 32 x 64 up to 24 rows per group
+// and on 64 x 64 up to 44: tiles of 32 rows would there read most groups' weights twice, under skewed routing (a group of 300 rows
+// in ten tiles) and uniform routing alike. us, the others / 32 x 32 / 32 x 64 / 64 x 64 / 64 x 128 (rows, groups, N x K):
+//    1 each in 5 of 41, 576 x 3520  19.8 / 10.5 / 12.3 / 15.0 / 22.2     9, 43, 2240 x 2752          123 / 92.4 / 86.5 / 88.7 / 110
+//   22, 7, 768 x 6656               35.8 / 19.6 / 27.1 / 30.8 / 45.5     46, 8, 1024 x 3648          22.7 / 21.0 / 18.0 / 22.3 / 32.1
+//   35, 48, 512 x 2432              39.2 / 40.4 / 40.6 / 30.4 / 28.3     52, 9, 2304 x 5568          66.4 / 76.9 / 64.7 / 61.5 / 53.2
+//  143, 6, 960 x 2400               27.2 / 28.2 / 22.8 / 17.7 / 27.3     282, 4, 1472 x 4992         46.0 / 72.6 / 58.8 / 42.8 / 37.9
+// and where the others stay: 40, 8, 7168 x 7168 (skewed) 144 / - / 182 / 165 / 143; 28, 8, 7168 x 1536 (skewed) 37.9 / - / 47.5 / 40.4 /
+// 42.8; 40, 128, 1792 x 7168 587 / - / 719 / 566 / 537; 28, 128, 4096 x 2880 516 / - / 611 / 532 / 542; 4, 8, 7168 x 2048 39.7 / - / 44.1 /
+// 45.7 / 46.6; 2, 53, 2240 x 512 23.3 / 35.8 / 29.4; 68, 41, 512 x 640 12.7 / 23.1 / 17.1 / 16.0 / 19.7.
+// Over 12204 products (4 to 128 groups, 0.06 to 400 rows per group, N and K of 512 to 14000, half of them with Zipf's routing, exponent
+// 1.2) the choice takes 0.907 of the others' time (geometric mean; the best of all five 0.88) and is more than 5 % behind them on 1.3 %.
 enum RingTile { NO_RING = 0, RING_32x32, RING_32x64, RING_64x64, RING_64x128 };
 
 RingTile grouped_ring(long long rows_hint, int groups, int N, int K) {
   constexpr double UNITS = 256;
   if (!tile_rows_in_range(128, K)) return NO_RING;
+  const int steps = (K + 63) / 64;
   const double rows = (double)rows_hint / groups, hit = 1.0 - std::exp(-rows);
-  auto tiles = [&](int high, int wide) {
+  auto per_unit = [&](int high, int wide) {
     const double of_a_group = rows < 0.7 ? hit : std::max(hit, rows / high + 0.5);
-    return of_a_group * groups * ((N + wide - 1) / wide);
+    return of_a_group * groups * ((N + wide - 1) / wide) / UNITS;
   };
-  if (rows <= 40) {
-    if (tiles(32, 32) <= UNITS) return RING_32x32;
-    return (K + 63) / 64 >= 24 || tiles(32, 64) <= UNITS ? RING_32x64 : NO_RING;
-  }
-  if (tiles(64, 128) > UNITS * 15 / 16) return NO_RING;
-  if (rows < 56) return tiles(32, 64) <= UNITS ? RING_32x64 : RING_64x128;
-  return tiles(64, 64) <= UNITS ? RING_64x64 : RING_64x128;
+  if (rows <= 40 && per_unit(32, 32) <= 1) return RING_32x32;
+  const double of_32 = per_unit(32, 64), of_64 = per_unit(64, 64), of_128 = per_unit(64, 128);
+  if (rows >= 56) return of_64 <= 1 ? RING_64x64 : of_128 <= 0.9 ? RING_64x128 : NO_RING;
+  if (rows > 40 && of_128 >= 0.6 && of_128 <= 0.9) return RING_64x128;
+  const bool far_ahead = streams_far_ahead(rows_hint, groups, N);
+  // (few rows hit now more groups, now less; where nothing else is under way either, more than a tile per unit is still ahead)
+  if (of_32 <= (rows < 2 && far_ahead ? 0.9 : rows < 1 ? 1.5 : 1.0)) return RING_32x64;
+  if (far_ahead) return rows > 24 && of_64 >= 0.75 && of_64 <= 0.95 ? RING_64x64 : NO_RING;
+  if (rows > 24 && of_64 <= 2) return RING_64x64;
+  const double tiles = rows <= 24 ? of_32 : of_64;
+  const bool long_walk = (steps >= 24 && tiles >= 5) || (steps >= 48 && (tiles < 3 || tiles >= 4));
+  if (rows > 44 || !long_walk) return NO_RING;
+  return rows <= 24 ? RING_32x64 : RING_64x64;
 }
 
 // The kernel of a plain product [M, N, K].

@@ -333,8 +333,8 @@ int moe_a2a_expert_scale(const moe_a2a_shape* shape, const void* expert_x,
  * Rows are processed in blocks found from the device-side counts, so the work
  * follows the rows, not the experts. rows_hint (the rows the caller expects
  * over all experts) picks the kernel and sizes the launch, and changes no bit
- * of the result: where tiles are few, tiles of 32 or 64 rows x 32 to 128 columns
- * whose workgroups keep up to 144 KB of K under way; else from 56 rows per expert on average, output tiles of 192, 256 or
+ * of the result: where tiles are few, or walks of K long, tiles of 32 or 64 rows x 32 to 128
+ * columns whose workgroups keep up to 144 KB of K under way; else from 56 rows per expert on average, output tiles of 192, 256 or
  * 320 rows x 256 columns or of 64 or 128 rows x 128 columns (whichever keeps the
  * GPU busiest) of the kernels behind moe_a2a_linear, numbered over the experts; below, a kernel
  * built around streaming every weight once, in blocks of 32, 64 or 128 tokens

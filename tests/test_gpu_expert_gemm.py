@@ -99,20 +99,24 @@ def test_small_integers_sum_exactly(H, dt):
                               want.astype(np.float32))
 
 
-# rows per expert (of five) -> rows of a tile, by (in_dim, out_dim); test_tile_rules.py holds the tiles to that
-TILES_OF_NARROW = {(96, 160): {56: 64, 768: 64, 3000: 128, 10000: 256}, (200, 64): {56: 64, 768: 64, 10000: 128},
-                   (128, 128): {56: 64, 768: 64, 10000: 128}}
+# experts, in_dim, out_dim -> counts of rows per expert and the kernel that they pick; test_tile_rules.py holds them to that
+KERNELS_OF_NARROW = {
+    (5, 96, 160): {0: "ring 32 x 32", 56: "ring 64 x 64", 768: "ring 64 x 64", 3000: "tiles 128", 10000: "tiles 256"},
+    (5, 200, 64): {0: "ring 32 x 32", 56: "ring 64 x 64", 768: "ring 64 x 64", 10000: "tiles 128"},
+    (5, 128, 128): {0: "ring 32 x 32", 56: "ring 64 x 64", 768: "ring 64 x 64", 10000: "tiles 128"},
+    (128, 96, 160): {2: "stream 32, four steps ahead", 60: "tiles 128"},
+    (300, 200, 160): {2: "stream 32, two steps ahead", 20: "stream 64", 50: "stream 128", 60: "tiles 64"}}
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("in_dim,out_dim", TILES_OF_NARROW)
-def test_bias_and_unequal_widths_on_every_kernel(in_dim, out_dim, dt):
+@pytest.mark.parametrize("nle,in_dim,out_dim", KERNELS_OF_NARROW)
+def test_bias_and_unequal_widths_on_every_kernel(nle, in_dim, out_dim, dt):
     """[nle, out_dim, in_dim] weights with a bias, small integers (every order of the sum agrees, and
-    both roundings are exact): the streaming kernel (row count 0) and the tiles that `TILES_OF_NARROW`
-    lists for counts of rows per expert all give the integers of `x @ w.T + b`."""
-    print(f"bias in={in_dim} out={out_dim} {dt}", flush=True)
+    both roundings are exact): the kernels that `KERNELS_OF_NARROW` lists for counts of rows per expert
+    all give the integers of `x @ w.T + b`."""
+    print(f"bias nle={nle} in={in_dim} out={out_dim} {dt}", flush=True)
     rng = np.random.default_rng(in_dim * 7 + out_dim)
-    W, nle, max_tokens = 1, 5, 300
+    W, max_tokens = 1, 300 if nle < 10 else 140
     a, cfg = rank_object(W, nle, in_dim, max_tokens, dt)
     counts = ragged_counts(rng, nle, max_tokens, [max_tokens, 0, 65, 129])
     x = rng.integers(-1, 2, (nle, max_tokens, in_dim))
@@ -121,7 +125,7 @@ def test_bias_and_unequal_widths_on_every_kernel(in_dim, out_dim, dt):
     ex, wt, bt = (torch.from_numpy(v).to(dt).to(DEV) for v in (x, w, b))
     num = torch.tensor(counts, dtype=torch.int32, device=DEV)
     name = dtype_name(dt)
-    for hint in [0] + [rows * nle for rows in TILES_OF_NARROW[in_dim, out_dim]]:
+    for hint in [rows * nle for rows in KERNELS_OF_NARROW[nle, in_dim, out_dim]]:
         out = torch.empty(nle, max_tokens, out_dim, dtype=dt, device=DEV)
         out.view(torch.int16).fill_(SENTINEL)
         got = a.expert_gemm(ex, num, wt, bias=bt, rows_hint=hint, out=out)
@@ -279,18 +283,18 @@ def test_wide_workgroups_of_every_width(H, width):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("nle,H,max_tokens,counts", [
     # ragged last tiles in both directions, an empty expert, exact multiples of the tile, few rows: the row counts
-    # below take tiles of 64, 128 and 192 rows, and of 192 and 256
+    # below take tiles of 128 and 192 rows, and of 192 and 256
     (6, 416, 400, [384, 0, 5, 400, 131, 256]),
     (5, 7168, 300, [290, 213, 0, 256, 129]),
-    # several tiles per expert: of 64 and 192 rows, and of 64, 128 and 192
+    # several tiles per expert: of 192 rows, and of 128 and 192
     (3, 320, 1100, [1100, 770, 513]),
     (2, 1024, 1030, [1025, 1024]),
 ])
 def test_tiles_for_experts_with_hundreds_of_rows(nle, H, max_tokens, counts, dt):
     """From 56 rows per expert (judged from the row count the caller passes) the product runs on tiles, found
     over the experts from the device-side counts. The row count only picks the
-    kernel and sizes the launch: every value of it gives the same bits, those of the streaming kernel
-    (hint 0) included, within the float32 bound, and rows past the counts stay untouched."""
+    kernel and sizes the launch: every value of it gives the same bits, those of the rings of few tiles
+    (0 rows: 32 x 32) included, within the float32 bound, and rows past the counts stay untouched."""
     print(f"gemm tiles nle={nle} H={H} counts={counts} {dt}", flush=True)
     a, cfg = rank_object(1, nle, H, max_tokens, dt)
     total = sum(counts)
@@ -300,7 +304,7 @@ def test_tiles_for_experts_with_hundreds_of_rows(nle, H, max_tokens, counts, dt)
 
 
 def test_graph_replays_of_both_products_match_eager():
-    """The grouped product (on tiles, and the streaming kernel through a low row count) and the gemm-rs
+    """The grouped product (on tiles and on a ring, by the row count) and the gemm-rs
     product captured in a HIP graph after one warm-up call each (the first call on a GPU sets kernel
     attributes): every replay, with new operands and eager work in between, gives the eager bits."""
     from amd_distributed_2025_amd import gemm_rs
@@ -313,10 +317,12 @@ def test_graph_replays_of_both_products_match_eager():
     w = (torch.randn(nle, H, H, generator=g, device=DEV) / H ** 0.5).to(dt)
     lin = gemm_rs.generate_input(0, 8, 512, 4096, 12288, True, 663, device=DEV)
     lin_out = torch.empty(512, 4096, dtype=dt, device=DEV)
+    ring_out = torch.empty(nle, T, H, dtype=dt, device=DEV)
     outs = {}
 
     def step():
-        outs["tiles"] = a.expert_gemm(ex, num, w, rows_hint=sum(counts))
+        outs["ring"] = a.expert_gemm(ex, num, w, rows_hint=sum(counts), out=ring_out)
+        outs["tiles"] = a.expert_gemm(ex, num, w, rows_hint=600 * nle)
         outs["linear"] = gemm_rs.local_product(lin, out=lin_out)
 
     side = torch.cuda.Stream()
@@ -334,12 +340,12 @@ def test_graph_replays_of_both_products_match_eager():
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
-        got_tiles, got_lin = outs["tiles"].clone(), outs["linear"].clone()
-        want_tiles = a.expert_gemm(ex, num, w, rows_hint=0).clone()   # eager, the streaming kernel: the same bits
+        got, got_lin = {k: outs[k].clone() for k in ("ring", "tiles")}, outs["linear"].clone()
+        want = a.expert_gemm(ex, num, w, rows_hint=0).clone()   # eager, on other tiles: the same bits
         want_lin = gemm_rs.local_product(lin).clone()
         torch.cuda.synchronize()
         for le, c in enumerate(counts):
-            assert torch.equal(got_tiles[le, :c], want_tiles[le, :c]), f"replay {i}, expert {le}"
+            assert all(torch.equal(g[le, :c], want[le, :c]) for g in got.values()), f"replay {i}, expert {le}"
         assert torch.equal(got_lin, want_lin), f"replay {i}: linear"
 
 
@@ -363,11 +369,12 @@ def _random_layouts(seed, count):
 
 @pytest.mark.parametrize("nle,H,max_tokens,counts", _random_layouts(77, 14))
 def test_random_layouts_give_the_same_bits_on_every_kernel(nle, H, max_tokens, counts):
-    """Random numbers of experts, row lengths and ragged counts: the streaming kernel (row count 0) and the
-    tiles that the true row count (56 per expert at least) and one of 768 per expert pick give the same bits,
-    inside the float32 bound, and leave the rows past the counts alone."""
+    """Random numbers of experts, row lengths and ragged counts: the ring that a row count of 0 picks, what 2, 20 and 52
+    rows per expert pick (the streaming kernel where that makes many tiles), and the tiles of the true row count (56 per
+    expert at least) and one of 768 per expert give the same bits, inside the float32 bound, and leave the rows past the
+    counts alone."""
     print(f"gemm random layout nle={nle} H={H} T={max_tokens} rows={sum(counts)}", flush=True)
     a, cfg = rank_object(1, nle, H, max_tokens, torch.bfloat16)
     base = random_case(a, cfg, 1, counts, seed=nle * 1000 + H, hint=0, check_experts=[0, nle - 1])
-    for hint in (max(sum(counts), 56 * nle), 768 * nle):
+    for hint in (2 * nle, 20 * nle, 52 * nle, max(sum(counts), 56 * nle), 768 * nle):
         assert np.array_equal(run_gemm_same(a, cfg, 1, counts, nle * 1000 + H, hint), base), f"hint {hint}"

@@ -9,10 +9,12 @@ from amd_distributed_2025_amd import HIPAllToAll, MoEConfig
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-# rows per group -> kernel and rows of a tile, by groups, at N = 7168 and K of 2048 or 2112 (csrc/tile_rules.h;
-# test_tile_rules.py holds the tiles to that)
-ROWS_FOR_TILE = {3: {20: "stream 32, four steps ahead", 50: "stream 128", 60: 64, 100: 128, 150: 192, 600: 256, 800: 320},
-                 5: {8: "stream 32, two steps ahead", 20: "stream 64", 100: 192, 230: 256, 300: 320}}
+# rows per group -> the kernel, by groups, at N = 7168 and every K below (csrc/tile_rules.h; test_tile_rules.py holds the
+# kernels to that)
+KERNELS = {3: {20: "stream 32, four steps ahead", 0: "ring 32 x 32", 50: "ring 64 x 128", 60: "tiles 64", 100: "tiles 128",
+               150: "tiles 192", 600: "tiles 256", 800: "tiles 320"},
+           5: {8: "stream 32, two steps ahead", 20: "stream 64", 50: "stream 128", 100: "tiles 192", 230: "tiles 256",
+               300: "tiles 320"}}
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
@@ -23,7 +25,7 @@ ROWS_FOR_TILE = {3: {20: "stream 32, four steps ahead", 50: "stream 128", 60: 64
     (5, [704, 704, 650, 704, 704]),  # more rows than any of the row counts: workgroups take a second tile, some a third
 ])
 @pytest.mark.parametrize("K", [8, 200, 2048, 2112])  # one short step; a tail; a walk that starts apart; one that does not
-def test_every_tile_gives_the_same_bits(groups, counts, K, bias, dt):
+def test_every_kernel_gives_the_same_bits(groups, counts, K, bias, dt):
     print(f"tiles groups={groups} counts={counts} K={K} bias={bias} {dt}", flush=True)
     N, T = 7168, 704
     a = HIPAllToAll(MoEConfig(groups, 1, K, T, dt, dt), 0, 1, device=torch.device(DEV))
@@ -38,7 +40,7 @@ def test_every_tile_gives_the_same_bits(groups, counts, K, bias, dt):
         out = torch.full((*rows.shape[:-1], N), 7.0, dtype=dt, device=DEV)
         return a.expert_gemm(rows, num, w, b, rows_hint=hint, out=out)
 
-    base = run(x, 0)  # streams in blocks of 32 rows, four steps ahead
+    base = run(x, next(iter(KERNELS[groups])) * groups)  # (streams the weights in blocks of 32 rows)
     ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dt]  # of one rounding, to either side
     for e, c in enumerate(counts):
         want = x[e, :c].double() @ w[e].double().T
@@ -49,7 +51,7 @@ def test_every_tile_gives_the_same_bits(groups, counts, K, bias, dt):
             bound = (1 + ulp) * bound + ulp * want.abs()
         assert ((base[e, :c].double() - want).abs() <= bound + 2.0 ** -24).all(), f"group {e}"
         assert (base[e, c:] == 7).all()
-    for rows in ROWS_FOR_TILE[groups]:
+    for rows in KERNELS[groups]:
         got = run(x, rows * groups)
         assert torch.equal(got, base), f"row count {rows} per group"
         got = run(flat, rows * groups)
@@ -82,27 +84,31 @@ def test_few_steps_on_the_ring_of_half_steps(K):
             assert (out[e, c:] == 7).all()
 
 
-# groups, K -> rows per group and the tile (0: a block that streams the weights) of weights of 256 MB and more at N = 7168,
-# which are read with loads that leave nothing in the caches: every kernel of the grouped product has such a form
-PAST_THE_CACHE = {(3, 6272): {20: 0, 50: 0, 60: 64, 100: 128, 150: 192}, (5, 3752): {8: 0, 30: 0, 230: 256, 300: 320}}
+# groups, N, K -> rows per group and the kernel, for weights of 256 MB and more, which are read with loads that leave nothing
+# in the caches: every kernel of the grouped product has such a form
+PAST_THE_CACHE = {(3, 7168, 6272): {20: "stream 32, four steps ahead", 50: "ring 64 x 128", 60: "tiles 64", 100: "tiles 128",
+                                    150: "tiles 192"},
+                  (5, 7168, 3752): {8: "ring 32 x 64", 30: "ring 64 x 64", 230: "tiles 256", 300: "tiles 320"},
+                  (8, 1024, 16384): {1: "ring 32 x 32"},
+                  (64, 2048, 1024): {2: "stream 32, two steps ahead", 20: "stream 64", 50: "stream 128"}}
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("groups,K", PAST_THE_CACHE)
-def test_weights_that_the_cache_cannot_hold(groups, K, dt):
+@pytest.mark.parametrize("groups,N,K", PAST_THE_CACHE)
+def test_weights_that_the_cache_cannot_hold(groups, N, K, dt):
     """Small integers, whose sums every order gives exactly (|sums| < 2^11 here, which float16 holds; bfloat16
     rounds them once)."""
-    print(f"past the cache groups={groups} K={K} {dt}", flush=True)
-    N, T = 7168, 330
+    print(f"past the cache groups={groups} N={N} K={K} {dt}", flush=True)
+    T = 330
     a = HIPAllToAll(MoEConfig(groups, 1, K, T, dt, dt), 0, 1, device=torch.device(DEV))
     g = torch.Generator(device=DEV).manual_seed(K)
     x = torch.randint(-1, 2, (groups, T, K), generator=g, device=DEV).to(dt)
     w = torch.randint(-1, 2, (groups, N, K), generator=g, device=DEV).to(dt)
     b = torch.randint(-9, 10, (groups, N), generator=g, device=DEV).to(dt)
-    counts = [257, 0, 33, 321, 1][:groups]
+    counts = ([257, 0, 33, 321, 1] + [0, 64, 2, 31] * 15)[:groups]
     num = torch.tensor(counts, dtype=torch.int32, device=DEV)
     want = [((x[e, :c].double() @ w[e].double().T).to(dt).double() + b[e].double()).to(dt) for e, c in enumerate(counts)]
-    for rows in PAST_THE_CACHE[groups, K]:
+    for rows in PAST_THE_CACHE[groups, N, K]:
         out = a.expert_gemm(x, num, w, b, rows_hint=rows * groups, out=torch.full((groups, T, N), 7.0, dtype=dt, device=DEV))
         for e, c in enumerate(counts):
             assert torch.equal(out[e, :c], want[e]), (rows, e)

@@ -8,8 +8,8 @@ from amd_distributed_2025_amd import HIPAllToAll, MoEConfig, gemm_rs
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 # tile (RingTile) -> groups, out_dim, rows per group that the caller promises (test_tile_rules.py holds the rule to that)
-RING_TILES = {1: (3, 96, 8), 2: (5, 3872, 9), 3: (3, 160, 70), 4: (6, 2080, 80)}
-RING_STEPS = [8, 64, 136, 256, 320, 328, 384, 448, 512, 520, 1000, 2048]  # from 24 steps on the streaming kernel has some fewer
+RING_TILES = {1: (3, 96, 8), 2: (5, 2080, 9), 3: (3, 160, 70), 4: (6, 2080, 80)}
+RING_STEPS = [8, 64, 136, 256, 320, 328, 384, 448, 512, 520, 1000, 2048]
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
