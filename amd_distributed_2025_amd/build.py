@@ -23,7 +23,7 @@ PKG_DIR = Path(__file__).resolve().parent
 REPO_DIR = PKG_DIR.parent
 SOURCE = PKG_DIR / "csrc" / "moe_a2a.hip"
 ABI_HEADER = REPO_DIR / "include" / "moe_a2a.h"
-HEADERS = [PKG_DIR / "csrc" / "tile_rules.h", ABI_HEADER]
+HEADERS = [PKG_DIR / "csrc" / "stream_rules.h", PKG_DIR / "csrc" / "tile_rules.h", ABI_HEADER]
 LIBRARY = PKG_DIR / "libmoe_a2a.so"
 EXT_SOURCE = PKG_DIR / "csrc" / "moe_a2a_torch.cpp"
 CALLS_SOURCE = PKG_DIR / "csrc" / "host_calls.cpp"

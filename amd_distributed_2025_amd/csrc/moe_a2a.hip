@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "moe_a2a.h"
+#include "stream_rules.h"
 #include "tile_rules.h"
 
 // Device memory of moe_a2a_dispatch_recv_static: the send-back plan of one call, held by the
@@ -42,12 +43,7 @@ static __device__ __align__(256) int32_t scratch[2 * MOE_A2A_STATIC_PLAN_EXPERTS
 namespace {
 
 constexpr int META = MOE_A2A_META_DIM;
-constexpr int BLOCK = 256;            // lanes of the block-per-row kernels and counting workgroups
 constexpr int NWAVES = BLOCK / 64;
-#ifndef MOE_A2A_ROWS
-#define MOE_A2A_ROWS 4
-#endif
-constexpr int ROWS = MOE_A2A_ROWS;    // rows (= waves) per workgroup of a ranked row move
 constexpr int COMBINE_CAP = 64;       // addends per token handled by the fast path
 constexpr int COMBINE_WEIGHTS = 128;  // weights of one token staged in LDS
 constexpr int COMBINE_BATCH = 8;      // addend rows loaded before accumulating
@@ -775,13 +771,8 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
 // nothing in the scan is skipped by a branch (with up to 16 keys per lane skipped in this way 3.23 us instead of 2.57 for
 // the 32 entries of 12 KB below, 2.83 with up to 8). us, one launch after another in a graph, before / here: 72 entries
 // of 1 KB, 6 per token 4.38 / 2.77, 32 of 12 KB, 2 per token 3.92 / 2.57, 500 of 5.8 KB, 4 per token 3.85 / 3.30, 720 of
-// 2 KB, 8 per token 5.27 / 3.61, 800 of 14 KB, 8 per token 6.17 / 4.66. Beyond 1024 entries the keys of all waves go through
-// the unit's one path to L1 too often; and tokens with fewer than four entries and much to move are better off with a wave
-// per entry (900 of 14 KB, 2 per token 5.26 / 5.70).
-constexpr int FEW_ENTRIES = 64 * 16;
-constexpr int FEW_MAX_K = 64;            // a lane of the wave for each
-constexpr long long FEW_BYTES = 8 << 20; // (of tokens with fewer than MOE_A2A_FANOUT_MIN_K entries)
-
+// 2 KB, 8 per token 5.27 / 3.61, 800 of 14 KB, 8 per token 6.17 / 4.66. With more keys, or more pieces of rows that each hold
+// them, they go through the unit's one path to L1 too often (send_way).
 template <typename V, int KEYS, bool POW2>
 __global__ __launch_bounds__(BLOCK) void dispatch_few_kernel(
     const V* __restrict__ x, const int* __restrict__ indices, int T, int K, int W, int chunks, int row_vecs, int E,
@@ -856,9 +847,6 @@ __global__ __launch_bounds__(BLOCK) void dispatch_few_kernel(
 // 2787 tokens of 4 KB, 4 per token 33.4 / 14.6 (the rows alone 10.4 at 5.3 TB/s), 4096 of 14 KB, 8 per token 118.9 / 102.5
 // (99.7), 4096 of 512 bytes, 8 per token 109 / 23.6, 1500 of 1 KB, 6 per token 17.6 / 7.3, 700 of 3.4 KB, 5 per token 8.1 / 5.6,
 // 3626 of 8150 bytes, moved by elements, 3 per token 109 / 37.
-constexpr int BLOCK_RANKS = 8;
-constexpr int BLOCK_MAX_ENTRIES = 255 * BLOCK;  // keys that 256 lanes count in bytes
-
 template <typename V, int NVW, bool POW2>
 __global__ __launch_bounds__(64 * ROWS) void dispatch_block_kernel(
     const V* __restrict__ x, const int* __restrict__ indices, int T, int K, int W, int chunks, int row_vecs, int E,
@@ -4402,8 +4390,6 @@ int mover_blocks(long long items) {
   return (int)(g < 1 ? 1 : g);
 }
 
-bool items_fit(long long rows, int chunks) { return rows * chunks <= INT_MAX / 2; }
-
 int launch_status() { return hipGetLastError() == hipSuccess ? MOE_A2A_OK : MOE_A2A_ELAUNCH; }
 
 // Picks the <vector type, vectors per lane> instantiation for a geometry.
@@ -4512,23 +4498,15 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
   const Geometry g = geometry(s, x, send_buf);
   if (!items_fit(S, g.wchunks)) return MOE_A2A_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  // Tokens with several entries: one workgroup per (token, 256-vector chunk) stores the chunk to
-  // all of the token's slots (measured at K = 8, H = 7168: 8.4 us against 8.8 us with a wave per
-  // entry; one chunk per workgroup beats two or four). With one or two entries per token the
-  // wave-per-entry kernel scans fewer keys per byte moved.
-#ifndef MOE_A2A_FANOUT_MIN_K
-#define MOE_A2A_FANOUT_MIN_K 4
-#endif
   Geometry f = g;
   f.nv = 1;
   f.chunks = (f.row_vecs + BLOCK - 1) / BLOCK;
-  // (a job without tokens goes to the kernels below, which then read nothing)
-  if (S > 0 && S <= FEW_ENTRIES && s->experts_per_token <= FEW_MAX_K && (long long)num_tokens * f.chunks <= 1 << 20 &&
-      (s->experts_per_token >= MOE_A2A_FANOUT_MIN_K || S * s->hidden_dim * 2 <= FEW_BYTES)) {
+  const SendWay way = send_way(num_tokens, s->experts_per_token, s->world_size, g.row_vecs, g.vec16);
+  if (way == SEND_FEW) {
     int order_bits = 1, nle_shift = 0;
     while ((1 << order_bits) < S) ++order_bits;
     while ((1 << nle_shift) < g.nle) ++nle_shift;
-    const int few_grid = s->world_size + num_tokens * f.chunks;
+    const int few_grid = s->world_size + num_tokens * f.chunks, keys = few_keys(S);
 #define LAUNCH_K(V, KEYS, POW2)                                                                  \
   dispatch_few_kernel<V, KEYS, POW2><<<few_grid, BLOCK, 0, st>>>(                                \
       (const V*)x, indices, num_tokens, s->experts_per_token, s->world_size, f.chunks,           \
@@ -4536,10 +4514,10 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
       (V*)send_buf, send_meta, send_counts, send_slot)
 #define LAUNCH(V, POW2)                                  \
   do {                                                   \
-    if (S <= 64 * 2) LAUNCH_K(V, 2, POW2);               \
-    else if (S <= 64 * 4) LAUNCH_K(V, 4, POW2);          \
-    else if (S <= 64 * 8) LAUNCH_K(V, 8, POW2);          \
-    else if (S <= 64 * 12) LAUNCH_K(V, 12, POW2);        \
+    if (keys == 2) LAUNCH_K(V, 2, POW2);                 \
+    else if (keys == 4) LAUNCH_K(V, 4, POW2);            \
+    else if (keys == 8) LAUNCH_K(V, 8, POW2);            \
+    else if (keys == 12) LAUNCH_K(V, 12, POW2);          \
     else LAUNCH_K(V, 16, POW2);                          \
   } while (0)
     if ((g.nle & (g.nle - 1)) == 0) { if (f.vec16) LAUNCH(b128, true); else LAUNCH(uint16_t, true); }
@@ -4548,29 +4526,14 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
 #undef LAUNCH_K
     return launch_status();
   }
-  // Longer streams go to the kernel that ranks four tokens in one pass over the keys, but for two kinds of short ones, where
-  // a pass is little beside the rows and the kernels below store them faster: fewer than four entries per token up to
-  // 1280 of them (600 tokens of 14 KB, 2 per token 6.2 / 6.4 us), and long rows as long as a pass over the keys is short
-  // beside the rows of a token, which the tokens and the vectors of a row measure: before / here 8 per token of 14 KB, 1024
-  // tokens 26.2 / 27.8, 1400 34.3 / 36.9, 1800 43.7 / 48.9, 4096 118.9 / 102.5; 4 of 10 KB, 1000 tokens 10.7 / 11.1, 1500
-  // 16.2 / 16.3; 6 of 13.7 KB, 600 tokens 12.0 / 13.0; but 3 of 9.2 KB, 500 tokens 5.6 / 5.4, and rows moved by elements 18.1 /
-  // 10.2 (6 of 4111, 500 tokens).
-  const bool few_entries = s->experts_per_token < MOE_A2A_FANOUT_MIN_K && S <= 1280;
-  const bool long_rows = s->experts_per_token >= MOE_A2A_FANOUT_MIN_K && f.vec16 && f.row_vecs > 2 * BLOCK &&
-                         num_tokens <= 3 * f.row_vecs;
-  if (S > 0 && S <= BLOCK_MAX_ENTRIES && s->world_size <= BLOCK_RANKS && s->experts_per_token * ROWS <= 64 && !few_entries &&
-      !long_rows) {
+  if (way == SEND_BLOCK) {
     Geometry b = g;
-    const int groups = (num_tokens + ROWS - 1) / ROWS;
-    // Rows are cut into pieces of two vectors per lane where there are few workgroups otherwise, else of four: pieces of 2 / 4 /
-    // whole rows: 250 tokens of 5.8 KB, 8 per token 4.8 / 5.1 / 5.5 us, 1440 of 7.4 KB, 4 per token 11.6 / 12.3 / 12.1, 4096 of
-    // 14 KB, 8 per token 129 / 102 / 106. With one entry a piece would do little but rank: 2000 of 14 KB 13.4 / 10.7 / 9.6.
-    if (b.vec16 && s->experts_per_token > 1) b.nvw = std::min(b.nvw, groups <= 400 ? 2 : 4);
+    b.nvw = block_piece(num_tokens, s->experts_per_token, b.nvw, b.vec16);
     b.wchunks = (b.row_vecs + 64 * b.nvw - 1) / (64 * b.nvw);
     int nle_shift = 0;
     while ((1 << nle_shift) < g.nle) ++nle_shift;
     const bool pow2 = (g.nle & (g.nle - 1)) == 0;
-    const int block_grid = groups * b.wchunks;
+    const int block_grid = (num_tokens + ROWS - 1) / ROWS * b.wchunks;
 #define LAUNCH_B(V, NVW, POW2)                                                                \
   dispatch_block_kernel<V, NVW, POW2><<<block_grid, 64 * ROWS, 0, st>>>(                      \
       (const V*)x, indices, num_tokens, s->experts_per_token, s->world_size, b.wchunks,       \
@@ -4586,14 +4549,10 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
 #undef LAUNCH_B
     return launch_status();
   }
-  if (s->experts_per_token >= MOE_A2A_FANOUT_MIN_K && (s->world_size + 2ll) * S <= INT_MAX &&
-      items_fit(num_tokens, f.chunks)) {
+  if (way == SEND_FANOUT || way == SEND_FANOUT_WIDE) {
     const int fan = fan_of(S);
-#ifndef MOE_A2A_FANOUT_WIDE
-#define MOE_A2A_FANOUT_WIDE 1
-#endif
-    constexpr int WIDE = 2 * BLOCK;  // rows of more than one 256-lane chunk: 512-lane workgroups
-    if (MOE_A2A_FANOUT_WIDE && f.row_vecs > BLOCK && S < 65536 && s->world_size < 16384) {
+    constexpr int WIDE = 2 * BLOCK;  // 512-lane workgroups
+    if (way == SEND_FANOUT_WIDE) {
       // Rows of more than 512 vectors: two vectors per lane, so that a row of up to 1024 vectors
       // is one workgroup's and its entries are ranked once, not once per chunk (measured at
       // H = 7168: the whole step 0.4 us shorter; 256 lanes x 4 and 1024 lanes x 1 were slower).

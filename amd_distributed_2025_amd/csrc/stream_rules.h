@@ -1,0 +1,89 @@
+// Which kernels the stages of a job run on: plain arithmetic on its sizes, so that a host compiler can take it as well.
+#pragma once
+
+#include <limits.h>
+
+#include <algorithm>
+
+namespace {
+
+constexpr int BLOCK = 256;            // lanes of the block-per-row kernels and counting workgroups
+#ifndef MOE_A2A_ROWS
+#define MOE_A2A_ROWS 4
+#endif
+constexpr int ROWS = MOE_A2A_ROWS;    // rows (= waves) per workgroup of a ranked row move
+
+bool items_fit(long long rows, int chunks) { return rows * chunks <= INT_MAX / 2; }
+
+// ---------------------------------------------------------------- stage 1
+
+constexpr int FANOUT_MIN_K = 4;
+constexpr int FEW_ENTRIES = 64 * 16;
+constexpr int FEW_MAX_K = 64;            // a lane of the wave for each
+constexpr int BLOCK_RANKS = 8;
+constexpr int BLOCK_MAX_ENTRIES = 255 * BLOCK;  // keys that 256 lanes count in bytes
+
+enum SendWay {
+  SEND_BY_ENTRY,     // dispatch_send_kernel
+  SEND_FEW,          // dispatch_few_kernel
+  SEND_BLOCK,        // dispatch_block_kernel
+  SEND_FANOUT,       // dispatch_fanout_kernel
+  SEND_FANOUT_WIDE   // dispatch_fanout_wide_kernel: rows of more than one 256-lane chunk
+};
+
+// Keys per lane of a wave that holds all of a stream: the smallest of the numbers that there are kernels for.
+int few_keys(long long entries) {
+  for (const int keys : {2, 4, 8, 12})
+    if (entries <= 64 * keys) return keys;
+  return 16;
+}
+
+// `row_vecs`: vectors of 16 bytes in a row, or its elements where those cannot be used (vec16).
+//
+// Up to 1024 entries every wave holds all keys. That costs each workgroup, which moves a piece of 256 vectors, as many loads and
+// compares as there are keys per lane, and pays up to about 16000 of them over all pieces, 12000 where a vector is one
+// element. Beyond (many tokens with long rows and few entries) a wave per entry is ahead; only tokens with four and more
+// entries of whole vectors then have as much to store per piece. us, held by every wave / a wave per entry: 1 per token, 500 of
+// 14 KB (16000) 4.4 / 4.6, 728 of 4.6 KB (17472) 4.5 / 4.0, 918 of 13 KB (58752) 8.1 / 5.9; of single elements 60 tokens of 7167,
+// 2 each (3360) 3.6 / 4.1, 179 of 1971, 2 each (11456) 4.1 / 4.2, 126 of 6277, 2 each (12600) 5.0 / 4.6, 500 of 7167 (112000) 14.1 /
+// 5.4, 200 of 4097, 4 each (54400) 8.8 / 6.3.
+//
+// Longer streams go to the kernel that ranks four tokens in one pass over the keys, but for two kinds of short ones, where
+// a pass is little beside the rows and the others store them faster: fewer than four entries per token up to
+// 1280 of them (600 tokens of 14 KB, 2 per token 6.2 / 6.4 us), and long rows as long as a pass over the keys is short
+// beside the rows of a token, which the tokens and the vectors of a row measure: the others / that kernel 8 per token of 14 KB, 1024
+// tokens 26.2 / 27.8, 1400 34.3 / 36.9, 1800 43.7 / 48.9, 4096 118.9 / 102.5; 4 of 10 KB, 1000 tokens 10.7 / 11.1, 1500
+// 16.2 / 16.3; 6 of 13.7 KB, 600 tokens 12.0 / 13.0; but 3 of 9.2 KB, 500 tokens 5.6 / 5.4, and rows moved by elements 18.1 /
+// 10.2 (6 of 4111, 500 tokens).
+//
+// The others: tokens with several entries have one workgroup per (token, 256-vector chunk) that stores the chunk to
+// all of the token's slots (measured at K = 8, H = 7168: 8.4 us against 8.8 us with a wave per
+// entry; one chunk per workgroup beats two or four). With one or two entries per token the
+// wave-per-entry kernel scans fewer keys per byte moved.
+SendWay send_way(long long tokens, int per_token, int ranks, int row_vecs, bool vec16) {
+  const long long entries = tokens * per_token;
+  const int pieces = (row_vecs + BLOCK - 1) / BLOCK;
+  // (a job without tokens goes to the kernels below, which then read nothing)
+  if (entries > 0 && entries <= FEW_ENTRIES && per_token <= FEW_MAX_K && tokens * pieces <= 1 << 20) {
+    if (vec16 && per_token >= FANOUT_MIN_K) return SEND_FEW;
+    return tokens * pieces * few_keys(entries) <= (vec16 ? 16000 : 12000) ? SEND_FEW : SEND_BY_ENTRY;
+  }
+  const bool few_entries = per_token < FANOUT_MIN_K && entries <= 1280;
+  const bool long_rows = per_token >= FANOUT_MIN_K && vec16 && row_vecs > 2 * BLOCK && tokens <= 3ll * row_vecs;
+  if (entries > 0 && entries <= BLOCK_MAX_ENTRIES && ranks <= BLOCK_RANKS && per_token * ROWS <= 64 && !few_entries && !long_rows)
+    return SEND_BLOCK;
+  if (per_token >= FANOUT_MIN_K && (ranks + 2ll) * entries <= INT_MAX && items_fit(tokens, pieces))
+    return row_vecs > BLOCK && entries < 65536 && ranks < 16384 ? SEND_FANOUT_WIDE : SEND_FANOUT;
+  return SEND_BY_ENTRY;
+}
+
+// Vectors per lane of a wave of dispatch_block_kernel, for rows that a wave has in one go with `nvw`. Rows
+// are cut into pieces of two vectors per lane where there are few workgroups otherwise, else of four: pieces of 2 / 4 /
+// whole rows: 250 tokens of 5.8 KB, 8 per token 4.8 / 5.1 / 5.5 us, 1440 of 7.4 KB, 4 per token 11.6 / 12.3 / 12.1, 4096 of
+// 14 KB, 8 per token 129 / 102 / 106. With one entry a piece would do little but rank: 2000 of 14 KB 13.4 / 10.7 / 9.6.
+int block_piece(long long tokens, int per_token, int nvw, bool vec16) {
+  if (!vec16 || per_token == 1) return nvw;
+  return std::min(nvw, (tokens + ROWS - 1) / ROWS <= 400 ? 2 : 4);
+}
+
+}  // namespace

@@ -1,5 +1,5 @@
-"""Stage 1 of long streams (`dispatch_block_kernel`: four tokens per workgroup, keys counted by destination in bytes) against a
-stable sort, at the numbers of tokens, entries and ranks where it begins and ends."""
+"""Stage 1 against a stable sort: `dispatch_block_kernel` (four tokens per workgroup, keys counted by destination in bytes) on every
+cut of a row, and the numbers of tokens, entries, ranks and row lengths where it and the kernels of short streams begin and end."""
 import numpy as np
 import pytest
 import torch
@@ -25,10 +25,24 @@ def check(W, E, K, H, T, indices):
     assert torch.equal(buf[:T * K].cpu().view(torch.int16), x.view(torch.int16)[torch.from_numpy(token)])
 
 
-@pytest.mark.parametrize("W,E,K,H,T", [
-    (8, 16, 1, 8, 1281), (1, 3, 3, 24, 427), (8, 64, 4, 64, 257), (3, 15, 5, 1032, 410), (2, 6, 16, 37, 66), (8, 256, 8, 520, 1023),
-    (7, 21, 6, 4104, 345), (8, 88, 2, 2048, 1601), (5, 10, 7, 7168, 1799), (8, 8, 8, 16, 4096), (4, 32, 4, 8, 16320), (4, 32, 4, 8, 16321),
-    (9, 18, 4, 8, 400), (8, 32, 17, 8, 70)])  # (the last three are other kernels')
+# ranks, experts, entries per token, hidden, tokens -> the kernel, and for dispatch_block_kernel vectors per lane and pieces of a
+# row (csrc/stream_rules.h; test_stream_rules.py holds the cases to that)
+CASES = {
+    (8, 16, 1, 8, 1281): ("block", 1, 1), (1, 3, 3, 24, 427): ("block", 1, 1), (8, 64, 4, 64, 257): ("block", 1, 1),
+    (2, 2, 1, 1000, 1282): ("block", 2, 1), (8, 256, 8, 520, 1023): ("block", 2, 1), (3, 15, 5, 1032, 410): ("block", 2, 2),
+    (5, 10, 3, 4104, 700): ("block", 2, 5), (4, 4, 1, 1032, 1290): ("block", 4, 1), (8, 88, 2, 2048, 1601): ("block", 4, 1),
+    (4, 8, 4, 4104, 1601): ("block", 4, 3), (8, 16, 2, 7168, 1605): ("block", 4, 4), (2, 4, 1, 2056, 1300): ("block", 6, 1),
+    (8, 8, 1, 4096, 1300): ("block", 8, 1), (3, 3, 1, 6144, 1285): ("block", 12, 1), (2, 4, 1, 7168, 1301): ("block", 14, 1),
+    (2, 2, 1, 8192, 1283): ("block", 16, 1), (2, 2, 1, 8200, 1282): ("block", 16, 2),
+    (2, 6, 16, 37, 66): ("block", 16, 1), (4, 8, 5, 2051, 300): ("block", 16, 3), (2, 4, 1, 3001, 1290): ("block", 16, 3),  # single elements
+    (8, 8, 8, 16, 4096): ("block", 1, 1), (4, 32, 4, 8, 16320): ("block", 1, 1),
+    (4, 32, 4, 8, 16321): "fanout", (9, 18, 4, 8, 400): "fanout", (8, 32, 17, 8, 70): "fanout",
+    (7, 21, 6, 4104, 345): "wide fanout", (5, 10, 7, 7168, 1799): "wide fanout", (9, 18, 2, 24, 700): "by entry",
+    (4, 8, 1, 7167, 100): "few", (4, 8, 1, 7167, 300): "by entry", (8, 16, 4, 4097, 60): "few", (8, 16, 4, 4097, 100): "by entry",
+    (16, 32, 8, 2049, 120): "by entry", (8, 64, 1, 7168, 500): "few", (2, 4, 1, 2304, 728): "by entry"}
+
+
+@pytest.mark.parametrize("W,E,K,H,T", CASES)
 @pytest.mark.parametrize("ids", ["any", "one", "stray"])
 def test_against_a_stable_sort(W, E, K, H, T, ids):
     print(f"block {W} {E} {K} {H} {T} {ids}", flush=True)

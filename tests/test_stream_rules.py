@@ -1,0 +1,84 @@
+"""The rules of csrc/stream_rules.h, built with the host's compiler: which kernels the stages of a job run on."""
+import ctypes as C
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from tests.test_gpu_block_streams import CASES
+
+CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
+SEND_WAYS = ["by entry", "few", "block", "fanout", "wide fanout"]  # SendWay
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not installed")
+    src = tmp_path_factory.mktemp("rules") / "rules.cpp"
+    src.write_text('#include "stream_rules.h"\n'
+                   'extern "C" int way(long long tokens, int k, int ranks, int row_vecs, int vec16) {\n'
+                   '  return send_way(tokens, k, ranks, row_vecs, vec16); }\n'
+                   'extern "C" int piece(long long tokens, int k, int nvw, int vec16) { return block_piece(tokens, k, nvw, vec16); }\n'
+                   'extern "C" int keys(long long entries) { return few_keys(entries); }\n')
+    lib = src.with_suffix(".so")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
+                    str(src), "-o", str(lib)], check=True)
+    dll = C.CDLL(str(lib))
+    dll.way.argtypes = [C.c_longlong] + [C.c_int] * 4
+    dll.piece.argtypes = [C.c_longlong] + [C.c_int] * 3
+    dll.keys.argtypes = [C.c_longlong]
+    return dll
+
+
+def row(hidden):
+    """Vectors of 16 bytes in a row, or its elements, and vectors per lane of a wave that moves it (row_geometry)."""
+    vec16 = hidden % 8 == 0
+    vecs = hidden // 8 if vec16 else hidden
+    nvw = next((n for n in (1, 2, 4, 6, 8, 12, 14) if vecs <= 64 * n), 16) if vec16 else 16
+    return vecs, vec16, nvw
+
+
+def way_of(rules, tokens, k, ranks, hidden):
+    vecs, vec16, nvw = row(hidden)
+    way = SEND_WAYS[rules.way(tokens, k, ranks, vecs, vec16)]
+    if way == "block":
+        nvw = rules.piece(tokens, k, nvw, vec16)
+        return way, nvw, -(-vecs // (64 * nvw))
+    return way
+
+
+@pytest.mark.parametrize("W,E,K,H,T", CASES)
+def test_kernels_of_stage_1_that_the_gpu_tests_mean(rules, W, E, K, H, T):
+    assert way_of(rules, T, K, W, H) == CASES[W, E, K, H, T]
+
+
+@pytest.mark.parametrize("tokens,k,hidden,way", [
+    (500, 1, 7167, "by entry"), (900, 1, 513, "by entry"), (500, 2, 1001, "by entry"), (300, 2, 4097, "by entry"),
+    (200, 4, 4097, "by entry"), (120, 8, 7167, "by entry"), (435, 1, 1235, "by entry"), (858, 1, 4491, "by entry"),
+    (728, 1, 2304, "by entry"), (918, 1, 6720, "by entry"), (100, 1, 7167, "few"), (60, 2, 7167, "few"), (100, 3, 1001, "few"),
+    (30, 8, 7167, "few"), (80, 6, 1561, "few"), (1000, 1, 2048, "few"), (250, 2, 7168, "few"), (120, 8, 7168, "few"), (16, 2, 6144, "few"),
+])
+def test_way_of_short_streams_that_was_faster(rules, tokens, k, hidden, way):
+    """Timed on the GPU: many pieces of rows that each rank all keys take up to 3.6 times as long as a wave per entry."""
+    assert way_of(rules, tokens, k, 8, hidden) == way
+
+
+def test_limits_of_the_kernels_of_stage_1(rules):
+    """(each of them addresses what its way promises: a key per lane and slot, bytes of counts, 32-bit order keys)"""
+    for tokens in (1, 2, 3, 63, 64, 65, 1023, 1024, 1025, 4095, 16320, 16321, 65280, 65281, 1 << 20):
+        for k in (1, 2, 3, 4, 8, 15, 16, 17, 63, 64, 65):
+            for ranks in (1, 8, 9, 64, 65536):
+                for vecs, vec16 in ((1, 1), (256, 1), (513, 1), (896, 1), (1 << 22, 1), (37, 0), (7167, 0), (1 << 25, 0)):
+                    way, entries = SEND_WAYS[rules.way(tokens, k, ranks, vecs, vec16)], tokens * k
+                    pieces = -(-vecs // 256)
+                    if way == "few":
+                        assert entries <= 64 * rules.keys(entries) <= 1024 and k <= 64 and tokens * pieces <= 1 << 20
+                    if way == "block":
+                        assert entries <= 65280 and ranks <= 8 and 4 * k <= 64
+                    if way == "fanout":
+                        assert (ranks + 2) * entries < 2 ** 31 and tokens * pieces < 2 ** 30
+                    if way == "wide fanout":
+                        assert (ranks + 1) << max(1, (entries - 1).bit_length()) < 2 ** 31 and tokens * pieces < 2 ** 30
+    assert rules.way(0, 2, 8, 896, 1) == 0 and SEND_WAYS[rules.way(0, 8, 8, 896, 1)] == "wide fanout"  # (which read nothing then)
