@@ -77,8 +77,7 @@ typedef unsigned int b128 __attribute__((ext_vector_type(4)));
 //  - exchange: 8 MB of rows for a rank (0.03 MB of 512 B 2.25 / 2.41, 3.9 MB 6.30 / 7.31; 8 MB of 2 KB 5.01 / 5.27, 16 MB 8.46
 //    / 7.80; 3.9 MB of 8 KB 3.18 / 3.31, 6.2 MB 3.67 / 3.61).
 enum Store { PLAIN, THROUGH, STREAM };
-constexpr int STAGE2_THROUGH_ROWS = 1024;
-constexpr long long STAGE2_THROUGH_BYTES = 8 << 20, JOB_THROUGH_BYTES = 1 << 20, EXCHANGE_THROUGH_BYTES = 8 << 20;
+constexpr long long JOB_THROUGH_BYTES = 1 << 20, EXCHANGE_THROUGH_BYTES = 8 << 20;  // (stage 2's: recv_through)
 // (a kernel for each kind: chosen inside one, the stores of 5.5 MB of rows took 0.3 us longer than either)
 template <typename V> constexpr Store THROUGH_OF = sizeof(V) == sizeof(b128) ? THROUGH : PLAIN;  // (of 16 bytes only)
 #ifndef MOE_A2A_STORE_SEND   /* stage 1 -> send buffer */
@@ -347,8 +346,10 @@ struct WavePayload {
 // issue order, so the keys arrive first and the slot is ready while the payload
 // is still in flight):  RowsScan scan(n, keys);  ...issue payload...;
 // scan.finish(keys, test, cnt);
-// SHORT: scans that mostly end inside a batch leave it there (the branches cost 0.5 us where batches are full: 20.2 against
-// 19.2 for the 4800 rows of a skewed job in the compact layout).
+// SHORT: scans that mostly end inside a batch leave it there. That pays while a unit has another workgroup to go on with (stage 2
+// with / without, 1422 rows of 14 KB 8.15 / 8.41 us, of 8 KB 6.05 / 6.25); with one workgroup on a unit the waits at the branches
+// cost more (900 rows of 14 KB 6.35 / 5.42), and so they do where batches are full (the 4800 rows of a skewed job in the
+// compact layout 20.2 / 19.2).
 template <typename Keys, bool SHORT = false, int UNROLL = SCAN_UNROLL>
 struct RowsScan {
   static constexpr int STEP = 64 * ROWS;
@@ -1243,7 +1244,7 @@ __device__ __forceinline__ void plan_expert(
   }
 }
 
-template <typename V, int NVW, bool PLAN, int MODE, Store HOW>
+template <typename V, int NVW, bool PLAN, int MODE, Store HOW, bool SHORT>
 __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
     const V* __restrict__ recv_buf, const int* __restrict__ recv_meta,
     const int* __restrict__ recv_counts, int W, int hint_rows, int movers, int chunks, int row_vecs, int nle,
@@ -1251,7 +1252,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
     V* __restrict__ expert_x, int* __restrict__ expert_meta, int* __restrict__ plan,
     const int* __restrict__ row_pos, int* __restrict__ expert_offsets) {
   constexpr bool POS = MODE == RECV_POS, COMPACT = MODE == RECV_COMPACT;
-  constexpr int UNROLL = HOW == PLAIN ? 4 : SCAN_UNROLL;  // (PLAIN: at most 1024 rows, mostly)
+  constexpr int UNROLL = HOW == PLAIN ? 4 : SCAN_UNROLL;  // (PLAIN: up to 1024 rows of elements, or of more than 64 experts)
   __shared__ int part[2 * ROWS * ROWS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const StridedKeys key{recv_meta, META};
@@ -1313,7 +1314,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
     if (c == 0 && lane < META) m = recv_meta[(size_t)ic * META + lane];
     // only rows before the group's last row can precede any of its rows in its expert; the rows of
     // lower experts, which the compact layout puts ahead of it, lie anywhere in the stream
-    RowsScan<StridedKeys, !COMPACT, UNROLL> scan(COMPACT ? limit : min(i0 + ROWS - 1, limit), key);
+    RowsScan<StridedKeys, SHORT, UNROLL> scan(COMPACT ? limit : min(i0 + ROWS - 1, limit), key);
     WavePayload<V, NVW> p;
     p.load(recv_buf + (size_t)ic * row_vecs, base, row_vecs, lane);
 
@@ -1375,7 +1376,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
 // hold hint_rows), with nothing to wait for but its own loads. As in dispatch_few_kernel the code that a wave runs through is
 // what counts. us, one launch after another in a graph, before / here: 72 rows of 1 KB 3.33 / 2.54, 32 of 12 KB 3.87 / 3.09,
 // 500 of 5.8 KB 4.11 / 3.44, 600 of 8 KB 4.45 / 4.11, 800 of 14 KB 6.17 / 5.75.
-template <typename V, int NVW, int KEYS, bool COMPACT>
+template <typename V, int NVW, int KEYS, bool COMPACT, Store HOW>
 __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_few_kernel(
     const V* __restrict__ recv_buf, const int* __restrict__ recv_meta,
     const int* __restrict__ recv_counts, int W, int hint_rows, int movers, int chunks, int row_vecs, int nle,
@@ -1433,7 +1434,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_few_kernel(
     }
     if (pos < max_recv) {
       const size_t row = COMPACT ? (size_t)pos : (size_t)le * max_recv + pos;
-      p.template store<PLAIN>(expert_x + row * row_vecs, base, row_vecs, lane);
+      p.template store<HOW>(expert_x + row * row_vecs, base, row_vecs, lane);
       if (c == 0 && lane < META) expert_meta[row * META + lane] = m;
     }
   }
@@ -4667,7 +4668,7 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
                                                     capacity_rows, g.nle, g.magic, expert_bits, row_position);
     const int grid = g.nle + mover_blocks(group_items(rows_hint, g));
 #define LAUNCH_P(V, NVW, PLAN)                                                              \
-  dispatch_recv_kernel<V, NVW, PLAN, RECV_POS, THROUGH><<<grid, 64 * ROWS, 0, st>>>(        \
+  dispatch_recv_kernel<V, NVW, PLAN, RECV_POS, THROUGH, false><<<grid, 64 * ROWS, 0, st>>>( \
       (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, grid - g.nle,    \
       g.wchunks, g.row_vecs, g.nle, capacity_rows, g.magic, g.max_recv, expert_num_tokens,   \
       (V*)expert_x, expert_meta, send_back_plan, row_position, nullptr)
@@ -4686,14 +4687,22 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   }
   // the stream can hold at most nle * max_recv rows that fit the expert buffers
   if (!items_fit((long long)g.nle * g.max_recv, g.wchunks)) return MOE_A2A_EINVAL;
-  if (planned && rows_hint > 0 && rows_hint <= FEW_ENTRIES) {  // (planned: at most 64 ranks)
+  const RecvFew few = planned ? recv_few(rows_hint, g.row_vecs, g.nvw, g.vec16, compact_rows > 0) : RECV_NOT_FEW;
+  if (few != RECV_NOT_FEW) {  // (planned: at most 64 ranks)
     const int few_grid = g.nle + mover_blocks(((long long)rows_hint * g.wchunks + ROWS - 1) / ROWS);
-#define LAUNCH_K(V, NVW, KEYS, COMPACT)                                                      \
-  dispatch_recv_few_kernel<V, NVW, KEYS, COMPACT><<<few_grid, 64 * ROWS, 0, st>>>(           \
+#define LAUNCH_H(V, NVW, KEYS, COMPACT, HOW)                                                 \
+  dispatch_recv_few_kernel<V, NVW, KEYS, COMPACT, HOW><<<few_grid, 64 * ROWS, 0, st>>>(      \
       (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint,                  \
       few_grid - g.nle, g.wchunks, g.row_vecs, g.nle, capacity_rows, g.magic,                \
       compact_rows > 0 ? compact_rows : g.max_recv, expert_num_tokens, (V*)expert_x,         \
       expert_meta, send_back_plan, expert_offsets)
+#define LAUNCH_K(V, NVW, KEYS, COMPACT)                                                         \
+  do {                                                                                          \
+    /* (a lane's vectors of a whole row of 8 MB in 1024: 6 and more) */                         \
+    constexpr Store LARGE = NVW == 8 || NVW == 12 || NVW == 16 ? THROUGH_OF<V> : PLAIN;         \
+    if (few == RECV_FEW_THROUGH) LAUNCH_H(V, NVW, KEYS, COMPACT, LARGE);                        \
+    else LAUNCH_H(V, NVW, KEYS, COMPACT, PLAIN);                                                \
+  } while (0)
 #define LAUNCH_C(V, NVW, COMPACT)                                       \
   do {                                                                  \
     if (rows_hint <= 64 * 4) LAUNCH_K(V, NVW, 4, COMPACT);              \
@@ -4710,21 +4719,26 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
 #undef LAUNCH
 #undef LAUNCH_C
 #undef LAUNCH_K
+#undef LAUNCH_H
     return launch_status();
   }
   const int grid = g.nle + mover_blocks(group_items(rows_hint, g));
-  const bool through =  // (Store)
-      rows_hint >= STAGE2_THROUGH_ROWS || (long long)rows_hint * s->hidden_dim * 2 >= STAGE2_THROUGH_BYTES;
-#define LAUNCH_S(V, NVW, PLAN, MODE, HOW)                                                   \
-  dispatch_recv_kernel<V, NVW, PLAN, MODE, HOW><<<grid, 64 * ROWS, 0, st>>>(                     \
+  const bool through = recv_through(rows_hint, 2ll * s->hidden_dim);  // (Store)
+#define LAUNCH_S(V, NVW, PLAN, MODE, HOW, SHORT)                                            \
+  dispatch_recv_kernel<V, NVW, PLAN, MODE, HOW, SHORT><<<grid, 64 * ROWS, 0, st>>>(         \
       (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, grid - g.nle,    \
       g.wchunks, g.row_vecs, g.nle, capacity_rows, g.magic,                                  \
       compact_rows > 0 ? compact_rows : g.max_recv,                                          \
       expert_num_tokens, (V*)expert_x, expert_meta, send_back_plan, nullptr, expert_offsets)
-#define LAUNCH_P(V, NVW, PLAN, MODE)                        \
-  do {                                                      \
-    if (through) LAUNCH_S(V, NVW, PLAN, MODE, THROUGH);     \
-    else LAUNCH_S(V, NVW, PLAN, MODE, PLAIN);               \
+#define LAUNCH_P(V, NVW, PLAN, MODE)                                                        \
+  do {                                                                                      \
+    /* (planned rows of vectors that come here are more than 1024, or 8 MB of 14 per lane,  \
+       a workgroup per unit: recv_few) */                                                   \
+    constexpr bool VECTORS = PLAN && sizeof(V) == sizeof(b128), SHORT = MODE == RECV_SCAN;  \
+    constexpr bool SHORT_FEW = SHORT && !(VECTORS && NVW == 14);                            \
+    if (!through) LAUNCH_S(V, NVW, PLAN, MODE, (VECTORS ? THROUGH : PLAIN), SHORT);         \
+    else if (rows_hint > FEW_ENTRIES) LAUNCH_S(V, NVW, PLAN, MODE, THROUGH, SHORT);         \
+    else LAUNCH_S(V, NVW, PLAN, MODE, THROUGH, SHORT_FEW);                                  \
   } while (0)
 #define LAUNCH(V, NVW)                                         \
   do {                                                         \

@@ -86,4 +86,34 @@ int block_piece(long long tokens, int per_token, int nvw, bool vec16) {
   return std::min(nvw, (tokens + ROWS - 1) / ROWS <= 400 ? 2 : 4);
 }
 
+// ---------------------------------------------------------------- stage 2
+
+constexpr int STAGE2_THROUGH_ROWS = 1024;
+constexpr long long STAGE2_THROUGH_BYTES = 8 << 20;
+
+bool recv_through(long long rows_hint, long long row_bytes) {
+  return rows_hint >= STAGE2_THROUGH_ROWS || rows_hint * row_bytes >= STAGE2_THROUGH_BYTES;
+}
+
+enum RecvFew { RECV_NOT_FEW, RECV_FEW_PLAIN, RECV_FEW_THROUGH };
+
+// Whether a planned stage 2 runs on dispatch_recv_few_kernel, where every wave holds all keys, and how that stores its rows
+// (Store). `nvw`: vectors per lane of the wave that moves a row, or a piece of one.
+//
+// Up to 1024 rows, but for two kinds. Elements: each of a row's pieces of 1024 ranks the row again, which costs more than
+// the other kernel's shared scan above 512 rows (padded; in the compact layout the scan is as long). us, held by every wave / scan: 900
+// rows of 5001 elements 8.3 / 6.6, 1000 of 2049 5.8 / 5.0, 700 of 7167 7.4 / 6.6; 512 of 2049 4.2 / 4.2, 256 4.1 / 4.4.
+// And 8 MB of rows of 13 or 14 vectors per lane: those and the keys leave room for fewer waves. us, held and plain / held and
+// past L2 / scan and past L2, 14 KB: 600 rows 5.15 / 4.93 / 4.78, 800 6.06 / 5.51 / 5.18, 900 6.44 / 5.94 / 5.42, 1024
+// 6.94 / 6.71 / 5.86; compact 900 6.62 / 6.03 / 5.93. Rows of other lengths stay, from 8 MB on past L2 as there: 900 of 10 KB 5.27 /
+// 4.77 / 5.31, 800 of 12 KB 5.49 / 5.20 / 5.59, 600 of 16 KB 5.67 / 5.43 / 6.20; longer ones, of several pieces, with plain
+// stores (800 of 28 KB 9.10 / 9.65 / 9.11, 500 of 56 KB 9.98 / 10.92 / 10.80).
+RecvFew recv_few(long long rows_hint, int row_vecs, int nvw, bool vec16, bool compact) {
+  if (rows_hint > FEW_ENTRIES) return RECV_NOT_FEW;
+  const bool pieces = row_vecs > 64 * nvw;
+  if (!vec16) return pieces && !compact && rows_hint > 512 ? RECV_NOT_FEW : RECV_FEW_PLAIN;
+  if (rows_hint * row_vecs * 16 < STAGE2_THROUGH_BYTES) return RECV_FEW_PLAIN;
+  return nvw == 14 ? RECV_NOT_FEW : pieces ? RECV_FEW_PLAIN : RECV_FEW_THROUGH;
+}
+
 }  // namespace

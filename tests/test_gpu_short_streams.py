@@ -109,3 +109,42 @@ def test_jobs_whose_lanes_move_several_vectors(world_size, hidden):
     ys = custom_kernel_job([(cfg, d, r, world_size) for r, d in enumerate(data)])
     for r in range(world_size):
         assert torch.equal(ys[r], want[r]), f"rank {r}"
+
+
+# hidden, rows, promised rows, layout -> the kernel of stage 2 and how it stores (csrc/stream_rules.h; test_stream_rules.py
+# holds the cases to that)
+RECV_CASES = {
+    (512, 300, 300, "padded"): "few, plain", (512, 300, 0, "padded"): "few, plain", (512, 300, 0, "compact"): "few, plain",
+    (4096, 1023, 1023, "padded"): "few, plain", (4096, 1024, 1024, "padded"): "few, through", (5120, 820, 820, "compact"): "few, through",
+    (8192, 512, 512, "padded"): "few, through", (8192, 700, 600, "compact"): "few, through", (6144, 700, 700, "padded"): "few, through",
+    (7168, 580, 580, "padded"): "few, plain", (7168, 600, 600, "padded"): "scan, through", (7168, 1024, 1024, "compact"): "scan, through",
+    (7168, 700, 600, "padded"): "scan, through", (7168, 590, 800, "compact"): "scan, through", (8200, 600, 600, "padded"): "few, plain",
+    (72, 1025, 1025, "padded"): "scan, through", (2049, 512, 512, "padded"): "few, plain", (2049, 513, 513, "padded"): "scan, plain",
+    (2049, 513, 513, "compact"): "few, plain", (1001, 1024, 1024, "padded"): "few, plain", (3001, 900, 700, "padded"): "scan, plain"}
+
+
+@pytest.mark.parametrize("hidden,rows,hint,layout", RECV_CASES)
+def test_kernels_of_stage_2(hidden, rows, hint, layout):
+    """Placement, counts and meta rows, and with them the order of the way back, which stage 3 takes from stage 2's plan."""
+    print(f"stage 2 {hidden} {rows} {hint} {layout}", flush=True)
+    W, nle = 3, 5
+    rng = np.random.default_rng(hidden + rows)
+    a = HIPAllToAll(MoEConfig(W * nle, 1, hidden, rows // W + 1, torch.bfloat16, torch.bfloat16), 1, W, device=DEV, layout=layout)
+    source = np.sort(rng.integers(0, W, rows))
+    meta = np.stack([nle + rng.integers(0, nle, rows), source, np.arange(rows), np.zeros(rows), np.zeros(rows)], 1).astype(np.int32)
+    buf = torch.from_numpy(rng.integers(-30000, 30000, (rows, hidden), dtype=np.int16))
+    counts = torch.from_numpy(np.bincount(source, minlength=W).astype(np.int32)).to(DEV)
+    num, ex, em = a.dispatch_recv(counts, buf.to(DEV).view(torch.bfloat16), torch.from_numpy(meta).to(DEV), hint)
+    back_counts, back, back_meta = a.combine_send(em, ex, num)
+    expert = meta[:, 0] - nle
+    assert np.array_equal(num.cpu().numpy(), np.bincount(expert, minlength=nle))
+    got_x, got_m = ex.cpu().view(torch.int16), em.cpu().numpy()
+    at = 0
+    for le in range(nle):
+        mine = np.flatnonzero(expert == le)
+        x, m = (got_x[at:at + len(mine)], got_m[at:at + len(mine)]) if layout == "compact" else (got_x[le, :len(mine)], got_m[le, :len(mine)])
+        assert torch.equal(x, buf[torch.from_numpy(mine)]) and np.array_equal(m, meta[mine]), le
+        at += len(mine)
+    order = np.lexsort((np.arange(rows), expert, source))
+    assert torch.equal(back_counts, counts) and np.array_equal(back_meta[:rows].cpu().numpy(), meta[order])
+    assert torch.equal(back[:rows].cpu().view(torch.int16), buf[torch.from_numpy(order)])

@@ -7,6 +7,7 @@ from pathlib import Path
 import pytest
 
 from tests.test_gpu_block_streams import CASES
+from tests.test_gpu_short_streams import RECV_CASES
 
 CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
 SEND_WAYS = ["by entry", "few", "block", "fanout", "wide fanout"]  # SendWay
@@ -21,6 +22,9 @@ def rules(tmp_path_factory):
                    'extern "C" int way(long long tokens, int k, int ranks, int row_vecs, int vec16) {\n'
                    '  return send_way(tokens, k, ranks, row_vecs, vec16); }\n'
                    'extern "C" int piece(long long tokens, int k, int nvw, int vec16) { return block_piece(tokens, k, nvw, vec16); }\n'
+                   'extern "C" int few(long long rows, int row_vecs, int nvw, int vec16, int compact) {\n'
+                   '  return recv_few(rows, row_vecs, nvw, vec16, compact); }\n'
+                   'extern "C" int through(long long rows, long long row_bytes) { return recv_through(rows, row_bytes); }\n'
                    'extern "C" int keys(long long entries) { return few_keys(entries); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
@@ -28,6 +32,8 @@ def rules(tmp_path_factory):
     dll = C.CDLL(str(lib))
     dll.way.argtypes = [C.c_longlong] + [C.c_int] * 4
     dll.piece.argtypes = [C.c_longlong] + [C.c_int] * 3
+    dll.few.argtypes = [C.c_longlong] + [C.c_int] * 4
+    dll.through.argtypes = [C.c_longlong, C.c_longlong]
     dll.keys.argtypes = [C.c_longlong]
     return dll
 
@@ -82,3 +88,29 @@ def test_limits_of_the_kernels_of_stage_1(rules):
                     if way == "wide fanout":
                         assert (ranks + 1) << max(1, (entries - 1).bit_length()) < 2 ** 31 and tokens * pieces < 2 ** 30
     assert rules.way(0, 2, 8, 896, 1) == 0 and SEND_WAYS[rules.way(0, 8, 8, 896, 1)] == "wide fanout"  # (which read nothing then)
+
+
+def recv_way(rules, rows, hidden, layout):
+    vecs, vec16, nvw = row(hidden)
+    few = rules.few(rows, vecs, nvw, vec16, layout == "compact")
+    if few:
+        return "few, through" if few == 2 else "few, plain"
+    return "scan, through" if rules.through(rows, 2 * hidden) else "scan, plain"
+
+
+@pytest.mark.parametrize("hidden,rows,hint,layout", RECV_CASES)
+def test_kernels_of_stage_2_that_the_gpu_tests_mean(rules, hidden, rows, hint, layout):
+    assert recv_way(rules, hint, hidden, layout) == RECV_CASES[hidden, rows, hint, layout]
+
+
+def test_ways_of_stage_2_that_there_are_kernels_for(rules):
+    """Stores past L2 from the kernel that holds all keys are built for 8, 12 and 16 vectors per lane, plain ones of the scan
+    only for rows of elements (with a plan)."""
+    for hidden in [*range(8, 9000, 8), 12288, 16384, 65536, 37, 1025, 7167]:
+        vecs, vec16, nvw = row(hidden)
+        for rows in (0, 1, 256, 512, 513, 600, 1000, 1024, 1025, 5000):
+            for layout in ("padded", "compact"):
+                way = recv_way(rules, rows, hidden, layout)
+                assert way != "few, through" or (vec16 and nvw in (8, 12, 16)), (hidden, rows)
+                assert way != "scan, plain" or not vec16, (hidden, rows)
+                assert way.startswith("scan") or rows <= 1024
