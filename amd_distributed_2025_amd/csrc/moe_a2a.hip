@@ -4113,8 +4113,7 @@ __global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
 // job in a graph with partial counts added up over the waves and tables of 64 ranks / here: 8 ranks x 16 tokens x 2, hidden
 // 6144 10.9 / 7.9, x 30 x 4, 2880 11.9 / 10.3, x 7 x 6, 7168 13.5 / 9.3, x 24 x 8, 4096 13.0 / 12.4 (16.2 with keys that every
 // wave picks up by itself); one rank's dispatch, expert and combine, 16 tokens x 2, hidden 256 10.5 / 9.3, 180 x 8, 4096 18.9 /
-// 17.7. NV: with more than 16 keys per lane and two workgroups per unit a lane moves two vectors of the row, or four, so that
-// half as many workgroups hold the keys (8 ranks x 49 x 5, 3856, partial counts / one vector / two: 13.2 / 13.7 / 12.6 us).
+// 17.7. NV: vectors of the row that a lane moves (local_few_vecs).
 template <typename V, int DIN, int DOUT, Store HOW, int R, int KEYS, int NV>
 __global__ __launch_bounds__(BLOCK) void local_dispatch_few_kernel(
     const void* x0, const int* indices0, int T, int K, int E, int chunks, int row_vecs, bool counts, bool compact, int max_recv,
@@ -5601,38 +5600,41 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
   hipStream_t st = (hipStream_t)stream;
   const bool through = (long long)S * s->hidden_dim * 2 >= JOB_THROUGH_BYTES;  // (Store)
   // Few ranks with few entries: the mover ranks them
-  int few_nv = 1;
-  auto chunks_of = [&](int nv) { return (g.row_vecs + BLOCK * nv - 1) / (BLOCK * nv); };
-  while (S > 64 * 16 && few_nv < 4 && chunks_of(few_nv) > 1 && tokens * chunks_of(few_nv) > 512) few_nv *= 2;
-  const int few_chunks = chunks_of(few_nv);
+  const int few_nv = local_few_vecs(tokens, S, W, g.row_vecs, g.vec16);
+  const int few_chunks = (g.row_vecs + BLOCK * few_nv - 1) / (BLOCK * few_nv);
   if (W <= LOCAL_FEW_RANKS && S > 0 && S <= LOCAL_RANK_ENTRIES && rank_limit == 0 && items_fit(tokens, few_chunks)) {
     const bool counts = expert_num_tokens || expert_offsets;
     const int grid = (counts ? 1 : 0) + (int)(tokens * few_chunks);
 #define LAUNCH_H(V, DI, DO, HOW, R, KEYS, NV)                                                              \
-  local_dispatch_few_kernel<V, DI, DO, HOW, R, KEYS, NV><<<grid, BLOCK, 0, st>>>(                              \
+  local_dispatch_few_kernel<V, DI, DO, HOW, R, KEYS, NV><<<grid, BLOCK, 0, st>>>(                          \
       x[0], indices[0], (int)tokens, K, E, few_chunks, g.row_vecs, counts, compact, g.max_recv, expert_limit, \
       g.nle, g.magic, W, entry_row, expert_num_tokens, expert_offsets, (V*)expert_rows, expert_meta,       \
       sources(LocalSources<R>{}))
-#define LAUNCH_T(V, DI, DO, R, KEYS, NV)                                                                    \
+#define LAUNCH_T(V, DI, DO, R, KEYS, NV)                                                                   \
   do {                                                                                                     \
-    if (through) LAUNCH_H(V, DI, DO, THROUGH_OF<V>, R, KEYS, NV);                                              \
-    else LAUNCH_H(V, DI, DO, PLAIN, R, KEYS, NV);                                                              \
+    if (through) LAUNCH_H(V, DI, DO, THROUGH_OF<V>, R, KEYS, NV);                                          \
+    else LAUNCH_H(V, DI, DO, PLAIN, R, KEYS, NV);                                                          \
   } while (0)
-#define LAUNCH_S(V, R, KEYS, NV)                                                                               \
+#define LAUNCH_S(V, R, KEYS, NV)                                                                           \
   do {                                                                                                     \
-    if (!standin) LAUNCH_T(V, -1, -1, R, KEYS, NV);                                                            \
+    if (!standin) LAUNCH_T(V, -1, -1, R, KEYS, NV);                                                        \
     else if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_T(V, MOE_A2A_BF16, MOE_A2A_BF16, R, KEYS, NV); \
     else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_T(V, MOE_A2A_F16, MOE_A2A_F16, R, KEYS, NV); \
-    else if (in_dtype == MOE_A2A_F16) LAUNCH_T(V, MOE_A2A_F16, MOE_A2A_BF16, R, KEYS, NV);                     \
-    else LAUNCH_T(V, MOE_A2A_BF16, MOE_A2A_F16, R, KEYS, NV);                                                  \
+    else if (in_dtype == MOE_A2A_F16) LAUNCH_T(V, MOE_A2A_F16, MOE_A2A_BF16, R, KEYS, NV);                 \
+    else LAUNCH_T(V, MOE_A2A_BF16, MOE_A2A_F16, R, KEYS, NV);                                              \
+  } while (0)
+#define LAUNCH_N(V, R, KEYS)                                                                               \
+  do {                                                                                                     \
+    constexpr int MORE = sizeof(V) == sizeof(b128) ? 2 : 4;  /* (local_few_vecs) */                        \
+    if (few_nv == 1) LAUNCH_S(V, R, KEYS, 1);                                                              \
+    else if (few_nv == MORE) LAUNCH_S(V, R, KEYS, MORE);                                                   \
+    else LAUNCH_S(V, R, KEYS, 2 * MORE);                                                                   \
   } while (0)
 #define LAUNCH_K(V, R)                                                                                     \
   do {                                                                                                     \
-    if (S <= 64 * 4) LAUNCH_S(V, R, 4, 1);                                                                    \
-    else if (S <= 64 * 16) LAUNCH_S(V, R, 16, 1);                                                             \
-    else if (few_nv == 4) LAUNCH_S(V, R, 32, 4);         \
-    else if (few_nv == 2) LAUNCH_S(V, R, 32, 2);         \
-    else LAUNCH_S(V, R, 32, 1);                                                                             \
+    if (S <= 64 * 4 && few_nv == 1) LAUNCH_S(V, R, 4, 1);                                                  \
+    else if (S <= 64 * 16) LAUNCH_N(V, R, 16);                                                             \
+    else LAUNCH_N(V, R, 32);                                                                               \
   } while (0)
 #define LAUNCH(V)                                                                                          \
   do {                                                                                                     \
@@ -5643,6 +5645,7 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
     else LAUNCH(uint16_t);
 #undef LAUNCH
 #undef LAUNCH_K
+#undef LAUNCH_N
 #undef LAUNCH_S
 #undef LAUNCH_T
 #undef LAUNCH_H

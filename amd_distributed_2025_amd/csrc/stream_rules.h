@@ -116,4 +116,22 @@ RecvFew recv_few(long long rows_hint, int row_vecs, int nvw, bool vec16, bool co
   return nvw == 14 ? RECV_NOT_FEW : pieces ? RECV_FEW_PLAIN : RECV_FEW_THROUGH;
 }
 
+// ---------------------------------------------------------------- jobs on one GPU
+
+// Vectors of a row that a lane of local_dispatch_few_kernel moves: one, two or four, of single elements one, four or eight. Every
+// workgroup holds all keys, so that many pieces of rows cost more than the rows: beyond two workgroups per unit with tables of
+// several ranks or more than 1024 keys, else beyond four, a lane moves more. (Up to 256 keys are so few that pieces of
+// whole vectors stay as they are.) us, one / two / four / eight vectors (ranks x tokens x entries, hidden): 8 x 60 x 2, 7168 8.1 / 6.7 / 5.8 / 6.6,
+// 8 x 100 x 1, 7168 9.9 / 7.7 / 6.5 / 8.3, 8 x 16 x 4, 7168 5.1 / 5.2 / 6.2, 1 x 900 x 1, 7168 7.1 / 5.6 / 5.1 / 6.9, 1 x 128 x 8,
+// 7168 5.7 / 6.0 / 8.1; single elements 8 x 64 x 2, 7167 30.0 / 18.2 / 12.4 / 10.3, 8 x 16 x 8, 3001 9.3 / 7.3 / 7.2 / 8.2, 1 x 250 x 8, 5001
+// 24.3 / 15.9 / 11.7 / 11.2, 1 x 1000 x 1, 513 5.1 / 4.5 / 3.6 / 4.0, 1 x 16 x 8, 7167 3.8 / 4.4 / 5.1 / 6.3.
+int local_few_vecs(long long tokens, long long entries, int ranks, int row_vecs, bool vec16) {
+  if (row_vecs <= BLOCK || (vec16 && entries <= 64 * 4)) return 1;
+  auto workgroups = [&](int vecs) { return tokens * ((row_vecs + BLOCK * vecs - 1) / (BLOCK * vecs)); };
+  const int limit = entries > 64 * 16 || (ranks > 1 && entries > 64 * 4) ? 512 : 1024;
+  if (workgroups(1) <= limit) return 1;
+  const int more = vec16 ? 2 : 4;
+  return row_vecs <= BLOCK * more || workgroups(more) <= (vec16 ? limit : 1024) ? more : 2 * more;
+}
+
 }  // namespace

@@ -538,7 +538,7 @@ int moe_a2a_exchange_gather_local(int32_t world_size, int32_t hidden_dim,
  *   expert_offsets      int32[num_experts + 1] out, or NULL (compact layout only)
  *   expert_meta   int32[rows, 5] out (expert, source rank, token, k, 0), or NULL
  * Limits: world_size <= 64, num_experts <= 1024, experts_per_token <= 64
- * (MOE_A2A_EINVAL). One launch for one rank with up to 2048 entries, else two.
+ * (MOE_A2A_EINVAL). One launch for up to 8 ranks with up to 2048 entries, else two.
  * The first call on a GPU sets kernel attributes: make it outside a graph capture.
  */
 int moe_a2a_local_dispatch(const moe_a2a_shape* shape, const void* const* x,

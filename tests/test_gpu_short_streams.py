@@ -148,3 +148,23 @@ def test_kernels_of_stage_2(hidden, rows, hint, layout):
     order = np.lexsort((np.arange(rows), expert, source))
     assert torch.equal(back_counts, counts) and np.array_equal(back_meta[:rows].cpu().numpy(), meta[order])
     assert torch.equal(back[:rows].cpu().view(torch.int16), buf[torch.from_numpy(order)])
+
+
+# ranks, tokens of each, entries per token, hidden -> vectors of a row that a lane moves (csrc/stream_rules.h; test_stream_rules.py
+# holds the cases to that)
+LANES = {(1, 16, 8, 7168): 1, (2, 100, 1, 513): 1, (8, 16, 4, 7168): 1, (3, 60, 2, 7168): 2, (1, 300, 1, 7168): 2, (8, 40, 2, 7168): 4,
+         (1, 900, 1, 7168): 4, (2, 20, 3, 7167): 4, (1, 1000, 1, 513): 4, (5, 30, 6, 4100): 4, (8, 26, 1, 7167): 8, (1, 300, 4, 5001): 8,
+         (2, 300, 2, 2049): 8}
+
+
+@pytest.mark.parametrize("world_size,tokens,topk,hidden", LANES)
+@pytest.mark.parametrize("dtypes", ["bf16 fp16", "fp16 fp16"])
+def test_lanes_that_move_several_vectors_of_short_jobs(world_size, tokens, topk, hidden, dtypes):
+    print(f"lanes {world_size} {tokens} {topk} {hidden} {dtypes}", flush=True)
+    din, dout = ({"bf16": torch.bfloat16, "fp16": torch.float16}[d] for d in dtypes.split())
+    cfg = config(8 * world_size, topk, hidden, tokens, din, dout)
+    data = [rank_data(cfg, tokens - r, 5 * r) for r in range(world_size)]
+    want = [y.clone() for y in LocalWorld(cfg, world_size, device=DEV).run(data)]
+    ys = custom_kernel_job([(cfg, d, r, world_size) for r, d in enumerate(data)])
+    for r in range(world_size):
+        assert torch.equal(ys[r], want[r]), f"rank {r}"

@@ -7,7 +7,7 @@ from pathlib import Path
 import pytest
 
 from tests.test_gpu_block_streams import CASES
-from tests.test_gpu_short_streams import RECV_CASES
+from tests.test_gpu_short_streams import LANES, RECV_CASES
 
 CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
 SEND_WAYS = ["by entry", "few", "block", "fanout", "wide fanout"]  # SendWay
@@ -25,6 +25,8 @@ def rules(tmp_path_factory):
                    'extern "C" int few(long long rows, int row_vecs, int nvw, int vec16, int compact) {\n'
                    '  return recv_few(rows, row_vecs, nvw, vec16, compact); }\n'
                    'extern "C" int through(long long rows, long long row_bytes) { return recv_through(rows, row_bytes); }\n'
+                   'extern "C" int lanes(long long tokens, long long entries, int ranks, int row_vecs, int vec16) {\n'
+                   '  return local_few_vecs(tokens, entries, ranks, row_vecs, vec16); }\n'
                    'extern "C" int keys(long long entries) { return few_keys(entries); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
@@ -34,6 +36,7 @@ def rules(tmp_path_factory):
     dll.piece.argtypes = [C.c_longlong] + [C.c_int] * 3
     dll.few.argtypes = [C.c_longlong] + [C.c_int] * 4
     dll.through.argtypes = [C.c_longlong, C.c_longlong]
+    dll.lanes.argtypes = [C.c_longlong, C.c_longlong] + [C.c_int] * 3
     dll.keys.argtypes = [C.c_longlong]
     return dll
 
@@ -114,3 +117,22 @@ def test_ways_of_stage_2_that_there_are_kernels_for(rules):
                 assert way != "few, through" or (vec16 and nvw in (8, 12, 16)), (hidden, rows)
                 assert way != "scan, plain" or not vec16, (hidden, rows)
                 assert way.startswith("scan") or rows <= 1024
+
+
+@pytest.mark.parametrize("W,T,K,H", LANES)
+def test_vectors_of_a_lane_that_the_gpu_tests_mean(rules, W, T, K, H):
+    vecs, vec16, _ = row(H)
+    tokens = W * T - W * (W - 1) // 2  # (rank r has r tokens less)
+    assert rules.lanes(tokens, tokens * K, W, vecs, vec16) == LANES[W, T, K, H] and tokens * K <= 2048
+
+
+@pytest.mark.parametrize("W,T,K,H,lanes", [
+    (8, 60, 2, 7168, 4), (8, 100, 1, 7168, 4), (1, 900, 1, 7168, 4), (1, 1000, 1, 4096, 2), (1, 500, 2, 7168, 2), (4, 60, 4, 7168, 2),
+    (2, 200, 2, 4096, 2), (1, 128, 8, 7168, 1), (8, 30, 4, 4096, 1), (8, 8, 4, 7168, 1), (1, 256, 1, 7168, 1), (1, 250, 8, 7168, 2),
+    (8, 64, 2, 7167, 8), (8, 16, 8, 3001, 4), (1, 1000, 1, 7167, 8), (1, 200, 4, 3001, 4), (8, 60, 2, 1001, 4), (4, 20, 6, 4097, 4),
+    (8, 8, 4, 7167, 4), (1, 16, 8, 7167, 1), (8, 4, 8, 7167, 1), (1, 16, 2, 257, 1), (1, 250, 8, 5001, 8),
+])
+def test_vectors_of_a_lane_that_were_fastest(rules, W, T, K, H, lanes):
+    """Timed on the GPU, of one, two, four and eight: the fastest or within a tenth of it."""
+    vecs, vec16, _ = row(H)
+    assert rules.lanes(W * T, W * T * K, W, vecs, vec16) == lanes
