@@ -125,6 +125,8 @@ bool streams_far_ahead(long long rows_hint, int groups, int N) {
 // and where the others stay: 40, 8, 7168 x 7168 (skewed) 144 / - / 182 / 165 / 143; 28, 8, 7168 x 1536 (skewed) 37.9 / - / 47.5 / 40.4 /
 // 42.8; 40, 128, 1792 x 7168 587 / - / 719 / 566 / 537; 28, 128, 4096 x 2880 516 / - / 611 / 532 / 542; 4, 8, 7168 x 2048 39.7 / - / 44.1 /
 // 45.7 / 46.6; 2, 53, 2240 x 512 23.3 / 35.8 / 29.4; 68, 41, 512 x 640 12.7 / 23.1 / 17.1 / 16.0 / 19.7.
+// A ring is filled whatever the walk: with fewer than five steps of K (three on 32 x 32, eight on 64 x 128) that takes longer than the
+// others' whole product: 57, 5, 2816 x 8 4.9 / 6.8 on 64 x 128 and 48, 10, 896 x 360 8.2 / 9.8; but 25, 11, 512 x 216 5.5 / 4.9 on 32 x 32.
 // Over 12204 products (4 to 128 groups, 0.06 to 400 rows per group, N and K of 512 to 14000, half of them with Zipf's routing, exponent
 // 1.2) the choice takes 0.907 of the others' time (geometric mean; the best of all five 0.88) and is more than 5 % behind them on 1.3 %.
 enum RingTile { NO_RING = 0, RING_32x32, RING_32x64, RING_64x64, RING_64x128 };
@@ -133,15 +135,18 @@ RingTile grouped_ring(long long rows_hint, int groups, int N, int K) {
   constexpr double UNITS = 256;
   if (!tile_rows_in_range(128, K)) return NO_RING;
   const int steps = (K + 63) / 64;
+  if (steps < 3) return NO_RING;
   const double rows = (double)rows_hint / groups, hit = 1.0 - std::exp(-rows);
   auto per_unit = [&](int high, int wide) {
     const double of_a_group = rows < 0.7 ? hit : std::max(hit, rows / high + 0.5);
     return of_a_group * groups * ((N + wide - 1) / wide) / UNITS;
   };
   if (rows <= 40 && per_unit(32, 32) <= 1) return RING_32x32;
+  if (steps < 5) return NO_RING;
   const double of_32 = per_unit(32, 64), of_64 = per_unit(64, 64), of_128 = per_unit(64, 128);
-  if (rows >= 56) return of_64 <= 1 ? RING_64x64 : of_128 <= 0.9 ? RING_64x128 : NO_RING;
-  if (rows > 40 && of_128 >= 0.6 && of_128 <= 0.9) return RING_64x128;
+  const bool one_per_unit = steps >= 8 && of_128 <= 0.9;
+  if (rows >= 56) return of_64 <= 1 ? RING_64x64 : one_per_unit ? RING_64x128 : NO_RING;
+  if (rows > 40 && of_128 >= 0.6 && one_per_unit) return RING_64x128;
   const bool far_ahead = streams_far_ahead(rows_hint, groups, N);
   // (few rows hit now more groups, now less; where nothing else is under way either, more than a tile per unit is still ahead)
   if (of_32 <= (rows < 2 && far_ahead ? 0.9 : rows < 1 ? 1.5 : 1.0)) return RING_32x64;
@@ -229,7 +234,8 @@ LinearWay linear_way(long long M, long long N, long long K, long long* least_cos
 }
 
 // Whether a plain product goes to ring_gemm_kernel instead. With K too short to be split it is ahead on tiles of 32 x 32 as
-// long as every unit has one at most. Above, tiles of 64 x 64, which it has under way for longer than dense_gemm_kernel and which fetch
+// long as every unit has one at most, but for walks that end before the ring is filled: 1 to 7 steps take 1.11, 1.07, 1.05, 1.01, 0.99,
+// 0.96 and 0.93 of the others' time (284 products). Above, tiles of 64 x 64, which it has under way for longer than dense_gemm_kernel and which fetch
 // no more than skinny_gemm_kernel does, fill a gap between those two; a wait of 300 in the comparison above finds them (280 to 320 choose
 // the same of 95 shapes), from 12 steps on (shorter ones are as fast elsewhere). us, linear_way's choice / here:
 //   137 x 4320 x 5440  47.9 / 25.7     200 x 4096 x 4096  36.9 / 21.4     82 x 6592 x 2816  27.1 / 16.9
@@ -239,7 +245,7 @@ LinearWay linear_way(long long M, long long N, long long K, long long* least_cos
 RingTile linear_ring(long long M, long long N, long long K) {
   constexpr long long UNITS = 256, WAIT = 300;
   const long long steps = (K + 63) / 64;
-  if (steps < 8) return (M + 31) / 32 * ((N + 31) / 32) <= UNITS ? RING_32x32 : NO_RING;
+  if (steps < 8) return steps >= 5 && (M + 31) / 32 * ((N + 31) / 32) <= UNITS ? RING_32x32 : NO_RING;
   if (steps < 12 || M <= 64) return NO_RING;
   const long long n = (M + 63) / 64 * ((N + 63) / 64);
   long long least = 0;  // (more than a unit's tile each, or one of the largest tiles: not compared)

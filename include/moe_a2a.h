@@ -379,7 +379,7 @@ int moe_a2a_expert_gemm(const moe_a2a_shape* shape, const void* expert_x,
  * 64 and n <= 24448 and else where larger tiles would leave compute units without
  * work; kernels bound by the matrix cores, whose workgroups own output tiles of
  * 256 x 256, 192 x 128, 128 x 128 or 64 x 128 (all of them add the same terms in
- * the same order); where tiles of 64 x 64 (of 32 x 32 for k <= 448) are at most one
+ * the same order); where tiles of 64 x 64 (of 32 x 32 for 256 < k <= 448) are at most one
  * per compute unit and the others would take longer, the kernel that
  * moe_a2a_expert_gemm has for few tiles, in that order too; for shapes beyond their index ranges, the kernel of moe_a2a_expert_gemm
  * with one group of m rows.

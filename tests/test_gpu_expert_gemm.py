@@ -101,9 +101,9 @@ def test_small_integers_sum_exactly(H, dt):
 
 # experts, in_dim, out_dim -> counts of rows per expert and the kernel that they pick; test_tile_rules.py holds them to that
 KERNELS_OF_NARROW = {
-    (5, 96, 160): {0: "ring 32 x 32", 56: "ring 64 x 64", 768: "ring 64 x 64", 3000: "tiles 128", 10000: "tiles 256"},
-    (5, 200, 64): {0: "ring 32 x 32", 56: "ring 64 x 64", 768: "ring 64 x 64", 10000: "tiles 128"},
-    (5, 128, 128): {0: "ring 32 x 32", 56: "ring 64 x 64", 768: "ring 64 x 64", 10000: "tiles 128"},
+    (5, 96, 160): {0: "stream 32, four steps ahead", 56: "tiles 64", 768: "tiles 64", 3000: "tiles 128", 10000: "tiles 256"},
+    (5, 200, 64): {0: "ring 32 x 32", 56: "tiles 64", 768: "tiles 64", 10000: "tiles 128"},
+    (5, 328, 128): {0: "ring 32 x 32", 56: "ring 64 x 64", 768: "ring 64 x 64", 10000: "tiles 128"},
     (128, 96, 160): {2: "stream 32, four steps ahead", 60: "tiles 128"},
     (300, 200, 160): {2: "stream 32, two steps ahead", 20: "stream 64", 50: "stream 128", 60: "tiles 64"}}
 

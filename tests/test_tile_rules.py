@@ -89,10 +89,10 @@ def test_every_count_of_rows_has_a_tile(rules):
 
 @pytest.mark.parametrize("K", [8, 200, 2048, 2112])
 def test_the_kernels_that_the_gpu_tests_mean(rules, K):
-    """(with few steps of K other tiles are picked, but a streaming kernel stays one)"""
+    """(with few steps of K other tiles and no rings are picked, but a streaming kernel stays one)"""
     for groups, kernels in KERNELS.items():
         picked = {rows: kernel_of(rules, rows, groups, 7168, K) for rows in kernels}
-        assert picked == kernels if K > 2000 else all(picked[r].split()[0] == k.split()[0] for r, k in kernels.items())
+        assert picked == kernels if K > 2000 else all(picked[r].split()[0] == k.split()[0] for r, k in kernels.items() if "ring" not in k)
     tested = {k for kernels in KERNELS.values() for k in kernels.values()}
     assert tested >= {f"tiles {t}" for t in (64, 128, 192, 256, 320)} | {f"stream {s}" for s in ("64", "128")}
     assert {f"stream 32, {n} steps ahead" for n in ("two", "four")} <= tested
@@ -191,7 +191,7 @@ def test_ways_of_a_product_stay_in_the_range_of_their_kernels(rules):
 @pytest.mark.parametrize("tile", RING_TILES)
 def test_rings_that_the_gpu_tests_mean(rules, tile):
     groups, n, rows = RING_TILES[tile]
-    for k in [*RING_STEPS, 1544, 2112]:
+    for k in [*RING_STEPS[tile], 1544, 2112]:
         assert rules.ring(rows * groups, groups, n, k) == tile, k
     assert rules.ring(30000 * groups, groups, n, 2048) == 0
 
@@ -202,6 +202,7 @@ def test_rings_that_the_gpu_tests_mean(rules, tile):
     (144, 64, 1024, 2048, 0), (144, 64, 2048, 1024, 0), (118, 53, 2240, 512, 0), (2792, 41, 512, 640, 0), (2468, 48, 1856, 1184, 0),
     (320, 8, 7168, 7168, 0), (224, 8, 7168, 1536, 0), (32, 8, 7168, 2048, 0), (1280, 32, 2048, 1536, 0), (128, 32, 2048, 2880, 0),
     (8192, 32, 2048, 4096, 0), (0, 3, 7168, 200, 1), (7, 48, 832, 1 << 23, 0),
+    (4, 44, 1728, 8, 0), (275, 11, 512, 216, 1), (285, 5, 2816, 8, 0), (480, 10, 896, 360, 0),
 ])
 def test_ring_that_was_fastest(rules, rows_hint, groups, n, k, tile):
     """(a tenth slower on tiles of 32 x 64, uniform or skewed: 8 groups of 40 rows, 7168 x 7168, of 28, 7168 x 1536, of 4,
@@ -221,7 +222,7 @@ def test_many_rows_are_not_cut_into_tiles_of_32(rules, groups, n, k):
 @pytest.mark.parametrize("m,n,k,tile", [
     (137, 4320, 5440, 3), (200, 4096, 4096, 3), (82, 6592, 2816, 3), (494, 2048, 2176, 3), (195, 3008, 832, 3),
     (255, 1728, 3968, 0), (349, 4032, 2752, 0), (160, 4544, 512, 0), (64, 7168, 2304, 0), (8192, 8192, 3696, 0), (2048, 2880, 360, 0),
-    (15, 5888, 448, 1), (80, 2176, 448, 1), (33, 4608, 352, 0), (1, 32, 8, 1), (100, 4096, 1 << 22, 0),
+    (15, 5888, 448, 1), (80, 2176, 448, 1), (33, 4608, 352, 0), (1, 32, 264, 1), (1, 32, 256, 0), (2, 1344, 64, 0), (100, 4096, 1 << 22, 0),
 ])
 def test_plain_products_on_rings(rules, m, n, k, tile):
     assert rules.linear_ring_of(m, n, k) == tile
