@@ -56,6 +56,7 @@ HIPCC_FLAGS = [
     # keep the compiler from forming packed-fp32 instructions
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
+EXT_CFLAGS = ["-O2", "-std=c++17"]
 
 
 def hipcc_path() -> str:
@@ -65,23 +66,23 @@ def hipcc_path() -> str:
     raise RuntimeError("hipcc not found (looked at $HIPCC, PATH and /opt/rocm/bin)")
 
 
-def _hash(*files: Path) -> str:
+def _hash(flags: list, *files: Path) -> str:
     import hashlib
 
-    h = hashlib.sha256()
+    h = hashlib.sha256("\0".join(flags).encode())
     for f in files:
         h.update(f.read_bytes())
     return h.hexdigest()[:16]
 
 
 def source_id() -> str:
-    """What `moe_a2a_build_id()` of a library built from the present sources returns."""
-    return _hash(SOURCE, *HEADERS)
+    """What `moe_a2a_build_id()` of a library built from the present sources, with the present flags, returns."""
+    return _hash(HIPCC_FLAGS, SOURCE, *HEADERS)
 
 
 def extension_id() -> str:
-    """What `a2a_extension_id()` of an extension built from the present sources returns."""
-    return _hash(EXT_SOURCE, CALLS_SOURCE, ABI_HEADER)
+    """What `a2a_extension_id()` of an extension built from the present sources, with the present flags, returns."""
+    return _hash(EXT_CFLAGS, EXT_SOURCE, CALLS_SOURCE, ABI_HEADER)
 
 
 def build_library(verbose: bool = False) -> Path:
@@ -113,7 +114,7 @@ def build_extension(verbose: bool = False) -> Path:
         name=EXT_NAME,
         cpp_sources=[f'#define A2A_EXTENSION_ID "{extension_id()}"', EXT_SOURCE.read_text(), CALLS_SOURCE.read_text()],
         functions=EXT_FUNCTIONS + EXT_CALLS,
-        extra_cflags=["-O2", "-std=c++17"],
+        extra_cflags=EXT_CFLAGS,
         extra_include_paths=[str(REPO_DIR / "include")],
         # $ORIGIN/.. is the package directory as seen from _ext/ ($$ is ninja's escape for $)
         extra_ldflags=[f"-L{PKG_DIR}", "-l:libmoe_a2a.so", "-Wl,-rpath,'$$ORIGIN/..'"],

@@ -35,6 +35,15 @@ def test_library_exports_every_declared_symbol():
     assert lib.moe_a2a_build_id().decode() == source_id()
 
 
+def test_ids_of_a_build_cover_its_flags(monkeypatch):
+    """A library built with other flags is another library: code generation, and with it figures, hang on them."""
+    from amd_distributed_2025_amd import build
+    library, extension = build.source_id(), build.extension_id()
+    monkeypatch.setattr(build, "HIPCC_FLAGS", build.HIPCC_FLAGS[:-1])
+    monkeypatch.setattr(build, "EXT_CFLAGS", ["-O1", "-std=c++17"])
+    assert build.source_id() != library and build.extension_id() != extension
+
+
 def test_argument_counts_match_the_header():
     """ctypes signatures and header prototypes must list the same number of parameters."""
     flat = re.sub(r"/\*.*?\*/", "", HEADER, flags=re.S)
