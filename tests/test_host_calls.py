@@ -1,6 +1,7 @@
 """csrc/host_calls.cpp without a GPU: whatever is not a plain tensor on the rank's GPU is refused before anything is
 launched, and the class surface does without the extension."""
 import copy
+import functools
 
 import pytest
 import torch
@@ -117,32 +118,70 @@ def _int(*shape):
     return torch.zeros(*shape, dtype=torch.int32)
 
 
-# method -> its arguments after the shape, and which of them may not be shorter (by place)
+# method -> its arguments (SHAPE goes ahead of them unless they begin with numbers); every tensor among them, in lists too, is
+# as small as it may be, but for the row and meta buffers whose rows the binding passes on as a capacity (by place)
 SIZED = {
-    "dispatch_recv": ([_bf(24, 64), _int(24, 5), _int(1), 24, _int(8), _bf(8, 12, 64), _int(8, 12, 5), None, 0], [2]),
-    "dispatch_recv_compact": ([_bf(24, 64), _int(24, 5), _int(1), 24, _int(8), _int(9), _bf(24, 64), _int(24, 5), None, 0], [2]),
-    "expert_scale": ([_bf(8, 12, 64), _int(8), 24, _bf(8, 12, 64), 0], [0, 1, 3]),
-    "expert_scale_compact": ([_bf(24, 64), _int(8), 24, _bf(24, 64), 0], [1]),
-    "expert_gemm": ([_bf(8, 12, 64), _int(8), 24, _bf(8, 32, 64), None, _bf(8, 12, 32), 0], [0, 1, 5]),
-    "expert_gemm_compact": ([_bf(24, 64), _int(8), 24, _bf(8, 32, 64), None, _bf(24, 32), 0], [1]),
-    "combine_send": ([_bf(8, 12, 64), _int(8, 12, 5), _int(8), 24, _bf(24, 64), _int(24, 5), _int(1), None, 0], [0, 1, 2]),
-    "combine_send_compact": ([_bf(24, 64), _int(24, 5), _int(8), 24, _bf(24, 64), _int(24, 5), _int(1), None, 0], [2]),
-    "combine_recv": ([_bf(24, 64), _int(24, 5), _int(1), 24, torch.zeros(12, 2), 12, _bf(12, 64), True, 0], [2, 4, 6]),
+    "dispatch_send": ([_bf(12, 64), _int(12, 2), 12, _bf(24, 64), _int(24, 5), _int(1), _int(24), 0], []),
+    "plan_send": ([_int(12, 2), 12, _int(1), _int(2), _int(8), _int(24), _int(24), 0], []),
+    "dispatch_recv": ([_bf(24, 64), _int(24, 5), _int(1), 24, _int(8), _bf(8, 12, 64), _int(8, 12, 5), _int(16), 0], [0, 1]),
+    "dispatch_recv_compact": ([_bf(24, 64), _int(24, 5), _int(1), 24, _int(8), _int(9), _bf(24, 64), _int(24, 5), _int(16), 0],
+                              [0, 1, 6, 7]),
+    "expert_scale": ([_bf(8, 12, 64), _int(8), 24, _bf(8, 12, 64), 0], []),
+    "expert_scale_compact": ([_bf(24, 64), _int(8), 24, _bf(24, 64), 0], [0, 3]),
+    "expert_gemm": ([_bf(8, 12, 64), _int(8), 24, _bf(8, 32, 64), _bf(8, 32), _bf(8, 12, 32), 0], []),
+    "expert_gemm_compact": ([_bf(24, 64), _int(8), 24, _bf(8, 32, 64), _bf(8, 32), _bf(24, 32), 0], [0, 5]),
+    "combine_send": ([_bf(8, 12, 64), _int(8, 12, 5), _int(8), 24, _bf(24, 64), _int(24, 5), _int(1), _int(16), 0], [4, 5]),
+    "combine_send_compact": ([_bf(24, 64), _int(24, 5), _int(8), 24, _bf(24, 64), _int(24, 5), _int(1), _int(16), 0], [0, 1, 4, 5]),
+    "combine_recv": ([_bf(24, 64), _int(24, 5), _int(1), 24, torch.zeros(12, 2), 12, _bf(12, 64), True, 0], [0, 1]),
+    "linear": ([_bf(12, 64), _bf(32, 64), _bf(32), _bf(12, 32), 0], [0, 1]),
+    "exchange_local": ([1, 64, _bf(24, 64), _int(24, 5), _int(1), 0, _bf(24, 64), _int(24, 5), _int(1), 0, 24, 0], [2, 3, 6, 7]),
+    "local_dispatch": ([[_bf(12, 64)], [_int(12, 2)], False, _int(24), _int(8), _int(9), _bf(8, 12, 64), _int(8, 12, 5), False, 0], [1]),
+    "local_combine": ([_bf(24, 64), _int(24), [torch.zeros(12, 2)], [12], [_bf(12, 64)], -1, False, 0], [0]),
 }
 
 
 @pytest.mark.parametrize("method", SIZED)
 def test_tensors_that_hold_less_than_a_call_addresses_are_refused(method):
-    args, sized = SIZED[method]
+    args, sets_a_capacity = SIZED[method]
     b = Recorded()
-    getattr(b, method)(SHAPE, *args)
+    call = getattr(b, method) if method in ("linear", "exchange_local") else functools.partial(getattr(b, method), SHAPE)
+    call(*args)
     assert len(b.called) == 1
-    for at in sized:
+    looked_at = 0
+    for at, arg in enumerate(args):
+        tensor = arg[0] if isinstance(arg, list) else arg
+        if at in sets_a_capacity or not isinstance(tensor, torch.Tensor):
+            continue
         short = list(args)
-        short[at] = args[at][:-1]
+        short[at] = [tensor[:-1]] if isinstance(arg, list) else tensor[:-1]
         with pytest.raises(ValueError, match="the call needs"):
-            getattr(b, method)(SHAPE, *short)
-    assert len(b.called) == 1
+            call(*short)
+        looked_at += 1
+    assert len(b.called) == 1 and looked_at
+
+
+def test_rows_that_set_a_capacity_are_held_to_it():
+    """Compact rows are as many as their buffer has of the layer's width, a weight's columns the input's, and a gather's sources as
+    many as its ranks."""
+    b = Recorded()
+    with pytest.raises(ValueError, match="expert_x"):
+        b.expert_gemm_compact(SHAPE, _bf(24, 63), _int(8), 24, _bf(8, 32, 64), None, _bf(24, 32), 0)
+    with pytest.raises(ValueError, match="expert_y"):
+        b.expert_gemm_compact(SHAPE, _bf(24, 64), _int(8), 24, _bf(8, 32, 64), None, _bf(24, 31), 0)
+    with pytest.raises(ValueError, match="weight"):
+        b.linear(_bf(12, 64), _bf(32, 63), None, _bf(12, 32), 0)
+    with pytest.raises(ValueError, match="rows"):
+        b.local_dispatch(SHAPE, [_bf(12, 64)], [_int(12, 2)], True, _int(24), None, None, _bf(24, 63), None, False, 0)
+    with pytest.raises(ValueError, match="send_counts"):
+        b.gather_sources(64, [_bf(24, 64)] * 2, [_int(24, 5)] * 2, [_int(2), _int(1)])
+    sources = b.gather_sources(64, [_bf(24, 64)] * 2, [_int(24, 5)] * 2, [_int(2), _int(2)])
+    with pytest.raises(ValueError, match="sources"):
+        b.exchange_gather(3, 64, sources, 0, _bf(24, 64), _int(24, 5), _int(3), 24, 0)
+    with pytest.raises(ValueError, match="recv_counts"):
+        b.exchange_gather(2, 64, sources, 0, _bf(24, 64), _int(24, 5), _int(1), 24, 0)
+    assert not b.called
+    b.exchange_gather(2, 64, sources, 0, _bf(24, 64), _int(24, 5), _int(2), 24, 0)
+    assert b.called == ["moe_a2a_exchange_gather_local"]
 
 
 @pytest.mark.parametrize("rows, taken", [(24, False), (96, True), (95, False)])
