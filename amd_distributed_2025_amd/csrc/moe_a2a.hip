@@ -5234,6 +5234,7 @@ int allow_large_lds() {
   allow((const void*)skinny_gemm_kernel<MOE_A2A_BF16, 2, 8, false>, skinny_lds_bytes(2, 8));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8, true>, skinny_lds_bytes(2, 8));
   allow((const void*)skinny_gemm_kernel<MOE_A2A_F16, 2, 8, false>, skinny_lds_bytes(2, 8));
+  allow((const void*)local_plan_kernel<1>, local_plan_lds_bytes(LOCAL_MAX_EXPERTS));
   allow((const void*)local_plan_kernel<LOCAL_FEW_RANKS>, local_plan_lds_bytes(LOCAL_MAX_EXPERTS));
   allow((const void*)local_plan_kernel<LOCAL_MAX_RANKS>, local_plan_lds_bytes(LOCAL_MAX_EXPERTS));
   if (!ok) return MOE_A2A_ELAUNCH;
@@ -5679,7 +5680,10 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
 #undef LAUNCH
 #undef LAUNCH_H
   };
-  if (W <= LOCAL_FEW_RANKS) launch(sources(LocalSources<LOCAL_FEW_RANKS>{}));
+  // (one rank: nothing to pick from. us, planned, with a table of eight / one: 13694 tokens of 1.2 KB 19.2 / 15.4, 5452 of 2019
+  // elements, 2 each, 22.5 / 19.3, 1753 of 6.5 KB, 2 each 10.4 / 9.9)
+  if (W == 1) launch(sources(LocalSources<1>{}));
+  else if (W <= LOCAL_FEW_RANKS) launch(sources(LocalSources<LOCAL_FEW_RANKS>{}));
   else launch(sources(LocalSources<LOCAL_MAX_RANKS>{}));
   return launch_status();
 }

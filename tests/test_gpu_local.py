@@ -41,7 +41,7 @@ def config(E, K, H, T, din=torch.bfloat16, dout=torch.bfloat16):
     (64, 8, 2048, 256, None), (64, 8, 64, 257, None),                      # 2048 entries and 8 more: ranked, planned
     (64, 7, 4104, 40, "ids"), (300, 6, 520, 1000, "ids"),                  # ids outside the range, both ways
     (40, 9, 1032, 33, None), (64, 64, 128, 20, "ids"), (64, 33, 72, 90, None),  # more than eight entries per token
-    (1024, 4, 96, 700, None), (16, 8, 512, 300, "twins"), (4, 4, 264, 64, "twins"),
+    (1024, 4, 96, 700, None), (5, 3, 101, 900, "ids"), (16, 8, 512, 300, "twins"), (4, 4, 264, 64, "twins"),
 ])
 def test_one_rank_matches_the_halves(E, K, H, T, spoil, layout, binding, monkeypatch):
     print(f"one rank E={E} K={K} H={H} T={T} {spoil} {layout} {binding}", flush=True)
