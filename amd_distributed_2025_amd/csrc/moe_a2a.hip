@@ -551,9 +551,7 @@ __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
     const int base = c * (BLOCK * NV);
     const int i0 = t * K;
 
-    // the token's own expert ids (as in the kernel below), first batch of keys, then the row: the keys come back first
-    const bool all_own = K <= 64;
-    const int own0 = indices[i0 + min(all_own ? lane : lane & (FAN - 1), K - 1)];
+    // first batch of keys, then the row: the keys come back first
     int key[SCAN_UNROLL];
 #pragma unroll
     for (int u = 0; u < SCAN_UNROLL; ++u) key[u] = indices[min(tid + u * BLOCK, S - 1)];
@@ -561,13 +559,11 @@ __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
     p.load(x + (size_t)t * row_vecs, base, row_vecs);
 
     for (int g0 = 0; g0 < K; g0 += FAN) {
-      int own = own0;
-      if (!all_own && g0 > 0) own = first_use(indices[i0 + min(g0 + (lane & (FAN - 1)), K - 1)]);
       int mine[FAN];
 #pragma unroll
       for (int g = 0; g < FAN; ++g) {
-        const int k = min(g0 + g, K - 1);
-        mine[g] = klass(__builtin_amdgcn_readlane(own, all_own ? k : g)) * S + i0 + k;
+        const int i = i0 + min(g0 + g, K - 1);
+        mine[g] = klass(indices[i]) * S + i;
       }
       int cnt[FAN];
 #pragma unroll
@@ -608,13 +604,11 @@ __global__ __launch_bounds__(BLOCK) void dispatch_fanout_kernel(
       }
       if (c == 0 && tid < live * META) {
         const int g = tid / META, f = tid - g * META;
-        int slot = 0, e = 0;
+        int slot = 0;
 #pragma unroll
         for (int w = 0; w < NWAVES; ++w) slot += half[w * FAN + g];
-#pragma unroll
-        for (int gg = 0; gg < FAN; ++gg) e = gg == g ? __builtin_amdgcn_readlane(own, all_own ? min(g0 + gg, K - 1) : gg) : e;
         const int i = i0 + g0 + g;
-        const int m = f == 0 ? e : f == 1 ? rank : f == 2 ? t : f == 3 ? g0 + g : 0;
+        const int m = f == 0 ? indices[i] : f == 1 ? rank : f == 2 ? t : f == 3 ? g0 + g : 0;
         send_meta[(size_t)slot * META + f] = m;
         if (f == 0 && send_slot) send_slot[i] = slot;
       }
@@ -672,9 +666,10 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
     const int i0 = t * K;
 
     // the token's own expert ids: lane l of every wave holds entry l, or entry g0 + l % FAN of a token with more than
-    // 64. One vector load issued ahead of the keys (as uniform loads they become scalar loads that are
+    // 64 and where eight are ranked per pass, which is mostly the only one (1500 tokens of 5 KB, 4 per token, 16 ranks 13.4 us
+    // with entries picked by their number, 13.0 here). One vector load issued ahead of the keys (as uniform loads they become scalar loads that are
     // waited for one by one in the middle of the ranking)
-    const bool all_own = K <= 64;
+    const bool all_own = FAN < 8 && K <= 64;
     const int own0 = indices[i0 + min(all_own ? lane : lane & (FAN - 1), K - 1)];
     int key[KEYS];
 #pragma unroll
@@ -700,7 +695,10 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
       auto consume = [&](const int (&k)[KEYS], int b) {
 #pragma unroll
         for (int u = 0; u < KEYS; ++u) {
-          if (b + u * BLK >= S) break;  // (with few entries that is most of the batch)
+          // Keys past the end of the stream are left out where a lane has two vectors of the row: 188 tokens of 14 KB, 8 per
+          // token 5.57 us, 6.49 with them. With one, the branches cost more than the compares: 400 of 5 KB, 4 per token, 16 ranks
+          // 4.44 with branches, 4.25 here; 1000 8.38 / 8.06.
+          if (NV > 1 && b + u * BLK >= S) break;
           const int i2 = b + tid + u * BLK;
           const int ck = i2 < S ? composite(k[u], i2) : INT_MAX;
 #pragma unroll
@@ -754,8 +752,9 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
 #pragma unroll
         for (int gg = 0; gg < FAN; ++gg) {
           mine_slot = gg == g ? slot[gg] : mine_slot;
-          e = gg == g ? __builtin_amdgcn_readlane(own, all_own ? min(g0 + gg, K - 1) : gg) : e;
+          if (FAN < 8) e = gg == g ? __builtin_amdgcn_readlane(own, all_own ? min(g0 + gg, K - 1) : gg) : e;
         }
+        if (FAN == 8) e = __shfl(own, g, 64);  // (lanes 0 .. FAN-1 of wave 0 are among the active ones)
         const int i = i0 + g0 + g;
         const int m = f == 0 ? e : f == 1 ? rank : f == 2 ? t : f == 3 ? g0 + g : 0;
         send_meta[(size_t)mine_slot * META + f] = m;

@@ -38,6 +38,9 @@ CASES = {
     (8, 8, 8, 16, 4096): ("block", 1, 1), (4, 32, 4, 8, 16320): ("block", 1, 1),
     (4, 32, 4, 8, 16321): "fanout", (9, 18, 4, 8, 400): "fanout", (8, 32, 17, 8, 70): "fanout",
     (7, 21, 6, 4104, 345): "wide fanout", (5, 10, 7, 7168, 1799): "wide fanout", (9, 18, 2, 24, 700): "by entry",
+    # two and eight entries ranked per pass, in one, two and nine passes, ids in registers and past them
+    (9, 36, 11, 2056, 400): "wide fanout", (9, 36, 11, 4104, 130): "wide fanout", (9, 18, 6, 2056, 700): "wide fanout",
+    (9, 90, 70, 4104, 60): "wide fanout", (9, 90, 70, 2056, 20): "wide fanout", (9, 36, 11, 520, 400): "fanout", (9, 90, 70, 24, 20): "fanout",
     (4, 8, 1, 7167, 100): "few", (4, 8, 1, 7167, 300): "by entry", (8, 16, 4, 4097, 60): "few", (8, 16, 4, 4097, 100): "by entry",
     (16, 32, 8, 2049, 120): "by entry", (8, 64, 1, 7168, 500): "few", (2, 4, 1, 2304, 728): "by entry"}
 
