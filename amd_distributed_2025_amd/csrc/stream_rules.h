@@ -50,7 +50,7 @@ int few_keys(long long entries) {
 //
 // Longer streams go to the kernel that ranks four tokens in one pass over the keys, but for two kinds of short ones, where
 // a pass is little beside the rows and the others store them faster: fewer than four entries per token up to
-// 1280 of them (600 tokens of 14 KB, 2 per token 6.2 / 6.4 us), and long rows as long as a pass over the keys is short
+// 1280 of them (600 tokens of 14 KB, 2 per token 6.2 / 6.4 us), with one entry per token further (stays_by_entry), and long rows as long as a pass over the keys is short
 // beside the rows of a token, which the tokens and the vectors of a row measure: the others / that kernel 8 per token of 14 KB, 1024
 // tokens 26.2 / 27.8, 1400 34.3 / 36.9, 1800 43.7 / 48.9, 4096 118.9 / 102.5; 4 of 10 KB, 1000 tokens 10.7 / 11.1, 1500
 // 16.2 / 16.3; 6 of 13.7 KB, 600 tokens 12.0 / 13.0; but 3 of 9.2 KB, 500 tokens 5.6 / 5.4, and rows moved by elements 18.1 /
@@ -60,6 +60,16 @@ int few_keys(long long entries) {
 // all of the token's slots (measured at K = 8, H = 7168: 8.4 us against 8.8 us with a wave per
 // entry; one chunk per workgroup beats two or four). With one or two entries per token the
 // wave-per-entry kernel scans fewer keys per byte moved.
+// With one entry per token a wave per entry only scans what lies ahead in the stream, where the other kernel's passes take 2048 keys.
+// Behind the first pass that is ahead up to 3000 entries, before its end on rows of 4 to 10 KB (shorter ones leave it idle, and of longer
+// ones the scan is little), on elements up to 2700. us, a wave per entry / four tokens in a pass: 1967 tokens of 5.8 KB 5.5 / 6.2, 2303 of 4.9
+// KB 6.6 / 7.6, 2440 of 768 bytes 5.3 / 5.6, 2862 of 3.7 KB 6.8 / 7.3, 2067 of 1452 elements 7.6 / 8.5; but 1823 of 1.4 KB 4.5 / 4.2, 1326
+// of 16 KB 9.1 / 8.7, 3642 of 1.2 KB 6.9 / 6.7, 3735 of 7.4 KB 11.3 / 10.2.
+bool stays_by_entry(long long entries, int row_vecs, bool vec16) {
+  if (!vec16) return entries <= 2700;
+  return entries <= 3000 && row_vecs <= 640 && (entries > 2048 || row_vecs > 256);
+}
+
 SendWay send_way(long long tokens, int per_token, int ranks, int row_vecs, bool vec16) {
   const long long entries = tokens * per_token;
   const int pieces = (row_vecs + BLOCK - 1) / BLOCK;
@@ -68,7 +78,7 @@ SendWay send_way(long long tokens, int per_token, int ranks, int row_vecs, bool 
     if (vec16 && per_token >= FANOUT_MIN_K) return SEND_FEW;
     return tokens * pieces * few_keys(entries) <= (vec16 ? 16000 : 12000) ? SEND_FEW : SEND_BY_ENTRY;
   }
-  const bool few_entries = per_token < FANOUT_MIN_K && entries <= 1280;
+  const bool few_entries = (per_token < FANOUT_MIN_K && entries <= 1280) || (per_token == 1 && stays_by_entry(entries, row_vecs, vec16));
   const bool long_rows = per_token >= FANOUT_MIN_K && vec16 && row_vecs > 2 * BLOCK && tokens <= 3ll * row_vecs;
   if (entries > 0 && entries <= BLOCK_MAX_ENTRIES && ranks <= BLOCK_RANKS && per_token * ROWS <= 64 && !few_entries && !long_rows)
     return SEND_BLOCK;
@@ -80,9 +90,13 @@ SendWay send_way(long long tokens, int per_token, int ranks, int row_vecs, bool 
 // Vectors per lane of a wave of dispatch_block_kernel, for rows that a wave has in one go with `nvw`. Rows
 // are cut into pieces of two vectors per lane where there are few workgroups otherwise, else of four: pieces of 2 / 4 /
 // whole rows: 250 tokens of 5.8 KB, 8 per token 4.8 / 5.1 / 5.5 us, 1440 of 7.4 KB, 4 per token 11.6 / 12.3 / 12.1, 4096 of
-// 14 KB, 8 per token 129 / 102 / 106. With one entry a piece would do little but rank: 2000 of 14 KB 13.4 / 10.7 / 9.6.
+// 14 KB, 8 per token 129 / 102 / 106. With one entry a piece would do little but rank: 2000 of 14 KB 13.4 / 10.7 / 9.6. Two and three
+// entries pay for a piece of long rows only, two for one of four vectors: 1292 of 5 KB, 2 per token 7.1 / 6.6 / 5.9, 1380 of 15 KB 14.0 /
+// 12.6 / 12.4, 1001 of 13.7 KB 8.5 / 8.0 / 9.2, 671 of 10.8 KB 6.1 / 5.5 / 5.8; 893 of 4.5 KB, 3 per token 6.1 / 5.5 / 5.3, 537 of 13.6 KB
+// 6.5 / 7.0 / 7.2.
 int block_piece(long long tokens, int per_token, int nvw, bool vec16) {
-  if (!vec16 || per_token == 1) return nvw;
+  if (!vec16 || per_token == 1 || (per_token < FANOUT_MIN_K && nvw <= 8)) return nvw;
+  if (per_token == 2) return std::min(nvw, 4);
   return std::min(nvw, (tokens + ROWS - 1) / ROWS <= 400 ? 2 : 4);
 }
 

@@ -31,18 +31,20 @@ CASES = {
     (8, 16, 1, 8, 1281): ("block", 1, 1), (1, 3, 3, 24, 427): ("block", 1, 1), (8, 64, 4, 64, 257): ("block", 1, 1),
     (2, 2, 1, 1000, 1282): ("block", 2, 1), (8, 256, 8, 520, 1023): ("block", 2, 1), (3, 15, 5, 1032, 410): ("block", 2, 2),
     (5, 10, 3, 4104, 700): ("block", 2, 5), (4, 4, 1, 1032, 1290): ("block", 4, 1), (8, 88, 2, 2048, 1601): ("block", 4, 1),
-    (4, 8, 4, 4104, 1601): ("block", 4, 3), (8, 16, 2, 7168, 1605): ("block", 4, 4), (2, 4, 1, 2056, 1300): ("block", 6, 1),
-    (8, 8, 1, 4096, 1300): ("block", 8, 1), (3, 3, 1, 6144, 1285): ("block", 12, 1), (2, 4, 1, 7168, 1301): ("block", 14, 1),
+    (4, 8, 4, 4104, 1601): ("block", 4, 3), (8, 16, 2, 7168, 1605): ("block", 4, 4), (2, 4, 1, 2056, 3001): ("block", 6, 1),
+    (8, 8, 1, 4096, 3007): ("block", 8, 1), (3, 3, 1, 6144, 1285): ("block", 12, 1), (2, 4, 1, 7168, 1301): ("block", 14, 1),
     (2, 2, 1, 8192, 1283): ("block", 16, 1), (2, 2, 1, 8200, 1282): ("block", 16, 2),
-    (2, 6, 16, 37, 66): ("block", 16, 1), (4, 8, 5, 2051, 300): ("block", 16, 3), (2, 4, 1, 3001, 1290): ("block", 16, 3),  # single elements
-    (8, 8, 8, 16, 4096): ("block", 1, 1), (4, 32, 4, 8, 16320): ("block", 1, 1),
+    (2, 6, 16, 37, 66): ("block", 16, 1), (4, 8, 5, 2051, 300): ("block", 16, 3), (2, 4, 1, 3001, 2710): ("block", 16, 3),  # single elements
+    (8, 16, 2, 2560, 700): ("block", 6, 1), (4, 8, 2, 4096, 661): ("block", 8, 1), (2, 4, 2, 7168, 650): ("block", 4, 4),
+    (8, 16, 3, 3072, 501): ("block", 6, 1), (8, 8, 8, 16, 4096): ("block", 1, 1), (4, 32, 4, 8, 16320): ("block", 1, 1),
     (4, 32, 4, 8, 16321): "fanout", (9, 18, 4, 8, 400): "fanout", (8, 32, 17, 8, 70): "fanout",
     (7, 21, 6, 4104, 345): "wide fanout", (5, 10, 7, 7168, 1799): "wide fanout", (9, 18, 2, 24, 700): "by entry",
     # two and eight entries ranked per pass, in one, two and nine passes, ids in registers and past them
     (9, 36, 11, 2056, 400): "wide fanout", (9, 36, 11, 4104, 130): "wide fanout", (9, 18, 6, 2056, 700): "wide fanout",
     (9, 90, 70, 4104, 60): "wide fanout", (9, 90, 70, 2056, 20): "wide fanout", (9, 36, 11, 520, 400): "fanout", (9, 90, 70, 24, 20): "fanout",
     (4, 8, 1, 7167, 100): "few", (4, 8, 1, 7167, 300): "by entry", (8, 16, 4, 4097, 60): "few", (8, 16, 4, 4097, 100): "by entry",
-    (16, 32, 8, 2049, 120): "by entry", (8, 64, 1, 7168, 500): "few", (2, 4, 1, 2304, 728): "by entry"}
+    (16, 32, 8, 2049, 120): "by entry", (8, 64, 1, 7168, 500): "few", (2, 4, 1, 2304, 728): "by entry",
+    (8, 16, 1, 2304, 3000): "by entry", (2, 4, 1, 5120, 1281): "by entry", (8, 16, 1, 72, 2049): "by entry", (8, 16, 1, 517, 2700): "by entry"}
 
 
 @pytest.mark.parametrize("W,E,K,H,T", CASES)
