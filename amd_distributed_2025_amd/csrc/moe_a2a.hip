@@ -5613,8 +5613,10 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
       sources(LocalSources<R>{}))
 #define LAUNCH_T(V, DI, DO, R, KEYS, NV)                                                                   \
   do {                                                                                                     \
+    /* (rows cut for several vectors per lane are 1 MB and more) */                                        \
+    constexpr Store SMALL = NV > 1 ? THROUGH_OF<V> : PLAIN;                                                \
     if (through) LAUNCH_H(V, DI, DO, THROUGH_OF<V>, R, KEYS, NV);                                          \
-    else LAUNCH_H(V, DI, DO, PLAIN, R, KEYS, NV);                                                          \
+    else LAUNCH_H(V, DI, DO, SMALL, R, KEYS, NV);                                                          \
   } while (0)
 #define LAUNCH_S(V, R, KEYS, NV)                                                                           \
   do {                                                                                                     \

@@ -149,3 +149,12 @@ def test_vectors_of_a_lane_that_were_fastest(rules, W, T, K, H, lanes):
     """Timed on the GPU, of one, two, four and eight: the fastest or within a tenth of it."""
     vecs, vec16, _ = row(H)
     assert rules.lanes(W * T, W * T * K, W, vecs, vec16) == lanes
+
+
+def test_lanes_that_move_several_vectors_have_stores_for_a_megabyte_and_more(rules):
+    """(there are no others: they store past L2)"""
+    for W in (1, 2, 8):
+        for K in (1, 2, 8):
+            for vecs in (256, 257, 300, 512, 513, 896, 1025, 4096):
+                least = next((T for T in range(W, 2048 // K + 1) if rules.lanes(T, T * K, W, vecs, 1) > 1), None)
+                assert least is None or least * K * vecs * 16 >= 1 << 20, (W, K, vecs)
