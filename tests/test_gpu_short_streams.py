@@ -120,6 +120,7 @@ RECV_CASES = {
     (7168, 580, 580, "padded"): "few, plain", (7168, 600, 600, "padded"): "scan, through", (7168, 1024, 1024, "compact"): "scan, through",
     (7168, 700, 600, "padded"): "scan, through", (7168, 590, 800, "compact"): "scan, through", (8200, 600, 600, "padded"): "few, plain",
     (72, 1025, 1025, "padded"): "scan, through", (2049, 512, 512, "padded"): "few, plain", (2049, 513, 513, "padded"): "scan, plain",
+    (264, 4097, 4097, "padded"): "scan, through", (512, 4096, 4096, "compact"): "scan, through", (512, 5003, 5003, "compact"): "scan, through",
     (2049, 513, 513, "compact"): "few, plain", (1001, 1024, 1024, "padded"): "few, plain", (3001, 900, 700, "padded"): "scan, plain"}
 
 
@@ -146,6 +147,11 @@ def test_kernels_of_stage_2(hidden, rows, hint, layout):
         assert torch.equal(x, buf[torch.from_numpy(mine)]) and np.array_equal(m, meta[mine]), le
         at += len(mine)
     order = np.lexsort((np.arange(rows), expert, source))
+    assert torch.equal(back_counts, counts) and np.array_equal(back_meta[:rows].cpu().numpy(), meta[order])
+    assert torch.equal(back[:rows].cpu().view(torch.int16), buf[torch.from_numpy(order)])
+    # (of other tensors: by a scan)
+    back.zero_(), back_meta.zero_()
+    back_counts, back, back_meta = a.combine_send(em.clone(), ex.clone(), num.clone())
     assert torch.equal(back_counts, counts) and np.array_equal(back_meta[:rows].cpu().numpy(), meta[order])
     assert torch.equal(back[:rows].cpu().view(torch.int16), buf[torch.from_numpy(order)])
 
