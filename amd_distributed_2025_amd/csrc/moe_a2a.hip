@@ -3777,9 +3777,10 @@ __global__ __launch_bounds__(512, 1) void phased_gemm_kernel(
 
 // ---------------------------------------------------------------- exchange stand-in
 
+// (ArgumentsLoaded: nothing waits for these arguments that the counts would not be waited for as well. A leg of 64 rows of 1 KB 2.12 / 2.01 us.)
 template <typename V, int NV, Store HOW>
 __global__ __launch_bounds__(BLOCK) void exchange_local_kernel(
-    const V* __restrict__ send_buf, const int* __restrict__ send_meta,
+    ArgumentsLoaded, const V* __restrict__ send_buf, const int* __restrict__ send_meta,
     const int* __restrict__ send_counts, int dst_rank, V* __restrict__ recv_buf,
     int* __restrict__ recv_meta, const int* __restrict__ recv_counts, int src_rank, int row_vecs,
     int chunks, int send_capacity_rows, int recv_capacity_rows) {
@@ -5504,7 +5505,7 @@ int moe_a2a_exchange_local(int32_t world_size, int32_t hidden_dim, const void* s
   hipStream_t st = (hipStream_t)stream;
 #define LAUNCH_H(V, NV, HOW)                                                                  \
   exchange_local_kernel<V, NV, HOW><<<grid, BLOCK, 0, st>>>(                                  \
-      (const V*)send_buf, send_meta, send_counts, dst_rank, (V*)recv_buf, recv_meta,          \
+      ArgumentsLoaded{}, (const V*)send_buf, send_meta, send_counts, dst_rank, (V*)recv_buf, recv_meta,          \
       recv_counts, src_rank, g.row_vecs, g.chunks, send_capacity_rows, recv_capacity_rows)
 #define LAUNCH(V, NV)                                    \
   do {                                                   \
