@@ -3866,6 +3866,10 @@ constexpr int LOCAL_MAX_RANKS = 64;
 constexpr int LOCAL_MAX_EXPERTS = 1024;     // counters of the plan in LDS
 constexpr int LOCAL_MAX_K = 64;             // entries of a token, one per lane
 constexpr int LOCAL_FEW_RANKS = 8;          // a table that a wave holds in scalar registers
+// Up to here in a launch. Picking costs each wave some fifty scalar instructions, which many short waves take longer for than for the
+// dependent load that lanes of other waves hide: us, job's way back with compares / loads by rank, 4792 tokens of 512 bytes, 2 per token 8.49 /
+// 8.03, 7944 of 640 bytes, 5 each 17.7 / 16.6, 2256 of 768 bytes, 3 each 5.97 / 5.63; planned dispatch of 18768 of 512 bytes 35.0 / 33.8.
+constexpr int LOCAL_FEW_WORKGROUPS = 2048;
 constexpr int LOCAL_RANK_BITS = 11;
 constexpr int LOCAL_RANK_ENTRIES = 1 << LOCAL_RANK_BITS;  // 32 keys per lane of a wave
 
@@ -5710,7 +5714,7 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
   // (one rank: nothing to pick from. us, planned, with a table of eight / one: 13694 tokens of 1.2 KB 19.2 / 15.4, 5452 of 2019
   // elements, 2 each, 22.5 / 19.3, 1753 of 6.5 KB, 2 each 10.4 / 9.9)
   if (W == 1) launch(sources(LocalSources<1>{}));
-  else if (W <= LOCAL_FEW_RANKS) launch(sources(LocalSources<LOCAL_FEW_RANKS>{}));
+  else if (W <= LOCAL_FEW_RANKS && tokens * g.chunks <= LOCAL_FEW_WORKGROUPS) launch(sources(LocalSources<LOCAL_FEW_RANKS>{}));
   else launch(sources(LocalSources<LOCAL_MAX_RANKS>{}));
   return launch_status();
 }
@@ -5759,6 +5763,7 @@ int moe_a2a_local_combine(const moe_a2a_shape* s, const void* expert_rows, const
   if (!items_fit(items, chunks)) return MOE_A2A_EINVAL;
   const int grid = (int)(items * chunks);
   hipStream_t st = (hipStream_t)stream;
+  const bool few_ranks = W <= LOCAL_FEW_RANKS && grid <= LOCAL_FEW_WORKGROUPS;
 #define LAUNCH_R(V, DT, NV, MANY, R)                                                                       \
   local_combine_kernel<V, DT, NV, MANY, R><<<grid, BLOCK, 0, st>>>(                                        \
       entry_row, weights[0], (const V*)expert_rows, out_tokens[0], K, chunks, g.row_vecs, first, accumulate, W, \
@@ -5766,7 +5771,7 @@ int moe_a2a_local_combine(const moe_a2a_shape* s, const void* expert_rows, const
 #define LAUNCH(V, DT, NV, MANY)                                                                            \
   do {                                                                                                     \
     if (W == 1) LAUNCH_R(V, DT, NV, MANY, 1);                                                              \
-    else if (W <= LOCAL_FEW_RANKS) LAUNCH_R(V, DT, NV, MANY, LOCAL_FEW_RANKS);                             \
+    else if (few_ranks) LAUNCH_R(V, DT, NV, MANY, LOCAL_FEW_RANKS);                                        \
     else LAUNCH_R(V, DT, NV, MANY, LOCAL_MAX_RANKS);                                                       \
   } while (0)
 #define PICK(V, DT)                                                                                        \

@@ -94,6 +94,8 @@ def test_combine_of_other_tensors_takes_the_halves():
     (1, 32, 12, 264, [300], None), (3, 9, 2, 7168, [11, 1, 40], None),
     # ranked by the mover: experts with more entries than room, ids outside the range, up to 2048 entries and just above
     (1, 4, 4, 264, [64], "twins"), (2, 16, 4, 72, [60, 50], "twins"), (8, 64, 8, 520, [32] * 8, "ids"),
+    # tables of up to eight ranks up to 2048 workgroups, and behind
+    (8, 16, 2, 64, [257] * 8, None), (2, 4, 2, 72, [1024, 1024], "ids"), (3, 9, 1, 101, [900, 249, 1000], None),
     (8, 64, 8, 64, [32] * 7 + [33], None), (7, 63, 9, 96, [32, 1, 60, 7, 33, 64, 30], None),
 ])
 def test_custom_kernel_matches_the_halves(W, E, K, H, tokens, spoil, din, dout):
