@@ -40,6 +40,16 @@ int few_keys(long long entries) {
 
 // `row_vecs`: vectors of 16 bytes in a row, or its elements where those cannot be used (vec16).
 //
+// With one entry per token a wave per entry only scans what lies ahead in the stream, where the other kernel's passes take 2048 keys.
+// Behind the first pass that is ahead up to 3000 entries, before its end on rows of 4 to 10 KB (shorter ones leave it idle, and of longer
+// ones the scan is little), on elements up to 2700. us, a wave per entry / four tokens in a pass: 1967 tokens of 5.8 KB 5.5 / 6.2, 2303 of 4.9
+// KB 6.6 / 7.6, 2440 of 768 bytes 5.3 / 5.6, 2862 of 3.7 KB 6.8 / 7.3, 2067 of 1452 elements 7.6 / 8.5; but 1823 of 1.4 KB 4.5 / 4.2, 1326
+// of 16 KB 9.1 / 8.7, 3642 of 1.2 KB 6.9 / 6.7, 3735 of 7.4 KB 11.3 / 10.2.
+bool stays_by_entry(long long entries, int row_vecs, bool vec16) {
+  if (!vec16) return entries <= 2700;
+  return entries <= 3000 && row_vecs <= 640 && (entries > 2048 || row_vecs > 256);
+}
+
 // Up to 1024 entries every wave holds all keys. That costs each workgroup, which moves a piece of 256 vectors, as many loads and
 // compares as there are keys per lane, and pays up to about 16000 of them over all pieces, 12000 where a vector is one
 // element. Beyond (many tokens with long rows and few entries) a wave per entry is ahead; only tokens with four and more
@@ -54,22 +64,15 @@ int few_keys(long long entries) {
 // beside the rows of a token, which the tokens and the vectors of a row measure: the others / that kernel 8 per token of 14 KB, 1024
 // tokens 26.2 / 27.8, 1400 34.3 / 36.9, 1800 43.7 / 48.9, 4096 118.9 / 102.5; 4 of 10 KB, 1000 tokens 10.7 / 11.1, 1500
 // 16.2 / 16.3; 6 of 13.7 KB, 600 tokens 12.0 / 13.0; but 3 of 9.2 KB, 500 tokens 5.6 / 5.4, and rows moved by elements 18.1 /
-// 10.2 (6 of 4111, 500 tokens).
+// 10.2 (6 of 4111, 500 tokens). Rows of 7 KB (6.4 of seven entries) are long in that sense beyond 4096 entries, where the others rank eight at a
+// time: 8 per token of 8 KB, 997 tokens 15.0 / 16.9, 1518 23.0 / 26.0, 5 per token, 919 10.5 / 11.8, 8 of 7.7 KB, 953 14.1 / 16.1, 7 of 6.7 KB, 648
+// 9.0 / 10.0; but 399 of 8 KB, 8 per token 8.2 / 7.8, and not with four entries (1156 of 7 KB 11.4 / 10.1), of which
+// rows of more than 4 KB up to 2048 of them: 492 tokens of 4.5 KB 4.4 / 4.7, 509 of 8 KB 4.8 / 5.4; but 523 of 5.1 KB 5.7 / 5.2.
 //
 // The others: tokens with several entries have one workgroup per (token, 256-vector chunk) that stores the chunk to
 // all of the token's slots (measured at K = 8, H = 7168: 8.4 us against 8.8 us with a wave per
 // entry; one chunk per workgroup beats two or four). With one or two entries per token the
 // wave-per-entry kernel scans fewer keys per byte moved.
-// With one entry per token a wave per entry only scans what lies ahead in the stream, where the other kernel's passes take 2048 keys.
-// Behind the first pass that is ahead up to 3000 entries, before its end on rows of 4 to 10 KB (shorter ones leave it idle, and of longer
-// ones the scan is little), on elements up to 2700. us, a wave per entry / four tokens in a pass: 1967 tokens of 5.8 KB 5.5 / 6.2, 2303 of 4.9
-// KB 6.6 / 7.6, 2440 of 768 bytes 5.3 / 5.6, 2862 of 3.7 KB 6.8 / 7.3, 2067 of 1452 elements 7.6 / 8.5; but 1823 of 1.4 KB 4.5 / 4.2, 1326
-// of 16 KB 9.1 / 8.7, 3642 of 1.2 KB 6.9 / 6.7, 3735 of 7.4 KB 11.3 / 10.2.
-bool stays_by_entry(long long entries, int row_vecs, bool vec16) {
-  if (!vec16) return entries <= 2700;
-  return entries <= 3000 && row_vecs <= 640 && (entries > 2048 || row_vecs > 256);
-}
-
 SendWay send_way(long long tokens, int per_token, int ranks, int row_vecs, bool vec16) {
   const long long entries = tokens * per_token;
   const int pieces = (row_vecs + BLOCK - 1) / BLOCK;
@@ -79,7 +82,9 @@ SendWay send_way(long long tokens, int per_token, int ranks, int row_vecs, bool 
     return tokens * pieces * few_keys(entries) <= (vec16 ? 16000 : 12000) ? SEND_FEW : SEND_BY_ENTRY;
   }
   const bool few_entries = (per_token < FANOUT_MIN_K && entries <= 1280) || (per_token == 1 && stays_by_entry(entries, row_vecs, vec16));
-  const bool long_rows = per_token >= FANOUT_MIN_K && vec16 && row_vecs > 2 * BLOCK && tokens <= 3ll * row_vecs;
+  const bool long_rows = per_token >= FANOUT_MIN_K && vec16 && tokens <= 3ll * row_vecs &&
+                         (row_vecs > 2 * BLOCK || (per_token > 4 && row_vecs >= (per_token > 6 ? 400 : 448) && entries > 4096) ||
+                          (per_token == 4 && row_vecs > BLOCK && entries <= 2048));
   if (entries > 0 && entries <= BLOCK_MAX_ENTRIES && ranks <= BLOCK_RANKS && per_token * ROWS <= 64 && !few_entries && !long_rows)
     return SEND_BLOCK;
   if (per_token >= FANOUT_MIN_K && (ranks + 2ll) * entries <= INT_MAX && items_fit(tokens, pieces))

@@ -44,6 +44,7 @@ CASES = {
     (9, 90, 70, 4104, 60): "wide fanout", (9, 90, 70, 2056, 20): "wide fanout", (9, 36, 11, 520, 400): "fanout", (9, 90, 70, 24, 20): "fanout",
     (4, 8, 1, 7167, 100): "few", (4, 8, 1, 7167, 300): "by entry", (8, 16, 4, 4097, 60): "few", (8, 16, 4, 4097, 100): "by entry",
     (16, 32, 8, 2049, 120): "by entry", (8, 64, 1, 7168, 500): "few", (2, 4, 1, 2304, 728): "by entry",
+    (8, 16, 4, 2304, 400): "wide fanout", (4, 16, 8, 4096, 520): "wide fanout", (8, 16, 8, 4096, 400): ("block", 2, 4),
     (8, 16, 1, 2304, 3000): "by entry", (2, 4, 1, 5120, 1281): "by entry", (8, 16, 1, 72, 2049): "by entry", (8, 16, 1, 517, 2700): "by entry"}
 
 
