@@ -115,7 +115,8 @@ bool streams_far_ahead(long long rows_hint, int groups, int N) {
 // where those are too many, and from 56 rows on of dense_gemm_kernel, on 64 x 64 and then 64 x 128 (of which nearly a unit's worth pays
 // from 40 rows on). With more tiles the kernel that streams the weights looks four steps ahead up to two blocks per unit and is as fast
 // or faster. Beyond, where it does not, walks of K that are long beside the start of a ring are ahead: of 48 steps with up to three
-// tiles per unit (between three and four the last round is nearly empty), of 24 with five or more, on 32 x 64 up to 24 rows per group
+// tiles per unit (just above that the last round, of two tiles on a unit, is nearly empty), of 24 with five or more, of 32 with just under
+// two (few rows in many groups: 36 in 78, 960 x 2496 31.1 / 26.2 on 32 x 64, 12 in 61, 2528 x 2400 30.6 / 25.7), on 32 x 64 up to 24 rows per group
 // and on 64 x 64 up to 44: tiles of 32 rows would there read most groups' weights twice, under skewed routing (a group of 300 rows
 // in ten tiles) and uniform routing alike. us, the others / 32 x 32 / 32 x 64 / 64 x 64 / 64 x 128 (rows, groups, N x K):
 //    1 each in 5 of 41, 576 x 3520  19.8 / 10.5 / 12.3 / 15.0 / 22.2     9, 43, 2240 x 2752          123 / 92.4 / 86.5 / 88.7 / 110
@@ -153,7 +154,8 @@ RingTile grouped_ring(long long rows_hint, int groups, int N, int K) {
   if (far_ahead) return rows > 24 && of_64 >= 0.75 && of_64 <= 0.95 ? RING_64x64 : NO_RING;
   if (rows > 24 && of_64 <= 2) return RING_64x64;
   const double tiles = rows <= 24 ? of_32 : of_64;
-  const bool long_walk = (steps >= 24 && tiles >= 5) || (steps >= 48 && (tiles < 3 || tiles >= 4));
+  const bool long_walk = (steps >= 24 && tiles >= 5) || (steps >= 48 && (tiles < 3 || tiles >= (rows <= 24 ? 3.5 : 4.0))) ||
+                         (steps >= 32 && tiles <= 1.9);
   if (rows > 44 || !long_walk) return NO_RING;
   return rows <= 24 ? RING_32x64 : RING_64x64;
 }

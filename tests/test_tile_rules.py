@@ -201,6 +201,7 @@ def test_rings_that_the_gpu_tests_mean(rules, tile):
     (368, 8, 1024, 3648, 2), (1704, 48, 512, 2432, 3), (858, 6, 960, 2400, 3), (1379, 7, 832, 6528, 4), (468, 9, 2304, 5568, 4),
     (144, 64, 1024, 2048, 0), (144, 64, 2048, 1024, 0), (118, 53, 2240, 512, 0), (2792, 41, 512, 640, 0), (2468, 48, 1856, 1184, 0),
     (320, 8, 7168, 7168, 0), (224, 8, 7168, 1536, 0), (32, 8, 7168, 2048, 0), (1280, 32, 2048, 1536, 0), (128, 32, 2048, 2880, 0),
+    (14, 55, 2048, 2816, 2), (36, 78, 960, 2496, 2), (12, 61, 2528, 2400, 2), (20, 31, 2368, 2560, 0), (35, 24, 5376, 7136, 2), (154, 70, 928, 2336, 0),
     (8192, 32, 2048, 4096, 0), (0, 3, 7168, 200, 1), (7, 48, 832, 1 << 23, 0),
     (4, 44, 1728, 8, 0), (275, 11, 512, 216, 1), (285, 5, 2816, 8, 0), (480, 10, 896, 360, 0),
 ])
