@@ -86,9 +86,6 @@ template <typename V> constexpr Store THROUGH_OF = sizeof(V) == sizeof(b128) ? T
 #ifndef MOE_A2A_STORE_CSEND  /* stage 3 -> send-back buffer */
 #define MOE_A2A_STORE_CSEND STREAM
 #endif
-#ifndef MOE_A2A_NT_LOAD
-#define MOE_A2A_NT_LOAD 0
-#endif
 template <Store HOW, typename V>
 __device__ __forceinline__ void row_store(V* p, const V& v) {
   if constexpr (HOW == STREAM) __builtin_nontemporal_store(v, p);
@@ -96,13 +93,11 @@ __device__ __forceinline__ void row_store(V* p, const V& v) {
     __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) b128*)p, v, "agent");
   else *p = v;
 }
-template <typename P>
-__device__ __forceinline__ auto stream_load(P p) {
-#if MOE_A2A_NT_LOAD
-  return __builtin_nontemporal_load(p);
-#else
-  return *p;
-#endif
+// PAST: nontemporal, for rows of streams that the caches do not hold (csrc/stream_rules.h).
+template <bool PAST, typename P>
+__device__ __forceinline__ auto row_load(P p) {
+  if constexpr (PAST) return __builtin_nontemporal_load(p);
+  else return *p;
 }
 
 // ---------------------------------------------------------------- wave / block primitives
@@ -251,6 +246,13 @@ __device__ __forceinline__ void dest_class(int e, int nle, int E, uint32_t magic
   }
 }
 
+// Rows cut into `per_row` pieces each; pieces are numbered along the stream.
+struct Pieces {
+  int per_row;
+  uint32_t magic, shift;  // q / per_row of 0 <= q < 2^31 is the high word of q * magic, shifted
+  __device__ __forceinline__ int row_of(int q) const { return per_row == 1 ? q : (int)(__umulhi((uint32_t)q, magic) >> shift); }
+};
+
 // NV vectors of one row chunk held in registers. Loads are unconditional
 // (lanes past the end of the row re-read its last vector), so all of them are
 // in flight at once; only the stores are predicated.
@@ -259,7 +261,7 @@ struct Payload {
   V v[NV];
   __device__ __forceinline__ void load(const V* __restrict__ row, int base, int row_vecs) {
 #pragma unroll
-    for (int j = 0; j < NV; ++j) v[j] = stream_load(row + min(base + j * BLOCK + (int)threadIdx.x, row_vecs - 1));
+    for (int j = 0; j < NV; ++j) v[j] = row[min(base + j * BLOCK + (int)threadIdx.x, row_vecs - 1)];
   }
   template <Store HOW>
   __device__ __forceinline__ void store(V* __restrict__ row, int base, int row_vecs) const {
@@ -332,10 +334,10 @@ struct StridedKeys {
 template <typename V, int NVW>
 struct WavePayload {
   V v[NVW];
-  template <typename P>  // const V* or global_ptr<V>
+  template <bool PAST = false, typename P>  // const V* or global_ptr<V>
   __device__ __forceinline__ void load(P row, int base, int row_vecs, int lane) {
 #pragma unroll
-    for (int j = 0; j < NVW; ++j) v[j] = stream_load(row + min(base + j * 64 + lane, row_vecs - 1));
+    for (int j = 0; j < NVW; ++j) v[j] = row_load<PAST>(row + min(base + j * 64 + lane, row_vecs - 1));
   }
   template <Store HOW>
   __device__ __forceinline__ void store(V* __restrict__ row, int base, int row_vecs, int lane) const {
@@ -683,7 +685,7 @@ __global__ __launch_bounds__(BLK) void dispatch_fanout_wide_kernel(
     for (int u = 0; u < KEYS; ++u) key[u] = indices[min(tid + u * BLK, S - 1)];
     V v[NV];
 #pragma unroll
-    for (int j = 0; j < NV; ++j) v[j] = stream_load(x + (size_t)t * row_vecs + min(col + j * BLK, row_vecs - 1));
+    for (int j = 0; j < NV; ++j) v[j] = x[(size_t)t * row_vecs + min(col + j * BLK, row_vecs - 1)];
 
     for (int g0 = 0; g0 < K; g0 += FAN) {
       // (a later group waits for its ids inside the branch: a wait at the place where the two paths
@@ -816,7 +818,7 @@ __global__ __launch_bounds__(BLOCK) void dispatch_few_kernel(
   const int i0 = t * K, col = c * BLOCK + tid;
   const int own = indices[i0 + min(lane, K - 1)];
   fetch();
-  const V v = stream_load(x + (size_t)t * row_vecs + min(col, row_vecs - 1));
+  const V v = x[(size_t)t * row_vecs + min(col, row_vecs - 1)];
 #pragma unroll
   for (int u = 0; u < KEYS; ++u)
     key[u] = lane + u * 64 < S ? composite(key[u], lane + u * 64) : INT_MAX;
@@ -1167,17 +1169,11 @@ __global__ __launch_bounds__(RPLAN_BLOCK) void plan_recv_kernel(
   }
 }
 
-// How a mover finds the place of a row:
-//   RECV_SCAN     by counting the earlier rows of the same expert (the padded layout of
-//                 all2all/reference.py:127-136: row pos of expert le at le * max_recv + pos);
-//   RECV_POS      from `row_pos` (plan_recv_kernel): the movers scan nothing (padded layout);
-//   RECV_COMPACT  the compact layout: the experts' rows back to back, row pos of expert le at
-//                 offset[le] + pos with offset = exclusive prefix of the rows per expert. A row's
-//                 place is then the number of rows of lower experts anywhere in the stream plus
-//                 the earlier rows of its own expert (one pass over all keys); `max_recv` is the
-//                 number of rows the compact buffers hold, and the counting workgroups also write
-//                 the offsets.
-enum { RECV_SCAN = 0, RECV_POS = 1, RECV_COMPACT = 2 };
+// COMPACT: the compact layout, the experts' rows back to back, row pos of expert le at offset[le] + pos with offset =
+// exclusive prefix of the rows per expert (padded: row pos of expert le at le * max_recv + pos, all2all/reference.py:127-136).
+// A row's place is then the number of rows of lower experts anywhere in the stream plus the earlier rows of its own
+// expert (one pass over all keys); `max_recv` is the number of rows the compact buffers hold, and the counting
+// workgroups also write the offsets.
 
 // A workgroup that plans expert blockIdx.x: its rows, where every source's run of them starts inside the expert and in the
 // send-back stream, and in the compact layout where the expert starts.
@@ -1250,14 +1246,33 @@ __device__ __forceinline__ void plan_expert(
   }
 }
 
-template <typename V, int NVW, bool PLAN, int MODE, Store HOW, bool SHORT>
+// A workgroup that only counts the rows of expert blockIdx.x. `red` is ROWS ints of LDS.
+template <bool COMPACT>
+__device__ __forceinline__ void count_expert(
+    const int* __restrict__ recv_meta, const int* __restrict__ recv_counts, int W, int nle, int capacity_rows, uint32_t magic,
+    int* red, int* __restrict__ expert_num_tokens, int* __restrict__ expert_offsets) {
+  const StridedKeys key{recv_meta, META};
+  const int R = min(sum_counts(recv_counts, W, capacity_rows), capacity_rows);
+  const int me = blockIdx.x, tid = threadIdx.x;
+  int c = count_keys<64 * ROWS>(R, key, [=](int e, int) { return floormod(e, nle, magic) == me; });
+  c = block_sum<ROWS>(c, red);
+  if (tid == 0) expert_num_tokens[me] = c;
+  if constexpr (COMPACT) {
+    int lower = count_keys<64 * ROWS>(R, key, [=](int e, int) { return floormod(e, nle, magic) < me; });
+    lower = block_sum<ROWS>(lower, red);
+    if (tid == 0) {
+      expert_offsets[me] = lower;
+      if (me == nle - 1) expert_offsets[nle] = lower + c;
+    }
+  }
+}
+
+template <typename V, int NVW, bool PLAN, bool COMPACT, Store HOW, bool SHORT>
 __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
     const V* __restrict__ recv_buf, const int* __restrict__ recv_meta,
     const int* __restrict__ recv_counts, int W, int hint_rows, int movers, int chunks, int row_vecs, int nle,
     int capacity_rows, uint32_t magic, int max_recv, int* __restrict__ expert_num_tokens,
-    V* __restrict__ expert_x, int* __restrict__ expert_meta, int* __restrict__ plan,
-    const int* __restrict__ row_pos, int* __restrict__ expert_offsets) {
-  constexpr bool POS = MODE == RECV_POS, COMPACT = MODE == RECV_COMPACT;
+    V* __restrict__ expert_x, int* __restrict__ expert_meta, int* __restrict__ plan, int* __restrict__ expert_offsets) {
   constexpr int UNROLL = HOW == PLAIN ? 4 : SCAN_UNROLL;  // (PLAIN: up to 1024 rows of elements, or of more than 64 experts)
   __shared__ int part[2 * ROWS * ROWS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -1272,19 +1287,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
   }
 
   if ((int)blockIdx.x < nle) {
-    const int R = min(sum_counts(recv_counts, W, capacity_rows), capacity_rows);
-    const int me = blockIdx.x;
-    int c = count_keys<64 * ROWS>(R, key, [=](int e, int) { return floormod(e, nle, magic) == me; });
-    c = block_sum<ROWS>(c, part);
-    if (tid == 0) expert_num_tokens[me] = c;
-    if constexpr (COMPACT) {
-      int lower = count_keys<64 * ROWS>(R, key, [=](int e, int) { return floormod(e, nle, magic) < me; });
-      lower = block_sum<ROWS>(lower, part);
-      if (tid == 0) {
-        expert_offsets[me] = lower;
-        if (me == nle - 1) expert_offsets[nle] = lower + c;
-      }
-    }
+    count_expert<COMPACT>(recv_meta, recv_counts, W, nle, capacity_rows, magic, part, expert_num_tokens, expert_offsets);
     return;
   }
 
@@ -1296,22 +1299,6 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
     const int i0 = grp * ROWS, i = i0 + wave;
     const int ic = min(i, limit - 1);
     const int base = c * (64 * NVW);
-
-    if constexpr (POS) {
-      const int e = recv_meta[(size_t)ic * META];
-      const int pos = row_pos[ic];
-      int m = 0;
-      if (c == 0 && lane < META) m = recv_meta[(size_t)ic * META + lane];
-      WavePayload<V, NVW> p;
-      p.load(recv_buf + (size_t)ic * row_vecs, base, row_vecs, lane);
-      const int R = rows_known();
-      if (i < R && (uint32_t)pos < (uint32_t)max_recv) {
-        const size_t row = (size_t)floormod(e, nle, magic) * max_recv + pos;
-        p.template store<HOW>(expert_x + row * row_vecs, base, row_vecs, lane);
-        if (c == 0 && lane < META) expert_meta[row * META + lane] = m;
-      }
-      return R;
-    }
 
     int re[ROWS];
 #pragma unroll
@@ -1376,6 +1363,56 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
   }
   const int items = (R + ROWS - 1) / ROWS * chunks;
   for (; q < items; q += movers) move(q, R, [&] { return R; });
+}
+
+// The movers of a long stream, with the positions that plan_recv_kernel left: a wave per piece of 64 * NVW vectors of a row, in
+// the order of the stream. Memory bounds it, and what shaped it is how few places of the streams are open at a time (planned_recv_vecs and
+// RECV_PAST_BYTES, csrc/stream_rules.h): 32768 rows of 14 KB 160 us with a workgroup on the same piece of four rows and plain loads of four
+// vectors, 137 here (6.9 TB/s); with a stage before and behind it 12000 rows of 4 KB 53.6 / 47.0.
+template <typename V, int NVW, bool PLAN, Store HOW, bool PAST>
+__global__ __launch_bounds__(64 * ROWS) void dispatch_recv_planned_kernel(
+    const int* __restrict__ recv_meta, const int* __restrict__ row_pos, const int* __restrict__ recv_counts,
+    const V* __restrict__ recv_buf, int W, int hint_rows, int movers, Pieces pieces, int row_vecs, int nle, int capacity_rows,
+    uint32_t magic, int max_recv, V* __restrict__ expert_x, int* __restrict__ expert_meta,
+    int* __restrict__ expert_num_tokens, int* __restrict__ plan) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if ((int)blockIdx.x < nle) {
+    if constexpr (PLAN) {
+      plan_expert<false, SCAN_UNROLL>(recv_meta, recv_counts, W, hint_rows, nle, capacity_rows, magic, expert_num_tokens, plan,
+                                      nullptr);
+    } else {
+      __shared__ int red[ROWS];
+      count_expert<false>(recv_meta, recv_counts, W, nle, capacity_rows, magic, red, expert_num_tokens, nullptr);
+    }
+    return;
+  }
+  const bool lanes_hold_counts = W <= 64;
+  const int raw_count = recv_counts[min(lane, W - 1)];
+  int R = -1;  // not known yet
+  auto rows = [&] {
+    const int my_count = lane < W ? min(max(first_use(raw_count), 0), capacity_rows) : 0;
+    return min(lanes_hold_counts ? wave_sum(my_count) : sum_counts(recv_counts, W, capacity_rows), capacity_rows);
+  };
+  for (int q = ((int)blockIdx.x - nle) * ROWS + wave;; q += movers * ROWS) {
+    const int i = pieces.row_of(q), c = q - i * pieces.per_row, base = c * (64 * NVW);
+    if (R >= 0 || i >= hint_rows) {  // (rows below the hint can be read before the count is known)
+      if (R < 0) R = rows();
+      if (i >= R) return;
+    }
+    const int e = recv_meta[(size_t)i * META], pos = row_pos[i];
+    int m = 0;
+    if (c == 0 && lane < META) m = recv_meta[(size_t)i * META + lane];
+    WavePayload<V, NVW> p;
+    p.template load<PAST>(unknown_origin(recv_buf + (size_t)i * row_vecs), base, row_vecs, lane);
+    issued_here();
+    if (R < 0) R = rows();
+    if (i >= R) return;
+    if ((uint32_t)pos < (uint32_t)max_recv) {
+      const size_t row = (size_t)floormod(e, nle, magic) * max_recv + pos;
+      p.template store<HOW>(expert_x + row * row_vecs, base, row_vecs, lane);
+      if (c == 0 && lane < META) expert_meta[row * META + lane] = m;
+    }
+  }
 }
 
 // The same for a short stream: every wave ranks a row of its own against all keys it needs (KEYS per lane, the fewest that
@@ -1613,7 +1650,7 @@ struct WaveStreamKeys {
 // buffers when no expert overflowed max_recv; if one did, every workgroup sees
 // it in the counts and takes the scan instead.
 
-template <typename V, int NVW, bool SMALL, bool PLAN, typename... Loaded>
+template <typename V, int NVW, bool SMALL, bool PLAN, bool PAST, typename... Loaded>
 __global__ __launch_bounds__(64 * ROWS) void combine_send_kernel(
     Loaded..., const int* __restrict__ expert_num_tokens, const int* __restrict__ plan,
     const int* __restrict__ expert_meta, const V* __restrict__ expert_y, int nle, int W, int chunks, int max_recv,
@@ -1661,7 +1698,7 @@ __global__ __launch_bounds__(64 * ROWS) void combine_send_kernel(
         int m = 0;
         if (c == 0 && lane < META) m = expert_meta[row * META + lane];
         WavePayload<V, NVW> p;
-        p.load(unknown_origin(expert_y + row * row_vecs), base, row_vecs, lane);
+        p.template load<PAST>(unknown_origin(expert_y + row * row_vecs), base, row_vecs, lane);
         // (the row is only used by the stores below, which depend on the slot: without this the
         // compiler moves the loads down behind the plan's round trip)
         issued_here();
@@ -2220,8 +2257,9 @@ __global__ __launch_bounds__(BLOCK) void expert_scale_kernel(
 
 // The same for at most 64 local experts and 16-byte vectors: a wave per (row,
 // chunk of 64 * NVW vectors), the expert prefix in one register per lane, the
-// row found with one ballot. No LDS table, no barrier.
-template <int NVW, int DIN, int DOUT, Store HOW>
+// row found with one ballot. No LDS table, no barrier. Long streams take two vectors per lane and nontemporal loads (PAST; EXPERT_PAST_BYTES,
+// csrc/stream_rules.h): 470 MB of rows among the other stages 170 -> 153 us, 29 MB 13.4 -> 12.8 (between events).
+template <int NVW, int DIN, int DOUT, Store HOW, bool PAST>
 __global__ __launch_bounds__(64 * ROWS) void expert_scale_wave_kernel(
     const b128* __restrict__ expert_x, const int* __restrict__ expert_num_tokens, int nle,
     int max_recv, float scale, int row_vecs, int chunks, b128* __restrict__ expert_y, int compact_rows) {
@@ -2236,7 +2274,7 @@ __global__ __launch_bounds__(64 * ROWS) void expert_scale_wave_kernel(
     wp.locate(g, le, first);
     const size_t row = compact_rows > 0 ? (size_t)g : (size_t)le * max_recv + (g - first);
     WavePayload<b128, NVW> p;
-    p.load(expert_x + row * row_vecs, base, row_vecs, lane);
+    p.template load<PAST>(expert_x + row * row_vecs, base, row_vecs, lane);
 #pragma unroll
     for (int j = 0; j < NVW; ++j) p.v[j] = standin_expert<b128, DIN, DOUT>(p.v[j], scale);
     p.template store<HOW>(expert_y + row * row_vecs, base, row_vecs, lane);
@@ -4436,9 +4474,16 @@ int launch_status() { return hipGetLastError() == hipSuccess ? MOE_A2A_OK : MOE_
     }                                             \
   } while (0)
 
-#ifndef MOE_A2A_PLANNED_NVW
-#define MOE_A2A_PLANNED_NVW 4  // vectors per lane of a mover that scans nothing
-#endif
+Pieces pieces_of(int per_row) {
+  Pieces p{per_row, 0, 0};
+  if (per_row > 1) {
+    int bits = 1;  // per_row <= 1 << bits
+    while ((1ll << bits) < per_row) ++bits;
+    p.magic = (uint32_t)((1ull << (31 + bits)) / (uint32_t)per_row + 1);
+    p.shift = bits - 1;
+  }
+  return p;
+}
 
 // The send-back plan is kept by the lanes of one wave: one lane per source rank
 // in stage 2, one lane per local expert in stage 3.
@@ -4665,9 +4710,9 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   hipStream_t st = (hipStream_t)stream;
   const bool planned = send_back_plan && plan_supported(s);
   if (row_position && g.nle <= RPLAN_MAX_EXPERTS && capacity_rows > 0) {
-    // no scan to repeat per chunk: a row is split among more waves, as in the planned stage 3
-    if (g.vec16 && g.nvw > MOE_A2A_PLANNED_NVW) {
-      g.nvw = MOE_A2A_PLANNED_NVW;
+    // no scan to repeat per piece: a row is split among more waves, as in the planned stage 3
+    if (g.vec16) {
+      g.nvw = planned_recv_vecs(g.row_vecs);
       g.wchunks = (g.row_vecs + 64 * g.nvw - 1) / (64 * g.nvw);
     }
     if (!items_fit((long long)g.nle * g.max_recv, g.wchunks)) return MOE_A2A_EINVAL;
@@ -4676,12 +4721,23 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
     while ((1 << expert_bits) < g.nle) ++expert_bits;
     plan_recv_kernel<<<tiles, RPLAN_BLOCK, 0, st>>>(recv_meta, recv_counts, s->world_size, rows_hint,
                                                     capacity_rows, g.nle, g.magic, expert_bits, row_position);
-    const int grid = g.nle + mover_blocks(group_items(rows_hint, g));
-#define LAUNCH_P(V, NVW, PLAN)                                                              \
-  dispatch_recv_kernel<V, NVW, PLAN, RECV_POS, THROUGH, false><<<grid, 64 * ROWS, 0, st>>>( \
-      (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, grid - g.nle,    \
-      g.wchunks, g.row_vecs, g.nle, capacity_rows, g.magic, g.max_recv, expert_num_tokens,   \
-      (V*)expert_x, expert_meta, send_back_plan, row_position, nullptr)
+    const int movers = mover_blocks(((long long)rows_hint * g.wchunks + ROWS - 1) / ROWS);
+    const bool past = (long long)rows_hint * s->hidden_dim * 2 >= RECV_PAST_BYTES;
+#define LAUNCH_L(V, NVW, PLAN, PAST)                                                                           \
+  dispatch_recv_planned_kernel<V, NVW, PLAN, THROUGH, PAST><<<g.nle + movers, 64 * ROWS, 0, st>>>(             \
+      recv_meta, row_position, recv_counts, (const V*)recv_buf, s->world_size, rows_hint, movers,              \
+      pieces_of(g.wchunks), g.row_vecs, g.nle, capacity_rows, g.magic, g.max_recv, (V*)expert_x, expert_meta,  \
+      expert_num_tokens, send_back_plan)
+#define LAUNCH_P(V, NVW, PLAN)                        \
+  do {                                                \
+    if constexpr (sizeof(V) == sizeof(b128)) {        \
+      if (past) {                                     \
+        LAUNCH_L(V, NVW, PLAN, true);                 \
+        break;                                        \
+      }                                               \
+    }                                                 \
+    LAUNCH_L(V, NVW, PLAN, false);                    \
+  } while (0)
 #define LAUNCH(V, NVW)                     \
   do {                                     \
     if (planned) LAUNCH_P(V, NVW, true);   \
@@ -4689,10 +4745,10 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   } while (0)
     if (!g.vec16) LAUNCH(uint16_t, 16);
     else if (g.nvw == 1) LAUNCH(b128, 1);
-    else if (g.nvw == 2) LAUNCH(b128, 2);
-    else LAUNCH(b128, 4);
+    else LAUNCH(b128, 2);
 #undef LAUNCH
 #undef LAUNCH_P
+#undef LAUNCH_L
     return launch_status();
   }
   // the stream can hold at most nle * max_recv rows that fit the expert buffers
@@ -4734,30 +4790,30 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   }
   const int grid = g.nle + mover_blocks(group_items(rows_hint, g));
   const bool through = recv_through(rows_hint, 2ll * s->hidden_dim);  // (Store)
-#define LAUNCH_S(V, NVW, PLAN, MODE, HOW, SHORT)                                            \
-  dispatch_recv_kernel<V, NVW, PLAN, MODE, HOW, SHORT><<<grid, 64 * ROWS, 0, st>>>(         \
+#define LAUNCH_S(V, NVW, PLAN, COMPACT, HOW, SHORT)                                         \
+  dispatch_recv_kernel<V, NVW, PLAN, COMPACT, HOW, SHORT><<<grid, 64 * ROWS, 0, st>>>(      \
       (const V*)recv_buf, recv_meta, recv_counts, s->world_size, rows_hint, grid - g.nle,    \
       g.wchunks, g.row_vecs, g.nle, capacity_rows, g.magic,                                  \
       compact_rows > 0 ? compact_rows : g.max_recv,                                          \
-      expert_num_tokens, (V*)expert_x, expert_meta, send_back_plan, nullptr, expert_offsets)
-#define LAUNCH_P(V, NVW, PLAN, MODE)                                                        \
+      expert_num_tokens, (V*)expert_x, expert_meta, send_back_plan, expert_offsets)
+#define LAUNCH_P(V, NVW, PLAN, COMPACT)                                                        \
   do {                                                                                      \
     /* (planned rows of vectors that come here are more than 1024, or 8 MB of 14 per lane,  \
        a workgroup per unit: recv_few) */                                                   \
-    constexpr bool VECTORS = PLAN && sizeof(V) == sizeof(b128), SHORT = MODE == RECV_SCAN;  \
+    constexpr bool VECTORS = PLAN && sizeof(V) == sizeof(b128), SHORT = !COMPACT;           \
     constexpr bool SHORT_FEW = SHORT && !(VECTORS && NVW == 14);                            \
-    if (!through) LAUNCH_S(V, NVW, PLAN, MODE, (VECTORS ? THROUGH : PLAIN), SHORT);         \
-    else if (rows_hint > FEW_ENTRIES) LAUNCH_S(V, NVW, PLAN, MODE, THROUGH, SHORT);         \
-    else LAUNCH_S(V, NVW, PLAN, MODE, THROUGH, SHORT_FEW);                                  \
+    if (!through) LAUNCH_S(V, NVW, PLAN, COMPACT, (VECTORS ? THROUGH : PLAIN), SHORT);         \
+    else if (rows_hint > FEW_ENTRIES) LAUNCH_S(V, NVW, PLAN, COMPACT, THROUGH, SHORT);         \
+    else LAUNCH_S(V, NVW, PLAN, COMPACT, THROUGH, SHORT_FEW);                                  \
   } while (0)
 #define LAUNCH(V, NVW)                                         \
   do {                                                         \
     if (compact_rows > 0) {                                    \
-      if (planned) LAUNCH_P(V, NVW, true, RECV_COMPACT);       \
-      else LAUNCH_P(V, NVW, false, RECV_COMPACT);              \
+      if (planned) LAUNCH_P(V, NVW, true, true);               \
+      else LAUNCH_P(V, NVW, false, true);                      \
     } else {                                                   \
-      if (planned) LAUNCH_P(V, NVW, true, RECV_SCAN);          \
-      else LAUNCH_P(V, NVW, false, RECV_SCAN);                 \
+      if (planned) LAUNCH_P(V, NVW, true, false);              \
+      else LAUNCH_P(V, NVW, false, false);                     \
     }                                                          \
   } while (0)
   MOE_A2A_FOR_WAVE_KERNEL(g, LAUNCH);
@@ -4829,11 +4885,12 @@ int launch_combine_send(const moe_a2a_shape* s, const void* expert_y, const int3
     g.max_recv = compact_rows;  // no expert has more rows than the buffers hold
   }
   const bool planned = send_back_plan && plan_supported(s);
-  // The planned path has no scan to repeat per chunk, so a row can be split among more waves:
-  // 4 vectors per lane (a 256-vector chunk per wave) made the whole step 0.5 us shorter at
-  // H = 7168 than the 14 the scan path uses; 2, 6 and 8 were no better than 14.
-  if (planned && g.vec16 && g.nvw > MOE_A2A_PLANNED_NVW) {
-    g.nvw = MOE_A2A_PLANNED_NVW;
+  // (the planned path has no scan to repeat per piece, so a row can be split among more waves)
+  const long long stream_bytes = (long long)rows_hint * s->hidden_dim * 2;
+  const bool past = stream_bytes >= EXPERT_PAST_BYTES;
+  const int planned_nvw = planned_send_vecs(stream_bytes, g.row_vecs);
+  if (planned && g.vec16 && g.nvw > planned_nvw) {
+    g.nvw = planned_nvw;
     g.wchunks = (g.row_vecs + 64 * g.nvw - 1) / (64 * g.nvw);
   }
   if (!items_fit(compact_rows > 0 ? (long long)compact_rows : (long long)g.nle * g.max_recv, g.wchunks))
@@ -4842,23 +4899,33 @@ int launch_combine_send(const moe_a2a_shape* s, const void* expert_y, const int3
   hipStream_t st = (hipStream_t)stream;
   // (ArgumentsLoaded) Rows of up to 1 KB, a wave each. us with arguments in registers / loaded: 5056 rows of 512 bytes 3.67 / 3.29, 35928
   // of 512 14.0 / 12.8, 32102 of 1 KB 16.3 / 15.1, its scan 391 / 372; some 3000 the same, fewer are better off with registers.
-#define LAUNCH_A(V, NVW, SMALL, PLAN, ...)                                                     \
+#define LAUNCH_A(V, NVW, SMALL, PLAN, PAST, ...)                                               \
   do {                                                                                         \
-    auto kernel = combine_send_kernel<V, NVW, SMALL, PLAN __VA_OPT__(,) __VA_ARGS__>;          \
+    auto kernel = combine_send_kernel<V, NVW, SMALL, PLAN, PAST __VA_OPT__(,) __VA_ARGS__>;    \
     kernel<<<grid, 64 * ROWS, 0, st>>>(                                                        \
         __VA_OPT__(__VA_ARGS__{},) expert_num_tokens, send_back_plan, expert_meta,             \
         (const V*)expert_y, g.nle, s->world_size, g.wchunks, g.max_recv, compact_rows,         \
         g.row_vecs, capacity_rows, (V*)send_buf, send_meta, send_counts);                      \
   } while (0)
-#define LAUNCH_S(V, NVW, SMALL, PLAN)                                                          \
+#define LAUNCH_R(V, NVW, SMALL, PLAN, PAST)                                                    \
   do {                                                                                         \
     if constexpr (NVW == 1) {                                                                  \
       if (rows_hint > LOADED_MIN_ROWS) {                                                       \
-        LAUNCH_A(V, NVW, SMALL, PLAN, ArgumentsLoaded);                                        \
+        LAUNCH_A(V, NVW, SMALL, PLAN, PAST, ArgumentsLoaded);                                  \
         break;                                                                                 \
       }                                                                                        \
     }                                                                                          \
-    LAUNCH_A(V, NVW, SMALL, PLAN);                                                             \
+    LAUNCH_A(V, NVW, SMALL, PLAN, PAST);                                                       \
+  } while (0)
+#define LAUNCH_S(V, NVW, SMALL, PLAN)                                                          \
+  do {                                                                                         \
+    if constexpr (PLAN && sizeof(V) == sizeof(b128) && NVW <= 8) {                             \
+      if (past) {                                                                              \
+        LAUNCH_R(V, NVW, SMALL, PLAN, true);                                                   \
+        break;                                                                                 \
+      }                                                                                        \
+    }                                                                                          \
+    LAUNCH_R(V, NVW, SMALL, PLAN, false);                                                      \
   } while (0)
 #define LAUNCH(V, NVW)                                   \
   do {                                                   \
@@ -4869,6 +4936,7 @@ int launch_combine_send(const moe_a2a_shape* s, const void* expert_y, const int3
   MOE_A2A_FOR_WAVE_KERNEL(g, LAUNCH);
 #undef LAUNCH
 #undef LAUNCH_S
+#undef LAUNCH_R
 #undef LAUNCH_A
   return launch_status();
 }
@@ -5046,18 +5114,27 @@ int launch_expert_scale(const moe_a2a_shape* s, const void* expert_x, const int3
 #define MOE_A2A_SCALE_WAVES 1
 #endif
   if (MOE_A2A_SCALE_WAVES && g.vec16 && g.nle <= 64) {
-    const int nvw = g.nvw < 4 ? g.nvw : 4;  // 1, 2 or 4 vectors per lane
+    const long long stream_bytes = (long long)rows_hint * s->hidden_dim * 2;
+    const bool past = stream_bytes >= EXPERT_PAST_BYTES;
+    const int nvw = std::min(g.nvw, past ? 2 : 4);  // 1, 2 or 4 vectors per lane
     const int wchunks = (g.row_vecs + 64 * nvw - 1) / (64 * nvw);
     if (!items_fit(most_rows, wchunks)) return MOE_A2A_EINVAL;
     const int wgrid = mover_blocks(((long long)rows_hint * wchunks + ROWS - 1) / ROWS);
-#define LAUNCH_WH(NVW, DI, DO, HOW)                                                            \
-  expert_scale_wave_kernel<NVW, DI, DO, HOW><<<wgrid, 64 * ROWS, 0, st>>>(                     \
+#define LAUNCH_WH(NVW, DI, DO, HOW, PAST)                                                      \
+  expert_scale_wave_kernel<NVW, DI, DO, HOW, PAST><<<wgrid, 64 * ROWS, 0, st>>>(                     \
       (const b128*)expert_x, expert_num_tokens, g.nle, g.max_recv, scale, g.row_vecs, wchunks,  \
       (b128*)expert_y, compact_rows)
 #define LAUNCH_WT(NVW, DI, DO)                                                                 \
   do {                                                                                         \
-    if (through) LAUNCH_WH(NVW, DI, DO, THROUGH);                                              \
-    else LAUNCH_WH(NVW, DI, DO, PLAIN);                                                        \
+    if constexpr (NVW <= 2) {                                                                  \
+      if (past) {                                                                              \
+        if (stream_bytes >= EXPERT_STREAM_BYTES) LAUNCH_WH(NVW, DI, DO, STREAM, true);         \
+        else LAUNCH_WH(NVW, DI, DO, THROUGH, true);                                            \
+        break;                                                                                 \
+      }                                                                                        \
+    }                                                                                          \
+    if (through) LAUNCH_WH(NVW, DI, DO, THROUGH, false);                                       \
+    else LAUNCH_WH(NVW, DI, DO, PLAIN, false);                                                 \
   } while (0)
 #define LAUNCH_W(NVW)                                                                          \
   do {                                                                                         \

@@ -15,6 +15,32 @@ constexpr int ROWS = MOE_A2A_ROWS;    // rows (= waves) per workgroup of a ranke
 
 bool items_fit(long long rows, int chunks) { return rows * chunks <= INT_MAX / 2; }
 
+// ---------------------------------------------------------------- streams beyond the caches
+//
+// Streams that do not stay in L2 (32 MB) on their way from one stage to the next, nor in the 256 MB behind it, are bound by what memory
+// takes at a time. Rows of them are read with nontemporal loads, which push nothing of what is being written out of the caches, and
+// in small pieces along the stream, so that fewer places of it are open at once: a plain copy of 470 MB runs at 5.4 TB/s with 14 vectors per
+// lane, 5.7 with four, 6.1 with one, and 6.5 with nontemporal loads and one; of 28 MB, at 6.1 to 6.4 with any of them.
+// us of a graph of stages 1, 2, expert, 3 and 4, plain / nontemporal loads in one stage (8 entries per token, 14 KB but where said):
+//  - expert, four vectors per lane / two and nontemporal: 2.3 MB 17.8 / 17.8, 15 MB 29.9 / 30.0, 29 MB 49.5 / 47.0, 46 MB 78.8 / 74.3, 134
+//    MB of 4 KB 214 / 198, 235 MB 377 / 348, 470 MB 720 / 716 (its rows then fill the cache behind L2 for stage 3 to push out: below)
+//  - stage 3: 15 MB 29.7 / 30.2, 29 MB 47.2 / 47.0, 46 MB 72.1 / 71.0, 69 MB 99.8 / 98.3, 134 MB of 4 KB 193.9 / 189.0, 235 MB 340 / 329
+//  - stage 2, four vectors per lane / two / two and nontemporal: 29 MB 47.2 / 46.6 / 47.2, 46 MB - / 74.2 / 72.0, 69 MB 102.2 / 102.1 /
+//    101.1, 134 MB of 8 KB 196.0 / 194.2 / 192.7, 275 MB 395 / 393 / 378, 470 MB 682 / 676 / 663; of rows of up to 4 KB one vector per lane:
+//    134 MB of 4 KB, two / one 195.2 / 193.5, 67 MB of 2 KB 128.0 / 123.9, 16 MB of 2 KB 48.8 / 47.8.
+constexpr long long EXPERT_PAST_BYTES = 24ll << 20, RECV_PAST_BYTES = 40ll << 20;
+
+// The expert's results go past the cache behind L2 only where it could hold little of them, else through it (Store):
+// 134 MB 198 / 205, 268 MB 497 / 510, 336 MB 708 / 685 and, the other stages at their best, 658 / 664; 470 MB 716 / 682 and 649 / 637.
+constexpr long long EXPERT_STREAM_BYTES = 384ll << 20;
+
+int planned_recv_vecs(int row_vecs) { return row_vecs > BLOCK ? 2 : 1; }
+
+// Vectors per lane of a planned stage 3: four (a 256-vector piece per wave) made a whole step 0.5 us shorter at 2048 rows of 14 KB than the
+// 14 of the scan path; 2, 6 and 8 were no better than 14. Long rows beyond the cache take eight: 470 MB 660 / 654 us as above, 336 MB of 10 KB
+// 670 / 665, 275 MB 378 / 376, but 235 MB 329 / 331 and, a whole row in eight, 268 MB of 8 KB 485 / 497.
+int planned_send_vecs(long long bytes, int row_vecs) { return bytes >= 256ll << 20 && row_vecs > 2 * BLOCK ? 8 : 4; }
+
 // ---------------------------------------------------------------- stage 1
 
 constexpr int FANOUT_MIN_K = 4;

@@ -1,0 +1,72 @@
+"""Streams that the caches do not hold: rows read past them, in pieces of one, two, four or eight vectors per lane
+(`csrc/stream_rules.h`). Results are the ones of the other kernels, bit for bit."""
+import pytest
+import torch
+
+from amd_distributed_2025_amd import HIPAllToAll, _lib, generate_world
+from amd_distributed_2025_amd.task import MoEConfig
+from tests.test_gpu_long_streams import run_long
+from tests.test_gpu_parity import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+# rows of each stream: 42 to 49 MB, above the lines of the expert, of stage 3 and of stage 2
+@pytest.mark.parametrize("hidden_dim,tokens,K,dtype", [
+    (1032, 2560, 8, "bf16"),   # 129 vectors: a piece of one vector, one lane of it used
+    (2048, 2816, 4, "fp16"),   # 256: whole pieces of one
+    (2056, 2816, 4, "bf16"),   # 257: pieces of two, and one lane of the last
+    (4104, 704, 8, "fp16"),    # 513
+])
+def test_streams_of_more_than_40_mb(hidden_dim, tokens, K, dtype):
+    print(f"{tokens * K} rows of {hidden_dim}", flush=True)
+    assert tokens * K * hidden_dim * 2 > 40 << 20
+    spec = dict(world_size=2, num_experts=16, experts_per_token=K, hidden_dim=hidden_dim, max_num_tokens=tokens,
+                num_tokens="full", routing="uniform", weights="softmax", dtype=dtype)
+    run_long(generate_world(spec, 3), long_stream_rows=0)
+
+
+@pytest.mark.parametrize("hidden_dim", [8, 520, 1024, 1032, 4096, 4104, 7168])
+@pytest.mark.parametrize("layout", ["padded", "compact"])
+def test_a_few_rows_in_a_launch_for_hundreds_of_megabytes(hidden_dim, layout):
+    """The expert and stage 3 size their launches and choose their kernels by the caller's row count, which may lie above the
+    rows that there are: below and above 24, 256 and 384 MB the same rows give the same results."""
+    nle, tokens = 3, 37
+    cfg = MoEConfig(nle, 2, hidden_dim, tokens, torch.bfloat16, torch.bfloat16)
+    results = []
+    for megabytes in (0, 25, 300, 400):
+        a = HIPAllToAll(cfg, 0, 1, device=DEV, layout=layout, compact_rows=96 if layout == "compact" else None)
+        gen = torch.Generator(device=DEV)
+        gen.manual_seed(7)
+        rows = tokens * 2
+        hint = max(rows, (megabytes << 20) // (2 * hidden_dim))
+        recv = torch.randn(rows, hidden_dim, device=DEV, generator=gen).to(torch.bfloat16)
+        meta = torch.zeros(rows, 5, dtype=torch.int32, device=DEV)
+        meta[:, 0] = torch.arange(rows, device=DEV) * 7 % nle
+        meta[:, 2] = torch.arange(rows, device=DEV) // 2
+        meta[:, 3] = torch.arange(rows, device=DEV) % 2
+        counts = torch.tensor([rows], dtype=torch.int32, device=DEV)
+        num, ex, em = a.dispatch_recv(counts, recv, meta, rows)
+        ex_rows, plan = ex.shape[0], a._ws["send_back_plan"]
+        ey, back = torch.zeros_like(ex), torch.zeros_like(recv)
+        back_meta, back_counts = torch.zeros_like(meta), torch.zeros_like(counts)
+        p, st = _lib_pointer, torch.cuda.current_stream().cuda_stream
+        print(f"{layout}, {hidden_dim}, launches for {megabytes} MB", flush=True)
+        if layout == "compact":
+            _lib.call("moe_a2a_expert_scale_compact", a.shape, p(ex), p(num), hint, ex_rows, _lib.BF16, _lib.BF16, p(ey), st)
+            _lib.call("moe_a2a_combine_send_compact", a.shape, p(ey), p(em), p(num), hint, ex_rows, rows, p(back),
+                      p(back_meta), p(back_counts), p(plan), st)
+        else:
+            _lib.call("moe_a2a_expert_scale", a.shape, p(ex), p(num), hint, _lib.BF16, _lib.BF16, p(ey), st)
+            _lib.call("moe_a2a_combine_send", a.shape, p(ey), p(em), p(num), hint, rows, p(back), p(back_meta), p(back_counts),
+                      p(plan), st)
+        torch.cuda.synchronize()
+        order = torch.argsort(meta[:, 0], stable=True)
+        assert torch.equal(back, recv[order]) and torch.equal(back_meta, meta[order])  # (rank 0: times one)
+        results.append((ey, back_counts))
+    for ey, back_counts in results[1:]:
+        assert torch.equal(ey, results[0][0]) and torch.equal(back_counts, results[0][1])
+
+
+def _lib_pointer(t):
+    return t.data_ptr()
