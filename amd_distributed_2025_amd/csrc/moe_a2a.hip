@@ -2107,6 +2107,88 @@ __global__ __launch_bounds__(BLK) void combine_recv_kernel(
   }
 }
 
+// Stage 4 of a long stream with its table (return_map_kernel), for up to eight entries per token: a wave per (token, piece
+// of 64 * NV vectors), with nothing to wait for but its own loads. Lane k (and those 8, 16, .. on) holds entry k: the rows that the
+// table names are ordered by arrival and asked for while the meta rows that say whether they are the token's are on their way. Memory
+// bounds it, on short rows the two dependent trips. us with the launch that makes the table, a workgroup of 256 lanes per piece that takes
+// these steps one after the other with barriers between them / here: 2500 tokens of 2 KB, 1 per token 14.3 / 10.4, 1600 of 2 KB, 2 each 13.1 / 10.2,
+// 4096 of 8 KB, 2 each 34.3 / 24.5, 3 each 37.4 / 29.7, 4096 of 14 KB, 8 each 109.5 / 96.0 (5.8 TB/s).
+template <int DT, int NV, int ADDENDS, bool PAST>
+__global__ __launch_bounds__(BLOCK) void combine_recv_mapped_kernel(
+    const int* __restrict__ entry_row, const int* __restrict__ recv_counts, const float* __restrict__ weights,
+    const int* __restrict__ recv_meta, int W, int T, int K, Pieces pieces, int capacity_rows,
+    const b128* __restrict__ recv_buf, int row_vecs, int accumulate, b128* __restrict__ out) {
+  constexpr int N = Words<b128>::N, FAST = 8;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int items = T * pieces.per_row, waves = gridDim.x * NWAVES;
+  const int raw_count = recv_counts[min(lane, W - 1)];
+  int R = -1;
+  for (int q = blockIdx.x * NWAVES + wave; q < items; q += waves) {
+    const int t = pieces.row_of(q), base = (q - t * pieces.per_row) * (64 * NV);
+    const int k = lane & (FAST - 1), kc = min(k, K - 1);
+    const int i = entry_row[(size_t)t * K + kc];
+    const float w = weights[(size_t)t * K + kc];
+    b128* __restrict__ orow = out + (size_t)t * row_vecs;
+    PairAcc<DT> acc[NV][N];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      b128 o{};
+      if (accumulate) o = orow[min(base + j * 64 + lane, row_vecs - 1)];
+#pragma unroll
+      for (int e = 0; e < N; ++e) acc[j][e].set(get_word(o, e));
+    }
+    if (R < 0) {
+      const int my_count = lane < W ? min(max(first_use(raw_count), 0), capacity_rows) : 0;
+      R = min(W <= 64 ? wave_sum(my_count) : sum_counts(recv_counts, W, capacity_rows), capacity_rows);
+    }
+    const bool named = k < K && (uint32_t)i < (uint32_t)R;
+    int tk[2] = {-1, -1};
+    if (named) __builtin_memcpy(tk, recv_meta + (size_t)i * META + 2, 8);
+    // (as in combine_recv_kernel; a stale entry may name a row that another one names as well: the entry decides between them)
+    const uint32_t key = named ? (uint32_t)i << 3 | k : UINT_MAX;
+    int place = 0;
+#define MOE_A2A_ROT(S) place += (int)((uint32_t)__builtin_amdgcn_update_dpp(0, (int)key, 0x120 + S, 0xf, 0xf, false) < key)
+    MOE_A2A_ROT(1); MOE_A2A_ROT(2); MOE_A2A_ROT(3); MOE_A2A_ROT(4); MOE_A2A_ROT(5); MOE_A2A_ROT(6); MOE_A2A_ROT(7);
+#undef MOE_A2A_ROT
+    const int to = ((lane & ~(FAST - 1)) | place) << 2;
+    const int ordered_row = __builtin_amdgcn_ds_permute(to, i), ordered_w = __builtin_amdgcn_ds_permute(to, __float_as_int(w));
+    const int n = __popcll(__ballot(named) & 0xff);
+    b128 v[ADDENDS][NV];
+#pragma unroll
+    for (int u = 0; u < ADDENDS; ++u) {
+      if (u < n) {
+        const b128* row = recv_buf + (size_t)__builtin_amdgcn_readlane(ordered_row, u) * row_vecs;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) v[u][j] = row_load<PAST>(unknown_origin(row) + min(base + j * 64 + lane, row_vecs - 1));
+      }
+    }
+    issued_here();
+    // which of the ordered rows are addends: those whose meta row names this token and entry
+    const int ordered_ok = __builtin_amdgcn_ds_permute(to, (int)(named && tk[0] == t && tk[1] == k));
+    const unsigned long long ok = __ballot(ordered_ok != 0);
+#pragma unroll
+    for (int u = 0; u < ADDENDS; ++u) {
+      if (u < n && (ok >> u & 1)) {
+        const float wu = __int_as_float(__builtin_amdgcn_readlane(ordered_w, u));
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+          for (int e = 0; e < N; ++e) acc[j][e].step(get_word(v[u][j], e), wu);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int idx = base + j * 64 + lane;
+      if (idx < row_vecs) {
+        uint32_t h[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) h[e] = acc[j][e].word();
+        row_store<THROUGH>(orow + idx, from_words<b128>(h));
+      }
+    }
+  }
+}
+
 // The same for a short stream (hint_rows <= 64 * KEYS): every wave looks through all of it by itself. The rows of 64 keys
 // that are the token's come out of a ballot in arrival order, so there is nothing to sort and no other wave to wait for.
 // ADDENDS: rows under way at a time. us, one launch after another in a graph, before / here: 72 rows of 1 KB, 6 per token
@@ -4976,6 +5058,35 @@ int launch_combine_recv(const moe_a2a_shape* s, const void* recv_buf, const int3
     const int mgrid = (int)std::min<long long>(((long long)rows_hint + BLOCK - 1) / BLOCK + 1, 1 << 16);
     return_map_kernel<<<mgrid, BLOCK, 0, st>>>(recv_meta, recv_counts, W, rows_hint, capacity_rows,
                                                num_tokens, K, entry_row);
+  }
+  // Up to eight entries per token a wave has the rows of its piece in one go (combine_recv_mapped_kernel).
+  if (mapped && g.vec16 && K <= 8 && capacity_rows < 1 << 28) {
+    const bool past = ((long long)rows_hint + num_tokens) * s->hidden_dim * 2 >= COMBINE_PAST_BYTES;
+    const int mnv = mapped_vecs(K, g.row_vecs, past), pieces = (g.row_vecs + 64 * mnv - 1) / (64 * mnv);
+    if (items_fit(num_tokens, pieces)) {
+      const int fgrid = mover_blocks(((long long)num_tokens * pieces + NWAVES - 1) / NWAVES);
+#define LAUNCH_P(DT, NV, ADDENDS, PAST)                                                                          \
+  combine_recv_mapped_kernel<DT, NV, ADDENDS, PAST><<<fgrid, BLOCK, 0, st>>>(                                    \
+      entry_row, recv_counts, weights, recv_meta, W, num_tokens, K, pieces_of(pieces), capacity_rows,            \
+      (const b128*)recv_buf, g.row_vecs, accumulate, (b128*)out_tokens)
+#define LAUNCH_A(DT, NV, ADDENDS)                          \
+  do {                                                     \
+    if (past) LAUNCH_P(DT, NV, ADDENDS, true);             \
+    else LAUNCH_P(DT, NV, ADDENDS, false);                 \
+  } while (0)
+#define LAUNCH(DT)                                                                                               \
+  do {                                                                                                           \
+    if (K <= 2) { if (mnv == 2) LAUNCH_A(DT, 2, 2); else LAUNCH_A(DT, 1, 2); }                                   \
+    else if (K <= 4) { if (mnv == 2) LAUNCH_A(DT, 2, 4); else LAUNCH_A(DT, 1, 4); }                              \
+    else LAUNCH_A(DT, 1, 8);                                                                                     \
+  } while (0)
+      if (dtype == MOE_A2A_BF16) LAUNCH(MOE_A2A_BF16);
+      else LAUNCH(MOE_A2A_F16);
+#undef LAUNCH
+#undef LAUNCH_A
+#undef LAUNCH_P
+      return launch_status();
+    }
   }
   // Up to 512 rows every wave looks through the stream by itself (combine_recv_few_kernel); above that the waves share the
   // scan (601 rows of 8 KB: 4.17 us shared, 4.68 by each wave), with code for what there is of it up to 1024.

@@ -163,6 +163,16 @@ RecvFew recv_few(long long rows_hint, int row_vecs, int nvw, bool vec16, bool co
   return nvw == 14 ? RECV_NOT_FEW : pieces ? RECV_FEW_PLAIN : RECV_FEW_THROUGH;
 }
 
+// ---------------------------------------------------------------- stage 4
+
+// Vectors per lane of combine_recv_mapped_kernel, and whether it reads rows past the caches. One vector with more than two entries per token, or
+// four of a large stream: of fewer a wave has little to do but to find them. us of the graph of stages as above, one / two: 8 per token
+// of 14 KB, 69 MB 100.8 / 101.8; 4 of 5.8 KB, 18 MB 38.6 / 39.3; 3 of 8 KB, 20 MB 40.7 / 41.2, 101 MB 143.2 / 142.3; 2 of 8 KB, 67 MB 105.7 / 103.4; 1
+// of 8 KB, 34 MB 69.2 / 67.3. Plain / nontemporal loads (rows and results): 78 MB 100.8 / 101.4, 100 MB (2 per token) 111.4 / 103.4, 118 MB
+// 151.1 / 148.0, 134 MB 149.2 / 142.3, 528 MB 652.7 / 641.6; of 67 MB (1 per token) 67.3 / 65.7, of 52 MB 72.5 / 73.6.
+constexpr long long COMBINE_PAST_BYTES = 80ll << 20;
+int mapped_vecs(int per_token, int row_vecs, bool past) { return row_vecs > 64 && per_token <= (past ? 4 : 2) ? 2 : 1; }
+
 // ---------------------------------------------------------------- jobs on one GPU
 
 // Vectors of a row that a lane of local_dispatch_few_kernel moves: one, two or four, of single elements one, four or eight. Every
