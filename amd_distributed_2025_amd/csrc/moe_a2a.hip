@@ -954,6 +954,112 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_block_kernel(
   }
 }
 
+// The same for longer streams yet: a workgroup of sixteen waves owns `own_tokens` tokens (of at most 64 entries), so that fewer of them
+// pass over all keys, and its waves take pieces of 64 vectors of the tokens' rows in turn, along the stream, so that few places of
+// the send buffer are open at a time. What bounds it is the stores of the rows, of short ones the keys. us, dispatch_block_kernel /
+// here: 3090 tokens of 1.1 KB, 4 per token 13.5 / 8.8; 3123 of 1 KB, 2 each 9.9 / 6.8; 3630 of 1.5 KB, 8 each 24.8 / 19.4; 3554 of 8.6 KB, 2
+// each 21.4 / 18.0; 3001 of 12 KB, 5 each 42.9 / 38.7; 4096 of 14 KB, 8 each, behind the other stages, 118 / 111.
+template <bool POW2>
+__global__ __launch_bounds__(LONG_BLOCK) void dispatch_long_kernel(
+    const b128* __restrict__ x, const int* __restrict__ indices, int T, int K, int W, int own_tokens, Pieces pieces, int row_vecs,
+    int E, uint32_t magic, int nle_shift, int rank,
+    b128* __restrict__ send_buf, int* __restrict__ send_meta, int* __restrict__ send_counts,
+    int* __restrict__ send_slot) {
+  constexpr int KEYS = 8, BATCH = KEYS * LONG_BLOCK, WORDS = 4, NW = LONG_BLOCK / 64;
+  __shared__ int part[2 * WORDS][NW];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int S = T * K;
+  const int t0 = blockIdx.x * own_tokens, i0 = t0 * K, tokens = min(own_tokens, T - t0), own = tokens * K;  // (own <= 64)
+  auto klass = [&](int e) {
+    const int d = POW2 ? e >> nle_shift : (int)__umulhi((uint32_t)e, magic);
+    return (uint32_t)e >= (uint32_t)E ? BLOCK_RANKS : d;
+  };
+  const int mine = indices[i0 + min(lane, own - 1)];
+  int key[KEYS];
+  auto fetch = [&](int b) {
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) key[u] = indices[min(b + tid + u * LONG_BLOCK, S - 1)];
+  };
+  fetch(0);
+  issued_here();
+  const int items = tokens * pieces.per_row;
+  auto vector_of = [&](int q) {
+    const int tl = pieces.row_of(q), at = (q - tl * pieces.per_row) * 64 + lane;
+    return x[(size_t)(t0 + tl) * row_vecs + min(at, row_vecs - 1)];
+  };
+  b128 v{};
+  if (wave < items) v = vector_of(wave);
+
+  uint32_t ahead[2] = {}, others[2] = {};
+  auto count = [&](uint32_t (&n)[2], int b, int from, int to) {
+#pragma unroll
+    for (int u = 0; u < KEYS; ++u) {
+      const int i = b + tid + u * LONG_BLOCK;
+      const int d = (i >= from) & (i < to) ? klass(key[u]) : BLOCK_RANKS;
+      const uint32_t one = 1u << ((d & 3) * 8);
+      n[0] += d < 4 ? one : 0;
+      n[1] += (uint32_t)(d - 4) < 4u ? one : 0;
+    }
+  };
+  for (int b = 0; b < S; b += BATCH) {
+    if (b > 0) fetch(b);
+    if (b < i0) count(ahead, b, 0, i0);
+    if (b + BATCH > i0) count(others, b, i0, S);
+  }
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    const int a0 = wave_sum((int)(ahead[w] & 0x00ff00ffu)), a1 = wave_sum((int)((ahead[w] >> 8) & 0x00ff00ffu));
+    const int o0 = wave_sum((int)(others[w] & 0x00ff00ffu)), o1 = wave_sum((int)((others[w] >> 8) & 0x00ff00ffu));
+    if (lane == 0) {
+      part[w * 2][wave] = a0;
+      part[w * 2 + 1][wave] = a1;
+      part[WORDS + w * 2][wave] = o0;
+      part[WORDS + w * 2 + 1][wave] = o1;
+    }
+  }
+  lds_barrier();
+  const int word = (lane >> 2 & 1) * 2 + (lane & 1), half = (lane >> 1 & 1) * 16;
+  int before = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    before += part[word][w] >> half & 0xffff;
+    total += part[WORDS + word][w] >> half & 0xffff;
+  }
+  const bool is_rank = lane < W;
+  before = is_rank ? before : 0;
+  total = is_rank ? total + before : 0;
+  const int upto = wave_inclusive_scan(total), all_before = wave_inclusive_scan(before);
+  const int first = lane < BLOCK_RANKS ? upto - total + before : upto + i0 - all_before;
+  if (blockIdx.x == 0 && wave == 0 && is_rank) send_counts[lane] = total;
+  const int d = lane < own ? klass(mine) : -1;
+  int slot = __shfl(first, d < 0 ? 0 : d, 64);
+#pragma unroll
+  for (int r = 0; r <= BLOCK_RANKS; ++r) {
+    const unsigned long long same = __ballot(d == r);
+    slot += d == r ? __popcll(same & ((1ull << lane) - 1)) : 0;
+  }
+
+  for (int b = wave * 64; b < own * META; b += LONG_BLOCK) {
+    const int m = b + lane, k = min(m / META, own - 1), f = m - k * META;
+    const int to = __shfl(slot, k, 64), e = __shfl(mine, k, 64);
+    if (m < own * META) {
+      const int tl = k / K;
+      send_meta[(size_t)to * META + f] = f == 0 ? e : f == 1 ? rank : f == 2 ? t0 + tl : f == 3 ? k - tl * K : 0;
+      if (f == 0 && send_slot) send_slot[i0 + k] = to;
+    }
+  }
+  for (int q = wave; q < items;) {
+    const int tl = pieces.row_of(q), at = (q - tl * pieces.per_row) * 64 + lane;
+    const b128 out = v;
+    q += NW;
+    if (q < items) v = vector_of(q);
+    for (int k = 0; k < K; ++k) {
+      const int to = __builtin_amdgcn_readlane(slot, tl * K + k);
+      if (at < row_vecs) row_store<MOE_A2A_STORE_SEND>(send_buf + (size_t)to * row_vecs + at, out);
+    }
+  }
+}
+
 // ---------------------------------------------------------------- send plan (counts, offsets, maps)
 //
 // The stable counting sort of stage 1 made explicit, for callers that want the
@@ -4662,6 +4768,20 @@ int moe_a2a_dispatch_send(const moe_a2a_shape* s, const void* x, const int32_t* 
     else { if (f.vec16) LAUNCH(b128, false); else LAUNCH(uint16_t, false); }
 #undef LAUNCH
 #undef LAUNCH_K
+    return launch_status();
+  }
+  if (const int own = long_tokens(way, num_tokens, s->experts_per_token, s->world_size, g.row_vecs, g.vec16)) {
+    int nle_shift = 0;
+    while ((1 << nle_shift) < g.nle) ++nle_shift;
+    const int long_grid = (num_tokens + own - 1) / own;
+#define LAUNCH(POW2)                                                                             \
+  dispatch_long_kernel<POW2><<<long_grid, LONG_BLOCK, 0, st>>>(                                  \
+      (const b128*)x, indices, num_tokens, s->experts_per_token, s->world_size, own,             \
+      pieces_of((g.row_vecs + 63) / 64), g.row_vecs, s->num_experts, g.magic, nle_shift, s->rank, \
+      (b128*)send_buf, send_meta, send_counts, send_slot)
+    if ((g.nle & (g.nle - 1)) == 0) LAUNCH(true);
+    else LAUNCH(false);
+#undef LAUNCH
     return launch_status();
   }
   if (way == SEND_BLOCK) {

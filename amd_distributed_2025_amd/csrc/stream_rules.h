@@ -48,6 +48,8 @@ constexpr int FEW_ENTRIES = 64 * 16;
 constexpr int FEW_MAX_K = 64;            // a lane of the wave for each
 constexpr int BLOCK_RANKS = 8;
 constexpr int BLOCK_MAX_ENTRIES = 255 * BLOCK;  // keys that 256 lanes count in bytes
+constexpr int LONG_BLOCK = 1024;                // lanes of dispatch_long_kernel
+constexpr int LONG_ENTRIES = 5120, LONG_MAX_ENTRIES = 255 * LONG_BLOCK;
 
 enum SendWay {
   SEND_BY_ENTRY,     // dispatch_send_kernel
@@ -118,6 +120,24 @@ SendWay send_way(long long tokens, int per_token, int ranks, int row_vecs, bool 
   if (per_token >= FANOUT_MIN_K && (ranks + 2ll) * entries <= INT_MAX && items_fit(tokens, pieces))
     return row_vecs > BLOCK && entries < 65536 && ranks < 16384 ? SEND_FANOUT_WIDE : SEND_FANOUT;
   return SEND_BY_ENTRY;
+}
+
+// Tokens of a workgroup of dispatch_long_kernel, or 0 where a stream stays with its choice above. From 5120 entries on it takes whole vectors over from
+// dispatch_block_kernel, and from 65281 on from all others, which compare every key with every entry: over 288 streams of 5120 to 32768 entries, one to
+// eight per token, rows of 512 bytes to 14 KB, 0.90 of their time, 17 of them more than 3 % behind (2803 tokens of 1.9 KB, 6 per token
+// 14.75 / 16.6). Below it is behind: 4900 entries (613 tokens of 900 bytes) 6.2 / 6.4, 3100 (777 of 1.4 KB) 5.5 / 6.3.
+//
+// About one workgroup per unit where rows are short, which leaves the passes over the keys to the fewest, two where the rows take longer
+// than that. us, with 128 / 256 / 512 / 1024 workgroups: 3590 tokens of 1 KB, 3 per token 7.9 /
+// 8.0 / 11.2 / 15.1; 3649 of 1.5 KB, 5 each 14.4 (192) / 14.4 / 22.1 (912); 2803 of 1.9 KB, 6 each - / 16.6 / 15.1 / 23.1; 3554 of 8.6 KB, 2
+// each 18.1 / 18.0 / 18.0 / 19.6; 3001 of 12 KB, 5 each - / 41.2 / 39.9 / 38.7; 4096 of 14 KB, 8 each - / - / 113 / 111.
+int long_tokens(SendWay way, long long tokens, int per_token, int ranks, int row_vecs, bool vec16) {
+  const long long entries = tokens * per_token;
+  if (!vec16 || ranks > BLOCK_RANKS || per_token > 64 || entries < LONG_ENTRIES || entries > LONG_MAX_ENTRIES ||
+      (way != SEND_BLOCK && entries <= BLOCK_MAX_ENTRIES))
+    return 0;
+  const int workgroups = row_vecs <= 400 ? 256 : 512;
+  return (int)std::min<long long>(64 / per_token, (tokens + workgroups - 1) / workgroups);
 }
 
 // Vectors per lane of a wave of dispatch_block_kernel, for rows that a wave has in one go with `nvw`. Rows

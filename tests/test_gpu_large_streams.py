@@ -26,6 +26,38 @@ def test_streams_of_more_than_40_mb(hidden_dim, tokens, K, dtype):
     run_long(generate_world(spec, 3), long_stream_rows=0)
 
 
+@pytest.mark.parametrize("W,E,K,hidden_dim,tokens", [
+    (8, 16, 1, 8, 5120),     # the shortest it takes, one entry per token; a vector per row, 20 tokens a workgroup
+    (3, 15, 5, 520, 1024),   # 65 vectors, experts per rank no power of two
+    (2, 6, 6, 1032, 2561),   # 60 entries in a workgroup, the last of which owns one token
+    (8, 8, 7, 64, 2311),     # an expert per rank, nine tokens each
+    (4, 256, 64, 16, 81),    # a token per workgroup, with 64 entries
+    (5, 20, 3, 3208, 1800),  # 401 vectors: twice as many workgroups
+    (2, 4, 2, 8, 32641),     # 65282 entries, more than the kernel before it takes
+    (1, 2, 1, 7168, 5121),
+])
+def test_stage_one_of_long_streams(W, E, K, hidden_dim, tokens):
+    print(f"stage 1, {W} ranks x {tokens} tokens x {K} of {hidden_dim}", flush=True)
+    spec = dict(world_size=W, num_experts=E, experts_per_token=K, hidden_dim=hidden_dim, max_num_tokens=tokens,
+                num_tokens="full", routing="zipf" if K < E else "uniform", weights="softmax", dtype="bf16")
+    world = generate_world(spec, 9)[:1]
+    cfg, d = world[0][0], world[0][1]
+    ids = d.indices.to(DEV)
+    ids[tokens // 2] = E + 3  # names no expert: behind all ranks' rows
+    a = HIPAllToAll(cfg, 0, W, device=DEV)
+    x = d.x.to(DEV)
+    counts, buf, meta = a.dispatch_send(x, ids)
+    torch.cuda.synchronize()
+    flat = ids.flatten().long()
+    dest = torch.where(flat < E, flat // (E // W), W)
+    order = torch.argsort(dest, stable=True)
+    rows = order.numel()
+    assert torch.equal(counts.long(), torch.bincount(dest, minlength=W + 1)[:W])
+    assert torch.equal(buf[:rows], x[order // K])
+    want = torch.stack([flat[order], torch.zeros_like(order), order // K, order % K, torch.zeros_like(order)], 1).int()
+    assert torch.equal(meta[:rows], want)
+
+
 @pytest.mark.parametrize("hidden_dim", [8, 520, 1024, 1032, 4096, 4104, 7168])
 @pytest.mark.parametrize("layout", ["padded", "compact"])
 def test_a_few_rows_in_a_launch_for_hundreds_of_megabytes(hidden_dim, layout):
