@@ -193,16 +193,21 @@ class CtypesBinding:
     # ---- the compact expert-major layout (rows of the experts back to back)
 
     def dispatch_recv_compact(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens,
-                              expert_offsets, expert_x, expert_meta, send_back_plan, stream):
+                              expert_offsets, expert_x, expert_meta, send_back_plan, stream, row_position=None):
         _holds("recv_counts", recv_counts, shape.world_size)
         _holds_counts(shape, expert_num_tokens)
         _holds("expert_offsets", expert_offsets, shape.num_experts // shape.world_size + 1)
         _holds_plan(shape, send_back_plan)
         capacity = _rows(recv_buf, recv_meta, shape.hidden_dim)
-        self._call("moe_a2a_dispatch_recv_compact", shape, _ptr(recv_buf), _ptr(recv_meta),
-                  _ptr(recv_counts), min(rows_hint, capacity), capacity, _ptr(expert_num_tokens),
-                  _ptr(expert_offsets), _ptr(expert_x), _ptr(expert_meta),
-                  _rows(expert_x, expert_meta, shape.hidden_dim), _ptr(send_back_plan), stream)
+        args = (shape, _ptr(recv_buf), _ptr(recv_meta), _ptr(recv_counts), min(rows_hint, capacity), capacity,
+                _ptr(expert_num_tokens), _ptr(expert_offsets), _ptr(expert_x), _ptr(expert_meta),
+                _rows(expert_x, expert_meta, shape.hidden_dim), _ptr(send_back_plan))
+        if row_position is None:
+            self._call("moe_a2a_dispatch_recv_compact", *args, stream)
+        else:  # long streams: places from a planning launch
+            if row_position.numel() < capacity:
+                raise ValueError("row_position must hold one int per row of the receive buffers")
+            self._call("moe_a2a_dispatch_recv_compact_long", *args, _ptr(row_position), stream)
 
     def expert_scale_compact(self, shape, expert_x, expert_num_tokens, rows_hint, expert_y, stream):
         capacity = min(expert_x.shape[0], expert_y.shape[0])
@@ -343,10 +348,13 @@ class ExtBinding:
                                    recv_meta, recv_counts, src_rank, rows_hint, stream)
 
     def dispatch_recv_compact(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens,
-                              expert_offsets, expert_x, expert_meta, send_back_plan, stream):
-        self._m.a2a_dispatch_recv_compact(self._shape(shape), recv_buf, recv_meta, recv_counts, rows_hint,
-                                          expert_num_tokens, expert_offsets, expert_x, expert_meta,
-                                          send_back_plan, stream)
+                              expert_offsets, expert_x, expert_meta, send_back_plan, stream, row_position=None):
+        args = (self._shape(shape), recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens, expert_offsets,
+                expert_x, expert_meta, send_back_plan)
+        if row_position is None:
+            self._m.a2a_dispatch_recv_compact(*args, stream)
+        else:
+            self._m.a2a_dispatch_recv_compact_long(*args, row_position, stream)
 
     def expert_scale_compact(self, shape, expert_x, expert_num_tokens, rows_hint, expert_y, stream):
         self._m.a2a_expert_scale_compact(self._shape(shape), expert_x, expert_num_tokens, rows_hint, expert_y,

@@ -52,6 +52,7 @@ SIGNATURES = {
     "moe_a2a_exchange_local": [_I, _I, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P],
     "moe_a2a_exchange_gather_local": [_I, _I, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _P],
     "moe_a2a_dispatch_recv_compact": [_SP, _P, _P, _P, _I, _I, _P, _P, _P, _P, _I, _P, _P],
+    "moe_a2a_dispatch_recv_compact_long": [_SP, _P, _P, _P, _I, _I, _P, _P, _P, _P, _I, _P, _P, _P],
     "moe_a2a_expert_scale_compact": [_SP, _P, _P, _I, _I, _I, _I, _P, _P],
     "moe_a2a_expert_gemm_compact": [_SP, _P, _P, _I, _I, _P, _P, _I, _I, _I, _P, _P],
     "moe_a2a_combine_send_compact": [_SP, _P, _P, _P, _I, _I, _I, _P, _P, _P, _P, _P],

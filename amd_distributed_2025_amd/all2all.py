@@ -36,12 +36,13 @@ from .task import MoEConfig, RankTestData
 
 META_DIM = 5
 # Streams of more rows than this take the entry points that rank in a planning launch of their
-# own (moe_a2a_dispatch_recv_long, moe_a2a_combine_recv_long); shorter ones the one-launch
-# entry points, whose movers rank by scanning. Results are the same; the second launch costs
-# about 5 us, which the combine has earned back at 4096 rows and the dispatch, whose scans hide
-# behind its payload for longer, at 8192 (measured at hidden_dim 7168; at 12288 rows the two
-# together are 17 % ahead, at 32768 rows 40 %).
-LONG_STREAM_ROWS = {"dispatch": 8192, "combine": 4096}
+# own (moe_a2a_dispatch_recv_long, moe_a2a_dispatch_recv_compact_long, moe_a2a_combine_recv_long); shorter ones the
+# one-launch entry points, whose movers rank by scanning. Results are the same. The second launch costs
+# about 5 us, which the combine has earned back at 4096 rows, the dispatch, whose scans hide
+# behind its payload for longer, at 6144 (5500 rows of 512 bytes 10.7 us scanned, 10.9 planned, of 14 KB 26.0 / 26.7; 7500 13.4 / 12.8
+# and 42.5 / 33.3), and the compact dispatch, which scans all rows instead of those ahead, at 4096 (3000 rows of 1.3 KB 9.7 / 9.7, of 14 KB
+# 14.6 / 19.2; 4096 12.6 / 10.3 and 23.0 / 23.0; 7500 29.5 / 14.1 and 53.5 / 34.5).
+LONG_STREAM_ROWS = {"dispatch": 6144, "compact": 4096, "combine": 4096}
 
 
 # what moe_a2a_local_dispatch takes
@@ -330,15 +331,16 @@ class HIPAllToAll:
         else:
             ex = self._buf("expert_x", (nle, self.max_recv, cfg.hidden_dim), cfg.in_dtype)
             em = self._buf("expert_meta", (nle, self.max_recv, META_DIM), torch.int32)
-            pos = self._buf("row_position", (capacity,), torch.int32) if hint > self._long_from("dispatch") else None
+        long_from = self._long_from("compact" if compact else "dispatch")
+        if hint > long_from:
+            pos = self._buf("row_position", (capacity,), torch.int32)
         self._plan_made_for = None if plan is None else (em.data_ptr(), num.data_ptr())
-        fresh = self._learn("recv", "learn_recv", num, ex, em, self.expert_offsets if compact else None, plan,
-                            0x7fffffff if compact else self._long_from("dispatch"))
+        fresh = self._learn("recv", "learn_recv", num, ex, em, self.expert_offsets if compact else None, plan, long_from)
         if fresh and self._calls.dispatch_recv(recv_counts, recv_buf, recv_meta, hint) is not None:
             pass
         elif compact:
             self.binding.dispatch_recv_compact(self.shape, recv_buf, recv_meta, recv_counts, hint, num,
-                                               self.expert_offsets, ex, em, plan, _stream(self.device))
+                                               self.expert_offsets, ex, em, plan, _stream(self.device), pos)
         else:
             self.binding.dispatch_recv(self.shape, recv_buf, recv_meta, recv_counts, hint, num, ex, em, plan,
                                        _stream(self.device), pos)

@@ -120,7 +120,7 @@ struct GemmOut {
 struct Workspace {
   Tensor send_counts, send_buf, send_meta;
   Tensor num, expert_x, expert_meta, offsets, plan;
-  int64_t long_rows = 0;  // longer streams take the entry points with a planning launch (padded layout)
+  int64_t long_rows = 0;  // longer streams take the entry points with a planning launch
   Tensor expert_y;
   Tensor back_counts, back_buf, back_meta, back_plan;
   Tensor where, direct_num, direct_x, direct_meta, direct_offsets;
@@ -287,7 +287,7 @@ PyObject* dispatch_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   if (capacity > INT32_MAX) REFUSE;
   rows = std::min(rows, capacity);
   const bool compact = ws->offsets.defined();
-  if (!compact && rows > ws->long_rows) REFUSE;
+  if (rows > ws->long_rows) REFUSE;
   void* stream;
   if (!stream_of(s.raw_stream, s.device_index, &stream)) return nullptr;
   const bool ok =

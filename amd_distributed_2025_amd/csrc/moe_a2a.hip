@@ -1208,19 +1208,31 @@ constexpr int PLAN_INTS = 2;  // ints per (local expert, source rank) of the sen
 // expert (the set of those lanes from one ballot per bit of the expert number), the waves ordered
 // by a prefix over their per-expert counts. row_pos[i] = #{rows before i with the same local expert}, which is
 // the slot the reference's running counter hands out (all2all/reference.py:140-146). The movers
-// then read one int per row instead of scanning.
+// then read one int per row instead of scanning. COMPACT: plus where the row's expert starts, from the same counts
+// of all rows. Stage 2, us with scans / planned: 10000 rows of 512 bytes, padded 22.0 / 15.5, compact 43.6 / 16.6; 20000 of 3 KB 67.6 /
+// 31.8 and 147 / 33; 7500 of 14 KB 42.5 / 33.3 and 53.5 / 34.5; 4096 of 3 KB 8.9 / 9.6 and 12.9 / 10.4, of 14 KB 19.3 / 21.9 and 23.0 / 23.0;
+// 3000 of 1.3 KB compact 9.7 / 9.7, of 14 KB 14.6 / 19.2.
 constexpr int RPLAN_BLOCK = 1024;
 constexpr int RPLAN_WAVES = RPLAN_BLOCK / 64;
 constexpr int RPLAN_MAX_EXPERTS = 256;  // local experts with a counter per wave in LDS
+constexpr int RPLAN_SPREAD = 32;
 
+template <bool COMPACT>
 __global__ __launch_bounds__(RPLAN_BLOCK) void plan_recv_kernel(
     const int* __restrict__ recv_meta, const int* __restrict__ recv_counts, int W, int hint_rows,
     int capacity_rows, int nle, uint32_t magic, int expert_bits, int* __restrict__ row_pos) {
-  __shared__ int ahead[RPLAN_MAX_EXPERTS];                  // rows of each expert before the tile
+  __shared__ int ahead[RPLAN_MAX_EXPERTS];                 // rows of each expert before the tile, in several copies and then summed
+  __shared__ int all[COMPACT ? RPLAN_MAX_EXPERTS : 1];      // rows of each expert, likewise, and then where they start
   __shared__ int in_wave[RPLAN_WAVES][RPLAN_MAX_EXPERTS];   // rows of each expert in each wave of the tile
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const unsigned long long lanes_below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   int R = -1;  // not known yet
+  // Lanes of a wave that count for the same expert do so one after the other, so few experts get several copies of their counters.
+  // Stage 2 of 7500 rows of 512 bytes, us with one copy / these: one expert, padded 16.0 / 12.6, compact 22.8 / 13.6; copies beyond that
+  // only have to be summed (32 experts with 32 copies, 4096 rows 9.3 / 10.5).
+  int copies = 1;
+  while (copies * nle < RPLAN_SPREAD) copies *= 2;
+  const int my_copy = (lane & (copies - 1)) * nle;
   auto rows = [&] { return min(sum_counts(recv_counts, W, capacity_rows), capacity_rows); };
   for (int first = blockIdx.x * RPLAN_BLOCK;; first += gridDim.x * RPLAN_BLOCK) {
     // A tile that lies wholly below the readable bound sends its loads off before the row
@@ -1233,26 +1245,41 @@ __global__ __launch_bounds__(RPLAN_BLOCK) void plan_recv_kernel(
     const int last = early ? first + RPLAN_BLOCK - 1 : R - 1;  // last row that may be read
     const int i = first + tid;
     const int mine = recv_meta[(size_t)min(i, last) * META];
+    // the first keys: of rows ahead, or (COMPACT) of all that may be read
+    constexpr int BATCH = SCAN_UNROLL * RPLAN_BLOCK;
+    const int got = min(BATCH, COMPACT ? (early ? hint_rows : R) : first);
     int e2[SCAN_UNROLL];
+    auto fetch = [&](int from, int to) {
 #pragma unroll
-    for (int u = 0; u < SCAN_UNROLL; ++u)
-      e2[u] = recv_meta[(size_t)min(tid + u * RPLAN_BLOCK, max(first - 1, 0)) * META];
-    for (int j = tid; j < nle; j += RPLAN_BLOCK) ahead[j] = 0;
+      for (int u = 0; u < SCAN_UNROLL; ++u) e2[u] = recv_meta[(size_t)min(from + tid + u * RPLAN_BLOCK, max(to - 1, 0)) * META];
+    };
+    fetch(0, got);
+    for (int j = tid; j < copies * nle; j += RPLAN_BLOCK) {
+      ahead[j] = 0;
+      if constexpr (COMPACT) all[j] = 0;
+    }
     for (int j = tid; j < RPLAN_WAVES * RPLAN_MAX_EXPERTS; j += RPLAN_BLOCK) (&in_wave[0][0])[j] = 0;
     if (R < 0) R = rows();
     lds_barrier();
     if (first >= R) break;  // (uniform over the workgroup)
     const bool ok = i < R;
     const int le = floormod(mine, nle, magic);
-    for (int b = 0; b < first; b += SCAN_UNROLL * RPLAN_BLOCK) {
-      if (b > 0) {
+    auto count = [&](int from, int to) {
 #pragma unroll
-        for (int u = 0; u < SCAN_UNROLL; ++u)
-          e2[u] = recv_meta[(size_t)min(b + tid + u * RPLAN_BLOCK, first - 1) * META];
+      for (int u = 0; u < SCAN_UNROLL; ++u) {
+        const int at = from + tid + u * RPLAN_BLOCK;
+        if (at < to) {
+          const int le2 = floormod(e2[u], nle, magic);
+          if (!COMPACT || at < first) atomicAdd(&ahead[my_copy + le2], 1);
+          if constexpr (COMPACT) atomicAdd(&all[my_copy + le2], 1);
+        }
       }
-#pragma unroll
-      for (int u = 0; u < SCAN_UNROLL; ++u)
-        if (b + tid + u * RPLAN_BLOCK < first) atomicAdd(&ahead[floormod(e2[u], nle, magic)], 1);
+    };
+    const int end = COMPACT ? R : first;
+    count(0, min(got, end));
+    for (int b = got; b < end; b += BATCH) {
+      fetch(b, end);
+      count(b, end);
     }
     // the lanes of this wave with the same expert, from one ballot per bit of the expert number
     // (a loop over the experts present in the wave costs a round per expert: 3.8 us of issue
@@ -1266,8 +1293,40 @@ __global__ __launch_bounds__(RPLAN_BLOCK) void plan_recv_kernel(
     const int rank_in_wave = __popcll(same & lanes_below);
     if (ok && rank_in_wave == 0) in_wave[wave][le] = __popcll(same);
     lds_barrier();
+    if (copies > 1) {
+      if (tid < nle) {
+        int n = 0, n_all = 0;
+        for (int c = tid; c < copies * nle; c += nle) {
+          n += ahead[c];
+          if constexpr (COMPACT) n_all += all[c];
+        }
+        ahead[tid] = n;
+        if constexpr (COMPACT) all[tid] = n_all;
+      }
+      lds_barrier();
+    }
+    if constexpr (COMPACT) {  // where each expert's rows start: a prefix by one wave, four experts per lane
+      if (wave == 0) {
+        int n[RPLAN_MAX_EXPERTS / 64], sum = 0;
+#pragma unroll
+        for (int j = 0; j < RPLAN_MAX_EXPERTS / 64; ++j) {
+          const int x = lane * (RPLAN_MAX_EXPERTS / 64) + j;
+          n[j] = x < nle ? all[x] : 0;
+          sum += n[j];
+        }
+        int before = wave_inclusive_scan(sum) - sum;
+#pragma unroll
+        for (int j = 0; j < RPLAN_MAX_EXPERTS / 64; ++j) {
+          const int x = lane * (RPLAN_MAX_EXPERTS / 64) + j;
+          if (x < nle) all[x] = before;
+          before += n[j];
+        }
+      }
+      lds_barrier();
+    }
     if (ok) {
       int pos = ahead[le] + rank_in_wave;
+      if constexpr (COMPACT) pos += all[le];
       for (int w = 0; w < wave; ++w) pos += in_wave[w][le];
       row_pos[i] = pos;
     }
@@ -1475,20 +1534,20 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
 // the order of the stream. Memory bounds it, and what shaped it is how few places of the streams are open at a time (planned_recv_vecs and
 // RECV_PAST_BYTES, csrc/stream_rules.h): 32768 rows of 14 KB 160 us with a workgroup on the same piece of four rows and plain loads of four
 // vectors, 137 here (6.9 TB/s); with a stage before and behind it 12000 rows of 4 KB 53.6 / 47.0.
-template <typename V, int NVW, bool PLAN, Store HOW, bool PAST>
+template <typename V, int NVW, bool PLAN, bool COMPACT, Store HOW, bool PAST>
 __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_planned_kernel(
     const int* __restrict__ recv_meta, const int* __restrict__ row_pos, const int* __restrict__ recv_counts,
     const V* __restrict__ recv_buf, int W, int hint_rows, int movers, Pieces pieces, int row_vecs, int nle, int capacity_rows,
     uint32_t magic, int max_recv, V* __restrict__ expert_x, int* __restrict__ expert_meta,
-    int* __restrict__ expert_num_tokens, int* __restrict__ plan) {
+    int* __restrict__ expert_num_tokens, int* __restrict__ plan, int* __restrict__ expert_offsets) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if ((int)blockIdx.x < nle) {
     if constexpr (PLAN) {
-      plan_expert<false, SCAN_UNROLL>(recv_meta, recv_counts, W, hint_rows, nle, capacity_rows, magic, expert_num_tokens, plan,
-                                      nullptr);
+      plan_expert<COMPACT, SCAN_UNROLL>(recv_meta, recv_counts, W, hint_rows, nle, capacity_rows, magic, expert_num_tokens, plan,
+                                        expert_offsets);
     } else {
       __shared__ int red[ROWS];
-      count_expert<false>(recv_meta, recv_counts, W, nle, capacity_rows, magic, red, expert_num_tokens, nullptr);
+      count_expert<COMPACT>(recv_meta, recv_counts, W, nle, capacity_rows, magic, red, expert_num_tokens, expert_offsets);
     }
     return;
   }
@@ -1514,7 +1573,7 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_planned_kernel(
     if (R < 0) R = rows();
     if (i >= R) return;
     if ((uint32_t)pos < (uint32_t)max_recv) {
-      const size_t row = (size_t)floormod(e, nle, magic) * max_recv + pos;
+      const size_t row = COMPACT ? (size_t)pos : (size_t)floormod(e, nle, magic) * max_recv + pos;
       p.template store<HOW>(expert_x + row * row_vecs, base, row_vecs, lane);
       if (c == 0 && lane < META) expert_meta[row * META + lane] = m;
     }
@@ -4903,7 +4962,7 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   if (!shape_ok(s) || rows_hint < 0 || capacity_rows < 0 || !recv_counts || !expert_num_tokens ||
       !expert_x || !expert_meta)
     return MOE_A2A_EINVAL;
-  if (compact_rows > 0 && (!expert_offsets || row_position)) return MOE_A2A_EINVAL;
+  if (compact_rows > 0 && !expert_offsets) return MOE_A2A_EINVAL;
   if (!counts_fit(capacity_rows, s->world_size)) return MOE_A2A_EINVAL;
   if (rows_hint > capacity_rows) rows_hint = capacity_rows;
   if (capacity_rows > 0 && (!recv_buf || !recv_meta)) return MOE_A2A_EINVAL;
@@ -4921,15 +4980,22 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
     const int tiles = (int)std::min<long long>(((long long)rows_hint + RPLAN_BLOCK - 1) / RPLAN_BLOCK + 1, 1 << 16);
     int expert_bits = 0;  // nle <= 1 << expert_bits
     while ((1 << expert_bits) < g.nle) ++expert_bits;
-    plan_recv_kernel<<<tiles, RPLAN_BLOCK, 0, st>>>(recv_meta, recv_counts, s->world_size, rows_hint,
-                                                    capacity_rows, g.nle, g.magic, expert_bits, row_position);
+    auto plan_rows = compact_rows > 0 ? plan_recv_kernel<true> : plan_recv_kernel<false>;
+    plan_rows<<<tiles, RPLAN_BLOCK, 0, st>>>(recv_meta, recv_counts, s->world_size, rows_hint, capacity_rows, g.nle, g.magic,
+                                             expert_bits, row_position);
     const int movers = mover_blocks(((long long)rows_hint * g.wchunks + ROWS - 1) / ROWS);
     const bool past = (long long)rows_hint * s->hidden_dim * 2 >= RECV_PAST_BYTES;
-#define LAUNCH_L(V, NVW, PLAN, PAST)                                                                           \
-  dispatch_recv_planned_kernel<V, NVW, PLAN, THROUGH, PAST><<<g.nle + movers, 64 * ROWS, 0, st>>>(             \
+#define LAUNCH_C(V, NVW, PLAN, COMPACT, PAST)                                                                  \
+  dispatch_recv_planned_kernel<V, NVW, PLAN, COMPACT, THROUGH, PAST><<<g.nle + movers, 64 * ROWS, 0, st>>>(    \
       recv_meta, row_position, recv_counts, (const V*)recv_buf, s->world_size, rows_hint, movers,              \
-      pieces_of(g.wchunks), g.row_vecs, g.nle, capacity_rows, g.magic, g.max_recv, (V*)expert_x, expert_meta,  \
-      expert_num_tokens, send_back_plan)
+      pieces_of(g.wchunks), g.row_vecs, g.nle, capacity_rows, g.magic,                                         \
+      COMPACT ? compact_rows : g.max_recv, (V*)expert_x, expert_meta, expert_num_tokens, send_back_plan,       \
+      expert_offsets)
+#define LAUNCH_L(V, NVW, PLAN, PAST)                            \
+  do {                                                          \
+    if (compact_rows > 0) LAUNCH_C(V, NVW, PLAN, true, PAST);   \
+    else LAUNCH_C(V, NVW, PLAN, false, PAST);                   \
+  } while (0)
 #define LAUNCH_P(V, NVW, PLAN)                        \
   do {                                                \
     if constexpr (sizeof(V) == sizeof(b128)) {        \
@@ -4951,6 +5017,7 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
 #undef LAUNCH
 #undef LAUNCH_P
 #undef LAUNCH_L
+#undef LAUNCH_C
     return launch_status();
   }
   // the stream can hold at most nle * max_recv rows that fit the expert buffers
@@ -5278,6 +5345,17 @@ int moe_a2a_dispatch_recv_compact(const moe_a2a_shape* s, const void* recv_buf, 
   if (compact_capacity_rows < 1 || !expert_offsets) return MOE_A2A_EINVAL;
   return launch_dispatch_recv(s, recv_buf, recv_meta, recv_counts, rows_hint, capacity_rows, expert_num_tokens,
                               expert_x, expert_meta, send_back_plan, nullptr, stream, compact_capacity_rows,
+                              expert_offsets);
+}
+
+int moe_a2a_dispatch_recv_compact_long(const moe_a2a_shape* s, const void* recv_buf, const int32_t* recv_meta,
+                                       const int32_t* recv_counts, int32_t rows_hint, int32_t capacity_rows,
+                                       int32_t* expert_num_tokens, int32_t* expert_offsets, void* expert_x,
+                                       int32_t* expert_meta, int32_t compact_capacity_rows,
+                                       int32_t* send_back_plan, int32_t* row_position, void* stream) {
+  if (compact_capacity_rows < 1 || !expert_offsets || !row_position) return MOE_A2A_EINVAL;
+  return launch_dispatch_recv(s, recv_buf, recv_meta, recv_counts, rows_hint, capacity_rows, expert_num_tokens,
+                              expert_x, expert_meta, send_back_plan, row_position, stream, compact_capacity_rows,
                               expert_offsets);
 }
 

@@ -315,10 +315,11 @@ int64_t compact_rows(const torch::Tensor& rows, const char* what) {
 }
 }  // namespace
 
-void a2a_dispatch_recv_compact(std::vector<int64_t> shape, torch::Tensor recv_buf, torch::Tensor recv_meta,
-                               torch::Tensor recv_counts, int64_t rows_hint, torch::Tensor expert_num_tokens,
-                               torch::Tensor expert_offsets, torch::Tensor expert_x, torch::Tensor expert_meta,
-                               c10::optional<torch::Tensor> send_back_plan, int64_t stream) {
+// Stage 2 in the compact layout; `row_position`: the place of every row from a planning launch, or null.
+static void recv_compact(const std::vector<int64_t>& shape, torch::Tensor& recv_buf, torch::Tensor& recv_meta,
+                         torch::Tensor& recv_counts, int64_t rows_hint, torch::Tensor& expert_num_tokens,
+                         torch::Tensor& expert_offsets, torch::Tensor& expert_x, torch::Tensor& expert_meta,
+                         c10::optional<torch::Tensor>& send_back_plan, torch::Tensor* row_position, int64_t stream) {
   const moe_a2a_shape s = shape_of(shape);
   const auto dt = rows_type(recv_buf, "recv_buf");
   const int64_t nle = s.world_size > 0 ? s.num_experts / s.world_size : 0;
@@ -334,6 +335,17 @@ void a2a_dispatch_recv_compact(std::vector<int64_t> shape, torch::Tensor recv_bu
   need(expert_meta, "expert_meta", torch::kInt32, room * MOE_A2A_META_DIM, &recv_buf);
   if (send_back_plan.has_value())
     need(*send_back_plan, "send_back_plan", torch::kInt32, 2 * (int64_t)s.num_experts, &recv_buf);
+  if (row_position) {
+    need(*row_position, "row_position", torch::kInt32, capacity, &recv_buf);
+    status(moe_a2a_dispatch_recv_compact_long(&s, recv_buf.data_ptr(), ints(recv_meta), ints(recv_counts),
+                                              to_i32(std::min(rows_hint, capacity), "rows_hint"),
+                                              to_i32(capacity, "capacity_rows"), ints(expert_num_tokens),
+                                              ints(expert_offsets), expert_x.data_ptr(), ints(expert_meta),
+                                              to_i32(room, "compact_capacity_rows"), ints_or_null(send_back_plan),
+                                              ints(*row_position), stream_of(stream)),
+           "moe_a2a_dispatch_recv_compact_long");
+    return;
+  }
   status(moe_a2a_dispatch_recv_compact(&s, recv_buf.data_ptr(), ints(recv_meta), ints(recv_counts),
                                        to_i32(std::min(rows_hint, capacity), "rows_hint"),
                                        to_i32(capacity, "capacity_rows"), ints(expert_num_tokens),
@@ -341,6 +353,23 @@ void a2a_dispatch_recv_compact(std::vector<int64_t> shape, torch::Tensor recv_bu
                                        to_i32(room, "compact_capacity_rows"), ints_or_null(send_back_plan),
                                        stream_of(stream)),
          "moe_a2a_dispatch_recv_compact");
+}
+
+void a2a_dispatch_recv_compact(std::vector<int64_t> shape, torch::Tensor recv_buf, torch::Tensor recv_meta,
+                               torch::Tensor recv_counts, int64_t rows_hint, torch::Tensor expert_num_tokens,
+                               torch::Tensor expert_offsets, torch::Tensor expert_x, torch::Tensor expert_meta,
+                               c10::optional<torch::Tensor> send_back_plan, int64_t stream) {
+  recv_compact(shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens, expert_offsets, expert_x, expert_meta,
+               send_back_plan, nullptr, stream);
+}
+
+void a2a_dispatch_recv_compact_long(std::vector<int64_t> shape, torch::Tensor recv_buf, torch::Tensor recv_meta,
+                                    torch::Tensor recv_counts, int64_t rows_hint, torch::Tensor expert_num_tokens,
+                                    torch::Tensor expert_offsets, torch::Tensor expert_x, torch::Tensor expert_meta,
+                                    c10::optional<torch::Tensor> send_back_plan, torch::Tensor row_position,
+                                    int64_t stream) {
+  recv_compact(shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens, expert_offsets, expert_x, expert_meta,
+               send_back_plan, &row_position, stream);
 }
 
 void a2a_expert_scale_compact(std::vector<int64_t> shape, torch::Tensor expert_x, torch::Tensor expert_num_tokens,

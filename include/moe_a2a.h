@@ -171,7 +171,7 @@ int moe_a2a_dispatch_recv(const moe_a2a_shape* shape, const void* recv_buf,
  *                every received row inside its expert
  *
  * Two launches instead of one: at hidden_dim 7168 this form pays from about
- * 8192 rows (at 32768 rows: 200 us against 323 us). With more than 256 local
+ * 6144 rows (at 20000 rows: 86 us against 155 us). With more than 256 local
  * experts the call falls back to the scanning kernel.
  */
 int moe_a2a_dispatch_recv_long(const moe_a2a_shape* shape, const void* recv_buf,
@@ -445,7 +445,7 @@ int moe_a2a_exchange_local(int32_t world_size, int32_t hidden_dim,
  * Every mover workgroup counts the rows of lower experts over the whole stream
  * (one pass over all keys instead of the keys ahead of it), so this entry point
  * is meant for the streams of a few thousand rows the one-launch entry points
- * serve; there is no long-stream form of it.
+ * serve; moe_a2a_dispatch_recv_compact_long is the form for longer ones.
  */
 int moe_a2a_dispatch_recv_compact(const moe_a2a_shape* shape, const void* recv_buf,
                                   const int32_t* recv_meta, const int32_t* recv_counts,
@@ -454,6 +454,24 @@ int moe_a2a_dispatch_recv_compact(const moe_a2a_shape* shape, const void* recv_b
                                   void* expert_x, int32_t* expert_meta,
                                   int32_t compact_capacity_rows, int32_t* send_back_plan,
                                   void* stream);
+
+/*
+ * moe_a2a_dispatch_recv_compact for long streams: the rows' places come from a
+ * planning launch, as in moe_a2a_dispatch_recv_long. Same arguments and the same
+ * results, bit for bit, plus
+ *
+ *   row_position [capacity_rows] int32 workspace, overwritten: the place of
+ *                every received row among the compact rows
+ *
+ * With more than 256 local experts the call falls back to the scanning kernel.
+ */
+int moe_a2a_dispatch_recv_compact_long(const moe_a2a_shape* shape, const void* recv_buf,
+                                       const int32_t* recv_meta, const int32_t* recv_counts,
+                                       int32_t rows_hint, int32_t capacity_rows,
+                                       int32_t* expert_num_tokens, int32_t* expert_offsets,
+                                       void* expert_x, int32_t* expert_meta,
+                                       int32_t compact_capacity_rows, int32_t* send_back_plan,
+                                       int32_t* row_position, void* stream);
 
 /* moe_a2a_expert_scale on compact buffers: expert_x, expert_y [compact_capacity_rows, H]. */
 int moe_a2a_expert_scale_compact(const moe_a2a_shape* shape, const void* expert_x,

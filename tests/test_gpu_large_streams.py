@@ -1,12 +1,14 @@
 """Streams that the caches do not hold: rows read past them, in pieces of one, two, four or eight vectors per lane
 (`csrc/stream_rules.h`). Results are the ones of the other kernels, bit for bit."""
+import numpy as np
 import pytest
 import torch
 
-from amd_distributed_2025_amd import HIPAllToAll, _lib, generate_world
+from amd_distributed_2025_amd import HIPAllToAll, LocalWorld, WORKLOADS, _lib, generate_world
 from amd_distributed_2025_amd.task import MoEConfig
+from tests.helpers import bits, run_oracle
 from tests.test_gpu_long_streams import run_long
-from tests.test_gpu_parity import DEV
+from tests.test_gpu_parity import DEV, EDGE
 
 pytestmark = pytest.mark.gpu
 
@@ -102,3 +104,38 @@ def test_a_few_rows_in_a_launch_for_hundreds_of_megabytes(hidden_dim, layout):
 
 def _lib_pointer(t):
     return t.data_ptr()
+
+
+def run_compact(world, binding="ctypes", exact_hints=True):
+    cfg, W = world[0][0], len(world)
+    lw = LocalWorld(cfg, W, device=DEV, layout="compact", long_stream_rows=0, binding=binding, exact_hints=exact_hints)
+    ys = lw.run([d.to(DEV) for _, d, _, _ in world])
+    torch.cuda.synchronize()
+    want = run_oracle(world)
+    for r in range(W):
+        g, a = lw.trace[r], lw.ranks[r]
+        num = want[r].expert_num_tokens
+        R = int(num.sum())
+        assert np.array_equal(g["expert_num_tokens"].cpu().numpy(), num), r
+        assert np.array_equal(a.expert_offsets.cpu().numpy(), np.concatenate([[0], np.cumsum(num)])), r
+        assert np.array_equal(bits(g["expert_x"][:R]), want[r].expert_rows), r
+        assert np.array_equal(g["expert_meta"][:R].cpu().numpy(), want[r].expert_meta_rows), r
+        assert np.array_equal(bits(ys[r]), want[r].y), r
+
+
+@pytest.mark.parametrize("name", ["C1", "C2", "C3", "C4", "C5"] + sorted(EDGE))
+def test_planned_places_in_the_compact_layout(name):
+    print(f"compact, planned, {name}", flush=True)
+    spec = WORKLOADS[name] if name in WORKLOADS else dict(dict(routing="uniform", weights="rand"), **EDGE[name])
+    run_compact(generate_world(spec, 17))
+
+
+@pytest.mark.parametrize("W,nle,K,tokens", [(2, 256, 8, 1500), (4, 3, 5, 2600), (1, 64, 8, 1025), (3, 257, 2, 300)])
+@pytest.mark.parametrize("exact_hints", [True, False])
+def test_planned_places_of_many_tiles(W, nle, K, tokens, exact_hints):
+    """Several tiles of 1024 rows, more rows than the first batch of a tile (8192), up to 256 experts (257: the scan), hints above
+    and, under skewed routing, below the rows that arrive; the extension's wrapper."""
+    print(f"compact, planned, {W} x {nle} experts, {tokens} tokens x {K}", flush=True)
+    spec = dict(world_size=W, num_experts=W * nle, experts_per_token=K, hidden_dim=16, max_num_tokens=tokens,
+                num_tokens="full", routing="zipf", weights="rand", dtype="bf16")
+    run_compact(generate_world(spec, 5), exact_hints=exact_hints, binding="ext" if exact_hints else "ctypes")
