@@ -223,6 +223,11 @@ class HIPAllToAll:
             self._kept[name] = (shape, dtype)
         return self._ws[name]
 
+    def _at_least(self, name: str, ints: int) -> torch.Tensor:
+        """A workspace of that many ints, or the larger one that an earlier call has made."""
+        kept = self._ws.get(name)
+        return kept if kept is not None and kept.numel() >= ints else self._buf(name, (ints,), torch.int32)
+
     def workspace_bytes(self) -> int:
         """Device memory of the buffers this object has made so far."""
         return sum(t.numel() * t.element_size() for t in self._ws.values())
@@ -333,9 +338,11 @@ class HIPAllToAll:
             em = self._buf("expert_meta", (nle, self.max_recv, META_DIM), torch.int32)
         long_from = self._long_from("compact" if compact else "dispatch")
         if hint > long_from:
-            pos = self._buf("row_position", (capacity,), torch.int32)
+            pos = self._at_least("row_position", capacity)
         self._plan_made_for = None if plan is None else (em.data_ptr(), num.data_ptr())
         fresh = self._learn("recv", "learn_recv", num, ex, em, self.expert_offsets if compact else None, plan, long_from)
+        if pos is not None:
+            fresh = self._learn("positions", "learn_positions", pos) or fresh
         if fresh and self._calls.dispatch_recv(recv_counts, recv_buf, recv_meta, hint) is not None:
             pass
         elif compact:
@@ -491,7 +498,11 @@ class HIPAllToAll:
         hint = min(capacity, T * cfg.experts_per_token)
         table = None
         if unique_pairs and hint > self._long_from("combine"):
-            table = self._buf("entry_row", (cfg.max_num_tokens * cfg.experts_per_token,), torch.int32)
+            table = self._at_least("entry_row", cfg.max_num_tokens * cfg.experts_per_token)
+            if (self._learn("table", "learn_table", table)
+                    and self._calls.combine_recv(out_tokens, weights, ret_counts, ret_buf, ret_meta, accumulate,
+                                                 self._long_from("combine"))):
+                return out_tokens
         self.binding.combine_recv(self.shape, ret_buf, ret_meta, ret_counts, hint, weights, T, out_tokens,
                                   accumulate, _stream(self.device), table)
         return out_tokens

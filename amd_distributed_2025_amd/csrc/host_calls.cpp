@@ -121,6 +121,7 @@ struct Workspace {
   Tensor send_counts, send_buf, send_meta;
   Tensor num, expert_x, expert_meta, offsets, plan;
   int64_t long_rows = 0;  // longer streams take the entry points with a planning launch
+  Tensor row_position, entry_row;  // what those launches work out (stages 2 and 4)
   Tensor expert_y;
   Tensor back_counts, back_buf, back_meta, back_plan;
   Tensor where, direct_num, direct_x, direct_meta, direct_offsets;
@@ -270,6 +271,14 @@ PyObject* learn_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// (row_position)
+PyObject* learn_positions(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TAKES(1)
+  return learn(state(self), a, {&Workspace::row_position});
+  END_HANDLE_TH_ERRORS
+}
+
 // (counts, buf, meta, rows) -> rows that sized the launch
 PyObject* dispatch_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -287,15 +296,22 @@ PyObject* dispatch_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   if (capacity > INT32_MAX) REFUSE;
   rows = std::min(rows, capacity);
   const bool compact = ws->offsets.defined();
-  if (rows > ws->long_rows) REFUSE;
+  const bool planned = rows > ws->long_rows;
+  if (planned && (!ws->row_position.defined() || ws->row_position.numel() < capacity)) REFUSE;
   void* stream;
   if (!stream_of(s.raw_stream, s.device_index, &stream)) return nullptr;
+  const int32_t hint = (int32_t)rows, room = (int32_t)capacity, compact_room = compact ? (int32_t)ws->expert_x.size(0) : 0;
+  void *const from = buf->data_ptr(), *const to = ws->expert_x.data_ptr();
+  int32_t *const m = ints(*meta), *const c = ints(*counts), *const num = ints(ws->num), *const to_meta = ints(ws->expert_meta);
+  int32_t *const plan = ints(ws->plan), *const offsets = ints(ws->offsets);
+  int32_t* const position = planned ? ints(ws->row_position) : nullptr;
   const bool ok =
-      compact ? launched(moe_a2a_dispatch_recv_compact, &s.shape, buf->data_ptr(), ints(*meta), ints(*counts), (int32_t)rows,
-                         (int32_t)capacity, ints(ws->num), ints(ws->offsets), ws->expert_x.data_ptr(), ints(ws->expert_meta),
-                         (int32_t)ws->expert_x.size(0), ints(ws->plan), stream)
-              : launched(moe_a2a_dispatch_recv, &s.shape, buf->data_ptr(), ints(*meta), ints(*counts), (int32_t)rows,
-                         (int32_t)capacity, ints(ws->num), ws->expert_x.data_ptr(), ints(ws->expert_meta), ints(ws->plan), stream);
+      compact && planned ? launched(moe_a2a_dispatch_recv_compact_long, &s.shape, from, m, c, hint, room, num, offsets, to, to_meta,
+                                    compact_room, plan, position, stream)
+      : compact ? launched(moe_a2a_dispatch_recv_compact, &s.shape, from, m, c, hint, room, num, offsets, to, to_meta, compact_room,
+                           plan, stream)
+      : planned ? launched(moe_a2a_dispatch_recv_long, &s.shape, from, m, c, hint, room, num, to, to_meta, plan, position, stream)
+                : launched(moe_a2a_dispatch_recv, &s.shape, from, m, c, hint, room, num, to, to_meta, plan, stream);
   if (!ok) REFUSE;
   return PyLong_FromLongLong(rows);
   END_HANDLE_TH_ERRORS
@@ -442,6 +458,14 @@ bool takes_results(const State& s, const Tensor& out, const Tensor& weights) {
          dense(weights, at::kFloat, s.device);
 }
 
+// (entry_row)
+PyObject* learn_table(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TAKES(1)
+  return learn(state(self), a, {&Workspace::entry_row});
+  END_HANDLE_TH_ERRORS
+}
+
 // (out, weights, counts, buf, meta, accumulate, rows from which streams are long) -> True
 PyObject* combine_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -455,13 +479,21 @@ PyObject* combine_recv(PyObject* self, PyObject* const* a, Py_ssize_t n) {
       !dense(*buf, s.out, s.device) || !dense(*meta, at::kInt, s.device))
     REFUSE;
   const int64_t T = weights->size(0), capacity = std::min(buf->size(0), meta->size(0)), rows = std::min(capacity, T * s.topk);
-  if (capacity > INT32_MAX || rows > long_rows) REFUSE;
+  const auto ws = s.ws;
+  const bool mapped = rows > long_rows;
+  if (capacity > INT32_MAX || (mapped && (!ws->entry_row.defined() || ws->entry_row.numel() < T * s.topk))) REFUSE;
   void* stream;
   if (!stream_of(s.raw_stream, s.device_index, &stream)) return nullptr;
   const int32_t accumulate = a[5] == Py_True;
-  if (!launched(moe_a2a_combine_recv, &s.shape, buf->data_ptr(), ints(*meta), ints(*counts), (int32_t)rows, (int32_t)capacity,
-                static_cast<const float*>(weights->data_ptr()), (int32_t)T, out->data_ptr(), accumulate, code(s.out), stream))
-    REFUSE;
+  void *const from = buf->data_ptr(), *const to = out->data_ptr();
+  int32_t *const m = ints(*meta), *const c = ints(*counts);
+  const float* const w = static_cast<const float*>(weights->data_ptr());
+  int32_t* const table = mapped ? ints(ws->entry_row) : nullptr;
+  const bool ok = mapped ? launched(moe_a2a_combine_recv_long, &s.shape, from, m, c, (int32_t)rows, (int32_t)capacity, w, (int32_t)T, to,
+                                    accumulate, code(s.out), table, stream)
+                         : launched(moe_a2a_combine_recv, &s.shape, from, m, c, (int32_t)rows, (int32_t)capacity, w, (int32_t)T, to,
+                                    accumulate, code(s.out), stream);
+  if (!ok) REFUSE;
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -676,6 +708,7 @@ PyMethodDef rank_methods[] = {
     FAST(learn_send, "(counts, buf, meta)"),
     FAST(dispatch_send, "(x, indices) -> tokens or None"),
     FAST(learn_recv, "(num, expert_x, expert_meta, offsets, plan, long_rows)"),
+    FAST(learn_positions, "(row_position)"),
     FAST(dispatch_recv, "(counts, buf, meta, rows) -> rows or None"),
     FAST(learn_scale, "(expert_y)"),
     FAST(expert_scale, "(expert_x, num, rows) -> expert_y or None"),
@@ -683,6 +716,7 @@ PyMethodDef rank_methods[] = {
     FAST(expert_gemm, "(expert_x, num, weights, bias, rows) -> out or None"),
     FAST(learn_back, "(counts, buf, meta, plan)"),
     FAST(combine_send, "(expert_meta, expert_y, num, rows, planned_for) -> True or None"),
+    FAST(learn_table, "(entry_row)"),
     FAST(combine_recv, "(out, weights, counts, buf, meta, accumulate, long_rows) -> True or None"),
     FAST(learn_direct, "(num, expert_x, expert_meta, where, offsets)"),
     FAST(direct_dispatch, "(x, indices) -> tokens or None"),
