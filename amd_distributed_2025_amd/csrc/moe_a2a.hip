@@ -3018,7 +3018,7 @@ __global__ __launch_bounds__(64 * KW) void skinny_gemm_kernel(
 //
 // C[M, N] = A[M, K] @ B[N, K]^T for outputs that tiles of 256 columns (phased_gemm_kernel) would spread over
 // too few compute units, and for experts' rows (GROUPED) also where those would leave much of a last round idle. A
-// workgroup of four waves owns a BM x BN tile of C (64 or 128 x 128) and walks K in steps of
+// workgroup of four waves owns a BM x BN tile of C (128 x 128; 64 x 128 and products of one round are sliced_gemm_kernel's) and walks K in steps of
 // 64 elements. Per step the workgroup copies BM + BN rows of 128 bytes into LDS once (through registers, two LDS
 // buffers, one barrier per step), and every wave reads each operand fragment it needs once per 16-element slice
 // of the step for a whole row or column of its MFMA tiles, issued one slice ahead.
@@ -3510,17 +3510,17 @@ __device__ __forceinline__ GroupTile find_group_tile(int tile, const int* __rest
 
 // ---------------------------------------------------------------- products of few tiles
 //
-// The experts' product, or a plain one, where its tiles leave a unit with one or two workgroups (and some with long walks of K,
-// grouped_ring): nothing then hides the way of a step's rows from memory but the steps that are already under way. Four waves fetch the rows of a tile of 32 TM x 32 TN straight
-// into a ring of DEPTH steps in LDS (64 to 144 KB of them) and multiply a quarter of the tile each. One barrier per step:
+// The experts' product of few rows per expert, on tiles of 32 x 32 or 32 x 64, where they leave a unit with one or two workgroups (and some with long
+// walks of K, grouped_ring): nothing then hides the way of a step's rows from memory but the steps that are already under way. Four waves fetch the
+// rows of a tile of 32 TM x 32 TN straight into a ring of DEPTH steps in LDS (64 to 72 KB of them) and multiply a quarter of the tile each. One barrier per step:
 // behind it step s + 1 is there for everybody, and everybody holds the fragments of step s, so that its place is free for
 // step s + DEPTH, and the fragments of step s + 1 are read beside the MFMAs of step s (without that, and with all of a tile's
 // 32 columns on one wave, 1 row in 1024 x 7168 took 27.6 us instead of 17.1).
 // LDS rows, fragments and the order of K are those of phased_gemm_kernel.
 // What bounds it: with few tiles the chain of a step (barrier, fragments, two MFMAs: 0.14 us), with more HBM (5 to 6 TB/s
-// from 400 tiles on), on 64 x 128 the fragments' way out of LDS. us, expert_gemm_kernel or dense_gemm_kernel / here: 7 of 48
-// groups with a row, 832 x 3840 21.7 / 11.3; 2 of 8, 2048 x 4096 23.0 / 11.8; 4 groups of 1 row, 2048 x 7168 38.1 / 22.5; 8 of
-// 70, 2048 x 4096 42.4 / 32.3; 7 of 197, 832 x 6528 66.3 / 42.4; 19 of 2, 6272 x 3360 157.0 / 120.6.
+// from 400 tiles on). us, expert_gemm_kernel / here: 7 of 48
+// groups with a row, 832 x 3840 21.7 / 11.3; 2 of 8, 2048 x 4096 23.0 / 11.8; 4 groups of 1 row, 2048 x 7168 38.1 / 22.5; 19 of 2, 6272 x
+// 3360 157.0 / 120.6. (Larger tiles are sliced_gemm_kernel's. On these it is up to 7 % behind: 101 products of 32 x 64 1.02 of the time here.)
 
 constexpr size_t ring_lds_bytes(int TM, int TN, int DEPTH) { return (size_t)DEPTH * (TM + TN) * 32 * 128; }
 
@@ -3656,6 +3656,200 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
         }
       }
     }
+  }
+}
+
+// ---------------------------------------------------------------- products of a few hundred tiles
+//
+// The experts' product or a plain one where its tiles make for about one workgroup per unit, or two. WM x WN waves, two or four of them on a SIMD,
+// fetch the rows of a tile straight into a ring of DEPTH steps in LDS. A wave holds the fragments of one slice of 32 inputs while those of the
+// next are on their way, so that its reads are behind MFMAs and the waves of a SIMD fill each other's gaps; one barrier per step, in its
+// middle. LDS rows, fragments, results and the order of K are those of phased_gemm_kernel, so the choice changes no bit.
+// What bounds it: rows out of L2, some 17 TB/s over the chip on any tile (32 x 64 to 192 x 128: 0.2 to 0.67 us a step), and 3.5 to 5 us around
+// the walk (launch, first rows, results). us, the kernel that had the product / here:
+//   plain, on one group of ring_gemm_kernel, whose workgroups search the groups for their tile: 77 x 7360 x 768 7.84 / 5.74, 351 x 1728 x 832
+//     8.19 / 6.04, 202 x 2432 x 6272 26.7 / 21.7, 24 x 2176 x 384 5.31 / 4.38; on 64 x 128 of dense_gemm_kernel, whose rows go through registers
+//     into two buffers: 786 x 1984 x 4608 28.4 / 25.5, 297 x 1152 x 408 5.79 / 4.77, 37 x 7808 x 8 4.33 / 3.75; split over K: 64 x 7168 x 2304
+//     10.56 / 9.60, 88 x 5056 x 2432 11.75 / 9.95
+//   experts': 15 of 400 rows, 576 x 640 (dense_gemm_kernel, 64 x 128) 23.9 / 16.8; 5 of 253, 896 x 1856 (a ring of 64 x 128) 17.3 / 14.0; 11 of 50,
+//     1248 x 6240 69.4 / 45.0; 22 of 239, 640 x 1280 (dense_gemm_kernel, 128 x 128) 25.0 / 17.2; 13 of 377, 1024 x 4032
+//     (phased_gemm_kernel, 192 x 256) 72.0 / 52.6; 18 of 39, 960 x 1408 (expert_gemm_kernel) 22.2 / 13.0
+template <int WM_, int WN_, int TM_, int TN_, int DEPTH_, int ON_UNIT_>
+struct Slices {
+  static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, DEPTH = DEPTH_, ON_UNIT = ON_UNIT_;  // (workgroups on a unit)
+  static constexpr int ROWS = WM * TM * 16, COLS = WN * TN * 16, LANES = 64 * WM * WN;
+  static constexpr size_t LDS_BYTES = (size_t)DEPTH * (ROWS + COLS) * 128;
+};
+using Slices32x64 = Slices<2, 2, 1, 2, 6, 2>;
+using Slices64x64 = Slices<4, 2, 1, 2, 4, 2>;
+using Slices64x128 = Slices<2, 4, 2, 2, 3, 2>;
+using Slices128x128 = Slices<4, 2, 2, 4, 4, 1>;
+using Slices192x128 = Slices<4, 2, 3, 4, 3, 1>;
+
+// (Rings of twice the depth where every unit has a tile at most, of 144 KB of LDS: 0.4 to 1.2 us longer, as two launches in a row do not overlap then; with
+// weights that HBM has to deliver as well, 64 x 7168 x 2304 12.0 / 13.0, 85 x 5376 x 1856 9.6 / 10.6, 200 x 4096 x 4096 18.8 / 17.7.)
+template <int DT, typename TILE, bool GROUPED, bool STREAMED>
+__global__ __launch_bounds__(64 * TILE::WM * TILE::WN, TILE::ON_UNIT * TILE::WM * TILE::WN / 4) void sliced_gemm_kernel(
+    const b128* __restrict__ A, const b128* __restrict__ B, const uint16_t* __restrict__ bias, uint16_t* __restrict__ C, int M, int N, int K,
+    int tiles_m, int tiles_n, const int* __restrict__ rows_of_group, int groups, int max_rows, int compact) {
+  constexpr int WM = TILE::WM, WN = TILE::WN, TM = TILE::TM, TN = TILE::TN, DEPTH = TILE::DEPTH;
+  constexpr int NW = WM * WN, NT = 64 * NW, BM = TILE::ROWS, BN = TILE::COLS, GROUP_M = 4;
+  constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW;  // direct loads (8 rows each) of a wave per step
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole loads");
+  constexpr int STEP_BYTES = (BM + BN) * 128, B_AT = BM * 128, RING_BYTES = DEPTH * STEP_BYTES;
+  constexpr int YOUNGER = (LA + LB) * (DEPTH - 2);  // a wave's loads that may be under way when step s + 1 has to be there
+  static_assert(DEPTH >= 2 && YOUNGER + LA + LB < 64, "loads that the wait can count");
+  extern __shared__ b128 tile_lds[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int row_vecs = K / 8, row_bytes = K * 2, steps = (K + GEMM_KSTEP - 1) / GEMM_KSTEP;
+  const int tail_vecs = row_vecs - (steps - 1) * 8;
+  // load i of a wave takes rows (i * NW + wave) * 8 .. + 7 of an operand, a lane the vector that belongs at its place
+  const int lrow = wave * 8 + (lane >> 3);
+  const int vec = (lane & 7) ^ ((lrow >> 1) & 7);
+  const int off = lrow * row_bytes + vec * 16;
+  const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) b128*)tile_lds + wave * 1024;
+  // fragment of a slice of 32 inputs: row r of a band of 16, vector 4 * slice + q of the step
+  const int r = lane & 15, q = lane >> 4, swz = (r >> 1) & 7;
+  [[maybe_unused]] const int total_tiles = tiles_m * tiles_n;  // (GROUPED: counted by find_group_tile)
+
+  for (int tile = blockIdx.x;; tile += gridDim.x) {
+    int n0, rows_left;         // first column of the tile; rows of the matrix from the tile's first one on
+    size_t row_at, b_at;       // the tile's first rows of A and C, and of B
+    const uint16_t* bias_row;  // the bias of the tile's group, or null
+    [[maybe_unused]] int k_first = 0;
+    if constexpr (GROUPED) {
+      const GroupTile at = find_group_tile<NT, BM>(tile, rows_of_group, groups, max_rows, tiles_n, compact, (int*)tile_lds);
+      if (tile >= at.total) return;
+      lds_barrier();
+      n0 = at.tn * BN;
+      rows_left = at.rows;
+      row_at = at.row_at;
+      b_at = (size_t)at.group * N + n0;
+      k_first = first_kstep(at.group, groups, K) * (GEMM_KSTEP * 2);
+      bias_row = bias ? bias + (size_t)at.group * N : nullptr;
+    } else {
+      if (tile >= total_tiles) return;
+      const int logical = xcd_contiguous(tile, total_tiles);
+      const int per_group = GROUP_M * tiles_n, group = logical / per_group, in = logical - group * per_group;
+      const int group_rows = min(GROUP_M, tiles_m - group * GROUP_M);
+      const int tn = in / group_rows, tm = group * GROUP_M + in - tn * group_rows;
+      n0 = tn * BN;
+      rows_left = M - tm * BM;
+      row_at = (size_t)tm * BM;
+      b_at = n0;
+      bias_row = bias;
+    }
+    const b128 abuf = buffer_words(A + row_at * row_vecs, min(BM, rows_left) * row_bytes);
+    const b128 bbuf = buffer_words(B + b_at * row_vecs, min(BN, N - n0) * row_bytes);
+    int past = 0, soff = k_first;  // past the end of the rows in their last step, and everywhere behind it: out of range
+    unsigned fill = 0, use = 0;
+    auto range = [&](int step) __attribute__((always_inline)) {  // before a step near the end is asked for
+      if (step == steps - 1) past = vec >= tail_vecs ? OUT_OF_RANGE : 0;
+      else if (step >= steps) past = OUT_OF_RANGE;
+    };
+    auto load = [&]() __attribute__((always_inline)) {
+      unrolled<0, LA>([&](auto c) __attribute__((always_inline)) {
+        constexpr int i = decltype(c)::value;
+        load_to_lds<i * NW * 1024>(base + fill, off + i * 8 * NW * row_bytes + past, abuf, soff);
+      });
+      unrolled<0, LB>([&](auto c) __attribute__((always_inline)) {
+        constexpr int i = decltype(c)::value;
+        load_to_lds<B_AT + i * NW * 1024, STREAMED>(base + fill, off + i * 8 * NW * row_bytes + past, bbuf, soff);
+      });
+      fill = fill == RING_BYTES - STEP_BYTES ? 0u : fill + STEP_BYTES;
+      soff += GEMM_KSTEP * 2;
+      if (GROUPED && k_first && soff == row_bytes) soff = 0;
+    };
+#pragma unroll 1
+    for (int step = 0; step < DEPTH; ++step) {
+      range(step);
+      load();
+    }
+    f32x4 acc[TM][TN] = {};
+    b128 af[2][TM], bf[2][TN];  // [slice]
+    auto read_frags = [&](auto slice) __attribute__((always_inline)) {  // of the step in `use`
+      constexpr int s = decltype(slice)::value;
+      const int v = ((s * 4 + q) ^ swz) * 16;
+      const char* as = (const char*)tile_lds + use + (wm * TM * 16 + r) * 128 + v;
+      const char* bs = (const char*)tile_lds + use + B_AT + (wn * TN * 16 + r) * 128 + v;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bf[s][j] = *(const b128*)(bs + j * (16 * 128));
+#pragma unroll
+      for (int i = 0; i < TM; ++i) af[s][i] = *(const b128*)(as + i * (16 * 128));
+    };
+    auto mfmas = [&](auto slice) __attribute__((always_inline)) {
+      constexpr int s = decltype(slice)::value;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = Mfma16x16x32<DT>::mma(bf[s][j], af[s][i], acc[i][j]);
+    };
+    constexpr std::integral_constant<int, 0> first{};
+    constexpr std::integral_constant<int, 1> second{};
+    auto one_step = [&]() __attribute__((always_inline)) {
+      read_frags(second);  // (the first slice is in registers)
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(first);
+      __builtin_amdgcn_sched_barrier(0);
+      // everybody has read this step's rows, whose place the step DEPTH on takes, and the next one's are there for everybody
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(YOUNGER) : "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      load();
+      use = use == RING_BYTES - STEP_BYTES ? 0u : use + STEP_BYTES;
+      read_frags(first);
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(second);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER + LA + LB) : "memory");
+    lds_barrier();
+    read_frags(first);
+    int step = 0;
+    for (; step + DEPTH + 1 < steps; ++step) one_step();  // (what these ask for lies before the last step)
+    for (; step < steps; ++step) {
+      range(step + DEPTH);
+      one_step();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the loads past the last step write zeros)
+    __syncthreads();
+
+    // Out through LDS as in phased_gemm_kernel, a band of 16 rows at a time.
+    constexpr int VR = TN * 2, PITCH = TN * 32 + 16, ROWS_PER_READ = 64 / VR;
+    static_assert(ROWS_PER_READ <= 16 && NW * 16 * PITCH <= RING_BYTES, "bands that a wave reads in whole turns");
+    char* park = (char*)tile_lds + wave * (16 * PITCH);
+    uint16_t* const c_tile = C + row_at * N;
+    const int ncol = n0 + wn * TN * 16;
+    uint32_t bias2[TN][2] = {};
+    if (bias_row) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        if (ncol + j * 16 < N) __builtin_memcpy(bias2[j], bias_row + ncol + j * 16 + q * 4, 8);
+    }
+    const int rrow = lane / VR, rvec = lane % VR;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const f32x4& c = acc[i][j];
+        uint32_t two[2] = {Pair16<DT>::canonical(Pair16<DT>::round(c[0], c[1])), Pair16<DT>::canonical(Pair16<DT>::round(c[2], c[3]))};
+        if (bias_row) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            two[e] = Pair16<DT>::canonical(Pair16<DT>::round(__fadd_rn(Pair16<DT>::lo(two[e]), Pair16<DT>::lo(bias2[j][e])),
+                                                             __fadd_rn(Pair16<DT>::hi(two[e]), Pair16<DT>::hi(bias2[j][e]))));
+        }
+        __builtin_memcpy(park + r * PITCH + (j * 16 + q * 4) * 2, two, 8);
+      }
+#pragma unroll
+      for (int p = 0; p < 16 / ROWS_PER_READ; ++p) {
+        const int row = p * ROWS_PER_READ + rrow;
+        const b128 v = *(const b128*)(park + row * PITCH + rvec * 16);
+        const int m = (wm * TM + i) * 16 + row, n = ncol + rvec * 8;
+        if (m < rows_left && n < N) row_store<THROUGH>((b128*)(c_tile + (size_t)m * N + n), v);
+      }
+    }
+    lds_barrier();  // the results are out of LDS
   }
 }
 
@@ -5625,9 +5819,15 @@ int allow_large_lds() {
     allow((const void*)dense_gemm_kernel<DT, 2, 2, 2, 2, true, S>, dense_lds_bytes(128, 128));
     allow((const void*)ring_gemm_kernel<DT, 1, 1, 8, S>, ring_lds_bytes(1, 1, 8));
     allow((const void*)ring_gemm_kernel<DT, 1, 2, 6, S>, ring_lds_bytes(1, 2, 6));
-    allow((const void*)ring_gemm_kernel<DT, 2, 2, 4, S>, ring_lds_bytes(2, 2, 4));
-    allow((const void*)ring_gemm_kernel<DT, 2, 4, 6, S>, ring_lds_bytes(2, 4, 6));
-    allow((const void*)dense_gemm_kernel<DT, 2, 2, 1, 2, true, S>, dense_lds_bytes(64, 128));
+    allow((const void*)sliced_gemm_kernel<DT, Slices64x64, true, S>, Slices64x64::LDS_BYTES);
+    allow((const void*)sliced_gemm_kernel<DT, Slices64x128, true, S>, Slices64x128::LDS_BYTES);
+    allow((const void*)sliced_gemm_kernel<DT, Slices128x128, true, S>, Slices128x128::LDS_BYTES);
+    allow((const void*)sliced_gemm_kernel<DT, Slices192x128, true, S>, Slices192x128::LDS_BYTES);
+    if constexpr (!S) {
+      allow((const void*)sliced_gemm_kernel<DT, Slices32x64, false, false>, Slices32x64::LDS_BYTES);
+      allow((const void*)sliced_gemm_kernel<DT, Slices64x64, false, false>, Slices64x64::LDS_BYTES);
+      allow((const void*)sliced_gemm_kernel<DT, Slices64x128, false, false>, Slices64x128::LDS_BYTES);
+    }
   };
   allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 8, 4, 3, 4, false, false>, phased_lds_bytes(8, 4, 3, 4));
   allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 8, 4, 3, 4, false, false>, phased_lds_bytes(8, 4, 3, 4));
@@ -5637,9 +5837,7 @@ int allow_large_lds() {
   allow((const void*)phased_gemm_kernel<MOE_A2A_BF16, 6, 2, 3, 4, false, false>, phased_lds_bytes(6, 2, 3, 4));
   allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 4, 2, 3, 4, false, false>, phased_lds_bytes(4, 2, 3, 4));
   allow((const void*)phased_gemm_kernel<MOE_A2A_F16, 6, 2, 3, 4, false, false>, phased_lds_bytes(6, 2, 3, 4));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_BF16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
-  allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 1, 2, false>, dense_lds_bytes(64, 128));
   allow((const void*)dense_gemm_kernel<MOE_A2A_F16, 2, 2, 2, 2, false>, dense_lds_bytes(128, 128));
   allow_grouped(std::integral_constant<int, MOE_A2A_BF16>{}, std::false_type{});
   allow_grouped(std::integral_constant<int, MOE_A2A_BF16>{}, std::true_type{});
@@ -5657,11 +5855,10 @@ int allow_large_lds() {
   return MOE_A2A_OK;
 }
 
-// A product on ring_gemm_kernel, in the tiles that grouped_ring or linear_ring has chosen (rows_of_group null: max_rows rows in
-// every group). MOE_A2A_NOT_DENSE where it has too many.
+// A product on ring_gemm_kernel, in the tiles that grouped_ring has chosen. MOE_A2A_NOT_DENSE where it has too many.
 int launch_grouped_ring(const void* x, const int32_t* rows_of_group, const void* w, const void* bias, void* y, int groups,
                         long long max_rows, long long rows_hint, int N, int K, int dtype, hipStream_t st, int compact, RingTile way) {
-  const int BM = way == RING_32x32 || way == RING_32x64 ? 32 : 64, BN = way == RING_32x32 ? 32 : way == RING_64x128 ? 128 : 64;
+  const int BM = 32, BN = way == RING_32x32 ? 32 : 64;
   const long long tiles_n = (N + BN - 1) / BN;
   // Every group that has a row can end in a partly filled row tile; the kernel strides over what the hint misses. (Workgroups
   // without a tile are not free with so much LDS: 6 rows of 95 groups, 1152 x 192 9.7 us with one for every group.)
@@ -5678,9 +5875,7 @@ int launch_grouped_ring(const void* x, const int32_t* rows_of_group, const void*
                                                                          (uint16_t*)y, N, K, (int)tiles_n, groups, (int)max_rows, compact);
     };
     if (way == RING_32x32) start(ring_gemm_kernel<DT, 1, 1, 8, S>, 8);
-    else if (way == RING_32x64) start(ring_gemm_kernel<DT, 1, 2, 6, S>, 6);
-    else if (way == RING_64x64) start(ring_gemm_kernel<DT, 2, 2, 4, S>, 4);
-    else start(ring_gemm_kernel<DT, 2, 4, 6, S>, 6);
+    else start(ring_gemm_kernel<DT, 1, 2, 6, S>, 6);
   };
   auto launch_of = [&](auto dtype_const) {
     if (streamed) launch(dtype_const, std::true_type{});
@@ -5691,10 +5886,50 @@ int launch_grouped_ring(const void* x, const int32_t* rows_of_group, const void*
   return launch_status();
 }
 
+// A product on sliced_gemm_kernel, in the tiles that grouped_slices or linear_slices has chosen. MOE_A2A_NOT_DENSE where it has too many.
+int launch_slices(const void* x, const int32_t* rows_of_group, const void* w, const void* bias, void* y, int groups, long long max_rows,
+                  long long rows_hint, int N, int K, int dtype, hipStream_t st, int compact, SlicedTile way) {
+  const int BM = sliced_rows(way), BN = sliced_cols(way);
+  const long long tiles_m = (max_rows + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  if (tiles_m * groups * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
+  // (GROUPED: every group that has a row can end in a partly filled row tile; the kernel strides over what the hint misses)
+  const long long pairs = rows_of_group ? (rows_hint / BM + std::min<long long>(groups, std::max(rows_hint, 1ll))) * tiles_n : tiles_m * tiles_n;
+  const int grid = mover_blocks(pairs);
+  if (const int rc = allow_large_lds()) return rc;
+  const bool streamed = rows_of_group && weights_past_the_cache(groups, rows_hint, N, K) && rows_hint <= (long long)groups * BM;
+  auto start = [&](auto dtype_const, auto tile, auto grouped, auto streamed_const) {
+    using TILE = decltype(tile);
+    sliced_gemm_kernel<decltype(dtype_const)::value, TILE, decltype(grouped)::value, decltype(streamed_const)::value>
+        <<<grid, TILE::LANES, TILE::LDS_BYTES, st>>>((const b128*)x, (const b128*)w, (const uint16_t*)bias, (uint16_t*)y, (int)max_rows, N, K,
+                                                     (int)tiles_m, (int)tiles_n, rows_of_group, groups, (int)max_rows, compact);
+  };
+  auto launch_of = [&](auto dtype_const) {
+    auto grouped = [&](auto tile) {
+      if (streamed) start(dtype_const, tile, std::true_type{}, std::true_type{});
+      else start(dtype_const, tile, std::true_type{}, std::false_type{});
+    };
+    auto plain = [&](auto tile) { start(dtype_const, tile, std::false_type{}, std::false_type{}); };
+    if (rows_of_group) {
+      if (way == SLICES_64x64) grouped(Slices64x64{});
+      else if (way == SLICES_64x128) grouped(Slices64x128{});
+      else if (way == SLICES_128x128) grouped(Slices128x128{});
+      else grouped(Slices192x128{});
+    } else {
+      if (way == SLICES_32x64) plain(Slices32x64{});
+      else if (way == SLICES_64x64) plain(Slices64x64{});
+      else plain(Slices64x128{});
+    }
+  };
+  if (dtype == MOE_A2A_BF16) launch_of(std::integral_constant<int, MOE_A2A_BF16>{});
+  else launch_of(std::integral_constant<int, MOE_A2A_F16>{});
+  return launch_status();
+}
+
 // A plain product on tiles that workgroups own whole, as linear_way has chosen.
 int launch_linear_tiles(const void* a, const void* b, const void* bias, void* c, int M, int N, int K, int dtype,
                         LinearWay way, hipStream_t st) {
-  const int BM = way == PHASED_256 ? 256 : way == PHASED_192 ? 192 : way == TILES_64x128 ? 64 : 128;
+  if (way == TILES_64x128) return MOE_A2A_NOT_DENSE;  // (linear_slices: sliced_gemm_kernel has these)
+  const int BM = way == PHASED_256 ? 256 : way == PHASED_192 ? 192 : 128;
   const int BN = way == PHASED_256 ? 256 : 128;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + BN - 1) / BN;
   if (tiles_m * tiles_n > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
@@ -5715,8 +5950,7 @@ int launch_linear_tiles(const void* a, const void* b, const void* bias, void* c,
     else if (way == PHASED_256) LAUNCH_P(DT, 8, 4, false);                                       \
     else if (way == PHASED_192) LAUNCH_P(DT, 6, 2, false);                                       \
     else if (way == PHASED_128) LAUNCH_P(DT, 4, 2, false);                                       \
-    else if (way == TILES_128x128) LAUNCH_D(DT, 2, 2, dense_lds_bytes(128, 128));                \
-    else LAUNCH_D(DT, 1, 2, dense_lds_bytes(64, 128));                                           \
+    else LAUNCH_D(DT, 2, 2, dense_lds_bytes(128, 128));                                          \
   } while (0)
   if (dtype == MOE_A2A_BF16) LAUNCH_DT(MOE_A2A_BF16);
   else LAUNCH_DT(MOE_A2A_F16);
@@ -5738,14 +5972,19 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
-  if (const RingTile ring = rows_of_group && max_rows <= INT_MAX / 2 ? grouped_ring(rows_hint, groups, N, K) : NO_RING) {
+  if (!rows_of_group || max_rows > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
+  const RingTile ring = grouped_ring(rows_hint, groups, N, K);
+  if (ring == RING_32x32 || ring == RING_32x64) {
     const int rc = launch_grouped_ring(x, rows_of_group, w, bias, y, groups, max_rows, rows_hint, N, K, dtype, st, compact, ring);
     if (rc != MOE_A2A_NOT_DENSE) return rc;
   }
-  if (!rows_of_group || rows_hint < (long long)MOE_A2A_GROUPED_DENSE_MIN_ROWS * groups) return MOE_A2A_NOT_DENSE;
-  if (max_rows > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
-  const int bands = grouped_tile_bands(rows_hint, groups, N, K);
-  if (!bands) return MOE_A2A_NOT_DENSE;
+  const bool tiled = rows_hint >= (long long)MOE_A2A_GROUPED_DENSE_MIN_ROWS * groups;
+  const int bands = tiled && !ring ? grouped_tile_bands(rows_hint, groups, N, K) : 0;
+  if (const SlicedTile slices = grouped_slices(ring, bands, rows_hint, groups, N)) {
+    const int rc = launch_slices(x, rows_of_group, w, bias, y, groups, max_rows, rows_hint, N, K, dtype, st, compact, slices);
+    if (rc != MOE_A2A_NOT_DENSE) return rc;
+  }
+  if (!bands || bands == 2) return MOE_A2A_NOT_DENSE;
   const int BM = bands * 32, BN = bands <= 4 ? 128 : 256;
   const long long tiles_n = (N + BN - 1) / BN;
   // every group can end in a partly filled row tile; the kernel strides over what the hint misses
@@ -5767,8 +6006,7 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
     if (bands == 10) phased(phased_gemm_kernel<DT, 10, 4, 2, 5, false, true, S>, phased_lds_bytes(10, 4, 2, 5));
     else if (bands == 8) phased(phased_gemm_kernel<DT, 8, 4, 2, 6, false, true, S>, phased_lds_bytes(8, 4, 2, 6));
     else if (bands == 6) phased(phased_gemm_kernel<DT, 6, 4, 2, 6, false, true, S>, phased_lds_bytes(6, 4, 2, 6));
-    else if (bands == 4) dense(dense_gemm_kernel<DT, 2, 2, 2, 2, true, S>, dense_lds_bytes(128, 128));
-    else dense(dense_gemm_kernel<DT, 2, 2, 1, 2, true, S>, dense_lds_bytes(64, 128));
+    else dense(dense_gemm_kernel<DT, 2, 2, 2, 2, true, S>, dense_lds_bytes(128, 128));
   };
   auto launch_of = [&](auto dtype_const) {
     if (streamed) launch(dtype_const, std::true_type{});
@@ -5816,11 +6054,12 @@ int launch_linear(const void* x, const void* w, const void* bias, void* y, int M
   if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
-  if (const RingTile ring = linear_ring(M, N, K)) {
-    const int rc = launch_grouped_ring(x, nullptr, w, bias, y, 1, M, M, N, K, dtype, st, 0, ring);
+  const RingTile ring = linear_ring(M, N, K);
+  const LinearWay way = ring ? STREAM_WEIGHTS : linear_way(M, N, K);
+  if (const SlicedTile slices = linear_slices(ring, way, M, N, K)) {
+    const int rc = launch_slices(x, nullptr, w, bias, y, 1, M, M, N, K, dtype, st, 0, slices);
     if (rc != MOE_A2A_NOT_DENSE) return rc;
   }
-  const LinearWay way = linear_way(M, N, K);
   int rc = MOE_A2A_NOT_DENSE;
   if (way == SPLIT_32 || way == SPLIT_64) rc = launch_linear_split(x, w, bias, y, M, N, K, dtype, way == SPLIT_32 ? 1 : 2, st);
   else if (way != STREAM_WEIGHTS) rc = launch_linear_tiles(x, w, bias, y, M, N, K, dtype, way, st);

@@ -255,4 +255,48 @@ RingTile linear_ring(long long M, long long N, long long K) {
   return WAIT * UNITS + n * (64 + 64) < least ? RING_64x64 : NO_RING;
 }
 
+// Tiles of sliced_gemm_kernel (rows x columns), or none.
+enum SlicedTile { NO_SLICES = 0, SLICES_32x64, SLICES_64x64, SLICES_64x128, SLICES_128x128, SLICES_192x128 };
+int sliced_rows(SlicedTile t) { return t == SLICES_32x64 ? 32 : t <= SLICES_64x128 ? 64 : t == SLICES_128x128 ? 128 : 192; }
+int sliced_cols(SlicedTile t) { return t <= SLICES_64x64 ? 64 : 128; }
+
+// For a grouped product; `ring` and `bands`: what grouped_ring and (from 56 rows per group on, else 0) grouped_tile_bands have chosen. It takes 64 x
+// 64 and 64 x 128 over from both, and where uniform routing would make for 0.8 of a round of them over the units at most, 128 x 128 from
+// dense_gemm_kernel and 192 x 128 from that and from 192 x 256. (Above, one group of many rows makes a second round: 341 rows in 6 groups by Zipf's
+// routing, 4992 x 672, 0.91 of a round for uniform routing, 16.2 / 24.1 us on 64 x 128 / 128 x 128.) Of 500 products (4 to 64 groups, 1 to 3500 rows
+// per group, N and K of 512 to 7168, a third of them with Zipf's routing) 90 go there, and take of the others' time, as geometric means: those of 64 x
+// 128 of a ring 0.85 and of dense_gemm_kernel 0.67, of 64 x 64 0.94 (2 of 26 more than 3 % behind), of dense_gemm_kernel's 128 x 128 0.84, of 192 x 256
+// 0.80. With fewer rows expert_gemm_kernel stays, whose small blocks read weights from HBM as fast: 42 groups of 25, 1280 x 896, on
+// 64 x 128 23.6 / 23.4 us, 896 x 1280 28.2 / 30.2, and where those are few 41.9 / 54.7 (20 of 23, 768 x 6464).
+SlicedTile grouped_slices(RingTile ring, int bands, long long rows_hint, int groups, int N) {
+  constexpr double UNITS = 256, MOST = 0.8;
+  if (ring) return ring == RING_64x64 ? SLICES_64x64 : ring == RING_64x128 ? SLICES_64x128 : NO_SLICES;
+  if (bands == 2) return SLICES_64x128;
+  auto of_a_unit = [&](int high) {
+    return tiles_of_groups((double)rows_hint / groups, groups, high).each * groups * ((N + 127) / 128) / UNITS;
+  };
+  if (bands == 4 && of_a_unit(128) <= MOST) return SLICES_128x128;
+  return (bands == 4 || bands == 6) && of_a_unit(192) <= MOST ? SLICES_192x128 : NO_SLICES;
+}
+
+// For a plain product; `ring` and `way`: what linear_ring and, without one, linear_way have chosen. It takes over all of the ring's tiles, all of 64 x
+// 128 (on the smallest tiles of which every unit has one at most, else as they are), and of the products split over K those of 33 to 96 rows that
+// give nearly every unit a tile of 32 x 64; up to 64 of them only with weights that the L2s hold: two tiles wait for the same rows out of HBM. Of 300
+// products (16 to 8192 rows, N 1024 to 8192, K 256 to 8192) 98, at 0.86 of the others' time, none behind, and 11 split ones at 0.91 (one 4 % behind: 70 x
+// 4704 x 688 5.10 / 5.29). us, 37 x 7808 x 448 on 64 x 128 / 64 x 64 / 32 x 64: 5.59 / 4.82 / 4.76; 148 x 3680 x 448 (87, 174 and 290 tiles) 5.71 /
+// 4.92 / 5.86; 500 x 2976 x 448 (192, 376, 752) 5.86 / 6.56 / 8.28. Split over K / here, the same weights again and others out of HBM: 64 x 7168 x 2304
+// (32 MiB) 9.3 / 8.9, 12.1 / 12.0; 88 x 5056 x 2432 10.2 / 8.6, 13.8 / 11.8; 90 x 4480 x 6000 24.4 / 19.9, 31.8 / 30.3; but 64 x 7008 x 3008 11.3 /
+// 10.2, 14.2 / 14.9; 33 x 7776 x 8080 25.7 / 31.4, 35.5 / 32.8. With fewer tiles or more rows splitting K stays ahead: 52 x 5824 x 3624 (182 tiles)
+// 0.99 of its time here, 183 x 1120 x 960 (108) 1.24, 295 x 1536 x 8000 (240) 1.12.
+// 192 x 128 stay phased_gemm_kernel's: launched one after the other in a graph they are up to 4 % ahead here, in calls of their own 2 to 3 % behind
+// (2048 x 2880 x 360 9.98 / 10.16, 1399 x 3904 x 3016 42.6 / 43.8).
+SlicedTile linear_slices(RingTile ring, LinearWay way, long long M, long long N, long long K) {
+  constexpr long long UNITS = 256;
+  auto tiles = [&](int rows, int columns) { return (M + rows - 1) / rows * ((N + columns - 1) / columns); };
+  if (ring == RING_64x64) return SLICES_64x64;
+  if (ring || way == TILES_64x128) return tiles(32, 64) <= UNITS ? SLICES_32x64 : tiles(64, 64) <= UNITS ? SLICES_64x64 : SLICES_64x128;
+  const bool split = way == SPLIT_32 || way == SPLIT_64, held = M > 64 || N * K * 2 <= 32 << 20;
+  return split && held && M > 32 && M <= 96 && tiles(32, 64) >= 200 && tiles(32, 64) <= UNITS ? SLICES_32x64 : NO_SLICES;
+}
+
 }  // namespace
