@@ -77,6 +77,12 @@ typedef unsigned int b128 __attribute__((ext_vector_type(4)));
 //  - exchange: 8 MB of rows for a rank (0.03 MB of 512 B 2.25 / 2.41, 3.9 MB 6.30 / 7.31; 8 MB of 2 KB 5.01 / 5.27, 16 MB 8.46
 //    / 7.80; 3.9 MB of 8 KB 3.18 / 3.31, 6.2 MB 3.67 / 3.61).
 enum Store { PLAIN, THROUGH, STREAM };
+//  - results of a job whose ranks share the GPU, past the cache behind L2, where they and the rows they are added up from are 80 MB, with several ranks
+//    128 MB: what is left dirty there goes out line by line among the reads of whatever comes next. us of the whole call, plain / stream: layer of 32
+//    experts, 2048 x 4096, 2048 tokens, 4 per token (84 MB) 337 / 333, of 64, 1024 x 4096, 2048 tokens, 8 per token (151 MB) 413 / 410; 8 ranks of
+//    256 tokens, 8 per token of 14 KB (264 MB) 92.5 / 91.4, of 8 KB (151 MB) 55.7 / 55.4, but of 189, 4 per token of 11 KB (84 MB) 38.1 / 38.7.
+//    Nontemporal loads of the rows as well: 330, 410; 94.3, 54.6.
+constexpr long long JOB_STREAM_BYTES = 80ll << 20, JOB_RANKS_STREAM_BYTES = 128ll << 20;
 constexpr long long JOB_THROUGH_BYTES = 1 << 20, EXCHANGE_THROUGH_BYTES = 8 << 20;  // (stage 2's: recv_through)
 // (a kernel for each kind: chosen inside one, the stores of 5.5 MB of rows took 0.3 us longer than either)
 template <typename V> constexpr Store THROUGH_OF = sizeof(V) == sizeof(b128) ? THROUGH : PLAIN;  // (of 16 bytes only)
@@ -4736,13 +4742,16 @@ __global__ __launch_bounds__(BLOCK) void local_dispatch_few_kernel(
   }
 }
 
-// MANY: more than eight entries per token.
+// ADDENDS: 2, 4, 6 or 8, no fewer than a token's entries, whose rows are all under way at once; 0 for more of them, in batches of 8. Past the last one
+// its row is loaded again, which costs as much as another (us, all with 8 / as many as here, 3 per token: 3907 tokens of 4.3 KB 15.4 / 14.2; 2 per token:
+// 2987 of 6.4 KB 17.4 / 13.2; 1: 3683 of 7.2 KB 17.4 / 13.2; 6, of 8 ranks: 238 of 4.5 KB 13.7 / 12.4).
 // weights0 and out0 are rank 0's, which is all that a job of one rank has (R = 1).
-template <typename V, int DT, int NV, bool MANY, int R>
+template <typename V, int DT, int NV, int ADDENDS, Store HOW, int R>
 __global__ __launch_bounds__(BLOCK) void local_combine_kernel(
     const int* __restrict__ entry_row, const float* weights0, const V* __restrict__ rows, void* out0, int K, int chunks,
     int row_vecs, int first_token, int accumulate, int W, LocalResults<R> dst) {
-  constexpr int N = Words<V>::N, BATCH = 8;
+  constexpr int N = Words<V>::N, BATCH = ADDENDS ? ADDENDS : 8, RUN = BATCH > 4 ? 8 : 4;
+  constexpr bool MANY = ADDENDS == 0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int q = blockIdx.x;
   const int item = chunks == 1 ? q : q / chunks, c = q - item * chunks;
@@ -4758,8 +4767,8 @@ __global__ __launch_bounds__(BLOCK) void local_combine_kernel(
   }
   const int base = c * (BLOCK * NV);
   V* __restrict__ orow = (V*)out + (size_t)local_t * row_vecs;
-  // entry of this lane; lanes repeat the entries in runs of 8 unless there are more
-  const int k = MANY ? lane : lane & (BATCH - 1);
+  // entry of this lane; lanes repeat the entries in runs of 4 or 8 unless there are more
+  const int k = MANY ? lane : lane & (RUN - 1);
   const bool there = k < K;
   const int loaded = entry_row[(size_t)t * K + min(k, K - 1)];
   const float w_loaded = weights[(size_t)local_t * K + min(k, K - 1)];
@@ -4772,17 +4781,18 @@ __global__ __launch_bounds__(BLOCK) void local_combine_kernel(
     for (int e = 0; e < N; ++e) acc[j][e].set(get_word(o, e));
   }
   const int mine = there && loaded >= 0 ? loaded : INT_MAX;
-  const int n = __popcll(__ballot(mine != INT_MAX && lane < (MANY ? 64 : BATCH)));
+  const int n = __popcll(__ballot(mine != INT_MAX && lane < (MANY ? 64 : RUN)));
   // place of this lane's row among the token's rows (all different), then rows and weights in order
   int place = 0;
   if constexpr (MANY) {
     for (int b = 0; b < K; ++b) place += (int)(__builtin_amdgcn_readlane(mine, b) < mine);
   } else {
 #define MOE_A2A_ROT(S) place += (int)(__builtin_amdgcn_update_dpp(0, mine, 0x120 + S, 0xf, 0xf, false) < mine)
-    MOE_A2A_ROT(1); MOE_A2A_ROT(2); MOE_A2A_ROT(3); MOE_A2A_ROT(4); MOE_A2A_ROT(5); MOE_A2A_ROT(6); MOE_A2A_ROT(7);
+    MOE_A2A_ROT(1); MOE_A2A_ROT(2); MOE_A2A_ROT(3);
+    if constexpr (RUN > 4) { MOE_A2A_ROT(4); MOE_A2A_ROT(5); MOE_A2A_ROT(6); MOE_A2A_ROT(7); }
 #undef MOE_A2A_ROT
   }
-  const int to = (MANY ? place : (lane & ~(BATCH - 1)) | place) << 2;  // (lanes without a row all get place n, which nothing reads)
+  const int to = (MANY ? place : (lane & ~(RUN - 1)) | place) << 2;  // (lanes without a row all get place n, which nothing reads)
   const int ordered_row = __builtin_amdgcn_ds_permute(to, mine);
   const int ordered_w = __builtin_amdgcn_ds_permute(to, __float_as_int(w_loaded));
   for (int a0 = 0; a0 < n; a0 += BATCH) {
@@ -4815,7 +4825,7 @@ __global__ __launch_bounds__(BLOCK) void local_combine_kernel(
       uint32_t h[N];
 #pragma unroll
       for (int e = 0; e < N; ++e) h[e] = acc[j][e].word();
-      orow[idx] = from_words<V>(h);
+      row_store<HOW>(orow + idx, from_words<V>(h));
     }
   }
 }
@@ -6389,28 +6399,44 @@ int moe_a2a_local_combine(const moe_a2a_shape* s, const void* expert_rows, const
   const int grid = (int)(items * chunks);
   hipStream_t st = (hipStream_t)stream;
   const bool few_ranks = W <= LOCAL_FEW_RANKS && grid <= LOCAL_FEW_WORKGROUPS;
-#define LAUNCH_R(V, DT, NV, MANY, R)                                                                       \
-  local_combine_kernel<V, DT, NV, MANY, R><<<grid, BLOCK, 0, st>>>(                                        \
+  const bool streams = g.vec16 && (items * K + items) * s->hidden_dim * 2 >= (W == 1 ? JOB_STREAM_BYTES : JOB_RANKS_STREAM_BYTES);
+  // (of rows in several chunks three entries and more stay with eight, whose workgroups, fewer on a unit, have fewer rows open at once: 8 ranks, us
+  // with 8 / as many as there are, 193 tokens of 12 KB, 3 per token 13.7 / 14.0, 184 of 10.7 KB, 4 per token 14.5 / 15.0, 162 of 11 KB, 6 17.2 / 17.6)
+  const bool long_rows = g.row_vecs > 2 * BLOCK;
+#define LAUNCH_R(V, DT, NV, ADDENDS, HOW, R)                                                               \
+  local_combine_kernel<V, DT, NV, ADDENDS, HOW, R><<<grid, BLOCK, 0, st>>>(                                \
       entry_row, weights[0], (const V*)expert_rows, out_tokens[0], K, chunks, g.row_vecs, first, accumulate, W, \
       results(LocalResults<R>{}))
-#define LAUNCH(V, DT, NV, MANY)                                                                            \
+#define LAUNCH(V, DT, NV, ADDENDS, HOW)                                                                    \
   do {                                                                                                     \
-    if (W == 1) LAUNCH_R(V, DT, NV, MANY, 1);                                                              \
-    else if (few_ranks) LAUNCH_R(V, DT, NV, MANY, LOCAL_FEW_RANKS);                                        \
-    else LAUNCH_R(V, DT, NV, MANY, LOCAL_MAX_RANKS);                                                       \
+    if (W == 1) LAUNCH_R(V, DT, NV, ADDENDS, HOW, 1);                                                      \
+    else if (few_ranks) LAUNCH_R(V, DT, NV, ADDENDS, HOW, LOCAL_FEW_RANKS);                                \
+    else LAUNCH_R(V, DT, NV, ADDENDS, HOW, LOCAL_MAX_RANKS);                                               \
   } while (0)
-#define PICK(V, DT)                                                                                        \
+#define LAUNCH_N(V, DT, ADDENDS, HOW)                                                                      \
   do {                                                                                                     \
-    if (K <= 8) { if (nv == 1) LAUNCH(V, DT, 1, false); else LAUNCH(V, DT, 2, false); }                    \
-    else { if (nv == 1) LAUNCH(V, DT, 1, true); else LAUNCH(V, DT, 2, true); }                             \
+    if (nv == 1) LAUNCH(V, DT, 1, ADDENDS, HOW);                                                           \
+    else LAUNCH(V, DT, 2, ADDENDS, HOW);                                                                   \
   } while (0)
-  if (g.vec16) {
-    if (dtype == MOE_A2A_BF16) PICK(b128, MOE_A2A_BF16);
-    else PICK(b128, MOE_A2A_F16);
-  } else {
-    if (dtype == MOE_A2A_BF16) PICK(uint16_t, MOE_A2A_BF16);
-    else PICK(uint16_t, MOE_A2A_F16);
-  }
+#define LAUNCH_H(DT, ADDENDS)                                                                              \
+  do {                                                                                                     \
+    if (streams) LAUNCH_N(b128, DT, ADDENDS, STREAM);                                                      \
+    else LAUNCH_N(b128, DT, ADDENDS, PLAIN);                                                               \
+  } while (0)
+#define PICK(DT)                                                                                           \
+  do {                                                                                                     \
+    if (!g.vec16 && K <= 8) LAUNCH_N(uint16_t, DT, 8, PLAIN);                                              \
+    else if (!g.vec16) LAUNCH_N(uint16_t, DT, 0, PLAIN);                                                   \
+    else if (K <= 2) LAUNCH_H(DT, 2);                                                                      \
+    else if (K <= 4 && !long_rows) LAUNCH_H(DT, 4);                                                        \
+    else if (K <= 6 && !long_rows) LAUNCH_H(DT, 6);                                                        \
+    else if (K <= 8) LAUNCH_H(DT, 8);                                                                      \
+    else LAUNCH_H(DT, 0);                                                                                  \
+  } while (0)
+  if (dtype == MOE_A2A_BF16) PICK(MOE_A2A_BF16);
+  else PICK(MOE_A2A_F16);
+#undef LAUNCH_H
+#undef LAUNCH_N
 #undef PICK
 #undef LAUNCH
 #undef LAUNCH_R
