@@ -2360,6 +2360,109 @@ __global__ __launch_bounds__(BLOCK) void combine_recv_mapped_kernel(
   }
 }
 
+// Stage 4 for up to eight entries per token without a table: one pass of sixteen waves over the arriving meta rows notes what is addressed to any
+// of the workgroup's tokens, in whatever order; then a wave per (token, piece of 64 vectors) orders the token's rows by arrival and has all of
+// them under way at once. A token with more than ADDENDS rows (pairs that arrive twice) is added up from another walk over the stream.
+// Bound by the trips (counts and metas, rows) and, with many tokens, by the rows: a workgroup per token and 256 vectors, each of which reads all
+// metas, spent most of its time on those. us, that / here: 885 tokens of 5.8 KB, 4 per token 10.8 / 7.2, 939 of 8.4 KB, 2 each 10.2 / 6.8, 1428
+// of 7.6 KB, 2 each 11.7 / 7.8, 1622 of 1 KB, 1 each 6.2 / 4.3, 377 of 10 KB, 6 each 8.4 / 7.4. Results stored plainly 0.1 to 0.4 us longer.
+template <int DT, int ADDENDS>
+__global__ __launch_bounds__(COMBINE_BLOCK) void combine_recv_block_kernel(
+    const int* __restrict__ recv_meta, const int* __restrict__ recv_counts, const float* __restrict__ weights, int W, int hint_rows, int T,
+    int K, int tokens, Pieces pieces, int capacity_rows, const b128* __restrict__ recv_buf, int row_vecs, int accumulate,
+    b128* __restrict__ out) {
+  constexpr int N = Words<b128>::N, FAST = 8, UNROLL = 4, WAVES = COMBINE_BLOCK / 64;
+  __shared__ int hits[COMBINE_TOKENS], hit[COMBINE_TOKENS * FAST];  // rows of a token; their numbers * 8 + entry
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int t0 = blockIdx.x * tokens, here = min(tokens, T - t0);
+  const int raw_count = recv_counts[min(lane, W - 1)];
+  if (tid < COMBINE_TOKENS) hits[tid] = 0;
+  int tk[UNROLL][2];
+  auto fetch = [&](int b, int end) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u)
+      __builtin_memcpy(tk[u], recv_meta + (size_t)min(b + tid + u * COMBINE_BLOCK, end - 1) * META + 2, 8);
+  };
+  auto note = [&](int b, int end) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int row = b + tid + u * COMBINE_BLOCK, t = tk[u][0] - t0;
+      if (row < end && (uint32_t)t < (uint32_t)here && (uint32_t)tk[u][1] < (uint32_t)K) {
+        const int p = atomicAdd(&hits[t], 1);
+        if (p < FAST) hit[t * FAST + p] = row << 3 | tk[u][1];
+      }
+    }
+  };
+  const int ahead = min(hint_rows, UNROLL * COMBINE_BLOCK);  // (readable whatever the counts say; more than none)
+  fetch(0, ahead);
+  lds_barrier();
+  const int my_count = lane < W ? min(max(first_use(raw_count), 0), capacity_rows) : 0;
+  const int R = min(W <= 64 ? wave_sum(my_count) : sum_counts(recv_counts, W, capacity_rows), capacity_rows);
+  note(0, min(ahead, R));
+  for (int b = ahead; b < R; b += UNROLL * COMBINE_BLOCK) {
+    fetch(b, R);
+    note(b, R);
+  }
+  lds_barrier();
+
+  const int items = here * pieces.per_row;
+  for (int q = wave; q < items; q += WAVES) {
+    const int item = pieces.row_of(q), at = (q - item * pieces.per_row) * 64 + lane, col = min(at, row_vecs - 1), t = t0 + item;
+    const int n = __builtin_amdgcn_readfirstlane(hits[item]);
+    const float* const w_row = weights + (size_t)t * K;
+    b128* __restrict__ orow = out + (size_t)t * row_vecs;
+    PairAcc<DT> acc[N];
+    b128 o{};
+    if (accumulate) o = orow[col];
+#pragma unroll
+    for (int e = 0; e < N; ++e) acc[e].set(get_word(o, e));
+    if (n <= ADDENDS) {
+      const int p = lane & (FAST - 1);
+      const int mine = p < n ? hit[item * FAST + p] : INT_MAX;
+      const float w = w_row[p < n ? mine & 7 : 0];
+      int place = 0;
+#define MOE_A2A_ROT(S) place += (int)(__builtin_amdgcn_update_dpp(0, mine, 0x120 + S, 0xf, 0xf, false) < mine)
+      MOE_A2A_ROT(1); MOE_A2A_ROT(2); MOE_A2A_ROT(3); MOE_A2A_ROT(4); MOE_A2A_ROT(5); MOE_A2A_ROT(6); MOE_A2A_ROT(7);
+#undef MOE_A2A_ROT
+      const int to = ((lane & ~(FAST - 1)) | place) << 2;  // (lanes without a row all get place n, which nothing reads)
+      const int ordered = __builtin_amdgcn_ds_permute(to, mine);
+      b128 v[ADDENDS];
+#pragma unroll
+      for (int u = 0; u < ADDENDS; ++u)
+        if (u < n) v[u] = *(unknown_origin(recv_buf + (size_t)(__builtin_amdgcn_readlane(ordered, u) >> 3) * row_vecs) + col);
+      issued_here();
+      const int ordered_w = __builtin_amdgcn_ds_permute(to, __float_as_int(w));
+#pragma unroll
+      for (int u = 0; u < ADDENDS; ++u) {
+        if (u < n) {
+          const float wu = __int_as_float(__builtin_amdgcn_readlane(ordered_w, u));
+#pragma unroll
+          for (int e = 0; e < N; ++e) acc[e].step(get_word(v[u], e), wu);
+        }
+      }
+    } else {
+      for (int b = 0; b < R; b += 64) {
+        int key[2];
+        __builtin_memcpy(key, recv_meta + (size_t)min(b + lane, R - 1) * META + 2, 8);
+        unsigned long long mine = __ballot(b + lane < R && key[0] == t && (uint32_t)key[1] < (uint32_t)K);
+        for (; mine; mine &= mine - 1) {
+          const int l = __builtin_ctzll(mine);
+          const float wu = w_row[__builtin_amdgcn_readlane(key[1], l)];
+          const b128 v = recv_buf[(size_t)(b + l) * row_vecs + col];
+#pragma unroll
+          for (int e = 0; e < N; ++e) acc[e].step(get_word(v, e), wu);
+        }
+      }
+    }
+    if (at < row_vecs) {
+      uint32_t h[N];
+#pragma unroll
+      for (int e = 0; e < N; ++e) h[e] = acc[e].word();
+      row_store<THROUGH>(orow + at, from_words<b128>(h));
+    }
+  }
+}
+
 // The same for a short stream (hint_rows <= 64 * KEYS): every wave looks through all of it by itself. The rows of 64 keys
 // that are the token's come out of a ballot in arrival order, so there is nothing to sort and no other wave to wait for.
 // ADDENDS: rows under way at a time. us, one launch after another in a graph, before / here: 72 rows of 1 KB, 6 per token
@@ -5502,6 +5605,28 @@ int launch_combine_recv(const moe_a2a_shape* s, const void* recv_buf, const int3
     else { if (nv == 1) LAUNCH(MOE_A2A_F16, 1); else LAUNCH(MOE_A2A_F16, 2); }
 #undef LAUNCH
 #undef LAUNCH_K
+#undef LAUNCH_A
+    return launch_status();
+  }
+  // Above one token per unit a workgroup looks through the stream for several at once (combine_block).
+  const int block_pieces = (g.row_vecs + 63) / 64;
+  const int block_tokens = mapped || !g.vec16 || capacity_rows >= 1 << 28 || block_pieces > INT_MAX / 2 / COMBINE_TOKENS
+                               ? 0 : combine_block(num_tokens, rows_hint, K);
+  if (block_tokens) {
+    const int block_grid = (num_tokens + block_tokens - 1) / block_tokens;
+#define LAUNCH_A(DT, ADDENDS)                                                                                    \
+  combine_recv_block_kernel<DT, ADDENDS><<<block_grid, COMBINE_BLOCK, 0, st>>>(                                  \
+      recv_meta, recv_counts, weights, W, rows_hint, num_tokens, K, block_tokens, pieces_of(block_pieces),       \
+      capacity_rows, (const b128*)recv_buf, g.row_vecs, accumulate, (b128*)out_tokens)
+#define LAUNCH(DT)                   \
+  do {                               \
+    if (K <= 2) LAUNCH_A(DT, 2);     \
+    else if (K <= 4) LAUNCH_A(DT, 4); \
+    else LAUNCH_A(DT, 8);            \
+  } while (0)
+    if (dtype == MOE_A2A_BF16) LAUNCH(MOE_A2A_BF16);
+    else LAUNCH(MOE_A2A_F16);
+#undef LAUNCH
 #undef LAUNCH_A
     return launch_status();
   }

@@ -193,6 +193,17 @@ RecvFew recv_few(long long rows_hint, int row_vecs, int nvw, bool vec16, bool co
 constexpr long long COMBINE_PAST_BYTES = 80ll << 20;
 int mapped_vecs(int per_token, int row_vecs, bool past) { return row_vecs > 64 && per_token <= (past ? 4 : 2) ? 2 : 1; }
 
+// Tokens of a workgroup of combine_recv_block_kernel, or 0 where a workgroup looks for the rows of one token: up to as many tokens as there are units
+// that has no less to share (256 of 14 KB, 8 per token 8.1 / 8.7 us, 128 of 11 KB, 7 each 5.1 / 5.4; 278 of 8.6 KB, 4 each 5.4 / 5.4). One workgroup
+// per unit, two where there are three tokens for each. us, with 256 / 512 / 1024 of them: 377 of 10 KB, 6 each 7.4 / 8.0 / 8.0; 531 of 6.4
+// KB, 2 each 4.9 / 5.2 / 5.6; 885 of 5.8 KB, 4 each 7.5 / 7.2 / 9.3; 1428 of 7.6 KB, 2 each 8.8 / 7.8 / 9.2; 1622 of 1 KB 4.5 / 4.4 / 5.2.
+constexpr int COMBINE_BLOCK = 1024, COMBINE_TOKENS = 64;  // lanes, and most tokens, of a workgroup
+int combine_block(long long tokens, long long rows_hint, int per_token) {
+  if (tokens <= 256 || rows_hint <= 512 || per_token > 8) return 0;
+  const int workgroups = tokens >= 768 ? 512 : 256;
+  return (int)std::min<long long>(COMBINE_TOKENS, (tokens + workgroups - 1) / workgroups);
+}
+
 // ---------------------------------------------------------------- jobs on one GPU
 
 // Vectors of a row that a lane of local_dispatch_few_kernel moves: one, two or four, of single elements one, four or eight. Every
