@@ -4441,7 +4441,8 @@ __global__ __launch_bounds__(BLOCK) void exchange_gather_kernel(
 //   local_plan_kernel      the expert-buffer row of every (rank, token, k) entry (entry_row), in the order in
 //                          which the stages would have put it there: by source rank, token and k inside an
 //                          expert. Left out for up to LOCAL_FEW_RANKS ranks with LOCAL_RANK_ENTRIES entries
-//                          between them, whose mover ranks them itself (local_dispatch_few_kernel).
+//                          between them, whose mover ranks them itself (local_dispatch_few_kernel), and for up to
+//                          32768 entries of whole vectors (local_dispatch_long_kernel).
 //   local_dispatch_kernel  one workgroup per (token, chunk of its row) reads the chunk once and stores it to
 //                          all of the token's expert rows, as it is or through the stand-in expert.
 //   local_combine_kernel   one workgroup per (token, chunk): gathers the token's expert rows and adds them up
@@ -4514,11 +4515,12 @@ constexpr int LPLAN_BLOCK = 1024, LPLAN_WAVES = LPLAN_BLOCK / 64;
 //   rank_limit     > 0: entries past that many of their destination rank are dropped (what its receive
 //                  buffer holds). Reached only by tokens that name an expert more than once.
 // Entries with an expert outside [0, E) have no row. The last workgroup writes the rows per expert.
+// Here: the row of the lane's entry, of up to one per lane from `begin` to before `end`; `entry_expert` is what the entry names.
 template <int R>
-__global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
-    LocalSources<R> src, int W, int S, int K, int E, int nle, int expert_bits, int rank_bits, bool compact, int max_recv,
-    int expert_limit, int rank_limit, int* __restrict__ entry_row, int* __restrict__ expert_num_tokens,
-    int* __restrict__ expert_offsets) {
+__device__ __forceinline__ int local_plan(
+    const LocalSources<R>& src, int W, int S, int K, int E, int nle, int expert_bits, int rank_bits, bool compact, int max_recv,
+    int expert_limit, int rank_limit, int begin, int end, int* __restrict__ expert_num_tokens,
+    int* __restrict__ expert_offsets, int& entry_expert) {
   extern __shared__ int plan_lds[];            // before[E], total[E], in_wave[LPLAN_WAVES][E]
   int* const before = plan_lds;
   int* const total = plan_lds + E;
@@ -4530,7 +4532,6 @@ __global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
   __shared__ int red[LPLAN_WAVES];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const unsigned long long lanes_below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-  const int begin = blockIdx.x * LPLAN_BLOCK;
   const bool last = blockIdx.x == gridDim.x - 1;
   if (tid <= W) first_entry[tid] = src.first[tid] * K;
   if (tid < W) keys_of[tid] = src.indices[tid];
@@ -4548,7 +4549,8 @@ __global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
     return keys_of[r][i - first_entry[r]];
   };
   const int i = begin + tid;
-  const int e = i < S ? key_at(i) : -1;
+  const int e = i < end ? key_at(i) : -1;
+  entry_expert = e;
   const int scanned = compact ? S : begin;
   // compact: both counts of an expert in one word where they fit, all entries below, those before the tile above
   const bool packed = compact && S <= 0xffff;
@@ -4657,7 +4659,19 @@ __global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
       expert_num_tokens[j] = n;
     }
   }
-  if (i < S) entry_row[i] = !keep ? -1 : compact ? total[e] + pos : e * max_recv + pos;
+  return !keep ? -1 : compact ? total[e] + pos : e * max_recv + pos;
+}
+
+template <int R>
+__global__ __launch_bounds__(LPLAN_BLOCK) void local_plan_kernel(
+    LocalSources<R> src, int W, int S, int K, int E, int nle, int expert_bits, int rank_bits, bool compact, int max_recv,
+    int expert_limit, int rank_limit, int* __restrict__ entry_row, int* __restrict__ expert_num_tokens,
+    int* __restrict__ expert_offsets) {
+  const int begin = blockIdx.x * LPLAN_BLOCK, i = begin + threadIdx.x;
+  int e;
+  const int row = local_plan<R>(src, W, S, K, E, nle, expert_bits, rank_bits, compact, max_recv, expert_limit, rank_limit, begin,
+                                min(S, begin + LPLAN_BLOCK), expert_num_tokens, expert_offsets, e);
+  if (i < S) entry_row[i] = row;
 }
 
 // The token's row, held by the workgroup, to its K places: row_of and own hold the places and experts of entries, one per
@@ -4703,6 +4717,62 @@ __global__ __launch_bounds__(BLOCK) void local_dispatch_kernel(
   p.load((const V*)of_rank<R>(src.x, r) + (size_t)local_t * row_vecs, base, row_vecs);
   local_rows_out<DIN, DOUT, HOW>(p, base, row_vecs, K, row_of, own, nle, magic, rows);
   if (c == 0 && meta) local_meta_out(K, row_of, own, r, local_t, meta);
+}
+
+// The same with the plan in it: a workgroup ranks the entries of `tokens` tokens and its waves move their rows, pieces of 64 * NV vectors, the first
+// ones of which are on their way while it counts. Every workgroup counts up to all keys, at once and about as long as the last one of a plan, whose
+// launch is saved. Bound by memory, on small jobs by that count. us of both launches / here: 8 ranks, 2048 tokens of 14 KB, 8 per token 49.3 /
+// 47.6 (6.4 TB/s in the rows), 1920 of 11 KB, 7 each 34.9 / 31.9, 1528 of 7 KB, 4 each 16.0 / 14.1, 520 of 8.6 KB, 5 each 13.8 / 11.2; one rank, 2048 of 8 KB,
+// 4 each 20.2 / 17.7, 3084 of 1.6 KB, 2 each 9.9 / 7.2.
+template <int NV, int DIN, int DOUT, int R>
+__global__ __launch_bounds__(LPLAN_BLOCK) void local_dispatch_long_kernel(
+    LocalSources<R> src, int W, int S, int K, int E, int nle, uint32_t magic, int expert_bits, int rank_bits, bool compact, int max_recv,
+    int expert_limit, int rank_limit, int tokens, Pieces pieces, int row_vecs, int* __restrict__ entry_row,
+    int* __restrict__ expert_num_tokens, int* __restrict__ expert_offsets, b128* __restrict__ rows, int* __restrict__ meta) {
+  __shared__ int places[LOCAL_LONG_ENTRIES], experts[LOCAL_LONG_ENTRIES];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int t0 = blockIdx.x * tokens, begin = t0 * K, end = min(S, begin + tokens * K);
+  const int items = (end - begin) / K * pieces.per_row;
+  WavePayload<b128, NV> p;
+  auto load = [&](int q) __attribute__((always_inline)) {
+    const int item = pieces.row_of(q), r = rank_of_token<R>(src.first, W, t0 + item), local_t = t0 + item - of_rank<R>(src.first, r);
+    p.load((const b128*)of_rank<R>(src.x, r) + (size_t)local_t * row_vecs, (q - item * pieces.per_row) * (64 * NV), row_vecs, lane);
+  };
+  if (wave < items) load(wave);
+  int e;
+  const int row = local_plan<R>(src, W, S, K, E, nle, expert_bits, rank_bits, compact, max_recv, expert_limit, rank_limit, begin, end,
+                                expert_num_tokens, expert_offsets, e);
+  if (begin + tid < end) {
+    entry_row[begin + tid] = row;
+    places[tid] = row;
+    experts[tid] = e;
+  }
+  lds_barrier();
+  for (int q = wave; q < items; q += LPLAN_WAVES) {
+    if (q != wave) load(q);
+    const int item = pieces.row_of(q), base = (q - item * pieces.per_row) * (64 * NV);
+    const int row_of = places[item * K + min(lane, K - 1)], own = experts[item * K + min(lane, K - 1)];
+    for (int k = 0; k < K; ++k) {
+      const int to = __builtin_amdgcn_readlane(row_of, k);
+      if (to < 0) continue;
+      WavePayload<b128, NV> y = p;
+      if constexpr (DIN >= 0) {
+        const int of = __builtin_amdgcn_readlane(own, k);
+        const float scale = (float)(1 + (nle == 1 ? of : (int)__umulhi((uint32_t)of, magic)));
+#pragma unroll
+        for (int j = 0; j < NV; ++j) y.v[j] = standin_expert<b128, DIN, DOUT>(p.v[j], scale);
+      }
+      y.template store<THROUGH>(rows + (size_t)to * row_vecs, base, row_vecs, lane);
+    }
+    if (base == 0 && meta) {
+      const int t = t0 + item, r = rank_of_token<R>(src.first, W, t), local_t = t - of_rank<R>(src.first, r);
+      for (int m0 = 0; m0 < K * META; m0 += 64) {  // (the same trips for every lane: they shuffle)
+        const int m = m0 + lane, k = min(m / META, K - 1), f = m - k * META;
+        const int to = __shfl(row_of, k, 64), of = __shfl(own, k, 64);
+        if (m < K * META && to >= 0) meta[(size_t)to * META + f] = f == 0 ? of : f == 1 ? r : f == 2 ? local_t : f == 3 ? k : 0;
+      }
+    }
+  }
 }
 
 // The same without a plan, for few entries of few ranks: every wave holds all keys (KEYS per lane) and ranks entries of its own
@@ -6448,6 +6518,33 @@ int moe_a2a_local_dispatch(const moe_a2a_shape* s, const void* const* x, const i
   while ((1 << expert_bits) < E) ++expert_bits;
   while ((1 << rank_bits) < W) ++rank_bits;
   if (const int rc = allow_large_lds()) return rc;
+  if (const int each = g.vec16 ? local_long_tokens(tokens, K, W, E) : 0) {  // the movers rank theirs themselves
+    const int nv = local_long_vecs((long long)S * s->hidden_dim * 2, g.row_vecs), pieces = (g.row_vecs + 64 * nv - 1) / (64 * nv);
+    const int grid = (int)((tokens + each - 1) / each);
+    auto start = [&](auto table) {
+      constexpr int R = sizeof(table.x) / sizeof(table.x[0]);
+#define LAUNCH_H(NV, DI, DO)                                                                               \
+  local_dispatch_long_kernel<NV, DI, DO, R><<<grid, LPLAN_BLOCK, local_plan_lds_bytes(E), st>>>(           \
+      table, W, S, K, E, g.nle, g.magic, expert_bits, rank_bits, compact, g.max_recv, expert_limit, rank_limit, each, \
+      pieces_of(pieces), g.row_vecs, entry_row, expert_num_tokens, expert_offsets, (b128*)expert_rows, expert_meta)
+#define LAUNCH(NV)                                                                                         \
+  do {                                                                                                     \
+    if (!standin) LAUNCH_H(NV, -1, -1);                                                                    \
+    else if (in_dtype == MOE_A2A_BF16 && out_dtype == MOE_A2A_BF16) LAUNCH_H(NV, MOE_A2A_BF16, MOE_A2A_BF16); \
+    else if (in_dtype == MOE_A2A_F16 && out_dtype == MOE_A2A_F16) LAUNCH_H(NV, MOE_A2A_F16, MOE_A2A_F16);  \
+    else if (in_dtype == MOE_A2A_F16) LAUNCH_H(NV, MOE_A2A_F16, MOE_A2A_BF16);                             \
+    else LAUNCH_H(NV, MOE_A2A_BF16, MOE_A2A_F16);                                                          \
+  } while (0)
+      if (nv == 1) LAUNCH(1);
+      else if (nv == 2) LAUNCH(2);
+      else LAUNCH(4);
+#undef LAUNCH
+#undef LAUNCH_H
+    };
+    if (W == 1) start(sources(LocalSources<1>{}));
+    else start(sources(LocalSources<LOCAL_FEW_RANKS>{}));
+    return launch_status();
+  }
   const int tiles = std::max(1, (S + LPLAN_BLOCK - 1) / LPLAN_BLOCK);
   auto launch = [&](auto table) {
     constexpr int R = sizeof(table.x) / sizeof(table.x[0]);

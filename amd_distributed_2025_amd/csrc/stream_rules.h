@@ -206,6 +206,19 @@ int combine_block(long long tokens, long long rows_hint, int per_token) {
 
 // ---------------------------------------------------------------- jobs on one GPU
 
+// Tokens of a workgroup of local_dispatch_long_kernel, or 0 where a launch of its own plans the rows: more ranks than its tables have, more experts than
+// it counts in 64 KB, or so many keys that what 256 workgroups read of them (a 256 KB stream 64 MB out of L2) is not little beside the rows. One
+// workgroup per unit: us of whole calls, plan / with 256 / 512 / 1024 workgroups, 8 ranks of 238 tokens of 4.5 KB, 6 each 34.8 / 32.8 / 33.6 / 46, of
+// 65 of 8.6 KB, 5 each 18.4 / 15.7 / 16.7 / 27; one rank of 3084 of 1.6 KB, 2 each 24.8 / 21.0 / 22.6 / 26.
+constexpr int LOCAL_LONG_ENTRIES = 512;  // entries of a workgroup
+int local_long_tokens(long long tokens, int per_token, int ranks, int experts) {
+  const long long entries = tokens * per_token;
+  if (entries < 1 || entries > 32768 || per_token > 64 || ranks > 8 || experts > 512) return 0;
+  return (int)std::min<long long>(LOCAL_LONG_ENTRIES / per_token, (tokens + 255) / 256);
+}
+// Vectors per lane of its pieces: two, of many long rows four (235 MB 58.9 / 56.4 us, 146 MB 39.8 / 39.0, but 92 MB 41.5 / 41.6, 24 MB 15.6 / 16.9).
+int local_long_vecs(long long bytes, int row_vecs) { return row_vecs <= 64 ? 1 : row_vecs > 128 && bytes >= 128ll << 20 ? 4 : 2; }
+
 // Vectors of a row that a lane of local_dispatch_few_kernel moves: one, two or four, of single elements one, four or eight. Every
 // workgroup holds all keys, so that many pieces of rows cost more than the rows: beyond two workgroups per unit with tables of
 // several ranks or more than 1024 keys, else beyond four, a lane moves more. (Up to 256 keys are so few that pieces of
