@@ -5347,13 +5347,14 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   Geometry g = geometry(s, recv_buf, expert_x);
   hipStream_t st = (hipStream_t)stream;
   const bool planned = send_back_plan && plan_supported(s);
-  if (row_position && g.nle <= RPLAN_MAX_EXPERTS && capacity_rows > 0) {
-    // no scan to repeat per piece: a row is split among more waves, as in the planned stage 3
-    if (g.vec16) {
-      g.nvw = planned_recv_vecs(g.row_vecs);
-      g.wchunks = (g.row_vecs + 64 * g.nvw - 1) / (64 * g.nvw);
-    }
-    if (!items_fit((long long)g.nle * g.max_recv, g.wchunks)) return MOE_A2A_EINVAL;
+  // the stream can hold at most nle * max_recv rows that fit the expert buffers
+  if (!items_fit((long long)g.nle * g.max_recv, g.wchunks)) return MOE_A2A_EINVAL;
+  // no scan to repeat per piece: a row is split among more waves, as in the planned stage 3
+  const int piece_vecs = g.vec16 ? planned_recv_vecs(g.row_vecs) : g.nvw, pieces = (g.row_vecs + 64 * piece_vecs - 1) / (64 * piece_vecs);
+  // (what a launch numbers are the pieces of the rows that arrive, however many the experts could take; more than it can number are scanned for)
+  if (row_position && g.nle <= RPLAN_MAX_EXPERTS && capacity_rows > 0 && items_fit(capacity_rows, pieces)) {
+    g.nvw = piece_vecs;
+    g.wchunks = pieces;
     const int tiles = (int)std::min<long long>(((long long)rows_hint + RPLAN_BLOCK - 1) / RPLAN_BLOCK + 1, 1 << 16);
     int expert_bits = 0;  // nle <= 1 << expert_bits
     while ((1 << expert_bits) < g.nle) ++expert_bits;
@@ -5397,8 +5398,6 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
 #undef LAUNCH_C
     return launch_status();
   }
-  // the stream can hold at most nle * max_recv rows that fit the expert buffers
-  if (!items_fit((long long)g.nle * g.max_recv, g.wchunks)) return MOE_A2A_EINVAL;
   const RecvFew few = planned ? recv_few(rows_hint, g.row_vecs, g.nvw, g.vec16, compact_rows > 0) : RECV_NOT_FEW;
   if (few != RECV_NOT_FEW) {  // (planned: at most 64 ranks)
     const int few_grid = g.nle + mover_blocks(((long long)rows_hint * g.wchunks + ROWS - 1) / ROWS);

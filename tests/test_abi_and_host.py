@@ -151,6 +151,18 @@ def test_bad_arguments_are_rejected_without_touching_the_gpu():
         _lib.call("moe_a2a_dispatch_send", None, one, one, 1, one, one, one, None, None)
 
 
+def test_planned_places_bound_the_rows_that_arrive_not_those_the_experts_could_take():
+    """128 experts of 8 x 150000 tokens are more pieces of rows than a launch numbers, the 4200 rows of the buffers are not."""
+    if torch.cuda.is_available():
+        pytest.skip("addresses that are never launched with")
+    lib, one, shape = _lib.load(), C.c_void_p(16), _lib.Shape(8, 0, 1024, 8, 7168, 150000)
+    args = [C.byref(shape), one, one, one, 4200, 4200, one, one, one, one, 4200, None]
+    assert lib.moe_a2a_dispatch_recv_compact(*args, None) == lib.moe_a2a_dispatch_recv_compact_long(*args, one, None) == -3  # (no GPU)
+    # (what the padded layout could hold stays refused)
+    args = [C.byref(_lib.Shape(8, 0, 1024, 8, 7168, 1 << 24)), one, one, one, 4200, 4200, one, one, one, None]
+    assert lib.moe_a2a_dispatch_recv(*args, None) == lib.moe_a2a_dispatch_recv_long(*args, one, None) == -1
+
+
 def test_no_silent_cpu_fallback():
     from amd_distributed_2025_amd import HIPAllToAll, custom_kernel
 

@@ -139,3 +139,21 @@ def test_planned_places_of_many_tiles(W, nle, K, tokens, exact_hints):
     spec = dict(world_size=W, num_experts=W * nle, experts_per_token=K, hidden_dim=16, max_num_tokens=tokens,
                 num_tokens="full", routing="zipf", weights="rand", dtype="bf16")
     run_compact(generate_world(spec, 5), exact_hints=exact_hints, binding="ext" if exact_hints else "ctypes")
+
+
+def test_planned_places_of_a_shape_that_could_hold_far_more():
+    """128 experts that could each take 1.2 million rows, of which 4100 arrive: more than the experts' pieces could be numbered."""
+    W, nle, H, R = 8, 128, 7168, 4100
+    a = HIPAllToAll(MoEConfig(W * nle, 1, H, 150000, torch.bfloat16, torch.bfloat16), 3, W, device=DEV, layout="compact", compact_rows=4200)
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(1)
+    recv = torch.randn(R, H, device=DEV, generator=gen).to(torch.bfloat16)
+    meta = torch.randint(0, 1000, (R, 5), device=DEV, generator=gen, dtype=torch.int32)
+    meta[:, 0] = 3 * nle + torch.randint(0, nle, (R,), device=DEV, generator=gen, dtype=torch.int32)
+    counts = torch.tensor([R - 70] + [10] * 7, dtype=torch.int32, device=DEV)
+    num, ex, em = a.dispatch_recv(counts, recv, meta, R)
+    torch.cuda.synchronize()
+    order = torch.argsort(meta[:, 0], stable=True)
+    assert torch.equal(ex[:R], recv[order]) and torch.equal(em[:R], meta[order])
+    want = torch.bincount(meta[:, 0] - 3 * nle, minlength=nle)
+    assert torch.equal(num.long(), want) and torch.equal(a.expert_offsets[1:].long(), want.cumsum(0))
