@@ -1538,8 +1538,9 @@ __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_kernel(
 
 // The movers of a long stream, with the positions that plan_recv_kernel left: a wave per piece of 64 * NVW vectors of a row, in
 // the order of the stream. Memory bounds it, and what shaped it is how few places of the streams are open at a time (planned_recv_vecs and
-// RECV_PAST_BYTES, csrc/stream_rules.h): 32768 rows of 14 KB 160 us with a workgroup on the same piece of four rows and plain loads of four
-// vectors, 137 here (6.9 TB/s); with a stage before and behind it 12000 rows of 4 KB 53.6 / 47.0.
+// RECV_PAST_BYTES, csrc/stream_rules.h): 32768 rows of 14 KB between the other stages 160 us with a workgroup on the same piece of four rows and plain
+// loads of four vectors, 137 here (6.9 TB/s); what a graph of stages 1 to 4 loses without stage 2, its plan with it, 192 / 192 (203 with two vectors per
+// lane); with a stage before and behind it 12000 rows of 4 KB 53.6 / 47.0.
 template <typename V, int NVW, bool PLAN, bool COMPACT, Store HOW, bool PAST>
 __global__ __launch_bounds__(64 * ROWS) void dispatch_recv_planned_kernel(
     const int* __restrict__ recv_meta, const int* __restrict__ row_pos, const int* __restrict__ recv_counts,
@@ -5350,7 +5351,8 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
   // the stream can hold at most nle * max_recv rows that fit the expert buffers
   if (!items_fit((long long)g.nle * g.max_recv, g.wchunks)) return MOE_A2A_EINVAL;
   // no scan to repeat per piece: a row is split among more waves, as in the planned stage 3
-  const int piece_vecs = g.vec16 ? planned_recv_vecs(g.row_vecs) : g.nvw, pieces = (g.row_vecs + 64 * piece_vecs - 1) / (64 * piece_vecs);
+  const long long stream_bytes = (long long)rows_hint * s->hidden_dim * 2;
+  const int piece_vecs = g.vec16 ? planned_recv_vecs(stream_bytes, g.row_vecs) : g.nvw, pieces = (g.row_vecs + 64 * piece_vecs - 1) / (64 * piece_vecs);
   // (what a launch numbers are the pieces of the rows that arrive, however many the experts could take; more than it can number are scanned for)
   if (row_position && g.nle <= RPLAN_MAX_EXPERTS && capacity_rows > 0 && items_fit(capacity_rows, pieces)) {
     g.nvw = piece_vecs;
@@ -5362,7 +5364,7 @@ int launch_dispatch_recv(const moe_a2a_shape* s, const void* recv_buf, const int
     plan_rows<<<tiles, RPLAN_BLOCK, 0, st>>>(recv_meta, recv_counts, s->world_size, rows_hint, capacity_rows, g.nle, g.magic,
                                              expert_bits, row_position);
     const int movers = mover_blocks(((long long)rows_hint * g.wchunks + ROWS - 1) / ROWS);
-    const bool past = (long long)rows_hint * s->hidden_dim * 2 >= RECV_PAST_BYTES;
+    const bool past = stream_bytes >= RECV_PAST_BYTES;
 #define LAUNCH_C(V, NVW, PLAN, COMPACT, PAST)                                                                  \
   dispatch_recv_planned_kernel<V, NVW, PLAN, COMPACT, THROUGH, PAST><<<g.nle + movers, 64 * ROWS, 0, st>>>(    \
       recv_meta, row_position, recv_counts, (const V*)recv_buf, s->world_size, rows_hint, movers,              \

@@ -41,7 +41,11 @@ bool send_past(long long bytes, int row_vecs) { return bytes >= (row_vecs > BLOC
 // 134 MB 198 / 205, 268 MB 497 / 510, 336 MB 708 / 685 and, the other stages at their best, 658 / 664; 470 MB 716 / 682 and 649 / 637.
 constexpr long long EXPERT_STREAM_BYTES = 384ll << 20;
 
-int planned_recv_vecs(int row_vecs) { return row_vecs > BLOCK ? 2 : 1; }
+// Vectors per lane of the movers of a planned stage 2: one for rows of up to 4 KB, and for those of more than 8 KB that the cache behind L2 holds none
+// of; us of stages 1, 2, 3 and 4, and of a whole step, two / one: 14 KB 185 MB 216.5 / 219.1, 318.3 / 319.4, 240 MB 279.6 / 285.7, 411.6 / 413.3, 294 MB
+// 366.9 / 362.1, 531.8 / 533.1, 348 MB 435.8 / 425.8, 634.8 / 638.2, 446 MB 549.1 / 538.6, 803.5 / 802.6; 10 KB 319 MB 389.5 / 385.9, 510.6 / 511.9; 8 KB 312
+// MB 389.6 / 390.8, 513.3 / 515.8; 6 KB 328 MB 429.8 / 427.1, 557.4 / 559.7.
+int planned_recv_vecs(long long bytes, int row_vecs) { return row_vecs > BLOCK && (row_vecs <= 2 * BLOCK || bytes < 288ll << 20) ? 2 : 1; }
 
 // Vectors per lane of a planned stage 3: four (a 256-vector piece per wave) made a whole step 0.5 us shorter at 2048 rows of 14 KB than the
 // 14 of the scan path; 2, 6 and 8 were no better than 14. Long rows beyond the cache take eight: 470 MB 660 / 654 us as above, 336 MB of 10 KB

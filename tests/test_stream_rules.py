@@ -28,6 +28,7 @@ def rules(tmp_path_factory):
                    'extern "C" int lanes(long long tokens, long long entries, int ranks, int row_vecs, int vec16) {\n'
                    '  return local_few_vecs(tokens, entries, ranks, row_vecs, vec16); }\n'
                    'extern "C" int past_in_stage_3(long long bytes, int row_vecs) { return send_past(bytes, row_vecs); }\n'
+                   'extern "C" int vecs_of_stage_2(long long bytes, int row_vecs) { return planned_recv_vecs(bytes, row_vecs); }\n'
                    'extern "C" int keys(long long entries) { return few_keys(entries); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
@@ -39,7 +40,7 @@ def rules(tmp_path_factory):
     dll.through.argtypes = [C.c_longlong, C.c_longlong]
     dll.lanes.argtypes = [C.c_longlong, C.c_longlong] + [C.c_int] * 3
     dll.keys.argtypes = [C.c_longlong]
-    dll.past_in_stage_3.argtypes = [C.c_longlong, C.c_int]
+    dll.vecs_of_stage_2.argtypes = dll.past_in_stage_3.argtypes = [C.c_longlong, C.c_int]
     return dll
 
 
@@ -182,3 +183,12 @@ def test_lanes_that_move_several_vectors_have_stores_for_a_megabyte_and_more(rul
 def test_rows_of_stage_3_past_the_caches(rules, rows, hidden, past):
     """Timed on the GPU, with an expert in front and without: rows that the cache behind L2 still holds lose up to 8 % of the four stages."""
     assert rules.past_in_stage_3(rows * hidden * 2, hidden // 8) == past
+
+
+@pytest.mark.parametrize("rows,hidden,vecs", [
+    (6278, 7168, 2), (17530, 7168, 2), (21496, 7168, 1), (32613, 7168, 1), (32690, 5120, 1), (39957, 4096, 2), (32690, 4096, 2),
+    (11900, 4096, 2), (32945, 2560, 2), (55992, 3072, 2), (17946, 2048, 1), (64029, 2048, 1),
+])
+def test_pieces_of_a_planned_stage_2(rules, rows, hidden, vecs):
+    """Timed on the GPU: beyond the cache two vectors per lane of long rows take 2 % more of the four stages."""
+    assert rules.vecs_of_stage_2(rows * hidden * 2, hidden // 8) == vecs
