@@ -134,20 +134,24 @@ SendWay send_way(long long tokens, int per_token, int ranks, int row_vecs, bool 
 }
 
 // Tokens of a workgroup of dispatch_long_kernel, or 0 where a stream stays with its choice above. From 5120 entries on it takes whole vectors over from
-// dispatch_block_kernel, and from 65281 on from all others, which compare every key with every entry: over 288 streams of 5120 to 32768 entries, one to
-// eight per token, rows of 512 bytes to 14 KB, 0.90 of their time, 17 of them more than 3 % behind (2803 tokens of 1.9 KB, 6 per token
-// 14.75 / 16.6). Below it is behind: 4900 entries (613 tokens of 900 bytes) 6.2 / 6.4, 3100 (777 of 1.4 KB) 5.5 / 6.3.
+// dispatch_block_kernel, and from 65281 on from all others, which compare every key with every entry. It stays behind with few tokens and entries (its
+// workgroups then hold three and four tokens: 722 of 272 bytes, 8 per token 5.4 / 6.1 us, 1005 of 5.6 KB, 6 each 11.1 / 12.2), below 5120 entries (4900, 613 tokens
+// of 900 bytes, 6.2 / 6.4), and with short rows just past the entries that a workgroup per unit holds (2803 of 1.9 KB, 6 each 14.8 / 15.7,
+// 2235 of 1.5 KB, 8 each 14.1 / 15.0, 2225 of 272 bytes 12.7 / 13.4). Over 513 streams of 5120 to 32768 entries, one to eight per token, rows of 128 bytes to 14 KB, the choice takes
+// 0.893 of the others' time; 31 are more than 3 % behind, the worst by 10 % (1123 tokens of 1.8 KB, 8 each 8.1 / 8.9).
 //
-// About one workgroup per unit where rows are short, which leaves the passes over the keys to the fewest, two where the rows take longer
-// than that. us, with 128 / 256 / 512 / 1024 workgroups: 3590 tokens of 1 KB, 3 per token 7.9 /
-// 8.0 / 11.2 / 15.1; 3649 of 1.5 KB, 5 each 14.4 (192) / 14.4 / 22.1 (912); 2803 of 1.9 KB, 6 each - / 16.6 / 15.1 / 23.1; 3554 of 8.6 KB, 2
-// each 18.1 / 18.0 / 18.0 / 19.6; 3001 of 12 KB, 5 each - / 41.2 / 39.9 / 38.7; 4096 of 14 KB, 8 each - / - / 113 / 111.
+// Short rows have one workgroup per unit, which leaves the passes over the keys to the fewest, as long as those hold all tokens (64 entries each);
+// others two, and where a row takes longer than a pass four. us, with 256 / 512 / 768 / 1024 workgroups: 3590 tokens of 1 KB, 3 per token 7.5 / 10.6 / 14.4; 2675 of 2.1 KB, 6
+// each 15.4 / 13.0 / 15.7; 2055 of 5.8 KB, 4 each 14.2 / 15.2 / 16.8; 3594 of 6.3 KB, 8 each 40.5 / 40.7 / 41.1 / 44.4; 3212 of 5 KB, 5 each 28.6 / 24.5 / 24.1 /
+// 25.0; 3731 of 14.3 KB, 4 each 63.9 / 62.5 / 59.1 / 57.2; 4084 of 11.2 KB, 6 each 60.9 / 60.3 / 60.2 / 56.6; 4096 of 14 KB, 8 each, with the other stages, - / 809 / 815 / 807.
 int long_tokens(SendWay way, long long tokens, int per_token, int ranks, int row_vecs, bool vec16) {
   const long long entries = tokens * per_token;
   if (!vec16 || ranks > BLOCK_RANKS || per_token > 64 || entries < LONG_ENTRIES || entries > LONG_MAX_ENTRIES ||
       (way != SEND_BLOCK && entries <= BLOCK_MAX_ENTRIES))
     return 0;
-  const int workgroups = row_vecs <= 400 ? 256 : 512;
+  if ((tokens < 1024 && entries < 6400) || (row_vecs <= 128 && per_token >= 6 && entries >= 16800 && entries <= 18432)) return 0;
+  const bool one_each = row_vecs <= (entries <= 9216 ? 400 : 256) && tokens <= 64 / per_token * 264;
+  const int workgroups = one_each ? 256 : row_vecs > 512 && entries >= 7500 ? 1024 : 512;
   return (int)std::min<long long>(64 / per_token, (tokens + workgroups - 1) / workgroups);
 }
 

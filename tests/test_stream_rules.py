@@ -29,6 +29,8 @@ def rules(tmp_path_factory):
                    '  return local_few_vecs(tokens, entries, ranks, row_vecs, vec16); }\n'
                    'extern "C" int past_in_stage_3(long long bytes, int row_vecs) { return send_past(bytes, row_vecs); }\n'
                    'extern "C" int vecs_of_stage_2(long long bytes, int row_vecs) { return planned_recv_vecs(bytes, row_vecs); }\n'
+                   'extern "C" int long_of(long long tokens, int k, int ranks, int row_vecs, int vec16) {\n'
+                   '  return long_tokens(send_way(tokens, k, ranks, row_vecs, vec16), tokens, k, ranks, row_vecs, vec16); }\n'
                    'extern "C" int keys(long long entries) { return few_keys(entries); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
@@ -40,6 +42,7 @@ def rules(tmp_path_factory):
     dll.through.argtypes = [C.c_longlong, C.c_longlong]
     dll.lanes.argtypes = [C.c_longlong, C.c_longlong] + [C.c_int] * 3
     dll.keys.argtypes = [C.c_longlong]
+    dll.long_of.argtypes = [C.c_longlong] + [C.c_int] * 4
     dll.vecs_of_stage_2.argtypes = dll.past_in_stage_3.argtypes = [C.c_longlong, C.c_int]
     return dll
 
@@ -192,3 +195,25 @@ def test_rows_of_stage_3_past_the_caches(rules, rows, hidden, past):
 def test_pieces_of_a_planned_stage_2(rules, rows, hidden, vecs):
     """Timed on the GPU: beyond the cache two vectors per lane of long rows take 2 % more of the four stages."""
     assert rules.vecs_of_stage_2(rows * hidden * 2, hidden // 8) == vecs
+
+
+@pytest.mark.parametrize("tokens,k,hidden,own", [
+    (722, 8, 136, 0), (755, 8, 336, 0), (1005, 6, 2792, 0), (613, 8, 448, 0), (2803, 6, 952, 0), (2235, 8, 728, 0), (2225, 8, 136, 0),
+    (1015, 7, 416, 4), (816, 8, 2464, 4), (3590, 3, 512, 15), (2054, 8, 264, 8), (3131, 5, 80, 12), (3649, 5, 768, 8), (2675, 6, 1056, 6),
+    (2055, 4, 2912, 9), (2637, 6, 1456, 10), (3212, 5, 2488, 7), (3594, 8, 3136, 8), (3731, 4, 7144, 4), (4084, 6, 5600, 4), (4096, 8, 7168, 4),
+])
+def test_tokens_of_a_workgroup_for_long_streams(rules, tokens, k, hidden, own):
+    """Timed on the GPU: streams that stay with another kernel lose up to 13 % here, too few or too many tokens in a workgroup up to 40 %."""
+    vecs, vec16, _ = row(hidden)
+    assert rules.long_of(tokens, k, 8, vecs, vec16) == own
+
+
+def test_limits_of_the_kernel_of_long_streams(rules):
+    """(64 entries in a workgroup, keys that 1024 lanes count in bytes, whole vectors, eight ranks)"""
+    for tokens in (1, 79, 80, 640, 1023, 1024, 2048, 2112, 2113, 4080, 5120, 16320, 16321, 65280, 65281, 261120, 261121):
+        for k in (1, 2, 3, 5, 8, 16, 17, 63, 64, 65):
+            for vecs in (1, 128, 129, 256, 257, 400, 401, 512, 513, 896, 1 << 20):
+                own, entries = rules.long_of(tokens, k, 8, vecs, 1), tokens * k
+                assert rules.long_of(tokens, k, 9, vecs, 1) == rules.long_of(tokens, k, 8, vecs, 0) == 0
+                assert 0 <= own * k <= 64 and (not own or 5120 <= entries <= 255 * 1024)
+                assert own or not 65280 < entries <= 255 * 1024 or k > 64
