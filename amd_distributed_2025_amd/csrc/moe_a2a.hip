@@ -3774,13 +3774,14 @@ __global__ __launch_bounds__(256, 1) void ring_gemm_kernel(
 // The experts' product or a plain one where its tiles make for about one workgroup per unit, or two. WM x WN waves, two or four of them on a SIMD,
 // fetch the rows of a tile straight into a ring of DEPTH steps in LDS. A wave holds the fragments of one slice of 32 inputs while those of the
 // next are on their way, so that its reads are behind MFMAs and the waves of a SIMD fill each other's gaps; one barrier per step, in its
-// middle. LDS rows, fragments, results and the order of K are those of phased_gemm_kernel, so the choice changes no bit.
+// middle. LDS rows, fragments, results and the order of K are those of phased_gemm_kernel, so among kernels that walk K whole the choice changes no
+// bit (products that were split over K before round their sums elsewhere: a single one instead of one per wave).
 // What bounds it: rows out of L2, some 17 TB/s over the chip on any tile (32 x 64 to 192 x 128: 0.2 to 0.67 us a step), and 3.5 to 5 us around
 // the walk (launch, first rows, results). us, the kernel that had the product / here:
 //   plain, on one group of ring_gemm_kernel, whose workgroups search the groups for their tile: 77 x 7360 x 768 7.84 / 5.74, 351 x 1728 x 832
 //     8.19 / 6.04, 202 x 2432 x 6272 26.7 / 21.7, 24 x 2176 x 384 5.31 / 4.38; on 64 x 128 of dense_gemm_kernel, whose rows go through registers
-//     into two buffers: 786 x 1984 x 4608 28.4 / 25.5, 297 x 1152 x 408 5.79 / 4.77, 37 x 7808 x 8 4.33 / 3.75; split over K: 64 x 7168 x 2304
-//     10.56 / 9.60, 88 x 5056 x 2432 11.75 / 9.95
+//     into two buffers: 786 x 1984 x 4608 28.4 / 25.5, 297 x 1152 x 408 5.79 / 4.77, 37 x 7808 x 8 4.33 / 3.75; split over K, in calls: 64 x 7168 x 2304
+//     9.1 / 8.7 (on 64 x 32), 88 x 5056 x 2432 10.4 / 8.7
 //   experts': 15 of 400 rows, 576 x 640 (dense_gemm_kernel, 64 x 128) 23.9 / 16.8; 5 of 253, 896 x 1856 (a ring of 64 x 128) 17.3 / 14.0; 11 of 50,
 //     1248 x 6240 69.4 / 45.0; 22 of 239, 640 x 1280 (dense_gemm_kernel, 128 x 128) 25.0 / 17.2; 13 of 377, 1024 x 4032
 //     (phased_gemm_kernel, 192 x 256) 72.0 / 52.6; 18 of 39, 960 x 1408 (expert_gemm_kernel) 22.2 / 13.0
@@ -3791,6 +3792,7 @@ struct Slices {
   static constexpr size_t LDS_BYTES = (size_t)DEPTH * (ROWS + COLS) * 128;
 };
 using Slices32x64 = Slices<2, 2, 1, 2, 6, 2>;
+using Slices64x32 = Slices<4, 1, 1, 2, 6, 2>;
 using Slices64x64 = Slices<4, 2, 1, 2, 4, 2>;
 using Slices64x128 = Slices<2, 4, 2, 2, 3, 2>;
 using Slices128x128 = Slices<4, 2, 2, 4, 4, 1>;
@@ -6030,6 +6032,7 @@ int allow_large_lds() {
     allow((const void*)sliced_gemm_kernel<DT, Slices128x128, true, S>, Slices128x128::LDS_BYTES);
     allow((const void*)sliced_gemm_kernel<DT, Slices192x128, true, S>, Slices192x128::LDS_BYTES);
     if constexpr (!S) {
+      allow((const void*)sliced_gemm_kernel<DT, Slices64x32, false, false>, Slices64x32::LDS_BYTES);
       allow((const void*)sliced_gemm_kernel<DT, Slices32x64, false, false>, Slices32x64::LDS_BYTES);
       allow((const void*)sliced_gemm_kernel<DT, Slices64x64, false, false>, Slices64x64::LDS_BYTES);
       allow((const void*)sliced_gemm_kernel<DT, Slices64x128, false, false>, Slices64x128::LDS_BYTES);
@@ -6121,7 +6124,8 @@ int launch_slices(const void* x, const int32_t* rows_of_group, const void* w, co
       else if (way == SLICES_128x128) grouped(Slices128x128{});
       else grouped(Slices192x128{});
     } else {
-      if (way == SLICES_32x64) plain(Slices32x64{});
+      if (way == SLICES_64x32) plain(Slices64x32{});
+      else if (way == SLICES_32x64) plain(Slices32x64{});
       else if (way == SLICES_64x64) plain(Slices64x64{});
       else plain(Slices64x128{});
     }
