@@ -7,6 +7,9 @@ from pathlib import Path
 import pytest
 
 from tests.test_gpu_block_streams import CASES
+from tests.test_gpu_combine_block import CASES as COMBINE_CASES
+from tests.test_gpu_large_streams import LONG_CASES, MAPPED_PAST_CASES, RECV_PAST_CASES
+from tests.test_gpu_local_long import CASES as LOCAL_LONG_CASES
 from tests.test_gpu_short_streams import LANES, RECV_CASES
 
 CSRC = Path(__file__).resolve().parent.parent / "amd_distributed_2025_amd" / "csrc"
@@ -31,6 +34,14 @@ def rules(tmp_path_factory):
                    'extern "C" int vecs_of_stage_2(long long bytes, int row_vecs) { return planned_recv_vecs(bytes, row_vecs); }\n'
                    'extern "C" int long_of(long long tokens, int k, int ranks, int row_vecs, int vec16) {\n'
                    '  return long_tokens(send_way(tokens, k, ranks, row_vecs, vec16), tokens, k, ranks, row_vecs, vec16); }\n'
+                   'extern "C" int vecs_of_stage_3(long long bytes, int row_vecs) { return planned_send_vecs(bytes, row_vecs); }\n'
+                   'extern "C" int vecs_of_stage_4(int k, int row_vecs, int past) { return mapped_vecs(k, row_vecs, past); }\n'
+                   'extern "C" int tokens_of_stage_4(long long tokens, long long rows, int k) { return combine_block(tokens, rows, k); }\n'
+                   'extern "C" int tokens_of_jobs(long long tokens, int k, int ranks, int experts) {\n'
+                   '  return local_long_tokens(tokens, k, ranks, experts); }\n'
+                   'extern "C" int vecs_of_jobs(long long bytes, int row_vecs) { return local_long_vecs(bytes, row_vecs); }\n'
+                   'extern "C" long long line(int which) {\n'
+                   '  return which == 0 ? RECV_PAST_BYTES : which == 1 ? COMBINE_PAST_BYTES : which == 2 ? COMBINE_TOKENS : LOCAL_LONG_ENTRIES; }\n'
                    'extern "C" int keys(long long entries) { return few_keys(entries); }\n')
     lib = src.with_suffix(".so")
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-shared", "-fPIC", f"-I{CSRC}",
@@ -43,6 +54,10 @@ def rules(tmp_path_factory):
     dll.lanes.argtypes = [C.c_longlong, C.c_longlong] + [C.c_int] * 3
     dll.keys.argtypes = [C.c_longlong]
     dll.long_of.argtypes = [C.c_longlong] + [C.c_int] * 4
+    dll.line.restype = C.c_longlong
+    dll.tokens_of_stage_4.argtypes = [C.c_longlong, C.c_longlong, C.c_int]
+    dll.tokens_of_jobs.argtypes = [C.c_longlong] + [C.c_int] * 3
+    dll.vecs_of_stage_3.argtypes = dll.vecs_of_jobs.argtypes = [C.c_longlong, C.c_int]
     dll.vecs_of_stage_2.argtypes = dll.past_in_stage_3.argtypes = [C.c_longlong, C.c_int]
     return dll
 
@@ -56,6 +71,7 @@ def row(hidden):
 
 
 def way_of(rules, tokens, k, ranks, hidden):
+    """(as dispatch_long_kernel finds them, which takes streams of 5120 entries and more over)"""
     vecs, vec16, nvw = row(hidden)
     way = SEND_WAYS[rules.way(tokens, k, ranks, vecs, vec16)]
     if way == "block":
@@ -66,7 +82,9 @@ def way_of(rules, tokens, k, ranks, hidden):
 
 @pytest.mark.parametrize("W,E,K,H,T", CASES)
 def test_kernels_of_stage_1_that_the_gpu_tests_mean(rules, W, E, K, H, T):
-    assert way_of(rules, T, K, W, H) == CASES[W, E, K, H, T]
+    vecs, vec16, _ = row(H)
+    own = rules.long_of(T, K, W, vecs, vec16)
+    assert (("long", own) if own else way_of(rules, T, K, W, H)) == CASES[W, E, K, H, T]
 
 
 @pytest.mark.parametrize("tokens,k,hidden,way", [
@@ -217,3 +235,53 @@ def test_limits_of_the_kernel_of_long_streams(rules):
                 assert rules.long_of(tokens, k, 9, vecs, 1) == rules.long_of(tokens, k, 8, vecs, 0) == 0
                 assert 0 <= own * k <= 64 and (not own or 5120 <= entries <= 255 * 1024)
                 assert own or not 65280 < entries <= 255 * 1024 or k > 64
+
+
+def test_long_streams_of_stage_1_that_the_gpu_tests_mean(rules):
+    for (W, E, K, H, T), own in LONG_CASES.items():
+        vecs, vec16, _ = row(H)
+        assert rules.long_of(T, K, W, vecs, vec16) == own, (W, E, K, H, T)
+
+
+def test_large_streams_that_the_gpu_tests_mean(rules):
+    """(those that stages 2 and 4 read past the caches, and on pieces of one vector per lane and of two)"""
+    for (hidden, rows), vecs in RECV_PAST_CASES.items():
+        assert rows * hidden * 2 >= rules.line(0) and rules.vecs_of_stage_2(rows * hidden * 2, hidden // 8) == vecs, (hidden, rows)
+    for (hidden, k, tokens), vecs in MAPPED_PAST_CASES.items():
+        assert tokens * (k + 1) * hidden * 2 >= rules.line(1) and rules.vecs_of_stage_4(k, hidden // 8, 1) == vecs, (hidden, k, tokens)
+    assert {k > 2 for (_, k, _), vecs in MAPPED_PAST_CASES.items() if vecs == 2} == {True, False}
+
+
+@pytest.mark.parametrize("k,hidden,past,vecs", [
+    (8, 7168, 1, 1), (4, 2880, 0, 1), (3, 4096, 0, 1), (3, 4096, 1, 2), (2, 4096, 0, 2), (1, 4096, 0, 2), (1, 512, 1, 1), (5, 4096, 1, 1),
+])
+def test_vectors_of_stage_4_that_were_faster(rules, k, hidden, past, vecs):
+    """(timed on the GPU)"""
+    assert rules.vecs_of_stage_4(k, hidden // 8, past) == vecs
+
+
+@pytest.mark.parametrize("megabytes,hidden,vecs", [(470, 7168, 8), (336, 5120, 8), (275, 7168, 8), (235, 7168, 4), (268, 4096, 4), (29, 7168, 4)])
+def test_pieces_of_a_planned_stage_3(rules, megabytes, hidden, vecs):
+    """Timed on the GPU (megabytes of 10^6): eight vectors per lane of rows of more than 8 KB beyond the cache, else four."""
+    assert rules.vecs_of_stage_3(megabytes * 10 ** 6, hidden // 8) == vecs
+
+
+def test_tokens_of_stage_4_that_the_gpu_tests_mean(rules):
+    for (T, K, H, W), tokens in COMBINE_CASES.items():
+        assert rules.tokens_of_stage_4(T, T * K, K) == tokens, (T, K)
+    for T in (1, 256, 257, 767, 768, 4096, 32768, 32769, 1 << 20):
+        for K in (1, 2, 8, 9):
+            tokens = rules.tokens_of_stage_4(T, T * K, K)
+            assert tokens <= rules.line(2) and (tokens == 0) == (T <= 256 or T * K <= 512 or K > 8)
+
+
+def test_movers_of_jobs_that_the_gpu_tests_mean(rules):
+    for (E, K, H, T), (tokens, vecs) in LOCAL_LONG_CASES.items():
+        assert rules.tokens_of_jobs(T, K, 1, E) == tokens and rules.vecs_of_jobs(T * K * H * 2, H // 8) == vecs, (E, K, H, T)
+    for T in (0, 1, 255, 256, 257, 511, 512, 513, 4096, 16384, 32767, 32768, 32769):
+        for K in (1, 2, 3, 8, 63, 64, 65):
+            tokens = rules.tokens_of_jobs(T, K, 8, 512)
+            assert (tokens == 0) == (not 1 <= T * K <= 32768 or K > 64) and tokens * K <= rules.line(3)
+    assert rules.tokens_of_jobs(300, 8, 9, 9) == rules.tokens_of_jobs(300, 8, 8, 513) == 0
+    for megabytes, hidden, vecs in ((235, 7168, 4), (146, 4096, 4), (92, 7168, 2), (24, 2048, 2), (300, 512, 1), (300, 1024, 2)):
+        assert rules.vecs_of_jobs(megabytes * 10 ** 6, hidden // 8) == vecs
