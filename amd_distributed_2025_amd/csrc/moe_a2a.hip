@@ -3541,7 +3541,7 @@ constexpr size_t phased_lds_bytes(int TM, int TN, int NA, int HB) {  // NA buffe
 }
 
 // Tiles of a grouped product: A is [groups, max_rows, K], B [groups, N, K], C [groups, max_rows, N], and group g
-// has rows_of_group[g] rows (read here, clamped to max_rows; null: max_rows). A group's rows are spread evenly over the fewest
+// has rows_of_group[g] rows (read here, clamped to max_rows). A group's rows are spread evenly over the fewest
 // tiles of BM rows, in whole bands of 32; tiles are numbered by group, column tile and row tile, so that
 // neighbours share the group's weights. compact: A and C hold the groups' rows back to back in buffers of
 // max_rows rows. The rows ahead of a group are a prefix over the counts, and a group only has the rows that
@@ -3565,7 +3565,7 @@ __device__ __forceinline__ GroupTile find_group_tile(int tile, const int* __rest
   int* const red_rows = lds + 8;
   int* const home = lds + 16;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  auto rows_of = [=](int g) { return rows_of_group ? min(max(rows_of_group[g], 0), max_rows) : max_rows; };
+  auto rows_of = [=](int g) { return min(max(rows_of_group[g], 0), max_rows); };
   auto kept_of = [=](int g, int ahead) {
     const int n = rows_of(g);
     return compact ? min(ahead + n, max_rows) - min(ahead, max_rows) : n;
@@ -6138,7 +6138,6 @@ int launch_slices(const void* x, const int32_t* rows_of_group, const void* w, co
 // A plain product on tiles that workgroups own whole, as linear_way has chosen.
 int launch_linear_tiles(const void* a, const void* b, const void* bias, void* c, int M, int N, int K, int dtype,
                         LinearWay way, hipStream_t st) {
-  if (way == TILES_64x128) return MOE_A2A_NOT_DENSE;  // (linear_slices: sliced_gemm_kernel has these)
   const int BM = way == PHASED_256 ? 256 : way == PHASED_192 ? 192 : 128;
   const int BN = way == PHASED_256 ? 256 : 128;
   const long long tiles_m = ((long long)M + BM - 1) / BM, tiles_n = ((long long)N + BN - 1) / BN;
@@ -6182,7 +6181,7 @@ int launch_grouped_dense(const void* x, const int32_t* rows_of_group, const void
   if (dtype != MOE_A2A_F16 && dtype != MOE_A2A_BF16) return MOE_A2A_EINVAL;
   if (N % 32 != 0 || K % 8 != 0) return MOE_A2A_EINVAL;
   if (!all_aligned(16, x, w, y) || !all_aligned(8, bias)) return MOE_A2A_EALIGN;
-  if (!rows_of_group || max_rows > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
+  if (max_rows > INT_MAX / 2) return MOE_A2A_NOT_DENSE;
   const RingTile ring = grouped_ring(rows_hint, groups, N, K);
   if (ring == RING_32x32 || ring == RING_32x64) {
     const int rc = launch_grouped_ring(x, rows_of_group, w, bias, y, groups, max_rows, rows_hint, N, K, dtype, st, compact, ring);
@@ -6272,7 +6271,7 @@ int launch_linear(const void* x, const void* w, const void* bias, void* y, int M
   }
   int rc = MOE_A2A_NOT_DENSE;
   if (way == SPLIT_32 || way == SPLIT_64) rc = launch_linear_split(x, w, bias, y, M, N, K, dtype, way == SPLIT_32 ? 1 : 2, st);
-  else if (way != STREAM_WEIGHTS) rc = launch_linear_tiles(x, w, bias, y, M, N, K, dtype, way, st);
+  else if (way != STREAM_WEIGHTS && way != TILES_64x128) rc = launch_linear_tiles(x, w, bias, y, M, N, K, dtype, way, st);
   if (rc != MOE_A2A_NOT_DENSE) return rc;
   return launch_grouped_gemm(x, nullptr, w, bias, y, 1, M, M, N, K, dtype, st);
 }

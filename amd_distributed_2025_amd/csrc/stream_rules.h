@@ -157,8 +157,8 @@ int long_tokens(SendWay way, long long tokens, int per_token, int ranks, int row
 
 // Vectors per lane of a wave of dispatch_block_kernel, for rows that a wave has in one go with `nvw`. Rows
 // are cut into pieces of two vectors per lane where there are few workgroups otherwise, else of four: pieces of 2 / 4 /
-// whole rows: 250 tokens of 5.8 KB, 8 per token 4.8 / 5.1 / 5.5 us, 1440 of 7.4 KB, 4 per token 11.6 / 12.3 / 12.1, 4096 of
-// 14 KB, 8 per token 129 / 102 / 106. With one entry a piece would do little but rank: 2000 of 14 KB 13.4 / 10.7 / 9.6. Two and three
+// whole rows: 250 tokens of 5.8 KB, 8 per token 4.8 / 5.1 / 5.5 us. (Whole vectors come here with up to 5119 entries, and with some more of short rows:
+// long_tokens. So pieces of four are rows of more than 8 KB with three entries and more than 1600 tokens.) With one entry a piece would do little but rank: 2000 of 14 KB 13.4 / 10.7 / 9.6. Two and three
 // entries pay for a piece of long rows only, two for one of four vectors: 1292 of 5 KB, 2 per token 7.1 / 6.6 / 5.9, 1380 of 15 KB 14.0 /
 // 12.6 / 12.4, 1001 of 13.7 KB 8.5 / 8.0 / 9.2, 671 of 10.8 KB 6.1 / 5.5 / 5.8; 893 of 4.5 KB, 3 per token 6.1 / 5.5 / 5.3, 537 of 13.6 KB
 // 6.5 / 7.0 / 7.2.
@@ -222,14 +222,15 @@ int combine_block(long long tokens, long long rows_hint, int per_token) {
 // ---------------------------------------------------------------- jobs on one GPU
 
 // Tokens of a workgroup of local_dispatch_long_kernel, or 0 where a launch of its own plans the rows: more ranks than its tables have, more experts than
-// it counts in 64 KB, or so many keys that what 256 workgroups read of them (a 256 KB stream 64 MB out of L2) is not little beside the rows. One
+// it counts in 36 KB, or so many keys that what 256 workgroups read of them (of 128 KB, 32 MB out of L2) is not little beside the rows. One
 // workgroup per unit: us of whole calls, plan / with 256 / 512 / 1024 workgroups, 8 ranks of 238 tokens of 4.5 KB, 6 each 34.8 / 32.8 / 33.6 / 46, of
 // 65 of 8.6 KB, 5 each 18.4 / 15.7 / 16.7 / 27; one rank of 3084 of 1.6 KB, 2 each 24.8 / 21.0 / 22.6 / 26.
-constexpr int LOCAL_LONG_ENTRIES = 512;  // entries of a workgroup
+constexpr int LOCAL_LONG_KEYS = 32768, LOCAL_LONG_MAX_K = 64;
+constexpr int LOCAL_LONG_ENTRIES = LOCAL_LONG_KEYS / 256 + LOCAL_LONG_MAX_K;  // most entries of a workgroup
 int local_long_tokens(long long tokens, int per_token, int ranks, int experts) {
   const long long entries = tokens * per_token;
-  if (entries < 1 || entries > 32768 || per_token > 64 || ranks > 8 || experts > 512) return 0;
-  return (int)std::min<long long>(LOCAL_LONG_ENTRIES / per_token, (tokens + 255) / 256);
+  if (entries < 1 || entries > LOCAL_LONG_KEYS || per_token > LOCAL_LONG_MAX_K || ranks > 8 || experts > 512) return 0;
+  return (int)((tokens + 255) / 256);
 }
 // Vectors per lane of its pieces: two, of many long rows four (235 MB 58.9 / 56.4 us, 146 MB 39.8 / 39.0, but 92 MB 41.5 / 41.6, 24 MB 15.6 / 16.9).
 int local_long_vecs(long long bytes, int row_vecs) { return row_vecs <= 64 ? 1 : row_vecs > 128 && bytes >= 128ll << 20 ? 4 : 2; }

@@ -34,7 +34,7 @@ bool weights_past_the_cache(int groups, long long rows_hint, int N, int K) {
 }
 
 // How a grouped product is cut: the height of its tiles in bands of 32 rows (10, 8, 6: phased_gemm_kernel, 256
-// columns; 4, 2: dense_gemm_kernel, 128 columns), 0 where rows of K are too long for any. `rows_hint` rows over all
+// columns; 4: dense_gemm_kernel, 2: sliced_gemm_kernel, 128 columns, and grouped_slices on some of the others), 0 where rows of K are too long for any. `rows_hint` rows over all
 // groups are taken to be spread as uniform routing spreads them: a group's number is normal around the average.
 //
 // A tile costs per step of K what its unit has to fetch, in rows of 128 bytes, about 3 ns each (32 groups of 256 rows,
@@ -108,7 +108,8 @@ bool streams_far_ahead(long long rows_hint, int groups, int N) {
   return groups * std::max(1.0 - std::exp(-average), average / 32 + 0.5) * ((N + 63) / 64) <= 512;
 }
 
-// Tiles of ring_gemm_kernel (rows x columns), or none, for a grouped product. Groups with a row, and their row tiles, are
+// Tiles of a ring of steps (rows x columns), or none, for a grouped product: those of 32 rows are ring_gemm_kernel's, those of 64, which it had when the
+// times below were taken, sliced_gemm_kernel's by now (grouped_slices). Groups with a row, and their row tiles, are
 // counted as uniform routing would have them, and `of_*` is how many tiles that makes per unit.
 //
 // As long as every unit has one tile at most a ring is ahead of expert_gemm_kernel, on 32 x 32 up to 40 rows per group, on 32 x 64
@@ -191,7 +192,7 @@ RingTile grouped_ring(long long rows_hint, int groups, int N, int K) {
 // 4096 x 4096 x 512 (256) 22.2 / 27.4; 8192 x 8192 x 3696 (1024) 407 / 622.
 enum LinearWay {
   SPLIT_32, SPLIT_64,                  // skinny_gemm_kernel, 32 or 64 rows x 32 columns
-  TILES_64x128, TILES_128x128,         // dense_gemm_kernel
+  TILES_64x128, TILES_128x128,         // sliced_gemm_kernel (linear_slices), dense_gemm_kernel
   PHASED_128, PHASED_192, PHASED_256,  // phased_gemm_kernel, 128 x 128, 192 x 128 or 256 x 256
   STREAM_WEIGHTS                       // expert_gemm_kernel, as one group
 };
@@ -235,7 +236,7 @@ LinearWay linear_way(long long M, long long N, long long K, long long* least_cos
   return best;
 }
 
-// Whether a plain product goes to ring_gemm_kernel instead. With K too short to be split it is ahead on tiles of 32 x 32 as
+// Whether a plain product goes to a ring of steps instead (ring_gemm_kernel's when the times below were taken, sliced_gemm_kernel's by now). With K too short to be split it is ahead on tiles of 32 x 32 as
 // long as every unit has one at most, but for walks that end before the ring is filled: 1 to 7 steps take 1.11, 1.07, 1.05, 1.01, 0.99,
 // 0.96 and 0.93 of the others' time (284 products). Above, tiles of 64 x 64, which it has under way for longer than dense_gemm_kernel and which fetch
 // no more than skinny_gemm_kernel does, fill a gap between those two; a wait of 300 in the comparison above finds them (280 to 320 choose
