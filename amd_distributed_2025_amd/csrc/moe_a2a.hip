@@ -5536,7 +5536,7 @@ int launch_combine_send(const moe_a2a_shape* s, const void* expert_y, const int3
   const bool planned = send_back_plan && plan_supported(s);
   // (the planned path has no scan to repeat per piece, so a row can be split among more waves)
   const long long stream_bytes = (long long)rows_hint * s->hidden_dim * 2;
-  const bool past = g.vec16 && send_past(stream_bytes, g.row_vecs);
+  const bool past = stream_bytes >= EXPERT_PAST_BYTES;
   const int planned_nvw = planned_send_vecs(stream_bytes, g.row_vecs);
   if (planned && g.vec16 && g.nvw > planned_nvw) {
     g.nvw = planned_nvw;

@@ -24,18 +24,15 @@ bool items_fit(long long rows, int chunks) { return rows * chunks <= INT_MAX / 2
 // us of a graph of stages 1, 2, expert, 3 and 4, plain / nontemporal loads in one stage (8 entries per token, 14 KB but where said):
 //  - expert, four vectors per lane / two and nontemporal: 2.3 MB 17.8 / 17.8, 15 MB 29.9 / 30.0, 29 MB 49.5 / 47.0, 46 MB 78.8 / 74.3, 134
 //    MB of 4 KB 214 / 198, 235 MB 377 / 348, 470 MB 720 / 716 (its rows then fill the cache behind L2 for stage 3 to push out: below)
-//  - stage 3: 15 MB 29.7 / 30.2, 29 MB 47.2 / 47.0, 46 MB 72.1 / 71.0, 69 MB 99.8 / 98.3, 134 MB of 4 KB 193.9 / 189.0, 235 MB 340 / 329. Rows that
-//    no expert has just written are still in the cache behind L2, where nontemporal loads lose; graph of stages 1, 2, 3 and 4, and of those with the
-//    expert, plain / nontemporal: 28 MB 35.4 / 38.4, 45.1 / 45.3, 43 MB 55.3 / 58.3, 69.1 / 68.3, 51 MB 64.2 / 65.4, 78.6 / 76.6, 54 MB 69.5 / 69.4, 84.8 /
-//    81.7, 58 MB of 10 KB 85.2 / 80.1, 100.6 / 93.9, 62 MB of 8 KB 83.5 / 85.2, 100.8 / 99.8, 110 MB 131.5 / 134.6, 161.3 / 159.5; rows of up to 4 KB have it
-//    later: 16 MB of 4 KB 30.0 / 31.8, 36.6 / 37.4, 47 MB of 2 KB 82.1 / 88.1, 96.8 / 96.9, 70 MB of 4 KB 98.6 / 104.1, 120.2 / 120.2, 125 MB of 4 KB 161.6 /
-//    160.0, 190.8 / 189.8, 187 MB 259 / 236, 286 / 281.
+//  - stage 3: 15 MB 29.7 / 30.2, 29 MB 47.2 / 47.0, 46 MB 72.1 / 71.0, 69 MB 99.8 / 98.3, 134 MB of 4 KB 193.9 / 189.0, 235 MB 340 / 329. That is one set of
+//    buffers again and again, most of which the caches keep. Whole calls of a rank on six sets in turn, and by themselves between fills of 700 MB: 29 MB 53.5 / 51.1,
+//    64.3 / 61.4, compact and skewed 49.6 / 48.0, 55.1 / 52.1, 24 MB of 5.8 KB 54.7 / 53.3, 65.1 / 62.3, 31 MB of 4 KB 66.9 / 65.4, 78.5 / 75.3, 47 MB of 2 KB 103.1 /
+//    100.4, 112.7 / 105.2, 45 MB 78.2 / 74.8, 94.2 / 91.7; on one set 44.8 / 45.3, 36.8 / 36.9, 48.0 / 47.9, 59.2 / 59.5, 96.5 / 96.7, 68.9 / 69.1. What loses is a stage 3 whose
+//    rows no expert has written since it last read them: the graph of stages 1, 2, 3 and 4 alone, 28 MB 35.4 / 38.4, 43 MB 55.3 / 58.3, 54 MB 69.5 / 69.4. A job has an expert there.
 //  - stage 2, four vectors per lane / two / two and nontemporal: 29 MB 47.2 / 46.6 / 47.2, 46 MB - / 74.2 / 72.0, 69 MB 102.2 / 102.1 /
 //    101.1, 134 MB of 8 KB 196.0 / 194.2 / 192.7, 275 MB 395 / 393 / 378, 470 MB 682 / 676 / 663; of rows of up to 4 KB one vector per lane:
 //    134 MB of 4 KB, two / one 195.2 / 193.5, 67 MB of 2 KB 128.0 / 123.9, 16 MB of 2 KB 48.8 / 47.8.
 constexpr long long EXPERT_PAST_BYTES = 24ll << 20, RECV_PAST_BYTES = 40ll << 20;
-
-bool send_past(long long bytes, int row_vecs) { return bytes >= (row_vecs > BLOCK ? 48ll << 20 : 120ll << 20); }
 
 // The expert's results go past the cache behind L2 only where it could hold little of them, else through it (Store):
 // 134 MB 198 / 205, 268 MB 497 / 510, 336 MB 708 / 685 and, the other stages at their best, 658 / 664; 470 MB 716 / 682 and 649 / 637.

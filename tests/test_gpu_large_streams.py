@@ -13,7 +13,7 @@ from tests.test_gpu_parity import DEV, EDGE
 pytestmark = pytest.mark.gpu
 
 
-# rows of each stream: 42 to 49 MB, above the lines of the expert and of stage 2
+# rows of each stream: 42 to 49 MB, above the lines of the expert, of stage 3 and of stage 2
 @pytest.mark.parametrize("hidden_dim,tokens,K,dtype", [
     (1032, 2560, 8, "bf16"),   # 129 vectors: a piece of one vector, one lane of it used
     (2048, 2816, 4, "fp16"),   # 256: whole pieces of one
@@ -69,11 +69,11 @@ def test_stage_one_of_long_streams(W, E, K, hidden_dim, tokens):
 @pytest.mark.parametrize("layout", ["padded", "compact"])
 def test_a_few_rows_in_a_launch_for_hundreds_of_megabytes(hidden_dim, layout):
     """The expert and stage 3 size their launches and choose their kernels by the caller's row count, which may lie above the
-    rows that there are: below and above 24, 48, 120, 256 and 384 MB the same rows give the same results."""
+    rows that there are: below and above 24, 256 and 384 MB the same rows give the same results."""
     nle, tokens = 3, 37
     cfg = MoEConfig(nle, 2, hidden_dim, tokens, torch.bfloat16, torch.bfloat16)
     results = []
-    for megabytes in (0, 25, 50, 125, 300, 400):
+    for megabytes in (0, 25, 50, 300, 400):
         a = HIPAllToAll(cfg, 0, 1, device=DEV, layout=layout, compact_rows=96 if layout == "compact" else None)
         gen = torch.Generator(device=DEV)
         gen.manual_seed(7)

@@ -30,7 +30,6 @@ def rules(tmp_path_factory):
                    'extern "C" int through(long long rows, long long row_bytes) { return recv_through(rows, row_bytes); }\n'
                    'extern "C" int lanes(long long tokens, long long entries, int ranks, int row_vecs, int vec16) {\n'
                    '  return local_few_vecs(tokens, entries, ranks, row_vecs, vec16); }\n'
-                   'extern "C" int past_in_stage_3(long long bytes, int row_vecs) { return send_past(bytes, row_vecs); }\n'
                    'extern "C" int vecs_of_stage_2(long long bytes, int row_vecs) { return planned_recv_vecs(bytes, row_vecs); }\n'
                    'extern "C" int long_of(long long tokens, int k, int ranks, int row_vecs, int vec16) {\n'
                    '  return long_tokens(send_way(tokens, k, ranks, row_vecs, vec16), tokens, k, ranks, row_vecs, vec16); }\n'
@@ -58,7 +57,7 @@ def rules(tmp_path_factory):
     dll.tokens_of_stage_4.argtypes = [C.c_longlong, C.c_longlong, C.c_int]
     dll.tokens_of_jobs.argtypes = [C.c_longlong] + [C.c_int] * 3
     dll.vecs_of_stage_3.argtypes = dll.vecs_of_jobs.argtypes = [C.c_longlong, C.c_int]
-    dll.vecs_of_stage_2.argtypes = dll.past_in_stage_3.argtypes = [C.c_longlong, C.c_int]
+    dll.vecs_of_stage_2.argtypes = [C.c_longlong, C.c_int]
     return dll
 
 
@@ -195,15 +194,6 @@ def test_lanes_that_move_several_vectors_have_stores_for_a_megabyte_and_more(rul
             for vecs in (256, 257, 300, 512, 513, 896, 1025, 4096):
                 least = next((T for T in range(W, 2048 // K + 1) if rules.lanes(T, T * K, W, vecs, 1) > 1), None)
                 assert least is None or least * K * vecs * 16 >= 1 << 20, (W, K, vecs)
-
-
-@pytest.mark.parametrize("rows,hidden,past", [
-    (2013, 7168, False), (3145, 7168, False), (3981, 7168, True), (4819, 7168, True), (5964, 5120, True), (32613, 7168, True),
-    (4102, 2048, False), (17946, 2048, False), (23895, 1024, False), (47920, 2048, True),
-])
-def test_rows_of_stage_3_past_the_caches(rules, rows, hidden, past):
-    """Timed on the GPU, with an expert in front and without: rows that the cache behind L2 still holds lose up to 8 % of the four stages."""
-    assert rules.past_in_stage_3(rows * hidden * 2, hidden // 8) == past
 
 
 @pytest.mark.parametrize("rows,hidden,vecs", [
