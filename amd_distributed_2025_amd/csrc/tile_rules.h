@@ -257,8 +257,8 @@ RingTile linear_ring(long long M, long long N, long long K) {
 }
 
 // Tiles of sliced_gemm_kernel (rows x columns), or none.
-enum SlicedTile { NO_SLICES = 0, SLICES_64x32, SLICES_32x64, SLICES_64x64, SLICES_64x128, SLICES_128x128, SLICES_192x128 };
-int sliced_rows(SlicedTile t) { return t == SLICES_32x64 ? 32 : t <= SLICES_64x128 ? 64 : t == SLICES_128x128 ? 128 : 192; }
+enum SlicedTile { NO_SLICES = 0, SLICES_32x64, SLICES_64x64, SLICES_64x128, SLICES_128x128, SLICES_192x128, SLICES_64x32 };
+int sliced_rows(SlicedTile t) { return t == SLICES_32x64 ? 32 : t <= SLICES_64x128 || t == SLICES_64x32 ? 64 : t == SLICES_128x128 ? 128 : 192; }
 int sliced_cols(SlicedTile t) { return t == SLICES_64x32 ? 32 : t <= SLICES_64x64 ? 64 : 128; }
 
 // For a grouped product; `ring` and `bands`: what grouped_ring and (from 56 rows per group on, else 0) grouped_tile_bands have chosen. It takes 64 x
@@ -282,15 +282,19 @@ SlicedTile grouped_slices(RingTile ring, int bands, long long rows_hint, int gro
 
 // For a plain product; `ring` and `way`: what linear_ring and, without one, linear_way have chosen. It takes over all of the ring's tiles, all of 64 x
 // 128 (on the smallest tiles of which every unit has one at most, else as they are), and of the products split over K those of 33 to 96 rows that
-// give nearly every unit a tile: of 64 x 32 up to 64 rows, with weights that the L2s hold, and of 32 x 64 above, from 14 steps on. Of 300
-// products (16 to 8192 rows, N 1024 to 8192, K 256 to 8192) 98, at 0.86 of the others' time, none behind. us, 37 x 7808 x 448 on 64 x 128 / 64 x 64 / 32 x 64: 5.59 / 4.82 / 4.76; 148 x 3680 x 448 (87, 174 and 290 tiles) 5.71 /
-// 4.92 / 5.86; 500 x 2976 x 448 (192, 376, 752) 5.86 / 6.56 / 8.28. Up to 64 rows, split over K /
-// 32 x 64, of which two wait for the same weights / 64 x 32, calls with the same weights and with others out of HBM: 64 x 7168 x 2304 (31.5 MiB) 9.1 / 8.8 / 8.7,
-// 12.2 / 12.3 / 11.9; 60 x 7616 x 1688 8.3 / 7.2 / 7.1, 12.1 / 12.7 / 12.2; 52 x 7904 x 1592 7.5 / 6.9 / 6.8, 11.0 / 11.5 / 10.9; 64 x 8192 x 1024 6.1 /
-// 5.9 / 5.9, 7.8 / 7.7 / 7.5; but larger weights out of HBM 64 x 7008 x 3008 14.3 / 15.2 / 14.7 (and one launch right behind the other 64 x 7168 x 2304 12.2 / 13.8 / 13.4).
-// Above, in a graph, split / 32 x 64: 88 x 5056 x 2432 10.4 / 8.8, 13.9 / 12.3; 90 x 4480 x 6000 26.0 / 20.7, 32.2 / 30.7; of short walks 70 x 4704 x 688
-// 4.38 / 4.56, 5.74 / 5.82, 65 x 5056 x 568 4.12 / 4.18, 5.20 / 5.39; 66 x 5312 x 872 5.15 / 4.99, 6.63 / 6.63. With fewer tiles or more rows splitting K stays ahead: 52 x 5824 x 3624 (182 tiles)
-// 0.99 of its time here, 183 x 1120 x 960 (108) 1.24, 295 x 1536 x 8000 (240) 1.12.
+// give nearly every unit a tile: up to 64 rows, with weights that the L2s hold, of 64 x 32, which read every weight once (walks of eight steps, the
+// shortest that are split, of 32 x 64 as above), and of 32 x 64 above, from 14 steps on. Of 300 products (16 to 8192 rows, N 1024 to 8192, K 256 to
+// 8192) 98, at 0.86 of the others' time, none behind. us, 37 x 7808 x 448 on 64 x 128 / 64 x 64 / 32 x 64: 5.59 / 4.82 / 4.76; 148 x 3680 x 448 (87,
+// 174 and 290 tiles) 5.71 / 4.92 / 5.86; 500 x 2976 x 448 (192, 376, 752) 5.86 / 6.56 / 8.28.
+// Up to 64 rows, split over K / 32 x 64, of which two wait for the same weights / 64 x 32, calls with the same weights and with others out of HBM: 64 x
+// 7168 x 2304 (31.5 MiB) 9.1 / 8.8 / 8.7, 12.2 / 12.3 / 11.9; 60 x 7616 x 1688 8.3 / 7.2 / 7.1, 12.1 / 12.7 / 12.2; 52 x 7904 x 1592 7.5 / 6.9 / 6.8,
+// 11.0 / 11.5 / 10.9; 64 x 8192 x 1024 6.1 / 5.9 / 5.9, 7.8 / 7.7 / 7.5. In a graph: 62 x 6976 x 1960 8.7 / 7.6 / 7.7, 12.9 / 13.4 / 12.7; 33 x 7168 x
+// 1432 6.6 / 6.2 / 6.0, 9.5 / 8.7 / 8.2; 63 x 8160 x 568 4.6 / 4.2 / 4.2, 6.3 / 6.1 / 6.0; 33 x 7008 x 512 3.9 / 3.8 / 3.8, 5.0 / 4.8 / 4.7; over 33
+// products of 33 to 64 rows 64 x 32 takes 0.91 and 0.93 of the split's time, at worst 0.99 and 1.01. But larger weights out of HBM 64 x 7008 x 3008
+// 14.3 / 15.2 / 14.7 in calls.
+// Above, in a graph, split / 32 x 64: 88 x 5056 x 2432 10.4 / 8.8, 13.9 / 12.3; 90 x 4480 x 6000 26.0 / 20.7, 32.2 / 30.7; of short walks 70 x 4704 x
+// 688 4.38 / 4.56, 5.74 / 5.82, 65 x 5056 x 568 4.12 / 4.18, 5.20 / 5.39; 66 x 5312 x 872 5.15 / 4.99, 6.63 / 6.63. With fewer tiles or more rows
+// splitting K stays ahead: 52 x 5824 x 3624 (182 tiles) 0.99 of its time here, 183 x 1120 x 960 (108) 1.24, 295 x 1536 x 8000 (240) 1.12.
 // 192 x 128 stay phased_gemm_kernel's: launched one after the other in a graph they are up to 4 % ahead here, in calls of their own 2 to 3 % behind
 // (2048 x 2880 x 360 9.98 / 10.16, 1399 x 3904 x 3016 42.6 / 43.8).
 SlicedTile linear_slices(RingTile ring, LinearWay way, long long M, long long N, long long K) {
@@ -301,8 +305,9 @@ SlicedTile linear_slices(RingTile ring, LinearWay way, long long M, long long N,
   if ((way != SPLIT_32 && way != SPLIT_64) || M <= 32 || M > 96) return NO_SLICES;
   const long long of_round = M <= 64 ? tiles(64, 32) : tiles(32, 64);
   if (of_round < 200 || of_round > UNITS) return NO_SLICES;
-  if (M <= 64) return N * K * 2 <= 32 << 20 ? SLICES_64x32 : NO_SLICES;
-  return (K + 63) / 64 >= 14 ? SLICES_32x64 : NO_SLICES;
+  const long long steps = (K + 63) / 64;
+  if (M <= 64) return N * K * 2 > 32 << 20 ? NO_SLICES : steps > 8 ? SLICES_64x32 : SLICES_32x64;
+  return steps >= 14 ? SLICES_32x64 : NO_SLICES;
 }
 
 }  // namespace

@@ -12,7 +12,7 @@ from amd_distributed_2025_amd import HIPAllToAll, MoEConfig, gemm_rs
 
 DEV = "cuda:0"
 DT = pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-TILES = ["64x32", "32x64", "64x64", "64x128", "128x128", "192x128"]  # SlicedTile, from 1 on
+TILES = ["32x64", "64x64", "64x128", "128x128", "192x128"]  # SlicedTile, from 1 on
 STEPS = [8, 64, 72, 128, 136, 192, 200, 264, 328, 512]
 # tile -> groups, out_dim, rows per group that the caller promises; K
 GROUPED = {"64x64": (3, 160, 70, [264, 320, 328, 384, 1000, 2048]), "64x128": (3, 2080, 200, STEPS), "128x128": (3, 2080, 400, STEPS),
@@ -20,8 +20,7 @@ GROUPED = {"64x64": (3, 160, 70, [264, 320, 328, 384, 1000, 2048]), "64x128": (3
 # weights that are read past the caches (rows of one tile per group)
 STREAMED = {"64x64": (8, 1024, 60, 16384), "64x128": (8, 3072, 58, 5632), "128x128": (8, 2048, 115, 8192), "192x128": (8, 2048, 150, 8192)}
 # rows, out_dim, K
-PLAIN = {"32x64": [(m, n, k) for m, n in [(1, 1056), (65, 2016)] for k in [8, 64, 128, 192, 200]] + [(70, 5024, 1544), (96, 5440, 2048), (65, 4288, 840)],
-         "64x32": [(33, 6400, 512), (64, 8192, 520), (50, 7008, 2048), (64, 7168, 2304), (48, 6432, 1000), (63, 8160, 1544)],
+PLAIN = {"32x64": [(m, n, k) for m, n in [(1, 1056), (65, 2016)] for k in [8, 64, 128, 192, 200]] + [(70, 5024, 1544), (96, 5440, 2048), (33, 7008, 512)],
          "64x64": [(m, n, k) for m, n in [(513, 1056), (300, 2016)] for k in [8, 64, 128, 192, 200]] + [(200, 4064, 1544), (511, 2016, 2048)],
          "64x128": [(m, n, k) for m, n in [(700, 2016), (321, 4128)] for k in STEPS] + [(700, 2016, 2048)]}
 
@@ -62,13 +61,6 @@ def test_the_sizes_here_reach_every_tile(chosen):
     for tile, shapes in PLAIN.items():
         for shape in shapes:
             assert TILES[chosen.plain(*shape) - 1] == tile, (tile, shape)
-
-
-@pytest.mark.parametrize("shape", [(70, 4704, 688), (65, 5056, 568), (79, 4576, 664), (96, 5376, 832), (64, 7008, 3008), (64, 8224, 520), (64, 6368, 520),
-                                   (32, 8192, 1024), (97, 4096, 2048)])
-def test_products_that_stay_split_over_k(chosen, shape):
-    """Timed on the GPU, the first three and the fifth: up to 8 % slower on tiles that walk K whole, from HBM or from L2. The others lie past the rule's lines."""
-    assert chosen.plain(*shape) == 0
 
 
 def check_grouped(tile, groups, N, rows, K, counts, bias, dt):
