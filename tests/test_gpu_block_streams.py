@@ -1,6 +1,5 @@
 """Stage 1 against a stable sort: `dispatch_block_kernel` (four tokens per workgroup, keys counted by destination in bytes) on every
-cut of a row, `dispatch_long_kernel` (up to 64 entries per workgroup, counted likewise), and the numbers of tokens, entries, ranks and row
-lengths where they and the kernels of short streams begin and end."""
+cut of a row, and the numbers of tokens, entries, ranks and row lengths where it and the kernels of short streams begin and end."""
 import numpy as np
 import pytest
 import torch
@@ -27,21 +26,18 @@ def check(W, E, K, H, T, indices):
 
 
 # ranks, experts, entries per token, hidden, tokens -> the kernel, and for dispatch_block_kernel vectors per lane and pieces of a
-# row, for dispatch_long_kernel tokens of a workgroup (csrc/stream_rules.h; test_stream_rules.py holds the cases to that)
+# row (csrc/stream_rules.h; test_stream_rules.py holds the cases to that)
 CASES = {
     (8, 16, 1, 8, 1281): ("block", 1, 1), (1, 3, 3, 24, 427): ("block", 1, 1), (8, 64, 4, 64, 257): ("block", 1, 1),
-    (2, 2, 1, 1000, 1282): ("block", 2, 1), (8, 256, 8, 520, 1023): ("long", 4), (8, 256, 8, 520, 639): ("block", 2, 1), (3, 15, 5, 1032, 410): ("block", 2, 2),
+    (2, 2, 1, 1000, 1282): ("block", 2, 1), (8, 256, 8, 520, 1023): ("block", 2, 1), (3, 15, 5, 1032, 410): ("block", 2, 2),
     (5, 10, 3, 4104, 700): ("block", 2, 5), (4, 4, 1, 1032, 1290): ("block", 4, 1), (8, 88, 2, 2048, 1601): ("block", 4, 1),
-    (4, 8, 4, 4104, 1601): ("long", 4), (4, 8, 3, 6144, 1650): ("block", 4, 3), (8, 16, 2, 7168, 1605): ("block", 4, 4), (2, 4, 1, 2056, 3001): ("block", 6, 1),
+    (4, 8, 4, 4104, 1601): ("block", 4, 3), (8, 16, 2, 7168, 1605): ("block", 4, 4), (2, 4, 1, 2056, 3001): ("block", 6, 1),
     (8, 8, 1, 4096, 3007): ("block", 8, 1), (3, 3, 1, 6144, 1285): ("block", 12, 1), (2, 4, 1, 7168, 1301): ("block", 14, 1),
     (2, 2, 1, 8192, 1283): ("block", 16, 1), (2, 2, 1, 8200, 1282): ("block", 16, 2),
     (2, 6, 16, 37, 66): ("block", 16, 1), (4, 8, 5, 2051, 300): ("block", 16, 3), (2, 4, 1, 3001, 2710): ("block", 16, 3),  # single elements
     (8, 16, 2, 2560, 700): ("block", 6, 1), (4, 8, 2, 4096, 661): ("block", 8, 1), (2, 4, 2, 7168, 650): ("block", 4, 4),
-    (8, 16, 3, 3072, 501): ("block", 6, 1), (8, 8, 8, 16, 4096): ("long", 8), (4, 32, 4, 8, 16320): ("long", 16),
-    (4, 32, 4, 3, 16320): ("block", 16, 1), (4, 32, 4, 3, 16321): "fanout",  # the most keys that 256 lanes count in bytes, and more
-    (4, 32, 4, 8, 16321): ("long", 16), (4, 32, 4, 8, 65280): ("long", 16), (4, 32, 4, 8, 65281): "fanout",  # and that 1024 do
-    (4, 256, 64, 16, 1021): ("long", 1), (8, 40, 20, 64, 3300): ("long", 3), (8, 16, 16, 1032, 4090): ("long", 4),  # many entries per token
-    (4, 16, 8, 728, 2235): ("block", 2, 1), (8, 64, 6, 1456, 2637): ("long", 10), (8, 8, 4, 4608, 3500): ("long", 4), (9, 18, 4, 8, 400): "fanout", (8, 32, 17, 8, 70): "fanout",
+    (8, 16, 3, 3072, 501): ("block", 6, 1), (8, 8, 8, 16, 4096): ("block", 1, 1), (4, 32, 4, 8, 16320): ("block", 1, 1),
+    (4, 32, 4, 8, 16321): "fanout", (9, 18, 4, 8, 400): "fanout", (8, 32, 17, 8, 70): "fanout",
     (7, 21, 6, 4104, 345): "wide fanout", (5, 10, 7, 7168, 1799): "wide fanout", (9, 18, 2, 24, 700): "by entry",
     # two and eight entries ranked per pass, in one, two and nine passes, ids in registers and past them
     (9, 36, 11, 2056, 400): "wide fanout", (9, 36, 11, 4104, 130): "wide fanout", (9, 18, 6, 2056, 700): "wide fanout",

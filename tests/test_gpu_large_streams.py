@@ -28,21 +28,16 @@ def test_streams_of_more_than_40_mb(hidden_dim, tokens, K, dtype):
     run_long(generate_world(spec, 3), long_stream_rows=0)
 
 
-# ranks, experts, entries per token, hidden, tokens -> tokens of a workgroup of dispatch_long_kernel
-LONG_CASES = {
-    (8, 16, 1, 8, 5120): 20,     # the shortest it takes, one entry per token; a vector per row
-    (3, 15, 5, 520, 1024): 4,    # 65 vectors, experts per rank no power of two
-    (2, 6, 6, 1032, 2561): 10,   # 60 entries in a workgroup, the last of which owns one token
-    (8, 8, 7, 64, 2311): 9,      # an expert per rank
-    (4, 256, 64, 16, 1021): 1,   # 64 entries of a token, more entries than the kernel before it takes
-    (5, 20, 3, 3208, 1800): 4,   # 401 vectors: twice as many workgroups
-    (4, 8, 4, 4104, 2000): 2,    # 513: four times
-    (2, 4, 2, 8, 32641): 32,     # 65282 entries
-    (1, 2, 1, 7168, 5121): 11,
-}
-
-
-@pytest.mark.parametrize("W,E,K,hidden_dim,tokens", LONG_CASES)
+@pytest.mark.parametrize("W,E,K,hidden_dim,tokens", [
+    (8, 16, 1, 8, 5120),     # the shortest it takes, one entry per token; a vector per row, 20 tokens a workgroup
+    (3, 15, 5, 520, 1024),   # 65 vectors, experts per rank no power of two
+    (2, 6, 6, 1032, 2561),   # 60 entries in a workgroup, the last of which owns one token
+    (8, 8, 7, 64, 2311),     # an expert per rank, nine tokens each
+    (4, 256, 64, 16, 81),    # a token per workgroup, with 64 entries
+    (5, 20, 3, 3208, 1800),  # 401 vectors: twice as many workgroups
+    (2, 4, 2, 8, 32641),     # 65282 entries, more than the kernel before it takes
+    (1, 2, 1, 7168, 5121),
+])
 def test_stage_one_of_long_streams(W, E, K, hidden_dim, tokens):
     print(f"stage 1, {W} ranks x {tokens} tokens x {K} of {hidden_dim}", flush=True)
     spec = dict(world_size=W, num_experts=E, experts_per_token=K, hidden_dim=hidden_dim, max_num_tokens=tokens,
@@ -73,7 +68,7 @@ def test_a_few_rows_in_a_launch_for_hundreds_of_megabytes(hidden_dim, layout):
     nle, tokens = 3, 37
     cfg = MoEConfig(nle, 2, hidden_dim, tokens, torch.bfloat16, torch.bfloat16)
     results = []
-    for megabytes in (0, 25, 50, 300, 400):
+    for megabytes in (0, 25, 300, 400):
         a = HIPAllToAll(cfg, 0, 1, device=DEV, layout=layout, compact_rows=96 if layout == "compact" else None)
         gen = torch.Generator(device=DEV)
         gen.manual_seed(7)
@@ -144,83 +139,3 @@ def test_planned_places_of_many_tiles(W, nle, K, tokens, exact_hints):
     spec = dict(world_size=W, num_experts=W * nle, experts_per_token=K, hidden_dim=16, max_num_tokens=tokens,
                 num_tokens="full", routing="zipf", weights="rand", dtype="bf16")
     run_compact(generate_world(spec, 5), exact_hints=exact_hints, binding="ext" if exact_hints else "ctypes")
-
-
-def test_planned_places_of_a_shape_that_could_hold_far_more():
-    """128 experts that could each take 1.2 million rows, of which 4100 arrive: more than the experts' pieces could be numbered."""
-    W, nle, H, R = 8, 128, 7168, 4100
-    a = HIPAllToAll(MoEConfig(W * nle, 1, H, 150000, torch.bfloat16, torch.bfloat16), 3, W, device=DEV, layout="compact", compact_rows=4200)
-    gen = torch.Generator(device=DEV)
-    gen.manual_seed(1)
-    recv = torch.randn(R, H, device=DEV, generator=gen).to(torch.bfloat16)
-    meta = torch.randint(0, 1000, (R, 5), device=DEV, generator=gen, dtype=torch.int32)
-    meta[:, 0] = 3 * nle + torch.randint(0, nle, (R,), device=DEV, generator=gen, dtype=torch.int32)
-    counts = torch.tensor([R - 70] + [10] * 7, dtype=torch.int32, device=DEV)
-    num, ex, em = a.dispatch_recv(counts, recv, meta, R)
-    torch.cuda.synchronize()
-    order = torch.argsort(meta[:, 0], stable=True)
-    assert torch.equal(ex[:R], recv[order]) and torch.equal(em[:R], meta[order])
-    want = torch.bincount(meta[:, 0] - 3 * nle, minlength=nle)
-    assert torch.equal(num.long(), want) and torch.equal(a.expert_offsets[1:].long(), want.cumsum(0))
-
-
-# hidden, rows -> vectors per lane; more than the 40 MB from which stage 2 reads rows past the caches
-RECV_PAST_CASES = {(1032, 20500): 1, (2048, 10300): 1, (2056, 10300): 2, (7168, 3000): 2, (7168, 21200): 1}
-
-
-@pytest.mark.parametrize("hidden_dim,rows", RECV_PAST_CASES)
-@pytest.mark.parametrize("layout", ["padded", "compact"])
-@pytest.mark.parametrize("plan", [True, False])
-def test_stage_2_of_large_streams(hidden_dim, rows, layout, plan):
-    print(f"stage 2, {rows} rows of {hidden_dim}, {layout}, plan {plan}", flush=True)
-    W, nle = 2, 3
-    a = HIPAllToAll(MoEConfig(W * nle, 1, hidden_dim, rows, torch.bfloat16, torch.bfloat16), 1, W, device=DEV, reuse_placement=plan,
-                    layout=layout, compact_rows=rows + 5 if layout == "compact" else None)
-    a.long_stream_rows = 0
-    gen = torch.Generator(device=DEV)
-    gen.manual_seed(rows)
-    recv = torch.randint(-30000, 30000, (rows + 9, hidden_dim), device=DEV, generator=gen, dtype=torch.int16).view(torch.bfloat16)
-    meta = torch.randint(0, 1000, (rows + 9, 5), device=DEV, generator=gen, dtype=torch.int32)
-    meta[:, 0] = nle + torch.randint(0, nle, (rows + 9,), device=DEV, generator=gen, dtype=torch.int32)
-    counts = torch.tensor([rows - 700, 700], dtype=torch.int32, device=DEV)  # (nine rows more than arrived lie in the buffers)
-    num, ex, em = a.dispatch_recv(counts, recv, meta, rows)
-    torch.cuda.synchronize()
-    le = meta[:rows, 0] - nle
-    assert torch.equal(num.long(), torch.bincount(le, minlength=nle))
-    first = 0
-    for e in range(nle):
-        of, n = torch.nonzero(le == e).flatten(), int(num[e])
-        got, got_meta = (ex[first:first + n], em[first:first + n]) if layout == "compact" else (ex[e, :n], em[e, :n])
-        assert torch.equal(got.view(torch.int16), recv[of].view(torch.int16)) and torch.equal(got_meta, meta[of]), e
-        first += n
-
-
-# hidden, entries per token, tokens -> vectors per lane; rows and results of more than the 80 MB from which stage 4 reads past the caches
-MAPPED_PAST_CASES = {(2048, 1, 10300): 2, (7168, 2, 2000): 2, (4104, 3, 2560): 2, (2056, 4, 4100): 2, (512, 4, 16500): 1, (3080, 6, 1950): 1,
-                     (1032, 8, 4600): 1}
-
-
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("hidden_dim,K,tokens", MAPPED_PAST_CASES)
-def test_stage_4_of_large_streams(hidden_dim, K, tokens, dtype):
-    """With a table against the kernels that scan, which other files hold to the oracle. A third of the rows names other tokens' entries, and some lie past
-    the counts."""
-    print(f"stage 4, {tokens} tokens x {K} of {hidden_dim} {dtype}", flush=True)
-    a = HIPAllToAll(MoEConfig(16, K, hidden_dim, tokens, dtype, dtype), 0, 2, device=DEV)
-    a.long_stream_rows = 0
-    gen = torch.Generator(device=DEV)
-    gen.manual_seed(tokens)
-    S = tokens * K
-    order = torch.randperm(S, device=DEV, generator=gen)
-    meta = torch.stack([order, order, order // K, order % K, order], 1).int()
-    meta[::3, 2] += tokens
-    rows = torch.randn(S, hidden_dim, device=DEV, generator=gen).to(dtype)
-    weights = torch.rand(tokens, K, device=DEV, generator=gen)
-    counts = torch.tensor([S - 900, 800], dtype=torch.int32, device=DEV)
-    start = torch.randn(tokens, hidden_dim, device=DEV, generator=gen).to(dtype)
-    for accumulate in (True, False):
-        got = [start.clone() for _ in range(2)]
-        for y, unique in zip(got, (True, False)):
-            a.combine_recv(y, weights, counts, rows, meta, accumulate=accumulate, unique_pairs=unique)
-        torch.cuda.synchronize()
-        assert "entry_row" in a._ws and torch.equal(*[y.view(torch.int16) for y in got]), accumulate
