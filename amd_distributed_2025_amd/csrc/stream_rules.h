@@ -24,11 +24,13 @@ bool items_fit(long long rows, int chunks) { return rows * chunks <= INT_MAX / 2
 // us of a graph of stages 1, 2, expert, 3 and 4, plain / nontemporal loads in one stage (8 entries per token, 14 KB but where said):
 //  - expert, four vectors per lane / two and nontemporal: 2.3 MB 17.8 / 17.8, 15 MB 29.9 / 30.0, 29 MB 49.5 / 47.0, 46 MB 78.8 / 74.3, 134
 //    MB of 4 KB 214 / 198, 235 MB 377 / 348, 470 MB 720 / 716 (its rows then fill the cache behind L2 for stage 3 to push out: below)
-//  - stage 3: 15 MB 29.7 / 30.2, 29 MB 47.2 / 47.0, 46 MB 72.1 / 71.0, 69 MB 99.8 / 98.3, 134 MB of 4 KB 193.9 / 189.0, 235 MB 340 / 329. That is one set of
-//    buffers again and again, most of which the caches keep. Whole calls of a rank on six sets in turn, and by themselves between fills of 700 MB: 29 MB 53.5 / 51.1,
-//    64.3 / 61.4, compact and skewed 49.6 / 48.0, 55.1 / 52.1, 24 MB of 5.8 KB 54.7 / 53.3, 65.1 / 62.3, 31 MB of 4 KB 66.9 / 65.4, 78.5 / 75.3, 47 MB of 2 KB 103.1 /
-//    100.4, 112.7 / 105.2, 45 MB 78.2 / 74.8, 94.2 / 91.7; on one set 44.8 / 45.3, 36.8 / 36.9, 48.0 / 47.9, 59.2 / 59.5, 96.5 / 96.7, 68.9 / 69.1. What loses is a stage 3 whose
-//    rows no expert has written since it last read them: the graph of stages 1, 2, 3 and 4 alone, 28 MB 35.4 / 38.4, 43 MB 55.3 / 58.3, 54 MB 69.5 / 69.4. A job has an expert there.
+//  - stage 3: 15 MB 29.7 / 30.2, 29 MB 47.2 / 47.0, 46 MB 72.1 / 71.0, 69 MB 99.8 / 98.3, 134 MB of 4 KB 193.9 / 189.0, 235 MB 340 / 329.
+//    That is one set of buffers again and again, most of which the caches keep. Whole calls of a rank on six sets in turn, and by themselves between
+//    fills of 700 MB: 29 MB 53.1 / 50.8, 64.3 / 61.4, compact and skewed 53.0 / 51.7, 59.7 / 57.3, 24 MB of 5.8 KB 54.7 / 53.3, 65.1 / 62.3, 31 MB of 4
+//    KB 66.9 / 65.4, 78.5 / 75.3, 47 MB of 2 KB 103.1 / 100.4, 112.7 / 105.2, 45 MB 78.2 / 74.8, 94.2 / 91.7; on one set 46.3 / 46.3, 55.2 / 55.3,
+//    48.0 / 47.9, 59.2 / 59.5, 96.5 / 96.7, 68.9 / 69.1. What loses is a stage 3 whose rows no expert has written since it last read them, which the
+//    cache behind L2 then still holds: the graph of stages 1, 2, 3 and 4 alone, 28 MB 35.4 / 38.4, 43 MB 55.3 / 58.3, 54 MB 69.5 / 69.4. A job has an
+//    expert there. (Loads of another scope, sc0 and sc1, take the same as without, with and without nt.)
 //  - stage 2, four vectors per lane / two / two and nontemporal: 29 MB 47.2 / 46.6 / 47.2, 46 MB - / 74.2 / 72.0, 69 MB 102.2 / 102.1 /
 //    101.1, 134 MB of 8 KB 196.0 / 194.2 / 192.7, 275 MB 395 / 393 / 378, 470 MB 682 / 676 / 663; of rows of up to 4 KB one vector per lane:
 //    134 MB of 4 KB, two / one 195.2 / 193.5, 67 MB of 2 KB 128.0 / 123.9, 16 MB of 2 KB 48.8 / 47.8.
@@ -38,10 +40,10 @@ constexpr long long EXPERT_PAST_BYTES = 24ll << 20, RECV_PAST_BYTES = 40ll << 20
 // 134 MB 198 / 205, 268 MB 497 / 510, 336 MB 708 / 685 and, the other stages at their best, 658 / 664; 470 MB 716 / 682 and 649 / 637.
 constexpr long long EXPERT_STREAM_BYTES = 384ll << 20;
 
-// Vectors per lane of the movers of a planned stage 2: one for rows of up to 4 KB, and for those of more than 8 KB that the cache behind L2 holds none
-// of; us of stages 1, 2, 3 and 4, and of a whole step, two / one: 14 KB 185 MB 216.5 / 219.1, 318.3 / 319.4, 240 MB 279.6 / 285.7, 411.6 / 413.3, 294 MB
-// 366.9 / 362.1, 531.8 / 533.1, 348 MB 435.8 / 425.8, 634.8 / 638.2, 446 MB 549.1 / 538.6, 803.5 / 802.6; 10 KB 319 MB 389.5 / 385.9, 510.6 / 511.9; 8 KB 312
-// MB 389.6 / 390.8, 513.3 / 515.8; 6 KB 328 MB 429.8 / 427.1, 557.4 / 559.7.
+// Vectors per lane of the movers of a planned stage 2: one for rows of up to 4 KB, and for those of more than 8 KB that the cache behind L2 holds
+// none of; us of stages 1, 2, 3 and 4, and of a whole step, two / one: 14 KB 185 MB 216.5 / 219.1, 318.3 / 319.4, 240 MB 279.6 / 285.7, 411.6 / 413.3,
+// 294 MB 366.9 / 362.1, 531.8 / 533.1, 348 MB 435.8 / 425.8, 634.8 / 638.2, 446 MB 549.1 / 538.6, 803.5 / 802.6; 10 KB 319 MB 389.5 / 385.9, 510.6 /
+// 511.9; 8 KB 312 MB 389.6 / 390.8, 513.3 / 515.8; 6 KB 328 MB 429.8 / 427.1, 557.4 / 559.7.
 int planned_recv_vecs(long long bytes, int row_vecs) { return row_vecs > BLOCK && (row_vecs <= 2 * BLOCK || bytes < 288ll << 20) ? 2 : 1; }
 
 // Vectors per lane of a planned stage 3: four (a 256-vector piece per wave) made a whole step 0.5 us shorter at 2048 rows of 14 KB than the
@@ -131,22 +133,29 @@ SendWay send_way(long long tokens, int per_token, int ranks, int row_vecs, bool 
 }
 
 // Tokens of a workgroup of dispatch_long_kernel, or 0 where a stream stays with its choice above. From 5120 entries on it takes whole vectors over from
-// dispatch_block_kernel, and from 65281 on from all others, which compare every key with every entry. It stays behind with few tokens and entries (its
-// workgroups then hold three and four tokens: 722 of 272 bytes, 8 per token 5.4 / 6.1 us, 1005 of 5.6 KB, 6 each 11.1 / 12.2), below 5120 entries (4900, 613 tokens
-// of 900 bytes, 6.2 / 6.4), and with short rows just past the entries that a workgroup per unit holds (2803 of 1.9 KB, 6 each 14.8 / 15.7,
-// 2235 of 1.5 KB, 8 each 14.1 / 15.0, 2225 of 272 bytes 12.7 / 13.4). Over 513 streams of 5120 to 32768 entries, one to eight per token, rows of 128 bytes to 14 KB, the choice takes
-// 0.893 of the others' time; 31 are more than 3 % behind, the worst by 10 % (1123 tokens of 1.8 KB, 8 each 8.1 / 8.9).
+// dispatch_block_kernel, and from 65281 on from all others, which compare every key with every entry. It stays behind
+//  - below 5120 entries (4900, 613 tokens of 900 bytes, 6.2 / 6.4 us) and with few tokens and entries, of which a workgroup then holds three or four (722 of
+//    272 bytes, 8 per token 5.4 / 6.1, 1005 of 5.6 KB, 6 each 11.1 / 12.2),
+//  - with five and more entries per token, of which a workgroup holds few tokens, just past a batch of 8192 keys, which is another pass: rows of 1 to 6.4 KB,
+//    8193 to 10240 entries, 107 streams 1.03 on average (1836 of 2.3 KB, 5 each 9.2 / 10.1, 1627 of 2.7 KB, 6 each 10.3 / 11.3, 1046 of 1.9 KB, 8 each
+//    8.0 / 8.7; of up to 8192 entries 0.96, of up to 1 KB 0.99), and past two batches and the entries that a workgroup per unit holds rows of up to 3 KB
+//    (2803 of 1.9 KB, 6 each 14.8 / 15.7, 2235 of 1.5 KB, 8 each 14.1 / 15.0, 2225 of 272 bytes 12.7 / 13.4).
+// Over 700 streams of 5120 to 32768 entries, one to eight per token, rows of 128 bytes to 14 KB, one launch after another, the choice takes 0.74 of the
+// time of dispatch_block_kernel; 26 are more than 3 % behind, the worst by 10 % (4108 tokens of 11 KB, 3 each 35.3 / 39.0).
 //
 // Short rows have one workgroup per unit, which leaves the passes over the keys to the fewest, as long as those hold all tokens (64 entries each);
-// others two, and where a row takes longer than a pass four. us, with 256 / 512 / 768 / 1024 workgroups: 3590 tokens of 1 KB, 3 per token 7.5 / 10.6 / 14.4; 2675 of 2.1 KB, 6
-// each 15.4 / 13.0 / 15.7; 2055 of 5.8 KB, 4 each 14.2 / 15.2 / 16.8; 3594 of 6.3 KB, 8 each 40.5 / 40.7 / 41.1 / 44.4; 3212 of 5 KB, 5 each 28.6 / 24.5 / 24.1 /
-// 25.0; 3731 of 14.3 KB, 4 each 63.9 / 62.5 / 59.1 / 57.2; 4084 of 11.2 KB, 6 each 60.9 / 60.3 / 60.2 / 56.6; 4096 of 14 KB, 8 each, with the other stages, - / 809 / 815 / 807.
+// others two, and where a row takes longer than a pass four. us, with 256 / 512 / 768 / 1024 workgroups: 3590 tokens of 1 KB, 3 per token 7.5 / 10.6 /
+// 14.4; 2675 of 2.1 KB, 6 each 15.4 / 13.0 / 15.7; 2055 of 5.8 KB, 4 each 14.2 / 15.2 / 16.8; 3594 of 6.3 KB, 8 each 40.5 / 40.7 / 41.1 / 44.4; 3212 of
+// 5 KB, 5 each 28.6 / 24.5 / 24.1 / 25.0; 3731 of 14.3 KB, 4 each 63.9 / 62.5 / 59.1 / 57.2; 4084 of 11.2 KB, 6 each 60.9 / 60.3 / 60.2 / 56.6; 4096 of
+// 14 KB, 8 each, with the other stages, - / 809 / 815 / 807.
 int long_tokens(SendWay way, long long tokens, int per_token, int ranks, int row_vecs, bool vec16) {
   const long long entries = tokens * per_token;
   if (!vec16 || ranks > BLOCK_RANKS || per_token > 64 || entries < LONG_ENTRIES || entries > LONG_MAX_ENTRIES ||
       (way != SEND_BLOCK && entries <= BLOCK_MAX_ENTRIES))
     return 0;
-  if ((tokens < 1024 && entries < 6400) || (row_vecs <= 128 && per_token >= 6 && entries >= 16800 && entries <= 18432)) return 0;
+  if (tokens < 1024 && entries < 6400) return 0;
+  if (per_token >= 5 && row_vecs > 64 && row_vecs <= 400 && entries > 8192 && entries <= 10240) return 0;
+  if (per_token >= 6 && row_vecs <= 192 && entries >= 16800 && entries <= 18432) return 0;
   const bool one_each = row_vecs <= (entries <= 9216 ? 400 : 256) && tokens <= 64 / per_token * 264;
   const int workgroups = one_each ? 256 : row_vecs > 512 && entries >= 7500 ? 1024 : 512;
   return (int)std::min<long long>(64 / per_token, (tokens + workgroups - 1) / workgroups);
@@ -154,8 +163,8 @@ int long_tokens(SendWay way, long long tokens, int per_token, int ranks, int row
 
 // Vectors per lane of a wave of dispatch_block_kernel, for rows that a wave has in one go with `nvw`. Rows
 // are cut into pieces of two vectors per lane where there are few workgroups otherwise, else of four: pieces of 2 / 4 /
-// whole rows: 250 tokens of 5.8 KB, 8 per token 4.8 / 5.1 / 5.5 us. (Whole vectors come here with up to 5119 entries, and with some more of short rows:
-// long_tokens. So pieces of four are rows of more than 8 KB with three entries and more than 1600 tokens.) With one entry a piece would do little but rank: 2000 of 14 KB 13.4 / 10.7 / 9.6. Two and three
+// whole rows: 250 tokens of 5.8 KB, 8 per token 4.8 / 5.1 / 5.5 us. (Whole vectors come here with up to 5119 entries, and with some more of rows of up to
+// 6.4 KB: long_tokens.) With one entry a piece would do little but rank: 2000 of 14 KB 13.4 / 10.7 / 9.6. Two and three
 // entries pay for a piece of long rows only, two for one of four vectors: 1292 of 5 KB, 2 per token 7.1 / 6.6 / 5.9, 1380 of 15 KB 14.0 /
 // 12.6 / 12.4, 1001 of 13.7 KB 8.5 / 8.0 / 9.2, 671 of 10.8 KB 6.1 / 5.5 / 5.8; 893 of 4.5 KB, 3 per token 6.1 / 5.5 / 5.3, 537 of 13.6 KB
 // 6.5 / 7.0 / 7.2.

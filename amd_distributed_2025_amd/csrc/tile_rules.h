@@ -34,8 +34,8 @@ bool weights_past_the_cache(int groups, long long rows_hint, int N, int K) {
 }
 
 // How a grouped product is cut: the height of its tiles in bands of 32 rows (10, 8, 6: phased_gemm_kernel, 256
-// columns; 4: dense_gemm_kernel, 2: sliced_gemm_kernel, 128 columns, and grouped_slices on some of the others), 0 where rows of K are too long for any. `rows_hint` rows over all
-// groups are taken to be spread as uniform routing spreads them: a group's number is normal around the average.
+// columns; 4: dense_gemm_kernel, 2: sliced_gemm_kernel, 128 columns; grouped_slices has some of the others too), 0 where rows of K are too long
+// for any. `rows_hint` rows over all groups are taken to be spread as uniform routing spreads them: a group's number is normal around the average.
 //
 // A tile costs per step of K what its unit has to fetch, in rows of 128 bytes, about 3 ns each (32 groups of 256 rows,
 // 2048 x 4096, tiles of 192 rows: 37 KB a microsecond and unit, 40 without the MFMAs; the MFMAs without the loads take
@@ -236,10 +236,10 @@ LinearWay linear_way(long long M, long long N, long long K, long long* least_cos
   return best;
 }
 
-// Whether a plain product goes to a ring of steps instead (ring_gemm_kernel's when the times below were taken, sliced_gemm_kernel's by now). With K too short to be split it is ahead on tiles of 32 x 32 as
-// long as every unit has one at most, but for walks that end before the ring is filled: 1 to 7 steps take 1.11, 1.07, 1.05, 1.01, 0.99,
-// 0.96 and 0.93 of the others' time (284 products). Above, tiles of 64 x 64, which it has under way for longer than dense_gemm_kernel and which fetch
-// no more than skinny_gemm_kernel does, fill a gap between those two; a wait of 300 in the comparison above finds them (280 to 320 choose
+// Whether a plain product goes to a ring of steps instead (ring_gemm_kernel's when the times below were taken, sliced_gemm_kernel's by now). With K
+// too short to be split it is ahead on tiles of 32 x 32 as long as every unit has one at most, but for walks that end before the ring is filled: 1 to 7
+// steps take 1.11, 1.07, 1.05, 1.01, 0.99, 0.96 and 0.93 of the others' time (284 products). Above, tiles of 64 x 64, which it has under way for longer
+// than dense_gemm_kernel and which fetch no more than skinny_gemm_kernel does, fill a gap between those two; a wait of 300 in the comparison above finds them (280 to 320 choose
 // the same of 95 shapes), from 12 steps on (shorter ones are as fast elsewhere). us, linear_way's choice / here:
 //   137 x 4320 x 5440  47.9 / 25.7     200 x 4096 x 4096  36.9 / 21.4     82 x 6592 x 2816  27.1 / 16.9
 //   494 x 2048 x 2176  20.1 / 13.4     128 x 8192 x 2048  21.2 / 14.9    195 x 3008 x 832    7.7 /  7.5

@@ -74,6 +74,15 @@ def test_tokens_of_a_workgroup_for_long_streams(rules, tokens, k, hidden, own):
     assert rules.long_of(tokens, k, 8, *row(hidden)) == own
 
 
+@pytest.mark.parametrize("tokens,k,hidden,own", [
+    (1836, 5, 1144, 0), (1627, 6, 1336, 0), (1736, 5, 1416, 0), (1046, 8, 944, 0), (1892, 5, 1608, 0), (1443, 6, 2024, 0), (2573, 7, 1528, 0), (2290, 8, 1304, 0),
+    (1024, 8, 944, 4), (2049, 5, 1144, 9), (1836, 5, 512, 8), (1836, 5, 3208, 4), (2060, 4, 1144, 9), (2400, 7, 1544, 5),
+])
+def test_streams_just_past_a_batch_of_keys(rules, tokens, k, hidden, own):
+    """Timed on the GPU: with five and more entries per token another pass over the keys costs up to 10 % more than dispatch_block_kernel."""
+    assert rules.long_of(tokens, k, 8, *row(hidden)) == own
+
+
 def test_limits_of_the_kernel_of_long_streams(rules):
     """(64 entries in a workgroup, keys that 1024 lanes count in bytes, whole vectors, eight ranks)"""
     for tokens in (1, 79, 80, 640, 1023, 1024, 2048, 2112, 2113, 4080, 5120, 16320, 16321, 65280, 65281, 261120, 261121):
