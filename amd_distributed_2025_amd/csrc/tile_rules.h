@@ -239,8 +239,8 @@ LinearWay linear_way(long long M, long long N, long long K, long long* least_cos
 // Whether a plain product goes to a ring of steps instead (ring_gemm_kernel's when the times below were taken, sliced_gemm_kernel's by now). With K
 // too short to be split it is ahead on tiles of 32 x 32 as long as every unit has one at most, but for walks that end before the ring is filled: 1 to 7
 // steps take 1.11, 1.07, 1.05, 1.01, 0.99, 0.96 and 0.93 of the others' time (284 products). Above, tiles of 64 x 64, which it has under way for longer
-// than dense_gemm_kernel and which fetch no more than skinny_gemm_kernel does, fill a gap between those two; a wait of 300 in the comparison above finds them (280 to 320 choose
-// the same of 95 shapes), from 12 steps on (shorter ones are as fast elsewhere). us, linear_way's choice / here:
+// than dense_gemm_kernel and which fetch no more than skinny_gemm_kernel does, fill a gap between those two; a wait of 300 in the comparison
+// above finds them (280 to 320 choose the same of 95 shapes), from 12 steps on (shorter ones are as fast elsewhere). us, linear_way's choice / here:
 //   137 x 4320 x 5440  47.9 / 25.7     200 x 4096 x 4096  36.9 / 21.4     82 x 6592 x 2816  27.1 / 16.9
 //   494 x 2048 x 2176  20.1 / 13.4     128 x 8192 x 2048  21.2 / 14.9    195 x 3008 x 832    7.7 /  7.5
 // and on 32 x 32: 15 x 5888 x 448 5.5 / 4.7, 80 x 2176 x 448 5.6 / 4.8, 4 x 7104 x 280 5.0 / 4.4; but 33 x 4608 x 352 5.3 / 5.5.
@@ -262,22 +262,33 @@ int sliced_rows(SlicedTile t) { return t == SLICES_32x64 ? 32 : t <= SLICES_64x1
 int sliced_cols(SlicedTile t) { return t == SLICES_64x32 ? 32 : t <= SLICES_64x64 ? 64 : 128; }
 
 // For a grouped product; `ring` and `bands`: what grouped_ring and (from 56 rows per group on, else 0) grouped_tile_bands have chosen. It takes 64 x
-// 64 and 64 x 128 over from both, and where uniform routing would make for 0.8 of a round of them over the units at most, 128 x 128 from
-// dense_gemm_kernel and 192 x 128 from that and from 192 x 256. (Above, one group of many rows makes a second round: 341 rows in 6 groups by Zipf's
-// routing, 4992 x 672, 0.91 of a round for uniform routing, 16.2 / 24.1 us on 64 x 128 / 128 x 128.) Of 500 products (4 to 64 groups, 1 to 3500 rows
-// per group, N and K of 512 to 7168, a third of them with Zipf's routing) 90 go there, and take of the others' time, as geometric means: those of 64 x
-// 128 of a ring 0.85 and of dense_gemm_kernel 0.67, of 64 x 64 0.94 (2 of 26 more than 3 % behind), of dense_gemm_kernel's 128 x 128 0.84, of 192 x 256
-// 0.80. With fewer rows expert_gemm_kernel stays, whose small blocks read weights from HBM as fast: 42 groups of 25, 1280 x 896, on
+// 64 and 64 x 128 over from both: of 500 products (4 to 64 groups, 1 to 3500 rows per group, N and K of 512 to 7168, a third of them with Zipf's
+// routing) those of 64 x 128 of a ring take 0.85 and of dense_gemm_kernel 0.67 of the others' time, of 64 x 64 0.94 (2 of 26 more than 3 % behind).
+//
+// Taller tiles have a workgroup per unit, and a few tiles past a round make a second one. Skewed routing has more of them than uniform routing: by
+// Zipf's a group adds 0.6 of a tile to those that its rows fill (the median; nine of ten at most 0.7 of 128 rows, 0.75 of 192). So 128 x 128
+// from dense_gemm_kernel and 192 x 128 from 192 x 256 go there where such tiles fit a round, and uniform routing's 0.9 of one. Where 128 x 128 do not,
+// 192 x 128 do as well as dense_gemm_kernel while that has one round, and are up to 1.7 times as fast where it begins another. us, the kernel
+// before / here, with uniform and with Zipf's routing: 27 groups of 173, 864 x 2536, whose 192 x 128 are 0.79 of a round and 1.18, 47.8 / 37.0, 43.9 /
+// 67.3 (they stay); 30 of 152, 736 x 536, 1.4 rounds of 128 x 128, 20.6 / 13.0, 18.2 / 23.0; 8 of 214, 1984 x 6688 with a popularity that falls with
+// the root of the rank 106.6 / 73.7; 7 of 166, 2048 x 2576, 0.87 of a round of 128 x 128, on 192 x 128 30.3 / 33.7, 28.7 / 33.4 (128 x 128 it is).
+// Of 600 products (2 to 64 groups, 56 to 1500 rows per group, N and K of 512 to 7168, uniform routing's tiles 1.15 rounds at most), each with these three
+// kinds of routing, the choice takes 0.920 of the time of the kernels before, 22 of 1800 more than 3 % behind, by 26 % at most (with 0.8 of a round
+// for uniform routing as the only line 0.934, 57, 53 %; the fastest of the three tiles 0.865).
+// With fewer rows expert_gemm_kernel stays, whose small blocks read weights from HBM as fast: 42 groups of 25, 1280 x 896, on
 // 64 x 128 23.6 / 23.4 us, 896 x 1280 28.2 / 30.2, and where those are few 41.9 / 54.7 (20 of 23, 768 x 6464).
 SlicedTile grouped_slices(RingTile ring, int bands, long long rows_hint, int groups, int N) {
-  constexpr double UNITS = 256, MOST = 0.8;
+  constexpr double UNITS = 256;
   if (ring) return ring == RING_64x64 ? SLICES_64x64 : ring == RING_64x128 ? SLICES_64x128 : NO_SLICES;
   if (bands == 2) return SLICES_64x128;
-  auto of_a_unit = [&](int high) {
-    return tiles_of_groups((double)rows_hint / groups, groups, high).each * groups * ((N + 127) / 128) / UNITS;
-  };
-  if (bands == 4 && of_a_unit(128) <= MOST) return SLICES_128x128;
-  return (bands == 4 || bands == 6) && of_a_unit(192) <= MOST ? SLICES_192x128 : NO_SLICES;
+  if (bands != 4 && bands != 6) return NO_SLICES;
+  const double columns = (N + 127) / 128;
+  auto uniform = [&](int high) { return tiles_of_groups((double)rows_hint / groups, groups, high).each * groups * columns / UNITS; };
+  auto skewed = [&](int high, double of_group) { return ((double)rows_hint / high + of_group * groups) * columns / UNITS; };
+  if (bands == 6) return uniform(192) <= 0.9 && skewed(192, 0.7) <= 1 ? SLICES_192x128 : NO_SLICES;
+  if (uniform(128) <= 0.9 && skewed(128, 0.7) <= 1) return SLICES_128x128;
+  const bool second_round = uniform(128) > 0.95 && uniform(192) <= 0.8;
+  return second_round || (skewed(128, 1.0) > 1 && uniform(192) <= 0.9 && skewed(192, 0.8) <= 1) ? SLICES_192x128 : NO_SLICES;
 }
 
 // For a plain product; `ring` and `way`: what linear_ring and, without one, linear_way have chosen. It takes over all of the ring's tiles, all of 64 x
