@@ -337,7 +337,8 @@ class HIPAllToAll:
             ex = self._buf("expert_x", (nle, self.max_recv, cfg.hidden_dim), cfg.in_dtype)
             em = self._buf("expert_meta", (nle, self.max_recv, META_DIM), torch.int32)
         long_from = self._long_from("compact" if compact else "dispatch")
-        if hint > long_from:
+        # (a binding of the caller's own may know the compact call without places)
+        if hint > long_from and not (compact and type(self.binding) not in _binding.KINDS):
             pos = self._at_least("row_position", capacity)
         self._plan_made_for = None if plan is None else (em.data_ptr(), num.data_ptr())
         fresh = self._learn("recv", "learn_recv", num, ex, em, self.expert_offsets if compact else None, plan, long_from)
@@ -346,8 +347,8 @@ class HIPAllToAll:
         if fresh and self._calls.dispatch_recv(recv_counts, recv_buf, recv_meta, hint) is not None:
             pass
         elif compact:
-            self.binding.dispatch_recv_compact(self.shape, recv_buf, recv_meta, recv_counts, hint, num,
-                                               self.expert_offsets, ex, em, plan, _stream(self.device), pos)
+            self.binding.dispatch_recv_compact(self.shape, recv_buf, recv_meta, recv_counts, hint, num, self.expert_offsets,
+                                               ex, em, plan, _stream(self.device), *([] if pos is None else [pos]))
         else:
             self.binding.dispatch_recv(self.shape, recv_buf, recv_meta, recv_counts, hint, num, ex, em, plan,
                                        _stream(self.device), pos)

@@ -3,7 +3,7 @@ test_long_stream_rules.py holds the sizes to the kernels that they are meant for
 import pytest
 import torch
 
-from amd_distributed_2025_amd import HIPAllToAll
+from amd_distributed_2025_amd import HIPAllToAll, _binding
 from amd_distributed_2025_amd.task import MoEConfig
 from tests import test_gpu_block_streams as block_streams
 from tests import test_gpu_combine_block as combine_block
@@ -78,6 +78,32 @@ def test_planned_places_of_a_shape_that_could_hold_far_more():
     assert torch.equal(ex[:R], recv[order]) and torch.equal(em[:R], meta[order])
     want = torch.bincount(meta[:, 0] - 3 * nle, minlength=nle)
     assert torch.equal(num.long(), want) and torch.equal(a.expert_offsets[1:].long(), want.cumsum(0))
+
+
+@pytest.mark.parametrize("rows", [40, 4096, 5000])
+def test_a_binding_whose_compact_call_takes_no_places(rows):
+    class Own(_binding.CtypesBinding):
+        def dispatch_recv_compact(self, shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens, expert_offsets, expert_x,
+                                  expert_meta, send_back_plan, stream):
+            calls.append(rows_hint)
+            super().dispatch_recv_compact(shape, recv_buf, recv_meta, recv_counts, rows_hint, expert_num_tokens, expert_offsets, expert_x,
+                                          expert_meta, send_back_plan, stream)
+
+    calls, got = [], []
+    for own in (True, False):
+        a = HIPAllToAll(MoEConfig(6, 1, 64, 5000, torch.bfloat16, torch.bfloat16), 0, 2, device=DEV, layout="compact")
+        if own:
+            a.binding = Own()
+        gen = torch.Generator(device=DEV)
+        gen.manual_seed(rows)
+        recv = torch.randn(rows, 64, device=DEV, generator=gen).to(torch.bfloat16)
+        meta = torch.randint(0, 3, (rows, 5), device=DEV, generator=gen, dtype=torch.int32)
+        counts = torch.tensor([rows - 9, 9], dtype=torch.int32, device=DEV)
+        num, ex, em = a.dispatch_recv(counts, recv, meta, rows)
+        got.append((num, a.expert_offsets, ex[:rows], em[:rows]))
+    torch.cuda.synchronize()
+    assert calls == [rows]
+    assert all(torch.equal(p, q) for p, q in zip(*got))
 
 
 # hidden, rows -> vectors per lane; more than the 40 MB from which stage 2 reads rows past the caches
